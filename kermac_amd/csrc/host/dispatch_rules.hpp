@@ -21,6 +21,8 @@
     X(WIDE_K_CONTIGUOUS_MIN_TILES, 48)                                                                  \
     X(WIDE_K_CONTIGUOUS_MIN_TILES_TIMES_K, 36864)                                                       \
     X(WIDE_K_CONTIGUOUS_MIN_ROWS, 129)     /* in both directions */                                     \
+    /* the product kernel's tile: 256 x 128 from this many of them over the batch on, 128 x 128 below */    \
+    X(WIDE_LARGE_TILE_MIN_TILES, 4096)                                                                  \
     /* sums of products through the workspace (the alternative is the direct kernel) */                 \
     X(DOT_MIN_K, 128)                                                                                   \
     X(DOT_MIN_TILES, 64)                                                                                \

@@ -11,8 +11,8 @@
 //   gram_f16_split   scales every row by a power of two that puts its largest magnitude into
 //                    [2^14, 2^15), splits every scaled value x into h1 = fp16(x), h2 = fp16(x - h1)
 //                    and writes the pieces in the order the matrix instruction reads them.
-//   gram_f16_wide    one workgroup of 8 waves per 256 x 256 tile of the result: copies pieces from
-//                    the workspace into LDS and multiplies; a1 b1 + a1 b2 + a2 b1, fp32 accumulators.
+//   gram_f16_wide    one workgroup of 4 waves per 256 x 128 tile of the result (128 x 128 where those are few): copies
+//                    pieces from the workspace into LDS and multiplies; a1 b2 + a1 b1 + a2 b1, fp32 accumulators.
 //
 // Accuracy.  x - h1 is exact in fp32 and h2 keeps 11 of its bits: |x - h1 - h2| <= 2^-22 |x|, or
 // 2^-25 where h2 is subnormal, which is 2^-39 of the row's largest magnitude.  The dropped product
@@ -25,23 +25,21 @@
 // Scales are powers of two, so scaling and unscaling round nothing.  Rows that hold an infinity or
 // a NaN produce results that are not numbers, which are distrusted and recomputed like any other.
 //
-// Why two fp16 pieces and not the three bf16 pieces of gram_bf16_kernel.hpp: measured with this
-// same kernel structure at M = N = 30000, K = 1024, the board is power-limited (shader clock
-// 1.87 GHz with copies and matrix instructions running together, 2.37 GHz with either alone; the
-// matrix pipeline is busy two thirds of the cycles in all three cases), so time follows energy:
-// six products of three pieces 8.9 ms, three products of two pieces 5.4 ms.  Why a workspace: a
-// value is split once instead of once per tile that needs it (in the one-step kernel the split
-// takes as long as the matrix instructions it hides behind), a 256 x 256 tile asks the L2 for half
-// the bytes per matrix instruction of a 128 x 128 one, and the layout of an operand in memory
+// Why two fp16 pieces and not the three bf16 pieces of gram_bf16_kernel.hpp: the board is power-limited under this kernel
+// (at 16384 x 16384 x 4096 it multiplies at 1785 TFLOP/s on operands of zeros and at 1352 on normal ones, plain fp16
+// library products of the same size at 1718 and 1452), so time follows energy, and three products cost half of six.
+// Why a workspace: a value is split once instead of once per tile that needs it (in the one-step kernel the split
+// takes as long as the matrix instructions it hides behind), and the layout of an operand in memory
 // only matters to the split.
+//
+// What the shape of the product kernel is worth, whole call at M = N = 30000, K = 1024, and sums of products at
+// 16384 x 16384 x 256: one workgroup of 8 waves per 256 x 256 tile and CU on v_mfma_f32_32x32x16_f16, with nothing beside
+// its prologue and stores, 5.83 and 0.686 ms; two workgroups of 256 x 128 on v_mfma_f32_16x16x32_f16 4.87 and 0.513 ms.
 //
 // Workspace of one operand and batch entry, in 16-byte chunks of 8 fp16 (one row, one half of a
 // 16-deep K slice, one piece):  chunk[slice][piece][half][row 0 .. rows_pad),  rows_pad a multiple
 // of 256; rows that do not exist and k beyond K hold zeros, so the product kernel has no edge
-// handling in its walk.  Four slices more than K has are allocated and never multiplied.
-// Two compile-time switches leave a part of the product kernel out, for the measurements of what
-// bounds it (the results are then wrong): -DGW_ABLATE_NO_COPY issues no copies from the workspace,
-// -DGW_ABLATE_NO_EPILOGUE returns behind the walk.
+// handling in its walk.  K is padded to whole steps of 32.
 // Statistics: partial[range][row] for the sums of squares and for the magnitudes, one partial per
 // range of K slices that a workgroup walks, combined in the order of the ranges.
 // The reference has no such path (include/build_a_kernel.cuh:339-370 is SIMT only).
@@ -54,14 +52,10 @@ namespace kmc {
 typedef _Float16 gram_half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 gram_half2 __attribute__((ext_vector_type(2)));
 
-constexpr int GW_TILE = 256;                                  // rows of a and of b per workgroup
-constexpr int GW_THREADS = 512;
+constexpr int GW_TILE = 256;                                  // rows of an operand are padded to this
 constexpr int GW_PIECES = 2;
 constexpr int GW_SEGMENTS = 2 * GW_PIECES;                    // (piece, half) pairs of one slice
-constexpr int GW_OPERAND_CHUNKS = GW_SEGMENTS * GW_TILE;      // 16 KB
-constexpr int GW_BUFFER_CHUNKS = 2 * GW_OPERAND_CHUNKS;       // one slice of both operands: 32 KB
-constexpr int GW_EXTRA_SLICES = 4;                            // copied ahead of the walk, never multiplied
-constexpr int GW_BAND_N = 32;                                 // tile order: n tiles per band
+constexpr int GW_BAND_N = 64;                                 // tile order: n tiles per band
 constexpr int GW_ROW_THREADS = 256;
 constexpr int GW_SCALE_EXPONENT = 14;                         // a row's largest magnitude goes to [2^14, 2^15)
 
@@ -263,22 +257,44 @@ __global__ __launch_bounds__(GW_ROW_THREADS) void gram_f16_split_pair(const Gram
     }
 }
 
-// Workgroup -> tile, as tile_of_workgroup of build_kernel.hpp with bands of GW_BAND_N tiles: a
-// CU holds one workgroup, so the 32 of an XCD cover 4 n tiles x 8 m tiles of a band at a time.
-// SYMMETRIC (a panel against itself): the ids count through the tiles on and below the diagonal,
-// row r of the triangle starting at id r (r + 1) / 2.
-template <bool SYMMETRIC>
+// Tile shapes of the product kernel.  A workgroup is 4 waves; a wave owns WAVE_M rows of a and WAVE_N rows of b as
+// 16 x 16 blocks of the matrix instruction.  Two workgroups (three of the small shape) share a CU, so that one's
+// prologue, epilogue and result stores run beside the other's matrix instructions.
+template <int TILE_M_, int TILE_N_>
+struct WideTile {
+    static constexpr int TILE_M = TILE_M_, TILE_N = TILE_N_;
+    static constexpr int THREADS = 256, WAVES = 4;
+    static constexpr int WAVES_M = 2, WAVES_N = 2;
+    static constexpr int WAVE_M = TILE_M / WAVES_M, WAVE_N = TILE_N / WAVES_N;
+    static constexpr int MT = WAVE_M / 16, NT = WAVE_N / 16;
+    static constexpr int PARTS_M = TILE_M / 128, PARTS_N = TILE_N / 128, PARTS = PARTS_M * PARTS_N;
+    static constexpr int GRANULE_CHUNKS = 4 * (TILE_M + TILE_N);          // 32 k of one piece of a and one of b
+    static constexpr int COPIES_A = TILE_M / 64, COPIES_B = TILE_N / 64;  // runs of 64 chunks per wave and granule
+    static constexpr int COPIES = COPIES_A + COPIES_B;
+    static constexpr int SLOTS = 3;
+    static constexpr int MIN_WAVES = TILE_M * TILE_N >= 256 * 128 ? 2 : 3;      // per SIMD
+};
+typedef WideTile<256, 128> WideTileLarge;
+typedef WideTile<128, 128> WideTileSmall;
+
+// Workgroup -> tile, as tile_of_workgroup of build_kernel.hpp with bands of GW_BAND_N n tiles: n fastest inside a band,
+// so the workgroups resident on an XCD (the hardware deals ids round-robin) cover a block of about 8 n tiles x 8 m tiles.
+// SYMMETRIC (a panel against itself): the ids count through the 256 x 256 blocks on and below the diagonal (row r of
+// the triangle starts at block r (r + 1) / 2), each of them the tiles of TILE_M x TILE_N it holds.
+template <typename Tile, bool SYMMETRIC>
 __device__ __forceinline__ bool wide_tile_of_workgroup(const GramWideArgs &args, int &tile_m, int &tile_n)
 {
     const int rotated = blockIdx.x + blockIdx.y % gridDim.x;
     const int linear = rotated >= (int)gridDim.x ? rotated - (int)gridDim.x : rotated;
     if (SYMMETRIC) {
-        int row = (int)((sqrtf(8.0f * (float)linear + 1.0f) - 1.0f) * 0.5f);
-        while (row * (row + 1) / 2 > linear) row--;
-        while ((row + 1) * (row + 2) / 2 <= linear) row++;
-        tile_m = row;
-        tile_n = linear - row * (row + 1) / 2;
-        return true;
+        constexpr int PER_M = GW_TILE / Tile::TILE_M, PER_N = GW_TILE / Tile::TILE_N;
+        const int block = linear / (PER_M * PER_N), inside = linear - block * (PER_M * PER_N);
+        int row = (int)((sqrtf(8.0f * (float)block + 1.0f) - 1.0f) * 0.5f);
+        while (row * (row + 1) / 2 > block) row--;
+        while ((row + 1) * (row + 2) / 2 <= block) row++;
+        tile_m = row * PER_M + inside % PER_M;
+        tile_n = (block - row * (row + 1) / 2) * PER_N + inside / PER_M;
+        return tile_m < args.wide_tiles_m && tile_n < args.wide_tiles_n && tile_n * Tile::TILE_N < (tile_m + 1) * Tile::TILE_M;
     }
     const int band_tiles = GW_BAND_N * args.wide_tiles_m;
     const int band = linear / band_tiles;
@@ -289,27 +305,169 @@ __device__ __forceinline__ bool wide_tile_of_workgroup(const GramWideArgs &args,
     return tile_n < args.wide_tiles_n;
 }
 
-// Wave w of 8 owns rows wave_m .. +128 of a and wave_n .. +64 of b: 4 x 2 matrix-instruction
-// tiles of 32 x 32, 128 accumulator registers, 24 matrix instructions per slice.
+// The walk.  A step is 32 k: three products of pieces, a1 b2 + a1 b1 + a2 b1, on v_mfma_f32_16x16x32_f16.
 //
-// The pieces go from the workspace straight into LDS (global_load_lds_dwordx4: a wave copies 64
-// consecutive chunks, no registers involved), four slices in four buffers.  One barrier per
-// slice.  The operands of a slice are read into registers during the slice before it, so behind
-// the barrier of slice s the buffer of slice s is free and takes slice s + 4, and slice s + 1,
-// whose copies were issued three slices earlier, is complete and is read.
+// Why the 16 x 16 form: with real data in the registers this instruction sustains 1.93 PFLOP/s and the 32 x 32 x 16 one
+// 1.71 (2.47 both on zeros: the board is power-limited, and the smaller tile moves half the accumulator words per
+// multiply-add).
 //
-// The copies are written as instructions: through the compiler's builtin every later LDS read
-// waits for every copy under way (the copies carry no information on which array they fill), which
-// leaves nothing in flight.  The compiler therefore does not count these copies either; the walk
-// waits for them itself, and no other vector load is issued between the first copy and the wait
-// for all of them behind the walk.
+// The pieces go from the workspace straight into LDS (global_load_lds_dwordx4: a wave copies 64 consecutive chunks, no
+// registers involved) in granules of one piece of a and one of b, in the order the products need them: a granule G1 is
+// {a1, b2} of a step, G2 is {a2, b1}; three slots of LDS in turn.  One set of operand registers is enough: a1 and b2
+// are not needed behind the product a1 b1, so the G1 of the next step is read during a2 b1; b1 and a2 are free behind
+// a2 b1, so G2 is read during a1 b2.  A barrier stands in front of each read: behind it the granule to be read has
+// arrived for every wave, and the one read before is free to be filled again.
 //
-// SYMMETRIC: b is a, the result is symmetric, and it is made so bit for bit: one workgroup per
-// tile on or below the diagonal; what lies below the diagonal is stored a second time, mirrored;
-// of a 128 x 128 part on the diagonal the lower triangle is stored and mirrored (the two halves of
-// such a part are computed with the pieces in exchanged roles and differ in the last bit); the
-// part above the diagonal inside a diagonal tile is not stored from its own values at all.  A
-// distrusted part is left to the repair launch, which mirrors what it recomputes.
+// The copies are written as instructions: through the compiler's builtin every later LDS read waits for every copy
+// under way (the copies carry no information on which array they fill), which leaves nothing in flight.  The compiler
+// therefore does not count these copies either; the walk waits for them itself, and no other vector load is issued
+// between the first copy and the end of the walk.  Nothing is copied beyond the last step.
+template <typename Tile>
+struct WideWalk {
+    typedef const __attribute__((address_space(1))) char *global_address;
+    typedef __attribute__((address_space(3))) void *lds_address;
+
+    const char *run_a[Tile::COPIES_A], *run_b[Tile::COPIES_B];      // uniform: piece 1 of a, piece 1 of b, step 0
+    i64 piece_a, piece_b, step_a, step_b;                           // bytes
+    unsigned lane_offset, lds_base, lds_run_a[Tile::COPIES_A], lds_run_b[Tile::COPIES_B];
+    gram_chunk *ring;
+    int read_a, read_b;
+
+    __device__ __forceinline__ void init(const gram_chunk *pieces_a, int rows_pad_a, int m0, const gram_chunk *pieces_b, int rows_pad_b,
+                                         int n0, gram_chunk *ring_, int lane, int wave, int wave_m, int wave_n)
+    {
+        ring = ring_;
+        lane_offset = 16u * lane;
+        lds_base = (unsigned)(unsigned long)(lds_address)ring;
+        // quarter q of a step's 32 k: slice q / 2, half q % 2 of the workspace's [slice][piece][half][row]
+        auto segment = [](int quarter, int rows_pad) { return (i64)((quarter >> 1) * GW_SEGMENTS + (quarter & 1)) * rows_pad; };
+#pragma unroll
+        for (int j = 0; j < Tile::COPIES_A; j++) {
+            const int run = wave + Tile::WAVES * j, quarter = run / (Tile::TILE_M / 64), part = run % (Tile::TILE_M / 64);
+            run_a[j] = reinterpret_cast<const char *>(pieces_a + segment(quarter, rows_pad_a) + m0 + 64 * part);
+            lds_run_a[j] = 1024u * run;
+        }
+#pragma unroll
+        for (int j = 0; j < Tile::COPIES_B; j++) {
+            const int run = wave + Tile::WAVES * j, quarter = run / (Tile::TILE_N / 64), part = run % (Tile::TILE_N / 64);
+            run_b[j] = reinterpret_cast<const char *>(pieces_b + segment(quarter, rows_pad_b) + n0 + 64 * part);
+            lds_run_b[j] = 64u * Tile::TILE_M + 1024u * run;
+        }
+        piece_a = 32ll * rows_pad_a; piece_b = 32ll * rows_pad_b;              // two segments of rows_pad chunks
+        step_a = 2 * 16ll * GW_SEGMENTS * rows_pad_a; step_b = 2 * 16ll * GW_SEGMENTS * rows_pad_b;
+        read_a = (lane >> 4) * Tile::TILE_M + wave_m + (lane & 15);
+        read_b = 4 * Tile::TILE_M + (lane >> 4) * Tile::TILE_N + wave_n + (lane & 15);
+    }
+
+    // Granule SECOND (0: {a1, b2}, 1: {a2, b1}) of step `step` into slot `slot`.
+    template <int SECOND>
+    __device__ __forceinline__ void copy(int step, int slot) const
+    {
+        const unsigned to = lds_base + (unsigned)slot * (16u * Tile::GRANULE_CHUNKS);
+        const i64 at_a = (i64)step * step_a + (SECOND ? piece_a : 0), at_b = (i64)step * step_b + (SECOND ? 0 : piece_b);
+#pragma unroll
+        for (int j = 0; j < Tile::COPIES_A; j++)
+            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                         : : "v"(lane_offset), "s"((global_address)(run_a[j] + at_a)), "s"(to + lds_run_a[j]) : "memory", "m0");
+#pragma unroll
+        for (int j = 0; j < Tile::COPIES_B; j++)
+            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                         : : "v"(lane_offset), "s"((global_address)(run_b[j] + at_b)), "s"(to + lds_run_b[j]) : "memory", "m0");
+    }
+
+    __device__ __forceinline__ void read(gram_half8 (&fa)[Tile::MT], gram_half8 (&fb)[Tile::NT], int slot, bool b_first) const
+    {
+        const gram_chunk *from = ring + slot * Tile::GRANULE_CHUNKS;
+        if (b_first) {
+#pragma unroll
+            for (int nt = 0; nt < Tile::NT; nt++) fb[nt] = __builtin_bit_cast(gram_half8, from[read_b + 16 * nt]);
+        }
+#pragma unroll
+        for (int mt = 0; mt < Tile::MT; mt++) fa[mt] = __builtin_bit_cast(gram_half8, from[read_a + 16 * mt]);
+        if (!b_first) {
+#pragma unroll
+            for (int nt = 0; nt < Tile::NT; nt++) fb[nt] = __builtin_bit_cast(gram_half8, from[read_b + 16 * nt]);
+        }
+    }
+};
+
+template <int COUNT>
+__device__ __forceinline__ void wide_wait_copies()
+{
+    static_assert(COUNT < 64, "vmcnt has six bits");
+    __builtin_amdgcn_s_waitcnt(0x0F70 | (COUNT & 15) | ((COUNT >> 4) << 14));     // vmcnt(COUNT), nothing else
+}
+
+// The matrix instructions are written out: left to itself the compiler gives their results other registers than their
+// sums came from, which does not fit beside the operands.  Two products into the same sums are at least 16 matrix
+// instructions apart, and wide_walk ends with the wait states that vector instructions need before they read the sums.
+template <int MT, int NT, int FIRST, int LAST>
+__device__ __forceinline__ void wide_multiply(gram_float4 (&acc)[MT][NT], const gram_half8 (&fa)[MT], const gram_half8 (&fb)[NT])
+{
+#pragma unroll
+    for (int mt = FIRST; mt < LAST; mt++)
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++)
+            asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(acc[mt][nt]) : "v"(fa[mt]), "v"(fb[nt]));
+}
+
+template <typename Tile>
+__device__ __forceinline__ void wide_walk(gram_float4 (&acc)[Tile::MT][Tile::NT], const WideWalk<Tile> &walk, int steps)
+{
+    constexpr int MT = Tile::MT, NT = Tile::NT, COPIES = Tile::COPIES;
+    gram_half8 a1[MT], a2[MT], b1[NT], b2[NT];
+    walk.template copy<0>(0, 0);
+    walk.template copy<1>(0, 1);
+    if (steps > 1) {
+        walk.template copy<0>(1, 2);
+        wide_wait_copies<2 * COPIES>();
+    } else {
+        wide_wait_copies<COPIES>();
+    }
+    __syncthreads();
+    walk.read(a1, b2, 0, true);
+    int slot = 0;                                       // of this step's first granule
+    for (int step = 0; step < steps; step++) {
+        const int second = slot == 2 ? 0 : slot + 1, third = second == 2 ? 0 : second + 1;
+        const bool more = step + 1 < steps;
+        wide_multiply<MT, NT, 0, MT / 2>(acc, a1, b2);
+        __builtin_amdgcn_sched_barrier(0);
+        if (more) wide_wait_copies<COPIES>();            // the second granule has arrived; the next step's first may be under way
+        else wide_wait_copies<0>();
+        __syncthreads();
+        walk.read(a2, b1, second, true);
+        if (more) walk.template copy<1>(step + 1, slot);
+        __builtin_amdgcn_sched_barrier(0);
+        wide_multiply<MT, NT, MT / 2, MT>(acc, a1, b2);
+        wide_multiply<MT, NT, 0, MT>(acc, a1, b1);
+        __builtin_amdgcn_sched_barrier(0);
+        if (more) {
+            wide_wait_copies<COPIES>();
+            __syncthreads();
+            walk.read(a1, b2, third, true);
+            if (step + 2 < steps) walk.template copy<0>(step + 2, second);
+            __builtin_amdgcn_sched_barrier(0);
+        } else {
+            // said out loud: with unread operands on one of the two ways here, the products below would wait for the
+            // reads just issued on the other
+            __builtin_amdgcn_s_waitcnt(0xC07F);          // lgkmcnt(0), nothing else
+        }
+        wide_multiply<MT, NT, 0, MT>(acc, a2, b1);
+        __builtin_amdgcn_sched_barrier(0);
+        slot = third;
+    }
+    asm volatile("s_nop 15\n\ts_nop 15");
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++) asm volatile("" : "+v"(acc[mt][nt]));
+}
+
+// SYMMETRIC: b is a, the result is symmetric, and it is made so bit for bit: the tiles on or below the diagonal are
+// computed; what lies below the diagonal is stored a second time, mirrored; of a 128 x 128 part on the diagonal the
+// lower triangle is stored and mirrored (the two halves of such a part are computed with the pieces in exchanged
+// roles and differ in the last bit); a part above the diagonal inside a tile is not stored from its own values at
+// all.  A distrusted part is left to the repair launch, which mirrors what it recomputes.
 //
 // EPILOGUE GW_EPILOGUE_GRADIENT_L2: the same walk as a plain product of the pieces, for the gradient
 // of the L2 norm (norm_gradient_l2_wide.hpp): no norms, no trust check, the epilogue combines the
@@ -318,23 +476,21 @@ __device__ __forceinline__ bool wide_tile_of_workgroup(const GramWideArgs &args,
 // EPILOGUE GW_EPILOGUE_DOT: the inner operator DOT (sum_k a b): the product of the pieces is the
 // value itself, nothing cancels, so there is no trust check and no repair; outer power, kernel
 // function, regularised diagonal and the stores, mirrored ones included, are those of the distance.
-template <bool SYMMETRIC, int EPILOGUE = GW_EPILOGUE_DISTANCE>
-__global__ __launch_bounds__(GW_THREADS) void gram_f16_wide(const GramWideArgs args)
+template <typename Tile, bool SYMMETRIC, int EPILOGUE = GW_EPILOGUE_DISTANCE>
+__global__ __launch_bounds__(Tile::THREADS, Tile::MIN_WAVES) void gram_f16_wide(const GramWideArgs args)
 {
-    __shared__ gram_chunk lds0[GW_BUFFER_CHUNKS];
-    __shared__ gram_chunk lds1[GW_BUFFER_CHUNKS];
-    __shared__ gram_chunk lds2[GW_BUFFER_CHUNKS];
-    __shared__ gram_chunk lds3[GW_BUFFER_CHUNKS];
-    __shared__ __attribute__((aligned(16))) float lds_norm_a[GW_TILE], lds_norm_b[GW_TILE];
-    __shared__ __attribute__((aligned(16))) float lds_unscale_a[GW_TILE], lds_unscale_b[GW_TILE];
-    __shared__ int lds_distrust[4];
+    constexpr int TILE_M = Tile::TILE_M, TILE_N = Tile::TILE_N, MT = Tile::MT, NT = Tile::NT;
+    __shared__ gram_chunk ring[Tile::SLOTS * Tile::GRANULE_CHUNKS];
+    __shared__ __attribute__((aligned(16))) float lds_norm_a[TILE_M], lds_norm_b[TILE_N];
+    __shared__ __attribute__((aligned(16))) float lds_unscale_a[TILE_M], lds_unscale_b[TILE_N];
+    __shared__ int lds_distrust[Tile::PARTS];
 
     const int tid = threadIdx.x;
     const int batch = blockIdx.y;
     int tile_m, tile_n;
-    if (!wide_tile_of_workgroup<SYMMETRIC>(args, tile_m, tile_n)) return;
-    const int m0 = tile_m * GW_TILE;
-    const int n0 = tile_n * GW_TILE;
+    if (!wide_tile_of_workgroup<Tile, SYMMETRIC>(args, tile_m, tile_n)) return;
+    const int m0 = tile_m * TILE_M;
+    const int n0 = tile_n * TILE_N;
     const int m_valid = args.kernel.m - m0;
     const int n_valid = args.kernel.n - n0;
 
@@ -342,11 +498,11 @@ __global__ __launch_bounds__(GW_THREADS) void gram_f16_wide(const GramWideArgs a
         // The sample of the result says that the repair launch would redo (nearly) every part: stamp them all
         // and leave (the branch is uniform over the launch: every workgroup reads the same words).  Parts above the diagonal of a symmetric result belong to nobody.
         if (args.kernel.sample && sample_leaves_it_to_the_direct_kernel(args.kernel.sample)) {
-            if (tid < 4) {
-                const int part_m = tid & 1, part_n = tid >> 1;
-                const bool above = SYMMETRIC && tile_m == tile_n && part_m < part_n;
-                if (!above && part_m * 128 < m_valid && part_n * 128 < n_valid)
-                    args.kernel.c[batch * args.kernel.c_bs + (i64)(n0 + part_n * 128) * args.kernel.c_ld + m0 + part_m * 128] =
+            if (tid < Tile::PARTS) {
+                const int part_m = tid % Tile::PARTS_M * 128, part_n = tid / Tile::PARTS_M * 128;
+                const bool above = SYMMETRIC && m0 + part_m < n0 + part_n;
+                if (!above && part_m < m_valid && part_n < n_valid)
+                    args.kernel.c[batch * args.kernel.c_bs + (i64)(n0 + part_n) * args.kernel.c_ld + m0 + part_m] =
                         __uint_as_float(BK_REPAIR_MARKER);
             }
             return;
@@ -355,346 +511,253 @@ __global__ __launch_bounds__(GW_THREADS) void gram_f16_wide(const GramWideArgs a
 
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wave_m = (wave & 1) * 128;
-    const int wave_n = (wave >> 1) * 64;
-    const int h = lane >> 5;
-    const int i = lane & 31;
+    const int wave_m = (wave % Tile::WAVES_M) * Tile::WAVE_M;
+    const int wave_n = (wave / Tile::WAVES_M) * Tile::WAVE_N;
 
     // Norms of this tile's rows (the partial sums in the order of their ranges) and their scales.
-    {
-        const bool of_a = tid < GW_TILE;
-        const int r = of_a ? tid : tid - GW_TILE;
-        const float *partial = of_a ? args.squares_a + batch * args.stats_a_bs + m0 + r : args.squares_b + batch * args.stats_b_bs + n0 + r;
-        const int pitch = of_a ? args.rows_pad_a : args.rows_pad_b;
-        // all loads first, then the sum in range order: a loop would wait for each load in turn,
-        // eight memory latencies before the first copy of the walk is issued
-        float parts[GW_MAX_RANGES];
+    for (int at = tid; at < TILE_M + TILE_N; at += Tile::THREADS) {
+        const bool of_a = at < TILE_M;
+        const int r = of_a ? at : at - TILE_M;
+        if constexpr (EPILOGUE == GW_EPILOGUE_DISTANCE) {
+            const float *partial = of_a ? args.squares_a + batch * args.stats_a_bs + m0 + r : args.squares_b + batch * args.stats_b_bs + n0 + r;
+            const int pitch = of_a ? args.rows_pad_a : args.rows_pad_b;
+            // all loads first, then the sum in range order: a loop would wait for each load in turn
+            float parts[GW_MAX_RANGES];
 #pragma unroll
-        for (int range = 0; range < GW_MAX_RANGES; range++) parts[range] = range < args.ranges ? partial[(i64)range * pitch] : 0.0f;
-        float norm = 0.0f;
+            for (int range = 0; range < GW_MAX_RANGES; range++) parts[range] = range < args.ranges ? partial[(i64)range * pitch] : 0.0f;
+            float norm = 0.0f;
 #pragma unroll
-        for (int range = 0; range < GW_MAX_RANGES; range++) norm += range < args.ranges ? parts[range] : 0.0f;
-        (of_a ? lds_norm_a : lds_norm_b)[r] = norm;
+            for (int range = 0; range < GW_MAX_RANGES; range++) norm += range < args.ranges ? parts[range] : 0.0f;
+            (of_a ? lds_norm_a : lds_norm_b)[r] = norm;
+        }
         (of_a ? lds_unscale_a : lds_unscale_b)[r] =
             of_a ? args.unscale_a[batch * args.unscale_a_bs + m0 + r] : args.unscale_b[batch * args.unscale_b_bs + n0 + r];
-        if (tid < 4) lds_distrust[tid] = 0;
+    }
+    if (tid < Tile::PARTS) lds_distrust[tid] = 0;
+
+    gram_float4 acc[MT][NT];
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++) acc[mt][nt] = gram_float4{0.0f, 0.0f, 0.0f, 0.0f};
+    {
+        WideWalk<Tile> walk;
+        walk.init(args.pieces_a + batch * args.pieces_a_bs, args.rows_pad_a, m0, args.pieces_b + batch * args.pieces_b_bs, args.rows_pad_b, n0,
+                  ring, lane, wave, wave_m, wave_n);
+        wide_walk<Tile>(acc, walk, (args.slices + 1) / 2);
     }
 
-    auto buffer = [&](auto which) -> gram_chunk * {
-        constexpr int B = decltype(which)::value;
-        if constexpr (B == 0) return lds0;
-        else if constexpr (B == 1) return lds1;
-        else if constexpr (B == 2) return lds2;
-        else return lds3;
-    };
-
-    // Copies: 32 runs of 64 chunks per slice (operand, segment, quarter of the rows), 4 per wave:
-    // runs 0 .. 15 belong to a (q < 2 for every wave), 16 .. 31 to b.
-    typedef const __attribute__((address_space(1))) void *global_address;
-    typedef __attribute__((address_space(3))) void *lds_address;
-    const gram_chunk *src[4];
-    int dst[4];     // first chunk of the run in a buffer: uniform over the wave
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        const int run = wave + 8 * q;
-        const int operand = q < 2 ? 0 : 1, segment = (run % 16) / 4, quarter = run % 4;
-        const gram_chunk *base = operand == 0 ? args.pieces_a + batch * args.pieces_a_bs + (i64)segment * args.rows_pad_a + m0
-                                              : args.pieces_b + batch * args.pieces_b_bs + (i64)segment * args.rows_pad_b + n0;
-        src[q] = base + quarter * 64 + lane;
-        dst[q] = operand * GW_OPERAND_CHUNKS + segment * GW_TILE + quarter * 64;
-    }
-    const i64 step_a = (i64)GW_SEGMENTS * args.rows_pad_a, step_b = (i64)GW_SEGMENTS * args.rows_pad_b;
-    auto copy = [&](auto into, auto which_run) {
-        constexpr int q = decltype(which_run)::value;
-        const unsigned lds_byte = (unsigned)(unsigned long)(lds_address)(buffer(into) + dst[q]);
-#ifndef GW_ABLATE_NO_COPY
-        asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
-                     :
-                     : "v"((global_address)src[q]), "s"(lds_byte)
-                     : "memory", "m0");
-#endif
-        src[q] += q < 2 ? step_a : step_b;
-    };
-
-    gram_float16 acc[4][2];
-#pragma unroll
-    for (int mt = 0; mt < 4; mt++)
-#pragma unroll
-        for (int nt = 0; nt < 2; nt++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) acc[mt][nt][v] = 0.0f;
-
-    const int read_a = h * GW_TILE + wave_m + i;
-    const int read_b = GW_OPERAND_CHUNKS + h * GW_TILE + wave_n + i;
-    // fa[set][p], fb[set][p]: piece p (0 the larger) of this wave's rows, for slices of either parity
-    gram_half8 fa[2][GW_PIECES][4], fb[2][GW_PIECES][2];
-    auto read_operands = [&](auto set, auto from) {
-        constexpr int S = decltype(set)::value;
-#pragma unroll
-        for (int p = GW_PIECES - 1; p >= 0; p--) {
-#pragma unroll
-            for (int mt = 0; mt < 4; mt++)
-                fa[S][p][mt] = __builtin_bit_cast(gram_half8, buffer(from)[2 * p * GW_TILE + read_a + 32 * mt]);
-            if (p == GW_PIECES - 1) {
-#pragma unroll
-                for (int nt = 0; nt < 2; nt++)
-                    fb[S][0][nt] = __builtin_bit_cast(gram_half8, buffer(from)[read_b + 32 * nt]);
-            }
-        }
-#pragma unroll
-        for (int nt = 0; nt < 2; nt++)
-            fb[S][1][nt] = __builtin_bit_cast(gram_half8, buffer(from)[2 * GW_TILE + read_b + 32 * nt]);
-    };
-    auto multiply = [&](auto set, int pa, int pb) {
-        constexpr int S = decltype(set)::value;
-#pragma unroll
-        for (int mt = 0; mt < 4; mt++)
-#pragma unroll
-            for (int nt = 0; nt < 2; nt++)
-                acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[S][pa][mt], fb[S][pb][nt], acc[mt][nt], 0, 0, 0);
-    };
-
-    // The slice in buffer B, whose operands are in register set S.  The four copies of a slice
-    // are issued one per group of eight matrix instructions where they can be: three behind the
-    // barrier of the slice whose buffer they fill, the fourth in the first group of the next slice.
-    auto step = [&](auto set, auto which) {
-        constexpr int S = decltype(set)::value;
-        constexpr int B = decltype(which)::value;
-        const GramStep<(B + 1) % 4> next;
-        const GramStep<(B + 3) % 4> previous;
-        multiply(set, 1, 0);                                // a2 b1
-        copy(previous, GramStep<3>{});
-        __builtin_amdgcn_sched_barrier(0);
-        // what may still be under way: the eight copies issued last, of the two slices after the next one
-        __builtin_amdgcn_s_waitcnt(0x0F78);                 // vmcnt(8), nothing else
-        __syncthreads();
-        read_operands(GramStep<1 - S>{}, next);
-        copy(which, GramStep<0>{});
-        __builtin_amdgcn_sched_barrier(0);
-        multiply(set, 0, 0);                                // a1 b1
-        copy(which, GramStep<1>{});
-        __builtin_amdgcn_sched_barrier(0);
-        multiply(set, 0, 1);                                // a1 b2
-        copy(which, GramStep<2>{});
-        __builtin_amdgcn_sched_barrier(0);
-    };
-
-    // slices 0, 1 and 2, and three of the four copies of slice 3
-    copy(GramStep<0>{}, GramStep<0>{}); copy(GramStep<0>{}, GramStep<1>{}); copy(GramStep<0>{}, GramStep<2>{}); copy(GramStep<0>{}, GramStep<3>{});
-    copy(GramStep<1>{}, GramStep<0>{}); copy(GramStep<1>{}, GramStep<1>{}); copy(GramStep<1>{}, GramStep<2>{}); copy(GramStep<1>{}, GramStep<3>{});
-    copy(GramStep<2>{}, GramStep<0>{}); copy(GramStep<2>{}, GramStep<1>{}); copy(GramStep<2>{}, GramStep<2>{}); copy(GramStep<2>{}, GramStep<3>{});
-    copy(GramStep<3>{}, GramStep<0>{}); copy(GramStep<3>{}, GramStep<1>{}); copy(GramStep<3>{}, GramStep<2>{});
-    __builtin_amdgcn_s_waitcnt(0x0F7B);                     // vmcnt(11): slice 0 has arrived
-    __syncthreads();
-    read_operands(GramStep<0>{}, GramStep<0>{});
-    for (int slice = 0;;) {
-        step(GramStep<0>{}, GramStep<0>{});
-        if (++slice == args.slices) break;
-        step(GramStep<1>{}, GramStep<1>{});
-        if (++slice == args.slices) break;
-        step(GramStep<0>{}, GramStep<2>{});
-        if (++slice == args.slices) break;
-        step(GramStep<1>{}, GramStep<3>{});
-        if (++slice == args.slices) break;
-    }
-    // copies of slices that do not exist may still be under way: they must not land in what follows
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-    __syncthreads();
-
-#ifdef GW_ABLATE_NO_EPILOGUE
-    if (args.slices > 0) {      // keeps the accumulators alive without storing them
-        float sum = 0.0f;
-        for (int mt = 0; mt < 4; mt++)
-            for (int nt = 0; nt < 2; nt++)
-                for (int v = 0; v < 16; v++) sum += acc[mt][nt][v];
-        if (sum == 123.456f) args.kernel.c[tid] = sum;
-        return;
-    }
-#endif
-    const BuildKernelArgs &kernel = args.kernel;
+    // Everything behind the walk is derived from a copy of the lane id and of the argument block's address that the
+    // compiler cannot see through: computed before the walk and kept through it, it would push the walk's operands
+    // into scratch memory.
+    int lane_after = lane;
+    asm volatile("" : "+v"(lane_after));
+    typedef const __attribute__((address_space(4))) GramWideArgs *argument_pointer;
+    argument_pointer late = (argument_pointer)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(late));
+    const auto *kernel = &late->kernel;
+    // A lane holds, of every 16 x 16 block, one row of b (its lane number modulo 16) and 4 consecutive m:
+    //   acc[mt][nt][v]:  m = wave_m + 16 mt + 4 q + v,  n = wave_n + 16 nt + i
+    const int q = lane_after >> 4;
+    const int i = lane_after & 15;
+    const int rows = kernel->m - m0, columns = kernel->n - n0;      // of the result, from this tile's first element on
+    float *c_tile = kernel->c + batch * kernel->c_bs + (i64)n0 * kernel->c_ld + m0;
+    const i64 c_ld = kernel->c_ld;
+    const bool c_vec = kernel->c_vec != 0;
     if constexpr (EPILOGUE == GW_EPILOGUE_GRADIENT_L2) {
-        // A lane holds, of every 32 x 32 tile, one row r of b (its lane number modulo 32) and 16 m in 4 runs of 4.
-        const bool full = m_valid >= GW_TILE && n_valid >= GW_TILE;
-        float *c_tile = kernel.c + batch * kernel.c_bs + (i64)n0 * kernel.c_ld + m0;
+        const int gradient_n = late->gradient_n;
+        const i64 g_ld = late->gradient_g_ld;
+        const float *g_tile = late->gradient_g + batch * late->gradient_g_bs + (i64)m0 * g_ld;
+        const float *d_tile = late->gradient_d + batch * late->gradient_d_bs + m0;
+        const float *shifts = late->gradient_shift + batch * late->gradient_shift_bs;
+        const i64 d_ld = late->gradient_d_ld;
+        const bool full = rows >= TILE_M;
 #pragma unroll
-        for (int nt = 0; nt < 2; nt++) {
-            const int r_local = wave_n + nt * 32 + i;
-            if (!full && r_local >= n_valid) continue;
+        for (int nt = 0; nt < NT; nt++) {
+            const int r_local = wave_n + nt * 16 + i;
+            if (r_local >= columns) continue;
             const int r = n0 + r_local;
-            const int o = r / args.gradient_n, n = r - o * args.gradient_n;
+            const int o = r / gradient_n, n = r - o * gradient_n;
             const float unscale_b = lds_unscale_b[r_local];
-            const float shift = args.gradient_shift[batch * args.gradient_shift_bs + n];
-            const float *d_row = args.gradient_d + batch * args.gradient_d_bs + (i64)n * args.gradient_d_ld + m0;
-            const float *g_column = args.gradient_g + batch * args.gradient_g_bs + (i64)m0 * args.gradient_g_ld + o;
-            float *row = c_tile + (i64)r_local * kernel.c_ld;
+            const float shift = shifts[n];
+            const float *d_row = d_tile + (i64)n * d_ld;
+            float *row = c_tile + (i64)r_local * c_ld;
 #pragma unroll
-            for (int mt = 0; mt < 4; mt++)
+            for (int mt = 0; mt < MT; mt++) {
+                const int m_local = wave_m + mt * 16 + 4 * q;
+                const float4 unscale_a = *reinterpret_cast<const float4 *>(&lds_unscale_a[m_local]);
+                const float unscales_a[4] = {unscale_a.x, unscale_a.y, unscale_a.z, unscale_a.w};
+                float v4[4];
 #pragma unroll
-                for (int g = 0; g < 4; g++) {
-                    const int m_local = wave_m + mt * 32 + 8 * g + 4 * h;
-                    const float4 unscale_a = *reinterpret_cast<const float4 *>(&lds_unscale_a[m_local]);
-                    const float unscales_a[4] = {unscale_a.x, unscale_a.y, unscale_a.z, unscale_a.w};
-                    float v4[4];
-#pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        const bool exists = full || m_local + e < m_valid;
-                        const float d = exists ? d_row[m_local + e] - shift : 0.0f;
-                        const float weight = exists ? g_column[(i64)(m_local + e) * args.gradient_g_ld] : 0.0f;
-                        v4[e] = d * weight - (acc[mt][nt][4 * g + e] * unscales_a[e]) * unscale_b;
-                    }
-                    if (kernel.c_vec && (full || m_local + 3 < m_valid)) {
-                        *reinterpret_cast<float4 *>(row + m_local) = make_float4(v4[0], v4[1], v4[2], v4[3]);
-                    } else {
-#pragma unroll
-                        for (int e = 0; e < 4; e++)
-                            if (m_local + e < m_valid) row[m_local + e] = v4[e];
-                    }
+                for (int e = 0; e < 4; e++) {
+                    const bool exists = full || m_local + e < rows;
+                    const float d = exists ? d_row[m_local + e] - shift : 0.0f;
+                    const float weight = exists ? g_tile[(i64)(m_local + e) * g_ld + o] : 0.0f;
+                    v4[e] = d * weight - (acc[mt][nt][e] * unscales_a[e]) * unscale_b;
                 }
-        }
-        return;
-    }
-    // d^2 = |a|^2 + |b|^2 - 2 a.b, trust check per 128 x 128 part (the unit the repair launch
-    // works in; every wave lies inside one part), epilogue, stores.
-    const int outer_power = kernel.outer_power;
-    const int kernel_type = kernel.kernel_type;
-    float p_outer = 0.0f, neg_gamma = 0.0f, regularization = 0.0f;
-    if (outer_power == POW_POW) p_outer = kernel.p_outer ? kernel.p_outer[batch * kernel.p_outer_bs] : kernel.p_outer_value;
-    if (kernel_type != KERNEL_NONE) {
-        const float bw = kernel.bandwidth ? kernel.bandwidth[batch * kernel.bandwidth_bs] : kernel.bandwidth_value;
-        neg_gamma = kernel_neg_gamma(kernel_type, bw);
-        regularization = kernel.regularization ? kernel.regularization[batch * kernel.regularization_bs] : kernel.regularization_value;
-    }
-    const bool regularize = kernel_type != KERNEL_NONE && regularization != 0.0f;
-    const float diagonal_value = 1.0f + regularization;
-
-    // A lane holds, of every 32 x 32 tile, one n (its lane number modulo 32) and 16 m in 4 runs of 4:
-    //   acc[mt][nt][v]:  m = wave_m + 32 mt + 8 (v / 4) + 4 h + v % 4,  n = wave_n + 32 nt + i
-    // (With the rows of b as the first operand of the matrix instruction a lane holds one m and
-    // every store writes whole 128-byte lines, 32-bit stores instead of 128-bit ones: measured
-    // 2 % slower.)
-    //
-    // d^2 and the trust check first, without branches: norms and scales of a come as 128-bit
-    // reads; what is not trusted is collected as a lane mask in scalar registers.  A tile that is
-    // not a full one masks the rows and columns that do not exist.  The outer function follows
-    // with its switch outside the loop over the values.
-    const bool full = m_valid >= GW_TILE && n_valid >= GW_TILE;
-    unsigned long long distrusted = 0;
-    float norm_b[2], unscale_b[2];
-    int n_local[2];
-#pragma unroll
-    for (int nt = 0; nt < 2; nt++) {
-        n_local[nt] = wave_n + nt * 32 + i;
-        norm_b[nt] = lds_norm_b[n_local[nt]];
-        unscale_b[nt] = -2.0f * lds_unscale_b[n_local[nt]];
-    }
-    const float trust = kernel.gram_trust;
-#pragma unroll
-    for (int mt = 0; mt < 4; mt++)
-#pragma unroll
-        for (int g = 0; g < 4; g++) {
-            const int m_local = wave_m + mt * 32 + 8 * g + 4 * h;
-            const float4 norm_a = *reinterpret_cast<const float4 *>(&lds_norm_a[m_local]);
-            const float4 unscale_a = *reinterpret_cast<const float4 *>(&lds_unscale_a[m_local]);
-            const float norms_a[4] = {norm_a.x, norm_a.y, norm_a.z, norm_a.w};
-            const float unscales_a[4] = {unscale_a.x, unscale_a.y, unscale_a.z, unscale_a.w};
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-#pragma unroll
-                for (int nt = 0; nt < 2; nt++) {
-                    if constexpr (EPILOGUE == GW_EPILOGUE_DOT) {
-                        // unscale_b carries the factor -2 of the distance
-                        acc[mt][nt][4 * g + e] = (acc[mt][nt][4 * g + e] * unscales_a[e]) * (-0.5f * unscale_b[nt]);
-                    } else {
-                        const float norms = norms_a[e] + norm_b[nt];
-                        const float d2 = norms + (acc[mt][nt][4 * g + e] * unscales_a[e]) * unscale_b[nt];
-                        // not a number (overflowing squares, NaN data): not trusted either
-                        bool bad = !(d2 >= trust * norms);
-                        if (!full) bad = bad && m_local + e < m_valid && n_local[nt] < n_valid;
-                        distrusted |= __builtin_amdgcn_ballot_w64(bad);
-                        acc[mt][nt][4 * g + e] = fmaxf(d2, 0.0f);
-                    }
-                }
-        }
-    auto for_each = [&](auto &&f) {
-#pragma unroll
-        for (int mt = 0; mt < 4; mt++)
-#pragma unroll
-            for (int nt = 0; nt < 2; nt++)
-#pragma unroll
-                for (int v = 0; v < 16; v++) acc[mt][nt][v] = f(acc[mt][nt][v]);
-    };
-    // the outer function and the kernel function of epilogue_value (device_common.hpp)
-    switch (outer_power) {
-    case POW_ABS: for_each([](float v) { return fabsf(v); }); break;
-    case POW_SQUARE: for_each([](float v) { return v * v; }); break;
-    case POW_SQRT: for_each([](float v) { return __builtin_amdgcn_sqrtf(v); }); break;
-    case POW_POW: for_each([=](float v) { return epilogue_value(v, POW_POW, KERNEL_NONE, p_outer, 0.0f, 0.0f); }); break;
-    default: break;
-    }
-    if (kernel_type != KERNEL_NONE) {
-        const float epsilon = kernel.epsilon;
-        for_each([=](float v) { return epilogue_value(v, POW_NOOP, kernel_type, 0.0f, neg_gamma, epsilon); });
-    }
-    if (regularize) {
-#pragma unroll
-        for (int mt = 0; mt < 4; mt++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) {
-                const int m_local = wave_m + mt * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
-#pragma unroll
-                for (int nt = 0; nt < 2; nt++)
-                    if (kernel.reg_off_x + m0 + m_local == kernel.reg_off_y + n0 + n_local[nt]) acc[mt][nt][v] = diagonal_value;
-            }
-    }
-    const int part_m = wave & 1, part_n = wave >> 2;
-    const int part = part_m + 2 * part_n;
-    // where this wave's part lies: below the diagonal of the result (stored and mirrored), on it
-    // (lower triangle stored and mirrored), above it inside a diagonal tile (not stored)
-    const bool on_diagonal = SYMMETRIC && tile_m == tile_n && part_m == part_n;
-    const bool above = SYMMETRIC && tile_m == tile_n && part_m < part_n;
-    if (distrusted != 0 && lane == 0 && !above) lds_distrust[part] = 1;
-    __syncthreads();
-    if (above) return;
-    const bool repair = lds_distrust[part] != 0;
-    // the first element of a part is held by lane 0 of the wave that starts the part
-    if (repair && lane == 0 && (wave_n & 127) == 0) acc[0][0][0] = __uint_as_float(BK_REPAIR_MARKER);
-
-    float *c_tile = kernel.c + batch * kernel.c_bs + (i64)n0 * kernel.c_ld + m0;
-#pragma unroll
-    for (int nt = 0; nt < 2; nt++) {
-        if (!full && n_local[nt] >= n_valid) continue;
-        float *row = c_tile + (i64)n_local[nt] * kernel.c_ld;
-#pragma unroll
-        for (int mt = 0; mt < 4; mt++)
-#pragma unroll
-            for (int g = 0; g < 4; g++) {
-                const int m_local = wave_m + mt * 32 + 8 * g + 4 * h;
-                const float v4[4] = {acc[mt][nt][4 * g], acc[mt][nt][4 * g + 1], acc[mt][nt][4 * g + 2], acc[mt][nt][4 * g + 3]};
-                const bool whole = !on_diagonal || m_local >= n_local[nt];
-                if (kernel.c_vec && whole && (full || m_local + 3 < m_valid)) {
+                if (c_vec && (full || m_local + 3 < rows)) {
                     *reinterpret_cast<float4 *>(row + m_local) = make_float4(v4[0], v4[1], v4[2], v4[3]);
                 } else {
 #pragma unroll
                     for (int e = 0; e < 4; e++)
-                        if (m_local + e < m_valid && (!on_diagonal || m_local + e >= n_local[nt])) row[m_local + e] = v4[e];
+                        if (m_local + e < rows) row[m_local + e] = v4[e];
                 }
             }
+        }
+        return;
     }
 
-    // The same values at C(n, m), where the 32 consecutive n of a half wave are the contiguous ones.
-    if (SYMMETRIC && !repair) {
-        float *mirror = kernel.c + batch * kernel.c_bs + (i64)m0 * kernel.c_ld + n0;
+    const int part_m = wave_m / 128, part_n = wave_n / 128;
+    const int part = part_m + Tile::PARTS_M * part_n;
+    // where this wave's part lies: below the diagonal of the result (stored and mirrored), on it
+    // (lower triangle stored and mirrored), above it inside a tile (not stored)
+    const bool on_diagonal = SYMMETRIC && m0 + 128 * part_m == n0 + 128 * part_n;
+    const bool above = SYMMETRIC && m0 + 128 * part_m < n0 + 128 * part_n;
+
+    const int outer_power = kernel->outer_power;
+    const int kernel_type = kernel->kernel_type;
+    const float trust = kernel->gram_trust;
+    const float epsilon = kernel->epsilon;
+    float p_outer = 0.0f, neg_gamma = 0.0f, diagonal_value = 0.0f;
+    if (outer_power == POW_POW) p_outer = kernel->p_outer ? kernel->p_outer[batch * kernel->p_outer_bs] : kernel->p_outer_value;
+    // element (m, n) is regularised when reg_off_x + m == reg_off_y + n: 16 mt + 4 q + v == diagonal + 16 nt + i
+    const int diagonal = kernel->reg_off_y + n0 + wave_n - kernel->reg_off_x - m0 - wave_m;
+    bool regularize = false;
+    if (kernel_type != KERNEL_NONE) {
+        neg_gamma = kernel_neg_gamma(kernel_type, kernel->bandwidth ? kernel->bandwidth[batch * kernel->bandwidth_bs] : kernel->bandwidth_value);
+        const float regularization =
+            kernel->regularization ? kernel->regularization[batch * kernel->regularization_bs] : kernel->regularization_value;
+        diagonal_value = 1.0f + regularization;
+        regularize = regularization != 0.0f && diagonal < Tile::WAVE_M && diagonal > -Tile::WAVE_N;
+    }
+
+    // 16 columns n at a time: d^2 = |a|^2 + |b|^2 - 2 a.b and the trust check per 128 x 128 part (the unit the repair
+    // launch works in; every wave lies inside one part), the outer function and the kernel function, the stores.
+    // A result is trusted when d^2 >= trust * norms, judged as norms * (1 - trust) - 2 a.b >= 0; a lane keeps its least
+    // such margin (v_minimum3_f32 hands a NaN on: overflowing squares and NaN data are not trusted).  Rows and columns
+    // that do not exist have pieces and norms of zero: with a row or column that does exist they give d^2 = norms,
+    // which is trusted unless that row's norm is not a number -- and then its own elements are not trusted either.
+    // The stores go through this wave's share of the ring (idle: every copy has arrived, and no wave reads it any
+    // more), so that an instruction writes runs of WAVE_M floats of a column.
+    float least_margin = 0.0f;
+    float *stage = reinterpret_cast<float *>(ring) + wave * (4 * Tile::SLOTS * Tile::GRANULE_CHUNKS / Tile::WAVES);
+    {
+        constexpr int PITCH = Tile::WAVE_M + 4, LANES = Tile::WAVE_M / 4, PER_PASS = 64 / LANES;
+        static_assert(16 * PITCH <= 4 * Tile::SLOTS * Tile::GRANULE_CHUNKS / Tile::WAVES, "the staging fits a wave's share of the ring");
+        const int row = wave_m + 4 * (lane_after % LANES);
+        const bool whole = c_vec && row + 3 < rows;
 #pragma unroll
-        for (int nt = 0; nt < 2; nt++) {
-            if (!full && n_local[nt] >= n_valid) continue;
+        for (int nt = 0; nt < NT; nt++) {
+            const float norm_b = EPILOGUE == GW_EPILOGUE_DISTANCE ? lds_norm_b[wave_n + nt * 16 + i] : 0.0f;
+            const float unscale_b = (EPILOGUE == GW_EPILOGUE_DISTANCE ? -2.0f : 1.0f) * lds_unscale_b[wave_n + nt * 16 + i];
 #pragma unroll
-            for (int mt = 0; mt < 4; mt++)
+            for (int mt = 0; mt < MT; mt++) {
+                const int m_local = wave_m + mt * 16 + 4 * q;
+                const gram_float4 unscale_a = *reinterpret_cast<const gram_float4 *>(&lds_unscale_a[m_local]);
+                if constexpr (EPILOGUE == GW_EPILOGUE_DOT) {
 #pragma unroll
-                for (int v = 0; v < 16; v++) {
-                    const int m_local = wave_m + mt * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
-                    if ((full || m_local < m_valid) && (!on_diagonal || m_local > n_local[nt]))
-                        mirror[(i64)m_local * kernel.c_ld + n_local[nt]] = acc[mt][nt][v];
+                    for (int e = 0; e < 4; e++) acc[mt][nt][e] = (acc[mt][nt][e] * unscale_a[e]) * unscale_b;
+                } else {
+                    const gram_float4 norm_a = *reinterpret_cast<const gram_float4 *>(&lds_norm_a[m_local]);
+                    float margin[4];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const float norms = norm_a[e] + norm_b;
+                        const float minus_twice = (acc[mt][nt][e] * unscale_a[e]) * unscale_b;
+                        acc[mt][nt][e] = norms + minus_twice;
+                        margin[e] = norms * (1.0f - trust) + minus_twice;
+                    }
+                    asm("v_minimum3_f32 %0, %1, %2, %0" : "+v"(least_margin) : "v"(margin[0]), "v"(margin[1]));
+                    asm("v_minimum3_f32 %0, %1, %2, %0" : "+v"(least_margin) : "v"(margin[2]), "v"(margin[3]));
                 }
+            }
+            // the outer function and the kernel function of epilogue_value (device_common.hpp), the switches outside the loops
+            auto for_each = [&](auto &&f) {
+#pragma unroll
+                for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+                    for (int v = 0; v < 4; v++) acc[mt][nt][v] = f(acc[mt][nt][v]);
+            };
+            switch (outer_power) {
+            case POW_ABS: for_each([](float v) { return fabsf(v); }); break;
+            case POW_SQUARE: for_each([](float v) { return v * v; }); break;
+            case POW_SQRT: for_each([](float v) { return __builtin_amdgcn_sqrtf(v); }); break;
+            case POW_POW: for_each([=](float v) { return epilogue_value(v, POW_POW, KERNEL_NONE, p_outer, 0.0f, 0.0f); }); break;
+            default: break;
+            }
+            if (kernel_type != KERNEL_NONE) {
+                for_each([=](float v) { return epilogue_value(v, POW_NOOP, kernel_type, 0.0f, neg_gamma, epsilon); });
+                if (regularize) {
+#pragma unroll
+                    for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+                        for (int v = 0; v < 4; v++)
+                            acc[mt][nt][v] = 16 * mt + 4 * q + v == diagonal + 16 * nt + i ? diagonal_value : acc[mt][nt][v];
+                }
+            }
+            if (above) continue;
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++) *reinterpret_cast<gram_float4 *>(stage + i * PITCH + 16 * mt + 4 * q) = acc[mt][nt];
+#pragma unroll
+            for (int pass = 0; pass < 16 / PER_PASS; pass++) {
+                const int column = pass * PER_PASS + lane_after / LANES;
+                const gram_float4 v = *reinterpret_cast<const gram_float4 *>(stage + column * PITCH + 4 * (lane_after % LANES));
+                const int n_local = wave_n + 16 * nt + column;
+                float *to = c_tile + (i64)n_local * c_ld + row;
+                // on the diagonal only m >= n
+                const int first = SYMMETRIC && on_diagonal ? n0 + n_local - (m0 + row) : 0;
+                if (n_local < columns) {
+                    if (whole && first <= 0) {
+                        *reinterpret_cast<gram_float4 *>(to) = v;
+                    } else {
+                        for (int e = first > 0 ? first : 0; e < 4 && row + e < rows; e++) to[e] = e == 0 ? v[0] : e == 1 ? v[1] : e == 2 ? v[2] : v[3];
+                    }
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    if constexpr (EPILOGUE == GW_EPILOGUE_DISTANCE) {
+        // A part with a distrusted element is stamped: its first element, stored a second time by the wave that stored
+        // it first.  The repair launch recomputes the part (and mirrors it).
+        if (!(least_margin >= 0.0f) && !above) lds_distrust[part] = 1;
+        __syncthreads();
+        if (lds_distrust[part] != 0 && lane_after == 0 && !above && (wave_m & 127) == 0 && (wave_n & 127) == 0 && wave_m < rows && wave_n < columns)
+            c_tile[(i64)wave_n * c_ld + wave_m] = __uint_as_float(BK_REPAIR_MARKER);
+    }
+    if (above) return;
+
+    // The same values at C(n, m): 32 rows m at a time through the same memory.
+    if (SYMMETRIC) {
+        constexpr int PITCH = Tile::WAVE_N + 4, LANES = Tile::WAVE_N / 4, PER_PASS = 64 / LANES;
+        static_assert(32 * PITCH <= 4 * Tile::SLOTS * Tile::GRANULE_CHUNKS / Tile::WAVES, "the staging fits a wave's share of the ring");
+        float *mirror = kernel->c + batch * kernel->c_bs + (i64)m0 * c_ld + n0;
+        const int column = wave_n + 4 * (lane_after % LANES);
+        const bool whole = c_vec && column + 3 < columns;
+#pragma unroll
+        for (int pair = 0; pair < MT / 2; pair++) {
+#pragma unroll
+            for (int mt = 0; mt < 2; mt++)
+#pragma unroll
+                for (int nt = 0; nt < NT; nt++)
+#pragma unroll
+                    for (int v = 0; v < 4; v++) stage[(16 * mt + 4 * q + v) * PITCH + 16 * nt + i] = acc[2 * pair + mt][nt][v];
+#pragma unroll
+            for (int pass = 0; pass < 32 / PER_PASS; pass++) {
+                const int row = pass * PER_PASS + lane_after / LANES;
+                const gram_float4 v = *reinterpret_cast<const gram_float4 *>(stage + row * PITCH + 4 * (lane_after % LANES));
+                const int m_local = wave_m + 32 * pair + row;
+                float *to = mirror + (i64)m_local * c_ld + column;
+                // on the diagonal only n < m
+                const int last = on_diagonal ? m0 + m_local - (n0 + column) : 4;
+                if (m_local < rows) {
+                    if (whole && last >= 4) {
+                        *reinterpret_cast<gram_float4 *>(to) = v;
+                    } else {
+                        for (int e = 0; e < 4 && e < last && column + e < columns; e++) to[e] = e == 0 ? v[0] : e == 1 ? v[1] : e == 2 ? v[2] : v[3];
+                    }
+                }
+            }
         }
     }
 }

@@ -30,7 +30,7 @@ struct OperandRegions {
 
 struct WideLayout {
     int slices, slices_per_range, ranges;
-    int tiles_m, tiles_n, tiles_n_padded;
+    int tiles_m, tiles_n;       // of GW_TILE x GW_TILE
     OperandRegions a, b;
     int64_t sample;         // byte offset of the words of gram_probe_operands
     int64_t bytes;
@@ -98,7 +98,7 @@ void place_operand(OperandRegions &r, int rows, bool broadcast, int l, const Wid
 {
     r.rows_pad = (rows + kmc::GW_TILE - 1) / kmc::GW_TILE * kmc::GW_TILE;
     r.batches = broadcast ? 1 : l;
-    r.pieces_bs = static_cast<int64_t>(layout.slices + kmc::GW_EXTRA_SLICES) * kmc::GW_SEGMENTS * r.rows_pad;
+    r.pieces_bs = static_cast<int64_t>(2 * ((layout.slices + 1) / 2)) * kmc::GW_SEGMENTS * r.rows_pad;      // whole steps of the walk
     r.stats_bs = static_cast<int64_t>(layout.ranges) * r.rows_pad;
     r.pieces = place(cursor, r.batches * r.pieces_bs * 16);
     r.squares = place(cursor, r.batches * r.stats_bs * 4);
@@ -109,10 +109,8 @@ void place_operand(OperandRegions &r, int rows, bool broadcast, int l, const Wid
 // Grid, slices and the regions of both operands in the workspace; tiles_m and tiles_n are set.
 bool place_wide(int m, int n, int k, int l, bool a_once, bool b_once, bool symmetric, WideLayout *layout)
 {
-    int padded = (layout->tiles_n + kmc::BK_XCDS - 1) / kmc::BK_XCDS * kmc::BK_XCDS;
-    if ((padded - layout->tiles_n) * 8 > layout->tiles_n) padded = layout->tiles_n;
-    if (static_cast<int64_t>(layout->tiles_m) * padded > 0x7fffffff) return false;
-    layout->tiles_n_padded = padded;
+    // room for any tile of the product kernel in a grid, n tiles padded to the XCDs
+    if (static_cast<int64_t>(layout->tiles_m) * (layout->tiles_n + kmc::BK_XCDS) * 4 > 0x7fffffff) return false;
     layout->slices = (k + kmc::BK_TILE_K - 1) / kmc::BK_TILE_K;
     // at most 8 ranges of K per row: enough workgroups for the row kernels, few partial sums
     layout->slices_per_range = layout->slices / 8 > 8 ? (layout->slices + 7) / 8 : 8;
@@ -163,6 +161,7 @@ kmc::GramRowsArgs rows_args(const float *x, int64_t ld, int64_t bs, int rows, in
     rows_of.stats_bs = r.stats_bs; rows_of.unscale_bs = r.rows_pad;
     rows_of.rows_pad = r.rows_pad; rows_of.slices = layout.slices;
     rows_of.slices_per_range = layout.slices_per_range; rows_of.ranges = layout.ranges;
+    rows_of.zero_slices = layout.slices & 1;      // the walk takes two slices per step
     return rows_of;
 }
 
@@ -240,6 +239,36 @@ hipError_t launch_gram_rows_pair(const kmc::GramRowsArgs &first, int first_batch
     return launch(kmc::gram_f16_split_pair<0>, grid, dim3(kmc::GW_ROW_THREADS), stream, pair);
 }
 
+// The product kernel in tiles of TILE; extents, batch entries and operands of `wide` are set.
+template <typename Tile, bool SYMMETRIC, int EPILOGUE>
+hipError_t launch_product_in(kmc::GramWideArgs &wide, hipStream_t stream)
+{
+    wide.wide_tiles_m = (wide.kernel.m + Tile::TILE_M - 1) / Tile::TILE_M;
+    wide.wide_tiles_n = (wide.kernel.n + Tile::TILE_N - 1) / Tile::TILE_N;
+    int padded = (wide.wide_tiles_n + kmc::BK_XCDS - 1) / kmc::BK_XCDS * kmc::BK_XCDS;
+    if ((padded - wide.wide_tiles_n) * 8 > wide.wide_tiles_n) padded = wide.wide_tiles_n;
+    wide.wide_tiles_n_padded = padded;
+    const int64_t blocks = (wide.kernel.m + kmc::GW_TILE - 1) / kmc::GW_TILE;
+    const int64_t width = SYMMETRIC ? blocks * (blocks + 1) / 2 * (kmc::GW_TILE / Tile::TILE_M) * (kmc::GW_TILE / Tile::TILE_N)
+                                    : static_cast<int64_t>(wide.wide_tiles_m) * padded;
+    if (width > 0x7fffffff) return hipErrorInvalidValue;
+    return launch(kmc::gram_f16_wide<Tile, SYMMETRIC, EPILOGUE>, dim3(static_cast<unsigned>(width), wide.kernel.l, 1), dim3(Tile::THREADS), stream, wide);
+}
+
+// Tiles of 128 x 128 unless there are many: three of them share a CU and share the chip out more evenly, tiles of 256 x 128 ask
+// the L2 for three quarters of the bytes per multiply-add.  Time of a call in the small tiles over the large ones: 32 large
+// tiles 0.94 at K = 128, 0.75 at K = 2048; 288 tiles 0.92, 0.90; 512 tiles 0.99, 1.03; 800 tiles 0.97, 0.96; 1128 tiles
+// 0.89, 0.97; 2048 tiles 0.96, 1.03; 3160 tiles 0.91, 1.00; 8192 tiles 1.02 at K = 128, 1.01 at K = 512.
+template <bool SYMMETRIC, int EPILOGUE>
+hipError_t launch_product(kmc::GramWideArgs &wide, hipStream_t stream)
+{
+    using Large = kmc::WideTileLarge;
+    int64_t tiles = static_cast<int64_t>((wide.kernel.m + Large::TILE_M - 1) / Large::TILE_M) * ((wide.kernel.n + Large::TILE_N - 1) / Large::TILE_N) * wide.kernel.l;
+    if (SYMMETRIC) tiles /= 2;
+    return tiles >= kmc_rules::WIDE_LARGE_TILE_MIN_TILES ? launch_product_in<Large, SYMMETRIC, EPILOGUE>(wide, stream)
+                                                         : launch_product_in<kmc::WideTileSmall, SYMMETRIC, EPILOGUE>(wide, stream);
+}
+
 // Bytes of workspace the path needs for this problem; 0 when it does not apply.
 int64_t gram_f16_wide_bytes(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &args)
 {
@@ -292,7 +321,6 @@ hipError_t launch_gram_f16_wide(const kmc_build_kernel_params *p, const kmc::Bui
     wide.unscale_b_bs = layout.b.batches > 1 ? layout.b.rows_pad : 0;
     wide.rows_pad_a = layout.a.rows_pad; wide.rows_pad_b = layout.b.rows_pad;
     wide.slices = layout.slices; wide.ranges = layout.ranges;
-    wide.wide_tiles_m = layout.tiles_m; wide.wide_tiles_n = layout.tiles_n; wide.wide_tiles_n_padded = layout.tiles_n_padded;
     const bool products = p->inner_operator == KMC_OP_DOT;
     // Squared differences: a sample of the result first, so that data the trust rule would reject wholesale
     // (sets of near-duplicates) costs the direct kernel's time and little more, instead of both.
@@ -304,15 +332,10 @@ hipError_t launch_gram_f16_wide(const kmc_build_kernel_params *p, const kmc::Bui
         wide.kernel.sample = sample;
         if (sample_taken) *sample_taken = sample;
     }
-    if (args.symmetric) {
-        const dim3 grid(static_cast<unsigned>(layout.tiles_m) * (layout.tiles_m + 1) / 2, args.l, 1);
-        status = products ? launch(kmc::gram_f16_wide<true, kmc::GW_EPILOGUE_DOT>, grid, dim3(kmc::GW_THREADS), stream, wide)
-                          : launch(kmc::gram_f16_wide<true>, grid, dim3(kmc::GW_THREADS), stream, wide);
-    } else {
-        const dim3 grid(static_cast<unsigned>(layout.tiles_m) * layout.tiles_n_padded, args.l, 1);
-        status = products ? launch(kmc::gram_f16_wide<false, kmc::GW_EPILOGUE_DOT>, grid, dim3(kmc::GW_THREADS), stream, wide)
-                          : launch(kmc::gram_f16_wide<false>, grid, dim3(kmc::GW_THREADS), stream, wide);
-    }
+    if (args.symmetric)
+        status = products ? launch_product<true, kmc::GW_EPILOGUE_DOT>(wide, stream) : launch_product<true, kmc::GW_EPILOGUE_DISTANCE>(wide, stream);
+    else
+        status = products ? launch_product<false, kmc::GW_EPILOGUE_DOT>(wide, stream) : launch_product<false, kmc::GW_EPILOGUE_DISTANCE>(wide, stream);
     if (status == hipSuccess) *taken = true;
     return status;
 }
@@ -469,13 +492,11 @@ int launch_norm_gradient_l2_wide(const kmc_norm_gradient_params *p, hipStream_t 
     product.unscale_b_bs = wide.b.batches > 1 ? wide.b.rows_pad : 0;
     product.rows_pad_a = wide.a.rows_pad; product.rows_pad_b = wide.b.rows_pad;
     product.slices = wide.slices; product.ranges = wide.ranges;
-    product.wide_tiles_m = wide.tiles_m; product.wide_tiles_n = wide.tiles_n; product.wide_tiles_n_padded = wide.tiles_n_padded;
     product.gradient_d = p->d; product.gradient_d_ld = p->d_ld; product.gradient_d_bs = p->d_bs;
     product.gradient_g = g; product.gradient_g_ld = p->o; product.gradient_g_bs = weights.out_bs;
     product.gradient_shift = prepare.shift; product.gradient_shift_bs = prepare.shift_bs;
     product.gradient_n = p->n;
-    const dim3 grid(static_cast<unsigned>(wide.tiles_m) * wide.tiles_n_padded, p->l, 1);
-    status = launch(kmc::gram_f16_wide<false, kmc::GW_EPILOGUE_GRADIENT_L2>, grid, dim3(kmc::GW_THREADS), stream, product);
+    status = launch_product<false, kmc::GW_EPILOGUE_GRADIENT_L2>(product, stream);
     if (status != hipSuccess) return fail_hip(status, "gram_f16_wide (gradient) launch");
     *taken = true;
     return KMC_OK;

@@ -1,0 +1,55 @@
+"""The product kernel of the workspace route in both of its tiles (128 x 128, and 256 x 128 where those are many): edges of
+tiles and of steps of 32 k, one row and one column, sets against themselves, against float64 on a part of the batch."""
+import pytest
+import torch
+
+import kermac_amd as kermac
+
+pytestmark = pytest.mark.gpu
+
+# L x ceil(M / 256) x ceil(N / 128) says which tile runs: below 4096 the small one
+SHAPES = [
+    (1, 1, 1, 1), (1, 128, 128, 32), (1, 129, 127, 33), (3, 255, 257, 31), (2, 384, 130, 64), (1, 513, 640, 96),
+    (4100, 17, 9, 40), (1100, 300, 140, 33), (1030, 257, 256, 32), (2050, 1, 129, 65), (1030, 512, 129, 95),
+]
+
+
+def _truth(a, b, entries):
+    return (a[entries].double()[:, :, None, :] - b[entries].double()[:, None, :, :]).square().sum(-1).sqrt()
+
+
+@pytest.fixture(autouse=True)
+def any_size(monkeypatch):
+    monkeypatch.setenv("KERMAC_AMD_WIDE_MIN_TILES", "1")
+
+
+@pytest.mark.parametrize("L,M,N,K", SHAPES)
+@pytest.mark.parametrize("panel", [False, True])
+def test_distances_and_products(device, L, M, N, K, panel):
+    gen = torch.Generator(device=device).manual_seed(L + M + N + K)
+    a, b = (torch.randn(L, rows, K, device=device, generator=gen) for rows in (M, N))
+    if panel:
+        a, b = (x.transpose(1, 2).contiguous().transpose(1, 2) for x in (a, b))
+    entries = sorted({0, L // 2, L - 1})
+    with kermac.l2_mode("gram_bf16", min_k=1):
+        got = kermac.cdist(a, b, p=2.0)
+        dot = kermac.run_kernel(kermac.kernel_descriptor_mma, a, b)
+    truth = _truth(a, b, entries)
+    assert ((got[entries].double() - truth).abs() <= 1e-5 * truth).all()        # the route's stated tolerance
+    # error of the three products of pieces: below 3 * 2^-22 sum |a b|, beside the fp32 sum of K terms
+    exact = torch.matmul(a[entries].double(), b[entries].double().transpose(1, 2).contiguous())
+    scale = torch.matmul(a[entries].double().abs(), b[entries].double().abs().transpose(1, 2).contiguous())
+    assert ((dot[entries].double() - exact).abs() <= 1e-6 * scale).all()
+
+
+@pytest.mark.parametrize("L,M,K", [(1, 1, 5), (2, 130, 33), (1, 385, 64), (1400, 257, 40), (4200, 140, 32)])
+def test_a_set_against_itself(device, L, M, K):
+    gen = torch.Generator(device=device).manual_seed(M)
+    a = torch.randn(L, M, K, device=device, generator=gen)
+    entries = sorted({0, L // 2, L - 1})
+    with kermac.l2_mode("gram_bf16", min_k=1):
+        got = kermac.cdist(a, a, p=2.0)
+    truth = _truth(a, a, entries)
+    assert ((got[entries].double() - truth).abs() <= 1e-5 * truth).all()
+    assert torch.equal(got, got.transpose(1, 2))
+    assert (torch.diagonal(got, dim1=1, dim2=2) == 0).all()
