@@ -95,6 +95,18 @@ int prepare(const kmc_build_kernel_params *p, bool need_c, kmc::BuildKernelArgs 
     args->symmetric = need_c && !(p->flags & KMC_FLAG_NO_SYMMETRY) && exchangeable && p->a == p->b && p->m == p->n &&
                       p->a_ld == p->b_ld && p->a_bs == p->b_bs && p->a_majorness == p->b_majorness &&
                       p->regularization_offset_x == p->regularization_offset_y && tiles_m > 1;
+    // Rows of one set on both sides, possibly shifted: the same layout, and b starts a whole number of rows from a.
+    args->same_points = 0;
+    args->same_shift = 0;
+    if (p->inner_operator == KMC_OP_DIFF && p->a_majorness == p->b_majorness && p->a_ld == p->b_ld && p->a_bs == p->b_bs && p->a && p->b) {
+        const int64_t bytes = static_cast<int64_t>(reinterpret_cast<intptr_t>(p->b)) - static_cast<int64_t>(reinterpret_cast<intptr_t>(p->a));
+        const int64_t row = 4 * (p->a_majorness == KMC_ROW_MAJOR ? p->a_ld : 1);
+        const int64_t reach = static_cast<int64_t>(p->m) + p->n;
+        if (row > 0 && bytes % row == 0 && bytes / row < reach && bytes / row > -reach) {
+            args->same_points = 1;
+            args->same_shift = static_cast<int>(bytes / row);
+        }
+    }
     args->gram_trust = p->gram_trust > 0.0f ? p->gram_trust : 0.25f;
     if (p->k_total < 0) return fail(KMC_ERR_INVALID_ARGUMENT, "negative k_total %d", p->k_total);
     if (p->k_total > 0) {

@@ -637,9 +637,14 @@ __global__ __launch_bounds__(Tile::THREADS, Tile::MIN_WAVES) void gram_f16_wide(
     // such margin (v_minimum3_f32 hands a NaN on: overflowing squares and NaN data are not trusted).  Rows and columns
     // that do not exist have pieces and norms of zero: with a row or column that does exist they give d^2 = norms,
     // which is trusted unless that row's norm is not a number -- and then its own elements are not trusted either.
+    // A point against itself (BuildKernelArgs::same_points) is at distance zero, exactly, if its norm is a number: without
+    // that the parts on the diagonal are all distrusted, and the repair launch walks each of them on one CU (10000 points of
+    // K = 784 against themselves: 254 of 590 us; 338 with it).
     // The stores go through this wave's share of the ring (idle: every copy has arrived, and no wave reads it any
     // more), so that an instruction writes runs of WAVE_M floats of a column.
     float least_margin = 0.0f;
+    const int self_diagonal = n0 + wave_n + kernel->same_shift - m0 - wave_m;
+    const bool same_points = kernel->same_points != 0 && self_diagonal < Tile::WAVE_M && self_diagonal > -Tile::WAVE_N;
     float *stage = reinterpret_cast<float *>(ring) + wave * (4 * Tile::SLOTS * Tile::GRANULE_CHUNKS / Tile::WAVES);
     {
         constexpr int PITCH = Tile::WAVE_M + 4, LANES = Tile::WAVE_M / 4, PER_PASS = 64 / LANES;
@@ -666,6 +671,11 @@ __global__ __launch_bounds__(Tile::THREADS, Tile::MIN_WAVES) void gram_f16_wide(
                         const float minus_twice = (acc[mt][nt][e] * unscale_a[e]) * unscale_b;
                         acc[mt][nt][e] = norms + minus_twice;
                         margin[e] = norms * (1.0f - trust) + minus_twice;
+                        if (same_points) {
+                            const bool same = 16 * mt + 4 * q + e == self_diagonal + 16 * nt + i;
+                            acc[mt][nt][e] = same ? norms - norms : acc[mt][nt][e];
+                            margin[e] = same ? norms - norms : margin[e];
+                        }
                     }
                     asm("v_minimum3_f32 %0, %1, %2, %0" : "+v"(least_margin) : "v"(margin[0]), "v"(margin[1]));
                     asm("v_minimum3_f32 %0, %1, %2, %0" : "+v"(least_margin) : "v"(margin[2]), "v"(margin[3]));
