@@ -46,6 +46,7 @@
 #pragma once
 
 #include "gram_bf16_kernel.hpp"
+#include "gram_probe.hpp"
 
 namespace kmc {
 
@@ -81,7 +82,7 @@ struct GramWideArgs {
     i64 stats_a_bs, stats_b_bs;
     const float *unscale_a, *unscale_b;
     i64 unscale_a_bs, unscale_b_bs;
-    int rows_pad_a, rows_pad_b, slices, ranges;
+    int rows_pad_a, rows_pad_b, slices, ranges_a, ranges_b;
     int wide_tiles_m, wide_tiles_n, wide_tiles_n_padded;
     // GW_EPILOGUE_GRADIENT_L2 only: row r of b stands for (o, n) = (r / gradient_n, r % gradient_n) and
     // the result is (d[n][m] - shift[n]) * g[m][o] - a[m] . b[r]
@@ -167,6 +168,33 @@ __global__ __launch_bounds__(GW_ROW_THREADS) void gram_row_stats(const GramRowsA
     gram_row_stats_of(args, blockIdx.x);
 }
 
+// scale = 2^(GW_SCALE_EXPONENT - floor(log2 magnitude)), from the exponent field.  Rows of
+// zeros or of values below 2^-111 take the largest scale used, 2^125 (the scale and its
+// inverse must both be normal numbers); a row with a NaN or an infinity takes the smallest:
+// its products are not numbers whatever the scale.
+__device__ __forceinline__ int gram_scale_exponent(float magnitude)
+{
+    return max((int)(__float_as_uint(magnitude) >> 23) & 0xff, 16);
+}
+__device__ __forceinline__ float gram_scale(int exponent_field)
+{
+    return __uint_as_float((unsigned)(127 + GW_SCALE_EXPONENT + 127 - exponent_field) << 23);
+}
+__device__ __forceinline__ float gram_unscale(int exponent_field)
+{
+    return __uint_as_float((unsigned)(exponent_field - GW_SCALE_EXPONENT) << 23);
+}
+
+// Two scaled values into their two pieces, packed.
+__device__ __forceinline__ void gram_split_pair(float x0, float x1, unsigned &first, unsigned &second)
+{
+    const gram_half2 h1 = __builtin_convertvector(gram_float2{x0, x1}, gram_half2);
+    const gram_float2 back = __builtin_convertvector(h1, gram_float2);
+    const gram_half2 h2 = __builtin_convertvector(gram_float2{x0 - back.x, x1 - back.y}, gram_half2);
+    first = __builtin_bit_cast(unsigned, h1);
+    second = __builtin_bit_cast(unsigned, h2);
+}
+
 __device__ __forceinline__ void gram_f16_split_of(const GramRowsArgs &args, int block)
 {
     const int row = block * GW_ROW_THREADS + threadIdx.x;
@@ -174,21 +202,15 @@ __device__ __forceinline__ void gram_f16_split_of(const GramRowsArgs &args, int 
     const float *x = args.x + batch * args.bs;
     const float *centre = gram_rows_centre(args, batch);
 
-    // scale = 2^(GW_SCALE_EXPONENT - floor(log2 magnitude)), from the exponent field.  Rows of
-    // zeros or of values below 2^-111 take the largest scale used, 2^125 (the scale and its
-    // inverse must both be normal numbers); a row with a NaN or an infinity takes the smallest:
-    // its products are not numbers whatever the scale.
     float magnitude = 0.0f;
     for (int r = 0; r < args.ranges; r++) {
         const float part = args.magnitudes[batch * args.stats_bs + (i64)r * args.rows_pad + row];
         magnitude = part != part ? part : fmaxf(magnitude, part);
         if (part != part) break;
     }
-    int exponent_field = (__float_as_uint(magnitude) >> 23) & 0xff;
-    exponent_field = max(exponent_field, 16);
-    const float scale = __uint_as_float((unsigned)(127 + GW_SCALE_EXPONENT + 127 - exponent_field) << 23);
-    if (range == 0)
-        args.unscale[batch * args.unscale_bs + row] = __uint_as_float((unsigned)(exponent_field - GW_SCALE_EXPONENT) << 23);
+    const int exponent_field = gram_scale_exponent(magnitude);
+    const float scale = gram_scale(exponent_field);
+    if (range == 0) args.unscale[batch * args.unscale_bs + row] = gram_unscale(exponent_field);
 
     gram_chunk *pieces = args.pieces + batch * args.pieces_bs;
     const int first = range * args.slices_per_range;
@@ -198,14 +220,7 @@ __device__ __forceinline__ void gram_f16_split_of(const GramRowsArgs &args, int 
         gram_load_row_slice(args, x, centre, row, slice, v);
         unsigned int piece[GW_PIECES][8];
 #pragma unroll
-        for (int q = 0; q < 8; q++) {
-            const float x0 = v[2 * q] * scale, x1 = v[2 * q + 1] * scale;
-            const gram_half2 h1 = __builtin_convertvector(gram_float2{x0, x1}, gram_half2);
-            const gram_float2 back = __builtin_convertvector(h1, gram_float2);
-            const gram_half2 h2 = __builtin_convertvector(gram_float2{x0 - back.x, x1 - back.y}, gram_half2);
-            piece[0][q] = __builtin_bit_cast(unsigned int, h1);
-            piece[1][q] = __builtin_bit_cast(unsigned int, h2);
-        }
+        for (int q = 0; q < 8; q++) gram_split_pair(v[2 * q] * scale, v[2 * q + 1] * scale, piece[0][q], piece[1][q]);
         gram_chunk *dst = pieces + (i64)slice * GW_SEGMENTS * args.rows_pad + row;
 #pragma unroll
         for (int p = 0; p < GW_PIECES; p++)
@@ -255,6 +270,133 @@ __global__ __launch_bounds__(GW_ROW_THREADS) void gram_f16_split_pair(const Gram
     } else if ((int)blockIdx.z < pair.second_batches) {
         gram_f16_split_of(pair.second, blockIdx.x - pair.first_blocks);
     }
+}
+
+// Both steps in one pass for operands with k contiguous and at most GRO_MAX_K of them: a workgroup holds 16 whole rows in its
+// registers, so the values are read once and the scale is known before the pieces are written.  Wave w takes the slices w,
+// w + 4, ..; four lanes share a slice of a row, 4 k each (a load instruction reads 64 consecutive bytes of 16 rows, the four
+// waves together 256); two neighbours exchange halves so that one stores the chunk of the first piece and the other that
+// of the second, and a store instruction writes four runs of 256 bytes.  (A wave on four rows of 64 lanes' k wrote runs of 64
+// bytes.)  Bound by its bytes, 4 read and 4 written per value.  The squares are one sum
+// per row.  In front of the row workgroups in the grid stand those of the sample (gram_probe.hpp), which needs
+// nothing of theirs: at a few thousand rows every launch of this prelude is its own latency.  Statistics, split and sample in three launches, and now:
+// 1000 + 60000 rows of K = 784 53 + 89 + 12 -> 110 us, 10000 rows 12 + 13 + 10 -> 27 us, 2 x 2000 rows 10 + 12 + 11 -> 18 us.
+constexpr int GRO_ROWS = 16;                                  // per workgroup
+constexpr int GRO_WAVES = GW_ROW_THREADS / 64;
+constexpr int GRO_MAX_K = 1024;
+
+struct GramRowsOnceArgs {
+    GramRowsArgs first, second;
+    int samples, first_blocks;                 // workgroups along x: those of the sample (in the first batch), then of the first operand
+    int first_batches, second_batches;
+    GramProbeArgs probe;
+};
+
+template <int GROUPS>
+__device__ __forceinline__ void gram_rows_once_of(const GramRowsArgs &args, int block)
+{
+    __shared__ float squares[GRO_WAVES][GRO_ROWS], magnitudes[GRO_WAVES][GRO_ROWS];
+    const int wave = threadIdx.x >> 6, r = (threadIdx.x & 63) >> 2, quarter = threadIdx.x & 3;
+    const int row = block * GRO_ROWS + r, batch = blockIdx.z;
+    const bool live = row < args.rows;
+    const float *src = args.x + batch * args.bs + (i64)(live ? row : args.rows - 1) * args.ld;
+    const float *centre = gram_rows_centre(args, batch);
+    const int groups = (args.k + 63) / 64;
+    const int k0 = BK_TILE_K * wave + 4 * quarter;             // and every 64 behind it
+    float v[GROUPS][4];
+    // Loads of what does not exist go to the last element that does and are dropped: with a branch per load they would be
+    // waited for one by one (198 instead of 110 us for 61000 rows).
+    if (args.vec && args.k % 4 == 0) {
+#pragma unroll
+        for (int g = 0; g < GROUPS; g++) {
+            const float4 f = *reinterpret_cast<const float4 *>(src + min(64 * g + k0, args.k - 4));
+            v[g][0] = f.x; v[g][1] = f.y; v[g][2] = f.z; v[g][3] = f.w;
+        }
+    } else {
+#pragma unroll
+        for (int g = 0; g < GROUPS; g++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[g][e] = src[min(64 * g + k0 + e, args.k - 1)];
+    }
+    if (centre) {
+        // padded with zeros to whole groups of 64 k
+        const bool aligned = (reinterpret_cast<unsigned long>(centre) & 15) == 0;
+        const int last = 64 * (groups - 1);
+        if (aligned) {
+#pragma unroll
+            for (int g = 0; g < GROUPS; g++) {
+                const float4 f = *reinterpret_cast<const float4 *>(centre + min(64 * g, last) + k0);
+                v[g][0] -= f.x; v[g][1] -= f.y; v[g][2] -= f.z; v[g][3] -= f.w;
+            }
+        } else {
+#pragma unroll
+            for (int g = 0; g < GROUPS; g++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) v[g][e] -= centre[min(64 * g, last) + k0 + e];
+        }
+    }
+#pragma unroll
+    for (int g = 0; g < GROUPS; g++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[g][e] = live && 64 * g + k0 + e < args.k ? v[g][e] : 0.0f;
+    float square = 0.0f, magnitude = 0.0f;
+    bool not_a_number = false;
+#pragma unroll
+    for (int g = 0; g < GROUPS; g++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            square += v[g][e] * v[g][e];
+            magnitude = fmaxf(magnitude, fabsf(v[g][e]));      // skips NaNs
+            not_a_number |= v[g][e] != v[g][e];
+        }
+    if (not_a_number) magnitude = __builtin_inff();            // takes the same scale as a NaN
+#pragma unroll
+    for (int offset = 2; offset > 0; offset >>= 1) {
+        square += __shfl_xor(square, offset);
+        magnitude = fmaxf(magnitude, __shfl_xor(magnitude, offset));
+    }
+    if (quarter == 0) {
+        squares[wave][r] = square;
+        magnitudes[wave][r] = magnitude;
+    }
+    __syncthreads();
+    magnitude = fmaxf(fmaxf(magnitudes[0][r], magnitudes[1][r]), fmaxf(magnitudes[2][r], magnitudes[3][r]));
+    const int exponent_field = gram_scale_exponent(magnitude);
+    const float scale = gram_scale(exponent_field);
+    if (wave == 0 && quarter == 0) {
+        args.squares[batch * args.stats_bs + row] = (squares[0][r] + squares[1][r]) + (squares[2][r] + squares[3][r]);
+        args.unscale[batch * args.unscale_bs + row] = gram_unscale(exponent_field);
+    }
+    gram_chunk *pieces = args.pieces + batch * args.pieces_bs;
+    const int all_slices = args.slices + args.zero_slices;
+    const bool second = quarter & 1;
+    const int segment = 2 * (second ? 1 : 0) + (quarter >> 1);
+#pragma unroll
+    for (int g = 0; g < GROUPS; g++) {
+        const int slice = 4 * g + wave;
+        unsigned h1[2], h2[2];
+#pragma unroll
+        for (int q = 0; q < 2; q++) gram_split_pair(v[g][2 * q] * scale, v[g][2 * q + 1] * scale, h1[q], h2[q]);
+        // the even lane holds the first half of both pieces' chunks, the odd one the second half
+        const unsigned give0 = second ? h1[0] : h2[0], give1 = second ? h1[1] : h2[1];
+        const unsigned got0 = (unsigned)__shfl_xor((int)give0, 1), got1 = (unsigned)__shfl_xor((int)give1, 1);
+        const gram_chunk chunk = second ? gram_chunk{got0, got1, h2[0], h2[1]} : gram_chunk{h1[0], h1[1], got0, got1};
+        if (slice < all_slices) pieces[((i64)slice * GW_SEGMENTS + segment) * args.rows_pad + row] = chunk;
+    }
+}
+
+template <int GROUPS>
+__global__ __launch_bounds__(GW_ROW_THREADS, 2) void gram_rows_once(const GramRowsOnceArgs args)
+{
+    static_assert(GW_ROW_THREADS == GP_THREADS, "both parts of the launch");
+    const int block = (int)blockIdx.x - args.samples;
+    if (block < 0) {
+        if (blockIdx.z == 0) gram_probe_tile(args.probe, blockIdx.x);
+        return;
+    }
+    const bool first = block < args.first_blocks;
+    if ((int)blockIdx.z < (first ? args.first_batches : args.second_batches))
+        gram_rows_once_of<GROUPS>(first ? args.first : args.second, first ? block : block - args.first_blocks);
 }
 
 // Tile shapes of the product kernel.  A workgroup is 4 waves; a wave owns WAVE_M rows of a and WAVE_N rows of b as
@@ -520,14 +662,14 @@ __global__ __launch_bounds__(Tile::THREADS, Tile::MIN_WAVES) void gram_f16_wide(
         const int r = of_a ? at : at - TILE_M;
         if constexpr (EPILOGUE == GW_EPILOGUE_DISTANCE) {
             const float *partial = of_a ? args.squares_a + batch * args.stats_a_bs + m0 + r : args.squares_b + batch * args.stats_b_bs + n0 + r;
-            const int pitch = of_a ? args.rows_pad_a : args.rows_pad_b;
+            const int pitch = of_a ? args.rows_pad_a : args.rows_pad_b, ranges = of_a ? args.ranges_a : args.ranges_b;
             // all loads first, then the sum in range order: a loop would wait for each load in turn
             float parts[GW_MAX_RANGES];
 #pragma unroll
-            for (int range = 0; range < GW_MAX_RANGES; range++) parts[range] = range < args.ranges ? partial[(i64)range * pitch] : 0.0f;
+            for (int range = 0; range < GW_MAX_RANGES; range++) parts[range] = range < ranges ? partial[(i64)range * pitch] : 0.0f;
             float norm = 0.0f;
 #pragma unroll
-            for (int range = 0; range < GW_MAX_RANGES; range++) norm += range < args.ranges ? parts[range] : 0.0f;
+            for (int range = 0; range < GW_MAX_RANGES; range++) norm += range < ranges ? parts[range] : 0.0f;
             (of_a ? lds_norm_a : lds_norm_b)[r] = norm;
         }
         (of_a ? lds_unscale_a : lds_unscale_b)[r] =

@@ -23,13 +23,15 @@ constexpr int64_t REGION_ALIGN = 256;
 
 struct OperandRegions {
     int rows_pad, batches;
+    int slices_per_range, ranges;    // of the partial sums of squares
+    bool once;               // gram_rows_once makes the pieces
     int64_t pieces_bs;       // chunks per batch entry
     int64_t stats_bs;        // floats per batch entry, for the squares and for the magnitudes
     int64_t pieces, squares, magnitudes, unscale;   // byte offsets into the workspace
 };
 
 struct WideLayout {
-    int slices, slices_per_range, ranges;
+    int slices;
     int tiles_m, tiles_n;       // of GW_TILE x GW_TILE
     OperandRegions a, b;
     int64_t sample;         // byte offset of the words of gram_probe_operands
@@ -94,12 +96,17 @@ int64_t place(int64_t &cursor, int64_t bytes)
     return at;
 }
 
-void place_operand(OperandRegions &r, int rows, bool broadcast, int l, const WideLayout &layout, int64_t &cursor)
+void place_operand(OperandRegions &r, int rows, bool broadcast, int l, bool once, const WideLayout &layout, int64_t &cursor)
 {
+    // at most 8 ranges of K per row (9 by the rounding): enough workgroups for the row kernels, few partial sums
+    r.once = once;
+    r.slices_per_range = once ? layout.slices : layout.slices / 8 > 8 ? (layout.slices + 7) / 8 : 8;
+    r.ranges = (layout.slices + r.slices_per_range - 1) / r.slices_per_range;
+    static_assert(kmc::GW_MAX_RANGES == 9, "the two lines above");
     r.rows_pad = (rows + kmc::GW_TILE - 1) / kmc::GW_TILE * kmc::GW_TILE;
     r.batches = broadcast ? 1 : l;
     r.pieces_bs = static_cast<int64_t>(2 * ((layout.slices + 1) / 2)) * kmc::GW_SEGMENTS * r.rows_pad;      // whole steps of the walk
-    r.stats_bs = static_cast<int64_t>(layout.ranges) * r.rows_pad;
+    r.stats_bs = static_cast<int64_t>(r.ranges) * r.rows_pad;
     r.pieces = place(cursor, r.batches * r.pieces_bs * 16);
     r.squares = place(cursor, r.batches * r.stats_bs * 4);
     r.magnitudes = place(cursor, r.batches * r.stats_bs * 4);
@@ -107,19 +114,18 @@ void place_operand(OperandRegions &r, int rows, bool broadcast, int l, const Wid
 }
 
 // Grid, slices and the regions of both operands in the workspace; tiles_m and tiles_n are set.
-bool place_wide(int m, int n, int k, int l, bool a_once, bool b_once, bool symmetric, WideLayout *layout)
+// a_shared, b_shared: one operand for all batch entries.  a_rows, b_rows: its k are contiguous, so that one pass can make the
+// pieces of a short row (gram_rows_once).
+bool place_wide(int m, int n, int k, int l, bool a_shared, bool b_shared, bool a_rows, bool b_rows, bool symmetric, WideLayout *layout)
 {
     // room for any tile of the product kernel in a grid, n tiles padded to the XCDs
     if (static_cast<int64_t>(layout->tiles_m) * (layout->tiles_n + kmc::BK_XCDS) * 4 > 0x7fffffff) return false;
     layout->slices = (k + kmc::BK_TILE_K - 1) / kmc::BK_TILE_K;
-    // at most 8 ranges of K per row: enough workgroups for the row kernels, few partial sums
-    layout->slices_per_range = layout->slices / 8 > 8 ? (layout->slices + 7) / 8 : 8;
-    layout->ranges = (layout->slices + layout->slices_per_range - 1) / layout->slices_per_range;
-    if (layout->ranges > kmc::GW_MAX_RANGES) return false;       // 9 at most by the two lines above
     int64_t cursor = 0;
-    place_operand(layout->a, m, a_once, l, *layout, cursor);
+    const bool fits = k <= kmc::GRO_MAX_K;
+    place_operand(layout->a, m, a_shared, l, a_rows && fits, *layout, cursor);
     if (symmetric) layout->b = layout->a;      // one panel, split once
-    else place_operand(layout->b, n, b_once, l, *layout, cursor);
+    else place_operand(layout->b, n, b_shared, l, b_rows && fits, *layout, cursor);
     layout->sample = place(cursor, kmc::BK_SAMPLE_BYTES);
     layout->bytes = cursor;
     return true;
@@ -142,7 +148,8 @@ bool wide_layout(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &a
     // an operand that is the same for every batch entry is split once, unless the centre differs
     // (products have no centre: the caller's parameter block carries none into `args`)
     const bool one_centre = products || !args.centre || args.centre_bs == 0;
-    return place_wide(args.m, args.n, args.k, args.l, args.a_bs == 0 && one_centre, args.b_bs == 0 && one_centre, args.symmetric, layout);
+    return place_wide(args.m, args.n, args.k, args.l, args.a_bs == 0 && one_centre, args.b_bs == 0 && one_centre,
+                      p->a_majorness == KMC_ROW_MAJOR, p->b_majorness == KMC_ROW_MAJOR, args.symmetric, layout);
 }
 
 kmc::GramRowsArgs rows_args(const float *x, int64_t ld, int64_t bs, int rows, int majorness, bool scalar_only,
@@ -160,7 +167,7 @@ kmc::GramRowsArgs rows_args(const float *x, int64_t ld, int64_t bs, int rows, in
     rows_of.unscale = reinterpret_cast<float *>(workspace + r.unscale);
     rows_of.stats_bs = r.stats_bs; rows_of.unscale_bs = r.rows_pad;
     rows_of.rows_pad = r.rows_pad; rows_of.slices = layout.slices;
-    rows_of.slices_per_range = layout.slices_per_range; rows_of.ranges = layout.ranges;
+    rows_of.slices_per_range = r.slices_per_range; rows_of.ranges = r.ranges;
     rows_of.zero_slices = layout.slices & 1;      // the walk takes two slices per step
     return rows_of;
 }
@@ -212,6 +219,7 @@ void forget_split_in(const void *workspace)
 
 // Statistics and split of one operand (also used by the gradient's fp16 route).
 hipError_t launch_gram_probe(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &args, unsigned *sample, hipStream_t stream);   // gram_probe.hip
+kmc::GramProbeArgs gram_probe_args(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &args, unsigned *sample);                 // gram_probe.hip
 
 hipError_t launch_gram_rows(const kmc::GramRowsArgs &rows_of, int batches, hipStream_t stream)
 {
@@ -237,6 +245,32 @@ hipError_t launch_gram_rows_pair(const kmc::GramRowsArgs &first, int first_batch
     hipError_t status = launch(kmc::gram_row_stats_pair<0>, grid, dim3(kmc::GW_ROW_THREADS), stream, pair);
     if (status != hipSuccess) return status;
     return launch(kmc::gram_f16_split_pair<0>, grid, dim3(kmc::GW_ROW_THREADS), stream, pair);
+}
+
+// The pieces of the operands that are not null, and in front of them the sample if there is one, in one launch.
+hipError_t launch_gram_rows_once(const kmc::GramRowsArgs *first, int first_batches, const kmc::GramRowsArgs *second, int second_batches,
+                                 const kmc::GramProbeArgs &probe, bool take_sample, hipStream_t stream)
+{
+    kmc::GramRowsOnceArgs args = {};
+    args.probe = probe;
+    args.samples = take_sample ? kmc::BK_SAMPLE_TILES : 0;
+    int blocks = args.samples, k = 0, batches = 1;
+    if (first) {
+        args.first = *first; args.first_batches = batches = first_batches;
+        args.first_blocks = first->rows_pad / kmc::GRO_ROWS;
+        blocks += args.first_blocks;
+        k = first->k;
+    }
+    if (second) {
+        args.second = *second; args.second_batches = second_batches;
+        if (second_batches > batches) batches = second_batches;
+        blocks += second->rows_pad / kmc::GRO_ROWS;
+        k = second->k;
+    }
+    const dim3 grid(blocks, 1, batches), threads(kmc::GW_ROW_THREADS);
+    // registers for 64, 128 or 256 values of a row per lane group: the smallest that holds a row
+    return k <= 256 ? launch(kmc::gram_rows_once<4>, grid, threads, stream, args)
+         : k <= 512 ? launch(kmc::gram_rows_once<8>, grid, threads, stream, args) : launch(kmc::gram_rows_once<16>, grid, threads, stream, args);
 }
 
 // The product kernel in tiles of TILE; extents, batch entries and operands of `wide` are set.
@@ -291,25 +325,42 @@ hipError_t launch_gram_f16_wide(const kmc_build_kernel_params *p, const kmc::Bui
     const bool scalar_only = (p->flags & KMC_FLAG_FORCE_SCALAR_ACCESS) != 0;
     const kmc::GramRowsArgs rows_a = rows_args(args.a, args.a_ld, args.a_bs, args.m, p->a_majorness, scalar_only, args, layout, layout.a, workspace);
     const kmc::GramRowsArgs rows_b = rows_args(args.b, args.b_ld, args.b_bs, args.n, p->b_majorness, scalar_only, args, layout, layout.b, workspace);
-    // the region of a lies first in the workspace and its size does not depend on b
-    const bool a_is_kept = split_of_a_is_kept(p, args, layout);
-    hipError_t status = hipSuccess;
-    if (!a_is_kept && !args.symmetric) {
-        status = launch_gram_rows_pair(rows_a, layout.a.batches, rows_b, layout.b.batches, stream);
-    } else {
-        if (!a_is_kept) status = launch_gram_rows(rows_a, layout.a.batches, stream);
-        if (status == hipSuccess && !args.symmetric) status = launch_gram_rows(rows_b, layout.b.batches, stream);
-    }
-    if (status != hipSuccess) return status;
-
-    kmc::GramWideArgs wide = {};
-    wide.kernel = args;
     // The caller's trust rule grows with sqrt(k) (the error of a sum of k terms against the norms) and
     // passes 1 near k = 18000, where it would send every part to the repair launch -- whose own
     // fp32 sum over k is no better by then (measured at k = 20000 .. 200000: this walk, which rounds once
     // per 16 k, 4e-7 .. 2e-6 of d for points as far apart as their norms, the direct kernel 5e-6 .. 4e-5).
     // With a product worth half the norms the two are equally good, so that is where the rule stops.
+    kmc::GramWideArgs wide = {};
+    wide.kernel = args;
     if (wide.kernel.gram_trust > 0.5f) wide.kernel.gram_trust = 0.5f;
+    const bool products = p->inner_operator == KMC_OP_DOT;
+    // Squared differences: a sample of the result first, so that data the trust rule would reject wholesale
+    // (sets of near-duplicates) costs the direct kernel's time and little more, instead of both.
+    // KMC_FLAG_NO_PROBE leaves it out.
+    unsigned *sample = !products && !(p->flags & KMC_FLAG_NO_PROBE) ? reinterpret_cast<unsigned *>(workspace + layout.sample) : nullptr;
+    // the region of a lies first in the workspace and its size does not depend on b
+    const bool a_is_kept = split_of_a_is_kept(p, args, layout);
+    const bool split_a = !a_is_kept, split_b = !args.symmetric;
+    bool sampled = false;
+    hipError_t status = hipSuccess;
+    if ((split_a && layout.a.once) || (split_b && layout.b.once)) {
+        status = launch_gram_rows_once(split_a && layout.a.once ? &rows_a : nullptr, layout.a.batches, split_b && layout.b.once ? &rows_b : nullptr,
+                                       layout.b.batches, sample ? gram_probe_args(p, wide.kernel, sample) : kmc::GramProbeArgs{}, sample != nullptr, stream);
+        sampled = true;
+    }
+    if (status == hipSuccess && split_a && split_b && !layout.a.once && !layout.b.once) {
+        status = launch_gram_rows_pair(rows_a, layout.a.batches, rows_b, layout.b.batches, stream);
+    } else {
+        if (status == hipSuccess && split_a && !layout.a.once) status = launch_gram_rows(rows_a, layout.a.batches, stream);
+        if (status == hipSuccess && split_b && !layout.b.once) status = launch_gram_rows(rows_b, layout.b.batches, stream);
+    }
+    if (status == hipSuccess && sample && !sampled) status = launch_gram_probe(p, wide.kernel, sample, stream);
+    if (status != hipSuccess) return status;
+    if (sample) {
+        wide.kernel.sample = sample;
+        if (sample_taken) *sample_taken = sample;
+    }
+
     wide.pieces_a = rows_a.pieces; wide.pieces_b = rows_b.pieces;
     wide.pieces_a_bs = layout.a.batches > 1 ? layout.a.pieces_bs : 0;
     wide.pieces_b_bs = layout.b.batches > 1 ? layout.b.pieces_bs : 0;
@@ -320,18 +371,7 @@ hipError_t launch_gram_f16_wide(const kmc_build_kernel_params *p, const kmc::Bui
     wide.unscale_a_bs = layout.a.batches > 1 ? layout.a.rows_pad : 0;
     wide.unscale_b_bs = layout.b.batches > 1 ? layout.b.rows_pad : 0;
     wide.rows_pad_a = layout.a.rows_pad; wide.rows_pad_b = layout.b.rows_pad;
-    wide.slices = layout.slices; wide.ranges = layout.ranges;
-    const bool products = p->inner_operator == KMC_OP_DOT;
-    // Squared differences: a sample of the result first, so that data the trust rule would reject wholesale
-    // (sets of near-duplicates) costs the direct kernel's time and little more, instead of both.
-    // KMC_FLAG_NO_PROBE leaves it out.
-    if (!products && !(p->flags & KMC_FLAG_NO_PROBE)) {
-        unsigned *sample = reinterpret_cast<unsigned *>(workspace + layout.sample);
-        status = launch_gram_probe(p, wide.kernel, sample, stream);
-        if (status != hipSuccess) return status;
-        wide.kernel.sample = sample;
-        if (sample_taken) *sample_taken = sample;
-    }
+    wide.slices = layout.slices; wide.ranges_a = layout.a.ranges; wide.ranges_b = layout.b.ranges;
     if (args.symmetric)
         status = products ? launch_product<true, kmc::GW_EPILOGUE_DOT>(wide, stream) : launch_product<true, kmc::GW_EPILOGUE_DISTANCE>(wide, stream);
     else
@@ -390,7 +430,7 @@ bool gradient_l2_layout(const kmc_norm_gradient_params *p, GradientL2Layout *lay
     wide.tiles_m = (p->m + kmc::GW_TILE - 1) / kmc::GW_TILE;
     wide.tiles_n = static_cast<int>((rows + kmc::GW_TILE - 1) / kmc::GW_TILE);
     if (!gradient_l2_pays(p, wide.tiles_m, wide.tiles_n)) return false;
-    if (!place_wide(p->m, static_cast<int>(rows), p->k, p->l, p->a_bs == 0, false, false, &wide)) return false;
+    if (!place_wide(p->m, static_cast<int>(rows), p->k, p->l, p->a_bs == 0, false, false, false, false, &wide)) return false;
     int64_t cursor = wide.bytes;
     layout->products_ld = (p->k + 3) / 4 * 4;
     layout->products = place(cursor, static_cast<int64_t>(p->l) * rows * layout->products_ld * 4);
@@ -491,7 +531,7 @@ int launch_norm_gradient_l2_wide(const kmc_norm_gradient_params *p, hipStream_t 
     product.unscale_a_bs = wide.a.batches > 1 ? wide.a.rows_pad : 0;
     product.unscale_b_bs = wide.b.batches > 1 ? wide.b.rows_pad : 0;
     product.rows_pad_a = wide.a.rows_pad; product.rows_pad_b = wide.b.rows_pad;
-    product.slices = wide.slices; product.ranges = wide.ranges;
+    product.slices = wide.slices; product.ranges_a = wide.a.ranges; product.ranges_b = wide.b.ranges;
     product.gradient_d = p->d; product.gradient_d_ld = p->d_ld; product.gradient_d_bs = p->d_bs;
     product.gradient_g = g; product.gradient_g_ld = p->o; product.gradient_g_bs = weights.out_bs;
     product.gradient_shift = prepare.shift; product.gradient_shift_bs = prepare.shift_bs;

@@ -53,3 +53,39 @@ def test_a_set_against_itself(device, L, M, K):
     assert ((got[entries].double() - truth).abs() <= 1e-5 * truth).all()
     assert torch.equal(got, got.transpose(1, 2))
     assert (torch.diagonal(got, dim1=1, dim2=2) == 0).all()
+
+
+@pytest.mark.parametrize("K", [3, 255, 256, 257, 260, 511, 512, 513, 1000, 1023, 1024, 1025])
+@pytest.mark.parametrize("form", ["rows", "misaligned", "a_panel", "b_panel", "offset"])
+def test_rows_of_any_length(device, K, form):
+    """Pieces made in one pass (k contiguous, K up to 1024) and in two, in every mixture, with and without a centre."""
+    L, M, N = 2, 131, 47
+    gen = torch.Generator(device=device).manual_seed(K)
+    a, b = (torch.randn(L, rows, K, device=device, generator=gen) for rows in (M, N))
+    if form == "misaligned":
+        a, b = (torch.nn.functional.pad(x, (1, 0))[:, :, 1:] for x in (a, b))
+    elif form == "a_panel":
+        a = a.transpose(1, 2).contiguous().transpose(1, 2)
+    elif form == "b_panel":
+        b = b.transpose(1, 2).contiguous().transpose(1, 2)
+    elif form == "offset":
+        a, b = a + 30.0, b + 30.0
+    with kermac.l2_mode("gram_bf16", min_k=1):
+        got = kermac.cdist(a, b, p=2.0)
+        alone = kermac.cdist(a, a, p=2.0)
+    # the rounding of the offset operands themselves is in both sides
+    truth, truth_alone = _truth(a, b, [0, 1]), _truth(a, a, [0, 1])
+    assert ((got.double() - truth).abs() <= 1e-5 * truth).all()
+    assert ((alone.double() - truth_alone).abs() <= 1e-5 * truth_alone).all()
+
+
+def test_rows_that_are_not_numbers(device):
+    gen = torch.Generator(device=device).manual_seed(3)
+    a, b = (torch.randn(rows, 300, device=device, generator=gen) for rows in (200, 150))
+    a[5, 7], b[9, 299] = float("nan"), float("inf")
+    with kermac.l2_mode("gram_bf16", min_k=1):
+        got = kermac.cdist(a, b, p=2.0)[0]
+    truth = _truth(a[None], b[None], [0])[0]
+    assert torch.equal(torch.isnan(got), torch.isnan(truth)) and torch.equal(torch.isinf(got), torch.isinf(truth))
+    finite = torch.isfinite(truth)
+    assert ((got.double() - truth).abs() <= 1e-5 * truth)[finite].all()
