@@ -742,13 +742,20 @@ def _auto_matrix_core_flags(params, asked):
                 return 0
         finally:
             params.flags = kept
-    if not rows_contiguous:
+    if not rows_contiguous and not _against_itself(params):
         if (params.k >= _AUTO_FP32_MIN_K and _AUTO_FP32_MIN_TILES <= tiles * params.l <= _AUTO_FP32_MAX_TILES
                 and tiles >= _AUTO_FP32_MIN_TILES_PER_ENTRY):
             return _backend.FLAG_L2_GRAM
         if min(params.m, params.n) <= 128 and tiles * params.l >= _AUTO_FP32_MIN_TILES:      # one long row of tiles
             return _backend.FLAG_L2_GRAM
     return asked
+
+
+def _against_itself(params):
+    """Whether both operands are the same rows in memory.  The fp32 one-step kernel distrusts every tile on the diagonal of such
+    a result and leaves it to the repair launch, the split kernel knows that the distances there are zero."""
+    return (params.a == params.b and params.a_ld == params.b_ld and params.a_bs == params.b_bs
+            and params.a_majorness == params.b_majorness)
 
 
 def _workspace_route_applies(params, flags):

@@ -21,6 +21,12 @@
     X(WIDE_K_CONTIGUOUS_MIN_TILES, 48)                                                                  \
     X(WIDE_K_CONTIGUOUS_MIN_TILES_TIMES_K, 36864)                                                       \
     X(WIDE_K_CONTIGUOUS_MIN_ROWS, 129)     /* in both directions */                                     \
+    /* ... a set against itself, tiles of its triangle: k contiguous, and rows contiguous */              \
+    X(WIDE_SYMMETRIC_K_CONTIGUOUS_MIN_K, 128)                                                           \
+    X(WIDE_SYMMETRIC_K_CONTIGUOUS_MIN_TILES, 20)                                                        \
+    X(WIDE_SYMMETRIC_K_CONTIGUOUS_MIN_TILES_TIMES_K, 9000)                                              \
+    X(WIDE_SYMMETRIC_MIN_TILES, 32)                                                                     \
+    X(WIDE_SYMMETRIC_MIN_TILES_TIMES_K, 54000)                                                          \
     /* the product kernel's tile: 256 x 128 from this many of them over the batch on, 128 x 128 below */    \
     X(WIDE_LARGE_TILE_MIN_TILES, 4096)                                                                  \
     /* sums of products through the workspace (the alternative is the direct kernel) */                 \

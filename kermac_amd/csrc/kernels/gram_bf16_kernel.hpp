@@ -368,6 +368,7 @@ __global__ __launch_bounds__(BK_THREADS, RAGGED_K ? 2 : GB_WAVES) void gram_bf16
     }
     __syncthreads();
 
+    constexpr bool GRAM_SAME_POINTS = true;
 #include "gram_epilogue.inc"
 }
 

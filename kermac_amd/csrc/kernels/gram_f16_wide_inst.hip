@@ -67,8 +67,14 @@ struct WideLayout {
 // 2 x 118 tiles 1.07 at K = 256, 1.3 at K = 784; 36 tiles 0.9 / 1.2; 32 tiles as 8 entries of 2 x 2 0.75 / 0.8;
 // K = 128 never above 1).  Not for a dimension that half a tile holds, where the 128 x 128 tiles of the
 // one-step kernels waste half as much (100 x 50000: 0.87 at K = 784, 4 entries 0.73; 128 x 20000 0.8).
+//
+// A set against itself (the tiles of one triangle): one round of workgroups either way, whose walk is the route's faster one
+// (one-step split kernel / route, us, k contiguous: 1400 points, 21 tiles, at K = 784 77 / 63; 2000 at K = 256 66 / 52, at
+// K = 784 152 / 65, at K = 3072 502 / 160; 3000 at K = 128 59 / 50; 4 x 1000 at K = 784 163 / 67; 1000 at K = 784, 10 tiles, 63 / 61;
+// rows contiguous: 2000 at K = 784 82 / 85, at K = 3072 248 / 167; 2400 at K = 1024 106 / 90; 3500 at K = 512 95 / 88; 3000 at
+// K = 128 46 / 70).
 bool wide_pays(int64_t m, int64_t n, int64_t tiles_m, int64_t tiles_n, int64_t tiles, int k, bool products, bool k_contiguous,
-               bool batched)
+               bool batched, bool symmetric)
 {
     const char *text = std::getenv("KERMAC_AMD_WIDE_MIN_TILES");
     const int forced = text ? std::atoi(text) : 0;
@@ -76,6 +82,11 @@ bool wide_pays(int64_t m, int64_t n, int64_t tiles_m, int64_t tiles_n, int64_t t
     namespace r = kmc_rules;
     if (k_contiguous && !products && k >= r::WIDE_K_CONTIGUOUS_MIN_K && tiles >= r::WIDE_K_CONTIGUOUS_MIN_TILES &&
         tiles * k >= r::WIDE_K_CONTIGUOUS_MIN_TILES_TIMES_K && m >= r::WIDE_K_CONTIGUOUS_MIN_ROWS && n >= r::WIDE_K_CONTIGUOUS_MIN_ROWS)
+        return true;
+    if (symmetric && !products &&
+        (k_contiguous ? k >= r::WIDE_SYMMETRIC_K_CONTIGUOUS_MIN_K && tiles >= r::WIDE_SYMMETRIC_K_CONTIGUOUS_MIN_TILES &&
+                            tiles * k >= r::WIDE_SYMMETRIC_K_CONTIGUOUS_MIN_TILES_TIMES_K
+                      : tiles >= r::WIDE_SYMMETRIC_MIN_TILES && tiles * k >= r::WIDE_SYMMETRIC_MIN_TILES_TIMES_K))
         return true;
     const bool little_padding = 100 * m * n >= (100 - r::WIDE_MAX_PADDING_PERCENT) * (tiles_m * kmc::GW_TILE) * (tiles_n * kmc::GW_TILE);
     if (products && k >= r::DOT_LONG_K && tiles * k >= r::DOT_LONG_MIN_TILES_TIMES_K &&
@@ -144,7 +155,7 @@ bool wide_layout(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &a
                                          : static_cast<int64_t>(layout->tiles_m) * layout->tiles_n;
     const bool k_contiguous = p->a_majorness == KMC_ROW_MAJOR && p->b_majorness == KMC_ROW_MAJOR;
     const bool asked_for = (p->flags & KMC_FLAG_GRAM_WORKSPACE_ANY_SIZE) && args.k >= 1;
-    if (!asked_for && !wide_pays(args.m, args.n, layout->tiles_m, layout->tiles_n, tiles * args.l, args.k, products, k_contiguous, args.l > 1)) return false;
+    if (!asked_for && !wide_pays(args.m, args.n, layout->tiles_m, layout->tiles_n, tiles * args.l, args.k, products, k_contiguous, args.l > 1, args.symmetric)) return false;
     // an operand that is the same for every batch entry is split once, unless the centre differs
     // (products have no centre: the caller's parameter block carries none into `args`)
     const bool one_centre = products || !args.centre || args.centre_bs == 0;

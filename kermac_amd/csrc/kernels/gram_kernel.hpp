@@ -271,6 +271,8 @@ __global__ __launch_bounds__(BK_THREADS, GRAM_WAVES) void gram_l2_kernel(const B
     row_norms<LOAD_B>(load_b, square_b, lds_b, lds_norm_b, tid);
     __syncthreads();
 
+    // off: a set against itself gives the bits that the set against a copy of itself gives
+    constexpr bool GRAM_SAME_POINTS = false;
 #include "gram_epilogue.inc"
 }
 

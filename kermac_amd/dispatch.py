@@ -52,14 +52,17 @@ _ROWS = (
      "tiles · K ≥ {WIDE_MIN_TILES_TIMES_K} or ≥ {WIDE_TILES_FOR_ANY_K} tiles, per batch entry 2 · tiles_m · tiles_n ≥ "
      "{WIDE_MIN_TILES_PER_SIDE_X2} · (tiles_m + tiles_n), ≤ {WIDE_MAX_PADDING_PERCENT} % of the tiles' area padding; with k contiguous in both "
      "operands instead: K ≥ {WIDE_K_CONTIGUOUS_MIN_K}, ≥ {WIDE_K_CONTIGUOUS_MIN_TILES} tiles, tiles · K ≥ {WIDE_K_CONTIGUOUS_MIN_TILES_TIMES_K}, M and N ≥ "
-     "{WIDE_K_CONTIGUOUS_MIN_ROWS}",
-     "`gram_row_stats_pair` + `gram_f16_split_pair` (both operands per launch), `gram_probe_operands`, `gram_f16_wide` (fp16 pieces, 256 × 256 tiles), repair launch "
+     "{WIDE_K_CONTIGUOUS_MIN_ROWS}; or a set against itself of ≥ {WIDE_SYMMETRIC_MIN_TILES} tiles (of its triangle), tiles · K ≥ "
+     "{WIDE_SYMMETRIC_MIN_TILES_TIMES_K}, with k contiguous K ≥ {WIDE_SYMMETRIC_K_CONTIGUOUS_MIN_K}, ≥ {WIDE_SYMMETRIC_K_CONTIGUOUS_MIN_TILES} tiles, "
+     "tiles · K ≥ {WIDE_SYMMETRIC_K_CONTIGUOUS_MIN_TILES_TIMES_K}",
+     "`gram_rows_once` (k contiguous and K ≤ 1024, the sample in the same launch) or `gram_row_stats_pair` + `gram_f16_split_pair` + `gram_probe_operands`, "
+     "`gram_f16_wide` (fp16 pieces, tiles of 256 × 128 from {WIDE_LARGE_TILE_MIN_TILES} on, else 128 × 128), repair launch "
      "of the direct kernel"),
     ("",
      "K ≥ {build_a_kernel.AUTO_ONE_STEP_MIN_K}, trust < 1, "
      "and not (a call the direct path would cut over k on fewer than {build_a_kernel.AUTO_UNCUT_MIN_TILES_K_CONTIGUOUS} tiles of 128 × 128, "
      "{build_a_kernel.AUTO_UNCUT_MIN_TILES} with the rows contiguous)",
-     "one-step matrix-core kernel: `gram_l2_kernel` (fp32 matrix instruction) with k contiguous in an operand and K ≥ {build_a_kernel.AUTO_FP32_MIN_K} on "
+     "one-step matrix-core kernel: `gram_l2_kernel` (fp32 matrix instruction) for two different sets with k contiguous in an operand and K ≥ {build_a_kernel.AUTO_FP32_MIN_K} on "
      "{build_a_kernel.AUTO_FP32_MIN_TILES} … {build_a_kernel.AUTO_FP32_MAX_TILES} tiles over the batch and ≥ {build_a_kernel.AUTO_FP32_MIN_TILES_PER_ENTRY} per entry, "
      "or one dimension ≤ 128 with ≥ {build_a_kernel.AUTO_FP32_MIN_TILES} "
      "tiles; else `gram_bf16_l2_kernel` (three bf16 pieces); from M · N · K · L ≥ {build_a_kernel.L2_SAMPLE_MIN_TERMS} on `gram_probe_operands` in front "

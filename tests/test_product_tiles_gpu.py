@@ -55,6 +55,32 @@ def test_a_set_against_itself(device, L, M, K):
     assert (torch.diagonal(got, dim1=1, dim2=2) == 0).all()
 
 
+@pytest.mark.parametrize("L,M,K", [(1, 1, 130), (1, 129, 128), (2, 257, 140), (1, 385, 200), (3, 128, 33)])
+@pytest.mark.parametrize("panel", [False, True])
+def test_a_set_against_itself_in_one_step(device, monkeypatch, L, M, K, panel):
+    """The split kernel without a workspace: zero on the diagonal, symmetric bit for bit, also where the tile is recomputed
+    (a pair of near-duplicates, a row that is not a number), and a set against a run of its own rows."""
+    monkeypatch.setenv("KERMAC_AMD_L2_WORKSPACE", "0")
+    gen = torch.Generator(device=device).manual_seed(M + K)
+    a = torch.randn(L, M, K, device=device, generator=gen)
+    if M > 200:
+        a[0, 150] = a[0, 3] + 1e-3
+        a[-1, 200, 5] = float("nan")
+    if panel:
+        a = a.transpose(1, 2).contiguous().transpose(1, 2)
+    with kermac.l2_mode("gram_bf16", min_k=1):
+        got = kermac.cdist(a, a, p=2.0)
+        run = kermac.cdist(a[:, M // 3:], a, p=2.0)
+    truth = _truth(a, a, list(range(L)))
+    finite = torch.isfinite(truth)
+    assert torch.equal(torch.isfinite(got), finite)
+    assert ((got.double() - truth).abs() <= 1e-5 * truth)[finite].all()
+    clean = torch.where(finite, got, torch.zeros_like(got))
+    assert torch.equal(clean, clean.transpose(1, 2)) and (torch.diagonal(clean, dim1=1, dim2=2) == 0).all()
+    part = truth[:, M // 3:]
+    assert ((run.double() - part).abs() <= 1e-5 * part)[torch.isfinite(part)].all()
+
+
 @pytest.mark.parametrize("K", [3, 255, 256, 257, 260, 511, 512, 513, 1000, 1023, 1024, 1025])
 @pytest.mark.parametrize("form", ["rows", "misaligned", "a_panel", "b_panel", "offset"])
 def test_rows_of_any_length(device, K, form):
