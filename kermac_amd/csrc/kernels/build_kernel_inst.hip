@@ -8,6 +8,7 @@
 #include "launch.hpp"
 #include "build_kernel.hpp"
 #include "build_kernel_scalar_b.hpp"
+#include "build_kernel_small.hpp"
 #include "../host/dispatch_rules.hpp"
 
 #ifndef KMC_INNER_OP
@@ -99,8 +100,27 @@ hipError_t launch_scalar_b_if_the_sample_leaves(int load_a, int load_b, const km
 }
 #endif
 
+// Results of few tiles, in tiles of 64 x 64 (build_kernel_small.hpp).  128 x 128 / 64 x 64 tiles, us, p = 1 and p = 1.3 at
+// K = 400: 64 tiles 117 / 55 and 326 / 121; 121 tiles 133 / 58 and 347 / 187; 192 tiles 127 / 72 and 341 / 259; 256 tiles, one
+// for every CU, 127 / 86 and 342 / 334; a set against itself of 16 x 16 tiles 165 / 108 and 439 / 428.  Beyond that a single problem
+// still gains (360 tiles 136 / 124 and 647 / 481) but a batch loses (32 x 500 x 500 146 / 165 and 657 / 636, at K = 64 33 / 39), and
+// so does a set against itself, of which this kernel computes both halves (22 x 22 tiles 167 / 194 and 445 / 802).
+static bool small_applies(const kmc::BuildKernelArgs &args)
+{
+    if (args.repair_only || args.k_total != 0 || args.panels != 0) return false;
+    const int64_t tiles = static_cast<int64_t>(args.tiles_m) * args.tiles_n * args.l;
+    return tiles <= kmc_rules::DIRECT_SMALL_MAX_TILES;
+}
+
 hipError_t KMC_LAUNCHER_NAME(int load_a, int load_b, const kmc::BuildKernelArgs &args, dim3 grid, hipStream_t stream)
 {
+    if (small_applies(args)) {
+        const int across = (args.m + kmc::BKS_TILE - 1) / kmc::BKS_TILE, down = (args.n + kmc::BKS_TILE - 1) / kmc::BKS_TILE;
+        kmc::BuildKernelArgs copy = args;
+        void *kernel_args[] = {&copy, &load_a, &load_b, const_cast<int *>(&down)};
+        return hipLaunchKernel(reinterpret_cast<const void *>(kmc::build_kernel_small<KMC_INNER_OP, KMC_INNER_POW>),
+                               dim3(static_cast<unsigned>(across) * down, args.l), dim3(kmc::BK_THREADS), kernel_args, 0, stream);
+    }
     switch (load_a * 4 + load_b) {
     case 0: return launch_one<0, 0>(args, grid, stream);
     case 1: return launch_one<0, 1>(args, grid, stream);
