@@ -2,7 +2,7 @@
 //
 //   sum_k (b[n,k] - a[m,k])^2  =  |a_m|^2 + |b_n|^2 - 2 * sum_k a[m,k] * b[n,k]
 //
-// on the fp16 matrix instruction (v_mfma_f32_32x32x16_f16, the rate of the bf16 one), from two
+// on the fp16 matrix instruction (v_mfma_f32_16x16x32_f16, the rate of the bf16 one), from two
 // fp16 pieces per fp32 value and three piece products, in three launches with a workspace
 // between them:
 //
