@@ -688,6 +688,9 @@ __global__ __launch_bounds__(Tile::THREADS, Tile::MIN_WAVES) void gram_f16_wide(
                   ring, lane, wave, wave_m, wave_n);
         wide_walk<Tile>(acc, walk, (args.slices + 1) / 2);
     }
+    // The last barrier of the walk stands in front of its last reads; behind this one every wave has its operands, and the
+    // ring is free for the staging of the results (the gradient's epilogue stages nothing).
+    if constexpr (EPILOGUE != GW_EPILOGUE_GRADIENT_L2) __syncthreads();
 
     // Everything behind the walk is derived from a copy of the lane id and of the argument block's address that the
     // compiler cannot see through: computed before the walk and kept through it, it would push the walk's operands
@@ -782,8 +785,8 @@ __global__ __launch_bounds__(Tile::THREADS, Tile::MIN_WAVES) void gram_f16_wide(
     // A point against itself (BuildKernelArgs::same_points) is at distance zero, exactly, if its norm is a number: without
     // that the parts on the diagonal are all distrusted, and the repair launch walks each of them on one CU (10000 points of
     // K = 784 against themselves: 254 of 590 us; 338 with it).
-    // The stores go through this wave's share of the ring (idle: every copy has arrived, and no wave reads it any
-    // more), so that an instruction writes runs of WAVE_M floats of a column.
+    // The stores go through this wave's share of the ring (free since the barrier behind the walk), so that an instruction
+    // writes runs of WAVE_M floats of a column.
     float least_margin = 0.0f;
     const int self_diagonal = n0 + wave_n + kernel->same_shift - m0 - wave_m;
     const bool same_points = kernel->same_points != 0 && self_diagonal < Tile::WAVE_M && self_diagonal > -Tile::WAVE_N;
