@@ -540,6 +540,15 @@ __device__ __forceinline__ void wide_wait_copies()
     __builtin_amdgcn_s_waitcnt(0x0F70 | (COUNT & 15) | ((COUNT >> 4) << 14));     // vmcnt(COUNT), nothing else
 }
 
+// Between writes and reads of LDS through which the lanes of a wave hand values to each other: the hardware keeps a wave's LDS
+// instructions in order, the compiler by itself only those of one lane.  No instruction comes of it.
+__device__ __forceinline__ void wide_lanes_exchange()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // The matrix instructions are written out: left to itself the compiler gives their results other registers than their
 // sums came from, which does not fit beside the operands.  Two products into the same sums are at least 16 matrix
 // instructions apart, and wide_walk ends with the wait states that vector instructions need before they read the sums.
@@ -851,8 +860,10 @@ __global__ __launch_bounds__(Tile::THREADS, Tile::MIN_WAVES) void gram_f16_wide(
                 }
             }
             if (above) continue;
+            wide_lanes_exchange();
 #pragma unroll
             for (int mt = 0; mt < MT; mt++) *reinterpret_cast<gram_float4 *>(stage + i * PITCH + 16 * mt + 4 * q) = acc[mt][nt];
+            wide_lanes_exchange();
 #pragma unroll
             for (int pass = 0; pass < 16 / PER_PASS; pass++) {
                 const int column = pass * PER_PASS + lane_after / LANES;
@@ -891,12 +902,14 @@ __global__ __launch_bounds__(Tile::THREADS, Tile::MIN_WAVES) void gram_f16_wide(
         const bool whole = c_vec && column + 3 < columns;
 #pragma unroll
         for (int pair = 0; pair < MT / 2; pair++) {
+            wide_lanes_exchange();
 #pragma unroll
             for (int mt = 0; mt < 2; mt++)
 #pragma unroll
                 for (int nt = 0; nt < NT; nt++)
 #pragma unroll
                     for (int v = 0; v < 4; v++) stage[(16 * mt + 4 * q + v) * PITCH + 16 * nt + i] = acc[2 * pair + mt][nt][v];
+            wide_lanes_exchange();
 #pragma unroll
             for (int pass = 0; pass < 32 / PER_PASS; pass++) {
                 const int row = pass * PER_PASS + lane_after / LANES;

@@ -115,3 +115,22 @@ def test_no_wave_stages_results_over_operands_that_another_has_yet_to_read(listi
         assert reads
         without = reachable(reads, code.follow, stop=lambda at: code.ops[at] == "s_barrier") & staged
         assert not without, f"{name}: {[lines[at][1] for at in sorted(without)][:4]}"
+
+
+def test_lanes_of_a_wave_exchange_staged_results_in_order(listings):
+    """Lanes of a wave hand results to each other through LDS.  The compiler has to respect the order within one lane only, so a
+    barrier of the wave keeps the reads behind the other lanes' writes, and the next writes behind those reads."""
+    for name, lines in listings.items():
+        code = Listing(lines)
+        barrier = lambda at: code.ops[at] == "s_barrier"
+        ordered = lambda at: code.ops[at] in ("s_barrier", "wave_barrier")
+        reads = {at for at in code.all("ds_read", "ds_load") if at not in code.before_a_product}
+        # what is written and read with no barrier of the workgroup in between is exchanged within a wave
+        exchanged = {at for at in code.all("ds_write", "ds_store") if at not in code.before_a_product
+                     and reachable([at], code.follow, stop=barrier) & reads}
+        assert bool(exchanged) == ("ELi1EEEv" not in name), name        # the gradient's epilogue (1) stages nothing
+        early = reachable(exchanged, code.follow, stop=ordered) & reads
+        assert not early, name
+        behind = reads & reachable(exchanged, code.follow, stop=barrier)
+        overwritten = reachable(behind, code.follow, stop=ordered) & exchanged
+        assert not overwritten, name
