@@ -552,6 +552,9 @@ __device__ __forceinline__ void wide_lanes_exchange()
 // The matrix instructions are written out: left to itself the compiler gives their results other registers than their
 // sums came from, which does not fit beside the operands.  Two products into the same sums are at least 16 matrix
 // instructions apart, and wide_walk ends with the wait states that vector instructions need before they read the sums.
+// The compiler, which keeps such distances for instructions it knows, does not see these: nothing else may read or move a sum between
+// the first product and those wait states, which holds as long as the sums stay where they are (the test of the kernel's listing
+// looks at every instruction in between).
 template <int MT, int NT, int FIRST, int LAST>
 __device__ __forceinline__ void wide_multiply(gram_float4 (&acc)[MT][NT], const gram_half8 (&fa)[MT], const gram_half8 (&fb)[NT])
 {

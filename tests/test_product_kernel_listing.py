@@ -134,3 +134,28 @@ def test_lanes_of_a_wave_exchange_staged_results_in_order(listings):
         behind = reads & reachable(exchanged, code.follow, stop=barrier)
         overwritten = reachable(behind, code.follow, stop=ordered) & exchanged
         assert not overwritten, name
+
+
+def registers(text):
+    found = set()
+    for first, last in re.findall(r"\bv\[(\d+):(\d+)\]", text):
+        found |= set(range(int(first), int(last) + 1))
+    return found | {int(at) for at in re.findall(r"\bv(\d+)\b", text)}
+
+
+def test_nothing_but_the_products_touches_the_sums_in_the_walk(listings):
+    """The matrix instructions are inline assembly, so the compiler keeps no distance between one of them and an instruction that reads or
+    moves its sums.  Inside the walk there must be no such instruction; behind it only past the wait states that end it."""
+    for name, lines in listings.items():
+        code = Listing(lines)
+        products = set(code.products)
+        sums = set().union(*(registers(lines[at][1].split(",")[0]) for at in products))
+        for at in products:
+            to, _, _, added = (registers(x) for x in re.findall(r"v\[\d+:\d+\]", lines[at][1]))
+            assert to == added, "the sums stay in their registers"
+        # the wait states: at least 16 behind the last product before anything else reads or writes a sum
+        waited = lambda at: lines[at][1] == "s_nop 15"
+        close = reachable(products, code.follow, stop=waited) - products
+        for at in sorted(close):
+            assert not registers(lines[at][1]) & sums, f"{name}: {lines[at][1]}"
+        assert not code.all("scratch_", "buffer_store", "buffer_load"), f"{name} spills"
