@@ -51,14 +51,16 @@ static bool scalar_b_applies(const kmc::BuildKernelArgs &args, int64_t *grid_wid
            args.k >= kmc_rules::DIRECT_SCALAR_B_MIN_K;
 }
 
+constexpr bool HAS_SCALAR_B = KMC_INNER_OP == kmc::OP_DIFF &&
+                              (KMC_INNER_POW == kmc::POW_ABS || KMC_INNER_POW == kmc::POW_SQUARE || KMC_INNER_POW == kmc::POW_ABS_CUBE ||
+                               KMC_INNER_POW == kmc::POW_ABS_FOURTH);
+
 template <int LOAD_A, int LOAD_B>
 static hipError_t launch_one(const kmc::BuildKernelArgs &args, dim3 grid, hipStream_t stream)
 {
     // absolute differences, their squares, cubes and fourth powers, of large problems whose rows are contiguous on both
     // sides: b in scalar registers
-    if constexpr (LOAD_A == kmc::LOAD_COL_VEC && LOAD_B == kmc::LOAD_COL_VEC && KMC_INNER_OP == kmc::OP_DIFF &&
-                  (KMC_INNER_POW == kmc::POW_ABS || KMC_INNER_POW == kmc::POW_SQUARE || KMC_INNER_POW == kmc::POW_ABS_CUBE ||
-                   KMC_INNER_POW == kmc::POW_ABS_FOURTH)) {
+    if constexpr (LOAD_A == kmc::LOAD_COL_VEC && LOAD_B == kmc::LOAD_COL_VEC && HAS_SCALAR_B) {
         int64_t grid_width = 0;
         if (scalar_b_applies(args, &grid_width)) {
             kmc::BuildKernelArgs copy = args;
@@ -105,16 +107,21 @@ hipError_t launch_scalar_b_if_the_sample_leaves(int load_a, int load_b, const km
 // for every CU, 127 / 86 and 342 / 334; a set against itself of 16 x 16 tiles 165 / 108 and 439 / 428.  Beyond that a single problem
 // still gains (360 tiles 136 / 124 and 647 / 481) but a batch loses (32 x 500 x 500 146 / 165 and 657 / 636, at K = 64 33 / 39), and
 // so does a set against itself, of which this kernel computes both halves (22 x 22 tiles 167 / 194 and 445 / 802).
-static bool small_applies(const kmc::BuildKernelArgs &args)
+// KERMAC_AMD_DIRECT_SMALL_MAX_TILES=n replaces the limit (read on every call, so that a test can choose the kernel).
+static bool small_applies(int load_a, int load_b, const kmc::BuildKernelArgs &args)
 {
     if (args.repair_only || args.k_total != 0 || args.panels != 0) return false;
+    // never so by the size rules of the two kernels, but a test may send results of few tiles to the other one
+    int64_t grid_width = 0;
+    if (HAS_SCALAR_B && load_a == kmc::LOAD_COL_VEC && load_b == kmc::LOAD_COL_VEC && scalar_b_applies(args, &grid_width)) return false;
     const int64_t tiles = static_cast<int64_t>(args.tiles_m) * args.tiles_n * args.l;
-    return tiles <= kmc_rules::DIRECT_SMALL_MAX_TILES;
+    const char *limit = std::getenv("KERMAC_AMD_DIRECT_SMALL_MAX_TILES");
+    return tiles <= (limit ? std::atoi(limit) : kmc_rules::DIRECT_SMALL_MAX_TILES);
 }
 
 hipError_t KMC_LAUNCHER_NAME(int load_a, int load_b, const kmc::BuildKernelArgs &args, dim3 grid, hipStream_t stream)
 {
-    if (small_applies(args)) {
+    if (small_applies(load_a, load_b, args)) {
         const int across = (args.m + kmc::BKS_TILE - 1) / kmc::BKS_TILE, down = (args.n + kmc::BKS_TILE - 1) / kmc::BKS_TILE;
         kmc::BuildKernelArgs copy = args;
         void *kernel_args[] = {&copy, &load_a, &load_b, const_cast<int *>(&down)};

@@ -18,3 +18,11 @@ def device():
     if not torch.cuda.is_available():
         pytest.skip("no GPU")
     return torch.device("cuda:0")
+
+
+@pytest.fixture(params=["64x64", "128x128"])
+def direct_tile(request, monkeypatch):
+    """Both tiles of the direct kernel for the small results of a test: 64 x 64 by the library's rule, and the 128 x 128 of larger results."""
+    if request.param == "128x128":
+        monkeypatch.setenv("KERMAC_AMD_DIRECT_SMALL_MAX_TILES", "0")
+    return request.param

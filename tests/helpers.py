@@ -35,3 +35,13 @@ def l1_distances_float64(a: torch.Tensor, b: torch.Tensor, block: int = 16) -> t
     (torch.cdist with p = 1 in float64 has returned wrong rows on the GPU for some sizes)."""
     a, b = a.double(), b.double()
     return torch.cat([(a[i:i + block, None, :] - b[None]).abs().sum(-1) for i in range(0, a.size(0), block)])
+
+
+def kernels_of(call):
+    """The names of the kernels that a call launches, in their order."""
+    from torch.profiler import ProfilerActivity, profile
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA], acc_events=True) as prof:
+        call()
+        torch.cuda.synchronize()
+    return [event.name for event in prof.events() if event.device_type == torch.autograd.DeviceType.CUDA]

@@ -16,7 +16,7 @@ import kermac_amd as kermac
 from oracle import oracle
 from tests.helpers import assert_close_to_truth, make_operand
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("direct_tile")]
 
 GOLDEN = np.load(Path(__file__).resolve().parent / "golden" / "hot_path_vectors.npz")
 RTOL = {1.0: 1e-5, 2.0: 1e-5}

@@ -16,7 +16,7 @@ import kermac_amd as kermac
 from oracle import oracle
 from tests.helpers import assert_close_to_truth
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("direct_tile")]
 
 
 @pytest.fixture(autouse=True, params=["as launched", "workspace routes"])

@@ -10,7 +10,7 @@ import torch
 
 import kermac_amd as kermac
 from oracle import oracle
-from tests.helpers import assert_close_to_truth, l1_distances_float64
+from tests.helpers import assert_close_to_truth, kernels_of, l1_distances_float64
 
 pytestmark = pytest.mark.gpu
 
@@ -178,3 +178,21 @@ def test_a_large_problem_takes_the_kernel_by_itself(device):
                 x, y = a[rows], b[columns]
                 truth = l1_distances_float64(x, y) if p == 1.0 else torch.cdist(x.double(), y.double(), p=2.0, compute_mode="donot_use_mm_for_euclid_dist")
                 assert_close_to_truth(out[rows][:, columns], truth, rtol=1e-5, what=f"p={p} {M}x{N}")
+
+
+def test_the_switches_choose_the_kernel(device, monkeypatch):
+    """The comparisons above are between different kernels: results of few tiles, by the library's rule and sent to the others."""
+    a, b = panels(320, 80, 32, device, 1)          # multiples of 16 on both sides: the result may be computed transposed
+    own, _ = panels(1024, 16, 64, device, 2)
+    deep_a, deep_b = panels(320, 80, 256, device, 3)
+    calls = [lambda: kermac.cdist(a, b, p=1.0), lambda: kermac.cdist(own, own, p=1.0), lambda: kermac.cdist(deep_a, deep_b, p=1.0)]
+    ran = lambda: [[name for name in kernels_of(call) if "build_kernel" in name] for call in calls]
+    only = lambda kernel: [[kernel + "<" in name for name in names] for names in ran()] == [[True]] * 3
+    assert only("build_kernel_small")
+    monkeypatch.setenv("KERMAC_AMD_SCALAR_B_MIN_TILES", "1")
+    assert only("build_kernel_scalar_b")
+    monkeypatch.setenv("KERMAC_AMD_SCALAR_B_MIN_TILES", "1000000")
+    assert only("build_kernel_small")
+    monkeypatch.setenv("KERMAC_AMD_DIRECT_SMALL_MAX_TILES", "0")
+    tile, own_tile, deep = ran()
+    assert "build_kernel<" in tile[0] and "build_kernel<" in own_tile[0] and "build_kernel_four_waves<" in deep[0]

@@ -12,7 +12,7 @@ import kermac_amd as kermac
 from oracle import oracle
 from tests.helpers import assert_close_to_truth
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("direct_tile")]
 
 DESCRIPTORS = {
     "l1": (kermac.kernel_descriptor_l1_norm, {}, ("DIFF", "ABS", "NOOP", "NONE"), {}),
