@@ -52,8 +52,8 @@ HOST_SOURCES = [
 
 # Device translation units without per-variant defines.
 EXTRA_DEVICE_SOURCES = ["kernels/norm_gradient_inst.hip", "kernels/gram_kernel_inst.hip",
-                        "kernels/gram_coefficients_inst.hip", "kernels/gram_bf16_kernel_inst.hip",
-                        "kernels/finish_partials.hip", "kernels/cut_static_scratch.hip", "kernels/sample_mean.hip", "kernels/gram_probe.hip",
+                        "kernels/gram_coefficients_inst.hip", "kernels/finish_partials.hip",
+                        "kernels/cut_static_scratch.hip", "kernels/sample_mean.hip", "kernels/gram_probe.hip",
                         "kernels/gram_f16_wide_inst.hip", "kernels/norm_gradient_f16_inst.hip",
                         "kernels/matrix_times_coefficients.hip", "kernels/l1_fixed_inst.hip", "kernels/panel_copy.hip"]
 
@@ -77,6 +77,9 @@ def _jobs():
     for op, pw in AOT_COEFFICIENT_VARIANTS:
         jobs.append((inst, OBJ_DIR / f"kernel_coefficients_inst_{op}_{pw}.o",
                      [f"-DKMC_INNER_OP={op}", f"-DKMC_INNER_POW={pw}"]))
+    inst = CSRC / "kernels" / "gram_bf16_kernel_inst.hip"
+    for same_points in (0, 1):
+        jobs.append((inst, OBJ_DIR / f"gram_bf16_kernel_inst_{same_points}.o", [f"-DKMC_SAME_POINTS={same_points}"]))
     for rel in EXTRA_DEVICE_SOURCES:
         src = CSRC / rel
         jobs.append((src, OBJ_DIR / (src.stem + ".o"), []))

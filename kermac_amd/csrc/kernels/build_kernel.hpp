@@ -47,7 +47,7 @@ struct BuildKernelArgs {
     int repair_only;     // recompute only the tiles that carry BK_REPAIR_MARKER (see gram_kernel.hpp)
     int symmetric;       // A and B are the same panel and the result is symmetric: only tiles with
                          // tile_m >= tile_n are computed, each is also stored mirrored
-    // gram_f16_wide.hpp: with same_points, row m of a and row n of b are the same row in memory
+    // gram_f16_wide.hpp and gram_bf16_kernel.hpp: with same_points, row m of a and row n of b are the same row in memory
     // where m == n + same_shift (a set against itself or against a run of its own rows): their distance is zero, which
     // |a|^2 + |b|^2 - 2 a.b cannot tell.
     int same_points, same_shift;

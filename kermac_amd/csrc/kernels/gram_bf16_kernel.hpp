@@ -292,7 +292,12 @@ __device__ __forceinline__ void gram_bf16_walk(
 // budget for two waves per SIMD: within the budget for three the compiler spills 180.
 // CENTRED: args.centre is subtracted from both operands while they are staged (a kernel of its
 // own: a run-time switch inside the walk breaks the interleaving of matrix instructions and split).
-template <int LOAD_A, int LOAD_B, bool RAGGED_K = false, bool CENTRED = false>
+// SAME_POINTS: rows of one set on both sides (BuildKernelArgs::same_points), whose equal points the epilogue looks for.  A kernel of
+// its own as well: two different sets with the comparison and without, us: rows contiguous 4096 x 4096 x 128 70.1 / 68.0, 3000 x 3000 x 256
+// 69.0 / 65.8, 1400 x 300 x 300 x 128 667 / 620; k contiguous 16 x 500 x 500 x 512 114.4 / 106.9.
+// (Looking in passes of their own, in front of the walk over the elements and behind it, only in tiles that meet the diagonal, cost
+// registers: 1400 x 300 x 300 x 128, k contiguous, 1270 against 844.)
+template <int LOAD_A, int LOAD_B, bool RAGGED_K = false, bool CENTRED = false, bool SAME_POINTS = false>
 __global__ __launch_bounds__(BK_THREADS, RAGGED_K ? 2 : GB_WAVES) void gram_bf16_l2_kernel(const BuildKernelArgs args)
 {
     __shared__ gram_chunk lds_a[2 * GB_PANEL_CHUNKS];
@@ -368,7 +373,7 @@ __global__ __launch_bounds__(BK_THREADS, RAGGED_K ? 2 : GB_WAVES) void gram_bf16
     }
     __syncthreads();
 
-    constexpr bool GRAM_SAME_POINTS = true;
+    constexpr bool GRAM_SAME_POINTS = SAME_POINTS;
 #include "gram_epilogue.inc"
 }
 

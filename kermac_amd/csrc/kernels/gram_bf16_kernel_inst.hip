@@ -1,5 +1,7 @@
 // Ahead-of-time instantiations of the split-bf16 matrix-core L2 kernel for all 16
-// (A loader, B loader) pairs, plus the ragged-K variants of the pairs with 128-bit row-major loads.
+// (A loader, B loader) pairs, plus the ragged-K variants of the pairs with 128-bit row-major loads.  Compiled twice: with
+// KMC_SAME_POINTS=1 the variants that look for equal points (rows of one set on both sides), which have the same layout on both sides,
+// though not always the same alignment.
 #include <hip/hip_runtime.h>
 
 #include "launch.hpp"
@@ -7,24 +9,41 @@
 
 namespace kmc_host {
 
+#ifndef KMC_SAME_POINTS
+#error "compile with -DKMC_SAME_POINTS=0 and -DKMC_SAME_POINTS=1"
+#endif
+
 template <int LOAD_A, int LOAD_B>
 static hipError_t launch_one(const kmc::BuildKernelArgs &args, dim3 grid, hipStream_t stream)
 {
-    constexpr bool has_ragged_variant = LOAD_A == kmc::LOAD_ROW_VEC || LOAD_B == kmc::LOAD_ROW_VEC;
-    hipError_t status;
-    const bool ragged = has_ragged_variant && args.k % kmc::BK_TILE_K != 0;
-    if (args.centre) {
-        status = ragged ? launch(kmc::gram_bf16_l2_kernel<LOAD_A, LOAD_B, has_ragged_variant, true>, grid, dim3(kmc::BK_THREADS), stream, args)
-                        : launch(kmc::gram_bf16_l2_kernel<LOAD_A, LOAD_B, false, true>, grid, dim3(kmc::BK_THREADS), stream, args);
+    constexpr bool same_points = KMC_SAME_POINTS != 0;
+    constexpr bool a_rows = LOAD_A == kmc::LOAD_ROW_VEC || LOAD_A == kmc::LOAD_ROW_SCALAR;
+    constexpr bool b_rows = LOAD_B == kmc::LOAD_ROW_VEC || LOAD_B == kmc::LOAD_ROW_SCALAR;
+    if constexpr (same_points && a_rows != b_rows) {
+        return hipErrorInvalidValue;
     } else {
-        status = ragged ? launch(kmc::gram_bf16_l2_kernel<LOAD_A, LOAD_B, has_ragged_variant>, grid, dim3(kmc::BK_THREADS), stream, args)
-                        : launch(kmc::gram_bf16_l2_kernel<LOAD_A, LOAD_B>, grid, dim3(kmc::BK_THREADS), stream, args);
+        constexpr bool has_ragged_variant = LOAD_A == kmc::LOAD_ROW_VEC || LOAD_B == kmc::LOAD_ROW_VEC;
+        const bool ragged = has_ragged_variant && args.k % kmc::BK_TILE_K != 0;
+        if (args.centre)
+            return ragged ? launch(kmc::gram_bf16_l2_kernel<LOAD_A, LOAD_B, has_ragged_variant, true, same_points>, grid, dim3(kmc::BK_THREADS), stream, args)
+                          : launch(kmc::gram_bf16_l2_kernel<LOAD_A, LOAD_B, false, true, same_points>, grid, dim3(kmc::BK_THREADS), stream, args);
+        return ragged ? launch(kmc::gram_bf16_l2_kernel<LOAD_A, LOAD_B, has_ragged_variant, false, same_points>, grid, dim3(kmc::BK_THREADS), stream, args)
+                      : launch(kmc::gram_bf16_l2_kernel<LOAD_A, LOAD_B, false, false, same_points>, grid, dim3(kmc::BK_THREADS), stream, args);
     }
-    return status;
 }
 
+hipError_t launch_gram_bf16_l2_same_points(int load_a, int load_b, const kmc::BuildKernelArgs &args, dim3 grid, hipStream_t stream);
+
+#if KMC_SAME_POINTS
+hipError_t launch_gram_bf16_l2_same_points(int load_a, int load_b, const kmc::BuildKernelArgs &args, dim3 grid, hipStream_t stream)
+{
+#else
 hipError_t launch_gram_bf16_l2(int load_a, int load_b, const kmc::BuildKernelArgs &args, dim3 grid, hipStream_t stream)
 {
+    // A result of one row of tiles is left to the repair launch all the same: the host takes no such result for a symmetric one, and only
+    // the direct kernel gives both halves of it the same bits.
+    if (args.same_points && args.tiles_m > 1) return launch_gram_bf16_l2_same_points(load_a, load_b, args, grid, stream);
+#endif
     switch (load_a * 4 + load_b) {
     case 0: return launch_one<0, 0>(args, grid, stream);
     case 1: return launch_one<0, 1>(args, grid, stream);

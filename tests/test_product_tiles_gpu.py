@@ -4,6 +4,7 @@ import pytest
 import torch
 
 import kermac_amd as kermac
+from tests.helpers import kernels_of
 
 pytestmark = pytest.mark.gpu
 
@@ -115,3 +116,24 @@ def test_rows_that_are_not_numbers(device):
     assert torch.equal(torch.isnan(got), torch.isnan(truth)) and torch.equal(torch.isinf(got), torch.isinf(truth))
     finite = torch.isfinite(truth)
     assert ((got.double() - truth).abs() <= 1e-5 * truth)[finite].all()
+
+
+@pytest.mark.parametrize("panel", [False, True])
+def test_only_a_set_against_itself_looks_for_equal_points(device, panel):
+    """The one-step split kernel has a variant for it (its last template argument), whose comparisons cost any other call up to a tenth."""
+    gen = torch.Generator(device=device).manual_seed(5)
+    a, b = torch.randn(300, 256, device=device, generator=gen), torch.randn(260, 260, device=device, generator=gen)[:, :256]
+    if panel:
+        a, b = (x.t().contiguous().t() for x in (a, b))
+
+    def variants(x, y):
+        with kermac.l2_mode("gram_bf16", min_k=1):
+            return [name.split("gram_bf16_l2_kernel<")[1].split(">")[0].split(",")[-1].strip()
+                    for name in kernels_of(lambda: kermac.cdist(x, y, p=2.0)) if "gram_bf16_l2_kernel<" in name]
+
+    with pytest.MonkeyPatch.context() as patch:
+        patch.setenv("KERMAC_AMD_L2_WORKSPACE", "0")
+        assert variants(a, b) == ["false"]
+        assert variants(a, a) == ["true"]
+        assert variants(a[30:], a) == ["true"] and variants(a, a[30:]) == ["true"]
+        assert variants(a[:100], a[:100]) == ["false"]        # one tile is left to the repair launch
