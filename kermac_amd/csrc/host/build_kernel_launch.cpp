@@ -95,14 +95,14 @@ int prepare(const kmc_build_kernel_params *p, bool need_c, kmc::BuildKernelArgs 
     args->symmetric = need_c && !(p->flags & KMC_FLAG_NO_SYMMETRY) && exchangeable && p->a == p->b && p->m == p->n &&
                       p->a_ld == p->b_ld && p->a_bs == p->b_bs && p->a_majorness == p->b_majorness &&
                       p->regularization_offset_x == p->regularization_offset_y && tiles_m > 1;
-    // Rows of one set on both sides, possibly shifted: the same layout, and b starts a whole number of rows from a.
+    // Rows of one set on both sides, possibly shifted: the same layout, b starts a whole number of rows from a, and some row is on both sides
+    // (parts of one set, or sets that the allocator placed side by side, share none).
     args->same_points = 0;
     args->same_shift = 0;
     if (p->inner_operator == KMC_OP_DIFF && p->a_majorness == p->b_majorness && p->a_ld == p->b_ld && p->a_bs == p->b_bs && p->a && p->b) {
         const int64_t bytes = static_cast<int64_t>(reinterpret_cast<intptr_t>(p->b)) - static_cast<int64_t>(reinterpret_cast<intptr_t>(p->a));
         const int64_t row = 4 * (p->a_majorness == KMC_ROW_MAJOR ? p->a_ld : 1);
-        const int64_t reach = static_cast<int64_t>(p->m) + p->n;
-        if (row > 0 && bytes % row == 0 && bytes / row < reach && bytes / row > -reach) {
+        if (row > 0 && bytes % row == 0 && bytes / row < p->m && bytes / row > -static_cast<int64_t>(p->n)) {
             args->same_points = 1;
             args->same_shift = static_cast<int>(bytes / row);
         }

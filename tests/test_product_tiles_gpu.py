@@ -118,22 +118,37 @@ def test_rows_that_are_not_numbers(device):
     assert ((got.double() - truth).abs() <= 1e-5 * truth)[finite].all()
 
 
+def _variants(x, y):
+    """Whether the one-step split kernel that a call runs is the one that looks for equal points (its last template argument)."""
+    with kermac.l2_mode("gram_bf16", min_k=1):
+        return [name.split("gram_bf16_l2_kernel<")[1].split(">")[0].split(",")[-1].strip()
+                for name in kernels_of(lambda: kermac.cdist(x, y, p=2.0)) if "gram_bf16_l2_kernel<" in name]
+
+
 @pytest.mark.parametrize("panel", [False, True])
-def test_only_a_set_against_itself_looks_for_equal_points(device, panel):
-    """The one-step split kernel has a variant for it (its last template argument), whose comparisons cost any other call up to a tenth."""
+def test_only_a_set_against_itself_looks_for_equal_points(device, monkeypatch, panel):
+    """The comparisons of the variant cost any other call up to a tenth."""
+    monkeypatch.setenv("KERMAC_AMD_L2_WORKSPACE", "0")
     gen = torch.Generator(device=device).manual_seed(5)
     a, b = torch.randn(300, 256, device=device, generator=gen), torch.randn(260, 260, device=device, generator=gen)[:, :256]
     if panel:
         a, b = (x.t().contiguous().t() for x in (a, b))
+    assert _variants(a, b) == ["false"]
+    assert _variants(a, a) == ["true"]
+    assert _variants(a[30:], a) == ["true"] and _variants(a, a[30:]) == ["true"]
+    assert _variants(a[:100], a[:100]) == ["false"]        # one tile is left to the repair launch
 
-    def variants(x, y):
-        with kermac.l2_mode("gram_bf16", min_k=1):
-            return [name.split("gram_bf16_l2_kernel<")[1].split(">")[0].split(",")[-1].strip()
-                    for name in kernels_of(lambda: kermac.cdist(x, y, p=2.0)) if "gram_bf16_l2_kernel<" in name]
 
-    with pytest.MonkeyPatch.context() as patch:
-        patch.setenv("KERMAC_AMD_L2_WORKSPACE", "0")
-        assert variants(a, b) == ["false"]
-        assert variants(a, a) == ["true"]
-        assert variants(a[30:], a) == ["true"] and variants(a, a[30:]) == ["true"]
-        assert variants(a[:100], a[:100]) == ["false"]        # one tile is left to the repair launch
+@pytest.mark.parametrize("panel", [False, True])
+def test_parts_of_one_set_that_share_no_point(device, monkeypatch, panel):
+    monkeypatch.setenv("KERMAC_AMD_L2_WORKSPACE", "0")
+    gen = torch.Generator(device=device).manual_seed(6)
+    x = torch.randn(700, 256, device=device, generator=gen)
+    x = x.t().contiguous().t() if panel else x
+    for first, second in ((x[:300], x[300:]), (x[300:], x[:300]), (x[:150], x[400:])):
+        assert _variants(first, second) == ["false"]
+    assert _variants(x[:301], x[300:]) == ["true"] and _variants(x[300:], x[:301]) == ["true"]      # one point on both sides
+    with kermac.l2_mode("gram_bf16", min_k=1):
+        got = kermac.cdist(x[:301], x[300:], p=2.0)[0]
+    truth = _truth(x[None, :301], x[None, 300:], [0])[0]
+    assert got[300, 0] == 0 and ((got.double() - truth).abs() <= 1e-5 * truth).all()
