@@ -42,31 +42,38 @@ __device__ __forceinline__ i64 sampled_row(const SampleMeanArgs &args, int s)
     return (i64)run * (args.rows - SM_RUN) / (SM_RUNS - 1) + (s - run * SM_RUN);
 }
 
-// k contiguous (row-major panel): a workgroup owns 16 k, 64 groups of 16 lanes share the rows, and a lane has eight rows
-// under way at once (eight sums per lane, added in a fixed order at the end): the panel's rows lie K floats apart, so the
-// time is that of the loads' latency, not of their bytes.  64 k per workgroup and 16 groups left 13 workgroups with 32
-// round trips each at K = 784: 43 us for 4096 rows, 14 for 2000, against 16 and 7 now.
-constexpr int SM_ROW_K = 16;
+// k contiguous (row-major panel): a workgroup owns SPAN k, 1024 / SPAN groups of SPAN lanes share the rows, and a lane has eight
+// rows under way at once (eight sums per lane, added in a fixed order at the end): the panel's rows lie K floats apart, so the
+// time of a single panel is that of the loads' latency, not of their bytes, and shrinks with more groups: SPAN 16 instead of 64 is 64
+// groups instead of 16 and four times as many workgroups (K = 784, 4096 rows: 43 -> 16 us; 2000 rows 14 -> 7).  A batch that
+// fills the chip with workgroups of SPAN 64 is bound by what it loads and adds up, which runs of 64 k do better, and up to 128 rows are
+// one round trip either way.  SPAN 16 / SPAN 64, us, by workgroups of SPAN 64: 32 of them 4.7 / 7.8 for 1000 rows, 14 / 24 for 4096; 64
+// 4.8 / 7.8 and 22 / 27; 96 10.4 / 8.0 and 33 / 27; 128 12 / 8.8 and 41 / 28; 512 40 / 21 and 166 / 98; the sample of 30000 rows, 16
+// runs far apart, 96 34 / 44, 128 42 / 44, 156 48 / 46, 512 170 / 96; 100 rows 3.8 / 3.2 in 16 workgroups, 11 / 4 in 512.
 constexpr int SM_ROW_THREADS = 1024;
-constexpr int SM_ROW_GROUPS = SM_ROW_THREADS / SM_ROW_K;
 constexpr int SM_ROW_UNROLL = 8;
+constexpr int SM_ROW_WIDE_MIN_WORKGROUPS = 96;              // of SPAN 64, all rows averaged
+constexpr int SM_ROW_WIDE_MIN_WORKGROUPS_SAMPLED = 144;     // ... and where they are a sample
+constexpr int SM_ROW_WIDE_MAX_FEW_ROWS = 128;
 
+template <int SPAN>
 __global__ __launch_bounds__(SM_ROW_THREADS) void sample_mean_rows(const SampleMeanArgs args)
 {
-    __shared__ float partial[SM_ROW_GROUPS][SM_ROW_K];
-    __shared__ float partial_squares[SM_ROW_GROUPS][SM_ROW_K];
-    const int kk = threadIdx.x % SM_ROW_K, group = threadIdx.x / SM_ROW_K;
-    const int k = blockIdx.x * SM_ROW_K + kk;
+    constexpr int GROUPS = SM_ROW_THREADS / SPAN;
+    __shared__ float partial[GROUPS][SPAN];
+    __shared__ float partial_squares[GROUPS][SPAN];
+    const int kk = threadIdx.x % SPAN, group = threadIdx.x / SPAN;
+    const int k = blockIdx.x * SPAN + kk;
     const float *x = args.x + blockIdx.y * args.bs;
     float sum[SM_ROW_UNROLL], squares[SM_ROW_UNROLL];
 #pragma unroll
     for (int u = 0; u < SM_ROW_UNROLL; ++u) sum[u] = squares[u] = 0.0f;
     if (k < args.k) {
-        for (int first = group; first < args.samples; first += SM_ROW_UNROLL * SM_ROW_GROUPS) {
+        for (int first = group; first < args.samples; first += SM_ROW_UNROLL * GROUPS) {
             float v[SM_ROW_UNROLL];
 #pragma unroll
             for (int u = 0; u < SM_ROW_UNROLL; ++u) {
-                const int s = first + u * SM_ROW_GROUPS;
+                const int s = first + u * GROUPS;
                 v[u] = s < args.samples ? x[sampled_row(args, s) * args.ld + k] : 0.0f;
             }
 #pragma unroll
@@ -88,7 +95,7 @@ __global__ __launch_bounds__(SM_ROW_THREADS) void sample_mean_rows(const SampleM
     if (group == 0 && k < args.k_padded) {
         float total = 0.0f, total_squares = 0.0f;
 #pragma unroll 16
-        for (int w = 0; w < SM_ROW_GROUPS; ++w) {
+        for (int w = 0; w < GROUPS; ++w) {
             total += partial[w][kk];
             total_squares += partial_squares[w][kk];
         }
@@ -196,8 +203,13 @@ extern "C" int kmc_sample_mean(const float *x, int32_t majorness, int32_t rows, 
     args.mean = mean; args.mean_bs = mean_bs;
     args.samples = rows < kmc::SM_MAX_SAMPLES ? rows : kmc::SM_MAX_SAMPLES;
     hipError_t e;
-    if (majorness == KMC_ROW_MAJOR)
-        e = kmc_host::launch(kmc::sample_mean_rows, dim3(k_padded / kmc::SM_ROW_K, l), dim3(kmc::SM_ROW_THREADS), static_cast<hipStream_t>(stream), args);
+    const int64_t wide_workgroups = static_cast<int64_t>(k_padded / 64) * l;
+    const bool wide = rows <= kmc::SM_ROW_WIDE_MAX_FEW_ROWS ||
+                      wide_workgroups >= (rows > kmc::SM_MAX_SAMPLES ? kmc::SM_ROW_WIDE_MIN_WORKGROUPS_SAMPLED : kmc::SM_ROW_WIDE_MIN_WORKGROUPS);
+    if (majorness == KMC_ROW_MAJOR && wide)
+        e = kmc_host::launch(kmc::sample_mean_rows<64>, dim3(k_padded / 64, l), dim3(kmc::SM_ROW_THREADS), static_cast<hipStream_t>(stream), args);
+    else if (majorness == KMC_ROW_MAJOR)
+        e = kmc_host::launch(kmc::sample_mean_rows<16>, dim3(k_padded / 16, l), dim3(kmc::SM_ROW_THREADS), static_cast<hipStream_t>(stream), args);
     else
         e = kmc_host::launch(kmc::sample_mean_columns, dim3(k_padded / 4, l), dim3(256), static_cast<hipStream_t>(stream), args);
     if (e != hipSuccess) return kmc_host::fail_hip(e, "sample_mean launch");

@@ -12,7 +12,7 @@ import torch
 
 import kermac_amd as kermac
 from oracle import oracle
-from tests.helpers import assert_close_to_truth, make_operand
+from tests.helpers import assert_close_to_truth, kernels_of, make_operand
 
 pytestmark = pytest.mark.gpu
 
@@ -218,6 +218,25 @@ def test_sample_mean_through_the_c_abi(device):
         assert torch.all(mean[:, padded] == expect), f"flag rows={rows} K={K} shift={shift}: {mean[:, padded].tolist()}"
     with pytest.raises(_backend.BackendError, match="mean_bs"):
         _backend.sample_mean(x.data_ptr(), _backend.ROW_MAJOR, rows, K, ld, x.stride(0), 2, mean.data_ptr(), padded, stream)
+
+
+@pytest.mark.parametrize("rows,K,L,span", [(1, 70, 1, 64), (128, 200, 1, 64), (129, 200, 1, 16), (129, 70, 47, 16), (129, 70, 48, 64), (1000, 33, 95, 16),
+                                           (1000, 33, 96, 64), (4096, 65, 48, 64), (4097, 65, 71, 16), (4097, 65, 72, 64)])
+def test_means_of_single_panels_and_of_batches(device, rows, K, L, span):
+    """k contiguous: few workgroups take 16 k each, a batch that fills the chip 64 (the kernel's template argument)."""
+    from kermac_amd import _backend
+    x = torch.randn(L, rows, K, device=device, generator=torch.Generator(device=device).manual_seed(rows + L)) + 3.0
+    padded = -(-K // 64) * 64
+    width = 2 * padded + 64
+    mean = torch.full((L, width), -1.0, device=device)
+    names = kernels_of(lambda: _backend.sample_mean(x.data_ptr(), _backend.ROW_MAJOR, rows, K, K, rows * K, L, mean.data_ptr(), width,
+                                                    torch.cuda.current_stream(device).cuda_stream))
+    assert sum(f"sample_mean_rows<{span}>" in name for name in names) == 1
+    sample = x if rows <= 4096 else torch.cat([x[:, s:s + 256] for s in [(j * (rows - 256)) // 15 for j in range(16)]], dim=1)
+    assert_close_to_truth(mean[:, :K], sample.double().mean(dim=1), rtol=1e-5, what="mean")         # sums of values of order 1
+    assert_close_to_truth(mean[:, padded + 64:padded + 64 + K], sample.double().var(dim=1, unbiased=False), rtol=1e-3, atol=1e-5,
+                          what="variance")        # the difference of two sums of order 10
+    assert torch.all(mean[:, K:padded] == 0.0) and torch.all(mean[:, padded + 64 + K:] == 0.0)
 
 
 def test_a_negligible_centre_is_left_out(device, gram_mode, monkeypatch):
