@@ -292,6 +292,10 @@ hipError_t launch_product_in(kmc::GramWideArgs &wide, hipStream_t stream)
     wide.wide_tiles_n = (wide.kernel.n + Tile::TILE_N - 1) / Tile::TILE_N;
     int padded = (wide.wide_tiles_n + kmc::BK_XCDS - 1) / kmc::BK_XCDS * kmc::BK_XCDS;
     if ((padded - wide.wide_tiles_n) * 8 > wide.wide_tiles_n) padded = wide.wide_tiles_n;
+    // ... nor where a launch that fits the chip at once would no longer, since the padding's idle ids fall to some of the XCDs (2 x 2816 x 2816
+    // of K = 4096, 22 large tiles in n, 66 of them on 64 places: 604 -> 488 us)
+    const int64_t places = 32 * Tile::MIN_WAVES, rows_of_tiles = static_cast<int64_t>(wide.wide_tiles_m) * wide.kernel.l;
+    if (rows_of_tiles * (padded / kmc::BK_XCDS) > places && rows_of_tiles * wide.wide_tiles_n <= places * kmc::BK_XCDS) padded = wide.wide_tiles_n;
     wide.wide_tiles_n_padded = padded;
     const int64_t blocks = (wide.kernel.m + kmc::GW_TILE - 1) / kmc::GW_TILE;
     const int64_t width = SYMMETRIC ? blocks * (blocks + 1) / 2 * (kmc::GW_TILE / Tile::TILE_M) * (kmc::GW_TILE / Tile::TILE_N)
@@ -304,14 +308,31 @@ hipError_t launch_product_in(kmc::GramWideArgs &wide, hipStream_t stream)
 // the L2 for three quarters of the bytes per multiply-add.  Time of a call in the small tiles over the large ones: 32 large
 // tiles 0.94 at K = 128, 0.75 at K = 2048; 288 tiles 0.92, 0.90; 512 tiles 0.99, 1.03; 800 tiles 0.97, 0.96; 1128 tiles
 // 0.89, 0.97; 2048 tiles 0.96, 1.03; 3160 tiles 0.91, 1.00; 8192 tiles 1.02 at K = 128, 1.01 at K = 512.
+//
+// Above one round of small tiles (three on each of 256 CUs) the few of the second round have the chip to themselves; where the large
+// tiles are one round (two per CU) they are taken instead, as long as the second round of small ones is little or the contraction long.
+// Not for a set against itself, whose rounds are of unequal tiles.  Small / large, us, k contiguous: 800 small tiles, 8 x 1280 x 1280 of
+// K = 784 129.4 / 127.5, of K = 4096 644 / 617 (a workgroup of 256 x 256 per CU, the kernel before these, 147 and 570); 840, 28 x 640 x 768 of
+// K = 784 210 / 185, of K = 4096 1072 / 934; 784, 3584 x 3584 of K = 784 100 / 96, of K = 4096 395 / 371; 938, 200 x 60000 of K = 784 194.4 / 197.5,
+// of K = 2048 568 / 561; 1024, 4096 x 4096 of K = 784 103.1 / 103.8, of K = 4096 432 / 421; more than one round of either: 1156,
+// 4352 x 4352 of K = 2048 276 / 306.  A set against itself: 780, 4900 points of K = 784 110 / 120; 990, 5632 of K = 784 130 / 127.
+constexpr int64_t SMALL_TILES_PER_ROUND = kmc::WideTileSmall::MIN_WAVES * 256, LARGE_TILES_PER_ROUND = kmc::WideTileLarge::MIN_WAVES * 256;
+constexpr int64_t LITTLE_OF_A_ROUND = SMALL_TILES_PER_ROUND / 6;
+constexpr int LONG_CONTRACTION_SLICES = 2048 / kmc::BK_TILE_K;
+
 template <bool SYMMETRIC, int EPILOGUE>
 hipError_t launch_product(kmc::GramWideArgs &wide, hipStream_t stream)
 {
     using Large = kmc::WideTileLarge;
-    int64_t tiles = static_cast<int64_t>((wide.kernel.m + Large::TILE_M - 1) / Large::TILE_M) * ((wide.kernel.n + Large::TILE_N - 1) / Large::TILE_N) * wide.kernel.l;
-    if (SYMMETRIC) tiles /= 2;
-    return tiles >= kmc_rules::WIDE_LARGE_TILE_MIN_TILES ? launch_product_in<Large, SYMMETRIC, EPILOGUE>(wide, stream)
-                                                         : launch_product_in<kmc::WideTileSmall, SYMMETRIC, EPILOGUE>(wide, stream);
+    using Small = kmc::WideTileSmall;
+    auto tiles_of = [&](int tile_m, int tile_n) {
+        return static_cast<int64_t>((wide.kernel.m + tile_m - 1) / tile_m) * ((wide.kernel.n + tile_n - 1) / tile_n) * wide.kernel.l / (SYMMETRIC ? 2 : 1);
+    };
+    const int64_t large = tiles_of(Large::TILE_M, Large::TILE_N), small = tiles_of(Small::TILE_M, Small::TILE_N);
+    const bool one_round = !SYMMETRIC && small > SMALL_TILES_PER_ROUND && large <= LARGE_TILES_PER_ROUND &&
+                           (small <= SMALL_TILES_PER_ROUND + LITTLE_OF_A_ROUND || wide.slices >= LONG_CONTRACTION_SLICES);
+    return large >= kmc_rules::WIDE_LARGE_TILE_MIN_TILES || one_round ? launch_product_in<Large, SYMMETRIC, EPILOGUE>(wide, stream)
+                                                                      : launch_product_in<Small, SYMMETRIC, EPILOGUE>(wide, stream);
 }
 
 // Bytes of workspace the path needs for this problem; 0 when it does not apply.

@@ -16,7 +16,8 @@ SHAPES = [
 
 
 def _truth(a, b, entries):
-    return (a[entries].double()[:, :, None, :] - b[entries].double()[:, None, :, :]).square().sum(-1).sqrt()
+    return torch.stack([torch.cdist(a[e].double().cpu(), b[e].double().cpu(), p=2.0, compute_mode="donot_use_mm_for_euclid_dist")
+                        for e in entries]).to(a.device)
 
 
 @pytest.fixture(autouse=True)
@@ -41,6 +42,28 @@ def test_distances_and_products(device, L, M, N, K, panel):
     exact = torch.matmul(a[entries].double(), b[entries].double().transpose(1, 2).contiguous())
     scale = torch.matmul(a[entries].double().abs(), b[entries].double().abs().transpose(1, 2).contiguous())
     assert ((dot[entries].double() - exact).abs() <= 1e-6 * scale).all()
+
+
+@pytest.mark.parametrize("L,M,N,K,tile", [(192, 256, 256, 48, "128, 128"), (193, 256, 256, 48, "256, 128"), (224, 256, 256, 48, "256, 128"),
+                                          (225, 256, 256, 48, "128, 128"), (225, 256, 256, 2033, "256, 128"), (256, 256, 256, 2048, "256, 128"),
+                                          (257, 256, 256, 2048, "128, 128"), (769, 128, 128, 48, "128, 128"), (56, 600, 300, 48, "256, 128"),
+                                          (86, 300, 600, 48, "128, 128"), (2, 2816, 2810, 2048, "256, 128")])
+@pytest.mark.parametrize("same", [False, True])
+def test_which_tile_runs(device, L, M, N, K, tile, same):
+    """A round of the chip is 768 tiles of 128 x 128 or 512 of 256 x 128: the large ones where they are one round and the small ones are a
+    little more (up to 896) or K is long, but not for a set against itself."""
+    gen = torch.Generator(device=device).manual_seed(L)
+    # rows contiguous, the result too: M is the kernel's m
+    a, b = (torch.randn(L, K, rows, device=device, generator=gen).transpose(1, 2) for rows in (M, N))
+    b = a if same else b
+    out = torch.empty(L, b.size(1), M, device=device).transpose(1, 2)
+    with kermac.l2_mode("gram_bf16", min_k=1):
+        names = kernels_of(lambda: kermac.cdist(a, b, out=out, p=2.0))
+    ran = [name.split("WideTile<")[1].split(">")[0] for name in names if "gram_f16_wide<" in name]
+    assert ran == ["128, 128" if same else tile]
+    rows, columns = (sorted({min(at, n - 1) for at in (0, 1, 127, 128, 255, 256, n // 2, n - 129, n - 1)}) for n in (M, b.size(1)))
+    truth = _truth(a[:, rows], b[:, columns], [0, L - 1])
+    assert ((out[[0, L - 1]][:, rows][:, :, columns].double() - truth).abs() <= 1e-5 * truth).all()
 
 
 @pytest.mark.parametrize("L,M,K", [(1, 1, 5), (2, 130, 33), (1, 385, 64), (1400, 257, 40), (4200, 140, 32)])
