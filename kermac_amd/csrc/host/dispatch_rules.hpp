@@ -29,6 +29,8 @@
     X(WIDE_SYMMETRIC_MIN_TILES_TIMES_K, 54000)                                                          \
     /* the product kernel's tile: 256 x 128 from this many of them over the batch on, 128 x 128 below */    \
     X(WIDE_LARGE_TILE_MIN_TILES, 4096)                                                                  \
+    /* ... batches of entries of up to this many tiles of 128 x 128: an XCD for each of eight entries */     \
+    X(WIDE_ENTRY_PER_XCD_MAX_TILES, 128)                                                                \
     /* sums of products through the workspace (the alternative is the direct kernel) */                 \
     X(DOT_MIN_K, 128)                                                                                   \
     X(DOT_MIN_TILES, 64)                                                                                \

@@ -84,6 +84,7 @@ struct GramWideArgs {
     i64 unscale_a_bs, unscale_b_bs;
     int rows_pad_a, rows_pad_b, slices, ranges_a, ranges_b;
     int wide_tiles_m, wide_tiles_n, wide_tiles_n_padded;
+    int entry_per_xcd;                    // wide_tile_of_workgroup
     // GW_EPILOGUE_GRADIENT_L2 only: row r of b stands for (o, n) = (r / gradient_n, r % gradient_n) and
     // the result is (d[n][m] - shift[n]) * g[m][o] - a[m] . b[r]
     const float *gradient_d; i64 gradient_d_ld, gradient_d_bs;
@@ -423,11 +424,19 @@ typedef WideTile<128, 128> WideTileSmall;
 // so the workgroups resident on an XCD (the hardware deals ids round-robin) cover a block of about 8 n tiles x 8 m tiles.
 // SYMMETRIC (a panel against itself): the ids count through the 256 x 256 blocks on and below the diagonal (row r of
 // the triangle starts at block r (r + 1) / 2), each of them the tiles of TILE_M x TILE_N it holds.
+// args.entry_per_xcd (batches of small entries): of eight consecutive batch entries each has an XCD to itself, so that the tiles of
+// an entry read their operands through one L2 instead of each through another; what is left over behind the last eight goes the ordinary way.
 template <typename Tile, bool SYMMETRIC>
-__device__ __forceinline__ bool wide_tile_of_workgroup(const GramWideArgs &args, int &tile_m, int &tile_n)
+__device__ __forceinline__ bool wide_tile_of_workgroup(const GramWideArgs &args, int &batch, int &tile_m, int &tile_n)
 {
     const int rotated = blockIdx.x + blockIdx.y % gridDim.x;
-    const int linear = rotated >= (int)gridDim.x ? rotated - (int)gridDim.x : rotated;
+    int linear = rotated >= (int)gridDim.x ? rotated - (int)gridDim.x : rotated;
+    batch = blockIdx.y;
+    if (args.entry_per_xcd && (blockIdx.y | (BK_XCDS - 1)) < gridDim.y) {
+        const int in_eight = (int)((blockIdx.y % BK_XCDS) * gridDim.x + blockIdx.x);
+        batch = (int)(blockIdx.y / BK_XCDS * BK_XCDS) + in_eight % BK_XCDS;
+        linear = in_eight / BK_XCDS;
+    }
     if (SYMMETRIC) {
         constexpr int PER_M = GW_TILE / Tile::TILE_M, PER_N = GW_TILE / Tile::TILE_N;
         const int block = linear / (PER_M * PER_N), inside = linear - block * (PER_M * PER_N);
@@ -640,9 +649,8 @@ __global__ __launch_bounds__(Tile::THREADS, Tile::MIN_WAVES) void gram_f16_wide(
     __shared__ int lds_distrust[Tile::PARTS];
 
     const int tid = threadIdx.x;
-    const int batch = blockIdx.y;
-    int tile_m, tile_n;
-    if (!wide_tile_of_workgroup<Tile, SYMMETRIC>(args, tile_m, tile_n)) return;
+    int batch, tile_m, tile_n;
+    if (!wide_tile_of_workgroup<Tile, SYMMETRIC>(args, batch, tile_m, tile_n)) return;
     const int m0 = tile_m * TILE_M;
     const int n0 = tile_n * TILE_N;
     const int m_valid = args.kernel.m - m0;

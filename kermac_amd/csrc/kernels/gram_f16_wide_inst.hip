@@ -301,6 +301,13 @@ hipError_t launch_product_in(kmc::GramWideArgs &wide, hipStream_t stream)
     const int64_t width = SYMMETRIC ? blocks * (blocks + 1) / 2 * (kmc::GW_TILE / Tile::TILE_M) * (kmc::GW_TILE / Tile::TILE_N)
                                     : static_cast<int64_t>(wide.wide_tiles_m) * padded;
     if (width > 0x7fffffff) return hipErrorInvalidValue;
+    // An entry of a batch on one XCD, with how it was spread over all of them and with the kernel before these tiles (half as many reads of
+    // an operand), us: 64 x 300 x 300 x 4096, products, 866 / 1009 / 946; 16 x 1280 x 1280 x 4096 1010 / 1174 / 1108; 10 x 1100 x 1100 x 4096
+    // 637 / 733 / 664; 64 x 600 x 600 x 4096 1593 / 1993 / 1886; 500 x 300 x 300 x 784 1207 / 1408 / 1793; 40 sets of 900 points of K = 784
+    // against themselves 224 / 251; 10 x 1500 x 100 x 8 x 4000, the gradient, 738 / 836 / 754.  Larger entries keep an XCD's L2 busy by themselves
+    // and gain nothing: 20 x 2000 x 2000 (256 tiles each) 248 / 236 at K = 256, 536 / 535 at K = 784; 8 x 4096 x 4096 x 784 752 / 702.
+    wide.entry_per_xcd = wide.kernel.l >= kmc::BK_XCDS &&
+                         static_cast<int64_t>((wide.kernel.m + 127) / 128) * ((wide.kernel.n + 127) / 128) <= kmc_rules::WIDE_ENTRY_PER_XCD_MAX_TILES;
     return launch(kmc::gram_f16_wide<Tile, SYMMETRIC, EPILOGUE>, dim3(static_cast<unsigned>(width), wide.kernel.l, 1), dim3(Tile::THREADS), stream, wide);
 }
 

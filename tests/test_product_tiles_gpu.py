@@ -66,6 +66,29 @@ def test_which_tile_runs(device, L, M, N, K, tile, same):
     assert ((out[[0, L - 1]][:, rows][:, :, columns].double() - truth).abs() <= 1e-5 * truth).all()
 
 
+@pytest.mark.parametrize("L,M,N,K", [(7, 130, 129, 40), (8, 130, 257, 33), (9, 300, 140, 32), (23, 65, 129, 20), (8, 1024, 2048, 16), (8, 1024, 2049, 16),
+                                     (4100, 17, 9, 40), (4100, 129, 128, 8)])
+@pytest.mark.parametrize("same", [False, True])
+def test_every_entry_of_a_batch(device, L, M, N, K, same):
+    """Eight entries at a time have an XCD each, up to 128 tiles per entry; the entries behind the last eight, and larger ones, are spread over all."""
+    if same and M == 1024:
+        M = N = 1408 if N == 2048 else 1409             # 121 and 144 tiles
+    gen = torch.Generator(device=device).manual_seed(L + M)
+    a, b = (torch.randn(L, rows, K, device=device, generator=gen) for rows in (M, N))
+    b = a if same else b
+    with kermac.l2_mode("gram_bf16", min_k=1):
+        got = kermac.cdist(a, b, p=2.0)
+        dot = kermac.run_kernel(kermac.kernel_descriptor_mma, a, b)
+    for entry in range(0, L, 1 if L < 100 else 53):
+        x, y = a[entry].double(), b[entry].double()
+        exact, scale = x @ y.t().contiguous(), x.abs() @ y.abs().t().contiguous()
+        truth = ((x * x).sum(1)[:, None] + (y * y).sum(1)[None] - 2 * exact).clamp_min(0).sqrt()
+        if same:
+            truth.fill_diagonal_(0)
+        assert ((got[entry].double() - truth).abs() <= 1e-5 * truth).all()
+        assert ((dot[entry].double() - exact).abs() <= 1e-6 * scale).all()        # as above
+
+
 @pytest.mark.parametrize("L,M,K", [(1, 1, 5), (2, 130, 33), (1, 385, 64), (1400, 257, 40), (4200, 140, 32)])
 def test_a_set_against_itself(device, L, M, K):
     gen = torch.Generator(device=device).manual_seed(M)
