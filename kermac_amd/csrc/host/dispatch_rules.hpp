@@ -44,6 +44,7 @@
     X(SAMPLE_LEAVE_PER_16384, 2)           /* pairs below the trust threshold, spread over the tiles */ \
     /* the direct kernel in tiles of 64 x 64: up to this many tiles of 128 x 128 over the batch */        \
     X(DIRECT_SMALL_MAX_TILES, 256)                                                                      \
+    X(DIRECT_SMALL_MAX_TILES_ROOTS, 192)   /* ... and for fractional powers */                          \
     /* the direct kernel compiled for four waves per SIMD (k-major panels, no fractional power) */       \
     X(DIRECT_FOUR_WAVES_MIN_K, 256)                                                                     \
     /* ... and the one with b in scalar registers (absolute and squared differences, K and N multiples of 16): */ \

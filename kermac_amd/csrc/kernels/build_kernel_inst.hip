@@ -107,7 +107,14 @@ hipError_t launch_scalar_b_if_the_sample_leaves(int load_a, int load_b, const km
 // for every CU, 127 / 86 and 342 / 334; a set against itself of 16 x 16 tiles 165 / 108 and 439 / 428.  Beyond that a single problem
 // still gains (360 tiles 136 / 124 and 647 / 481) but a batch loses (32 x 500 x 500 146 / 165 and 657 / 636, at K = 64 33 / 39), and
 // so does a set against itself, of which this kernel computes both halves (22 x 22 tiles 167 / 194 and 445 / 802).
-// KERMAC_AMD_DIRECT_SMALL_MAX_TILES=n replaces the limit (read on every call, so that a test can choose the kernel).
+// Powers with a root or a transcendental function are bound by its issue, and there a fourth workgroup of 64 x 64 per CU is a round of
+// its own: up to 192 tiles, three per CU (192 x 128 x 128, p = 1.3, K = 16, 64 and 256 20.6 / 20.5, 59.0 / 50.6 and 213 / 173;
+// 208 x 128 x 128 20.6 / 24.0, 59.0 / 63.1 and 214 / 220, p = 0.5 at K = 64 38.2 / 40.9; 1792 x 1792, 196 tiles, p = 1.3 21.0 / 23.6, 58.9 / 61.8
+// and 213 / 215).
+// KERMAC_AMD_DIRECT_SMALL_MAX_TILES=n replaces both limits (read on every call, so that a test can choose the kernel).
+constexpr bool HAS_ROOT_OR_POWER = KMC_INNER_POW == kmc::POW_POW || KMC_INNER_POW == kmc::POW_SQRT || KMC_INNER_POW == kmc::POW_ABS_HALF ||
+                                   KMC_INNER_POW == kmc::POW_ABS_THREE_HALVES;
+
 static bool small_applies(int load_a, int load_b, const kmc::BuildKernelArgs &args)
 {
     if (args.repair_only || args.k_total != 0 || args.panels != 0) return false;
@@ -116,7 +123,7 @@ static bool small_applies(int load_a, int load_b, const kmc::BuildKernelArgs &ar
     if (HAS_SCALAR_B && load_a == kmc::LOAD_COL_VEC && load_b == kmc::LOAD_COL_VEC && scalar_b_applies(args, &grid_width)) return false;
     const int64_t tiles = static_cast<int64_t>(args.tiles_m) * args.tiles_n * args.l;
     const char *limit = std::getenv("KERMAC_AMD_DIRECT_SMALL_MAX_TILES");
-    return tiles <= (limit ? std::atoi(limit) : kmc_rules::DIRECT_SMALL_MAX_TILES);
+    return tiles <= (limit ? std::atoi(limit) : HAS_ROOT_OR_POWER ? kmc_rules::DIRECT_SMALL_MAX_TILES_ROOTS : kmc_rules::DIRECT_SMALL_MAX_TILES);
 }
 
 hipError_t KMC_LAUNCHER_NAME(int load_a, int load_b, const kmc::BuildKernelArgs &args, dim3 grid, hipStream_t stream)

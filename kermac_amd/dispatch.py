@@ -85,7 +85,7 @@ _ROWS = (
      "direct `build_kernel` (ahead of time for DIFF + NOOP/ABS/SQUARE/POW and DOT + NOOP, else compiled on first use); scalar p of 0.5, 1.5, 3, 4 on "
      "the exact-form variants"),
     ("every direct launch",
-     "≤ {DIRECT_SMALL_MAX_TILES} tiles of 128 × 128 over the batch, compiled ahead of time, not ranges of one contraction, not a repair launch",
+     "≤ {DIRECT_SMALL_MAX_TILES} tiles of 128 × 128 over the batch, ≤ {DIRECT_SMALL_MAX_TILES_ROOTS} for fractional powers, compiled ahead of time, not ranges of one contraction, not a repair launch",
      "`build_kernel_small` (tiles of 64 × 64)"),
     ("",
      "absolute differences, their squares, and the scalar exponents 3 and 4; both operands with m / n contiguous and 16-byte aligned, K and N multiples of 16, K ≥ {DIRECT_SCALAR_B_MIN_K}, "

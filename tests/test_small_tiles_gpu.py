@@ -4,6 +4,7 @@ import pytest
 import torch
 
 import kermac_amd as kermac
+from tests.helpers import kernels_of
 
 pytestmark = pytest.mark.gpu
 
@@ -49,3 +50,11 @@ def test_a_set_against_itself(device, M, K):
     other = kermac.cdist(a, a.clone(), p=1.0)[0]
     same = (got == other) | (torch.isnan(got) & torch.isnan(other))
     assert same.all() and ((got == got.t()) | torch.isnan(got)).all()
+
+
+@pytest.mark.parametrize("p,most", [(1.0, 256), (3.0, 256), (1.3, 192), (0.5, 192), (1.5, 192)])
+def test_up_to_how_many_tiles(device, p, most):
+    """Fractional powers lose on a fourth workgroup per CU, the others do not."""
+    x = torch.randn(most + 1, 40, 5, device=device, generator=torch.Generator(device=device).manual_seed(1))
+    ran = [[name for name in kernels_of(lambda: kermac.cdist(x[:tiles], x[:tiles] + 1.0, p=p)) if "build_kernel" in name] for tiles in (most, most + 1)]
+    assert ["build_kernel_small<" in name for names in ran for name in names] == [True, False]
