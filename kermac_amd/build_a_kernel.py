@@ -742,7 +742,7 @@ def _auto_matrix_core_flags(params, asked):
                 return 0
         finally:
             params.flags = kept
-    if not rows_contiguous and not _against_itself(params):
+    if not rows_contiguous and not _split_kernel_knows_equal_points(params, tiles * params.l):
         if (params.k >= _AUTO_FP32_MIN_K and _AUTO_FP32_MIN_TILES <= tiles * params.l <= _AUTO_FP32_MAX_TILES
                 and tiles >= _AUTO_FP32_MIN_TILES_PER_ENTRY):
             return _backend.FLAG_L2_GRAM
@@ -751,11 +751,21 @@ def _auto_matrix_core_flags(params, asked):
     return asked
 
 
-def _against_itself(params):
-    """Whether both operands are the same rows in memory.  The fp32 one-step kernel distrusts every tile on the diagonal of such
-    a result and leaves it to the repair launch, the split kernel knows that the distances there are zero."""
-    return (params.a == params.b and params.a_ld == params.b_ld and params.a_bs == params.b_bs
-            and params.a_majorness == params.b_majorness)
+# Rows that are not 16-byte aligned: the split kernel runs two workgroups per CU on them, and beyond one round of those the fp32
+# kernel is ahead in spite of the repairs (30000 points of K = 1030 against their first 100, 4 batch entries, 940 tiles, fp32 / split 690 / 1200 us;
+# 50000 against 100, 391 tiles, 540 / 375).
+_AUTO_EQUAL_POINTS_UNALIGNED_MAX_TILES = 512
+
+
+def _split_kernel_knows_equal_points(params, tiles):
+    """Whether both operands are the same rows in memory and the split kernel acts on it.  The fp32 one-step kernel distrusts every
+    tile on the diagonal of such a result and leaves it to the repair launch; the split kernel knows that the distances there are
+    zero, except in results of one row of tiles, which it leaves to the repair launch too (50000 points of K = 784 against their first
+    100, m = 50000: fp32 / split 463 / 225 us; m = 100: 414 / 456, in 4 batch entries of 30000 546 / 853)."""
+    if (params.a != params.b or params.a_ld != params.b_ld or params.a_bs != params.b_bs or params.a_majorness != params.b_majorness
+            or params.m <= 128):
+        return False
+    return params.a_ld % 4 == 0 or tiles <= _AUTO_EQUAL_POINTS_UNALIGNED_MAX_TILES
 
 
 def _workspace_route_applies(params, flags):

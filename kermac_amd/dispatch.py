@@ -62,7 +62,8 @@ _ROWS = (
      "K ≥ {build_a_kernel.AUTO_ONE_STEP_MIN_K}, trust < 1, "
      "and not (a call the direct path would cut over k on fewer than {build_a_kernel.AUTO_UNCUT_MIN_TILES_K_CONTIGUOUS} tiles of 128 × 128, "
      "{build_a_kernel.AUTO_UNCUT_MIN_TILES} with the rows contiguous)",
-     "one-step matrix-core kernel: `gram_l2_kernel` (fp32 matrix instruction) for two different sets with k contiguous in an operand and K ≥ {build_a_kernel.AUTO_FP32_MIN_K} on "
+     "one-step matrix-core kernel: `gram_l2_kernel` (fp32 matrix instruction), but for a set against rows of its own with M > 128 (and ld a multiple of 4 or ≤ "
+     "{build_a_kernel.AUTO_EQUAL_POINTS_UNALIGNED_MAX_TILES} tiles), with k contiguous in an operand and K ≥ {build_a_kernel.AUTO_FP32_MIN_K} on "
      "{build_a_kernel.AUTO_FP32_MIN_TILES} … {build_a_kernel.AUTO_FP32_MAX_TILES} tiles over the batch and ≥ {build_a_kernel.AUTO_FP32_MIN_TILES_PER_ENTRY} per entry, "
      "or one dimension ≤ 128 with ≥ {build_a_kernel.AUTO_FP32_MIN_TILES} "
      "tiles; else `gram_bf16_l2_kernel` (three bf16 pieces); from M · N · K · L ≥ {build_a_kernel.L2_SAMPLE_MIN_TERMS} on `gram_probe_operands` in front "

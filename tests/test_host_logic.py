@@ -331,13 +331,16 @@ def test_auto_mode_picks_the_kernel_by_shape_without_a_gpu(monkeypatch):
         monkeypatch.delenv(name, raising=False)
     core = _backend.FLAG_L2_GRAM | _backend.FLAG_L2_GRAM_BF16
 
-    def chosen(m, n, k, l=1, dot=False, rows_contiguous=False):
+    def chosen(m, n, k, l=1, dot=False, rows_contiguous=False, same=False):
         params = _backend.BuildKernelParams()
         params.a_majorness = params.b_majorness = _backend.COL_MAJOR if rows_contiguous else _backend.ROW_MAJOR
         params.inner_operator, params.inner_power, params.outer_power = (1, 0, 0) if dot else (0, 2, 3)
         params.m, params.n, params.k, params.l = m, n, k, l
         params.a, params.a_ld, params.a_bs = 4096, (m if rows_contiguous else k), m * k
         params.b, params.b_ld, params.b_bs = 4096 + 4 * m * k * l, (n if rows_contiguous else k), n * k
+        if same:                                                 # rows of one set of max(m, n) points
+            params.a_bs = params.b_bs = max(m, n) * k
+            params.b = params.a
         params.c, params.c_ld, params.c_bs = 256, m, m * n
         params.gram_trust = module._gram_trust(k, {"trust": None})
         return module._auto_matrix_core_flags(params, _backend.FLAG_DOT_PIECES if dot else core)
@@ -363,6 +366,12 @@ def test_auto_mode_picks_the_kernel_by_shape_without_a_gpu(monkeypatch):
     assert chosen(5000, 5000, 128, rows_contiguous=True) == core and chosen(5000, 5000, 128) == core and chosen(5000, 5000, 112) == 0
     assert chosen(1500, 1500, 1024, rows_contiguous=True) == core and chosen(1500, 1500, 400) == _backend.FLAG_L2_GRAM
     assert chosen(2000, 2000, 784, rows_contiguous=True) == core              # the split one-step kernel there
+    # a set against rows of its own: the split kernel knows the equal points, but not in a result of one row of tiles
+    assert chosen(50000, 100, 784, same=True) == core and chosen(50000, 100, 784) == _backend.FLAG_L2_GRAM
+    assert chosen(100, 50000, 784, same=True) == _backend.FLAG_L2_GRAM and chosen(100, 30000, 784, l=4, same=True) == _backend.FLAG_L2_GRAM
+    assert chosen(128, 128, 1030, l=128, same=True) == _backend.FLAG_L2_GRAM
+    assert chosen(50000, 100, 1030, same=True) == core           # rows that are not 16-byte aligned: up to 512 tiles
+    assert chosen(30000, 100, 1030, l=4, same=True) == _backend.FLAG_L2_GRAM and chosen(30000, 100, 1032, l=4, same=True) == core
     assert chosen(8192, 4096, 512, dot=True) == _backend.FLAG_DOT_PIECES
     assert chosen(300, 300, 512, dot=True) == 0
     # from K = 256 on: 32 tiles over a batch, 64 of a single problem (which the direct path would cut over k), any padding
