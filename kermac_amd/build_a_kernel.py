@@ -727,7 +727,7 @@ _AUTO_UNCUT_MIN_TILES_K_CONTIGUOUS = 192
 
 def _auto_matrix_core_flags(params, asked):
     """Which of the matrix-core flags `asked` (those the descriptor allows) this call gets in the l2 mode "auto"."""
-    if _workspace_route_applies(params, asked):
+    if _workspace_route_applies(params, asked) and not _route_splits_a_small_set_slowly(params, asked):
         return asked
     # operands with the rows contiguous (m or n, the kernels' own order) stage faster in the split kernel
     rows_contiguous = params.a_majorness == _backend.COL_MAJOR and params.b_majorness == _backend.COL_MAJOR
@@ -766,6 +766,21 @@ def _split_kernel_knows_equal_points(params, tiles):
             or params.m <= 128):
         return False
     return params.a_ld % 4 == 0 or tiles <= _AUTO_EQUAL_POINTS_UNALIGNED_MAX_TILES
+
+
+# A set of fewer than 1665 points against itself goes through the workspace instead of the direct path, cut over k, and that pays where
+# its rows are split in one pass or by 128-bit loads.  Rows that are neither (K > 1024, not 16-byte aligned) take two passes of single loads,
+# cut / route, us: 1400 points of K = 1001 82 / 65, of K = 1025 83 / 97, of K = 1030 84 / 100, of K = 1100 88 / 80, of K = 3001 194 / 202;
+# 1536 of K = 1030 80 / 100; 1664 of K = 1030 98 / 101, of K = 3001 225 / 209; 1700, uncut, of K = 1030 450 / 102.
+_AUTO_ROUTE_ONE_PASS_MAX_K = 1024
+
+
+def _route_splits_a_small_set_slowly(params, asked):
+    tiles = -(-params.m // 128)
+    return bool(asked & _backend.FLAG_L2_GRAM and params.l == 1 and params.k > _AUTO_ROUTE_ONE_PASS_MAX_K and params.a_ld % 4 != 0
+                and params.a == params.b and params.m == params.n and params.a_ld == params.b_ld
+                and params.a_majorness == params.b_majorness == _backend.ROW_MAJOR
+                and tiles * tiles < _AUTO_UNCUT_MIN_TILES_K_CONTIGUOUS)
 
 
 def _workspace_route_applies(params, flags):
