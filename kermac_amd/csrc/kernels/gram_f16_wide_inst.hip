@@ -338,8 +338,11 @@ hipError_t launch_product(kmc::GramWideArgs &wide, hipStream_t stream)
     const int64_t large = tiles_of(Large::TILE_M, Large::TILE_N), small = tiles_of(Small::TILE_M, Small::TILE_N);
     const bool one_round = !SYMMETRIC && small > SMALL_TILES_PER_ROUND && large <= LARGE_TILES_PER_ROUND &&
                            (small <= SMALL_TILES_PER_ROUND + LITTLE_OF_A_ROUND || wide.slices >= LONG_CONTRACTION_SLICES);
-    return large >= kmc_rules::WIDE_LARGE_TILE_MIN_TILES || one_round ? launch_product_in<Large, SYMMETRIC, EPILOGUE>(wide, stream)
-                                                                      : launch_product_in<Small, SYMMETRIC, EPILOGUE>(wide, stream);
+    // KERMAC_AMD_WIDE_LARGE_TILE_MIN_TILES=n replaces the number (read on every call, so that a test can send small shapes to the large tiles)
+    const char *text = std::getenv("KERMAC_AMD_WIDE_LARGE_TILE_MIN_TILES");
+    return large >= (text ? std::atoi(text) : kmc_rules::WIDE_LARGE_TILE_MIN_TILES) || one_round
+               ? launch_product_in<Large, SYMMETRIC, EPILOGUE>(wide, stream)
+               : launch_product_in<Small, SYMMETRIC, EPILOGUE>(wide, stream);
 }
 
 // Bytes of workspace the path needs for this problem; 0 when it does not apply.

@@ -26,3 +26,11 @@ def direct_tile(request, monkeypatch):
     if request.param == "128x128":
         monkeypatch.setenv("KERMAC_AMD_DIRECT_SMALL_MAX_TILES", "0")
     return request.param
+
+
+@pytest.fixture(params=["by the rule", "256x128"])
+def product_tile(request, monkeypatch):
+    """Both tiles of the workspace route's product kernel for the small results of a test: 128 x 128 by the library's rule, and 256 x 128."""
+    if request.param == "256x128":
+        monkeypatch.setenv("KERMAC_AMD_WIDE_LARGE_TILE_MIN_TILES", "1")
+    return request.param

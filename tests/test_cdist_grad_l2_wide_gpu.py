@@ -19,7 +19,7 @@ module = importlib.import_module("kermac_amd.cdist_grad")       # the package at
 from oracle import oracle
 from tests.helpers import assert_close_to_truth
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("product_tile")]
 
 
 @pytest.fixture

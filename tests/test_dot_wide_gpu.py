@@ -15,7 +15,7 @@ from kermac_amd import _backend, build_a_kernel as module
 from oracle import oracle
 from tests.helpers import assert_close_to_truth, make_operand
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("product_tile")]
 
 DOT = kermac.KernelDescriptor(kermac.InnerOperator.DOT, kermac.PowerType.NOOP, kermac.PowerType.NOOP, kermac.KernelType.NONE)
 POLYNOMIAL = kermac.KernelDescriptor(kermac.InnerOperator.DOT, kermac.PowerType.NOOP, kermac.PowerType.POW, kermac.KernelType.NONE)

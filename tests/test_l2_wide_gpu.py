@@ -17,7 +17,7 @@ from kermac_amd import _backend, build_a_kernel as module
 from oracle import oracle
 from tests.helpers import assert_close_to_truth, make_operand
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("product_tile")]
 
 
 @pytest.fixture

@@ -128,6 +128,39 @@ def test_a_set_against_itself_in_one_step(device, monkeypatch, L, M, K, panel):
     assert ((run.double() - part).abs() <= 1e-5 * part)[torch.isfinite(part)].all()
 
 
+@pytest.mark.parametrize("K", [20, 300])
+@pytest.mark.parametrize("panel", [False, True])
+def test_distrusted_parts_of_a_large_tile(device, monkeypatch, panel, K):
+    """A tile of 256 x 128 is two parts to the repair launch: a near-duplicate in one of them, in the other, in both, a row that is not a
+    number; of a set against itself also with twins on the diagonal and in the part above it inside a tile."""
+    monkeypatch.setenv("KERMAC_AMD_WIDE_LARGE_TILE_MIN_TILES", "1")
+    monkeypatch.setenv("KERMAC_AMD_L2_PROBE", "0")
+    gen = torch.Generator(device=device).manual_seed(K)
+    a, b = torch.randn(700, K, device=device, generator=gen), torch.randn(515, K, device=device, generator=gen)
+    b[5], b[130], b[300], b[301] = a[3] + 1e-3, a[140] + 1e-3, a[400] + 1e-3, a[513] + 1e-3
+    own = a.clone()
+    own[100], own[300], own[500] = own[20] + 1e-3, own[140] + 1e-3, own[390] + 1e-3      # one part, across parts, above the diagonal
+    a[650, K // 2], own[690, 0] = float("nan"), float("inf")
+
+    def stored(x):
+        return x.t().contiguous().t() if panel else x
+
+    a, b, own = stored(a), stored(b), stored(own)
+    calls = []
+    for x, y in ((a, b), (own, own)):
+        out = torch.empty(y.size(0), x.size(0), device=device).t()
+        with kermac.l2_mode("gram_bf16", min_k=1):
+            calls += [name for name in kernels_of(lambda: kermac.cdist(x, y, out=out, p=2.0)) if "gram_f16_wide<" in name]
+        truth = _truth(x[None], y[None], [0])[0]
+        finite = torch.isfinite(truth)
+        assert (torch.isfinite(out) == finite).all()
+        assert ((out.double() - truth).abs() <= 1e-5 * truth)[finite].all()
+        if y is x:
+            clean = torch.where(finite, out, torch.zeros_like(out))
+            assert torch.equal(clean, clean.t()) and (torch.diagonal(clean) == 0).all()
+    assert len(calls) == 2 and all("WideTile<256, 128>" in name for name in calls)
+
+
 @pytest.mark.parametrize("K", [3, 255, 256, 257, 260, 511, 512, 513, 1000, 1023, 1024, 1025])
 @pytest.mark.parametrize("form", ["rows", "misaligned", "a_panel", "b_panel", "offset"])
 def test_rows_of_any_length(device, K, form):

@@ -41,6 +41,31 @@ def test_the_bits_of_the_large_tile(device, M, N, K, form_a, form_b, p):
     assert ((small.reshape(M, N).double().cpu() - truth).abs() <= (1e-4 if p == 1.3 else 1e-5) * truth).all()
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (63, 65, 15), (65, 127, 33), (130, 61, 16), (129, 200, 47)])
+@pytest.mark.parametrize("form_a,form_b", [("rows", "rows"), ("panel", "panel"), ("misaligned", "panel"), ("misaligned_panel", "misaligned")])
+@pytest.mark.parametrize("operator", ["signed differences", "products"])
+def test_the_bits_of_the_large_tile_where_no_power_is_taken(device, M, N, K, form_a, form_b, operator):
+    gen = torch.Generator(device=device).manual_seed(M + N + K)
+    a, b = (torch.randn(rows, K, device=device, generator=gen) for rows in (M, N))
+    a_many, b_many = (_stored(x.expand(COPIES, *x.shape).contiguous(), f) for x, f in ((a, form_a), (b, form_b)))
+    inner = kermac.InnerOperator.DIFF if operator == "signed differences" else kermac.InnerOperator.DOT
+    descriptor = kermac.KernelDescriptor(inner, kermac.PowerType.NOOP, kermac.PowerType.NOOP, kermac.KernelType.NONE)
+    results = []
+    with kermac.l2_mode("direct"):
+        for x, y, kernel in ((_stored(a, form_a), _stored(b, form_b), True), (a_many, b_many, False)):
+            kept = []
+            ran = [name for name in kernels_of(lambda: kept.append(kermac.run_kernel(descriptor, x, y))) if "build_kernel" in name]
+            assert len(ran) == 1 and ("build_kernel_small<" in ran[0]) == kernel
+            results.append(kept[0])
+    assert torch.equal(results[0].reshape(M, N), results[1][COPIES - 1])
+    x, y = a.double(), b.double()
+    if operator == "products":
+        truth, scale = x @ y.t().contiguous(), x.abs() @ y.abs().t().contiguous()
+    else:
+        truth, scale = (x[:, None] - y[None]).sum(-1), (x[:, None] - y[None]).abs().sum(-1)
+    assert ((results[0].reshape(M, N).double() - truth).abs() <= 1e-5 * scale).all()         # fp32 sums of K terms
+
+
 @pytest.mark.parametrize("M,K", [(65, 20), (300, 6), (129, 64)])
 def test_a_set_against_itself(device, M, K):
     gen = torch.Generator(device=device).manual_seed(M)
