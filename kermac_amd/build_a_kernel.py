@@ -727,7 +727,7 @@ _AUTO_UNCUT_MIN_TILES_K_CONTIGUOUS = 192
 
 def _auto_matrix_core_flags(params, asked):
     """Which of the matrix-core flags `asked` (those the descriptor allows) this call gets in the l2 mode "auto"."""
-    if _workspace_route_applies(params, asked) and not _route_splits_a_small_set_slowly(params, asked):
+    if _workspace_route_applies(params, asked) and not _small_set_is_cut(params, asked):
         return asked
     # operands with the rows contiguous (m or n, the kernels' own order) stage faster in the split kernel
     rows_contiguous = params.a_majorness == _backend.COL_MAJOR and params.b_majorness == _backend.COL_MAJOR
@@ -735,13 +735,8 @@ def _auto_matrix_core_flags(params, asked):
         return 0
     tiles = -(-params.m // 128) * -(-params.n // 128)
     if tiles < (_AUTO_UNCUT_MIN_TILES if rows_contiguous else _AUTO_UNCUT_MIN_TILES_K_CONTIGUOUS):
-        kept = params.flags
-        params.flags &= ~asked                  # the question is what the direct path would do
-        try:
-            if _cut_over_contraction(params) is not None:
-                return 0
-        finally:
-            params.flags = kept
+        if _direct_path_would_cut(params, asked):
+            return 0
     if not rows_contiguous and not _split_kernel_knows_equal_points(params, tiles * params.l):
         if (params.k >= _AUTO_FP32_MIN_K and _AUTO_FP32_MIN_TILES <= tiles * params.l <= _AUTO_FP32_MAX_TILES
                 and tiles >= _AUTO_FP32_MIN_TILES_PER_ENTRY):
@@ -768,19 +763,26 @@ def _split_kernel_knows_equal_points(params, tiles):
     return params.a_ld % 4 == 0 or tiles <= _AUTO_EQUAL_POINTS_UNALIGNED_MAX_TILES
 
 
-# A set of fewer than 1665 points against itself goes through the workspace instead of the direct path, cut over k, and that pays where
-# its rows are split in one pass or by 128-bit loads.  Rows that are neither (K > 1024, not 16-byte aligned) take two passes of single loads,
-# cut / route, us: 1400 points of K = 1001 82 / 65, of K = 1025 83 / 97, of K = 1030 84 / 100, of K = 1100 88 / 80, of K = 3001 194 / 202;
-# 1536 of K = 1030 80 / 100; 1664 of K = 1030 98 / 101, of K = 3001 225 / 209; 1700, uncut, of K = 1030 450 / 102.
-_AUTO_ROUTE_ONE_PASS_MAX_K = 1024
+def _direct_path_would_cut(params, asked):
+    kept = params.flags
+    params.flags &= ~asked
+    try:
+        return _cut_over_contraction(params) is not None
+    finally:
+        params.flags = kept
 
 
-def _route_splits_a_small_set_slowly(params, asked):
+def _small_set_is_cut(params, asked):
+    """A set of up to 1664 points against itself is enough tiles for the workspace route, but where the direct path would cut the call over
+    k, its short fp32 sums hold more of the result than products of pieces and, above all, than the uncut walk that repairs the distrusted
+    parts of such a call.  Route / direct, error of all distances against float64 relative to their 2-norm: 1300 normal points of K = 4096
+    5.7e-8 / 5.1e-8, of K = 784 4.1e-8 / 5.5e-8, heavy-tailed ones of K = 4096 2.0e-7 / 8.0e-8, points in clusters 4.8e-7 / 4.7e-8.  The route
+    would be up to a quarter faster (1400 points of K = 784 77 / 63 us), and a quarter slower where it splits rows that are not 16-byte aligned
+    in two passes (1536 of K = 1030 80 / 100)."""
     tiles = -(-params.m // 128)
-    return bool(asked & _backend.FLAG_L2_GRAM and params.l == 1 and params.k > _AUTO_ROUTE_ONE_PASS_MAX_K and params.a_ld % 4 != 0
-                and params.a == params.b and params.m == params.n and params.a_ld == params.b_ld
-                and params.a_majorness == params.b_majorness == _backend.ROW_MAJOR
-                and tiles * tiles < _AUTO_UNCUT_MIN_TILES_K_CONTIGUOUS)
+    return bool(asked & _backend.FLAG_L2_GRAM and tiles * tiles < _AUTO_UNCUT_MIN_TILES_K_CONTIGUOUS and params.m == params.n
+                and params.a == params.b and params.a_ld == params.b_ld and params.a_majorness == params.b_majorness
+                and _direct_path_would_cut(params, asked))
 
 
 def _workspace_route_applies(params, flags):

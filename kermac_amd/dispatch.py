@@ -54,8 +54,8 @@ _ROWS = (
      "operands instead: K ≥ {WIDE_K_CONTIGUOUS_MIN_K}, ≥ {WIDE_K_CONTIGUOUS_MIN_TILES} tiles, tiles · K ≥ {WIDE_K_CONTIGUOUS_MIN_TILES_TIMES_K}, M and N ≥ "
      "{WIDE_K_CONTIGUOUS_MIN_ROWS}; or a set against itself of ≥ {WIDE_SYMMETRIC_MIN_TILES} tiles (of its triangle), tiles · K ≥ "
      "{WIDE_SYMMETRIC_MIN_TILES_TIMES_K}, with k contiguous K ≥ {WIDE_SYMMETRIC_K_CONTIGUOUS_MIN_K}, ≥ {WIDE_SYMMETRIC_K_CONTIGUOUS_MIN_TILES} tiles, "
-     "tiles · K ≥ {WIDE_SYMMETRIC_K_CONTIGUOUS_MIN_TILES_TIMES_K} (mode `\"auto\"`: not below "
-     "{build_a_kernel.AUTO_UNCUT_MIN_TILES_K_CONTIGUOUS} tiles of 128 × 128 with K > {build_a_kernel.AUTO_ROUTE_ONE_PASS_MAX_K} and ld no multiple of 4)",
+     "tiles · K ≥ {WIDE_SYMMETRIC_K_CONTIGUOUS_MIN_TILES_TIMES_K} (mode `\"auto\"`: not one that "
+     "the direct path would cut over k on fewer than {build_a_kernel.AUTO_UNCUT_MIN_TILES_K_CONTIGUOUS} tiles of 128 × 128)",
      "`gram_rows_once` (k contiguous and K ≤ 1024, the sample in the same launch) or `gram_row_stats_pair` + `gram_f16_split_pair` + `gram_probe_operands`, "
      "`gram_f16_wide` (fp16 pieces, tiles of 256 × 128 from {WIDE_LARGE_TILE_MIN_TILES} on or where those fit the chip at once and 128 × 128 do not, else 128 × 128; in batches of ≥ 8 entries of ≤ {WIDE_ENTRY_PER_XCD_MAX_TILES} tiles of 128 × 128 each entry on one XCD), repair launch "
      "of the direct kernel"),

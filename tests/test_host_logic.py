@@ -366,10 +366,9 @@ def test_auto_mode_picks_the_kernel_by_shape_without_a_gpu(monkeypatch):
     assert chosen(5000, 5000, 128, rows_contiguous=True) == core and chosen(5000, 5000, 128) == core and chosen(5000, 5000, 112) == 0
     assert chosen(1500, 1500, 1024, rows_contiguous=True) == core and chosen(1500, 1500, 400) == _backend.FLAG_L2_GRAM
     assert chosen(2000, 2000, 784, rows_contiguous=True) == core              # the split one-step kernel there
-    # a set of fewer than 192 tiles against itself: the workspace route, but not where splitting its rows takes two passes of single loads
-    assert all(chosen(1400, 1400, k, same=True) == core for k in (400, 784, 1001, 1024, 1100, 2048))
-    assert all(chosen(m, m, k, same=True) == 0 for m in (1300, 1400, 1664) for k in (1025, 1030, 3001))
-    assert all(chosen(m, m, 1030, same=True) == core for m in (1665, 1700, 2000)) and chosen(700, 700, 1030, l=4, same=True) == core
+    # a set of fewer than 192 tiles against itself stays with the direct path where that cuts it over k, and takes the workspace route elsewhere
+    assert all(chosen(m, m, k, same=True) == 0 for m in (1300, 1400, 1664) for k in (512, 784, 1030, 2048, 4096))
+    assert chosen(1400, 1400, 400, same=True) == core and chosen(1665, 1665, 784, same=True) == core and chosen(1000, 1000, 784, l=4, same=True) == core
     # a set against rows of its own: the split kernel knows the equal points, but not in a result of one row of tiles
     assert chosen(50000, 100, 784, same=True) == core and chosen(50000, 100, 784) == _backend.FLAG_L2_GRAM
     assert chosen(100, 50000, 784, same=True) == _backend.FLAG_L2_GRAM and chosen(100, 30000, 784, l=4, same=True) == _backend.FLAG_L2_GRAM

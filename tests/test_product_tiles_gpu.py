@@ -231,3 +231,50 @@ def test_parts_of_one_set_that_share_no_point(device, monkeypatch, panel):
         got = kermac.cdist(x[:301], x[300:], p=2.0)[0]
     truth = _truth(x[None, :301], x[None, 300:], [0])[0]
     assert got[300, 0] == 0 and ((got.double() - truth).abs() <= 1e-5 * truth).all()
+
+
+def _points(distribution, M, K, device):
+    gen = torch.Generator(device=device).manual_seed(M + K)
+    normal = lambda *shape: torch.randn(*shape, device=device, generator=gen)
+    if distribution == "uniform":
+        return torch.rand(M, K, device=device, generator=gen)
+    if distribution == "heavy tails":
+        return normal(M, K) * torch.exp(1.5 * normal(M, K))
+    if distribution == "mostly zeros":
+        return (normal(M, K) - 0.8).clamp_min(0)
+    if distribution == "clusters":                      # squared distances from about a quarter of the norms on, where trust ends
+        return normal(40, K)[torch.randint(0, 40, (M,), device=device, generator=gen)] + 0.75 * normal(M, K)
+    if distribution == "scaled rows":
+        return normal(M, K) * torch.exp(2.0 * normal(M, 1))
+    return normal(M, K)
+
+
+# the workspace route and the one-step split kernel, two storage orders
+@pytest.mark.parametrize("M,K,panel", [(1400, 400, False), (2000, 256, False), (2000, 1024, False), (1000, 200, True), (1500, 200, True), (2400, 1024, True)])
+@pytest.mark.parametrize("distribution", ["normal", "uniform", "heavy tails", "mostly zeros", "clusters", "scaled rows"])
+def test_the_error_of_a_set_against_itself_is_no_larger_than_the_direct_kernels(device, monkeypatch, M, K, panel, distribution):
+    """Sets against themselves multiply pieces of their values by default.  The direct kernel subtracts in fp32 and rounds once per term; the
+    pieces hold 22 or 24 bits, and the products round once per 16 or 32 terms, which leaves the error (2-norm, against float64) below the direct
+    kernel's, of the whole result and of the parts on its diagonal."""
+    x = _points(distribution, M, K, device)
+    stored = x.t().contiguous().t() if panel else x
+    centred = x.double() - x.double().mean(0)
+    squares = (centred * centred).sum(1)
+    truth = (squares[:, None] + squares[None] - 2 * (centred @ centred.t().contiguous())).clamp_min(0).sqrt().fill_diagonal_(0)
+    got = kermac.cdist(stored, stored, p=2.0)[0].double()
+    monkeypatch.setenv("KERMAC_AMD_NO_CUT", "1")
+    with kermac.l2_mode("direct"):
+        direct = kermac.cdist(stored, stored, p=2.0)[0].double()
+    diagonal = torch.block_diag(*[torch.ones(min(128, M - at), min(128, M - at), device=device, dtype=torch.bool) for at in range(0, M, 128)]).bool()
+    for part in (torch.ones_like(diagonal), diagonal):
+        assert (got - truth)[part].norm() <= (direct - truth)[part].norm()
+
+
+@pytest.mark.parametrize("M,K", [(1300, 512), (1400, 784), (1664, 1030), (1300, 4096)])
+@pytest.mark.parametrize("distribution", ["normal", "clusters"])
+def test_a_small_set_against_itself_keeps_the_short_sums_of_the_direct_path(device, M, K, distribution):
+    """Where the direct path is cut over k (512 terms and more, fewer than 192 tiles) its error is below that of the pieces."""
+    x = _points(distribution, M, K, device)
+    got = kermac.cdist(x, x, p=2.0)
+    with kermac.l2_mode("direct"):
+        assert torch.equal(got, kermac.cdist(x, x, p=2.0))
