@@ -109,7 +109,7 @@ enum kmc_flags {
     KMC_FLAG_GRAM_A_KEPT = 64,
     /* kmc_build_kernel, inner_operator DOT with inner_power NOOP (sum_k a b: linear and polynomial
      * kernels), with gram_workspace: large problems are multiplied on the fp16 matrix instruction
-     * from two fp16 pieces per value and a scale per row, in the 256 x 256 tiles of the route that
+     * from two fp16 pieces per value and a scale per row, by the route that
      * KMC_FLAG_L2_GRAM_BF16 describes (kmc_gram_workspace_bytes says which, and how much memory it
      * wants).  Error below 3 * 2^-22 sum_k |a b| + k * 2^-38 max|a[m]| max|b[n]| (a value below
      * 2^-28 of the largest of its row is kept to 2^-40 of that largest one, not to 2^-22 of
@@ -227,8 +227,8 @@ typedef struct kmc_build_kernel_params {
      * aligned, of at least the size kmc_gram_workspace_bytes reports for these parameters.  With
      * it, large problems take a faster route in three steps (statistics per row, both operands
      * split once into two fp16 pieces per value in the order the matrix instruction reads them,
-     * then 256 x 256 tiles on the fp16 matrix instruction; same trust rule, same repair launch,
-     * same tolerance: at M = N = 30000, K = 1024 6.1 ms instead of 10).  NULL, too small, or a
+     * then products of pieces on the fp16 matrix instruction; same trust rule, same repair launch,
+     * same tolerance: at M = N = 30000, K = 1024 4.9 ms instead of 10).  NULL, too small, or a
      * problem for which kmc_gram_workspace_bytes reports 0: the one-step kernel runs.  The
      * contents after the call do not matter; calls that share a workspace must be ordered.
      * With KMC_FLAG_L2_GRAM or KMC_FLAG_L2_GRAM_BF16 on a problem that runs a one-step kernel, a
@@ -345,7 +345,7 @@ typedef struct kmc_norm_gradient_params {
      * run as e = (d - s) g - p a with g[m][o] = sum_k a c, p[o n_rows + n][k] = c[o][k] (b[n][k] - s[n])
      * and s[n] the mean of row n of b (any s gives the same e; this one keeps both terms as small
      * as the data allows): p and a are split once into two fp16 pieces per value with a scale per
-     * row and multiplied in 256 x 256 tiles on the fp16 matrix instruction, g comes from the fp32
+     * row and multiplied on the fp16 matrix instruction, g comes from the fp32
      * matrix instruction; the workspace also holds p in fp32.  Error of the product from the pieces
      * below 3 * 2^-22 sum_k |c a (b - s)| + k * 2^-38 max_k|a[k][m]| max_k|p[r][k]|.
      * NULL, too small, or a problem for which the query reports 0: the fp32 kernels run. */
@@ -466,8 +466,8 @@ int kmc_build_kernel_load_modes(const kmc_build_kernel_params *params, int32_t *
 int kmc_abi_version(void);
 /* The thresholds of the library's rules for its routes through a workspace (which
  * kmc_gram_workspace_bytes and kmc_norm_gradient_workspace_bytes apply) as text, one
- * "NAME = integer" per line, into buf (4096 bytes are enough).  A tile is 256 x 256 for the
- * matrix-core routes and 128 x 128 for the fixed-point one.  No counterpart in the reference. */
+ * "NAME = integer" per line, into buf (4096 bytes are enough).  Tiles are counted in 256 x 256 for the
+ * matrix-core routes and in 128 x 128 for the fixed-point one.  No counterpart in the reference. */
 int kmc_dispatch_rules(char *buf, size_t buf_len);
 /* Message of the last failing call on this thread ("" if none). */
 const char *kmc_last_error(void);

@@ -807,7 +807,7 @@ _L2_SAMPLE_MIN_TERMS = 4_000_000_000
 
 def _attach_gram_workspace(params, device, switch="KERMAC_AMD_L2_WORKSPACE"):
     """Large squared-difference problems in the split-bf16 mode go through a workspace (include/
-    kermac_amd.h, gram_workspace: both operands split once into fp16 pieces, then 256 x 256 tiles);
+    kermac_amd.h, gram_workspace: both operands split once into fp16 pieces, then their products);
     the library says how much it wants for this call, 0 when it would not use one.
     KERMAC_AMD_L2_WORKSPACE=0 keeps every call on the one-step kernel."""
     if os.environ.get(switch, "1") in ("", "0"):

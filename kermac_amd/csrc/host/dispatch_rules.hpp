@@ -4,7 +4,7 @@
 // kernels/norm_gradient_f16_inst.hip, gradient_l2_pays in kernels/gram_f16_wide_inst.hip) read them
 // from here, kmc_dispatch_rules() prints them, and the Python layer builds its "which kernel runs
 // when" table from that print-out.  Where each number comes from (the sweeps) is told next to the rule
-// that uses it.  A "tile" is 256 x 256 for the matrix-core routes and 128 x 128 for the fixed-point one.
+// that uses it.  Tiles are counted in 256 x 256 for the matrix-core routes and in 128 x 128 for the others, where a line does not say otherwise.
 #pragma once
 
 // X(name, value)

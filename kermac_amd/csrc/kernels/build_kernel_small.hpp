@@ -5,7 +5,7 @@
 // and a workgroup of 4 waves a tile of 64 x 64, so that the same result is four times the workgroups at a quarter of the
 // serial work each.  LDS then feeds half as many terms per byte, which is why large results stay with the other
 // tile.  Whole calls, 128 x 128 / 64 x 64 tiles, us: 1024 x 1024 p = 1 at K = 64 24 / 18, at K = 400 117 / 55;
-// p = 1.3 58 / 26 and 326 / 121; p = 2 at K = 64 24 / 20 (the host's share of a call is 17).
+// p = 1.3 58 / 26 and 326 / 121; p = 2 at K = 64 24 / 18, of which the kernel takes 14 and the host, call after call, 15 to 16.
 //
 // The terms, their order in every sum and the epilogue are those of build_kernel: the bits are the same.  Slices of 32 k, double
 // buffered.  The loaders are chosen at run time (uniform branches in front of a slice's loads): few launches are worth sixteen instantiations.  A

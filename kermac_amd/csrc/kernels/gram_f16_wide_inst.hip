@@ -38,9 +38,12 @@ struct WideLayout {
     int64_t bytes;
 };
 
-// Whether the route pays for its extra launches and its coarser tiles (a CU holds one workgroup of
-// 256 x 256, so a few hundred tiles do not fill the chip as evenly as four times as many of
-// 128 x 128).  From sweeps against the one-step kernel, one-step / wide time:
+// Whether the route pays for its extra launches.  Tiles are counted in 256 x 256, the rows that an operand is padded to.  The sweeps
+// against the one-step kernel below are of the product kernel before the present tiles of 256 x 128 and 128 x 128, one workgroup of
+// 256 x 256 per CU; the present one is faster almost everywhere, so that these lines keep some calls on a slower kernel and send hardly any to one
+// (one-step / route, us, today, calls that the rule leaves to the one-step kernel: k contiguous 1500 x 1500 x 784 102 / 50, 2000 x 2000 x 256
+// 60 / 41, 8 x 512 x 512 x 784 64 / 53, 100 x 50000 x 784 185 / 142; rows contiguous 2000 x 2000 x 2048 173 / 117, 3000 x 3000 x 784
+// 140 / 98, 1000 x 30000 x 256 161 / 111; the other way round, 16 x 512 x 512 x 2048 with k contiguous, 144 / 171).  One-step / wide time then:
 //   * over all tiles of the batch: K = 1024 1.09 at 144 tiles, 1.3 at 256, 1.6 from 1024 on; K = 256 0.99
 //     at 576, 1.15 at 1024, 1.25 at 4096; K = 64 1.0 at 1024, 1.07 from 2304 on; K = 32 never above 1;
 //   * the split of the operands is paid once per row and earned back once per tile the row meets, so
@@ -71,7 +74,7 @@ struct WideLayout {
 // A set against itself (the tiles of one triangle): one round of workgroups either way, whose walk is the route's faster one
 // (one-step split kernel / route, us, k contiguous: 1400 points, 21 tiles, at K = 784 77 / 63; 2000 at K = 256 66 / 52, at
 // K = 784 152 / 65, at K = 3072 502 / 160; 3000 at K = 128 59 / 50; 4 x 1000 at K = 784 163 / 67; 1000 at K = 784, 10 tiles, 63 / 61;
-// rows contiguous: 2000 at K = 784 82 / 85, at K = 3072 248 / 167; 2400 at K = 1024 106 / 90; 3500 at K = 512 95 / 88; 3000 at
+// rows contiguous: 2000 at K = 784 82 / 85, at K = 3072 248 / 167; 2400 at K = 1024 106 / 90; 3500 at K = 512 95 / 88, a hair below the line; 3000 at
 // K = 128 46 / 70).
 bool wide_pays(int64_t m, int64_t n, int64_t tiles_m, int64_t tiles_n, int64_t tiles, int k, bool products, bool k_contiguous,
                bool batched, bool symmetric)
@@ -369,8 +372,9 @@ hipError_t launch_gram_f16_wide(const kmc_build_kernel_params *p, const kmc::Bui
     const kmc::GramRowsArgs rows_b = rows_args(args.b, args.b_ld, args.b_bs, args.n, p->b_majorness, scalar_only, args, layout, layout.b, workspace);
     // The caller's trust rule grows with sqrt(k) (the error of a sum of k terms against the norms) and
     // passes 1 near k = 18000, where it would send every part to the repair launch -- whose own
-    // fp32 sum over k is no better by then (measured at k = 20000 .. 200000: this walk, which rounds once
-    // per 16 k, 4e-7 .. 2e-6 of d for points as far apart as their norms, the direct kernel 5e-6 .. 4e-5).
+    // fp32 sum over k is no better by then (measured at k = 20000 .. 200000: products of pieces, rounded once
+    // per 16 k, 4e-7 .. 2e-6 of d for points as far apart as their norms, the direct kernel 5e-6 .. 4e-5; the present walk, once per
+    // 32 k, as that one: largest error 5.7e-7 at k = 20000, 9.3e-7 at k = 60000).
     // With a product worth half the norms the two are equally good, so that is where the rule stops.
     kmc::GramWideArgs wide = {};
     wide.kernel = args;
@@ -439,11 +443,12 @@ struct GradientL2Layout {
 //                  outputs, 0.028 o up to 8 (vector kernels), 0.27 up to 16, 0.56 up to 32, 0.0175 o beyond
 //                  (matrix-core kernels: a run of outputs costs what its 16 or 32 columns cost);
 //   this route     200 + 1.5e-6 (o n + m) k l for the products and the two splits, and for the walk
-//                  6.3e-9 per multiply-add of the padded tiles (1.7 us per 256 x 256 x 16 step of a CU with the
-//                  chip full) but not less than 0.056 k (a CU alone walks a step in 0.9 us).
-// Examples (fp32 / this route, measured): 8192 x 512 x 16 x 8192 2.7; o = 1 .. 8 there 2.8 .. 4.0; n = 64 1.75,
-// n = 32 0.96, n = 8 0.81; m = 1024 1.55, m = 512 0.86; k = 512 1.35, k = 256 0.92, k = 64 0.40;
-// 10000 x 1000 x 10 x 784 2.6.  KERMAC_AMD_GRADIENT_L2_MIN_TERMS replaces the rule by a number of terms
+//                  6.3e-9 per multiply-add of the padded tiles but not less than 0.056 k (fitted to the product kernel before
+//                  the present tiles: 1.7 us per 256 x 256 x 16 step of a CU with the chip full, 0.9 us alone; the present one takes
+//                  4.7e-9 with the chip full, so the rule leaves a few calls to the fp32 kernels that it would win).
+// Examples (fp32 / this route, measured with the present kernel): 8192 x 512 x 16 x 8192 3.0; o = 1 4.3, o = 32 3.2; n = 64 1.65;
+// m = 1024 1.6; k = 512 1.8, k = 256 1.2; 10000 x 1000 x 10 x 784 3.4.  With the kernel before: n = 32 0.96, n = 8 0.81;
+// m = 512 0.86; k = 64 0.40.  KERMAC_AMD_GRADIENT_L2_MIN_TERMS replaces the rule by a number of terms
 // (read on every call, so that a test can send small shapes down the route).
 bool gradient_l2_pays(const kmc_norm_gradient_params *p, int64_t tiles_m, int64_t tiles_n)
 {

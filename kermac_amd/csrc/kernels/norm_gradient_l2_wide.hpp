@@ -9,7 +9,7 @@
 // out and cancelled).  The second term is a product of an (O N) x K matrix with a K x M one: the
 // rows of p and the columns of a are split into two fp16 pieces per value with a scale per row,
 // exactly as the squared-difference route does it (gram_f16_wide.hpp), and the same kernel walks
-// the pieces (GW_EPILOGUE_GRADIENT_L2: three piece products per 16 k); its epilogue fetches d and g
+// the pieces (GW_EPILOGUE_GRADIENT_L2: three piece products per 32 k); its epilogue fetches d and g
 // and stores e.  Where the fp32 kernels build c a (d - b) value by value on the vector ALU and
 // contract it on the fp32 matrix instruction, this route has no work per (o, n, m, k) outside the
 // matrix instruction.  Error of the product from the pieces below 3 * 2^-22 sum_k |c a (b - s)|;

@@ -179,7 +179,7 @@ def _partial_products(parts, plan, device):
 
 
 # Squared differences and sums of products on the matrix cores: the route of kmc_build_kernel through a workspace
-# (operands split once into fp16 pieces, 256 x 256 tiles) builds the kernel matrix several times
+# (operands split once into fp16 pieces) builds the kernel matrix several times
 # faster than the fused kernel walks it, so a large product is taken panel by panel instead: the
 # kernel matrix of all rows against a few thousand centres is written into a buffer that is
 # reused, and kmc_matrix_times_coefficients contracts it with the coefficients of those centres.
@@ -445,7 +445,7 @@ def _run_in_panels(plan, shape, stream, device, debug):
 # into the result for the first panel and into a buffer that is added to the result for the others.  Gaussian
 # kernel, fp32 contraction -> pieces: L = 4, M = N = 16384, K = 256 at O = 256 9.6 -> 8.1 ms, O = 512 15.6 -> 9.4,
 # O = 1000 25.5 -> 12.0; M = 10000, N = 100000, K = 784, O = 1000 28.5 -> 17.2 ms.  The split of a panel costs what
-# its fp32 contraction with 64 columns does, and the product runs in tiles of 256 x 256 over (o, m): not below 256
+# its fp32 contraction with 64 columns does, and its rows o and m are padded to 256: not below 256
 # columns (O = 128: 6.7 -> 7.8 ms) nor below 128 tiles over the batch (M = 10000, O = 256, 40 tiles: 12.3 -> 16.1 ms;
 # M = 2000, O = 1000, 32 tiles: 1.2 -> 2.0 ms).  KERMAC_AMD_COEFFICIENT_PIECES_MIN_COLUMNS replaces both conditions
 # by a number of columns (tests send small shapes this way with 1).

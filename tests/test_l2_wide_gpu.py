@@ -1,7 +1,7 @@
 """GPU tests of the route that large squared-difference problems take in the split-bf16 mode when
 the caller brings a workspace (include/kermac_amd.h, gram_workspace): row statistics, both
 operands split once into two fp16 pieces per value with a power-of-two scale per row, then
-256 x 256 tiles on the fp16 matrix instruction.  Same stated tolerance as every p = 2 path: 1e-5
+their products on the fp16 matrix instruction, in both tiles of the product kernel.  Same stated tolerance as every p = 2 path: 1e-5
 relative to the float64 truth -- trusted 128 x 128 parts by the error bound of the expansion,
 distrusted parts because the direct kernel recomputes them.
 
