@@ -47,10 +47,6 @@ struct BuildKernelArgs {
     int repair_only;     // recompute only the tiles that carry BK_REPAIR_MARKER (see gram_kernel.hpp)
     int symmetric;       // A and B are the same panel and the result is symmetric: only tiles with
                          // tile_m >= tile_n are computed, each is also stored mirrored
-    // gram_f16_wide.hpp and gram_bf16_kernel.hpp: with same_points, row m of a and row n of b are the same row in memory
-    // where m == n + same_shift (a set against itself or against a run of its own rows): their distance is zero, which
-    // |a|^2 + |b|^2 - 2 a.b cannot tell.
-    int same_points, same_shift;
     float gram_trust;    // gram_kernel.hpp: distrust d^2 below gram_trust * (|a|^2 + |b|^2)
     int k_total;         // 0, or: the batch entries are consecutive ranges of k terms of one contraction of
                          // k_total terms, and the last entry walks only what is left
@@ -66,6 +62,10 @@ struct BuildKernelArgs {
     // kernel, which therefore runs whatever the size of the problem.  BK_PANELS_B_PADDED: the rows of b hold n rounded
     // up to 16 columns (zeros past n), so that a wave's 16 columns can always be loaded; columns below n are stored.
     int panels;
+    // gram_f16_wide.hpp and gram_bf16_kernel.hpp: with same_points, row m of a and row n of b are the same row in memory
+    // where m == n + same_shift (a set against itself or against a run of its own rows): their distance is zero, which
+    // |a|^2 + |b|^2 - 2 a.b cannot tell.  (The last fields, so that kernels that know nothing of them are compiled as they were.)
+    int same_points, same_shift;
 };
 
 constexpr int BK_PANELS_COPIED = 1;
