@@ -284,16 +284,16 @@ def bench_cdist_grad(kermac, device, args, steps=None, warmup=None):
     del out32
     log(f"  p=1, 32 outputs: {o32_ms:.2f} ms (slab err {o32_err:.2e}); on the fp32 matrix-core kernel {o32_fp32_ms:.2f} ms")
     check_parity("cdist_grad p=1, 32 outputs, slab, max abs err / mean |truth|", o32_err, 1e-4)
-    # Executed matrix work on the default route: three products of fp16 pieces, 2 * O flops each per (m, n, k),
-    # against the dense fp16 peak; the sign work on the vector ALU (2.5 instructions per (m, n, k)) is what bounds it.
-    ops = 3.0 * 2.0 * o * m_ref * n_ref * k_ref
+    # Executed matrix work on the default route: two products (the signs as 0 or 1, times a c in two fp16 pieces), 2 * O flops
+    # each per (m, n, k), against the dense fp16 peak; vector instructions beside the matrix ones (3.3 for each) are what bounds it.
+    ops = 2.0 * 2.0 * o * m_ref * n_ref * k_ref
     nbytes = 4.0 * (k_ref * m_ref + n_ref * k_ref + o * k_ref + n_ref * m_ref + o * n_ref * m_ref)
     return side_line("cdist_grad ms, Laplace-kernel RFM gradient M=8192 N=512 O=16 K=8192 p=1",
                      "cdist_grad p=1.0 fp32: a[8192,8192] U(0,1), b[512,8192], d[512,8192] N(0,1)/sqrt(512), "
                      "c[16,8192] N(0,1), out[16,512,8192] (BASELINE configs[3])",
                      wall_ms, kernel_ms, ops, nbytes, "mfma", 2500.0,
                      {"parity_max_err_over_mean": err, "tolerance": 1e-4,
-                      "route": "a and c split once into two fp16 pieces per value, sign of d - b on the pieces, v_mfma_f32_16x16x32_f16",
+                      "route": "rows of b and d ranked, d >= b as an exact 0 or 1 times a c in two fp16 pieces, v_mfma_f32_16x16x32_f16",
                       "useful_tflops": round((2.0 * o + 3.0) * m_ref * n_ref * k_ref / kernel_ms / 1e9, 2),
                       "fp32_kernels_same_run": {"ms": round(fp32_ms, 3), "parity_max_err_over_mean": fp32_err,
                                                 "frac_of_fp32_mfma_peak": round((2.0 * o + 3.0) * m_ref * n_ref * k_ref / fp32_ms / 1e9 / 157.3, 4)},
@@ -303,7 +303,7 @@ def bench_cdist_grad(kermac, device, args, steps=None, warmup=None):
                                            "mfma_tflops": round(3.0 * 2.0 * o * m_ref * n_ref * k_ref / l2_ms / 1e9, 2),
                                            "fp32_kernels_ms": round(l2_fp32_ms, 3), "fp32_kernels_parity_max_err_over_mean": l2_fp32_err},
                       "p1_32_outputs": {"ms": round(o32_ms, 3), "parity_max_err_over_mean": o32_err, "fp32_kernels_ms": round(o32_fp32_ms, 3),
-                                        "route": "tiles of 64 m x 16 n x 32 outputs: the signed pieces meet two blocks of 16 outputs"}},
+                                        "route": "two blocks of 16 outputs"}},
                      args)
 
 

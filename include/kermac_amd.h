@@ -336,9 +336,9 @@ typedef struct kmc_norm_gradient_params {
     const float *p; int64_t p_bs; float p_value;
     /* KMC_NORM_L1 and KMC_NORM_L2 (ignored otherwise): device memory the call may use, 256-byte
      * aligned, of at least the size kmc_norm_gradient_workspace_bytes reports for these parameters.
-     * With it, large problems run on the fp16 matrix instruction.  KMC_NORM_L1: a and c are split once into two fp16 pieces per
-     * value (a power-of-two scale per row m of a and per row o of c), the sign of d - b is put on
-     * the pieces of a exactly, and the contraction takes 3 matrix instructions per 32 k where the
+     * With it, large problems run on the fp16 matrix instruction.  KMC_NORM_L1: the rows n of b and d are
+     * ranked, so that d >= b is a comparison of 16-bit numbers, 0 or 1 and exact; its product with a * c, in two fp16
+     * pieces (a power-of-two scale per row m of a and per row o of c), takes 2 matrix instructions per 32 k where the
      * fp32 kernel issues 8 of twice the duration.  Error of e from the pieces below
      * 3 * 2^-22 sum_k |c a|, beside the rounding of the fp32 accumulation that both kernels have.
      * KMC_NORM_L2 with e_ld_o = n * e_ld_n (the planes of e one matrix of o * n rows): large problems

@@ -170,6 +170,10 @@ def cdist_grad(
     return plan.out
 
 
+def _workspace_enabled():
+    return os.environ.get("KERMAC_AMD_GRADIENT_WORKSPACE", "1") not in ("", "0")
+
+
 def _attach_workspace(params, device):
     """Large L1 and L2 gradients run on the fp16 matrix instruction through a workspace (include/
     kermac_amd.h, kmc_norm_gradient_params::workspace.  L1: a and c split once into two fp16 pieces
@@ -177,7 +181,7 @@ def _attach_workspace(params, device):
     (d - s) (c a) - (c (b - s)) a, one product of pieces); the library says how much it wants for
     this call, 0 when it would not use one.  KERMAC_AMD_GRADIENT_WORKSPACE=0 keeps every call on
     the fp32 kernels."""
-    if os.environ.get("KERMAC_AMD_GRADIENT_WORKSPACE", "1") in ("", "0"):
+    if not _workspace_enabled():
         return None
     needed = _backend.norm_gradient_workspace_bytes(params)
     if needed == 0:
@@ -203,6 +207,14 @@ _SPLIT_TARGET_WORKGROUPS = 3072
 _SPLIT_MIN_DEPTH = 512                      # from 512 workgroups on: 1024, and 2048 for the matrix-core kernels
 _SPLIT_MAX_SLICES = 24
 _SPLIT_MAX_PARTIAL_BYTES = 512 << 20
+# Calls that go to the fp16 matrix instruction (p = 1, a workspace granted): its workgroups own 16 (m) x 128 (n) x 16 (o)
+# results or more, one per CU at a time, and every slice ranks its rows again, so fewer slices are wanted: 2000 x 24 x 16 x 9000 in
+# 17 slices 166 us, in 5 147; 200 x 1000 x 16 x 12000 in 12 472, in 5 401.
+_SPLIT_F16_TARGET_WORKGROUPS = 512
+
+
+def _takes_f16_route(params):
+    return params.norm_type == _NORM_L1 and _workspace_enabled() and _backend.norm_gradient_workspace_bytes(params) > 0
 
 
 def _split_over_contraction(plan):
@@ -215,7 +227,11 @@ def _split_over_contraction(plan):
     min_depth = _SPLIT_MIN_DEPTH * (1 if workgroups < 512 else 2 if O <= 8 else 4)
     if workgroups >= _SPLIT_BELOW_WORKGROUPS or K < 2 * min_depth:
         return None
-    slices = min(max(2, round(_SPLIT_TARGET_WORKGROUPS / workgroups)), K // min_depth, _SPLIT_MAX_SLICES,
+    wanted = max(2, round(_SPLIT_TARGET_WORKGROUPS / workgroups))
+    if _takes_f16_route(plan.params):
+        f16_workgroups = -(-M // 16) * -(-N // 128) * -(-O // 16)
+        wanted = -(-_SPLIT_F16_TARGET_WORKGROUPS // f16_workgroups)
+    slices = min(wanted, K // min_depth, _SPLIT_MAX_SLICES,
                  _SPLIT_MAX_PARTIAL_BYTES // (4 * O * N * M) - 1)
     if slices < 2:
         return None

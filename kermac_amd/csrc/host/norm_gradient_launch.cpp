@@ -8,8 +8,7 @@ namespace kmc_host {
 hipError_t launch_norm_gradient(int norm_type, int o_tile, const kmc::NormGradientArgs &args, dim3 grid,
                                 hipStream_t stream);
 int64_t norm_gradient_f16_bytes(const kmc_norm_gradient_params *p);
-hipError_t launch_norm_gradient_f16(const kmc_norm_gradient_params *p, bool a_vec, bool c_vec, bool e_vec, hipStream_t stream,
-                                    bool *taken);
+hipError_t launch_norm_gradient_f16(const kmc_norm_gradient_params *p, bool a_vec, bool e_vec, hipStream_t stream, bool *taken);
 int64_t norm_gradient_l2_wide_bytes(const kmc_norm_gradient_params *p);
 int launch_norm_gradient_l2_wide(const kmc_norm_gradient_params *p, hipStream_t stream, bool *taken);
 }
@@ -66,9 +65,8 @@ extern "C" int kmc_norm_kernel_gradient(const kmc_norm_gradient_params *p, void 
         int ready = require_gfx950();
         if (ready != KMC_OK) return ready;
         bool taken = false;
-        hipError_t e = launch_norm_gradient_f16(p, vec_ok(p->a, p->a_ld, p->a_bs, 0, p->flags), vec_ok(p->c, p->c_ld, p->c_bs, 0, p->flags),
-                                                vec_ok(p->e, p->e_ld_n, p->e_ld_o, p->e_bs, p->flags), static_cast<hipStream_t>(stream),
-                                                &taken);
+        hipError_t e = launch_norm_gradient_f16(p, vec_ok(p->a, p->a_ld, p->a_bs, 0, p->flags),
+                                                vec_ok(p->e, p->e_ld_n, p->e_ld_o, p->e_bs, p->flags), static_cast<hipStream_t>(stream), &taken);
         if (e != hipSuccess) return fail_hip(e, "norm_gradient_l1_f16 launches");
         if (taken) return KMC_OK;
     }

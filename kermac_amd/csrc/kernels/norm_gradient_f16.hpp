@@ -3,48 +3,39 @@
 //   E[m, n, o, l] = sum_k C[o,k,l] * A[m,k,l] * s(m,n,k),     s = copysign(1, D[m,n,l] - B[n,k,l])
 //
 // (reference: include/p_norm_gradient.cuh:407-497 with NormType::L1, whose weight of a term is
-// the sign of d - b, :373-394).  The factor that depends on all of m, n and k is a sign, and a
-// sign can be put on a 16-bit piece exactly.  So A and C are split once, like the operands of
-// gram_f16_wide.hpp and by the same two kernels (a power-of-two scale per row m of A and per row
-// o of C, two fp16 pieces per scaled value, 16-byte chunks of 8 k in the order the matrix
-// instruction reads them), and the contraction over k runs on v_mfma_f32_16x16x32_f16 with
+// the sign of d - b, :373-394).  For a fixed m this is a product of two matrices,
 //
-//   T1 = +-a1, T2 = +-a2 (the sign bit of d - b flipped into both pieces),   T1 c1 + T1 c2 + T2 c1
+//   E[n, o] = sum_k (2 S[n, k] - 1) * W[k, o],     S = 1 where d >= b and 0 where not,    W[k, o] = A[m, k] * C[o, k],
 //
-// per 32 k: 3 matrix instructions of 16 cycles where the fp32 kernel (norm_gradient_mfma.hpp)
-// issues 8 of 32 cycles.  What a lane computes per (m, n, k) is one subtraction, half a byte
-// permute, half an AND and two halves of an XOR: 3 vector instructions, as many as the fp32
-// kernel spends, which now bound the kernel instead of the matrix pipeline.
-// Accuracy: as in gram_f16_wide.hpp, |x - h1 - h2| <= 2^-22 |x| per value and the dropped product
-// a2 c2 below 2^-22 |a c|: the error of E from the pieces is below 3 * 2^-22 sum_k |c a|, the size
-// of the rounding of an fp32 accumulation over a few terms, beside the fp32 accumulation itself.
+// whose left operand is exact in 16 bits.  W is what has to be split into two fp16 pieces, and it is made once per
+// (m, k, o) and meets every n, so a term (m, n, k) costs two matrix instruction slots (S w1 + S w2) and half a vector
+// instruction for S:
 //
-// Workgroup: 4 waves, 64 m x 32 n x 16 o (for more than 16 outputs 64 m x 16 n x 32 o or 64 m x 8 n x 64 o,
-// below); wave w owns the 8 (4, 2) n  8w .. 8w + 7  and all 64 m as 4 row blocks of 16.  Per 32 k it reads the pieces of C (2 x 16 bytes per lane) and of its A rows
-// (8 x 16 bytes), and per n the 8 values of B that match its 8 k (2 x 16 bytes, the same for the
-// 16 lanes of a row block).  B is copied once into a padded array in the workspace (rows to 32,
-// k to 32 plus what the walk copies ahead), so that everything the walk touches exists and all of
-// it arrives in LDS by global_load_lds_dwordx4, three steps in three buffers, as in
-// gram_f16_wide.hpp (the copies are inline instructions for the reason given there).
+// gradient_signs_prepare   per row n of B: the position of every b[n, k] in the sorted row, and for every d[n, m] how
+//                          many b of the row are not above it.  d >= b is then position < count, for integers below
+//                          14335, written as fp16 numbers that lie at least 1 apart (signs_half): one packed
+//                          subtraction with the clamp to [0, 1] compares two k and gives S in fp16.  The keys that are
+//                          sorted order -0 below +0, so that signed zeros and ties come out as copysign(1, d - b).
+//                          Rows of B longer than that are cut into chunks with positions of their own.
+//                          The same launch copies A into the order in which a wave reads it (and takes the largest
+//                          magnitude of every row m), and scales C by a power of two per row o.
+// norm_gradient_l1_f16     the product.
 //
-// Measured at M = K = 8192, N = 512, O = 16: 3.86 ms (O = 32 on the second shape 5.4 ms, O = 64 on the third 9.2 ms) for this kernel and 0.33 ms for the row kernels
-// against 9.85 ms on the fp32 kernels.  Counters: 2.5 vector instructions per (m, n, k) (the
-// compiler fuses AND and XOR into v_bitop3_b32), the matrix pipeline busy 46 % and the vector
-// pipeline about 44 % of the elapsed cycles, hardly ever together, shader clock 1.75 GHz.  Tried
-// against that and not kept: matrix instructions alternating between two accumulators (3.99 ms,
-// the same), a software pipeline that makes the pieces of the next (n, row block) between the three
-// matrix instructions of this one, pinned with scheduling groups (co-issue rises to 47 % of the
-// matrix cycles, but the kernel takes more cycles: 4.1 .. 4.3 ms), D parked in LDS to free registers.
-// Two compile-time switches leave a part of the walk out, for the measurement of what bounds it (the results are
-// then wrong): -DNGF_ABLATE_NO_SIGN multiplies the pieces of A as they are, -DNGF_ABLATE_NO_MFMA makes the signed
-// pieces and issues no matrix instruction.  Measured with them at M = K = 8192, N = 512, O = 16: matrix instructions and
-// copies alone 2.01 ms (3.46e6 cycles at 1.72 GHz, the matrix pipeline busy 91 % of them), sign work and copies alone
-// 2.04 ms (4.17e6 cycles at 2.05 GHz), both 3.72 ms (6.83e6 cycles at 1.84 GHz): the two parts take nine tenths of
-// the sum of their cycles, whichever wave they come from -- a source-level pipeline that puts the vector work of pair
-// i + 1 between the three dependent matrix instructions of pair i (one matrix instruction, seven vector instructions,
-// three times; 255 registers) took 4.28 ms against 4.12 ms on the same box.  This 16-bit matrix instruction and the
-// vector ALU do not run side by side here; the kernel is at the sum of two floors, each already at its minimum of
-// instructions (2.5 vector instructions per (m, n, k) without packed fp32; three piece products).
+// Accuracy: S is exact, a = a1 + a2 and c = c1 + c2 to 2^-22, w1 = fp16(a1 c1) and w2 = a1 c1 - w1 + a1 c2 + a2 c1 in fp16: below
+// 3 * 2^-22 |w| together, beside the fp32 accumulation.  The sums run over S W, so  1/2 sum_k W  is taken off them again: every 256
+// k, since a partial sum of S W alone drifts away from the one of the signed terms, and rounding follows the partial sums.
+//
+// Workgroup of norm_gradient_l1_f16: 8 waves, 16 m x 16 BLOCKS n x 16 o; wave w owns the 2 m  2w, 2w + 1  and all n, as
+// BLOCKS x 2 results of v_mfma_f32_16x16x32_f16 (rows n, columns o).  The more n a wave holds, the less W costs: at 256
+// n the 64 matrix instructions of a step of 32 k stand beside 128 packed subtractions and about 75 other instructions.
+// Bound by the two together: on registers alone a v_mfma_f32_16x16x32_f16 takes 16.5 cycles, 16.9 with two packed
+// subtractions beside it, and four more for every further vector instruction; the kernel takes about 26.
+// Measured at M = K = 8192, N = 512, O = 16: 1.9 ms with 0.19 ms of gradient_signs_prepare (3.65 ms for the kernel that
+// flipped the sign into both pieces of A: three products and 2.5 vector instructions per term), O = 32 3.7 ms (5.55).
+// Up to 8 outputs leave half of the columns unused: there the columns 8 .. 15 take the second pieces (PIECES_IN_COLUMNS),
+// one matrix instruction instead of two.  Everything a step reads arrives in LDS by global_load_lds, a stage of 64 k in
+// one of two buffers while the other is worked on; the copies are inline instructions for the reason given in
+// gram_f16_wide.hpp.
 #pragma once
 
 #include "gram_f16_wide.hpp"
@@ -54,266 +45,612 @@ namespace kmc {
 
 typedef float ngf_float4 __attribute__((ext_vector_type(4)));
 
-constexpr int NGF_TILE_M = 64;
-constexpr int NGF_STEP_K = 32;                 // two slices of the split
-constexpr int NGF_THREADS = 256;
-constexpr int NGF_AHEAD = 3;                   // steps copied ahead of the walk
-constexpr int NGF_N_PAD = 32;                  // rows of the padded copy of B come in whole multiples of this
-
-// Three shapes of the workgroup's tile, 64 m in all: 32 n x 16 o (O_BLOCKS = 1), 16 n x 32 o
-// (O_BLOCKS = 2) and 8 n x 64 o (O_BLOCKS = 4).  The signed pieces of A are made once per (m, n, k)
-// and meet every block of 16 outputs, so with more outputs the wider shapes divide the vector work
-// per result, which is what bounds the first (17 to 32 outputs: one pass instead of two of 16).
-template <int O_BLOCKS>
-struct GradientF16Tile {
-    static constexpr int TILE_N = 32 / O_BLOCKS;
-    static constexpr int TILE_O = 16 * O_BLOCKS;
-    static constexpr int WAVE_N = TILE_N / 4;
-    static constexpr int A_CHUNKS = 8 * NGF_TILE_M;    // per step: 8 runs (slice, piece, half) of 64 rows
-    static constexpr int C_CHUNKS = 8 * TILE_O;
-    static constexpr int B_CHUNKS = TILE_N * NGF_STEP_K / 4;
-    static constexpr int BUFFER_CHUNKS = A_CHUNKS + C_CHUNKS + B_CHUNKS;      // 14 KB (17 KB for 64 outputs)
-    static constexpr int COPIES = O_BLOCKS == 4 ? 5 : 4;                       // per wave and step
-};
+constexpr int NGF_STEP_K = 32;
+constexpr int NGF_STAGE_K = 64;                // two steps
+constexpr int NGF_WAVES = 8;
+constexpr int NGF_TILE_M = 2 * NGF_WAVES;
+constexpr int NGF_TILE_O = 16;
+constexpr int NGF_THREADS = 64 * NGF_WAVES;
+constexpr int NGF_N_PAD = 256;
+constexpr int NGF_CORRECT_STAGES = 4;          // 1/2 sum W is taken off every so many stages
+constexpr int NGF_PREPARE_THREADS = 256;
+constexpr int NGF_PREPARE_GROUP = 256;
+constexpr int NGF_COPY_M = 64;                 // tile of the copy of A: m, and k per workgroup
+constexpr int NGF_COPY_K = 512;
+constexpr float NGF_SCALE_A = 0x1p-7f;         // of what gram_scale gives (2^14 .. 2^15): A in [2^7, 2^8), C in [2^6, 2^7),
+constexpr float NGF_SCALE_C = 0x1p-8f;         // and W below 2^15
+constexpr int NGF_MAX_CHUNK = 14272;           // k per sorted chunk: whole stages, counts up to 14334 (signs_half)
 
 struct NormGradientF16Args {
-    NormGradientArgs g;                        // extents, d, e, strides, o_chunks (of the tile's outputs); a, b, c are not read
+    NormGradientArgs g;                        // extents, d, e, strides, o_chunks; a, b, c are not read
     int o_begin;                               // the launch covers the outputs from here on
-    const gram_chunk *pieces_a, *pieces_c;     // gram_f16_split of A (rows m) and of C (rows o)
-    i64 pieces_a_bs, pieces_c_bs;              // per batch entry, in chunks
-    const float *unscale_a, *unscale_c;
-    i64 unscale_a_bs, unscale_c_bs;
-    const float *b_padded;                     // [batch][n_pad][k_pad]
-    i64 b_padded_bs;
-    int rows_pad_a, rows_pad_c, k_pad, steps;
+    const unsigned short *positions;           // [batch][k / 8][n_pad][8]: of b in its sorted row
+    const unsigned short *counts;              // [batch][chunk][n_pad][m_pad]: b not above d
+    i64 positions_bs, counts_bs;               // in halves
+    const float *a_copy; i64 a_copy_bs;        // [batch][m_pad / 2][k_pad / 32][4][2][8]: 8 k of each of 2 m, 4 times
+    const float *a_magnitudes; i64 a_magnitudes_bs;    // [batch][ranges][m_pad]
+    const gram_chunk *c_pieces; i64 c_pieces_bs;       // [batch][o_pad / 16][k_pad / 8][2 pieces][16 o] of 8 k
+    const float *c_unscale; i64 c_unscale_bs;  // [batch][o_pad]
+    int n_pad, m_pad, k_pad, ranges;
+    int chunks, chunk_stages, stages;          // sorted chunks, their length (the last may be shorter), all stages
 };
 
-struct GradientPadArgs {
+struct GradientPrepareArgs {
+    int m, n, o, k;
+    const float *a; i64 a_ld, a_bs;
     const float *b; i64 b_ld, b_bs;
-    float *padded; i64 padded_bs;
-    int n, k, n_pad, k_pad;
+    const float *c; i64 c_ld, c_bs;
+    const float *d; i64 d_ld, d_bs;
+    unsigned short *positions, *counts; i64 positions_bs, counts_bs;
+    float *a_copy; i64 a_copy_bs;
+    float *a_magnitudes; i64 a_magnitudes_bs;
+    gram_chunk *c_pieces; i64 c_pieces_bs;
+    float *c_unscale; i64 c_unscale_bs;
+    int n_pad, m_pad, k_pad, o_pad, ranges, chunks, chunk_k;
+    int sort_d;                                // the rows of D are sorted, not those of B
+    int sort_blocks, copy_blocks;              // rows to sort, tiles of A, ...
+    int sort_groups, copy_groups;              // ... and how many groups of NGF_PREPARE_GROUP that makes; blockIdx.x also has the rows of C
+    int sort_batches, a_batches, c_batches;    // blockIdx.y
+    int a_vec;
 };
 
-// padded[batch][n][k] = b[batch][n][k], zeros beyond n and k.  One thread per 4 k.
-__global__ __launch_bounds__(256) void gradient_pad_b(const GradientPadArgs args)
+// The integer count - 7167, count in 0 .. 14334, as an fp16 number: itself up to 2048, and beyond that the next larger
+// fp16 numbers in turn, which lie 2, 4, .. 32 apart.  Larger counts give larger numbers, at least 1 larger.
+__device__ __forceinline__ unsigned signs_half(int count)
 {
-    const int quad = blockIdx.x * 256 + threadIdx.x;
-    const int n = blockIdx.y, batch = blockIdx.z;
-    if (quad * 4 >= args.k_pad) return;
-    const float *src = args.b + batch * args.b_bs + (i64)n * args.b_ld;
-    float v[4];
-#pragma unroll
-    for (int e = 0; e < 4; e++) v[e] = (n < args.n && quad * 4 + e < args.k) ? src[quad * 4 + e] : 0.0f;
-    *reinterpret_cast<float4 *>(args.padded + batch * args.padded_bs + (i64)n * args.k_pad + quad * 4) = make_float4(v[0], v[1], v[2], v[3]);
+    const int centred = count - 7167;
+    const unsigned magnitude = (unsigned)abs(centred);
+    const unsigned exact = __builtin_bit_cast(unsigned short, (_Float16)(float)magnitude);
+    const unsigned bits = magnitude < 1024 ? exact : 0x6000 + magnitude;      // 1024 is 0x6400
+    return bits | (centred < 0 ? 0x8000u : 0u);
 }
 
-template <int O_BLOCKS>
-__global__ __launch_bounds__(NGF_THREADS, 2) void norm_gradient_l1_f16(const NormGradientF16Args args)
+// Unsigned integers in the order of copysign(1, d - b): -0 below +0, everything else as the floats
+__device__ __forceinline__ unsigned signs_key(float x)
 {
-    using Tile = GradientF16Tile<O_BLOCKS>;
-    constexpr int WAVE_N = Tile::WAVE_N;
-    __shared__ gram_chunk lds0[Tile::BUFFER_CHUNKS];
-    __shared__ gram_chunk lds1[Tile::BUFFER_CHUNKS];
-    __shared__ gram_chunk lds2[Tile::BUFFER_CHUNKS];
+    const int bits = __float_as_int(x);
+    return (unsigned)(bits ^ ((bits >> 31) & 0x7fffffff)) ^ 0x80000000u;
+}
+
+// LDS word of element i of the sorted row: a word of padding in 32, or lanes that own consecutive runs meet in few banks
+__device__ __forceinline__ int signs_word(int i)
+{
+    return i + (i >> 5);
+}
+
+// Bitonic sort of 256 << LOG_R keys by 256 threads, LOG_R strides per pass through LDS: the 1 << LOG_R keys that a
+// thread holds differ in the bits lo .. lo + LOG_R - 1 of their index.  (8192 keys: 19 passes instead of 91.)
+template <int LOG_R>
+__device__ __forceinline__ void signs_sort(unsigned (&key)[1 << LOG_R], unsigned *sorted, int tid)
+{
+    constexpr int R = 1 << LOG_R;
+    constexpr int LOG_N = 8 + LOG_R;
+    auto compare = [&](int low, int high, bool descending) {
+        const unsigned smaller = min(key[low], key[high]), larger = max(key[low], key[high]);
+        key[low] = descending ? larger : smaller;
+        key[high] = descending ? smaller : larger;
+    };
+    // the keys arrive as consecutive runs of R: the first LOG_R levels need no exchange
+#pragma unroll
+    for (int level = 1; level <= LOG_R; level++)
+#pragma unroll
+        for (int bit = level - 1; bit >= 0; bit--)
+#pragma unroll
+            for (int e = 0; e < R; e++)
+                if (!(e >> bit & 1)) compare(e, e | 1 << bit, level == LOG_R ? (tid & 1) : (e >> level & 1));
+#pragma unroll
+    for (int e = 0; e < R; e++) sorted[signs_word(tid * R + e)] = key[e];
+    for (int level = LOG_R + 1; level <= LOG_N; level++) {
+        for (int high = level - 1; high >= 0;) {
+            const int lo = max(high - LOG_R + 1, 0);
+            const int first = (tid & ((1 << lo) - 1)) | (tid >> lo) << (lo + LOG_R);
+            const bool descending = first >> level & 1;
+            __syncthreads();
+#pragma unroll
+            for (int e = 0; e < R; e++) key[e] = sorted[signs_word(first + (e << lo))];
+#pragma unroll
+            for (int bit = LOG_R - 1; bit >= 0; bit--) {
+                if (bit > high - lo) continue;
+#pragma unroll
+                for (int e = 0; e < R; e++)
+                    if (!(e >> bit & 1)) compare(e, e | 1 << bit, descending);
+            }
+#pragma unroll
+            for (int e = 0; e < R; e++) sorted[signs_word(first + (e << lo))] = key[e];
+            high = lo - 1;
+        }
+    }
+    __syncthreads();
+}
+
+// How many of the 256 << LOG_R sorted keys are below x (NOT_ABOVE: not above x), for eight x side by side
+template <int LOG_R, bool NOT_ABOVE>
+__device__ __forceinline__ void signs_search(const unsigned *sorted, const unsigned (&x)[8], int (&count)[8])
+{
+#pragma unroll
+    for (int j = 0; j < 8; j++) count[j] = 0;
+    for (int half = 128 << LOG_R; half >= 1; half >>= 1) {
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const unsigned key = sorted[signs_word(count[j] + half - 1)];
+            if (NOT_ABOVE ? key <= x[j] : key < x[j]) count[j] += half;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        const unsigned key = sorted[signs_word(count[j])];       // at most the last one
+        if (NOT_ABOVE ? key <= x[j] : key < x[j]) count[j]++;
+    }
+}
+
+__device__ __forceinline__ gram_chunk signs_pack(const int (&count)[8])
+{
+    gram_chunk packed;
+#pragma unroll
+    for (int j = 0; j < 4; j++) packed[j] = signs_half(count[2 * j]) | signs_half(count[2 * j + 1]) << 16;
+    return packed;
+}
+
+// A row n of B and of D; the shorter one is sorted, the other one (and the sorted one itself) searched in it.  With b
+// sorted: position = how many b are below b[k], count = how many b are not above d[m].  With d sorted: position = how
+// many d are below b[k], count = 1 + how many d are below d[m].  Both ways count > position exactly if d >= b, equal keys
+// included.  Bound by LDS (the sort, then log2 of its length dependent reads per element searched).
+template <int LOG_R>
+__device__ __forceinline__ void signs_rank_row(const GradientPrepareArgs &args, int block, int batch, unsigned *sorted)
+{
+    constexpr int R = 1 << LOG_R;
+    const int tid = threadIdx.x;
+    const int n = block % args.n, chunk = block / args.n;
+    const int k0 = chunk * args.chunk_k;
+    const int ks = min(args.chunk_k, args.k - k0);
+    const int span = min(args.chunk_k, args.k_pad - k0);
+    const float *b_row = args.b + batch * args.b_bs + (i64)n * args.b_ld + k0;
+    const float *d_row = args.d + batch * args.d_bs + (i64)n * args.d_ld;
+    const float *sorted_row = args.sort_d ? d_row : b_row;
+    const int keys = args.sort_d ? args.m : ks;
+    {
+        unsigned key[R];
+#pragma unroll
+        for (int e = 0; e < R; e++) key[e] = tid * R + e < keys ? signs_key(sorted_row[tid * R + e]) : ~0u;
+        signs_sort<LOG_R>(key, sorted, tid);
+    }
+    gram_chunk *positions = reinterpret_cast<gram_chunk *>(args.positions + batch * args.positions_bs) + (i64)(k0 / 8) * args.n_pad + n;
+    for (int k = 8 * tid; k < span; k += 8 * NGF_PREPARE_THREADS) {
+        unsigned x[8];
+        int position[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) x[j] = k + j < ks ? signs_key(b_row[k + j]) : ~0u;
+        signs_search<LOG_R, false>(sorted, x, position);
+#pragma unroll
+        for (int j = 0; j < 8; j++) position[j] = min(position[j], keys);         // what lies beyond K meets W = 0
+        positions[(i64)(k / 8) * args.n_pad] = signs_pack(position);
+    }
+    unsigned short *counts = args.counts + batch * args.counts_bs + ((i64)chunk * args.n_pad + n) * args.m_pad;
+    for (int m = 8 * tid; m < args.m_pad; m += 8 * NGF_PREPARE_THREADS) {
+        unsigned x[8];
+        int count[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) x[j] = m + j < args.m ? signs_key(d_row[m + j]) : 0u;
+        if (args.sort_d) {
+            signs_search<LOG_R, false>(sorted, x, count);
+#pragma unroll
+            for (int j = 0; j < 8; j++) count[j]++;
+        } else {
+            signs_search<LOG_R, true>(sorted, x, count);
+        }
+#pragma unroll
+        for (int j = 0; j < 8; j++) count[j] = min(count[j], keys);               // the padding of the sort is not B's
+        *reinterpret_cast<gram_chunk *>(counts + m) = signs_pack(count);
+    }
+}
+
+// 64 m x 512 k of A into the order of the product's waves, and the largest magnitude per m.  Memory-bound.
+__device__ __forceinline__ void signs_copy_tile(const GradientPrepareArgs &args, int block, int batch, float *tile)
+{
+    constexpr int PITCH = NGF_COPY_M + 1;
+    constexpr int ROUNDS = NGF_STAGE_K * NGF_COPY_M / 4 / NGF_PREPARE_THREADS;      // of four values per thread, per 64 k
+    const int tid = threadIdx.x;
+    const int m_tiles = args.m_pad / NGF_COPY_M;
+    const int m0 = block % m_tiles * NGF_COPY_M, range = block / m_tiles;
+    const int k_end = min((range + 1) * NGF_COPY_K, args.k_pad);
+    const float *a = args.a + batch * args.a_bs;
+    float *copy = args.a_copy + batch * args.a_copy_bs;
+    // loads: 4 m of one k.  Stores: 4 k of one m, of pair `pair` (of 8 per round) and step `step` of the 64 k
+    const int load_k = tid >> 4, load_m = (tid & 15) * 4;
+    const int pair = tid >> 5, step = tid >> 4 & 1, q = tid >> 2 & 3, which = tid >> 1 & 1, low = (tid & 1) * 4;
+    auto load = [&](int k0, float (&v)[ROUNDS][4]) {
+#pragma unroll
+        for (int round = 0; round < ROUNDS; round++) {
+            const int k = k0 + load_k + 16 * round;
+            const float *src = a + (i64)k * args.a_ld + m0 + load_m;
+            if (k < args.k && args.a_vec && m0 + load_m + 4 <= args.m) {
+                const float4 f = *reinterpret_cast<const float4 *>(src);
+                v[round][0] = f.x; v[round][1] = f.y; v[round][2] = f.z; v[round][3] = f.w;
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; j++) v[round][j] = (k < args.k && m0 + load_m + j < args.m) ? src[j] : 0.0f;
+            }
+        }
+    };
+    float magnitude[ROUNDS] = {};
+    float v[ROUNDS][4];
+    load(range * NGF_COPY_K, v);
+    for (int k0 = range * NGF_COPY_K; k0 < k_end; k0 += NGF_STAGE_K) {
+        __syncthreads();
+#pragma unroll
+        for (int round = 0; round < ROUNDS; round++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) tile[(load_k + 16 * round) * PITCH + load_m + j] = v[round][j];
+        __syncthreads();
+        if (k0 + NGF_STAGE_K < k_end) load(k0 + NGF_STAGE_K, v);
+#pragma unroll
+        for (int round = 0; round < ROUNDS; round++) {
+            float w[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                w[j] = tile[(NGF_STEP_K * step + 8 * q + low + j) * PITCH + 2 * (pair + 8 * round) + which];
+                magnitude[round] = fmaxf(magnitude[round], fabsf(w[j]));      // skips NaNs, whose products are not numbers at any scale
+            }
+            float *dst = copy + ((i64)(m0 / 2 + pair + 8 * round) * (args.k_pad / NGF_STEP_K) + k0 / NGF_STEP_K + step) * 64 + (tid & 15) * 4;
+            *reinterpret_cast<float4 *>(dst) = make_float4(w[0], w[1], w[2], w[3]);
+        }
+    }
+    // the lanes that share m: all bits of the lane but 1 (which) and 5 (pair)
+#pragma unroll
+    for (int round = 0; round < ROUNDS; round++) {
+#pragma unroll
+        for (int bit : {1, 4, 8, 16}) magnitude[round] = fmaxf(magnitude[round], __shfl_xor(magnitude[round], bit));
+        if ((tid & 0x1d) == 0)
+            args.a_magnitudes[batch * args.a_magnitudes_bs + (i64)range * args.m_pad + m0 + 2 * (pair + 8 * round) + which] = magnitude[round];
+    }
+}
+
+// One row o of C as two fp16 pieces, its largest magnitude in [2^6, 2^7), zeros beyond K and O
+__device__ __forceinline__ void signs_split_row(const GradientPrepareArgs &args, int o, int batch, float *shared)
+{
+    const int tid = threadIdx.x;
+    const float *row = args.c + batch * args.c_bs + (i64)o * args.c_ld;
+    const bool live = o < args.o;
+    float magnitude = 0.0f;
+    if (live)
+        for (int k = tid; k < args.k; k += NGF_PREPARE_THREADS) magnitude = fmaxf(magnitude, fabsf(row[k]));
+#pragma unroll
+    for (int bit = 1; bit < 64; bit *= 2) magnitude = fmaxf(magnitude, __shfl_xor(magnitude, bit));
+    if ((tid & 63) == 0) shared[tid >> 6] = magnitude;
+    __syncthreads();
+#pragma unroll
+    for (int wave = 0; wave < NGF_PREPARE_THREADS / 64; wave++) magnitude = fmaxf(magnitude, shared[wave]);
+    const int exponent_field = gram_scale_exponent(magnitude);
+    const float scale = gram_scale(exponent_field) * NGF_SCALE_C;
+    if (tid == 0) args.c_unscale[batch * args.c_unscale_bs + o] = gram_unscale(exponent_field) * (1.0f / NGF_SCALE_C);
+    gram_chunk *pieces = args.c_pieces + batch * args.c_pieces_bs + (i64)(o / 16) * args.k_pad / 8 * 32 + o % 16;
+    for (int k = 8 * tid; k < args.k_pad; k += 8 * NGF_PREPARE_THREADS) {
+        gram_chunk first, second;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            unsigned h1, h2;
+            gram_split_pair(live && k + 2 * j < args.k ? row[k + 2 * j] * scale : 0.0f,
+                            live && k + 2 * j + 1 < args.k ? row[k + 2 * j + 1] * scale : 0.0f, h1, h2);
+            first[j] = h1; second[j] = h2;
+        }
+        pieces[(i64)(k / 8) * 32] = first;
+        pieces[(i64)(k / 8) * 32 + 16] = second;
+    }
+}
+
+// Rows to sort keep LDS busy, tiles of A the memory, so the two are dealt out in turn, in groups of one workgroup per
+// CU, spread evenly over the launch; the rows of C come last.
+template <int LOG_R>
+__global__ __launch_bounds__(NGF_PREPARE_THREADS) void gradient_signs_prepare(const GradientPrepareArgs args)
+{
+    constexpr int WORDS = (256 << LOG_R) + (8 << LOG_R);
+    constexpr int TILE_WORDS = NGF_STAGE_K * (NGF_COPY_M + 1);
+    __shared__ unsigned words[WORDS > TILE_WORDS ? WORDS : TILE_WORDS];
+    const int batch = blockIdx.y;
+    const i64 groups = args.sort_groups + args.copy_groups, group = blockIdx.x / NGF_PREPARE_GROUP;
+    const int within = blockIdx.x % NGF_PREPARE_GROUP;
+    if (group >= groups) {
+        if (batch < args.c_batches) signs_split_row(args, blockIdx.x - (int)groups * NGF_PREPARE_GROUP, batch, reinterpret_cast<float *>(words));
+        return;
+    }
+    const int sorts_before = (int)((group * args.sort_groups + groups - 1) / groups);
+    const int sorts_behind = (int)(((group + 1) * args.sort_groups + groups - 1) / groups);
+    if (sorts_behind > sorts_before) {
+        const int block = sorts_before * NGF_PREPARE_GROUP + within;
+        if (block < args.sort_blocks && batch < args.sort_batches) signs_rank_row<LOG_R>(args, block, batch, words);
+    } else {
+        const int block = ((int)group - sorts_before) * NGF_PREPARE_GROUP + within;
+        if (block < args.copy_blocks && batch < args.a_batches) signs_copy_tile(args, block, batch, reinterpret_cast<float *>(words));
+    }
+}
+
+typedef _Float16 ngf_half2 __attribute__((ext_vector_type(2)));
+
+// (by value: a bit cast of an element of a vector, in place, takes the first element)
+__device__ __forceinline__ ngf_half2 signs_halves(unsigned x)
+{
+    return __builtin_bit_cast(ngf_half2, x);
+}
+
+// 1 where count > position and 0 where not, in both halves: one v_pk_add_f16 with clamp
+__device__ __forceinline__ unsigned signs_compare(_Float16 count, unsigned positions)
+{
+    ngf_half2 x = ngf_half2{count, count} - signs_halves(positions);
+    x = __builtin_elementwise_min(__builtin_elementwise_max(x, ngf_half2{(_Float16)0, (_Float16)0}), ngf_half2{(_Float16)1, (_Float16)1});
+    return __builtin_bit_cast(unsigned, x);
+}
+
+template <int BLOCKS>
+struct GradientF16Tile {
+    static constexpr int TILE_N = 16 * BLOCKS;
+    static constexpr int POSITION_CHUNKS = 8 * TILE_N;                  // of 16 bytes, per stage
+    static constexpr int C_CHUNKS = NGF_STAGE_K * NGF_TILE_O / 4;
+    static constexpr int A_CHUNKS = NGF_STAGE_K * NGF_TILE_M / 4;
+    static constexpr int PASS_BLOCKS = BLOCKS < 4 ? BLOCKS : 2;         // of 16 n, per pass of the epilogue
+    static constexpr int RESULT_PITCH = NGF_TILE_M + 4;
+    static constexpr int PASS_CHUNKS = PASS_BLOCKS * 256 * RESULT_PITCH / 4;
+    // two stages of everything, of A as it is and in pieces: 88 KB at 256 n
+    static constexpr int STAGE_CHUNKS = 2 * (POSITION_CHUNKS + C_CHUNKS + A_CHUNKS + A_CHUNKS);
+    static constexpr int CHUNKS = STAGE_CHUNKS > PASS_CHUNKS ? STAGE_CHUNKS : PASS_CHUNKS;
+};
+
+template <int BLOCKS, bool PIECES_IN_COLUMNS>
+__global__ __launch_bounds__(NGF_THREADS, BLOCKS >= 8 ? 2 : 4) void norm_gradient_l1_f16(const NormGradientF16Args args)
+{
+    using Tile = GradientF16Tile<BLOCKS>;
+    constexpr int COLUMN_PIECES = PIECES_IN_COLUMNS ? 1 : GW_PIECES;
+    __shared__ gram_chunk lds[Tile::CHUNKS];
 
     const NormGradientArgs &g = args.g;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int q = lane >> 4;     // 8 k of a step (operands), row quad (result)
-    const int r = lane & 15;     // row m (T) / column o (C, result)
+    const int r = lane & 15;     // row n (S) / column (W, result)
     const int batch = blockIdx.z / g.o_chunks;
-    const int o0 = args.o_begin + (blockIdx.z % g.o_chunks) * Tile::TILE_O;
-    const int m0 = blockIdx.x * NGF_TILE_M;
+    const int o0 = args.o_begin + (blockIdx.z % g.o_chunks) * NGF_TILE_O;
+    // the tiles of an XCD (every eighth workgroup) lie side by side, so that two of them fill a line of E in its L2
+    const int xcd = blockIdx.x & 7, per_xcd = gridDim.x >> 3, longer = gridDim.x & 7;
+    const int m0 = (xcd * per_xcd + min(xcd, longer) + (int)(blockIdx.x >> 3)) * NGF_TILE_M;
     const int n0 = blockIdx.y * Tile::TILE_N;
 
-    auto buffer = [&](auto which) -> gram_chunk * {
-        constexpr int B = decltype(which)::value;
-        if constexpr (B == 0) return lds0;
-        else if constexpr (B == 1) return lds1;
-        else return lds2;
-    };
-
-    // Copies per step, four per wave (five for 64 outputs), the same number in every wave so that
-    // one count of copies under way serves all.  A: 8 runs of 64 chunks, two per wave.  C: 8 runs of
-    // 16, 32 or 64 chunks: with 16, two copies of 4 runs (waves 0 and 2 issue the first, 1 and 3 the
-    // second: the same bytes twice); with 32, one copy of 2 runs per wave; with 64, two copies of one
-    // run per wave.  B: rows of 128 bytes, 8 per copy: with 32 rows one copy per wave, with 16 rows
-    // waves 2 and 3 repeat the copies of waves 0 and 1, with 8 rows every wave issues the one copy.
-    // A run (slice, piece, half) of a step starts at chunk ((2 step + slice) * 4 + 2 piece + half) *
-    // rows_pad of an operand's pieces.
     typedef const __attribute__((address_space(1))) void *global_address;
     typedef __attribute__((address_space(3))) void *lds_address;
-    constexpr int COPIES = Tile::COPIES;
-    const gram_chunk *src[COPIES];
-    i64 advance[COPIES];
-    int dst[COPIES];
-    {
-        const gram_chunk *pieces_a = args.pieces_a + batch * args.pieces_a_bs + m0;
-        const gram_chunk *pieces_c = args.pieces_c + batch * args.pieces_c_bs + o0;
+    // Copies of 64 chunks per stage and wave, the same in every wave.  Positions: 8 runs (8 k each) of TILE_N chunks; a copy
+    // is a part of a run, or, of 32 n, two runs.  C: 256 chunks in a row.  A: the 512 bytes of the wave's own two m, as two copies of 4
+    // bytes per lane.
+    constexpr int POSITION_COPIES = 2 * BLOCKS / NGF_WAVES > 0 ? 2 * BLOCKS / NGF_WAVES : 1;
+    constexpr int COPIES_PER_RUN = BLOCKS >= 4 ? BLOCKS / 4 : 1;
+    const gram_chunk *position_src[POSITION_COPIES];
+    int position_dst[POSITION_COPIES];
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const int run = 2 * wave + j;
-            src[j] = pieces_a + (i64)run * args.rows_pad_a + lane;
-            advance[j] = (i64)8 * args.rows_pad_a;
-            dst[j] = run * NGF_TILE_M;
-        }
-        if constexpr (O_BLOCKS == 4) {
-#pragma unroll
-            for (int j = 0; j < 2; j++) {                                       // 64 chunks of the step's C each: one run
-                const int run = 2 * wave + j;
-                src[2 + j] = pieces_c + (i64)run * args.rows_pad_c + lane;
-                advance[2 + j] = (i64)8 * args.rows_pad_c;
-                dst[2 + j] = Tile::A_CHUNKS + 64 * run;
-            }
-        } else {
-            const int c_copy = O_BLOCKS == 1 ? (wave & 1) : wave;               // 64 chunks of the step's C each
-            const int c_run = O_BLOCKS == 1 ? 4 * c_copy + q : 2 * c_copy + (lane >> 5);
-            const int c_row = O_BLOCKS == 1 ? r : (lane & 31);
-            src[2] = pieces_c + (i64)c_run * args.rows_pad_c + c_row;
-            advance[2] = (i64)8 * args.rows_pad_c;
-            dst[2] = Tile::A_CHUNKS + 64 * c_copy;
-        }
-        // 8 rows of B per copy: lane -> row lane / 8, 16 bytes number lane % 8 of the step's 128
-        const int b_copy = O_BLOCKS == 1 ? wave : O_BLOCKS == 2 ? (wave & 1) : 0;
-        const float *b_row = args.b_padded + batch * args.b_padded_bs + (i64)(n0 + 8 * b_copy + (lane >> 3)) * args.k_pad + 4 * (lane & 7);
-        src[COPIES - 1] = reinterpret_cast<const gram_chunk *>(b_row);
-        advance[COPIES - 1] = NGF_STEP_K / 4;
-        dst[COPIES - 1] = Tile::A_CHUNKS + Tile::C_CHUNKS + 64 * b_copy;
+    for (int j = 0; j < POSITION_COPIES; j++) {
+        const int copy = (wave * POSITION_COPIES + j) % (2 * BLOCKS);
+        const int run = BLOCKS >= 4 ? copy / COPIES_PER_RUN : 2 * copy + (lane >> 5);
+        position_src[j] = reinterpret_cast<const gram_chunk *>(args.positions + batch * args.positions_bs) + (i64)run * args.n_pad + n0 +
+                          (BLOCKS >= 4 ? 64 * (copy % COPIES_PER_RUN) + lane : lane & 31);
+        position_dst[j] = 64 * copy;
     }
-    auto copy_step = [&](auto into) {
+    const gram_chunk *c_src = args.c_pieces + batch * args.c_pieces_bs + (i64)(o0 / 16) * args.k_pad / 8 * 32 + 64 * (wave & 3) + lane;
+    const float *a_src = args.a_copy + batch * args.a_copy_bs + (i64)(m0 / 2 + wave) * (args.k_pad / NGF_STEP_K) * 64 + lane;
+    auto copy16 = [&](const gram_chunk *src, gram_chunk *dst) {
+        const unsigned lds_byte = (unsigned)(unsigned long)(lds_address)dst;
+        asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"((global_address)src), "s"(lds_byte) : "memory", "m0");
+    };
+    auto copy4 = [&](const float *src, gram_chunk *dst) {
+        const unsigned lds_byte = (unsigned)(unsigned long)(lds_address)dst;
+        asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" : : "v"((global_address)src), "s"(lds_byte) : "memory", "m0");
+    };
+    gram_chunk *const lds_c = lds + 2 * Tile::POSITION_CHUNKS;
+    gram_chunk *const lds_a = lds_c + 2 * Tile::C_CHUNKS;
+    unsigned *const a_pieces = reinterpret_cast<unsigned *>(lds_a + 2 * Tile::A_CHUNKS) + 128 * wave;        // [stage % 2][wave][piece][64]
+    auto copy_stage = [&](int into) {
 #pragma unroll
-        for (int j = 0; j < COPIES; j++) {
-            const unsigned lds_byte = (unsigned)(unsigned long)(lds_address)(buffer(into) + dst[j]);
-            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
-                         :
-                         : "v"((global_address)src[j]), "s"(lds_byte)
-                         : "memory", "m0");
-            src[j] += advance[j];
+        for (int j = 0; j < POSITION_COPIES; j++) {
+            copy16(position_src[j], lds + into * Tile::POSITION_CHUNKS + position_dst[j]);
+            position_src[j] += (i64)8 * args.n_pad;
         }
+        copy16(c_src, lds_c + into * Tile::C_CHUNKS + 64 * (wave & 3));
+        c_src += Tile::C_CHUNKS;
+    };
+    auto copy_a = [&](int into) {
+#pragma unroll
+        for (int j = 0; j < 2; j++) copy4(a_src + 64 * j, lds_a + into * Tile::A_CHUNKS + 32 * wave + 16 * j);
+        a_src += 128;
     };
 
-    // D[m, n] of this lane's rows, for the n of the wave.
-    float dval[WAVE_N][4];
+    // scale of the lane's m in split_a: 8 k of m0 + 2 wave, 8 k of m0 + 2 wave + 1 and so on, two k per lane
+    float scale_a, unscale_a[2];
     {
-        const float *d_base = g.d + batch * g.d_bs;
+        const float *magnitudes = args.a_magnitudes + batch * args.a_magnitudes_bs + m0 + 2 * wave;
+        float largest[2] = {0.0f, 0.0f};
+        for (int range = lane; range < args.ranges; range += 64)
 #pragma unroll
-        for (int nb = 0; nb < WAVE_N; nb++) {
-            const int n = n0 + WAVE_N * wave + nb;
+            for (int i = 0; i < 2; i++) largest[i] = fmaxf(largest[i], magnitudes[(i64)range * args.m_pad + i]);
 #pragma unroll
-            for (int mb = 0; mb < 4; mb++) {
-                const int m = m0 + 16 * mb + r;
-                dval[nb][mb] = (n < g.n && m < g.m) ? d_base[(i64)n * g.d_ld + m] : 0.0f;
-            }
+        for (int i = 0; i < 2; i++) {
+#pragma unroll
+            for (int bit = 1; bit < 64; bit *= 2) largest[i] = fmaxf(largest[i], __shfl_xor(largest[i], bit));
+            unscale_a[i] = gram_unscale(gram_scale_exponent(largest[i])) * (1.0f / NGF_SCALE_A);
         }
+        scale_a = gram_scale(gram_scale_exponent(lane & 4 ? largest[1] : largest[0])) * NGF_SCALE_A;
     }
+    // counts of the lane's rows n for the wave's two m, one dword per block
+    const unsigned short *counts = args.counts + batch * args.counts_bs + (i64)(n0 + r) * args.m_pad + m0 + 2 * wave;
+    unsigned count[BLOCKS];
+    auto load_counts = [&](int chunk) {
+#pragma unroll
+        for (int block = 0; block < BLOCKS; block++)
+            count[block] = *reinterpret_cast<const unsigned *>(counts + ((i64)chunk * args.n_pad + 16 * block) * args.m_pad);
+    };
+    load_counts(0);
     // the copies are not counted by the compiler: nothing it loads may be under way beside them
     __builtin_amdgcn_s_waitcnt(0x0F70);
 
-    ngf_float4 acc[WAVE_N][4][O_BLOCKS];
+    ngf_float4 acc[2][BLOCKS];
 #pragma unroll
-    for (int nb = 0; nb < WAVE_N; nb++)
+    for (int i = 0; i < 2; i++)
 #pragma unroll
-        for (int mb = 0; mb < 4; mb++)
-#pragma unroll
-            for (int ob = 0; ob < O_BLOCKS; ob++) acc[nb][mb][ob] = ngf_float4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int block = 0; block < BLOCKS; block++) acc[i][block] = ngf_float4{0.0f, 0.0f, 0.0f, 0.0f};
+    float sum_w[2] = {0.0f, 0.0f};
+    const int column = PIECES_IN_COLUMNS ? (r & 7) : r;
 
-    // lane (q, r): its 8 k are slice q / 2, half q % 2 of the step
-    const int run_of_lane = 4 * (q >> 1) + (q & 1);      // + 2 piece
-    auto step = [&](auto which) {
-        const gram_chunk *lds = buffer(which);
-        gram_half8 fc[O_BLOCKS][GW_PIECES], fa[4][GW_PIECES];
+    // A of a stage into two pieces, by the wave that uses it
+    auto split_a = [&](int into) {
+        const float2 a = reinterpret_cast<const float2 *>(lds_a + into * Tile::A_CHUNKS)[64 * wave + lane];
+        unsigned h1, h2;
+        gram_split_pair(a.x * scale_a, a.y * scale_a, h1, h2);
+        a_pieces[128 * NGF_WAVES * into + lane] = h1;
+        a_pieces[128 * NGF_WAVES * into + 64 + lane] = h2;
+    };
+    auto step = [&](int from, int half) {
+        const gram_chunk *positions = lds + from * Tile::POSITION_CHUNKS + (4 * half + q) * Tile::TILE_N + r;
+        gram_chunk c[GW_PIECES];
 #pragma unroll
-        for (int ob = 0; ob < O_BLOCKS; ob++)
+        for (int piece = 0; piece < GW_PIECES; piece++) c[piece] = lds_c[from * Tile::C_CHUNKS + (4 * half + q) * 32 + 16 * piece + column];
+        gram_half8 w[2][COLUMN_PIECES];
 #pragma unroll
-            for (int p = 0; p < GW_PIECES; p++)
-                fc[ob][p] = __builtin_bit_cast(gram_half8, lds[Tile::A_CHUNKS + (run_of_lane + 2 * p) * Tile::TILE_O + 16 * ob + r]);
+        for (int i = 0; i < 2; i++) {
+            gram_chunk a[GW_PIECES];
 #pragma unroll
-        for (int mb = 0; mb < 4; mb++)
+            for (int piece = 0; piece < GW_PIECES; piece++)
+                a[piece] = reinterpret_cast<const gram_chunk *>(a_pieces + 128 * NGF_WAVES * from + 64 * piece)[8 * half + 2 * q + i];
+            gram_chunk first, second;
 #pragma unroll
-            for (int p = 0; p < GW_PIECES; p++)
-                fa[mb][p] = __builtin_bit_cast(gram_half8, lds[(run_of_lane + 2 * p) * NGF_TILE_M + 16 * mb + r]);
-        const float4 *b_rows = reinterpret_cast<const float4 *>(lds + Tile::A_CHUNKS + Tile::C_CHUNKS);
+            for (int j = 0; j < 4; j++) {
+                const ngf_half2 a1 = signs_halves(a[0][j]), a2 = signs_halves(a[1][j]);
+                const ngf_half2 c1 = signs_halves(c[0][j]), c2 = signs_halves(c[1][j]);
+                const ngf_half2 h1 = a1 * c1;
+                const ngf_half2 h2 = __builtin_elementwise_fma(a2, c1, __builtin_elementwise_fma(a1, c2, __builtin_elementwise_fma(a1, c1, -h1)));
+                first[j] = __builtin_bit_cast(unsigned, h1);
+                second[j] = __builtin_bit_cast(unsigned, h2);
+                const ngf_half2 one = {(_Float16)1, (_Float16)1};
+                sum_w[i] = __builtin_amdgcn_fdot2(h1, one, sum_w[i], false);
+                sum_w[i] = __builtin_amdgcn_fdot2(h2, one, sum_w[i], false);
+            }
+            if constexpr (PIECES_IN_COLUMNS) {
 #pragma unroll
-        for (int nb = 0; nb < WAVE_N; nb++) {
-            const float4 b_low = b_rows[(WAVE_N * wave + nb) * (NGF_STEP_K / 4) + 2 * q];
-            const float4 b_high = b_rows[(WAVE_N * wave + nb) * (NGF_STEP_K / 4) + 2 * q + 1];
-            const float bk[8] = {b_low.x, b_low.y, b_low.z, b_low.w, b_high.x, b_high.y, b_high.z, b_high.w};
-#pragma unroll
-            for (int mb = 0; mb < 4; mb++) {
-                gram_chunk t1 = __builtin_bit_cast(gram_chunk, fa[mb][0]);
-                gram_chunk t2 = __builtin_bit_cast(gram_chunk, fa[mb][1]);
-#ifndef NGF_ABLATE_NO_SIGN
-#pragma unroll
-                for (int pair = 0; pair < 4; pair++) {
-                    const unsigned low = __float_as_uint(dval[nb][mb] - bk[2 * pair]);
-                    const unsigned high = __float_as_uint(dval[nb][mb] - bk[2 * pair + 1]);
-                    // the two sign bits, at the sign bits of the two halves of a dword
-                    const unsigned flip = __builtin_amdgcn_perm(high, low, 0x070c030c) & 0x80008000u;
-                    t1[pair] ^= flip;
-                    t2[pair] ^= flip;
-                }
-                const gram_half8 h1 = __builtin_bit_cast(gram_half8, t1), h2 = __builtin_bit_cast(gram_half8, t2);
-#ifdef NGF_ABLATE_NO_MFMA
-                asm volatile("" : : "v"(h1), "v"(h2));      // the signed pieces are made and dropped
-#else
-#pragma unroll
-                for (int ob = 0; ob < O_BLOCKS; ob++) acc[nb][mb][ob] = __builtin_amdgcn_mfma_f32_16x16x32_f16(h2, fc[ob][0], acc[nb][mb][ob], 0, 0, 0);
-#pragma unroll
-                for (int ob = 0; ob < O_BLOCKS; ob++) acc[nb][mb][ob] = __builtin_amdgcn_mfma_f32_16x16x32_f16(h1, fc[ob][1], acc[nb][mb][ob], 0, 0, 0);
-#pragma unroll
-                for (int ob = 0; ob < O_BLOCKS; ob++) acc[nb][mb][ob] = __builtin_amdgcn_mfma_f32_16x16x32_f16(h1, fc[ob][0], acc[nb][mb][ob], 0, 0, 0);
-#endif
+                for (int j = 0; j < 4; j++) first[j] = r < 8 ? first[j] : second[j];
+                w[i][0] = __builtin_bit_cast(gram_half8, first);
+            } else {
+                w[i][0] = __builtin_bit_cast(gram_half8, first);
+                w[i][1] = __builtin_bit_cast(gram_half8, second);
             }
         }
-#endif
-        // the wave's own copies of the next step have arrived (the four of the step after it may
-        // still be under way); behind the barrier everybody's have, and this step's buffer is free
-        __builtin_amdgcn_s_waitcnt(0x0F70 | COPIES);            // vmcnt(COPIES)
-        __syncthreads();
-        copy_step(which);
+        gram_chunk p[3], s[2][2];
+        auto compare = [&](int block, const gram_chunk &at, gram_chunk (&into)[2]) {
+            const ngf_half2 pair = signs_halves(count[block]);
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) into[i][j] = signs_compare(pair[i], at[j]);
+        };
+#pragma unroll
+        for (int block = 0; block < 3 && block < BLOCKS; block++) p[block] = positions[16 * block];
+        compare(0, p[0], s[0]);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int block = 0; block < BLOCKS; block++) {
+            if (block + 3 < BLOCKS) p[block % 3] = positions[16 * (block + 3)];
+            if (block + 1 < BLOCKS) compare(block + 1, p[(block + 1) % 3], s[(block + 1) % 2]);
+#pragma unroll
+            for (int piece = COLUMN_PIECES - 1; piece >= 0; piece--)
+#pragma unroll
+                for (int i = 0; i < 2; i++)
+                    acc[i][block] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(gram_half8, s[block % 2][i]), w[i][piece], acc[i][block], 0, 0, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+#pragma unroll
+            for (int j = 0; j < 2 * COLUMN_PIECES; j++) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 4 / COLUMN_PIECES, 0);
+            }
+        }
+    };
+    // the sums over k of the four row quads, half of them off the results of the column (with the pieces in the
+    // columns: off the first piece's)
+    auto correct = [&]() {
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            float total = sum_w[i];
+            total += __shfl_xor(total, 16);
+            total += __shfl_xor(total, 32);
+            const float off = PIECES_IN_COLUMNS && r >= 8 ? 0.0f : 0.5f * total;
+#pragma unroll
+            for (int block = 0; block < BLOCKS; block++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) acc[i][block][j] -= off;
+            sum_w[i] = 0.0f;
+        }
     };
 
-    copy_step(GramStep<0>{});
-    copy_step(GramStep<1>{});
-    copy_step(GramStep<2>{});
-    __builtin_amdgcn_s_waitcnt(0x0F70 | (2 * COPIES));      // vmcnt(2 COPIES): step 0 has arrived
-    __syncthreads();
-    for (int done = 0;;) {
-        step(GramStep<0>{});
-        if (++done == args.steps) break;
-        step(GramStep<1>{});
-        if (++done == args.steps) break;
-        step(GramStep<2>{});
-        if (++done == args.steps) break;
-    }
+    // Positions and C are copied one stage ahead, A two: it is split in the stage before.  (Three buffers and copies two and
+    // three stages ahead: the same time; the copies' latency is not what bounds a stage.)
+    copy_a(0);
+    copy_stage(0);
+    if (args.stages > 1) copy_a(1);
     __builtin_amdgcn_s_waitcnt(0x0F70);
+    split_a(0);
+    int chunk = 0, chunk_left = args.chunk_stages;
+    for (int stage = 0; stage < args.stages; stage++) {
+        // the wave's own copies have arrived; behind the barrier everybody's have, and the other buffer is free
+        __builtin_amdgcn_s_waitcnt(0x0F70);
+        __syncthreads();
+        if (chunk_left == 0) {
+            load_counts(++chunk);
+            chunk_left = args.chunk_stages;
+            __builtin_amdgcn_s_waitcnt(0x0F70);
+        }
+        chunk_left--;
+        const int here = stage & 1, other = here ^ 1;
+        if (stage + 1 < args.stages) copy_stage(other);
+        if (stage + 2 < args.stages) copy_a(here);
+        if (stage + 1 < args.stages) split_a(other);
+        step(here, 0);
+        step(here, 1);
+        if (stage % NGF_CORRECT_STAGES == NGF_CORRECT_STAGES - 1 || stage + 1 == args.stages) correct();
+    }
 
-    // acc[nb][mb][ob][j]: m = m0 + 16 mb + 4 q + j, o = o0 + 16 ob + r, n = n0 + WAVE_N wave + nb
+    // acc[i][block][j]: m = m0 + 2 wave + i, n = n0 + 16 block + 4 q + j, o = o0 + column.  Through LDS, so that the 16 m
+    // of the workgroup are stored together.
+    if constexpr (PIECES_IN_COLUMNS) {
 #pragma unroll
-    for (int ob = 0; ob < O_BLOCKS; ob++) {
-        const int o = o0 + 16 * ob + r;
-        const float unscale_c = args.unscale_c[batch * args.unscale_c_bs + o];
-        float *e_base = g.e + batch * g.e_bs + (i64)o * g.e_ld_o;
+        for (int i = 0; i < 2; i++)
 #pragma unroll
-        for (int mb = 0; mb < 4; mb++) {
-            const int m = m0 + 16 * mb + 4 * q;
-            const float4 unscale_a = *reinterpret_cast<const float4 *>(args.unscale_a + batch * args.unscale_a_bs + m);
+            for (int block = 0; block < BLOCKS; block++)
 #pragma unroll
-            for (int nb = 0; nb < WAVE_N; nb++) {
-                const int n = n0 + WAVE_N * wave + nb;
-                if (n >= g.n || o >= g.o) continue;
-                const ngf_float4 sum = acc[nb][mb][ob];
-                const float v[4] = {sum[0] * unscale_a.x * unscale_c, sum[1] * unscale_a.y * unscale_c,
-                                    sum[2] * unscale_a.z * unscale_c, sum[3] * unscale_a.w * unscale_c};
-                float *dst = e_base + (i64)n * g.e_ld_n + m;
-                if (g.e_vec && m + 3 < g.m) {
-                    *reinterpret_cast<float4 *>(dst) = make_float4(v[0], v[1], v[2], v[3]);
-                } else {
+                for (int j = 0; j < 4; j++) acc[i][block][j] += __shfl_xor(acc[i][block][j], 8);
+    }
+    const float unscale_c = 2.0f * args.c_unscale[batch * args.c_unscale_bs + o0 + column];
+    float *results = reinterpret_cast<float *>(lds);
+    constexpr int PITCH = Tile::RESULT_PITCH;
 #pragma unroll
-                    for (int j = 0; j < 4; j++)
-                        if (m + j < g.m) dst[j] = v[j];
-                }
+    for (int pass = 0; pass < BLOCKS / Tile::PASS_BLOCKS; pass++) {
+        __syncthreads();
+#pragma unroll
+        for (int within = 0; within < Tile::PASS_BLOCKS; within++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int block = pass * Tile::PASS_BLOCKS + within;
+                *reinterpret_cast<float2 *>(results + ((16 * within + 4 * q + j) * 16 + r) * PITCH + 2 * wave) =
+                    make_float2(acc[0][block][j] * unscale_a[0] * unscale_c, acc[1][block][j] * unscale_a[1] * unscale_c);
+            }
+        __syncthreads();
+        constexpr int QUADS = NGF_TILE_M / 4;
+        const int quad = tid % QUADS;
+        const int m = m0 + 4 * quad;
+#pragma unroll
+        for (int row = tid / QUADS; row < 256 * Tile::PASS_BLOCKS; row += NGF_THREADS / QUADS) {
+            const int o = o0 + (row & 15), n = n0 + 16 * Tile::PASS_BLOCKS * pass + (row >> 4);
+            if (o >= g.o || n >= g.n || (PIECES_IN_COLUMNS && (row & 8))) continue;
+            const float4 v = *reinterpret_cast<const float4 *>(results + row * PITCH + 4 * quad);
+            float *dst = g.e + batch * g.e_bs + (i64)o * g.e_ld_o + (i64)n * g.e_ld_n + m;
+            if (g.e_vec && m + 3 < g.m) {
+                *reinterpret_cast<float4 *>(dst) = v;
+            } else {
+                if (m < g.m) dst[0] = v.x;
+                if (m + 1 < g.m) dst[1] = v.y;
+                if (m + 2 < g.m) dst[2] = v.z;
+                if (m + 3 < g.m) dst[3] = v.w;
             }
         }
     }

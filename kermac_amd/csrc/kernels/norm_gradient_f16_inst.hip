@@ -1,7 +1,5 @@
 // Host side of the L1 kernel gradient on the fp16 matrix instruction (norm_gradient_f16.hpp): when
-// it applies, how the caller's workspace is divided, and the launches: row statistics and split of
-// A (rows m) and of C (rows o) by the kernels of gram_f16_wide.hpp, a padded copy of B, the
-// contraction.
+// it applies, how the caller's workspace is divided, and the launches.
 #include <hip/hip_runtime.h>
 
 #include <cstdlib>
@@ -18,17 +16,13 @@ namespace {
 
 constexpr int64_t REGION_ALIGN = 256;
 
-struct RowsRegions {
-    int rows_pad, batches;
-    int64_t pieces_bs, stats_bs;
-    int64_t pieces, squares, magnitudes, unscale;     // byte offsets into the workspace
-};
-
 struct GradientLayout {
-    int slices, slices_alloc, slices_per_range, ranges, steps;
-    int n_pad, k_pad, b_batches;
-    RowsRegions a, c;
-    int64_t b_padded, b_padded_bs;
+    int stages, n_pad, m_pad, k_pad, o_pad, ranges;
+    int chunks, chunk_k, keys;
+    bool sort_d;
+    int sort_batches, a_batches, c_batches;
+    int64_t positions_bs, counts_bs, a_copy_bs, a_magnitudes_bs, c_pieces_bs;     // in elements, of C in chunks of 16 bytes
+    int64_t positions, counts, a_copy, a_magnitudes, c_pieces, c_unscale;         // byte offsets into the workspace
     int64_t bytes;
 };
 
@@ -39,17 +33,7 @@ int64_t place(int64_t &cursor, int64_t bytes)
     return at;
 }
 
-void place_rows(RowsRegions &r, int rows, int batches, const GradientLayout &layout, int64_t &cursor)
-{
-    r.rows_pad = (rows + kmc::GW_TILE - 1) / kmc::GW_TILE * kmc::GW_TILE;
-    r.batches = batches;
-    r.pieces_bs = static_cast<int64_t>(layout.slices_alloc) * kmc::GW_SEGMENTS * r.rows_pad;
-    r.stats_bs = static_cast<int64_t>(layout.ranges) * r.rows_pad;
-    r.pieces = place(cursor, r.batches * r.pieces_bs * 16);
-    r.squares = place(cursor, r.batches * r.stats_bs * 4);
-    r.magnitudes = place(cursor, r.batches * r.stats_bs * 4);
-    r.unscale = place(cursor, static_cast<int64_t>(r.batches) * r.rows_pad * 4);
-}
+int64_t round_up(int64_t value, int64_t multiple) { return (value + multiple - 1) / multiple * multiple; }
 
 // The route pays where the fp32 kernels are bound by their matrix or vector instructions: enough
 // terms to carry the five extra launches, and more than two outputs (its cost does not fall below
@@ -80,49 +64,92 @@ bool gradient_layout(const kmc_norm_gradient_params *p, GradientLayout *layout)
 {
     if (p->norm_type != KMC_NORM_L1 || p->m < 1 || p->n < 1 || p->o < 1 || p->k < 1 || p->l < 1) return false;
     if (!f16_pays(p)) return false;
-    layout->slices = (p->k + kmc::BK_TILE_K - 1) / kmc::BK_TILE_K;
-    layout->steps = (p->k + kmc::NGF_STEP_K - 1) / kmc::NGF_STEP_K;
-    layout->slices_alloc = 2 * (layout->steps + kmc::NGF_AHEAD);
-    layout->slices_per_range = layout->slices / 8 > 8 ? (layout->slices + 7) / 8 : 8;
-    layout->ranges = (layout->slices + layout->slices_per_range - 1) / layout->slices_per_range;
-    layout->n_pad = (p->n + kmc::NGF_N_PAD - 1) / kmc::NGF_N_PAD * kmc::NGF_N_PAD;
-    layout->k_pad = kmc::NGF_STEP_K * (layout->steps + kmc::NGF_AHEAD);
+    // a row n is a row of blockIdx.y in other kernels of its size: the fp32 kernels keep what they had
+    if (round_up(p->n, 32) > 65535 || static_cast<int64_t>(p->l) * (p->o / 64 + 1) > 65535) return false;
+    const int64_t k_pad = round_up(p->k, kmc::NGF_STAGE_K), m_pad = round_up(p->m, kmc::NGF_COPY_M);
+    const int64_t n_pad = round_up(p->n, kmc::NGF_N_PAD), o_pad = round_up(p->o, kmc::NGF_TILE_O);
+    // a dimension of a grid holds fewer than 2^32 threads
+    const int64_t threads = int64_t{1} << 32;
+    // the shorter row of a pair is sorted; rows of B longer than the sort takes are cut into chunks
+    layout->sort_d = p->m < p->k && p->m <= kmc::NGF_MAX_CHUNK;
+    layout->chunks = layout->sort_d ? 1 : (p->k + kmc::NGF_MAX_CHUNK - 1) / kmc::NGF_MAX_CHUNK;
+    layout->chunk_k = static_cast<int>(round_up((p->k + layout->chunks - 1) / layout->chunks, kmc::NGF_STAGE_K));
+    layout->chunks = (p->k + layout->chunk_k - 1) / layout->chunk_k;
+    layout->keys = layout->sort_d ? p->m : layout->chunk_k;
+    layout->ranges = static_cast<int>((k_pad + kmc::NGF_COPY_K - 1) / kmc::NGF_COPY_K);
+    const int64_t prepare_blocks = static_cast<int64_t>(p->n) * layout->chunks + m_pad / kmc::NGF_COPY_M * layout->ranges + o_pad +
+                                   2 * kmc::NGF_PREPARE_GROUP;
+    if (prepare_blocks * kmc::NGF_PREPARE_THREADS >= threads || m_pad / kmc::NGF_TILE_M * kmc::NGF_THREADS >= threads || k_pad > INT32_MAX ||
+        m_pad > INT32_MAX || o_pad > INT32_MAX)
+        return false;
+    layout->stages = static_cast<int>(k_pad / kmc::NGF_STAGE_K);
+    layout->n_pad = static_cast<int>(n_pad); layout->m_pad = static_cast<int>(m_pad);
+    layout->k_pad = static_cast<int>(k_pad); layout->o_pad = static_cast<int>(o_pad);
+    layout->sort_batches = p->b_bs == 0 && p->d_bs == 0 ? 1 : p->l;
+    layout->a_batches = p->a_bs == 0 ? 1 : p->l;
+    layout->c_batches = p->c_bs == 0 ? 1 : p->l;
+    layout->positions_bs = k_pad * n_pad;
+    layout->counts_bs = static_cast<int64_t>(layout->chunks) * n_pad * m_pad;
+    layout->a_copy_bs = m_pad * k_pad;
+    layout->a_magnitudes_bs = static_cast<int64_t>(layout->ranges) * m_pad;
+    layout->c_pieces_bs = o_pad * k_pad / 4;
     int64_t cursor = 0;
-    place_rows(layout->a, p->m, p->a_bs == 0 ? 1 : p->l, *layout, cursor);
-    place_rows(layout->c, p->o, p->c_bs == 0 ? 1 : p->l, *layout, cursor);
-    layout->b_batches = p->b_bs == 0 ? 1 : p->l;
-    layout->b_padded_bs = static_cast<int64_t>(layout->n_pad) * layout->k_pad;
-    layout->b_padded = place(cursor, layout->b_batches * layout->b_padded_bs * 4);
+    layout->positions = place(cursor, layout->sort_batches * layout->positions_bs * 2);
+    layout->counts = place(cursor, layout->sort_batches * layout->counts_bs * 2);
+    layout->a_copy = place(cursor, layout->a_batches * layout->a_copy_bs * 4);
+    layout->a_magnitudes = place(cursor, layout->a_batches * layout->a_magnitudes_bs * 4);
+    layout->c_pieces = place(cursor, layout->c_batches * layout->c_pieces_bs * 16);
+    layout->c_unscale = place(cursor, layout->c_batches * o_pad * 4);
     layout->bytes = cursor;
-    // blockIdx.z = batch entry x chunk of outputs; blockIdx.y = one padded row n for gradient_pad_b (the
-    // largest grid.y of the route; the contraction's tiles of 8, 16 or 32 n need fewer)
-    const int64_t grid_z = static_cast<int64_t>(p->l) * (p->o / 64 + 1);
-    if (grid_z > 65535 || layout->n_pad > 65535) return false;
     return true;
 }
 
-kmc::GramRowsArgs rows_args(const float *x, int64_t ld, int64_t bs, int rows, bool row_major, bool vec, int k,
-                            const GradientLayout &layout, const RowsRegions &r, char *workspace)
+// Tile of the product in n: 16, 8, 4 or 2 blocks of 16.  A wave takes about 84 cycles for the two matrix instructions, the
+// comparisons and the reads of a block and m, and 230 for W and the rest of a step (1580 cycles at 16 blocks, measured at
+// 8192 x 512 x 16 x 8192), so wide tiles are cheaper per result, unless they are too few for the 256 CUs: one
+// workgroup per CU is what the count of rounds assumes.
+int blocks_for(const kmc_norm_gradient_params *p, int o_chunks)
 {
-    kmc::GramRowsArgs rows_of = {};
-    rows_of.x = x; rows_of.ld = ld; rows_of.bs = bs;
-    rows_of.rows = rows; rows_of.k = k;
-    rows_of.row_major = row_major; rows_of.vec = row_major && vec;
-    rows_of.pieces = reinterpret_cast<kmc::gram_chunk *>(workspace + r.pieces); rows_of.pieces_bs = r.pieces_bs;
-    rows_of.squares = reinterpret_cast<float *>(workspace + r.squares);
-    rows_of.magnitudes = reinterpret_cast<float *>(workspace + r.magnitudes);
-    rows_of.unscale = reinterpret_cast<float *>(workspace + r.unscale);
-    rows_of.stats_bs = r.stats_bs; rows_of.unscale_bs = r.rows_pad;
-    rows_of.rows_pad = r.rows_pad; rows_of.slices = layout.slices;
-    rows_of.slices_per_range = layout.slices_per_range; rows_of.ranges = layout.ranges;
-    rows_of.zero_slices = 2 * layout.steps - layout.slices;      // the walk takes two slices per step
-    return rows_of;
+    int best = 16;
+    int64_t best_cost = INT64_MAX;
+    for (int blocks = 16; blocks >= 2; blocks /= 2) {
+        const int64_t tiles_n = (p->n + 16 * blocks - 1) / (16 * blocks), tiles_m = (p->m + kmc::NGF_TILE_M - 1) / kmc::NGF_TILE_M;
+        const int64_t rounds = (tiles_n * tiles_m * p->l * o_chunks + 255) / 256;
+        const int64_t cost = rounds * (84 * blocks + 230);
+        if (cost < best_cost) { best = blocks; best_cost = cost; }
+    }
+    return best;
+}
+
+template <int BLOCKS, bool PIECES_IN_COLUMNS>
+hipError_t launch_product(kmc::NormGradientF16Args &args, int o_begin, int o_chunks, hipStream_t stream)
+{
+    using Tile = kmc::GradientF16Tile<BLOCKS>;
+    const int per_launch = 65535 / args.g.l;         // blockIdx.z = batch entry x block of 16 outputs
+    for (int first = 0; first < o_chunks; first += per_launch) {
+        const int chunks = o_chunks - first < per_launch ? o_chunks - first : per_launch;
+        args.o_begin = o_begin + first * kmc::NGF_TILE_O;
+        args.g.o_chunks = chunks;
+        const dim3 grid((args.g.m + kmc::NGF_TILE_M - 1) / kmc::NGF_TILE_M, (args.g.n + Tile::TILE_N - 1) / Tile::TILE_N,
+                        static_cast<unsigned>(args.g.l) * chunks);
+        const hipError_t status = launch(kmc::norm_gradient_l1_f16<BLOCKS, PIECES_IN_COLUMNS>, grid, dim3(kmc::NGF_THREADS), stream, args);
+        if (status != hipSuccess) return status;
+    }
+    return hipSuccess;
+}
+
+template <bool PIECES_IN_COLUMNS>
+hipError_t launch_products(int blocks, kmc::NormGradientF16Args &args, int o_begin, int o_chunks, hipStream_t stream)
+{
+    switch (blocks) {
+    case 16: return launch_product<16, PIECES_IN_COLUMNS>(args, o_begin, o_chunks, stream);
+    case 8: return launch_product<8, PIECES_IN_COLUMNS>(args, o_begin, o_chunks, stream);
+    case 4: return launch_product<4, PIECES_IN_COLUMNS>(args, o_begin, o_chunks, stream);
+    default: return launch_product<2, PIECES_IN_COLUMNS>(args, o_begin, o_chunks, stream);
+    }
 }
 
 }  // namespace
-
-hipError_t launch_gram_rows_pair(const kmc::GramRowsArgs &first, int first_batches, const kmc::GramRowsArgs &second, int second_batches,
-                                 hipStream_t stream);     // gram_f16_wide_inst.hip
 
 int64_t norm_gradient_f16_bytes(const kmc_norm_gradient_params *p)
 {
@@ -131,8 +158,7 @@ int64_t norm_gradient_f16_bytes(const kmc_norm_gradient_params *p)
 }
 
 // `*taken` says whether the route applied (and the launches were made); if not, nothing was launched.
-hipError_t launch_norm_gradient_f16(const kmc_norm_gradient_params *p, bool a_vec, bool c_vec, bool e_vec, hipStream_t stream,
-                                    bool *taken)
+hipError_t launch_norm_gradient_f16(const kmc_norm_gradient_params *p, bool a_vec, bool e_vec, hipStream_t stream, bool *taken)
 {
     *taken = false;
     GradientLayout layout;
@@ -140,53 +166,57 @@ hipError_t launch_norm_gradient_f16(const kmc_norm_gradient_params *p, bool a_ve
         (reinterpret_cast<uintptr_t>(p->workspace) & (REGION_ALIGN - 1)) != 0)
         return hipSuccess;
     char *workspace = static_cast<char *>(p->workspace);
-    (void)a_vec;
-    const kmc::GramRowsArgs rows_a = rows_args(p->a, p->a_ld, p->a_bs, p->m, false, false, p->k, layout, layout.a, workspace);
-    const kmc::GramRowsArgs rows_c = rows_args(p->c, p->c_ld, p->c_bs, p->o, true, c_vec, p->k, layout, layout.c, workspace);
-    hipError_t status = launch_gram_rows_pair(rows_a, layout.a.batches, rows_c, layout.c.batches, stream);
-    if (status != hipSuccess) return status;
-
-    kmc::GradientPadArgs pad = {};
-    pad.b = p->b; pad.b_ld = p->b_ld; pad.b_bs = p->b_bs;
-    pad.padded = reinterpret_cast<float *>(workspace + layout.b_padded); pad.padded_bs = layout.b_padded_bs;
-    pad.n = p->n; pad.k = p->k; pad.n_pad = layout.n_pad; pad.k_pad = layout.k_pad;
-    status = launch(kmc::gradient_pad_b, dim3((layout.k_pad / 4 + 255) / 256, layout.n_pad, layout.b_batches), dim3(256), stream, pad);
+    kmc::GradientPrepareArgs prepare = {};
+    prepare.m = p->m; prepare.n = p->n; prepare.o = p->o; prepare.k = p->k;
+    prepare.a = p->a; prepare.a_ld = p->a_ld; prepare.a_bs = p->a_bs; prepare.a_vec = a_vec;
+    prepare.b = p->b; prepare.b_ld = p->b_ld; prepare.b_bs = p->b_bs;
+    prepare.c = p->c; prepare.c_ld = p->c_ld; prepare.c_bs = p->c_bs;
+    prepare.d = p->d; prepare.d_ld = p->d_ld; prepare.d_bs = p->d_bs;
+    prepare.positions = reinterpret_cast<unsigned short *>(workspace + layout.positions); prepare.positions_bs = layout.positions_bs;
+    prepare.counts = reinterpret_cast<unsigned short *>(workspace + layout.counts); prepare.counts_bs = layout.counts_bs;
+    prepare.a_copy = reinterpret_cast<float *>(workspace + layout.a_copy); prepare.a_copy_bs = layout.a_copy_bs;
+    prepare.a_magnitudes = reinterpret_cast<float *>(workspace + layout.a_magnitudes); prepare.a_magnitudes_bs = layout.a_magnitudes_bs;
+    prepare.c_pieces = reinterpret_cast<kmc::gram_chunk *>(workspace + layout.c_pieces); prepare.c_pieces_bs = layout.c_pieces_bs;
+    prepare.c_unscale = reinterpret_cast<float *>(workspace + layout.c_unscale); prepare.c_unscale_bs = layout.o_pad;
+    prepare.n_pad = layout.n_pad; prepare.m_pad = layout.m_pad; prepare.k_pad = layout.k_pad; prepare.o_pad = layout.o_pad;
+    prepare.sort_d = layout.sort_d;
+    prepare.ranges = layout.ranges; prepare.chunks = layout.chunks; prepare.chunk_k = layout.chunk_k;
+    prepare.sort_blocks = p->n * layout.chunks;
+    prepare.copy_blocks = layout.m_pad / kmc::NGF_COPY_M * layout.ranges;
+    prepare.sort_batches = layout.sort_batches; prepare.a_batches = layout.a_batches; prepare.c_batches = layout.c_batches;
+    const int batches = layout.sort_batches > 1 || layout.a_batches > 1 || layout.c_batches > 1 ? p->l : 1;
+    prepare.sort_groups = (prepare.sort_blocks + kmc::NGF_PREPARE_GROUP - 1) / kmc::NGF_PREPARE_GROUP;
+    prepare.copy_groups = (prepare.copy_blocks + kmc::NGF_PREPARE_GROUP - 1) / kmc::NGF_PREPARE_GROUP;
+    const dim3 prepare_grid((prepare.sort_groups + prepare.copy_groups) * kmc::NGF_PREPARE_GROUP + layout.o_pad, batches);
+    const dim3 prepare_threads(kmc::NGF_PREPARE_THREADS);
+    hipError_t status;
+    if (layout.keys <= 1024) status = launch(kmc::gradient_signs_prepare<2>, prepare_grid, prepare_threads, stream, prepare);
+    else if (layout.keys <= 2048) status = launch(kmc::gradient_signs_prepare<3>, prepare_grid, prepare_threads, stream, prepare);
+    else if (layout.keys <= 4096) status = launch(kmc::gradient_signs_prepare<4>, prepare_grid, prepare_threads, stream, prepare);
+    else if (layout.keys <= 8192) status = launch(kmc::gradient_signs_prepare<5>, prepare_grid, prepare_threads, stream, prepare);
+    else status = launch(kmc::gradient_signs_prepare<6>, prepare_grid, prepare_threads, stream, prepare);
     if (status != hipSuccess) return status;
 
     kmc::NormGradientF16Args args = {};
     args.g.m = p->m; args.g.n = p->n; args.g.o = p->o; args.g.k = p->k; args.g.l = p->l;
-    args.g.d = p->d; args.g.d_ld = p->d_ld; args.g.d_bs = p->d_bs;
     args.g.e = p->e; args.g.e_ld_n = p->e_ld_n; args.g.e_ld_o = p->e_ld_o; args.g.e_bs = p->e_bs;
     args.g.e_vec = e_vec;
-    args.pieces_a = rows_a.pieces; args.pieces_c = rows_c.pieces;
-    args.pieces_a_bs = layout.a.batches > 1 ? layout.a.pieces_bs : 0;
-    args.pieces_c_bs = layout.c.batches > 1 ? layout.c.pieces_bs : 0;
-    args.unscale_a = rows_a.unscale; args.unscale_c = rows_c.unscale;
-    args.unscale_a_bs = layout.a.batches > 1 ? layout.a.rows_pad : 0;
-    args.unscale_c_bs = layout.c.batches > 1 ? layout.c.rows_pad : 0;
-    args.b_padded = pad.padded;
-    args.b_padded_bs = layout.b_batches > 1 ? layout.b_padded_bs : 0;
-    args.rows_pad_a = layout.a.rows_pad; args.rows_pad_c = layout.c.rows_pad;
-    args.k_pad = layout.k_pad; args.steps = layout.steps;
-    // Outputs in chunks of 64 on the 8 n x 64 o tile while more than 32 are left, then one chunk of 32 on the
-    // 16 n x 32 o tile for 17 to 32 of them, or the 32 n x 16 o tile for up to 16.
-    int wide_chunks = p->o / 64;
-    int left = p->o % 64;
-    if (left > 32) { wide_chunks += 1; left = 0; }
-    const unsigned tiles_m = (p->m + kmc::NGF_TILE_M - 1) / kmc::NGF_TILE_M;
-    auto run = [&](auto blocks, int o_begin, int chunks) {
-        using Tile = kmc::GradientF16Tile<decltype(blocks)::value>;
-        args.o_begin = o_begin;
-        args.g.o_chunks = chunks;
-        const dim3 grid(tiles_m, (p->n + Tile::TILE_N - 1) / Tile::TILE_N, static_cast<unsigned>(p->l) * chunks);
-        return launch(kmc::norm_gradient_l1_f16<decltype(blocks)::value>, grid, dim3(kmc::NGF_THREADS), stream, args);
-    };
-    if (wide_chunks) {
-        status = run(std::integral_constant<int, 4>{}, 0, wide_chunks);
-        if (status != hipSuccess) return status;
-    }
-    if (left > 16) status = run(std::integral_constant<int, 2>{}, p->o - left, 1);
-    else if (left > 0) status = run(std::integral_constant<int, 1>{}, p->o - left, 1);
+    args.positions = prepare.positions; args.counts = prepare.counts;
+    args.positions_bs = layout.sort_batches > 1 ? layout.positions_bs : 0;
+    args.counts_bs = layout.sort_batches > 1 ? layout.counts_bs : 0;
+    args.a_copy = prepare.a_copy; args.a_copy_bs = layout.a_batches > 1 ? layout.a_copy_bs : 0;
+    args.a_magnitudes = prepare.a_magnitudes; args.a_magnitudes_bs = layout.a_batches > 1 ? layout.a_magnitudes_bs : 0;
+    args.c_pieces = prepare.c_pieces; args.c_pieces_bs = layout.c_batches > 1 ? layout.c_pieces_bs : 0;
+    args.c_unscale = prepare.c_unscale; args.c_unscale_bs = layout.c_batches > 1 ? layout.o_pad : 0;
+    args.n_pad = layout.n_pad; args.m_pad = layout.m_pad; args.k_pad = layout.k_pad; args.ranges = layout.ranges;
+    args.chunks = layout.chunks; args.chunk_stages = layout.chunk_k / kmc::NGF_STAGE_K; args.stages = layout.stages;
+    // blocks of 16 outputs; what is left up to 8 in the first half of the columns, its second pieces in the other
+    const int left = p->o % kmc::NGF_TILE_O;
+    const int in_columns = left > 0 && left <= 8 ? 1 : 0;
+    const int full_chunks = (p->o + kmc::NGF_TILE_O - 1) / kmc::NGF_TILE_O - in_columns;
+    const int blocks = blocks_for(p, full_chunks + in_columns);
+    if (full_chunks) status = launch_products<false>(blocks, args, 0, full_chunks, stream);
+    if (status == hipSuccess && in_columns) status = launch_products<true>(blocks, args, p->o - left, 1, stream);
     if (status == hipSuccess) *taken = true;
     return status;
 }

@@ -132,3 +132,43 @@ def test_without_a_workspace_the_fp32_kernels_run(device, f16_route, monkeypatch
         plan.params.workspace, plan.params.workspace_bytes = pointer, size
         _backend.norm_kernel_gradient(plan.params, stream)
         assert torch.equal(plan.out, reference), "null, short or misaligned workspace: expected the fp32 kernel's bits"
+
+
+@pytest.mark.parametrize("M,N,O,K", [(16, 33, 9, 64), (200, 257, 8, 65), (17, 129, 16, 63), (1025, 31, 3, 1024), (1024, 65, 16, 1025),
+                                     (2049, 10, 16, 2048), (4096, 6, 4, 4097), (300, 5, 17, 8192), (8193, 4, 2, 8200), (40, 300, 24, 700),
+                                     (600, 3, 1, 30000),            # more k than are sorted at once: the rows of d are
+                                     (14300, 2, 1, 14400)])         # more of both: b sorted in two chunks
+def test_signs_are_exact(device, f16_route, M, N, O, K):
+    """Small integers in a and c make every product and partial sum exact, so one wrong sign changes the result.  b and d
+    are drawn from few values (ties), with signed zeros and infinities among them."""
+    g = torch.Generator().manual_seed(M + N + O + K)
+    a = torch.randint(-3, 4, (K, M), generator=g).float().to(device)
+    c = torch.randint(-3, 4, (O, K), generator=g).float().to(device)
+    values = torch.cat([torch.linspace(-1, 1, 61), torch.tensor([0.0, -0.0, 1e-42, -1e-42, 3e38])])
+    b = values[torch.randint(len(values), (N, K), generator=g)].to(device)
+    d = values[torch.randint(len(values), (N, M), generator=g)].to(device)
+    d[0, 0], d[-1, -1] = float("inf"), float("-inf")
+    assert workspace_bytes(a, b, c, d) > 0
+    got = kermac.cdist_grad(a, b, c, d, p=1.0)[0]
+    for n in range(N):
+        sign = torch.copysign(torch.ones((), device=device), d[n][None, :] - b[n][:, None])
+        truth = c.double() @ (sign.double() * a.double())
+        assert torch.equal(got[:, n, :].double(), truth), f"n = {n}"
+
+
+def test_rounding_follows_the_signed_sums(device):
+    """The matrix instruction sums S a c with S in {0, 1}, half of sum a c taken off on the way: weights of one sign must not
+    lose more than the signed sums do.  Bound: the square root of 2 K / 32 roundings of 2^-24 of the root of K terms, and the
+    pieces' 3 * 2^-22 per term; the fp32 route's error is of the same size."""
+    g = torch.Generator().manual_seed(8)
+    M, N, O, K = 4096, 48, 16, 4096
+    a = torch.exp(-10 * torch.rand(K, M, generator=g)).to(device)
+    c = torch.randn(O, K, generator=g).to(device)
+    b, d = torch.randn(N, K, generator=g).to(device), torch.randn(N, M, generator=g).to(device)
+    got = kermac.cdist_grad(a, b, c, d, p=1.0)[0]
+    worst = 0.0
+    for n in range(0, N, 7):
+        sign = torch.copysign(torch.ones((), device=device), d[n][None, :] - b[n][:, None]).double()
+        truth = c.double() @ (sign * a.double())
+        worst = max(worst, float((got[:, n].double() - truth).norm() / truth.norm()))
+    assert worst < (2 * K / 32) ** 0.5 * 2.0 ** -24 + 3 * 2.0 ** -22
