@@ -45,6 +45,12 @@
     /* the direct kernel in tiles of 64 x 64: up to this many tiles of 128 x 128 over the batch */        \
     X(DIRECT_SMALL_MAX_TILES, 256)                                                                      \
     X(DIRECT_SMALL_MAX_TILES_ROOTS, 192)   /* ... and for fractional powers */                          \
+    /* the direct kernel for contractions of few terms (no root or fractional power), above those tiles; and for two different */ \
+    /* sets from so many columns on up to 12 terms, 13 to 16 where the result is not aligned, more from so many tiles on */  \
+    X(DIRECT_SHORT_ANY_MAX_K, 8)                                                                        \
+    X(DIRECT_SHORT_MAX_K, 24)                                                                           \
+    X(DIRECT_SHORT_MIN_COLUMNS, 1024)                                                                   \
+    X(DIRECT_SHORT_LONG_MIN_TILES, 1024)                                                                \
     /* the direct kernel compiled for four waves per SIMD (k-major panels, no fractional power) */       \
     X(DIRECT_FOUR_WAVES_MIN_K, 256)                                                                     \
     /* ... and the one with b in scalar registers (absolute and squared differences, K and N multiples of 16): */ \

@@ -8,6 +8,7 @@
 #include "launch.hpp"
 #include "build_kernel.hpp"
 #include "build_kernel_scalar_b.hpp"
+#include "build_kernel_short.hpp"
 #include "build_kernel_small.hpp"
 #include "../host/dispatch_rules.hpp"
 
@@ -126,8 +127,69 @@ static bool small_applies(int load_a, int load_b, const kmc::BuildKernelArgs &ar
     return tiles <= (limit ? std::atoi(limit) : HAS_ROOT_OR_POWER ? kmc_rules::DIRECT_SMALL_MAX_TILES_ROOTS : kmc_rules::DIRECT_SMALL_MAX_TILES);
 }
 
+// Contractions of up to 24 terms, whose launches the stores of the result bound (build_kernel_short.hpp).  It pays a load of all k of
+// its rows per workgroup and a term at 3.5 cycles an instruction, where the ordinary kernel pays whole slices of 16 k.  Ordinary / this kernel,
+// us, p = 1, K = 6, 10, 16, 24: 10000 x 10000, rows 16-byte aligned 99 / 80, 103 / 92, 105 / 112, 153 / 150; 2 x 7000 x 7001, result not
+// aligned 182 / 84, 184 / 99, 160 / 117, 231 / 154; 5000 x 5000 35 / 24, 37 / 28, 37 / 32, 49 / 45; 3000 x 2500 16.8 / 13.9, 16.7 / 15.8, 16.2 / 17.8,
+// 21.6 / 24.4; 30000 rows against 300, whose loads of a
+// meet few columns, 17.6 / 14.8, 17.5 / 17.8, 17.7 / 19.8, 26.0 / 24.2 and with k contiguous 19.5 / 18.4, 19.6 / 23.0, 19.6 / 23.8, 27.6 / 33.9.  A set against
+// itself, computed in full here, 2 x 10000, K = 6 and 12, Laplace kernel 226 / 196 and 223 / 233.
+// KERMAC_AMD_DIRECT_SHORT_MAX_K=n replaces the rule by "at most n terms" (read on every call, so that a test can choose the kernel).
+constexpr bool HAS_SHORT = !HAS_ROOT_OR_POWER;
+
+static bool short_applies(int load_a, int load_b, const kmc::BuildKernelArgs &args)
+{
+    if (!HAS_SHORT || args.repair_only || args.k_total != 0 || args.panels != 0 || args.k < 1 || args.k > kmc_rules::DIRECT_SHORT_MAX_K ||
+        args.l > 65535 || args.n > (1 << 22))
+        return false;
+    const char *limit = std::getenv("KERMAC_AMD_DIRECT_SHORT_MAX_K");
+    if (limit) return args.k <= std::atoi(limit);
+    // a test that chooses between the other kernels
+    int64_t grid_width = 0;
+    if (std::getenv("KERMAC_AMD_DIRECT_SMALL_MAX_TILES") ||
+        (HAS_SCALAR_B && load_a == kmc::LOAD_COL_VEC && load_b == kmc::LOAD_COL_VEC && scalar_b_applies(args, &grid_width)))
+        return false;
+    const int64_t tiles = static_cast<int64_t>(args.tiles_m) * args.tiles_n * args.l;
+    if (tiles <= kmc_rules::DIRECT_SMALL_MAX_TILES) return false;          // for build_kernel_small
+    if (args.k <= kmc_rules::DIRECT_SHORT_ANY_MAX_K) return true;
+    if (args.symmetric) return false;
+    if (args.n < kmc_rules::DIRECT_SHORT_MIN_COLUMNS) return false;
+    if (args.k <= 12) return true;
+    if (args.k <= kmc::BK_TILE_K) return !args.c_vec;
+    return tiles >= kmc_rules::DIRECT_SHORT_LONG_MIN_TILES;
+}
+
+template <int DEPTH>
+static hipError_t launch_short(int load_a, int load_b, const kmc::BuildKernelArgs &args, hipStream_t stream)
+{
+    // columns this many apart start at the same place in a line of 32 floats
+    int classes = kmc::BKT_LINE;
+    while (classes > 1 && args.c_ld % (2 * kmc::BKT_LINE / classes) == 0) classes /= 2;
+    const int64_t m_tiles = (static_cast<int64_t>(args.m) + kmc::BKT_LINE - 1 + kmc::BKT_TILE_M - 1) / kmc::BKT_TILE_M;
+    // rounds of 16 columns per workgroup: as many as the loads of a are worth, as few as fill the chip
+    int rounds = kmc::BKT_MAX_ROUNDS;
+    while (rounds > 1 && m_tiles * (args.n / (rounds * kmc::BKT_COLUMNS) + 1) * args.l < 1024) rounds /= 2;
+    const int64_t per_group = static_cast<int64_t>(rounds) * kmc::BKT_COLUMNS * classes;
+    const int64_t groups = (args.n + per_group - 1) / per_group * classes;
+    kmc::BuildKernelArgs copy = args;
+    void *kernel_args[] = {&copy, &load_a, &load_b, &rounds, &classes};
+    return hipLaunchKernel(reinterpret_cast<const void *>(kmc::build_kernel_short<KMC_INNER_OP, KMC_INNER_POW, DEPTH>),
+                           dim3(static_cast<unsigned>(m_tiles), static_cast<unsigned>(groups), args.l), dim3(kmc::BK_THREADS), kernel_args, 0, stream);
+}
+
 hipError_t KMC_LAUNCHER_NAME(int load_a, int load_b, const kmc::BuildKernelArgs &args, dim3 grid, hipStream_t stream)
 {
+    if constexpr (HAS_SHORT)
+        if (short_applies(load_a, load_b, args)) {
+            switch ((args.k + 3) / 4) {
+            case 1: return launch_short<4>(load_a, load_b, args, stream);
+            case 2: return launch_short<8>(load_a, load_b, args, stream);
+            case 3: return launch_short<12>(load_a, load_b, args, stream);
+            case 4: return launch_short<16>(load_a, load_b, args, stream);
+            case 5: return launch_short<20>(load_a, load_b, args, stream);
+            default: return launch_short<24>(load_a, load_b, args, stream);
+            }
+        }
     if (small_applies(load_a, load_b, args)) {
         const int across = (args.m + kmc::BKS_TILE - 1) / kmc::BKS_TILE, down = (args.n + kmc::BKS_TILE - 1) / kmc::BKS_TILE;
         kmc::BuildKernelArgs copy = args;

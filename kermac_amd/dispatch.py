@@ -87,6 +87,11 @@ _ROWS = (
      "direct `build_kernel` (ahead of time for DIFF + NOOP/ABS/SQUARE/POW and DOT + NOOP, else compiled on first use); scalar p of 0.5, 1.5, 3, 4 on "
      "the exact-form variants"),
     ("every direct launch",
+     "more than {DIRECT_SMALL_MAX_TILES} tiles of 128 × 128 over the batch and K ≤ {DIRECT_SHORT_ANY_MAX_K}, or, of two different sets and a result of ≥ "
+     "{DIRECT_SHORT_MIN_COLUMNS} columns, K ≤ 12 (≤ 16 where its rows are not 16-byte aligned, 17 … {DIRECT_SHORT_MAX_K} from "
+     "{DIRECT_SHORT_LONG_MIN_TILES} tiles on); no root or fractional power, compiled ahead of time, not ranges of one contraction, not a repair launch",
+     "`build_kernel_short` (all k of a lane's rows in registers, whole lines stored)"),
+    ("",
      "≤ {DIRECT_SMALL_MAX_TILES} tiles of 128 × 128 over the batch, ≤ {DIRECT_SMALL_MAX_TILES_ROOTS} for fractional powers, compiled ahead of time, not ranges of one contraction, not a repair launch",
      "`build_kernel_small` (tiles of 64 × 64)"),
     ("",
