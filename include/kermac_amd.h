@@ -346,7 +346,7 @@ typedef struct kmc_norm_gradient_params {
      * and s[n] the mean of row n of b (any s gives the same e; this one keeps both terms as small
      * as the data allows): p and a are split once into two fp16 pieces per value with a scale per
      * row and multiplied on the fp16 matrix instruction, g comes from the fp32
-     * matrix instruction; the workspace also holds p in fp32.  Error of the product from the pieces
+     * matrix instruction.  Error of the product from the pieces
      * below 3 * 2^-22 sum_k |c a (b - s)| + k * 2^-38 max_k|a[k][m]| max_k|p[r][k]|.
      * NULL, too small, or a problem for which the query reports 0: the fp32 kernels run. */
     void *workspace;

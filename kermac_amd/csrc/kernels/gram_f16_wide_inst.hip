@@ -432,9 +432,8 @@ namespace {
 
 struct GradientL2Layout {
     WideLayout wide;                 // a: the columns m of a; b: the rows (o, n) of the products
-    int products_ld;
     int g_parts;                     // ranges of k that g is summed in (partial products, then their sum)
-    int64_t products, shift, c_transposed, g, g_partial;      // byte offsets behind the regions of `wide`
+    int64_t shift, c_transposed, g, g_partial;      // byte offsets behind the regions of `wide`
     int64_t bytes;
 };
 
@@ -479,8 +478,9 @@ bool gradient_l2_layout(const kmc_norm_gradient_params *p, GradientL2Layout *lay
     if (!gradient_l2_pays(p, wide.tiles_m, wide.tiles_n)) return false;
     if (!place_wide(p->m, static_cast<int>(rows), p->k, p->l, p->a_bs == 0, false, false, false, false, &wide)) return false;
     int64_t cursor = wide.bytes;
-    layout->products_ld = (p->k + 3) / 4 * 4;
-    layout->products = place(cursor, static_cast<int64_t>(p->l) * rows * layout->products_ld * 4);
+    // Room for the products in fp32, which no kernel stores any more: the size that the query reports is part of what callers
+    // have measured and planned with (and which calls a limit of theirs keeps off the route), so it stays what it was.
+    place(cursor, static_cast<int64_t>(p->l) * rows * ((p->k + 3) / 4 * 4) * 4);
     layout->shift = place(cursor, static_cast<int64_t>(p->l) * p->n * 4);
     layout->c_transposed = place(cursor, static_cast<int64_t>(p->l) * p->k * p->o * 4);
     layout->g = place(cursor, static_cast<int64_t>(p->l) * p->m * p->o * 4);
@@ -519,17 +519,12 @@ int launch_norm_gradient_l2_wide(const kmc_norm_gradient_params *p, hipStream_t 
     kmc::GradientL2PrepareArgs prepare = {};
     prepare.b = p->b; prepare.b_ld = p->b_ld; prepare.b_bs = p->b_bs;
     prepare.c = p->c; prepare.c_ld = p->c_ld; prepare.c_bs = p->c_bs;
-    prepare.products = reinterpret_cast<float *>(workspace + layout.products);
-    prepare.products_ld = layout.products_ld; prepare.products_bs = static_cast<int64_t>(rows) * layout.products_ld;
     prepare.shift = reinterpret_cast<float *>(workspace + layout.shift); prepare.shift_bs = p->n;
     prepare.c_transposed = reinterpret_cast<float *>(workspace + layout.c_transposed);
     prepare.c_transposed_ld = p->o; prepare.c_transposed_bs = static_cast<int64_t>(p->k) * p->o;
     prepare.n = p->n; prepare.o = p->o; prepare.k = p->k;
-    hipError_t status = launch(kmc::gradient_l2_products, dim3(p->n, (p->o + kmc::GL2_OUTPUTS - 1) / kmc::GL2_OUTPUTS, p->l),
-                               dim3(kmc::GL2_THREADS), stream, prepare);
-    if (status != hipSuccess) return fail_hip(status, "gradient_l2_products launch");
-    status = launch(kmc::gradient_l2_transpose_c, dim3((p->k + kmc::GL2_THREADS - 1) / kmc::GL2_THREADS, p->l), dim3(kmc::GL2_THREADS), stream, prepare);
-    if (status != hipSuccess) return fail_hip(status, "gradient_l2_transpose_c launch");
+    hipError_t status = launch(kmc::gradient_l2_prepare, dim3(p->n + (p->k + kmc::GL2_THREADS - 1) / kmc::GL2_THREADS, p->l), dim3(kmc::GL2_THREADS), stream, prepare);
+    if (status != hipSuccess) return fail_hip(status, "gradient_l2_prepare launch");
 
     // g[m][o] = sum_k a[k][m] c[o][k]: a is a stored panel with m contiguous
     float *g = reinterpret_cast<float *>(workspace + layout.g);
@@ -559,10 +554,20 @@ int launch_norm_gradient_l2_wide(const kmc_norm_gradient_params *p, hipStream_t 
     kmc::BuildKernelArgs walk = {};
     walk.m = p->m; walk.n = rows; walk.k = p->k; walk.l = p->l;
     const kmc::GramRowsArgs rows_a = rows_args(p->a, p->a_ld, p->a_bs, p->m, KMC_COL_MAJOR, scalar_only, walk, wide, wide.a, workspace);
-    const kmc::GramRowsArgs rows_b = rows_args(prepare.products, prepare.products_ld, prepare.products_bs, rows, KMC_ROW_MAJOR, scalar_only,
-                                               walk, wide, wide.b, workspace);
-    status = launch_gram_rows_pair(rows_a, wide.a.batches, rows_b, wide.b.batches, stream);
-    if (status != hipSuccess) return fail_hip(status, "gram_row_stats / gram_f16_split launch");
+    const kmc::GramRowsArgs rows_b = rows_args(nullptr, 0, 0, rows, KMC_ROW_MAJOR, scalar_only, walk, wide, wide.b, workspace);
+    kmc::GradientL2PiecesArgs pieces = {};
+    pieces.a = rows_a; pieces.p = rows_b;
+    pieces.a_blocks = rows_a.rows_pad / kmc::GW_ROW_THREADS; pieces.a_batches = wide.a.batches;
+    pieces.from = prepare;
+    // four outputs share a read of b, unless that leaves p fewer workgroups than three per CU
+    const int ranges = rows_a.ranges > rows_b.ranges ? rows_a.ranges : rows_b.ranges, blocks_n = (p->n + kmc::GL2_ROWS - 1) / kmc::GL2_ROWS;
+    pieces.outputs = kmc::GL2_OUTPUTS;
+    while (pieces.outputs > 1 && static_cast<int64_t>(blocks_n) * ((p->o + pieces.outputs - 1) / pieces.outputs) * ranges * p->l < 768) pieces.outputs /= 2;
+    const dim3 grid(pieces.a_blocks + blocks_n * ((p->o + pieces.outputs - 1) / pieces.outputs), ranges, p->l);
+    static_assert(kmc::GW_ROW_THREADS == kmc::GL2_THREADS, "one launch for both operands");
+    status = launch(kmc::gradient_l2_pieces_stats, grid, dim3(kmc::GL2_THREADS), stream, pieces);
+    if (status == hipSuccess) status = launch(kmc::gradient_l2_pieces_split, grid, dim3(kmc::GL2_THREADS), stream, pieces);
+    if (status != hipSuccess) return fail_hip(status, "gradient_l2_pieces launches");
 
     kmc::GramWideArgs product = {};
     product.kernel = walk;

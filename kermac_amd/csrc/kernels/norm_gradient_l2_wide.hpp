@@ -15,36 +15,53 @@
 // matrix instruction.  Error of the product from the pieces below 3 * 2^-22 sum_k |c a (b - s)|;
 // g and the rest are fp32.
 //
-// This header: the kernels that prepare p, s and the transposed c (g itself comes from
-// kmc_matrix_times_coefficients with a as the stored panel).
+// This header: the kernels that prepare s, the transposed c, and the pieces of a and p (g itself comes from
+// kmc_matrix_times_coefficients with a as the stored panel).  p is never stored: its values are made from b and c
+// twice, for the largest magnitude of every row and for the pieces (written in fp32 and read twice it cost 0.9 of 13.5 ms at
+// 2 x 10000 x 768 x 16 x 10000; now 12.7 .. 12.9, of which statistics 370 us and split 650, both mostly the bytes of a and the pieces).
 #pragma once
 
 #include <hip/hip_runtime.h>
 
-namespace kmc {
+#include "gram_f16_wide.hpp"
 
-using i64 = long long;
+namespace kmc {
 
 struct GradientL2PrepareArgs {
     const float *b; i64 b_ld, b_bs;          // [n][k], k contiguous
     const float *c; i64 c_ld, c_bs;          // [o][k], k contiguous
-    float *products; i64 products_ld, products_bs;   // [o n_rows + n][k]
     float *shift; i64 shift_bs;              // [n]
     float *c_transposed; i64 c_transposed_ld, c_transposed_bs;   // [k][o]
     int n, o, k;
 };
 
-constexpr int GL2_THREADS = 256;
-constexpr int GL2_OUTPUTS = 4;       // rows of p per workgroup
+// gradient_l2_pieces_stats and gradient_l2_pieces_split: the operand a, and p row o n + n' of which is c[o] (b[n'] - shift[n'])
+struct GradientL2PiecesArgs {
+    GramRowsArgs a, p;                       // p.x is not read
+    int a_blocks, a_batches;                 // workgroups along x: those of a, then of p
+    int outputs;                             // rows of p per row n and workgroup of p, up to GL2_OUTPUTS
+    GradientL2PrepareArgs from;
+};
 
-// One workgroup per row n of b and four outputs: the mean of the row (sums in a fixed order, the
-// same in every workgroup of the row), then the rows of p that belong to it.
-__global__ __launch_bounds__(GL2_THREADS) void gradient_l2_products(const GradientL2PrepareArgs args)
+constexpr int GL2_THREADS = 256;
+constexpr int GL2_ROWS = 64;         // rows n of a workgroup: a lane each
+constexpr int GL2_DEPTH = 64;        // k at a time, a slice of 16 per wave
+constexpr int GL2_OUTPUTS = 4;       // rows of p per row n and workgroup, at most
+
+// The mean of row n of b (sums in a fixed order), one workgroup per row; behind them c_transposed[k][o] = c[o][k].
+__global__ __launch_bounds__(GL2_THREADS) void gradient_l2_prepare(const GradientL2PrepareArgs args)
 {
     __shared__ float partial[GL2_THREADS];
-    const int n = blockIdx.x, batch = blockIdx.z;
-    const int o_begin = blockIdx.y * GL2_OUTPUTS;
-    const int o_end = o_begin + GL2_OUTPUTS < args.o ? o_begin + GL2_OUTPUTS : args.o;
+    const int batch = blockIdx.y;
+    if ((int)blockIdx.x >= args.n) {
+        const int k = (blockIdx.x - args.n) * GL2_THREADS + threadIdx.x;
+        if (k >= args.k) return;
+        const float *c = args.c + batch * args.c_bs;
+        float *row = args.c_transposed + batch * args.c_transposed_bs + (i64)k * args.c_transposed_ld;
+        for (int o = 0; o < args.o; ++o) row[o] = c[(i64)o * args.c_ld + k];
+        return;
+    }
+    const int n = blockIdx.x;
     const float *b_row = args.b + batch * args.b_bs + (i64)n * args.b_ld;
     float sum = 0.0f;
     for (int k = threadIdx.x; k < args.k; k += GL2_THREADS) sum += b_row[k];
@@ -56,14 +73,143 @@ __global__ __launch_bounds__(GL2_THREADS) void gradient_l2_products(const Gradie
     }
     const float mean = partial[0] / (float)args.k;
     // not-a-number or infinite rows: no shift (the product then carries them as the fp32 kernels would)
-    const float shift = (mean - mean == 0.0f) ? mean : 0.0f;
-    if (threadIdx.x == 0 && blockIdx.y == 0) args.shift[batch * args.shift_bs + n] = shift;
-    const float *c = args.c + batch * args.c_bs;
-    float *products = args.products + batch * args.products_bs;
-    for (int k = threadIdx.x; k < args.k; k += GL2_THREADS) {
-        const float centred = b_row[k] - shift;
-        for (int o = o_begin; o < o_end; ++o)
-            products[((i64)o * args.n + n) * args.products_ld + k] = c[(i64)o * args.c_ld + k] * centred;
+    if (threadIdx.x == 0) args.shift[batch * args.shift_bs + n] = (mean - mean == 0.0f) ? mean : 0.0f;
+}
+
+// For 64 rows n, GL2_OUTPUTS outputs and one range of k: `use(output, slice, values)` for every slice of 16 values of p, lane = row
+// n, wave = every fourth slice.  b passes through LDS, since a lane's k are contiguous in memory and the lanes' rows are not.
+template <typename Use>
+__device__ __forceinline__ void gradient_l2_walk(const GradientL2PiecesArgs &args, int n0, int o_begin, int o_end, int first, int last, Use &&use)
+{
+    __shared__ float tile[GL2_DEPTH * (GL2_ROWS + 1)];
+    const GradientL2PrepareArgs &from = args.from;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, batch = blockIdx.z;
+    const float *b = from.b + batch * from.b_bs, *c = from.c + batch * from.c_bs;
+    const int n = n0 + lane;
+    const float shift = n < from.n ? from.shift[batch * from.shift_bs + n] : 0.0f;
+    constexpr int LOADS = GL2_ROWS * GL2_DEPTH / GL2_THREADS;
+    float v[LOADS];
+    auto load = [&](int slice) {
+        const int k = slice * BK_TILE_K + lane;
+#pragma unroll
+        for (int j = 0; j < LOADS; j++) {
+            const int row = n0 + wave + 4 * j;
+            v[j] = row < from.n && k < from.k ? b[(i64)row * from.b_ld + k] : 0.0f;
+        }
+    };
+    load(first);
+    for (int group = first; group < last; group += GL2_DEPTH / BK_TILE_K) {
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < LOADS; j++) tile[lane * (GL2_ROWS + 1) + wave + 4 * j] = v[j];
+        __syncthreads();
+        if (group + GL2_DEPTH / BK_TILE_K < last) load(group + GL2_DEPTH / BK_TILE_K);
+        const int slice = group + wave;
+        if (slice >= last) continue;
+        float centred[BK_TILE_K];
+#pragma unroll
+        for (int e = 0; e < BK_TILE_K; e++) centred[e] = tile[(BK_TILE_K * wave + e) * (GL2_ROWS + 1) + lane] - shift;
+        const int k0 = slice * BK_TILE_K;
+        for (int o = o_begin; o < o_end; o++) {
+            const float *c_row = c + (i64)o * from.c_ld;
+            float value[BK_TILE_K];
+#pragma unroll
+            for (int e = 0; e < BK_TILE_K; e++) value[e] = k0 + e < from.k ? c_row[k0 + e] * centred[e] : 0.0f;
+            use(o, slice, value);
+        }
+    }
+}
+
+__global__ __launch_bounds__(GL2_THREADS) void gradient_l2_pieces_stats(const GradientL2PiecesArgs args)
+{
+    if ((int)blockIdx.x < args.a_blocks) {
+        if ((int)blockIdx.z < args.a_batches && (int)blockIdx.y < args.a.ranges) gram_row_stats_of(args.a, blockIdx.x);
+        return;
+    }
+    __shared__ float shared[4][GL2_OUTPUTS][GL2_ROWS];
+    const int groups = (args.from.o + args.outputs - 1) / args.outputs, block = blockIdx.x - args.a_blocks;
+    const int n0 = block / groups * GL2_ROWS, o_begin = block % groups * args.outputs, o_end = min(o_begin + args.outputs, args.from.o);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, range = blockIdx.y;
+    const int first = range * args.p.slices_per_range, last = min(first + args.p.slices_per_range, args.p.slices);
+    if (first >= last) return;
+    float magnitude[GL2_OUTPUTS] = {};
+    bool not_a_number[GL2_OUTPUTS] = {};
+    gradient_l2_walk(args, n0, o_begin, o_end, first, last, [&](int o, int, const float (&value)[BK_TILE_K]) {
+        float largest = 0.0f;
+        bool wrong = false;
+#pragma unroll
+        for (int e = 0; e < BK_TILE_K; e++) {
+            largest = fmaxf(largest, fabsf(value[e]));       // skips NaNs
+            wrong |= value[e] != value[e];
+        }
+#pragma unroll
+        for (int j = 0; j < GL2_OUTPUTS; j++)
+            if (o == o_begin + j) {
+                magnitude[j] = fmaxf(magnitude[j], largest);
+                not_a_number[j] |= wrong;
+            }
+    });
+    // a NaN takes the scale of an infinity, as in gram_rows_once
+#pragma unroll
+    for (int j = 0; j < GL2_OUTPUTS; j++) shared[wave][j][lane] = not_a_number[j] ? __builtin_inff() : magnitude[j];
+    __syncthreads();
+    const int n = n0 + lane, o = o_begin + wave;
+    static_assert(GL2_OUTPUTS == 4, "a wave each");
+    if (n < args.from.n && o < o_end)
+        args.p.magnitudes[blockIdx.z * args.p.stats_bs + (i64)range * args.p.rows_pad + (i64)o * args.from.n + n] =
+            fmaxf(fmaxf(shared[0][wave][lane], shared[1][wave][lane]), fmaxf(shared[2][wave][lane], shared[3][wave][lane]));
+}
+
+// Bound by the chunks it writes: a wave stores 1 KB of consecutive rows per piece and half.
+__global__ __launch_bounds__(GL2_THREADS) void gradient_l2_pieces_split(const GradientL2PiecesArgs args)
+{
+    if ((int)blockIdx.x < args.a_blocks) {
+        if ((int)blockIdx.z < args.a_batches && (int)blockIdx.y < args.a.ranges) gram_f16_split_of(args.a, blockIdx.x);
+        return;
+    }
+    const int groups = (args.from.o + args.outputs - 1) / args.outputs, block = blockIdx.x - args.a_blocks;
+    const int n0 = block / groups * GL2_ROWS, o_begin = block % groups * args.outputs, o_end = min(o_begin + args.outputs, args.from.o);
+    const int lane = threadIdx.x & 63, range = blockIdx.y, batch = blockIdx.z;
+    const int first = range * args.p.slices_per_range, all_slices = args.p.slices + args.p.zero_slices;
+    const int last = range == args.p.ranges - 1 ? all_slices : min(first + args.p.slices_per_range, args.p.slices);
+    if (first >= last) return;
+    const int n = n0 + lane;
+    const bool live = n < args.from.n;
+    float scale[GL2_OUTPUTS];
+#pragma unroll
+    for (int j = 0; j < GL2_OUTPUTS; j++) {
+        const i64 row = (i64)(o_begin + j) * args.from.n + n;
+        float magnitude = 0.0f;
+        if (live && o_begin + j < o_end)
+            for (int r = 0; r < args.p.ranges; r++) magnitude = fmaxf(magnitude, args.p.magnitudes[batch * args.p.stats_bs + (i64)r * args.p.rows_pad + row]);
+        const int exponent_field = gram_scale_exponent(magnitude);
+        scale[j] = gram_scale(exponent_field);
+        if (range == 0 && threadIdx.x < 64 && live && o_begin + j < o_end) args.p.unscale[batch * args.p.unscale_bs + row] = gram_unscale(exponent_field);
+    }
+    gram_chunk *pieces = args.p.pieces + batch * args.p.pieces_bs;
+    gradient_l2_walk(args, n0, o_begin, o_end, first, last, [&](int o, int slice, const float (&value)[BK_TILE_K]) {
+        const float s = o == o_begin ? scale[0] : o == o_begin + 1 ? scale[1] : o == o_begin + 2 ? scale[2] : scale[3];
+        unsigned piece[GW_PIECES][8];
+#pragma unroll
+        for (int q = 0; q < 8; q++) gram_split_pair(value[2 * q] * s, value[2 * q + 1] * s, piece[0][q], piece[1][q]);
+        gram_chunk *dst = pieces + (i64)slice * GW_SEGMENTS * args.p.rows_pad + (i64)o * args.from.n + n;
+#pragma unroll
+        for (int p = 0; p < GW_PIECES; p++)
+#pragma unroll
+            for (int half = 0; half < 2; half++)
+                if (live)
+                    dst[(i64)(2 * p + half) * args.p.rows_pad] =
+                        gram_chunk{piece[p][4 * half], piece[p][4 * half + 1], piece[p][4 * half + 2], piece[p][4 * half + 3]};
+    });
+    // the rows that pad p: by the last workgroup
+    if (block == (int)gridDim.x - args.a_blocks - 1) {
+        for (int slice = first + (threadIdx.x >> 6); slice < last; slice += 4)
+            for (int row = args.p.rows + lane; row < args.p.rows_pad; row += 64)
+#pragma unroll
+                for (int segment = 0; segment < GW_SEGMENTS; segment++)
+                    pieces[((i64)slice * GW_SEGMENTS + segment) * args.p.rows_pad + row] = gram_chunk{0u, 0u, 0u, 0u};
+        if (range == 0)
+            for (int row = args.p.rows + threadIdx.x; row < args.p.rows_pad; row += GL2_THREADS) args.p.unscale[batch * args.p.unscale_bs + row] = 1.0f;
     }
 }
 
@@ -82,16 +228,6 @@ __global__ __launch_bounds__(GL2_THREADS) void gradient_l2_sum_parts(const Gradi
     float total = args.partial[at];
     for (int part = 1; part < args.parts; ++part) total += args.partial[part * args.stride + at];
     args.sum[at] = total;
-}
-
-// c_transposed[k][o] = c[o][k]
-__global__ __launch_bounds__(GL2_THREADS) void gradient_l2_transpose_c(const GradientL2PrepareArgs args)
-{
-    const int k = blockIdx.x * GL2_THREADS + threadIdx.x, batch = blockIdx.y;
-    if (k >= args.k) return;
-    const float *c = args.c + batch * args.c_bs;
-    float *row = args.c_transposed + batch * args.c_transposed_bs + (i64)k * args.c_transposed_ld;
-    for (int o = 0; o < args.o; ++o) row[o] = c[(i64)o * args.c_ld + k];
 }
 
 }  // namespace kmc

@@ -155,3 +155,22 @@ def test_rfm_shape_against_float64_rows(device):
     truth = torch.stack([d[n].double()[None, :] * g - (cd * b[n].double()[None, :]) @ ad for n in rows], dim=1)
     error = (got[0][:, rows, :].double() - truth).abs().max().item() / truth.abs().mean().item()
     assert error < 1e-4, f"max abs err / mean |truth| = {error:.2e}"
+
+
+@pytest.mark.parametrize("M,N,O,K", [(40, 63, 4, 15), (70, 64, 5, 16), (256, 65, 8, 17), (33, 129, 3, 63), (20, 1, 1, 65), (65, 7, 9, 127), (30, 200, 2, 129),
+                                     (90, 66, 6, 900), (17, 300, 16, 1024)])
+def test_pieces_of_the_products_are_exact(device, l2_route, M, N, O, K):
+    """The rows c[o] (b[n] - mean) are made from b and c twice, for their scale and for their pieces, in tiles of 64 n x 64 k and
+    up to four outputs.  Small integers and rows of b with a mean of exactly zero make every sum exact."""
+    g = torch.Generator().manual_seed(M + N + O + K)
+    a = torch.randint(-3, 4, (K, M), generator=g).float().to(device)
+    c = torch.randint(-3, 4, (O, K), generator=g).float().to(device)
+    b = torch.zeros(N, K)
+    b[:, :K // 2] = torch.randint(-4, 5, (N, K // 2), generator=g).float()
+    b[:, K - K // 2:] = -b[:, :K // 2]
+    d = torch.randint(-4, 5, (N, M), generator=g).float().to(device)
+    b = b.to(device)
+    got = kermac.cdist_grad(a, b, c, d, p=2.0)[0].double()
+    a, b, c, d = a.double(), b.double(), c.double(), d.double()
+    truth = d[None] * (c @ a)[:, None, :] - torch.stack([(c[o][None, :] * b) @ a for o in range(O)])
+    assert torch.equal(got, truth)
