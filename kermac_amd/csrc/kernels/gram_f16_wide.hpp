@@ -400,25 +400,35 @@ __global__ __launch_bounds__(GW_ROW_THREADS, 2) void gram_rows_once(const GramRo
         gram_rows_once_of<GROUPS>(first ? args.first : args.second, first ? block : block - args.first_blocks);
 }
 
-// Tile shapes of the product kernel.  A workgroup is 4 waves; a wave owns WAVE_M rows of a and WAVE_N rows of b as
+// Tile shapes of the product kernel.  A workgroup is 4 waves (8: EightWaves); a wave owns WAVE_M rows of a and WAVE_N rows of b as
 // 16 x 16 blocks of the matrix instruction.  Two workgroups (three of the small shape) share a CU, so that one's
 // prologue, epilogue and result stores run beside the other's matrix instructions.
-template <int TILE_M_, int TILE_N_>
-struct WideTile {
+template <int TILE_M_, int TILE_N_, int WAVES_N_, int SLOTS_>
+struct WideShape {
     static constexpr int TILE_M = TILE_M_, TILE_N = TILE_N_;
-    static constexpr int THREADS = 256, WAVES = 4;
-    static constexpr int WAVES_M = 2, WAVES_N = 2;
+    static constexpr int WAVES_M = 2, WAVES_N = WAVES_N_, WAVES = WAVES_M * WAVES_N, THREADS = 64 * WAVES;
     static constexpr int WAVE_M = TILE_M / WAVES_M, WAVE_N = TILE_N / WAVES_N;
     static constexpr int MT = WAVE_M / 16, NT = WAVE_N / 16;
     static constexpr int PARTS_M = TILE_M / 128, PARTS_N = TILE_N / 128, PARTS = PARTS_M * PARTS_N;
     static constexpr int GRANULE_CHUNKS = 4 * (TILE_M + TILE_N);          // 32 k of one piece of a and one of b
-    static constexpr int COPIES_A = TILE_M / 64, COPIES_B = TILE_N / 64;  // runs of 64 chunks per wave and granule
+    static constexpr int COPIES_A = TILE_M / 16 / WAVES, COPIES_B = TILE_N / 16 / WAVES;  // runs of 64 chunks per wave and granule
     static constexpr int COPIES = COPIES_A + COPIES_B;
-    static constexpr int SLOTS = 3;
-    static constexpr int MIN_WAVES = TILE_M * TILE_N >= 256 * 128 ? 2 : 3;      // per SIMD
+    static constexpr int SLOTS = SLOTS_;
+    static constexpr int PER_CU = WAVES == 8 || TILE_M * TILE_N >= 256 * 128 ? 2 : 3;      // workgroups
+    static constexpr int MIN_WAVES = PER_CU * WAVES / 4;                                   // per SIMD
 };
+template <int TILE_M, int TILE_N>
+struct WideTile : WideShape<TILE_M, TILE_N, 2, 3> {};
+// The small tile by 8 waves of 64 x 32, for results of at most two tiles per CU: four waves leave a SIMD one or two, and it waits at every
+// granule's barrier for the reads of its operands.  With 8 a SIMD has two or four, and LDS for two whole steps of k, one barrier each.
+// A workgroup reads half as much again from LDS, which is why three workgroups of four waves are the better where there are tiles for them.
+// Product alone, 2000 x 2000 (256 tiles), 4 waves / 8: K = 784 47.3 / 41.4 us at the profiler's clock, K = 3072 155.6 / 139.8; calls at the rule.
+// A ring of four steps in 128 KB, one workgroup per CU: 148.5 at K = 3072; XCDs that share rectangles of tiles in place of columns: 141.7.
+template <typename Tile>
+struct EightWaves : WideShape<Tile::TILE_M, Tile::TILE_N, 4, 4> {};
 typedef WideTile<256, 128> WideTileLarge;
 typedef WideTile<128, 128> WideTileSmall;
+typedef EightWaves<WideTileSmall> WideTileFew;
 
 // Workgroup -> tile, as tile_of_workgroup of build_kernel.hpp with bands of GW_BAND_N n tiles: n fastest inside a band,
 // so the workgroups resident on an XCD (the hardware deals ids round-robin) cover a block of about 8 n tiles x 8 m tiles.
@@ -560,7 +570,7 @@ __device__ __forceinline__ void wide_lanes_exchange()
 
 // The matrix instructions are written out: left to itself the compiler gives their results other registers than their
 // sums came from, which does not fit beside the operands.  Two products into the same sums are at least 16 matrix
-// instructions apart, and wide_walk ends with the wait states that vector instructions need before they read the sums.
+// instructions apart (8 in EightWaves), and the walk ends with the wait states that vector instructions need before they read the sums.
 // The compiler, which keeps such distances for instructions it knows, does not see these: nothing else may read or move a sum between
 // the first product and those wait states, which holds as long as the sums stay where they are (the test of the kernel's listing
 // looks at every instruction in between).
@@ -618,6 +628,56 @@ __device__ __forceinline__ void wide_walk(gram_float4 (&acc)[Tile::MT][Tile::NT]
         wide_multiply<MT, NT, 0, MT>(acc, a2, b1);
         __builtin_amdgcn_sched_barrier(0);
         slot = third;
+    }
+    asm volatile("s_nop 15\n\ts_nop 15");
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++) asm volatile("" : "+v"(acc[mt][nt]));
+}
+
+// The walk of EightWaves: a ring of two whole steps and one barrier per step, in front of the read of a step's first granule.  Behind it both
+// granules of that step have arrived for every wave, and the step before has been read.  The products go into a sum in wide_walk's order.
+template <typename Tile>
+__device__ __forceinline__ void wide_walk_steps(gram_float4 (&acc)[Tile::MT][Tile::NT], const WideWalk<Tile> &walk, int steps)
+{
+    static_assert(Tile::SLOTS == 4, "two steps of two granules");
+    constexpr int MT = Tile::MT, NT = Tile::NT, COPIES = Tile::COPIES;
+    gram_half8 a1[MT], a2[MT], b1[NT], b2[NT];
+    walk.template copy<0>(0, 0);
+    walk.template copy<1>(0, 1);
+    if (steps > 1) {
+        walk.template copy<0>(1, 2);
+        walk.template copy<1>(1, 3);
+        wide_wait_copies<2 * COPIES>();
+    } else {
+        wide_wait_copies<0>();
+    }
+    __syncthreads();
+    walk.read(a1, b2, 0, true);
+    int slot = 0;                                       // of this step's first granule
+    for (int step = 0; step < steps; step++) {
+        const int next = 2 - slot;
+        walk.read(a2, b1, slot + 1, true);
+        __builtin_amdgcn_sched_barrier(0);
+        wide_multiply<MT, NT, 0, MT>(acc, a1, b2);
+        wide_multiply<MT, NT, 0, MT>(acc, a1, b1);
+        __builtin_amdgcn_sched_barrier(0);
+        if (step + 1 < steps) {
+            wide_wait_copies<0>();                       // only the next step's copies are under way
+            __syncthreads();
+            walk.read(a1, b2, next, true);
+            if (step + 2 < steps) {
+                walk.template copy<0>(step + 2, slot);
+                walk.template copy<1>(step + 2, slot + 1);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        } else {
+            __builtin_amdgcn_s_waitcnt(0xC07F);          // lgkmcnt(0), nothing else; why: at the end of wide_walk
+        }
+        wide_multiply<MT, NT, 0, MT>(acc, a2, b1);
+        __builtin_amdgcn_sched_barrier(0);
+        slot = next;
     }
     asm volatile("s_nop 15\n\ts_nop 15");
 #pragma unroll
@@ -706,7 +766,8 @@ __global__ __launch_bounds__(Tile::THREADS, Tile::MIN_WAVES) void gram_f16_wide(
         WideWalk<Tile> walk;
         walk.init(args.pieces_a + batch * args.pieces_a_bs, args.rows_pad_a, m0, args.pieces_b + batch * args.pieces_b_bs, args.rows_pad_b, n0,
                   ring, lane, wave, wave_m, wave_n);
-        wide_walk<Tile>(acc, walk, (args.slices + 1) / 2);
+        if constexpr (Tile::SLOTS == 3) wide_walk<Tile>(acc, walk, (args.slices + 1) / 2);
+        else wide_walk_steps<Tile>(acc, walk, (args.slices + 1) / 2);
     }
     // The last barrier of the walk stands in front of its last reads; behind this one every wave has its operands, and the
     // ring is free for the staging of the results (the gradient's epilogue stages nothing).

@@ -297,7 +297,7 @@ hipError_t launch_product_in(kmc::GramWideArgs &wide, hipStream_t stream)
     if ((padded - wide.wide_tiles_n) * 8 > wide.wide_tiles_n) padded = wide.wide_tiles_n;
     // ... nor where a launch that fits the chip at once would no longer, since the padding's idle ids fall to some of the XCDs (2 x 2816 x 2816
     // of K = 4096, 22 large tiles in n, 66 of them on 64 places: 604 -> 488 us)
-    const int64_t places = 32 * Tile::MIN_WAVES, rows_of_tiles = static_cast<int64_t>(wide.wide_tiles_m) * wide.kernel.l;
+    const int64_t places = 32 * Tile::PER_CU, rows_of_tiles = static_cast<int64_t>(wide.wide_tiles_m) * wide.kernel.l;
     if (rows_of_tiles * (padded / kmc::BK_XCDS) > places && rows_of_tiles * wide.wide_tiles_n <= places * kmc::BK_XCDS) padded = wide.wide_tiles_n;
     wide.wide_tiles_n_padded = padded;
     const int64_t blocks = (wide.kernel.m + kmc::GW_TILE - 1) / kmc::GW_TILE;
@@ -326,9 +326,15 @@ hipError_t launch_product_in(kmc::GramWideArgs &wide, hipStream_t stream)
 // K = 784 210 / 185, of K = 4096 1072 / 934; 784, 3584 x 3584 of K = 784 100 / 96, of K = 4096 395 / 371; 938, 200 x 60000 of K = 784 194.4 / 197.5,
 // of K = 2048 568 / 561; 1024, 4096 x 4096 of K = 784 103.1 / 103.8, of K = 4096 432 / 421; more than one round of either: 1156,
 // 4352 x 4352 of K = 2048 276 / 306.  A set against itself: 780, 4900 points of K = 784 110 / 120; 990, 5632 of K = 784 130 / 127.
-constexpr int64_t SMALL_TILES_PER_ROUND = kmc::WideTileSmall::MIN_WAVES * 256, LARGE_TILES_PER_ROUND = kmc::WideTileLarge::MIN_WAVES * 256;
+constexpr int64_t SMALL_TILES_PER_ROUND = kmc::WideTileSmall::PER_CU * 256, LARGE_TILES_PER_ROUND = kmc::WideTileLarge::PER_CU * 256;
 constexpr int64_t LITTLE_OF_A_ROUND = SMALL_TILES_PER_ROUND / 6;
 constexpr int LONG_CONTRACTION_SLICES = 2048 / kmc::BK_TILE_K;
+// Two small tiles per CU: up to there a tile by 8 waves, beyond it three by 4 each.  By 4 / 8 waves, us of a call, k contiguous: 192 tiles,
+// 3000 x 1000 x 784 49.4 / 45.8; 256, 2000 x 2000 of K = 784 51.5 / 48.9, of K = 3072 152.6 / 149.2; 324, 2200 x 2200 x 784 63.5 / 63.1; 484,
+// 2700 x 2700 x 784 77.7 / 71.5, products 2800 x 2800 of K = 256 31.9 / 29.3, of K = 4096 272 / 228; 480, 20 x 500 x 700 x 784 102.2 / 102.5; beyond:
+// 529, 2880 x 2880 x 784 78.6 / 81.2; 676, 3300 x 3300 x 784 88.1 / 93.1.  A set against itself: 128, 2000 points of K = 784 63.0 / 52.5; 288,
+// 3000 of K = 512 67.1 / 61.1; 392, 3500 of K = 784 79.0 / 73.2; 480, 3900 of K = 784 93.5 / 92.7; 544, 4200 102.0 / 99.6.
+constexpr int64_t FEW_TILES = 2 * 256;
 
 template <bool SYMMETRIC, int EPILOGUE>
 hipError_t launch_product(kmc::GramWideArgs &wide, hipStream_t stream)
@@ -343,9 +349,9 @@ hipError_t launch_product(kmc::GramWideArgs &wide, hipStream_t stream)
                            (small <= SMALL_TILES_PER_ROUND + LITTLE_OF_A_ROUND || wide.slices >= LONG_CONTRACTION_SLICES);
     // KERMAC_AMD_WIDE_LARGE_TILE_MIN_TILES=n replaces the number (read on every call, so that a test can send small shapes to the large tiles)
     const char *text = std::getenv("KERMAC_AMD_WIDE_LARGE_TILE_MIN_TILES");
-    return large >= (text ? std::atoi(text) : kmc_rules::WIDE_LARGE_TILE_MIN_TILES) || one_round
-               ? launch_product_in<Large, SYMMETRIC, EPILOGUE>(wide, stream)
-               : launch_product_in<Small, SYMMETRIC, EPILOGUE>(wide, stream);
+    if (large >= (text ? std::atoi(text) : kmc_rules::WIDE_LARGE_TILE_MIN_TILES) || one_round) return launch_product_in<Large, SYMMETRIC, EPILOGUE>(wide, stream);
+    if (small <= FEW_TILES) return launch_product_in<kmc::WideTileFew, SYMMETRIC, EPILOGUE>(wide, stream);
+    return launch_product_in<Small, SYMMETRIC, EPILOGUE>(wide, stream);
 }
 
 // Bytes of workspace the path needs for this problem; 0 when it does not apply.
