@@ -104,14 +104,12 @@ hipError_t launch_scalar_b_if_the_sample_leaves(int load_a, int load_b, const km
 #endif
 
 // Results of few tiles, in tiles of 64 x 64 (build_kernel_small.hpp).  128 x 128 / 64 x 64 tiles, us, p = 1 and p = 1.3 at
-// K = 400: 64 tiles 117 / 55 and 326 / 121; 121 tiles 133 / 58 and 347 / 187; 192 tiles 127 / 72 and 341 / 259; 256 tiles, one
-// for every CU, 127 / 86 and 342 / 334; a set against itself of 16 x 16 tiles 165 / 108 and 439 / 428.  Beyond that a single problem
-// still gains (360 tiles 136 / 124 and 647 / 481) but a batch loses (32 x 500 x 500 146 / 165 and 657 / 636, at K = 64 33 / 39), and
-// so does a set against itself, of which this kernel computes both halves (22 x 22 tiles 167 / 194 and 445 / 802).
-// Powers with a root or a transcendental function are bound by its issue, and there a fourth workgroup of 64 x 64 per CU is a round of
-// its own: up to 192 tiles, three per CU (192 x 128 x 128, p = 1.3, K = 16, 64 and 256 20.6 / 20.5, 59.0 / 50.6 and 213 / 173;
-// 208 x 128 x 128 20.6 / 24.0, 59.0 / 63.1 and 214 / 220, p = 0.5 at K = 64 38.2 / 40.9; 1792 x 1792, 196 tiles, p = 1.3 21.0 / 23.6, 58.9 / 61.8
-// and 213 / 215).
+// K = 400: 64 tiles 111 / 30 and 324 / 91; 121 tiles 113 / 45 and 326 / 166; 196 tiles 124 / 85 and 341 / 321; 256 tiles, one
+// for every CU, 113 / 77 and 328 / 317; a set against itself of 16 x 16 tiles 142 / 79 and 343 / 318.  Beyond that most single problems
+// still gain (324 tiles 148 / 109 and 633 / 468; 400 117 / 126 and 621 / 543) but batches hardly (32 x 500 x 500 162 / 149 and 639 / 618, at
+// K = 64 32 / 32 and 113 / 111), and a set against itself, of which this kernel computes both halves, loses (22 x 22 tiles 146 / 144 and 345 / 619).
+// Powers with a root or a transcendental function are bound by its issue, and there a fourth workgroup of 64 x 64 per CU brings little:
+// up to 192 tiles, three per CU (208 x 128 x 128, p = 1.3, K = 64 58.8 / 58.2; 240 x 128 x 128 x 256 212 / 205; 1792 x 1792 x 256 213 / 205).
 // KERMAC_AMD_DIRECT_SMALL_MAX_TILES=n replaces both limits (read on every call, so that a test can choose the kernel).
 constexpr bool HAS_ROOT_OR_POWER = KMC_INNER_POW == kmc::POW_POW || KMC_INNER_POW == kmc::POW_SQRT || KMC_INNER_POW == kmc::POW_ABS_HALF ||
                                    KMC_INNER_POW == kmc::POW_ABS_THREE_HALVES;
@@ -195,7 +193,7 @@ hipError_t KMC_LAUNCHER_NAME(int load_a, int load_b, const kmc::BuildKernelArgs 
         kmc::BuildKernelArgs copy = args;
         void *kernel_args[] = {&copy, &load_a, &load_b, const_cast<int *>(&down)};
         return hipLaunchKernel(reinterpret_cast<const void *>(kmc::build_kernel_small<KMC_INNER_OP, KMC_INNER_POW>),
-                               dim3(static_cast<unsigned>(across) * down, args.l), dim3(kmc::BK_THREADS), kernel_args, 0, stream);
+                               dim3(static_cast<unsigned>(across) * down, args.l), dim3(kmc::BKS_THREADS), kernel_args, 0, stream);
     }
     switch (load_a * 4 + load_b) {
     case 0: return launch_one<0, 0>(args, grid, stream);

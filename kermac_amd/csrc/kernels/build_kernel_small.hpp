@@ -1,11 +1,16 @@
 // The direct kernel for results of few tiles: build_kernel.hpp in tiles of 64 x 64 instead of 128 x 128.
 //
 // A result of 1024 x 1024 is 64 tiles of 128 x 128: a quarter of the CUs work, each lane through 64 results of its own, and what
-// stands in front of and behind the walk (first loads, epilogue, stores) is hidden by nothing.  Here a lane holds 4 x 4 results
-// and a workgroup of 4 waves a tile of 64 x 64, so that the same result is four times the workgroups at a quarter of the
-// serial work each.  LDS then feeds half as many terms per byte, which is why large results stay with the other
-// tile.  Whole calls, 128 x 128 / 64 x 64 tiles, us: 1024 x 1024 p = 1 at K = 64 24 / 18, at K = 400 117 / 55;
-// p = 1.3 58 / 26 and 326 / 121; p = 2 at K = 64 24 / 18, of which the kernel takes 14 and the host, call after call, 15 to 16.
+// stands in front of and behind the walk (first loads, epilogue, stores) is hidden by nothing.  Here a workgroup of 8 waves holds a
+// tile of 64 x 64 and a lane 4 x 2 results, so that the same result is four times the workgroups at an eighth of the
+// serial work per lane.  LDS then feeds a third as many terms per byte, which is why large results stay with the other
+// tile.
+//
+// Up to 256 of these tiles a workgroup has its CU to itself, and two waves on a SIMD are what hides the reads from LDS: with 4 waves of 4 x 4
+// results per lane, one on each SIMD, a term of k took 0.11 us where it now takes 0.06 (LDS alone 0.04).  4 / 8 waves, kernels back to back, us:
+// 1024 x 1024 at K = 64 p = 1 13.9 / 8.0, p = 2 13.3 / 8.1, p = 1.3 24.8 / 18.5, at K = 400 p = 1 51 / 28, p = 1.3 117 / 89, |x|^4 61 / 34; 64 x 64 x 16
+// 6.3 / 4.4; 1200 x 1200 x 200 (361 tiles) p = 1 31.2 / 23.8; 2048 x 2048 x 128 (1024, four workgroups per CU) 31.1 / 28.3, |x|^4 42.9 / 37.7;
+// 192 x 128 x 128 x 64 18.3 / 15.5; no size of this kernel's range was slower.
 //
 // The terms, their order in every sum and the epilogue are those of build_kernel: the bits are the same.  Slices of 32 k, double
 // buffered.  The loaders are chosen at run time (uniform branches in front of a slice's loads): few launches are worth sixteen instantiations.  A
@@ -19,45 +24,41 @@ namespace kmc {
 constexpr int BKS_TILE = 64;
 constexpr int BKS_DEPTH = 32;
 constexpr int BKS_PITCH = BKS_TILE + 4;
+constexpr int BKS_THREADS = 512;
 
-// One operand's share of a 64 x 32 slice: 8 floats per lane, as two runs of 4.
+// One operand's share of a 64 x 32 slice: 4 consecutive floats per lane.
 struct SmallLoader {
     const float *base;      // row 0 of the tile, k = 0
     i64 ld;
     int rows, mode, tid;    // rows that exist from the tile's first on
 
-    // first row and k of run h, relative to the tile and the slice
+    // this lane's first row and k, relative to the tile and the slice
     __device__ __forceinline__ bool k_runs() const { return mode == LOAD_ROW_VEC || mode == LOAD_ROW_SCALAR; }
-    __device__ __forceinline__ int row_of(int h) const { return k_runs() ? (tid >> 3) + 32 * h : (tid & 15) * 4; }
-    __device__ __forceinline__ int k_of(int h) const { return k_runs() ? (tid & 7) * 4 : (tid >> 4) + 16 * h; }
+    __device__ __forceinline__ int row() const { return k_runs() ? tid >> 3 : (tid & 15) * 4; }
+    __device__ __forceinline__ int k_row() const { return k_runs() ? (tid & 7) * 4 : tid >> 4; }
 
-    __device__ __forceinline__ void load(float4 (&r)[2], int k0, int k) const
+    __device__ __forceinline__ float4 load(int k0, int k) const
     {
         const bool vec = mode == LOAD_COL_VEC || mode == LOAD_ROW_VEC;
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const int row = row_of(h), at = k0 + k_of(h);
-            if (k_runs()) r[h] = row < rows ? load4_guarded(base + (i64)row * ld + at, k - at, vec) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            else r[h] = at < k ? load4_guarded(base + (i64)at * ld + row, rows - row, vec) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        }
+        const int at = k0 + k_row();
+        const float4 nothing = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (k_runs()) return row() < rows ? load4_guarded(base + (i64)row() * ld + at, k - at, vec) : nothing;
+        return at < k ? load4_guarded(base + (i64)at * ld + row(), rows - row(), vec) : nothing;
     }
 
-    __device__ __forceinline__ void store(float *slice, const float4 (&r)[2]) const
+    __device__ __forceinline__ void store(float *slice, const float4 &r) const
     {
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            float *to = slice + k_of(h) * BKS_PITCH + row_of(h);
-            if (k_runs()) {
-                to[0] = r[h].x; to[BKS_PITCH] = r[h].y; to[2 * BKS_PITCH] = r[h].z; to[3 * BKS_PITCH] = r[h].w;
-            } else {
-                *reinterpret_cast<float4 *>(to) = r[h];
-            }
+        float *to = slice + k_row() * BKS_PITCH + row();
+        if (k_runs()) {
+            to[0] = r.x; to[BKS_PITCH] = r.y; to[2 * BKS_PITCH] = r.z; to[3 * BKS_PITCH] = r.w;
+        } else {
+            *reinterpret_cast<float4 *>(to) = r;
         }
     }
 };
 
 template <int INNER_OP, int INNER_POW>
-__global__ __launch_bounds__(BK_THREADS) void build_kernel_small(const BuildKernelArgs args, int load_a, int load_b, int tiles_n)
+__global__ __launch_bounds__(BKS_THREADS) void build_kernel_small(const BuildKernelArgs args, int load_a, int load_b, int tiles_n)
 {
     __shared__ __attribute__((aligned(16))) float lds_a[2][BKS_DEPTH * BKS_PITCH];
     __shared__ __attribute__((aligned(16))) float lds_b[2][BKS_DEPTH * BKS_PITCH];
@@ -71,34 +72,32 @@ __global__ __launch_bounds__(BK_THREADS) void build_kernel_small(const BuildKern
     const SmallLoader from_a{args.a + batch * args.a_bs + first(load_a, m0, args.a_ld), args.a_ld, args.m - m0, load_a, tid};
     const SmallLoader from_b{args.b + batch * args.b_bs + first(load_b, n0, args.b_ld), args.b_ld, args.n - n0, load_b, tid};
 
-    float acc[4][4];
+    float acc[2][4];
 #pragma unroll
-    for (int j = 0; j < 4; j++)
+    for (int j = 0; j < 2; j++)
 #pragma unroll
         for (int i = 0; i < 4; i++) acc[j][i] = 0.0f;
     if (args.k > 0) {
-        float4 stage_a[2], stage_b[2];
-        from_a.load(stage_a, 0, args.k);
-        from_b.load(stage_b, 0, args.k);
+        float4 stage_a = from_a.load(0, args.k), stage_b = from_b.load(0, args.k);
         from_a.store(lds_a[0], stage_a);
         from_b.store(lds_b[0], stage_b);
         __syncthreads();
         for (int k0 = 0, cur = 0; k0 < args.k; k0 += BKS_DEPTH, cur ^= 1) {
             const bool more = k0 + BKS_DEPTH < args.k;
             if (more) {
-                from_a.load(stage_a, k0 + BKS_DEPTH, args.k);
-                from_b.load(stage_b, k0 + BKS_DEPTH, args.k);
+                stage_a = from_a.load(k0 + BKS_DEPTH, args.k);
+                stage_b = from_b.load(k0 + BKS_DEPTH, args.k);
             }
-            const float *row_a = lds_a[cur] + 4 * tx, *row_b = lds_b[cur] + 4 * ty;
+            const float *row_a = lds_a[cur] + 4 * tx, *row_b = lds_b[cur] + 2 * ty;
             // padding of k up to a multiple of 16 takes part, as in the other tile
             const int depth = min(BKS_DEPTH, (args.k - k0 + BK_TILE_K - 1) / BK_TILE_K * BK_TILE_K);
 #pragma unroll 4
             for (int kk = 0; kk < depth; kk++) {
                 const float4 va = *reinterpret_cast<const float4 *>(row_a + kk * BKS_PITCH);
-                const float4 vb = *reinterpret_cast<const float4 *>(row_b + kk * BKS_PITCH);
-                const float fa[4] = {va.x, va.y, va.z, va.w}, fb[4] = {vb.x, vb.y, vb.z, vb.w};
+                const float2 vb = *reinterpret_cast<const float2 *>(row_b + kk * BKS_PITCH);
+                const float fa[4] = {va.x, va.y, va.z, va.w}, fb[2] = {vb.x, vb.y};
 #pragma unroll
-                for (int j = 0; j < 4; j++)
+                for (int j = 0; j < 2; j++)
 #pragma unroll
                     for (int i = 0; i < 4; i++) {
                         if (INNER_OP == OP_DIFF && INNER_POW == POW_SQUARE) {
@@ -127,8 +126,8 @@ __global__ __launch_bounds__(BK_THREADS) void build_kernel_small(const BuildKern
     const bool regularize = kernel_type != KERNEL_NONE && regularization != 0.0f;
     const int m = m0 + 4 * tx;
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const int n = n0 + 4 * ty + j;
+    for (int j = 0; j < 2; j++) {
+        const int n = n0 + 2 * ty + j;
         float v[4];
 #pragma unroll
         for (int i = 0; i < 4; i++) {
