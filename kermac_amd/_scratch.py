@@ -96,8 +96,15 @@ def operator(function):
     """Decorator of the public operators: the body runs inside ``operator_call()``; signature and docstring stay."""
     @functools.wraps(function)
     def wrapped(*args, **kwargs):
-        with operator_call():
+        # operator_call() written out: a generator's entry and exit are a microsecond of every call
+        state = _state()
+        if state["depth"] == 0:
+            state["used"] = 0
+        state["depth"] += 1
+        try:
             return function(*args, **kwargs)
+        finally:
+            state["depth"] -= 1
     return wrapped
 
 

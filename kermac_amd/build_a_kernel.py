@@ -60,6 +60,9 @@ _INNER_OPERATOR_ABI = {InnerOperator.DIFF: 0, InnerOperator.DOT: 1}
 _POWER_TYPE_ABI = {PowerType.NOOP: 0, PowerType.ABS: 1, PowerType.SQUARE: 2, PowerType.SQRT: 3, PowerType.POW: 4}
 _KERNEL_TYPE_ABI = {KernelType.NONE: 0, KernelType.LAPLACE: 1, KernelType.GAUSSIAN: 2}
 _MAJORNESS_ABI = {Majorness.COL_MAJOR: _backend.COL_MAJOR, Majorness.ROW_MAJOR: _backend.ROW_MAJOR}
+for _numbers in (_INNER_OPERATOR_ABI, _POWER_TYPE_ABI, _KERNEL_TYPE_ABI, _MAJORNESS_ABI):
+    for _member, _number in _numbers.items():
+        _member.abi = _number           # an enum member as a key is hashed in Python code: six times per call
 # (majorness, alignment) -> device loader variant (csrc/kernels/device_common.hpp LoadMode).
 _LOAD_MODE = {
     (Majorness.COL_MAJOR, Alignment.ALIGN_4): 0,
@@ -346,6 +349,10 @@ class _LaunchPlan:
     __slots__ = ("params", "out", "keepalive", "swapped", "L", "M", "N", "K", "l2_auto")
 
 
+def _as_float(x):
+    return float(x) if isinstance(x, int) and not isinstance(x, bool) else x
+
+
 def _plan_run_kernel(
     kernel_descriptor, a, b, out, p, inner_p, outer_p, bandwidth, epsilon, regularization,
     regularization_offset_x, regularization_offset_y, try_to_align, require_device=True, allocate_out=True,
@@ -374,19 +381,23 @@ def _plan_run_kernel(
     if p is not None and outer_p is not None:
         raise ValueError("'p' is not 'None' but 'outer_p' is also not 'None")
 
-    def as_float(x):
-        return float(x) if isinstance(x, int) and not isinstance(x, bool) else x
-
-    p, inner_p, outer_p = as_float(p), as_float(inner_p), as_float(outer_p)
-    bandwidth, regularization = as_float(bandwidth), as_float(regularization)
-
     # Batch size: every operand's batch is 1 or the common L (reference: :203-211).
     L = 1
-    L = merge_batch_size("p", L, p, expected_dims=0, can_be_none=True)
-    L = merge_batch_size("inner_p", L, inner_p, expected_dims=0, can_be_none=True)
-    L = merge_batch_size("outer_p", L, outer_p, expected_dims=0, can_be_none=True)
-    L = merge_batch_size("bandwidth", L, bandwidth, expected_dims=0, can_be_none=True)
-    L = merge_batch_size("regularization", L, regularization, expected_dims=0, can_be_none=True)
+    if p is not None:
+        p = _as_float(p)
+        L = merge_batch_size("p", L, p, expected_dims=0)
+    if inner_p is not None:
+        inner_p = _as_float(inner_p)
+        L = merge_batch_size("inner_p", L, inner_p, expected_dims=0)
+    if outer_p is not None:
+        outer_p = _as_float(outer_p)
+        L = merge_batch_size("outer_p", L, outer_p, expected_dims=0)
+    if bandwidth is not None:
+        bandwidth = _as_float(bandwidth)
+        L = merge_batch_size("bandwidth", L, bandwidth, expected_dims=0)
+    if regularization is not None:
+        regularization = _as_float(regularization)
+        L = merge_batch_size("regularization", L, regularization, expected_dims=0)
     if not isinstance(a, torch.Tensor) or not isinstance(b, torch.Tensor):
         raise TypeError("a and b must be PyTorch tensors")
     if out is not None and not isinstance(out, torch.Tensor):
@@ -449,11 +460,12 @@ def _plan_run_kernel(
                 raise ValueError("`p` tensor must be on the same CUDA device as inputs")
             inner_p = p.contiguous()
             outer_p = 1.0 / inner_p
-    pi_ptr, pi_bs, pi_val, pi_keep = _hyper_parameter("inner_p", inner_p, L, device, require_device)
-    po_ptr, po_bs, po_val, po_keep = _hyper_parameter("outer_p", outer_p, L, device, require_device)
-    bw_ptr, bw_bs, bw_val, bw_keep = _hyper_parameter("bandwidth", bandwidth, L, device, require_device)
-    rg_ptr, rg_bs, rg_val, rg_keep = _hyper_parameter("regularization", regularization, L, device, require_device)
-    keepalive += [pi_keep, po_keep, bw_keep, rg_keep]
+    # only those that are set: the parameter block starts as zeros
+    hyper_parameters = []
+    for name, field, value in (("inner_p", "p_inner", inner_p), ("outer_p", "p_outer", outer_p), ("bandwidth", "bandwidth", bandwidth),
+                               ("regularization", "regularization", regularization)):
+        if value is not None:
+            hyper_parameters.append((field, *_hyper_parameter(name, value, L, device, require_device)))
 
     # The kernel writes C with m contiguous.  A row-major out is the transpose of
     # that, so swap the operands (reference: :323-336).  The reference swaps neither the
@@ -474,14 +486,15 @@ def _plan_run_kernel(
         off_x, off_y = off_y, off_x
 
     params = _backend.BuildKernelParams()
-    params.inner_operator = _INNER_OPERATOR_ABI[d._inner_operator]
-    params.inner_power = _POWER_TYPE_ABI[d._inner_power]
-    params.outer_power = _POWER_TYPE_ABI[d._outer_power]
-    params.kernel_type = _KERNEL_TYPE_ABI[d._kernel_type]
-    params.a_majorness = _MAJORNESS_ABI[stats_a.majorness]
-    params.b_majorness = _MAJORNESS_ABI[stats_b.majorness]
+    params.inner_operator = d._inner_operator.abi
+    params.inner_power = d._inner_power.abi
+    params.outer_power = d._outer_power.abi
+    params.kernel_type = d._kernel_type.abi
+    params.a_majorness = stats_a.majorness.abi
+    params.b_majorness = stats_b.majorness.abi
     params.flags = 0 if swapped else _backend.FLAG_NEGATE_DIFF
-    if os.environ.get("KERMAC_AMD_NO_SYMMETRY", "0") not in ("", "0"):
+    a_pointer, b_pointer = a.data_ptr(), b.data_ptr()
+    if a_pointer == b_pointer and os.environ.get("KERMAC_AMD_NO_SYMMETRY", "0") not in ("", "0"):
         # the library computes x-against-x matrices from the tiles on and below the diagonal
         # (bit-identical result, about half the time); this keeps it to the full computation
         params.flags |= _backend.FLAG_NO_SYMMETRY
@@ -514,14 +527,17 @@ def _plan_run_kernel(
         if l1["tolerance"] is not None:
             params.gram_trust = float(l1["tolerance"])
     params.m, params.n, params.k, params.l = M, N, K, L
-    params.a, params.a_ld, params.a_bs = a.data_ptr(), stats_a.leading_dimension_stride, stats_a.batch_stride
-    params.b, params.b_ld, params.b_bs = b.data_ptr(), stats_b.leading_dimension_stride, stats_b.batch_stride
+    params.a, params.a_ld, params.a_bs = a_pointer, stats_a.leading_dimension_stride, stats_a.batch_stride
+    params.b, params.b_ld, params.b_bs = b_pointer, stats_b.leading_dimension_stride, stats_b.batch_stride
     if stats_c is not None:
         params.c, params.c_ld, params.c_bs = out.data_ptr(), stats_c.leading_dimension_stride, stats_c.batch_stride
-    params.p_inner, params.p_inner_bs, params.p_inner_value = pi_ptr, pi_bs, pi_val
-    params.p_outer, params.p_outer_bs, params.p_outer_value = po_ptr, po_bs, po_val
-    params.bandwidth, params.bandwidth_bs, params.bandwidth_value = bw_ptr, bw_bs, bw_val
-    params.regularization, params.regularization_bs, params.regularization_value = rg_ptr, rg_bs, rg_val
+    for field, pointer, batch_stride, by_value, keep in hyper_parameters:
+        if keep is None:
+            setattr(params, field + "_value", by_value)
+        else:
+            setattr(params, field, pointer)
+            setattr(params, field + "_bs", batch_stride)
+            keepalive.append(keep)
     params.regularization_offset_x, params.regularization_offset_y = off_x, off_y
     params.epsilon = 1e-5 if epsilon is None else float(epsilon)
 
@@ -787,12 +803,11 @@ def _small_set_is_cut(params, asked):
 
 def _workspace_route_applies(params, flags):
     """Whether kmc_build_kernel would take this call through a workspace, given these matrix-core flags."""
-    if os.environ.get("KERMAC_AMD_L2_WORKSPACE", "1") in ("", "0"):
-        return False
     kept = params.flags
     params.flags |= flags
     try:
-        return _backend.gram_workspace_bytes(params) > 0
+        # the environment last: a small call, which the library has no workspace for, is bound by the host
+        return _backend.gram_workspace_bytes(params) > 0 and os.environ.get("KERMAC_AMD_L2_WORKSPACE", "1") not in ("", "0")
     finally:
         params.flags = kept
 

@@ -131,17 +131,18 @@ class TensorStats:
     __slots__ = ("_shape", "_num_batches", "_batch_stride", "_majorness", "_alignment", "_ld")
 
     def __init__(self, tensor: torch.Tensor):
-        if tensor.dim() not in (2, 3):
+        shape, strides = tensor.shape, tensor.stride()
+        if len(shape) not in (2, 3):
             raise ValueError("Input tensor must be 2 or 3-dimensional")
         if tensor.dtype != torch.float32:
             raise TypeError("Input tensor must have dtype torch.float32")
 
-        batched = tensor.dim() == 3
-        self._num_batches = tensor.size(0) if batched else 1
-        self._batch_stride = tensor.stride(0) if batched and self._num_batches != 1 else 0
+        batched = len(shape) == 3
+        self._num_batches = shape[0] if batched else 1
+        self._batch_stride = strides[0] if batched and self._num_batches != 1 else 0
 
-        rows, cols = tensor.size(-2), tensor.size(-1)
-        row_stride, col_stride = tensor.stride(-2), tensor.stride(-1)
+        rows, cols = shape[-2:]
+        row_stride, col_stride = strides[-2:]
         self._shape = (self._num_batches, rows, cols)
 
         if col_stride == 1 and row_stride >= cols:
@@ -154,8 +155,7 @@ class TensorStats:
             )
 
         self._ld = max(row_stride, col_stride)
-        sixteen_byte = tensor.data_ptr() % 16 == 0 and self._ld % 4 == 0
-        if self._majorness is Majorness.COL_MAJOR and sixteen_byte:
+        if self._majorness is Majorness.COL_MAJOR and self._ld % 4 == 0 and tensor.data_ptr() % 16 == 0:
             self._alignment = Alignment.ALIGN_4
         else:
             self._alignment = Alignment.ALIGN_1
