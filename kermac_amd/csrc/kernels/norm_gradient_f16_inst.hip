@@ -104,15 +104,18 @@ bool gradient_layout(const kmc_norm_gradient_params *p, GradientLayout *layout)
     return true;
 }
 
-// Tile of the product in n: 16, 8, 4 or 2 blocks of 16.  A wave takes about 84 cycles for the two matrix instructions, the
+// Tile of the product in n: 16, 12, 8, 4 or 2 blocks of 16.  A wave takes about 84 cycles for the two matrix instructions, the
 // comparisons and the reads of a block and m, and 230 for W and the rest of a step (1580 cycles at 16 blocks, measured at
 // 8192 x 512 x 16 x 8192), so wide tiles are cheaper per result, unless they are too few for the 256 CUs: one
-// workgroup per CU is what the count of rounds assumes.
+// workgroup per CU is what the count of rounds assumes.  12 is for n that fill little of the second half of a larger tile: with the others only / with
+// 12, us: 3000 x 147 x 64 x 4000 714 / 577, 2000 x 300 x 20 x 2000 301 / 212, 4000 x 147 x 32 x 4000 481 / 399.
 int blocks_for(const kmc_norm_gradient_params *p, int o_chunks)
 {
     int best = 16;
     int64_t best_cost = INT64_MAX;
-    for (int blocks = 16; blocks >= 2; blocks /= 2) {
+    for (int blocks : {16, 12, 8, 4, 2}) {
+        // 12 where its last tile ends inside the padded rows
+        if (blocks == 12 && round_up(p->n, 16 * blocks) > round_up(p->n, kmc::NGF_N_PAD)) continue;
         const int64_t tiles_n = (p->n + 16 * blocks - 1) / (16 * blocks), tiles_m = (p->m + kmc::NGF_TILE_M - 1) / kmc::NGF_TILE_M;
         const int64_t rounds = (tiles_n * tiles_m * p->l * o_chunks + 255) / 256;
         const int64_t cost = rounds * (84 * blocks + 230);
@@ -143,6 +146,7 @@ hipError_t launch_products(int blocks, kmc::NormGradientF16Args &args, int o_beg
 {
     switch (blocks) {
     case 16: return launch_product<16, PIECES_IN_COLUMNS>(args, o_begin, o_chunks, stream);
+    case 12: return launch_product<12, PIECES_IN_COLUMNS>(args, o_begin, o_chunks, stream);
     case 8: return launch_product<8, PIECES_IN_COLUMNS>(args, o_begin, o_chunks, stream);
     case 4: return launch_product<4, PIECES_IN_COLUMNS>(args, o_begin, o_chunks, stream);
     default: return launch_product<2, PIECES_IN_COLUMNS>(args, o_begin, o_chunks, stream);

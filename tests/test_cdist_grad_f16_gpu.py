@@ -13,6 +13,7 @@ import pytest
 import torch
 
 import kermac_amd as kermac
+from tests.helpers import kernels_of
 from kermac_amd import _backend
 
 module = importlib.import_module("kermac_amd.cdist_grad")       # the package attribute of that name is the operator
@@ -172,3 +173,11 @@ def test_rounding_follows_the_signed_sums(device):
         truth = c.double() @ (sign * a.double())
         worst = max(worst, float((got[:, n].double() - truth).norm() / truth.norm()))
     assert worst < (2 * K / 32) ** 0.5 * 2.0 ** -24 + 3 * 2.0 ** -22
+
+
+@pytest.mark.parametrize("M,N,O,K", [(4000, 150, 16, 65), (4001, 192, 5, 64), (4090, 300, 20, 33)])
+def test_signs_are_exact_in_tiles_of_192(device, f16_route, M, N, O, K):
+    """Sizes at which a tile of 12 blocks of n is the cheapest: the last one ends inside the padded rows."""
+    zeros = [torch.zeros(rows, columns, device=device) for rows, columns in ((K, M), (N, K), (O, K), (N, M))]
+    assert any("norm_gradient_l1_f16<12," in name for name in kernels_of(lambda: kermac.cdist_grad(*zeros, p=1.0)))
+    test_signs_are_exact(device, f16_route, M, N, O, K)
