@@ -17,21 +17,27 @@
 //                          subtraction with the clamp to [0, 1] compares two k and gives S in fp16.  The keys that are
 //                          sorted order -0 below +0, so that signed zeros and ties come out as copysign(1, d - b).
 //                          Rows of B longer than that are cut into chunks with positions of their own.
-//                          The same launch copies A into the order in which a wave reads it (and takes the largest
-//                          magnitude of every row m), and scales C by a power of two per row o.
+//                          The same launch copies A into the order in which a wave reads it, scales C by a power of two per
+//                          row o, and estimates the largest |A[m, k] C[o, k]| over k for every m and o.
 // norm_gradient_l1_f16     the product.
 //
-// Accuracy: S is exact, a = a1 + a2 and c = c1 + c2 to 2^-22, w1 = fp16(a1 c1) and w2 = a1 c1 - w1 + a1 c2 + a2 c1 in fp16: below
-// 3 * 2^-22 |w| together, beside the fp32 accumulation.  The sums run over S W, so  1/2 sum_k W  is taken off them again: every 256
+// Accuracy: S is exact.  w = a c 2^F with its largest value over k in [2^14, 2^15.2), F of every m and o from the estimate; w1 =
+// fp16(w), w2 = fp16(w - w1), so |w - w1 - w2| <= 2^-22 |w| + 2^-39 max_k|w|, however far max_k|a c| is below max|a| max|c|.  Doubled
+// with the result, that is below 3 * 2^-22 sum_k |c a| up to K = 2^16, beside the fp32 accumulation.  (A scale per row m of A times one per
+// row o of C is not enough: in rows with a large value whose partner is zero, 1 beside 2^-16 say, fp16's smallest step takes the place
+// of the others' last bits, 6e-6 of sum_k |c a| and more.)  Zeros count as 2^-127 in the estimate, which shows where max|a| or max|c| is above
+// 2^100 times the products; rows of A below 2^-113 keep fewer bits.  The sums run over S W, so  1/2 sum_k W  is taken off them again: every 256
 // k, since a partial sum of S W alone drifts away from the one of the signed terms, and rounding follows the partial sums.
 //
 // Workgroup of norm_gradient_l1_f16: 8 waves, 16 m x 16 BLOCKS n x 16 o; wave w owns the 2 m  2w, 2w + 1  and all n, as
 // BLOCKS x 2 results of v_mfma_f32_16x16x32_f16 (rows n, columns o).  The more n a wave holds, the less W costs: at 256
-// n the 64 matrix instructions of a step of 32 k stand beside 128 packed subtractions and about 75 other instructions.
+// n the 64 matrix instructions of a step of 32 k stand beside 128 packed subtractions and about 100 other vector instructions, two
+// thirds of them the cheap ones of fp32.
 // Bound by the two together: on registers alone a v_mfma_f32_16x16x32_f16 takes 16.5 cycles, 16.9 with two packed
-// subtractions beside it, and four more for every further vector instruction; the kernel takes about 26.
-// Measured at M = K = 8192, N = 512, O = 16: 1.9 ms with 0.19 ms of gradient_signs_prepare (3.65 ms for the kernel that
-// flipped the sign into both pieces of A: three products and 2.5 vector instructions per term), O = 32 3.7 ms (5.55).
+// subtractions beside it, and four more for every further packed instruction; the kernel takes about 26.
+// Measured at M = K = 8192, N = 512, O = 16: 1.95 ms with 0.20 ms of gradient_signs_prepare (3.65 ms for the kernel that
+// flipped the sign into both pieces of A: three products and 2.5 vector instructions per term), O = 32 3.75 ms (5.55).  W from
+// pieces of A and C under a scale per row each, which loses bits as said above, took 1.94 and 3.70.
 // Up to 8 outputs leave half of the columns unused: there the columns 8 .. 15 take the second pieces (PIECES_IN_COLUMNS),
 // one matrix instruction instead of two.  Everything a step reads arrives in LDS by global_load_lds, a stage of 64 k in
 // one of two buffers while the other is worked on; the copies are inline instructions for the reason given in
@@ -55,10 +61,15 @@ constexpr int NGF_N_PAD = 256;
 constexpr int NGF_CORRECT_STAGES = 4;          // 1/2 sum W is taken off every so many stages
 constexpr int NGF_PREPARE_THREADS = 256;
 constexpr int NGF_PREPARE_GROUP = 256;
-constexpr int NGF_COPY_M = 64;                 // tile of the copy of A: m, and k per workgroup
-constexpr int NGF_COPY_K = 512;
-constexpr float NGF_SCALE_A = 0x1p-7f;         // of what gram_scale gives (2^14 .. 2^15): A in [2^7, 2^8), C in [2^6, 2^7),
-constexpr float NGF_SCALE_C = 0x1p-8f;         // and W below 2^15
+constexpr int NGF_M_PAD = 64;
+constexpr int NGF_COPY_M = 128;                // tile of the copy of A: m, and k per workgroup at most and at least
+constexpr int NGF_COPY_MAX_K = 512;
+constexpr int NGF_COPY_MIN_K = 64;
+constexpr int NGF_COPY_DEPTH = 16;             // k per lane at a time
+constexpr int NGF_COPY_C_PITCH = NGF_TILE_O + 4;       // words of LDS per two k of 16 o
+constexpr int NGF_EXPONENT_W = 14;             // largest W of a result in [2^14, 2^15.2): fp16 ends at 2^16
+constexpr int NGF_EXPONENT_C = 14;             // largest C of a row as it is copied, in [2^14, 2^15): A, which takes the rest of W's scale, is
+                                               // then brought to 1 or a little more
 constexpr int NGF_MAX_CHUNK = 14272;           // k per sorted chunk: whole stages, counts up to 14334 (signs_half)
 
 struct NormGradientF16Args {
@@ -69,10 +80,11 @@ struct NormGradientF16Args {
     i64 positions_bs, counts_bs;               // in halves
     const float *a_copy; i64 a_copy_bs;        // [batch][m_pad / 2][k_pad / 32][4][2][8]: 8 k of each of 2 m, 4 times
     const float *a_magnitudes; i64 a_magnitudes_bs;    // [batch][ranges][m_pad]
-    const gram_chunk *c_pieces; i64 c_pieces_bs;       // [batch][o_pad / 16][k_pad / 8][2 pieces][16 o] of 8 k
-    const float *c_unscale; i64 c_unscale_bs;  // [batch][o_pad]
-    int n_pad, m_pad, k_pad, ranges;
-    int chunks, chunk_stages, stages;          // sorted chunks, their length (the last may be shorter), all stages
+    const unsigned short *products; i64 products_bs;   // [batch][ranges][o_pad / 16][m_pad][16 o]: signs_product
+    const float *c_copy; i64 c_copy_bs;        // [batch][o_pad / 16][k_pad / 4][16 o][4 k], times 2^c_exponents
+    const int *c_exponents; i64 c_exponents_bs;        // [batch][o_pad]
+    int n_pad, m_pad, k_pad, o_pad, ranges;
+    int chunk_stages, stages;                  // length of the sorted chunks (the last may be shorter), all stages
 };
 
 struct GradientPrepareArgs {
@@ -84,13 +96,14 @@ struct GradientPrepareArgs {
     unsigned short *positions, *counts; i64 positions_bs, counts_bs;
     float *a_copy; i64 a_copy_bs;
     float *a_magnitudes; i64 a_magnitudes_bs;
-    gram_chunk *c_pieces; i64 c_pieces_bs;
-    float *c_unscale; i64 c_unscale_bs;
-    int n_pad, m_pad, k_pad, o_pad, ranges, chunks, chunk_k;
+    unsigned short *products; i64 products_bs;
+    float *c_copy; i64 c_copy_bs;
+    int *c_exponents; i64 c_exponents_bs;
+    int n_pad, m_pad, k_pad, o_pad, copy_k, ranges, chunk_k;
     int sort_d;                                // the rows of D are sorted, not those of B
-    int sort_blocks, copy_blocks;              // rows to sort, tiles of A, ...
+    int sort_blocks, copy_blocks;              // rows to sort, tiles of A times blocks of 16 o, ...
     int sort_groups, copy_groups;              // ... and how many groups of NGF_PREPARE_GROUP that makes; blockIdx.x also has the rows of C
-    int sort_batches, a_batches, c_batches;    // blockIdx.y
+    int sort_batches, a_batches, c_batches, product_batches;       // blockIdx.y
     int a_vec;
 };
 
@@ -244,115 +257,216 @@ __device__ __forceinline__ void signs_rank_row(const GradientPrepareArgs &args, 
     }
 }
 
-// 64 m x 512 k of A into the order of the product's waves, and the largest magnitude per m.  Memory-bound.
-__device__ __forceinline__ void signs_copy_tile(const GradientPrepareArgs &args, int block, int batch, float *tile)
+typedef unsigned short ngf_ushort2 __attribute__((ext_vector_type(2)));
+
+// The upper halves of |x0| and |x1|.  As an integer, that of x is 128 (127 + log2|x|), below it by no more than 128 * 0.094 (the
+// mantissa stands for its logarithm, and its last bits are missing), so the sum of two of them is the logarithm of a
+// product, and finding the largest product of a row takes an addition and a maximum of 16 bits per term.
+__device__ __forceinline__ ngf_ushort2 signs_logarithms(float x0, float x1)
 {
-    constexpr int PITCH = NGF_COPY_M + 1;
-    constexpr int ROUNDS = NGF_STAGE_K * NGF_COPY_M / 4 / NGF_PREPARE_THREADS;      // of four values per thread, per 64 k
-    const int tid = threadIdx.x;
-    const int m_tiles = args.m_pad / NGF_COPY_M;
-    const int m0 = block % m_tiles * NGF_COPY_M, range = block / m_tiles;
-    const int k_end = min((range + 1) * NGF_COPY_K, args.k_pad);
+    return __builtin_bit_cast(ngf_ushort2, __builtin_amdgcn_perm(__float_as_uint(x1), __float_as_uint(x0), 0x07060302u) & 0x7fff7fffu);
+}
+
+// 128 m x copy_k k of A into the order of the product's waves, the largest magnitude per m, and the logarithm of the largest |a c| per m
+// and o of one block of 16 outputs (the blocks after the first only that).  A lane holds 2 m and 16 k at a time, which are 128
+// bytes of the copy; a wave takes a quarter of the k; the logarithms of C stand in LDS and are read as broadcasts.  Memory-bound
+// together with the sorts beside it for 16 outputs (8192 x 512 x 16 x 8192: the launch 0.18 ms without the products, 0.20 with them), beyond that
+// bound by the vector ALU, 4.6 cycles of a SIMD per 64 terms: 4000 x 32 x 128 x 4000 0.05 without, 0.13 with them.
+__device__ __forceinline__ void signs_copy_tile(const GradientPrepareArgs &args, int block, int batch, unsigned *shared)
+{
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int o_blocks = args.o_pad / NGF_TILE_O, m_tiles = (args.m_pad + NGF_COPY_M - 1) / NGF_COPY_M;
+    // the blocks of outputs of a tile run one behind the other on one XCD, whose L2 then holds the tile for all but the first
+    const int o_block = block / BK_XCDS % o_blocks, at = block / BK_XCDS / o_blocks * BK_XCDS + block % BK_XCDS;
+    const int m0 = at % m_tiles * NGF_COPY_M, range = at / m_tiles;
+    if (range >= args.ranges) return;
+    const int o_count = min(args.o - NGF_TILE_O * o_block, NGF_TILE_O);
+    const int k_first = range * args.copy_k, k_count = min(args.copy_k, args.k_pad - k_first);
+    const bool copies = o_block == 0 && batch < args.a_batches;
+
+    // loads of what does not exist, of C and of A, go to the last element that does and are dropped: with a branch for each they would be
+    // waited for one by one
+    const float *c = args.c + batch * args.c_bs + (i64)NGF_TILE_O * o_block * args.c_ld;
+    for (int pair = tid; pair < k_count / 2; pair += NGF_PREPARE_THREADS) {
+        const int k = k_first + 2 * pair, at0 = min(k, args.k - 1), at1 = min(k + 1, args.k - 1);
+        float x[NGF_TILE_O][2];
+#pragma unroll
+        for (int o = 0; o < NGF_TILE_O; o++) {
+            const float *row = c + (i64)min(o, o_count - 1) * args.c_ld;
+            x[o][0] = row[at0];
+            x[o][1] = row[at1];
+        }
+#pragma unroll
+        for (int o = 0; o < NGF_TILE_O; o++) {
+            const bool live = o < o_count;
+            shared[pair * NGF_COPY_C_PITCH + o] =
+                __builtin_bit_cast(unsigned, signs_logarithms(live && k < args.k ? x[o][0] : 0.0f, live && k + 1 < args.k ? x[o][1] : 0.0f));
+        }
+    }
+
+    const int m = m0 + 2 * lane;
     const float *a = args.a + batch * args.a_bs;
-    float *copy = args.a_copy + batch * args.a_copy_bs;
-    // loads: 4 m of one k.  Stores: 4 k of one m, of pair `pair` (of 8 per round) and step `step` of the 64 k
-    const int load_k = tid >> 4, load_m = (tid & 15) * 4;
-    const int pair = tid >> 5, step = tid >> 4 & 1, q = tid >> 2 & 3, which = tid >> 1 & 1, low = (tid & 1) * 4;
-    auto load = [&](int k0, float (&v)[ROUNDS][4]) {
+    const bool aligned = args.a_vec && m0 + NGF_COPY_M <= args.m;
+    float2 v[NGF_COPY_DEPTH];
+    auto load = [&](int k0) {
+        if (aligned && k0 + NGF_COPY_DEPTH <= args.k) {
 #pragma unroll
-        for (int round = 0; round < ROUNDS; round++) {
-            const int k = k0 + load_k + 16 * round;
-            const float *src = a + (i64)k * args.a_ld + m0 + load_m;
-            if (k < args.k && args.a_vec && m0 + load_m + 4 <= args.m) {
-                const float4 f = *reinterpret_cast<const float4 *>(src);
-                v[round][0] = f.x; v[round][1] = f.y; v[round][2] = f.z; v[round][3] = f.w;
-            } else {
+            for (int j = 0; j < NGF_COPY_DEPTH; j++) v[j] = *reinterpret_cast<const float2 *>(a + (i64)(k0 + j) * args.a_ld + m);
+        } else {
+            const int at0 = min(m, args.m - 1), at1 = min(m + 1, args.m - 1);
 #pragma unroll
-                for (int j = 0; j < 4; j++) v[round][j] = (k < args.k && m0 + load_m + j < args.m) ? src[j] : 0.0f;
+            for (int j = 0; j < NGF_COPY_DEPTH; j++) {
+                const float *row = a + (i64)min(k0 + j, args.k - 1) * args.a_ld;
+                v[j] = make_float2(row[at0], row[at1]);
+            }
+#pragma unroll
+            for (int j = 0; j < NGF_COPY_DEPTH; j++) {
+                v[j].x = k0 + j < args.k && m < args.m ? v[j].x : 0.0f;
+                v[j].y = k0 + j < args.k && m + 1 < args.m ? v[j].y : 0.0f;
             }
         }
     };
-    float magnitude[ROUNDS] = {};
-    float v[ROUNDS][4];
-    load(range * NGF_COPY_K, v);
-    for (int k0 = range * NGF_COPY_K; k0 < k_end; k0 += NGF_STAGE_K) {
-        __syncthreads();
+    float magnitude[2] = {0.0f, 0.0f};
+    ngf_ushort2 largest[2][NGF_TILE_O];                    // over even and odd k
 #pragma unroll
-        for (int round = 0; round < ROUNDS; round++)
+    for (int i = 0; i < 2; i++)
 #pragma unroll
-            for (int j = 0; j < 4; j++) tile[(load_k + 16 * round) * PITCH + load_m + j] = v[round][j];
-        __syncthreads();
-        if (k0 + NGF_STAGE_K < k_end) load(k0 + NGF_STAGE_K, v);
+        for (int o = 0; o < NGF_TILE_O; o++) largest[i][o] = ngf_ushort2{0, 0};
+    const int k_wave = k_first + wave * (k_count / 4), k_end = k_wave + k_count / 4;        // k_count: a multiple of 64
+    load(k_wave);
+    __syncthreads();
+    for (int k0 = k_wave; k0 < k_end; k0 += NGF_COPY_DEPTH) {
+        ngf_ushort2 logarithms[2][NGF_COPY_DEPTH / 2];
 #pragma unroll
-        for (int round = 0; round < ROUNDS; round++) {
-            float w[4];
+        for (int j = 0; j < NGF_COPY_DEPTH / 2; j++) {
+            logarithms[0][j] = signs_logarithms(v[2 * j].x, v[2 * j + 1].x);
+            logarithms[1][j] = signs_logarithms(v[2 * j].y, v[2 * j + 1].y);
+        }
+        if (copies) {
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                w[j] = tile[(NGF_STEP_K * step + 8 * q + low + j) * PITCH + 2 * (pair + 8 * round) + which];
-                magnitude[round] = fmaxf(magnitude[round], fabsf(w[j]));      // skips NaNs, whose products are not numbers at any scale
+            for (int j = 0; j < NGF_COPY_DEPTH; j++) {     // skips NaNs, whose products are not numbers at any scale
+                magnitude[0] = fmaxf(magnitude[0], fabsf(v[j].x));
+                magnitude[1] = fmaxf(magnitude[1], fabsf(v[j].y));
             }
-            float *dst = copy + ((i64)(m0 / 2 + pair + 8 * round) * (args.k_pad / NGF_STEP_K) + k0 / NGF_STEP_K + step) * 64 + (tid & 15) * 4;
-            *reinterpret_cast<float4 *>(dst) = make_float4(w[0], w[1], w[2], w[3]);
+            if (m < args.m_pad) {
+                float4 *dst = reinterpret_cast<float4 *>(args.a_copy + batch * args.a_copy_bs + ((i64)(m / 2) * args.k_pad + k0) * 2);
+#pragma unroll
+                for (int eight = 0; eight < NGF_COPY_DEPTH; eight += 8)
+#pragma unroll
+                    for (int j = 0; j < 8; j += 4) {
+                        dst[eight / 2 + j / 4] = make_float4(v[eight + j].x, v[eight + j + 1].x, v[eight + j + 2].x, v[eight + j + 3].x);
+                        dst[eight / 2 + 2 + j / 4] = make_float4(v[eight + j].y, v[eight + j + 1].y, v[eight + j + 2].y, v[eight + j + 3].y);
+                    }
+            }
+        }
+        if (k0 + NGF_COPY_DEPTH < k_end) load(k0 + NGF_COPY_DEPTH);
+        const uint4 *of_c = reinterpret_cast<const uint4 *>(shared + (k0 - k_first) / 2 * NGF_COPY_C_PITCH);
+        // four outputs at a time, so that the reads of their logarithms stand side by side behind one branch
+#pragma unroll
+        for (int o4 = 0; o4 < NGF_TILE_O / 4; o4++) {
+            if (4 * o4 >= o_count) continue;
+#pragma unroll
+            for (int j = 0; j < NGF_COPY_DEPTH / 2; j++) {
+                const uint4 x = of_c[j * (NGF_COPY_C_PITCH / 4) + o4];
+                const unsigned words[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+                for (int o = 0; o < 4; o++)
+#pragma unroll
+                    for (int i = 0; i < 2; i++)
+                        largest[i][4 * o4 + o] = __builtin_elementwise_max(largest[i][4 * o4 + o], logarithms[i][j] + __builtin_bit_cast(ngf_ushort2, words[o]));
+            }
         }
     }
-    // the lanes that share m: all bits of the lane but 1 (which) and 5 (pair)
+    // the four waves' largest: [wave][i][two outputs to a word][lane], and behind them the magnitudes
+    constexpr int WORDS = NGF_TILE_O / 2;
+    float *const magnitudes = reinterpret_cast<float *>(shared + 4 * 2 * WORDS * 64);
+    __syncthreads();
 #pragma unroll
-    for (int round = 0; round < ROUNDS; round++) {
+    for (int i = 0; i < 2; i++) {
 #pragma unroll
-        for (int bit : {1, 4, 8, 16}) magnitude[round] = fmaxf(magnitude[round], __shfl_xor(magnitude[round], bit));
-        if ((tid & 0x1d) == 0)
-            args.a_magnitudes[batch * args.a_magnitudes_bs + (i64)range * args.m_pad + m0 + 2 * (pair + 8 * round) + which] = magnitude[round];
+        for (int j = 0; j < WORDS; j++) {
+            const ngf_ushort2 first = largest[i][2 * j], second = largest[i][2 * j + 1];
+            shared[((wave * 2 + i) * WORDS + j) * 64 + lane] = max(first.x, first.y) | (unsigned)max(second.x, second.y) << 16;
+        }
+        magnitudes[(wave * 2 + i) * 64 + lane] = magnitude[i];
+    }
+    __syncthreads();
+    const int to = m0 + (tid >> 1), i = tid >> 1 & 1;      // half of the outputs of one m per thread
+    if (to >= args.m_pad) return;
+    if (batch < args.product_batches) {
+        unsigned word[WORDS / 2];
+#pragma unroll
+        for (int j = 0; j < WORDS / 2; j++) {
+            ngf_ushort2 x = {0, 0};
+#pragma unroll
+            for (int part = 0; part < 4; part++)
+                x = __builtin_elementwise_max(x, __builtin_bit_cast(ngf_ushort2, shared[((part * 2 + i) * WORDS + WORDS / 2 * (tid & 1) + j) * 64 + (tid >> 2)]));
+            word[j] = __builtin_bit_cast(unsigned, x);
+        }
+        unsigned short *products = args.products + batch * args.products_bs + (((i64)range * o_blocks + o_block) * args.m_pad + to) * NGF_TILE_O;
+        reinterpret_cast<uint4 *>(products)[tid & 1] = make_uint4(word[0], word[1], word[2], word[3]);
+    }
+    if (copies && !(tid & 1)) {
+        float x = 0.0f;
+#pragma unroll
+        for (int part = 0; part < 4; part++) x = fmaxf(x, magnitudes[(part * 2 + i) * 64 + (tid >> 2)]);
+        args.a_magnitudes[batch * args.a_magnitudes_bs + (i64)range * args.m_pad + to] = x;
     }
 }
 
-// One row o of C as two fp16 pieces, its largest magnitude in [2^6, 2^7), zeros beyond K and O
-__device__ __forceinline__ void signs_split_row(const GradientPrepareArgs &args, int o, int batch, float *shared)
+// Exponent of the first bit of a number (of its scale, which the largest value of a row is)
+__device__ __forceinline__ int signs_exponent(float magnitude)
+{
+    return ((int)(__float_as_uint(magnitude) >> 23) & 0xff) - 127;
+}
+
+// One row o of C times the power of two that brings its largest magnitude to [2^14, 2^15), zeros beyond K and O
+__device__ __forceinline__ void signs_scale_row(const GradientPrepareArgs &args, int o, int batch, float *shared)
 {
     const int tid = threadIdx.x;
     const float *row = args.c + batch * args.c_bs + (i64)o * args.c_ld;
     const bool live = o < args.o;
     float magnitude = 0.0f;
     if (live)
-        for (int k = tid; k < args.k; k += NGF_PREPARE_THREADS) magnitude = fmaxf(magnitude, fabsf(row[k]));
+        for (int k = tid; k < args.k; k += 4 * NGF_PREPARE_THREADS)
+#pragma unroll
+            for (int j = 0; j < 4; j++) magnitude = fmaxf(magnitude, fabsf(row[min(k + j * NGF_PREPARE_THREADS, args.k - 1)]));
 #pragma unroll
     for (int bit = 1; bit < 64; bit *= 2) magnitude = fmaxf(magnitude, __shfl_xor(magnitude, bit));
     if ((tid & 63) == 0) shared[tid >> 6] = magnitude;
     __syncthreads();
 #pragma unroll
     for (int wave = 0; wave < NGF_PREPARE_THREADS / 64; wave++) magnitude = fmaxf(magnitude, shared[wave]);
-    const int exponent_field = gram_scale_exponent(magnitude);
-    const float scale = gram_scale(exponent_field) * NGF_SCALE_C;
-    if (tid == 0) args.c_unscale[batch * args.c_unscale_bs + o] = gram_unscale(exponent_field) * (1.0f / NGF_SCALE_C);
-    gram_chunk *pieces = args.c_pieces + batch * args.c_pieces_bs + (i64)(o / 16) * args.k_pad / 8 * 32 + o % 16;
-    for (int k = 8 * tid; k < args.k_pad; k += 8 * NGF_PREPARE_THREADS) {
-        gram_chunk first, second;
+    const int exponent = NGF_EXPONENT_C - signs_exponent(magnitude);
+    if (tid == 0) args.c_exponents[batch * args.c_exponents_bs + o] = exponent;
+    float4 *copy = reinterpret_cast<float4 *>(args.c_copy + batch * args.c_copy_bs) + (i64)(o / NGF_TILE_O) * args.k_pad / 4 * NGF_TILE_O + o % NGF_TILE_O;
+    for (int k = 4 * tid; k < args.k_pad; k += 4 * NGF_PREPARE_THREADS) {
+        float v[4];
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            unsigned h1, h2;
-            gram_split_pair(live && k + 2 * j < args.k ? row[k + 2 * j] * scale : 0.0f,
-                            live && k + 2 * j + 1 < args.k ? row[k + 2 * j + 1] * scale : 0.0f, h1, h2);
-            first[j] = h1; second[j] = h2;
-        }
-        pieces[(i64)(k / 8) * 32] = first;
-        pieces[(i64)(k / 8) * 32 + 16] = second;
+        for (int j = 0; j < 4; j++) v[j] = live ? row[min(k + j, args.k - 1)] : 0.0f;
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[j] = k + j < args.k ? __builtin_ldexpf(v[j], exponent) : 0.0f;
+        copy[(i64)(k / 4) * NGF_TILE_O] = make_float4(v[0], v[1], v[2], v[3]);
     }
 }
 
-// Rows to sort keep LDS busy, tiles of A the memory, so the two are dealt out in turn, in groups of one workgroup per
-// CU, spread evenly over the launch; the rows of C come last.
+// Rows to sort keep LDS busy, tiles of A the memory and the vector ALU, so the two are dealt out in turn, in groups of one workgroup per
+// CU, spread evenly over the launch (all sorts within its first half: 214 us in the place of 200 at 8192 x 512 x 16 x 8192).  The rows of C, few
+// and slow, come first.
 template <int LOG_R>
-__global__ __launch_bounds__(NGF_PREPARE_THREADS) void gradient_signs_prepare(const GradientPrepareArgs args)
+__global__ __launch_bounds__(NGF_PREPARE_THREADS, LOG_R < 6 ? 4 : 2) void gradient_signs_prepare(const GradientPrepareArgs args)
 {
     constexpr int WORDS = (256 << LOG_R) + (8 << LOG_R);
-    constexpr int TILE_WORDS = NGF_STAGE_K * (NGF_COPY_M + 1);
-    __shared__ unsigned words[WORDS > TILE_WORDS ? WORDS : TILE_WORDS];
-    const int batch = blockIdx.y;
-    const i64 groups = args.sort_groups + args.copy_groups, group = blockIdx.x / NGF_PREPARE_GROUP;
-    const int within = blockIdx.x % NGF_PREPARE_GROUP;
-    if (group >= groups) {
-        if (batch < args.c_batches) signs_split_row(args, blockIdx.x - (int)groups * NGF_PREPARE_GROUP, batch, reinterpret_cast<float *>(words));
+    constexpr int TILE_WORDS = NGF_COPY_MAX_K / 2 * NGF_COPY_C_PITCH;
+    static_assert(TILE_WORDS >= 4 * 64 * (NGF_TILE_O + 2), "the waves' results");
+    __shared__ __attribute__((aligned(16))) unsigned words[WORDS > TILE_WORDS ? WORDS : TILE_WORDS];
+    const int batch = blockIdx.y, block_behind_c = (int)blockIdx.x - args.o_pad;
+    if (block_behind_c < 0) {
+        if (batch < args.c_batches) signs_scale_row(args, blockIdx.x, batch, reinterpret_cast<float *>(words));
         return;
     }
+    const i64 groups = args.sort_groups + args.copy_groups, group = block_behind_c / NGF_PREPARE_GROUP;
+    const int within = block_behind_c % NGF_PREPARE_GROUP;
     const int sorts_before = (int)((group * args.sort_groups + groups - 1) / groups);
     const int sorts_behind = (int)(((group + 1) * args.sort_groups + groups - 1) / groups);
     if (sorts_behind > sorts_before) {
@@ -360,7 +474,7 @@ __global__ __launch_bounds__(NGF_PREPARE_THREADS) void gradient_signs_prepare(co
         if (block < args.sort_blocks && batch < args.sort_batches) signs_rank_row<LOG_R>(args, block, batch, words);
     } else {
         const int block = ((int)group - sorts_before) * NGF_PREPARE_GROUP + within;
-        if (block < args.copy_blocks && batch < args.a_batches) signs_copy_tile(args, block, batch, reinterpret_cast<float *>(words));
+        if (block < args.copy_blocks && batch < max(args.a_batches, args.product_batches)) signs_copy_tile(args, block, batch, words);
     }
 }
 
@@ -389,8 +503,8 @@ struct GradientF16Tile {
     static constexpr int PASS_BLOCKS = BLOCKS < 4 ? BLOCKS : 2;         // of 16 n, per pass of the epilogue
     static constexpr int RESULT_PITCH = NGF_TILE_M + 4;
     static constexpr int PASS_CHUNKS = PASS_BLOCKS * 256 * RESULT_PITCH / 4;
-    // two stages of everything, of A as it is and in pieces: 88 KB at 256 n
-    static constexpr int STAGE_CHUNKS = 2 * (POSITION_CHUNKS + C_CHUNKS + A_CHUNKS + A_CHUNKS);
+    // two stages of everything: 80 KB at 256 n
+    static constexpr int STAGE_CHUNKS = 2 * (POSITION_CHUNKS + C_CHUNKS + A_CHUNKS);
     static constexpr int CHUNKS = STAGE_CHUNKS > PASS_CHUNKS ? STAGE_CHUNKS : PASS_CHUNKS;
 };
 
@@ -431,7 +545,8 @@ __global__ __launch_bounds__(NGF_THREADS, BLOCKS >= 8 ? 2 : 4) void norm_gradien
                           (BLOCKS >= 4 ? 64 * (copy % COPIES_PER_RUN) + lane : lane & 31);
         position_dst[j] = 64 * copy;
     }
-    const gram_chunk *c_src = args.c_pieces + batch * args.c_pieces_bs + (i64)(o0 / 16) * args.k_pad / 8 * 32 + 64 * (wave & 3) + lane;
+    const gram_chunk *c_src = reinterpret_cast<const gram_chunk *>(args.c_copy + batch * args.c_copy_bs) +
+                              (i64)(o0 / NGF_TILE_O) * args.k_pad / 4 * NGF_TILE_O + 64 * (wave & 3) + lane;
     const float *a_src = args.a_copy + batch * args.a_copy_bs + (i64)(m0 / 2 + wave) * (args.k_pad / NGF_STEP_K) * 64 + lane;
     auto copy16 = [&](const gram_chunk *src, gram_chunk *dst) {
         const unsigned lds_byte = (unsigned)(unsigned long)(lds_address)dst;
@@ -443,7 +558,6 @@ __global__ __launch_bounds__(NGF_THREADS, BLOCKS >= 8 ? 2 : 4) void norm_gradien
     };
     gram_chunk *const lds_c = lds + 2 * Tile::POSITION_CHUNKS;
     gram_chunk *const lds_a = lds_c + 2 * Tile::C_CHUNKS;
-    unsigned *const a_pieces = reinterpret_cast<unsigned *>(lds_a + 2 * Tile::A_CHUNKS) + 128 * wave;        // [stage % 2][wave][piece][64]
     auto copy_stage = [&](int into) {
 #pragma unroll
         for (int j = 0; j < POSITION_COPIES; j++) {
@@ -452,28 +566,39 @@ __global__ __launch_bounds__(NGF_THREADS, BLOCKS >= 8 ? 2 : 4) void norm_gradien
         }
         copy16(c_src, lds_c + into * Tile::C_CHUNKS + 64 * (wave & 3));
         c_src += Tile::C_CHUNKS;
-    };
-    auto copy_a = [&](int into) {
 #pragma unroll
         for (int j = 0; j < 2; j++) copy4(a_src + 64 * j, lds_a + into * Tile::A_CHUNKS + 32 * wave + 16 * j);
         a_src += 128;
     };
 
-    // scale of the lane's m in split_a: 8 k of m0 + 2 wave, 8 k of m0 + 2 wave + 1 and so on, two k per lane
-    float scale_a, unscale_a[2];
+    // The lane's column, and the power of two for A of each of the wave's two m, which with the scale of C makes W's largest value 2^14 or a
+    // little more.  A stays finite with it (one that would not meets a C of zero, or of less than 2^-100 of its row).
+    const int column = PIECES_IN_COLUMNS ? (r & 7) : r;
+    float scale[2];
+    int unscale[2];
     {
         const float *magnitudes = args.a_magnitudes + batch * args.a_magnitudes_bs + m0 + 2 * wave;
-        float largest[2] = {0.0f, 0.0f};
-        for (int range = lane; range < args.ranges; range += 64)
+        const unsigned short *products = args.products + batch * args.products_bs + ((i64)(o0 / NGF_TILE_O) * args.m_pad + m0 + 2 * wave) * NGF_TILE_O + column;
+        float magnitude[2] = {0.0f, 0.0f};
+        int product[2] = {0, 0};
+        for (int range = q; range < args.ranges; range += 4)
 #pragma unroll
-            for (int i = 0; i < 2; i++) largest[i] = fmaxf(largest[i], magnitudes[(i64)range * args.m_pad + i]);
+            for (int i = 0; i < 2; i++) {
+                magnitude[i] = fmaxf(magnitude[i], magnitudes[(i64)range * args.m_pad + i]);
+                product[i] = max(product[i], (int)products[(i64)range * args.o_pad * args.m_pad + NGF_TILE_O * i]);
+            }
+        const int c_exponent = args.c_exponents[batch * args.c_exponents_bs + o0 + column];
 #pragma unroll
         for (int i = 0; i < 2; i++) {
 #pragma unroll
-            for (int bit = 1; bit < 64; bit *= 2) largest[i] = fmaxf(largest[i], __shfl_xor(largest[i], bit));
-            unscale_a[i] = gram_unscale(gram_scale_exponent(largest[i])) * (1.0f / NGF_SCALE_A);
+            for (int bit : {16, 32}) {
+                magnitude[i] = fmaxf(magnitude[i], __shfl_xor(magnitude[i], bit));
+                product[i] = max(product[i], __shfl_xor(product[i], bit));
+            }
+            const int exponent = min(min(NGF_EXPONENT_W - ((product[i] >> 7) - 254) - c_exponent, 126 - signs_exponent(magnitude[i])), 127);
+            scale[i] = __builtin_ldexpf(1.0f, exponent);
+            unscale[i] = 1 - exponent - c_exponent;          // doubled: 2 S - 1 is summed as S - 1/2
         }
-        scale_a = gram_scale(gram_scale_exponent(lane & 4 ? largest[1] : largest[0])) * NGF_SCALE_A;
     }
     // counts of the lane's rows n for the wave's two m, one dword per block
     const unsigned short *counts = args.counts + batch * args.counts_bs + (i64)(n0 + r) * args.m_pad + m0 + 2 * wave;
@@ -493,49 +618,48 @@ __global__ __launch_bounds__(NGF_THREADS, BLOCKS >= 8 ? 2 : 4) void norm_gradien
 #pragma unroll
         for (int block = 0; block < BLOCKS; block++) acc[i][block] = ngf_float4{0.0f, 0.0f, 0.0f, 0.0f};
     float sum_w[2] = {0.0f, 0.0f};
-    const int column = PIECES_IN_COLUMNS ? (r & 7) : r;
 
-    // A of a stage into two pieces, by the wave that uses it
-    auto split_a = [&](int into) {
-        const float2 a = reinterpret_cast<const float2 *>(lds_a + into * Tile::A_CHUNKS)[64 * wave + lane];
-        unsigned h1, h2;
-        gram_split_pair(a.x * scale_a, a.y * scale_a, h1, h2);
-        a_pieces[128 * NGF_WAVES * into + lane] = h1;
-        a_pieces[128 * NGF_WAVES * into + 64 + lane] = h2;
-    };
     auto step = [&](int from, int half) {
         const gram_chunk *positions = lds + from * Tile::POSITION_CHUNKS + (4 * half + q) * Tile::TILE_N + r;
-        gram_chunk c[GW_PIECES];
+        float c[8];
 #pragma unroll
-        for (int piece = 0; piece < GW_PIECES; piece++) c[piece] = lds_c[from * Tile::C_CHUNKS + (4 * half + q) * 32 + 16 * piece + column];
+        for (int j = 0; j < 2; j++) {
+            const float4 x = reinterpret_cast<const float4 *>(lds_c)[from * Tile::C_CHUNKS + (4 * half + q) * 32 + 16 * j + column];
+            c[4 * j] = x.x; c[4 * j + 1] = x.y; c[4 * j + 2] = x.z; c[4 * j + 3] = x.w;
+        }
         gram_half8 w[2][COLUMN_PIECES];
 #pragma unroll
         for (int i = 0; i < 2; i++) {
-            gram_chunk a[GW_PIECES];
+            float a[8];
 #pragma unroll
-            for (int piece = 0; piece < GW_PIECES; piece++)
-                a[piece] = reinterpret_cast<const gram_chunk *>(a_pieces + 128 * NGF_WAVES * from + 64 * piece)[8 * half + 2 * q + i];
+            for (int j = 0; j < 2; j++) {
+                const float4 x = reinterpret_cast<const float4 *>(lds_a)[from * Tile::A_CHUNKS + 32 * wave + 16 * half + 4 * q + 2 * i + j];
+                a[4 * j] = x.x; a[4 * j + 1] = x.y; a[4 * j + 2] = x.z; a[4 * j + 3] = x.w;
+            }
             gram_chunk first, second;
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                const ngf_half2 a1 = signs_halves(a[0][j]), a2 = signs_halves(a[1][j]);
-                const ngf_half2 c1 = signs_halves(c[0][j]), c2 = signs_halves(c[1][j]);
-                const ngf_half2 h1 = a1 * c1;
-                const ngf_half2 h2 = __builtin_elementwise_fma(a2, c1, __builtin_elementwise_fma(a1, c2, __builtin_elementwise_fma(a1, c1, -h1)));
-                first[j] = __builtin_bit_cast(unsigned, h1);
-                second[j] = __builtin_bit_cast(unsigned, h2);
-                const ngf_half2 one = {(_Float16)1, (_Float16)1};
-                sum_w[i] = __builtin_amdgcn_fdot2(h1, one, sum_w[i], false);
-                sum_w[i] = __builtin_amdgcn_fdot2(h2, one, sum_w[i], false);
+                const float a0 = a[2 * j] * scale[i], a1 = a[2 * j + 1] * scale[i];
+                const float w0 = a0 * c[2 * j], w1 = a1 * c[2 * j + 1];
+                sum_w[i] += w0;
+                sum_w[i] += w1;
+                // What a pair of W costs is its instructions: 2.4 cycles for one of fp32, 4.6 for a packed or mixed one or a conversion, 8.3
+                // for one that rounds into half a register (which the compiler takes for a difference that is rounded at once)
+                gram_half2 h1 = __builtin_convertvector(gram_float2{w0, w1}, gram_half2);
+                asm("" : "+v"(h1));
+                // columns with the first pieces take nothing off: what is left is then W, and its rounding the first piece
+                if constexpr (PIECES_IN_COLUMNS) h1 = __builtin_bit_cast(gram_half2, __builtin_bit_cast(unsigned, h1) & (r < 8 ? 0u : ~0u));
+                float left0 = __builtin_fmaf(a0, c[2 * j], -(float)h1.x), left1 = __builtin_fmaf(a1, c[2 * j + 1], -(float)h1.y);
+                asm("" : "+v"(left0), "+v"(left1));
+                const unsigned left = __builtin_bit_cast(unsigned, __builtin_convertvector(gram_float2{left0, left1}, gram_half2));
+                first[j] = PIECES_IN_COLUMNS ? left : __builtin_bit_cast(unsigned, h1);
+                second[j] = left;
             }
-            if constexpr (PIECES_IN_COLUMNS) {
-#pragma unroll
-                for (int j = 0; j < 4; j++) first[j] = r < 8 ? first[j] : second[j];
-                w[i][0] = __builtin_bit_cast(gram_half8, first);
-            } else {
-                w[i][0] = __builtin_bit_cast(gram_half8, first);
-                w[i][1] = __builtin_bit_cast(gram_half8, second);
-            }
+            w[i][0] = __builtin_bit_cast(gram_half8, first);
+            if constexpr (!PIECES_IN_COLUMNS) w[i][1] = __builtin_bit_cast(gram_half8, second);
+            // where 128 registers are all, W is summed here: left to itself the sum runs beside the matrix instructions, which is faster (8192 x
+            // 512 x 16 x 8192 2 %) but keeps a and c until then
+            if constexpr (PIECES_IN_COLUMNS && BLOCKS == 4) asm volatile("" : "+v"(sum_w[i]));
         }
         gram_chunk p[3], s[2][2];
         auto compare = [&](int block, const gram_chunk &at, gram_chunk (&into)[2]) {
@@ -583,13 +707,9 @@ __global__ __launch_bounds__(NGF_THREADS, BLOCKS >= 8 ? 2 : 4) void norm_gradien
         }
     };
 
-    // Positions and C are copied one stage ahead, A two: it is split in the stage before.  (Three buffers and copies two and
-    // three stages ahead: the same time; the copies' latency is not what bounds a stage.)
-    copy_a(0);
+    // Copies go one stage ahead.  (Three buffers and copies two and three stages ahead: the same time; the copies' latency is not
+    // what bounds a stage.)
     copy_stage(0);
-    if (args.stages > 1) copy_a(1);
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-    split_a(0);
     int chunk = 0, chunk_left = args.chunk_stages;
     for (int stage = 0; stage < args.stages; stage++) {
         // the wave's own copies have arrived; behind the barrier everybody's have, and the other buffer is free
@@ -603,8 +723,6 @@ __global__ __launch_bounds__(NGF_THREADS, BLOCKS >= 8 ? 2 : 4) void norm_gradien
         chunk_left--;
         const int here = stage & 1, other = here ^ 1;
         if (stage + 1 < args.stages) copy_stage(other);
-        if (stage + 2 < args.stages) copy_a(here);
-        if (stage + 1 < args.stages) split_a(other);
         step(here, 0);
         step(here, 1);
         if (stage % NGF_CORRECT_STAGES == NGF_CORRECT_STAGES - 1 || stage + 1 == args.stages) correct();
@@ -620,7 +738,6 @@ __global__ __launch_bounds__(NGF_THREADS, BLOCKS >= 8 ? 2 : 4) void norm_gradien
 #pragma unroll
                 for (int j = 0; j < 4; j++) acc[i][block][j] += __shfl_xor(acc[i][block][j], 8);
     }
-    const float unscale_c = 2.0f * args.c_unscale[batch * args.c_unscale_bs + o0 + column];
     float *results = reinterpret_cast<float *>(lds);
     constexpr int PITCH = Tile::RESULT_PITCH;
 #pragma unroll
@@ -632,7 +749,7 @@ __global__ __launch_bounds__(NGF_THREADS, BLOCKS >= 8 ? 2 : 4) void norm_gradien
             for (int j = 0; j < 4; j++) {
                 const int block = pass * Tile::PASS_BLOCKS + within;
                 *reinterpret_cast<float2 *>(results + ((16 * within + 4 * q + j) * 16 + r) * PITCH + 2 * wave) =
-                    make_float2(acc[0][block][j] * unscale_a[0] * unscale_c, acc[1][block][j] * unscale_a[1] * unscale_c);
+                    make_float2(__builtin_ldexpf(acc[0][block][j], unscale[0]), __builtin_ldexpf(acc[1][block][j], unscale[1]));
             }
         __syncthreads();
         constexpr int QUADS = NGF_TILE_M / 4;

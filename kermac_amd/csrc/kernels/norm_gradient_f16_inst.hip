@@ -18,11 +18,11 @@ constexpr int64_t REGION_ALIGN = 256;
 
 struct GradientLayout {
     int stages, n_pad, m_pad, k_pad, o_pad, ranges;
-    int chunks, chunk_k, keys;
+    int chunks, chunk_k, keys, copy_k, copy_blocks;
     bool sort_d;
-    int sort_batches, a_batches, c_batches;
-    int64_t positions_bs, counts_bs, a_copy_bs, a_magnitudes_bs, c_pieces_bs;     // in elements, of C in chunks of 16 bytes
-    int64_t positions, counts, a_copy, a_magnitudes, c_pieces, c_unscale;         // byte offsets into the workspace
+    int sort_batches, a_batches, c_batches, product_batches;
+    int64_t positions_bs, counts_bs, a_copy_bs, a_magnitudes_bs, products_bs, c_copy_bs;      // in elements
+    int64_t positions, counts, a_copy, a_magnitudes, products, c_copy, c_exponents;           // byte offsets into the workspace
     int64_t bytes;
 };
 
@@ -66,7 +66,7 @@ bool gradient_layout(const kmc_norm_gradient_params *p, GradientLayout *layout)
     if (!f16_pays(p)) return false;
     // a row n is a row of blockIdx.y in other kernels of its size: the fp32 kernels keep what they had
     if (round_up(p->n, 32) > 65535 || static_cast<int64_t>(p->l) * (p->o / 64 + 1) > 65535) return false;
-    const int64_t k_pad = round_up(p->k, kmc::NGF_STAGE_K), m_pad = round_up(p->m, kmc::NGF_COPY_M);
+    const int64_t k_pad = round_up(p->k, kmc::NGF_STAGE_K), m_pad = round_up(p->m, kmc::NGF_M_PAD);
     const int64_t n_pad = round_up(p->n, kmc::NGF_N_PAD), o_pad = round_up(p->o, kmc::NGF_TILE_O);
     // a dimension of a grid holds fewer than 2^32 threads
     const int64_t threads = int64_t{1} << 32;
@@ -76,12 +76,17 @@ bool gradient_layout(const kmc_norm_gradient_params *p, GradientLayout *layout)
     layout->chunk_k = static_cast<int>(round_up((p->k + layout->chunks - 1) / layout->chunks, kmc::NGF_STAGE_K));
     layout->chunks = (p->k + layout->chunk_k - 1) / layout->chunk_k;
     layout->keys = layout->sort_d ? p->m : layout->chunk_k;
-    layout->ranges = static_cast<int>((k_pad + kmc::NGF_COPY_K - 1) / kmc::NGF_COPY_K);
-    const int64_t prepare_blocks = static_cast<int64_t>(p->n) * layout->chunks + m_pad / kmc::NGF_COPY_M * layout->ranges + o_pad +
-                                   2 * kmc::NGF_PREPARE_GROUP;
+    // fewer k per tile of A where that leaves fewer tiles than two per CU
+    const int64_t tiles_m = (m_pad + kmc::NGF_COPY_M - 1) / kmc::NGF_COPY_M, tiles = tiles_m * (o_pad / kmc::NGF_TILE_O);
+    layout->copy_k = kmc::NGF_COPY_MAX_K;
+    while (layout->copy_k > kmc::NGF_COPY_MIN_K && tiles * p->l * ((k_pad + layout->copy_k - 1) / layout->copy_k) < 1024) layout->copy_k /= 2;
+    layout->ranges = static_cast<int>((k_pad + layout->copy_k - 1) / layout->copy_k);
+    const int64_t copy_blocks = round_up(tiles_m * layout->ranges, kmc::BK_XCDS) * (o_pad / kmc::NGF_TILE_O);
+    const int64_t prepare_blocks = static_cast<int64_t>(p->n) * layout->chunks + copy_blocks + o_pad + 2 * kmc::NGF_PREPARE_GROUP;
     if (prepare_blocks * kmc::NGF_PREPARE_THREADS >= threads || m_pad / kmc::NGF_TILE_M * kmc::NGF_THREADS >= threads || k_pad > INT32_MAX ||
         m_pad > INT32_MAX || o_pad > INT32_MAX)
         return false;
+    layout->copy_blocks = static_cast<int>(copy_blocks);
     layout->stages = static_cast<int>(k_pad / kmc::NGF_STAGE_K);
     layout->n_pad = static_cast<int>(n_pad); layout->m_pad = static_cast<int>(m_pad);
     layout->k_pad = static_cast<int>(k_pad); layout->o_pad = static_cast<int>(o_pad);
@@ -92,14 +97,17 @@ bool gradient_layout(const kmc_norm_gradient_params *p, GradientLayout *layout)
     layout->counts_bs = static_cast<int64_t>(layout->chunks) * n_pad * m_pad;
     layout->a_copy_bs = m_pad * k_pad;
     layout->a_magnitudes_bs = static_cast<int64_t>(layout->ranges) * m_pad;
-    layout->c_pieces_bs = o_pad * k_pad / 4;
+    layout->product_batches = layout->a_batches > 1 || layout->c_batches > 1 ? p->l : 1;
+    layout->products_bs = layout->ranges * o_pad * m_pad;
+    layout->c_copy_bs = o_pad * k_pad;
     int64_t cursor = 0;
     layout->positions = place(cursor, layout->sort_batches * layout->positions_bs * 2);
     layout->counts = place(cursor, layout->sort_batches * layout->counts_bs * 2);
     layout->a_copy = place(cursor, layout->a_batches * layout->a_copy_bs * 4);
     layout->a_magnitudes = place(cursor, layout->a_batches * layout->a_magnitudes_bs * 4);
-    layout->c_pieces = place(cursor, layout->c_batches * layout->c_pieces_bs * 16);
-    layout->c_unscale = place(cursor, layout->c_batches * o_pad * 4);
+    layout->products = place(cursor, layout->product_batches * layout->products_bs * 2);
+    layout->c_copy = place(cursor, layout->c_batches * layout->c_copy_bs * 4);
+    layout->c_exponents = place(cursor, layout->c_batches * o_pad * 4);
     layout->bytes = cursor;
     return true;
 }
@@ -180,14 +188,16 @@ hipError_t launch_norm_gradient_f16(const kmc_norm_gradient_params *p, bool a_ve
     prepare.counts = reinterpret_cast<unsigned short *>(workspace + layout.counts); prepare.counts_bs = layout.counts_bs;
     prepare.a_copy = reinterpret_cast<float *>(workspace + layout.a_copy); prepare.a_copy_bs = layout.a_copy_bs;
     prepare.a_magnitudes = reinterpret_cast<float *>(workspace + layout.a_magnitudes); prepare.a_magnitudes_bs = layout.a_magnitudes_bs;
-    prepare.c_pieces = reinterpret_cast<kmc::gram_chunk *>(workspace + layout.c_pieces); prepare.c_pieces_bs = layout.c_pieces_bs;
-    prepare.c_unscale = reinterpret_cast<float *>(workspace + layout.c_unscale); prepare.c_unscale_bs = layout.o_pad;
+    prepare.products = reinterpret_cast<unsigned short *>(workspace + layout.products); prepare.products_bs = layout.products_bs;
+    prepare.c_copy = reinterpret_cast<float *>(workspace + layout.c_copy); prepare.c_copy_bs = layout.c_copy_bs;
+    prepare.c_exponents = reinterpret_cast<int *>(workspace + layout.c_exponents); prepare.c_exponents_bs = layout.o_pad;
     prepare.n_pad = layout.n_pad; prepare.m_pad = layout.m_pad; prepare.k_pad = layout.k_pad; prepare.o_pad = layout.o_pad;
     prepare.sort_d = layout.sort_d;
-    prepare.ranges = layout.ranges; prepare.chunks = layout.chunks; prepare.chunk_k = layout.chunk_k;
+    prepare.copy_k = layout.copy_k; prepare.ranges = layout.ranges; prepare.chunk_k = layout.chunk_k;
     prepare.sort_blocks = p->n * layout.chunks;
-    prepare.copy_blocks = layout.m_pad / kmc::NGF_COPY_M * layout.ranges;
+    prepare.copy_blocks = layout.copy_blocks;
     prepare.sort_batches = layout.sort_batches; prepare.a_batches = layout.a_batches; prepare.c_batches = layout.c_batches;
+    prepare.product_batches = layout.product_batches;
     const int batches = layout.sort_batches > 1 || layout.a_batches > 1 || layout.c_batches > 1 ? p->l : 1;
     prepare.sort_groups = (prepare.sort_blocks + kmc::NGF_PREPARE_GROUP - 1) / kmc::NGF_PREPARE_GROUP;
     prepare.copy_groups = (prepare.copy_blocks + kmc::NGF_PREPARE_GROUP - 1) / kmc::NGF_PREPARE_GROUP;
@@ -210,10 +220,11 @@ hipError_t launch_norm_gradient_f16(const kmc_norm_gradient_params *p, bool a_ve
     args.counts_bs = layout.sort_batches > 1 ? layout.counts_bs : 0;
     args.a_copy = prepare.a_copy; args.a_copy_bs = layout.a_batches > 1 ? layout.a_copy_bs : 0;
     args.a_magnitudes = prepare.a_magnitudes; args.a_magnitudes_bs = layout.a_batches > 1 ? layout.a_magnitudes_bs : 0;
-    args.c_pieces = prepare.c_pieces; args.c_pieces_bs = layout.c_batches > 1 ? layout.c_pieces_bs : 0;
-    args.c_unscale = prepare.c_unscale; args.c_unscale_bs = layout.c_batches > 1 ? layout.o_pad : 0;
-    args.n_pad = layout.n_pad; args.m_pad = layout.m_pad; args.k_pad = layout.k_pad; args.ranges = layout.ranges;
-    args.chunks = layout.chunks; args.chunk_stages = layout.chunk_k / kmc::NGF_STAGE_K; args.stages = layout.stages;
+    args.products = prepare.products; args.products_bs = layout.product_batches > 1 ? layout.products_bs : 0;
+    args.c_copy = prepare.c_copy; args.c_copy_bs = layout.c_batches > 1 ? layout.c_copy_bs : 0;
+    args.c_exponents = prepare.c_exponents; args.c_exponents_bs = layout.c_batches > 1 ? layout.o_pad : 0;
+    args.n_pad = layout.n_pad; args.m_pad = layout.m_pad; args.k_pad = layout.k_pad; args.o_pad = layout.o_pad; args.ranges = layout.ranges;
+    args.chunk_stages = layout.chunk_k / kmc::NGF_STAGE_K; args.stages = layout.stages;
     // blocks of 16 outputs; what is left up to 8 in the first half of the columns, its second pieces in the other
     const int left = p->o % kmc::NGF_TILE_O;
     const int in_columns = left > 0 && left <= 8 ? 1 : 0;

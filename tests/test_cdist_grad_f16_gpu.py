@@ -181,3 +181,57 @@ def test_signs_are_exact_in_tiles_of_192(device, f16_route, M, N, O, K):
     zeros = [torch.zeros(rows, columns, device=device) for rows, columns in ((K, M), (N, K), (O, K), (N, M))]
     assert any("norm_gradient_l1_f16<12," in name for name in kernels_of(lambda: kermac.cdist_grad(*zeros, p=1.0)))
     test_signs_are_exact(device, f16_route, M, N, O, K)
+
+
+def _beside_large_values(kind, M, O, K, g):
+    """a [K, M] and c [O, K] whose products are all small beside max |a| max |c|."""
+    signs = torch.randint(0, 2, (O, K), generator=g).float() * 2 - 1
+    a, c = torch.rand(K, M, generator=g) + 0.5, signs * (torch.rand(O, K, generator=g) + 0.5)
+    at_a, at_c = torch.randint(K // 2, (M,), generator=g), K // 2 + torch.randint(K - K // 2, (O,), generator=g)
+    if kind == "one c of 2^16 that meets a = 0":
+        c[:, K - 1] = 2.0 ** 16
+        a[K - 1] = 0.0
+    elif kind == "one a of 1 that meets c = 0, the others 2^-16":
+        a *= 2.0 ** -16
+        a[3], c[:, 3] = 1.0, 0.0
+    elif kind == "a Laplace kernel: 1 that meets c = 0, beside exp(-20 +- 3)":
+        a = torch.exp(-20 + 3 * torch.randn(K, M, generator=g))
+        a[K // 3], c[:, K // 3] = 1.0, 0.0
+    elif kind == "one of 1 in each, apart, the others 2^-14":
+        a, c = a * 2.0 ** -14, c * 2.0 ** -14
+        a[at_a, torch.arange(M)] = 1.0
+        c[torch.arange(O), at_c] = -1.0
+        c[:, :K // 2] *= (torch.zeros(K // 2).index_fill_(0, at_a, 1.0) == 0).float()       # ... so that a product with one of them is 0
+        a[K // 2:] *= (torch.zeros(K - K // 2).index_fill_(0, at_c - K // 2, 1.0) == 0).float()[:, None]
+    elif kind == "neighbours of 1 in each that meet 0, the others 2^-30":
+        a, c = a * 2.0 ** -30, c * 2.0 ** -30
+        a[8], a[9], c[:, 8], c[:, 9] = 1.0, 0.0, 0.0, 1.0
+    elif kind == "outputs that see different rows of a":
+        a *= torch.pow(2.0, -40.0 * torch.rand(K, generator=g))[:, None]
+        c *= (torch.arange(K)[None] % O == torch.arange(O)[:, None]).float()
+    return a, c
+
+
+@pytest.mark.parametrize("kind", ["one c of 2^16 that meets a = 0", "one a of 1 that meets c = 0, the others 2^-16",
+                                  "a Laplace kernel: 1 that meets c = 0, beside exp(-20 +- 3)", "one of 1 in each, apart, the others 2^-14",
+                                  "neighbours of 1 in each that meet 0, the others 2^-30", "outputs that see different rows of a"])
+@pytest.mark.parametrize("M,N,O,K", [(70, 40, 16, 64), (130, 300, 5, 100), (40, 70, 20, 130), (4000, 150, 9, 40), (33, 40, 40, 600)])
+@pytest.mark.parametrize("powers", [(0, 0), (100, -60), (-60, 100)])
+def test_small_products_beside_large_values(device, f16_route, kind, M, N, O, K, powers):
+    """The error of every element is bounded by its own sum of |c a|, however small that is beside max |a| max |c|: 3 * 2^-22 of it
+    from the pieces, and 2^-24 for each of two roundings in two matrix instructions per 32 k and for the last roundings, doubled
+    with the result."""
+    g = torch.Generator().manual_seed(M + N + O + K)
+    a, c = _beside_large_values(kind, M, O, K, g)
+    a, c = (a * 2.0 ** powers[0]).to(device), (c * 2.0 ** powers[1]).to(device)
+    b, d = torch.randn(N, K, generator=g).to(device), torch.randn(N, M, generator=g).to(device)
+    assert workspace_bytes(a, b, c, d) > 0
+    got = kermac.cdist_grad(a, b, c, d, p=1.0)[0].double()
+    bound = (3 * 2.0 ** -22 + (4 * -(-K // 32) + 4) * 2.0 ** -23) * (c.double().abs() @ a.double().abs())       # [O, M]
+    worst = 0.0
+    for n in range(0, N, 3):
+        sign = torch.copysign(torch.ones((), device=device), d[n][None, :] - b[n][:, None])
+        error = (got[:, n] - c.double() @ (sign.double() * a.double())).abs()
+        assert torch.isfinite(error).all()
+        worst = max(worst, float((error / bound.clamp_min(1e-300)).max()))
+    assert worst <= 1.0, f"{worst:.3g} times the bound"
