@@ -133,6 +133,16 @@ def allocate(nbytes: int, device: torch.device) -> Optional[torch.Tensor]:
     return taken
 
 
+def mark() -> int:
+    """What this operator call has taken so far, for `give_back_to`."""
+    return _state()["used"]
+
+
+def give_back_to(taken: int) -> None:
+    """What was taken since `mark()` returned `taken` counts no more: the caller has dropped it, with nothing launched on it."""
+    _state()["used"] = taken
+
+
 def allocate_floats(shape, device: torch.device) -> Optional[torch.Tensor]:
     """A contiguous fp32 tensor of ``shape`` from ``allocate``."""
     count = 1

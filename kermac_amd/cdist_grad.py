@@ -158,16 +158,24 @@ def cdist_grad(
         ValueError: bad shapes, strides, batch sizes or devices.
     """
     plan = _plan_cdist_grad(a, b, c, d, out, p)
-    split = _split_over_contraction(plan) if _may_split else None
-    if split is not None and _run_split_over_contraction(split, plan, a, b, c, d, p, debug):
-        return plan.out
-    stream = _current_stream_for(a.device)
+    if _may_split:
+        for cut in _cuts_over_contraction(plan):
+            if _run_cut(cut, plan, a, b, c, d, p, debug):
+                return plan.out
+    _launch(plan, a.device, debug)
+    return plan.out
+
+
+def _launch(plan, device, debug, needs_workspace=False):
+    """Launches the call as it is; with `needs_workspace` only if it gets the workspace that the library wants for it."""
+    workspace = _attach_workspace(plan.params, device)
+    if needs_workspace and workspace is None:
+        return False
     if debug:
         print(f"(Kermac Debug) Launching kernel: norm_kernel_gradient<{('L1', 'L2', 'P')[plan.params.norm_type]}>")
-    workspace = _attach_workspace(plan.params, a.device)
-    _backend.norm_kernel_gradient(plan.params, stream)
+    _backend.norm_kernel_gradient(plan.params, _current_stream_for(device))
     del workspace           # the launches are queued: the allocator hands the memory on in stream order
-    return plan.out
+    return True
 
 
 def _workspace_enabled():
@@ -175,10 +183,9 @@ def _workspace_enabled():
 
 
 def _attach_workspace(params, device):
-    """Large L1 and L2 gradients run on the fp16 matrix instruction through a workspace (include/
-    kermac_amd.h, kmc_norm_gradient_params::workspace.  L1: a and c split once into two fp16 pieces
-    per value, the sign of d - b put on the pieces of a.  L2: the sum factors into
-    (d - s) (c a) - (c (b - s)) a, one product of pieces); the library says how much it wants for
+    """Large L1 and L2 gradients run on the fp16 matrix instruction through a workspace (include/kermac_amd.h,
+    kmc_norm_gradient_params::workspace.  L1: rows of b and d ranked, d >= b as an exact 0 or 1 times a c in two fp16 pieces.
+    L2: the sum factors into (d - s) (c a) - (c (b - s)) a, one product of pieces); the library says how much it wants for
     this call, 0 when it would not use one.  KERMAC_AMD_GRADIENT_WORKSPACE=0 keeps every call on
     the fp32 kernels."""
     if not _workspace_enabled():
@@ -207,46 +214,80 @@ _SPLIT_TARGET_WORKGROUPS = 3072
 _SPLIT_MIN_DEPTH = 512                      # from 512 workgroups on: 1024, and 2048 for the matrix-core kernels
 _SPLIT_MAX_SLICES = 24
 _SPLIT_MAX_PARTIAL_BYTES = 512 << 20
-# Calls that go to the fp16 matrix instruction (p = 1, a workspace granted): its workgroups own 16 (m) x 128 (n) x 16 (o)
+# Calls that go to the fp16 matrix instruction (p = 1, the workspace granted): its workgroups own 16 (m) x 128 (n) x 16 (o)
 # results or more, one per CU at a time, and every slice ranks its rows again, so fewer slices are wanted: 2000 x 24 x 16 x 9000 in
 # 17 slices 166 us, in 5 147; 200 x 1000 x 16 x 12000 in 12 472, in 5 401.
 _SPLIT_F16_TARGET_WORKGROUPS = 512
 
 
-def _takes_f16_route(params):
-    return params.norm_type == _NORM_L1 and _workspace_enabled() and _backend.norm_gradient_workspace_bytes(params) > 0
+def _takes_f16_route(params, slices=1, depth=None):
+    """Whether the library wants a workspace for this L1 gradient, or for `slices` of `depth` k each as a batch of one launch."""
+    if params.norm_type != _NORM_L1 or not _workspace_enabled():
+        return False
+    if slices > 1:
+        params = type(params).from_buffer_copy(params)
+        params.k, params.l = depth, slices
+        params.a_bs, params.b_bs, params.c_bs, params.d_bs = depth * params.a_ld, depth, depth, 0
+    return _backend.norm_gradient_workspace_bytes(params) > 0
 
 
-def _split_over_contraction(plan):
-    """(slices, k per slice, leftover k), or None when the call is launched as it is."""
+def _cuts_over_contraction(plan):
+    """How the call is cut over k: (slices, k per slice, leftover k, whether only with a workspace), the best first.  Behind the cuts for the fp16
+    matrix instruction stands the one for the fp32 kernels, which run where the workspace is refused; the last resort is the call as it is."""
     if plan.L != 1 or plan.M == 0 or plan.N == 0 or plan.O == 0 or not launch_cuts_enabled():
-        return None
+        return
     M, N, O, K = plan.M, plan.N, plan.O, plan.K
     n_tile = 32 if O <= 8 else 16
     workgroups = -(-M // 64) * -(-N // n_tile) * max(1, -(-O // 32))
     min_depth = _SPLIT_MIN_DEPTH * (1 if workgroups < 512 else 2 if O <= 8 else 4)
     if workgroups >= _SPLIT_BELOW_WORKGROUPS or K < 2 * min_depth:
-        return None
-    wanted = max(2, round(_SPLIT_TARGET_WORKGROUPS / workgroups))
+        return
+    most = min(K // min_depth, _SPLIT_MAX_SLICES, _SPLIT_MAX_PARTIAL_BYTES // (4 * O * N * M) - 1)
+
+    def cut(wanted):
+        depth = K // min(wanted, most) // 64 * 64       # whole K slices of the kernels; 16-byte alignment survives
+        slices = K // depth
+        return slices, depth, K - slices * depth
+
     if _takes_f16_route(plan.params):
         f16_workgroups = -(-M // 16) * -(-N // 128) * -(-O // 16)
         wanted = -(-_SPLIT_F16_TARGET_WORKGROUPS // f16_workgroups)
+        filled = wanted
         # a workgroup has its CU to itself: up to twice as many slices where their last round of 256 would be nearly empty
         # (1408 x 128 x 32 x 9522, 176 workgroups: 3 slices 424 us, 4 slices 354)
         if wanted > 1:
-            filled = [n * f16_workgroups / (256 * -(-n * f16_workgroups // 256)) for n in range(wanted, 2 * wanted + 1)]
-            wanted += next((extra for extra, part in enumerate(filled) if part >= 0.85), filled.index(max(filled)))
-    slices = min(wanted, K // min_depth, _SPLIT_MAX_SLICES,
-                 _SPLIT_MAX_PARTIAL_BYTES // (4 * O * N * M) - 1)
-    if slices < 2:
-        return None
-    depth = K // slices // 64 * 64       # whole K slices of the kernels; 16-byte alignment survives
-    slices = K // depth
-    return slices, depth, K - slices * depth
+            parts = [n * f16_workgroups / (256 * -(-n * f16_workgroups // 256)) for n in range(wanted, 2 * wanted + 1)]
+            filled += next((extra for extra, part in enumerate(parts) if part >= 0.85), parts.index(max(parts)))
+        # more slices take more memory: where that is refused, the fewer ones
+        for slices in dict.fromkeys((filled, wanted)):
+            if min(slices, most) < 2:
+                yield 1, K, 0, True
+            elif _takes_f16_route(plan.params, *cut(slices)[:2]):
+                yield (*cut(slices), True)
+    if most >= 2:
+        yield (*cut(max(2, round(_SPLIT_TARGET_WORKGROUPS / workgroups))), False)
 
 
-def _run_split_over_contraction(split, plan, a, b, c, d, p, debug):
-    slices, depth, leftover = split
+def _split_over_contraction(plan):
+    """(slices, k per slice, leftover k), or None when the call is launched as it is, if all the memory it asks for is granted."""
+    best = next(_cuts_over_contraction(plan), None)
+    return best[:3] if best is not None and best[0] > 1 else None
+
+
+def _run_cut(cut, plan, a, b, c, d, p, debug):
+    """Launches the call in slices, or returns False with nothing launched: no memory for the partial results, or for the workspace of a
+    cut that is none without."""
+    slices, depth, leftover, needs_workspace = cut
+    if slices == 1:
+        return _launch(plan, a.device, debug, needs_workspace)
+    taken = _scratch.mark()
+    if _run_slices(slices, depth, leftover, needs_workspace, plan, a, b, c, d, p, debug):
+        return True
+    _scratch.give_back_to(taken)
+    return False
+
+
+def _run_slices(slices, depth, leftover, needs_workspace, plan, a, b, c, d, p, debug):
     a2, b2, c2, d2 = (t[0] if t.dim() == 3 else t for t in (a, b, c, d))
     M, N, O = plan.M, plan.N, plan.O
     partial = _scratch.allocate_floats((slices + (1 if leftover else 0), O, N, M), a.device)
@@ -255,14 +296,15 @@ def _run_split_over_contraction(split, plan, a, b, c, d, p, debug):
     # bits of a contiguous one, through a buffer of its own
     staged = None if target.is_contiguous() or partial is None else _scratch.allocate_floats((O, N, M), a.device)
     if partial is None or (staged is None and not target.is_contiguous()):
-        return False            # no memory for the partial results: the call goes out as it is
+        return False
     a_slices = a2.as_strided((slices, depth, M), (depth * a2.stride(0), a2.stride(0), a2.stride(1)), a2.storage_offset())
     b_slices = b2.as_strided((slices, N, depth), (depth * b2.stride(1), b2.stride(0), b2.stride(1)), b2.storage_offset())
     c_slices = c2.as_strided((slices, O, depth), (depth * c2.stride(1), c2.stride(0), c2.stride(1)), c2.storage_offset())
-    cdist_grad(a_slices, b_slices, c_slices, d2, out=partial[:slices], p=p, debug=debug, _may_split=False)
+    if not _launch(_plan_cdist_grad(a_slices, b_slices, c_slices, d2, partial[:slices], p), a.device, debug, needs_workspace):
+        return False
     if leftover:
         done = slices * depth
-        cdist_grad(a2[done:], b2[:, done:], c2[:, done:], d2, out=partial[slices:], p=p, debug=debug, _may_split=False)
+        _launch(_plan_cdist_grad(a2[done:], b2[:, done:], c2[:, done:], d2, partial[slices:], p), a.device, debug)
     if staged is None:
         torch.sum(partial, dim=0, out=target)
     else:

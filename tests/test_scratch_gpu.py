@@ -3,11 +3,17 @@ at 0 a call allocates nothing -- the reference's contract (README.md:69,135: "as
 -- and inside `kermac.scratch(buffer)` it takes its buffers from the caller's memory and allocates nothing either.
 Allocations are counted by torch's allocator statistics around the call.
 """
+import contextlib
+import importlib
+
 import pytest
 import torch
 
 import kermac_amd as kermac
-from tests.helpers import assert_close_to_truth, l1_distances_float64
+from kermac_amd import _backend
+from tests.helpers import assert_close_to_truth, kernels_of, l1_distances_float64
+
+grad_module = importlib.import_module("kermac_amd.cdist_grad")      # the package attribute of that name is the operator
 
 pytestmark = pytest.mark.gpu
 
@@ -111,3 +117,60 @@ def test_fixed_point_route_and_cut_launches_respect_the_limit(device):
             assert count == 0
     finally:
         kermac.set_max_scratch_bytes(None)
+
+
+def _gradient(device, M, N, O, K):
+    g = torch.Generator(device=device).manual_seed(M + N)
+    a, b, c, d = (torch.randn(rows, columns, device=device, generator=g) for rows, columns in ((K, M), (N, K), (O, K), (N, M)))
+    return lambda: kermac.cdist_grad(a, b, c, d, p=1.0), grad_module._plan_cdist_grad(a, b, c, d, None, 1.0)
+
+
+def _bytes_of(plan, cut):
+    """Partial results and workspace of a call that is cut over k, each at a multiple of 256 bytes as in a supplied buffer."""
+    slices, depth, leftover, needs_workspace = cut
+    partial = -(-4 * (slices + (leftover > 0)) * plan.O * plan.N * plan.M // 256) * 256
+    params = type(plan.params).from_buffer_copy(plan.params)
+    params.k, params.l, params.d_bs = depth, slices, 0
+    params.a_bs, params.b_bs, params.c_bs = depth * params.a_ld, depth, depth
+    return partial + (_backend.norm_gradient_workspace_bytes(params) if needs_workspace else 0)
+
+
+@contextlib.contextmanager
+def _at_most(nbytes, how, device):
+    if how == "buffer":
+        with kermac.scratch(torch.empty(nbytes, dtype=torch.uint8, device=device)):
+            yield
+    else:
+        kermac.set_max_scratch_bytes(nbytes)
+        try:
+            yield
+        finally:
+            kermac.set_max_scratch_bytes(None)
+
+
+# f16 slices wanted: several, fewer than the fp32 kernels, none
+@pytest.mark.parametrize("M,N,O,K", [(2000, 24, 16, 9000), (4000, 100, 16, 10000), (8192, 128, 16, 8192)])
+@pytest.mark.parametrize("how", ["limit", "buffer"])
+def test_l1_gradient_without_its_workspace_is_cut_for_the_kernels_that_run(device, monkeypatch, how, M, N, O, K):
+    """A limit that holds the partial results of the fp32 kernels' slices, but not the workspace of the fp16 route: the bits of a
+    process without that route."""
+    call, plan = _gradient(device, M, N, O, K)
+    *on_f16, on_fp32 = grad_module._cuts_over_contraction(plan)
+    assert on_f16 and all(cut[3] for cut in on_f16) and not on_fp32[3]
+    enough = _bytes_of(plan, on_fp32)
+    assert all(_bytes_of(plan, cut) > enough + 4096 for cut in on_f16 if cut[0] > 1)
+    with _at_most(enough + 4096, how, device):
+        if on_f16[0][0] == 1:
+            assert _backend.norm_gradient_workspace_bytes(plan.params) > enough + 4096
+        got = call()
+    monkeypatch.setenv("KERMAC_AMD_GRADIENT_WORKSPACE", "0")
+    assert torch.equal(got, call())
+
+
+@pytest.mark.parametrize("how", ["limit", "buffer"])
+def test_l1_gradient_takes_fewer_slices_where_more_do_not_fit(device, how):
+    call, plan = _gradient(device, 1408, 128, 32, 9522)
+    more, fewer, _ = grad_module._cuts_over_contraction(plan)
+    assert more[0] > fewer[0] > 1 and _bytes_of(plan, more) > _bytes_of(plan, fewer) + 4096
+    with _at_most(_bytes_of(plan, fewer) + 4096, how, device):
+        assert any("norm_gradient_l1_f16" in name for name in kernels_of(call))
