@@ -81,9 +81,12 @@ __global__ __launch_bounds__(BK_THREADS) void build_kernel_short(const BuildKern
     float *const c_batch = args.c + batch * args.c_bs;
     // floats between the start of a line and C(0, n)
     const int shift = (int)((reinterpret_cast<unsigned long long>(c_batch) / 4 + (unsigned long long)n_first * (unsigned long long)args.c_ld) % BKT_LINE);
-    const int m0 = (int)blockIdx.x * BKT_TILE_M - shift;
-    const int m_first = m0 + 4 * lane;
-    if (m0 >= args.m) return;
+    // Rows are added up without a sign, and compared with differences of M: for M near 2^31 those beyond it are negative, not small.
+    if ((i64)blockIdx.x * BKT_TILE_M - shift >= args.m) return;
+    const int m0 = (int)(blockIdx.x * BKT_TILE_M - (unsigned)shift);
+    auto row_at = [m0](int at) { return (int)((unsigned)m0 + (unsigned)at); };
+    const int m_first = row_at(4 * lane);
+    const bool whole_quad = m_first >= 0 && m_first <= args.m - 4;
 
     const float *b = args.b + batch * args.b_bs;
     const bool b_rows = load_b == LOAD_ROW_VEC || load_b == LOAD_ROW_SCALAR;
@@ -104,7 +107,7 @@ __global__ __launch_bounds__(BK_THREADS) void build_kernel_short(const BuildKern
             float v[LOADS];
 #pragma unroll
             for (int j = 0; j < LOADS; j++) {
-                const int m = m0 + j * ROWS + row;
+                const int m = row_at(j * ROWS + row);
                 v[j] = m >= 0 && m < args.m && k0 + kk < args.k ? from[(i64)m * args.a_ld + k0 + kk] : 0.0f;
             }
             __syncthreads();
@@ -117,7 +120,7 @@ __global__ __launch_bounds__(BK_THREADS) void build_kernel_short(const BuildKern
                 a[k0 + j][0] = x.x; a[k0 + j][1] = x.y; a[k0 + j][2] = x.z; a[k0 + j][3] = x.w;
             }
         }
-    } else if (load_a == LOAD_COL_VEC && shift % 4 == 0 && m_first >= 0 && m_first + 3 < args.m) {
+    } else if (load_a == LOAD_COL_VEC && shift % 4 == 0 && whole_quad) {
 #pragma unroll
         for (int k = 0; k < DEPTH; k++) {
             const float4 v = k < args.k ? *reinterpret_cast<const float4 *>(from + (i64)k * args.a_ld + m_first) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -128,7 +131,7 @@ __global__ __launch_bounds__(BK_THREADS) void build_kernel_short(const BuildKern
         for (int k = 0; k < DEPTH; k++)
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                const int m = m_first + i;
+                const int m = row_at(4 * lane + i);
                 a[k][i] = m >= 0 && m < args.m && k < args.k ? from[(i64)k * args.a_ld + m] : 0.0f;
             }
     }
@@ -143,7 +146,7 @@ __global__ __launch_bounds__(BK_THREADS) void build_kernel_short(const BuildKern
     const float diff_sign = args.diff_sign, epsilon = args.epsilon;
     __syncthreads();
 
-    const bool whole = m0 >= 0 && m0 + BKT_TILE_M <= args.m;
+    const bool whole = m0 >= 0 && m0 <= args.m - BKT_TILE_M;
     for (int round = 0; round < rounds; round++) {
         // this wave's columns j: the waves side by side
         const int j_first = round * BKT_COLUMNS + wave;
@@ -189,15 +192,15 @@ __global__ __launch_bounds__(BK_THREADS) void build_kernel_short(const BuildKern
             if (regularize) {
 #pragma unroll
                 for (int i = 0; i < 4; i++)
-                    if (args.reg_off_x + m_first + i == args.reg_off_y + (int)n) acc[c][i] = 1.0f + regularization;
+                    if ((unsigned)args.reg_off_x + (unsigned)m_first + i == (unsigned)args.reg_off_y + (unsigned)n) acc[c][i] = 1.0f + regularization;
             }
             float *to = c_batch + n * args.c_ld + m_first;
-            if (whole || (m_first >= 0 && m_first + 3 < args.m)) {
+            if (whole || whole_quad) {
                 *reinterpret_cast<float4 *>(to) = make_float4(acc[c][0], acc[c][1], acc[c][2], acc[c][3]);
             } else {
 #pragma unroll
                 for (int i = 0; i < 4; i++)
-                    if (m_first + i >= 0 && m_first + i < args.m) to[i] = acc[c][i];
+                    if (row_at(4 * lane + i) >= 0 && row_at(4 * lane + i) < args.m) to[i] = acc[c][i];
             }
         }
     }

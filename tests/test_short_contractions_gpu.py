@@ -89,3 +89,19 @@ def test_a_set_against_itself(device, monkeypatch):
     x = torch.randn(3, 400, 6, generator=g).to(device)
     short, ordinary = both(monkeypatch, lambda: kermac.run_kernel(DESCRIPTORS["gaussian"], x, x, bandwidth=2.0, regularization=1e-3))
     assert torch.equal(short, ordinary) and torch.equal(short, short.transpose(1, 2))
+
+
+@pytest.mark.parametrize("M", [2 ** 31 - 1, 2 ** 31 - 1 - 200])
+@pytest.mark.parametrize("k_contiguous", [False, True])
+def test_a_result_of_nearly_2_to_the_31_rows(device, monkeypatch, M, k_contiguous):
+    """The last tiles' row numbers, which end at M, do not fit 32 bits once a tile is added.  K = 2 with k contiguous would be 16 GB: K = 1 there."""
+    monkeypatch.setenv("KERMAC_AMD_DIRECT_SHORT_MAX_K", "24")
+    x = torch.empty(M, 1, device=device) if k_contiguous else torch.empty(1, M, device=device).t()
+    x.copy_(torch.arange(M, dtype=torch.int32, device=device)[:, None] % 4093)
+    point = torch.full((1, 1), 17.0, device=device)
+    guard = torch.full((M + 64,), -5.0, device=device)
+    out = guard[33:33 + M].as_strided((M, 1), (1, M))
+    kermac.cdist(x, point, out=out, p=1.0)
+    assert bool((guard[:33] == -5.0).all()) and bool((guard[33 + M:] == -5.0).all())
+    x.sub_(17.0).abs_()
+    assert torch.equal(out, x)
