@@ -359,7 +359,7 @@ typedef struct kmc_norm_gradient_params {
  * of kmc_dispatch_rules(); 4e8 terms at 16 outputs), and n within one grid dimension; about 1.1 times the
  * bytes of a, b and c.  KMC_NORM_L2:
  * when a model of both times favours the route by 15 % (tiles of 256 x 256 over m and o * n, in
- * both directions, and a contraction of about 512 or more); about 4 (m + 2 o n) k bytes.
+ * both directions, and a contraction of about 512 or more); about 4 (m + o n) k bytes.
  * KMC_NORM_P: never.  No counterpart in the reference. */
 int kmc_norm_gradient_workspace_bytes(const kmc_norm_gradient_params *params, int64_t *bytes);
 

@@ -484,9 +484,6 @@ bool gradient_l2_layout(const kmc_norm_gradient_params *p, GradientL2Layout *lay
     if (!gradient_l2_pays(p, wide.tiles_m, wide.tiles_n)) return false;
     if (!place_wide(p->m, static_cast<int>(rows), p->k, p->l, p->a_bs == 0, false, false, false, false, &wide)) return false;
     int64_t cursor = wide.bytes;
-    // Room for the products in fp32, which no kernel stores any more: the size that the query reports is part of what callers
-    // have measured and planned with (and which calls a limit of theirs keeps off the route), so it stays what it was.
-    place(cursor, static_cast<int64_t>(p->l) * rows * ((p->k + 3) / 4 * 4) * 4);
     layout->shift = place(cursor, static_cast<int64_t>(p->l) * p->n * 4);
     layout->c_transposed = place(cursor, static_cast<int64_t>(p->l) * p->k * p->o * 4);
     layout->g = place(cursor, static_cast<int64_t>(p->l) * p->m * p->o * 4);

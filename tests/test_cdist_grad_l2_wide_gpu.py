@@ -62,7 +62,7 @@ def test_when_the_route_applies(device):
     needed = workspace_bytes(a, b, c, d)                                     # 16 x 32 tiles over k = 2048
     assert needed > 0
     operands = 4 * (a.numel() + 16 * b.numel())                              # a, and c b for every output
-    assert 1.5 * operands <= needed <= 2 * operands                          # the products in fp32 and in pieces, the pieces of a
+    assert operands <= needed <= 1.1 * operands                              # pieces of a and of the products, 4 bytes a value; g and statistics
     assert workspace_bytes(a, b, c, d, p=1.3) == 0
     assert workspace_bytes(a[:256], b[:, :256], c[:, :256], d) == 0          # k = 256: the walk is too short
     assert workspace_bytes(a, b[:8], c, d[:8]) == 0                          # 16 x 1 tiles

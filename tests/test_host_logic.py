@@ -587,7 +587,7 @@ def test_workspace_queries_need_no_gpu(monkeypatch):
     assert gradient(8192, 512, 16, 8192, norm_type=2) == 0
     # the L2 norm: one product of (o n) x k by k x m on the fp16 matrix instruction, by a model of both times
     monkeypatch.delenv("KERMAC_AMD_GRADIENT_L2_MIN_TERMS", raising=False)
-    assert gradient(8192, 512, 16, 8192, norm_type=1) > 3 * 4 * 8192 * 8192          # c b in fp32 and in pieces, the pieces of a
+    assert 2 * 4 * 8192 * 8192 < gradient(8192, 512, 16, 8192, norm_type=1) < 2.2 * 4 * 8192 * 8192     # the pieces of c b and of a
     assert gradient(8192, 512, 16, 256, norm_type=1) == 0                            # a short contraction
     assert gradient(8192, 8, 16, 8192, norm_type=1) == 0                             # 32 x 1 tiles
     assert gradient(512, 512, 16, 8192, norm_type=1) == 0                            # 2 x 32 tiles

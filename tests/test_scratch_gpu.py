@@ -174,3 +174,12 @@ def test_l1_gradient_takes_fewer_slices_where_more_do_not_fit(device, how):
     assert more[0] > fewer[0] > 1 and _bytes_of(plan, more) > _bytes_of(plan, fewer) + 4096
     with _at_most(_bytes_of(plan, fewer) + 4096, how, device):
         assert any("norm_gradient_l1_f16" in name for name in kernels_of(call))
+
+
+@pytest.mark.parametrize("how", ["limit", "buffer"])
+def test_l2_gradient_asks_for_its_pieces_and_no_more(device, how):
+    """Two fp16 pieces per value of a and of the products c (b - s), 4 bytes, are what the route cannot do without: a tenth more holds it."""
+    M, N, O, K = 4096, 512, 16, 2048
+    a, b, c, d = (torch.randn(rows, columns, device=device) for rows, columns in ((K, M), (N, K), (O, K), (N, M)))
+    with _at_most(int(1.1 * 4 * (M + O * N) * K), how, device):
+        assert any("gram_f16_wide" in name for name in kernels_of(lambda: kermac.cdist_grad(a, b, c, d, p=2.0)))
