@@ -112,22 +112,26 @@ bool gradient_layout(const kmc_norm_gradient_params *p, GradientLayout *layout)
     return true;
 }
 
-// Tile of the product in n: 16, 12, 8, 4 or 2 blocks of 16.  A wave takes about 84 cycles for the two matrix instructions, the
-// comparisons and the reads of a block and m, and 230 for W and the rest of a step (1580 cycles at 16 blocks, measured at
-// 8192 x 512 x 16 x 8192), so wide tiles are cheaper per result, unless they are too few for the 256 CUs: one
-// workgroup per CU is what the count of rounds assumes.  12 is for n that fill little of the second half of a larger tile: with the others only / with
+// Tile of the product in n: 16, 12, 8, 4 or 2 blocks of 16, as blocks and us of two rounds of the 256 CUs at K = 8192, the second with the pieces in the
+// columns.  A step costs about as much as 8 blocks beside its blocks, W above all, so wide tiles are cheaper per result, unless they are too few for the
+// CUs or their last round is nearly empty.  Up to 4 blocks two workgroups share a CU and take as long as one behind the other, but need
+// no whole rounds; 8 % are taken off for what they hide of each other's ends (378, 431, 338 and 377 with the chip full; 2100 x 260 x 10 x 5000 in tiles
+// of 4 and 12 blocks 329 and 363 us, 1500 x 300 x 17 x 1500 138 and 146).
+// 12 is for n that fill little of the second half of a larger tile: with the others only / with
 // 12, us: 3000 x 147 x 64 x 4000 714 / 577, 2000 x 300 x 20 x 2000 301 / 212, 4000 x 147 x 32 x 4000 481 / 399.
-int blocks_for(const kmc_norm_gradient_params *p, int o_chunks)
+constexpr struct { int blocks, us, us_in_columns; } PRODUCT_TILES[] = {{16, 936, 743}, {12, 772, 642}, {8, 621, 536}, {4, 397, 347}, {2, 348, 311}};
+
+int blocks_for(const kmc_norm_gradient_params *p, int o_chunks, bool pieces_in_columns)
 {
-    int best = 16;
+    int best = 0;
     int64_t best_cost = INT64_MAX;
-    for (int blocks : {16, 12, 8, 4, 2}) {
+    for (const auto &tile : PRODUCT_TILES) {
+        const int tile_n = 16 * tile.blocks;
         // 12 where its last tile ends inside the padded rows
-        if (blocks == 12 && round_up(p->n, 16 * blocks) > round_up(p->n, kmc::NGF_N_PAD)) continue;
-        const int64_t tiles_n = (p->n + 16 * blocks - 1) / (16 * blocks), tiles_m = (p->m + kmc::NGF_TILE_M - 1) / kmc::NGF_TILE_M;
-        const int64_t rounds = (tiles_n * tiles_m * p->l * o_chunks + 255) / 256;
-        const int64_t cost = rounds * (84 * blocks + 230);
-        if (cost < best_cost) { best = blocks; best_cost = cost; }
+        if (tile.blocks == 12 && round_up(p->n, tile_n) > round_up(p->n, kmc::NGF_N_PAD)) continue;
+        const int64_t workgroups = static_cast<int64_t>((p->n + tile_n - 1) / tile_n) * ((p->m + kmc::NGF_TILE_M - 1) / kmc::NGF_TILE_M) * p->l * o_chunks;
+        const int64_t cost = (tile.blocks > 4 ? round_up(workgroups, 256) : workgroups > 256 ? workgroups : 256) * (pieces_in_columns ? tile.us_in_columns : tile.us);
+        if (cost < best_cost) { best = tile.blocks; best_cost = cost; }
     }
     return best;
 }
@@ -229,9 +233,9 @@ hipError_t launch_norm_gradient_f16(const kmc_norm_gradient_params *p, bool a_ve
     const int left = p->o % kmc::NGF_TILE_O;
     const int in_columns = left > 0 && left <= 8 ? 1 : 0;
     const int full_chunks = (p->o + kmc::NGF_TILE_O - 1) / kmc::NGF_TILE_O - in_columns;
-    const int blocks = blocks_for(p, full_chunks + in_columns);
-    if (full_chunks) status = launch_products<false>(blocks, args, 0, full_chunks, stream);
-    if (status == hipSuccess && in_columns) status = launch_products<true>(blocks, args, p->o - left, 1, stream);
+    // two launches, one behind the other: a tile for each
+    if (full_chunks) status = launch_products<false>(blocks_for(p, full_chunks, false), args, 0, full_chunks, stream);
+    if (status == hipSuccess && in_columns) status = launch_products<true>(blocks_for(p, 1, true), args, p->o - left, 1, stream);
     if (status == hipSuccess) *taken = true;
     return status;
 }

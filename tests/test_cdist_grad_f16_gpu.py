@@ -235,3 +235,14 @@ def test_small_products_beside_large_values(device, f16_route, kind, M, N, O, K,
         assert torch.isfinite(error).all()
         worst = max(worst, float((error / bound.clamp_min(1e-300)).max()))
     assert worst <= 1.0, f"{worst:.3g} times the bound"
+
+
+@pytest.mark.parametrize("M,N,O,tiles", [(2000, 700, 18, {"<12, false", "<12, true"}),      # two launches of 500 tiles of 192 n, two rounds each
+                                         (9000, 200, 20, {"<16, false", "<16, true"}),      # 563 of 256 n: three
+                                         (1500, 300, 17, {"<4, false", "<4, true"}),        # 470 of 64 n, two on a CU
+                                         (2000, 200, 37, {"<16, false", "<8, true"})])      # 250 of 256 n, one round; 250 of 128 n, one round
+def test_each_launch_of_a_call_has_its_own_tile(device, f16_route, M, N, O, tiles):
+    """The blocks of 16 outputs and the rest of up to 8 are launches one behind the other."""
+    zeros = [torch.zeros(rows, columns, device=device) for rows, columns in ((40, M), (N, 40), (O, 40), (N, M))]
+    names = kernels_of(lambda: kermac.cdist_grad(*zeros, p=1.0))
+    assert {tile for tile in tiles if any("norm_gradient_l1_f16" + tile in name for name in names)} == tiles, names
