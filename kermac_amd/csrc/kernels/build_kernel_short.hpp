@@ -86,7 +86,7 @@ __global__ __launch_bounds__(BK_THREADS) void build_kernel_short(const BuildKern
     const int m0 = (int)(blockIdx.x * BKT_TILE_M - (unsigned)shift);
     auto row_at = [m0](int at) { return (int)((unsigned)m0 + (unsigned)at); };
     const int m_first = row_at(4 * lane);
-    const bool whole_quad = m_first >= 0 && m_first <= args.m - 4;
+    const bool whole = m0 >= 0 && m0 <= args.m - BKT_TILE_M, whole_quad = m_first >= 0 && m_first <= args.m - 4;
 
     const float *b = args.b + batch * args.b_bs;
     const bool b_rows = load_b == LOAD_ROW_VEC || load_b == LOAD_ROW_SCALAR;
@@ -120,20 +120,33 @@ __global__ __launch_bounds__(BK_THREADS) void build_kernel_short(const BuildKern
                 a[k0 + j][0] = x.x; a[k0 + j][1] = x.y; a[k0 + j][2] = x.z; a[k0 + j][3] = x.w;
             }
         }
-    } else if (load_a == LOAD_COL_VEC && shift % 4 == 0 && whole_quad) {
+    } else if (load_a == LOAD_COL_VEC && shift % 4 == 0 && whole) {
 #pragma unroll
         for (int k = 0; k < DEPTH; k++) {
             const float4 v = k < args.k ? *reinterpret_cast<const float4 *>(from + (i64)k * args.a_ld + m_first) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             a[k][0] = v.x; a[k][1] = v.y; a[k][2] = v.z; a[k][3] = v.w;
         }
     } else {
+        // m contiguous, but not where a lane could load its 4 rows at once: 8 k of all rows at a time through LDS, lanes along m.  Loads of what does
+        // not exist go to the last row and k that do, and are dropped: with a branch for each they would be waited for one by one
+        const int m = row_at(tid);
+        const bool live = m >= 0 && m < args.m;
+        const float *column = from + min(max(m, 0), args.m - 1);
 #pragma unroll
-        for (int k = 0; k < DEPTH; k++)
+        for (int k0 = 0; k0 < DEPTH; k0 += BKT_CHUNK) {
+            float v[BKT_CHUNK];
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int m = row_at(4 * lane + i);
-                a[k][i] = m >= 0 && m < args.m && k < args.k ? from[(i64)k * args.a_ld + m] : 0.0f;
+            for (int j = 0; j < BKT_CHUNK && k0 + j < DEPTH; j++) v[j] = column[(i64)min(k0 + j, args.k - 1) * args.a_ld];
+            __syncthreads();
+#pragma unroll
+            for (int j = 0; j < BKT_CHUNK && k0 + j < DEPTH; j++) staged[j * BKT_PITCH + tid] = live && k0 + j < args.k ? v[j] : 0.0f;
+            __syncthreads();
+#pragma unroll
+            for (int j = 0; j < BKT_CHUNK && k0 + j < DEPTH; j++) {
+                const float4 x = *reinterpret_cast<const float4 *>(staged + j * BKT_PITCH + 4 * lane);
+                a[k0 + j][0] = x.x; a[k0 + j][1] = x.y; a[k0 + j][2] = x.z; a[k0 + j][3] = x.w;
             }
+        }
     }
     const int outer_power = args.outer_power, kernel_type = args.kernel_type;
     float p_outer = 0.0f, neg_gamma = 0.0f, regularization = 0.0f;
@@ -146,7 +159,6 @@ __global__ __launch_bounds__(BK_THREADS) void build_kernel_short(const BuildKern
     const float diff_sign = args.diff_sign, epsilon = args.epsilon;
     __syncthreads();
 
-    const bool whole = m0 >= 0 && m0 <= args.m - BKT_TILE_M;
     for (int round = 0; round < rounds; round++) {
         // this wave's columns j: the waves side by side
         const int j_first = round * BKT_COLUMNS + wave;
