@@ -163,7 +163,13 @@ static hipError_t launch_short(int load_a, int load_b, const kmc::BuildKernelArg
     // columns this many apart start at the same place in a line of 32 floats
     int classes = kmc::BKT_LINE;
     while (classes > 1 && args.c_ld % (2 * kmc::BKT_LINE / classes) == 0) classes /= 2;
-    const int64_t m_tiles = (static_cast<int64_t>(args.m) + kmc::BKT_LINE - 1 + kmc::BKT_TILE_M - 1) / kmc::BKT_TILE_M;
+    // floats between the start of a line and a column, at most
+    uint64_t shift = args.l > 1 && args.c_bs % kmc::BKT_LINE ? kmc::BKT_LINE - 1 : 0;
+    for (int column = 0; column < classes; column++) {
+        const uint64_t start = reinterpret_cast<uintptr_t>(args.c) / 4 + static_cast<uint64_t>(column) * static_cast<uint64_t>(args.c_ld);
+        shift = start % kmc::BKT_LINE > shift ? start % kmc::BKT_LINE : shift;
+    }
+    const int64_t m_tiles = (static_cast<int64_t>(args.m) + shift + kmc::BKT_TILE_M - 1) / kmc::BKT_TILE_M;
     // rounds of 16 columns per workgroup: as many as the loads of a are worth, as few as fill the chip
     int rounds = kmc::BKT_MAX_ROUNDS;
     while (rounds > 1 && m_tiles * (args.n / (rounds * kmc::BKT_COLUMNS) + 1) * args.l < 1024) rounds /= 2;

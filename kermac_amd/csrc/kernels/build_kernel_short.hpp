@@ -82,8 +82,11 @@ __global__ __launch_bounds__(BK_THREADS) void build_kernel_short(const BuildKern
     // floats between the start of a line and C(0, n)
     const int shift = (int)((reinterpret_cast<unsigned long long>(c_batch) / 4 + (unsigned long long)n_first * (unsigned long long)args.c_ld) % BKT_LINE);
     // Rows are added up without a sign, and compared with differences of M: for M near 2^31 those beyond it are negative, not small.
-    if ((i64)blockIdx.x * BKT_TILE_M - shift >= args.m) return;
-    const int m0 = (int)(blockIdx.x * BKT_TILE_M - (unsigned)shift);
+    // The last tile exists for some shifts only.  Tiles are dealt out in another order for every group of columns, or it would fall to
+    // the same of the 8 XCDs each time and leave them idle.
+    const unsigned m_tile = (blockIdx.x + blockIdx.y) % gridDim.x;
+    if ((i64)m_tile * BKT_TILE_M - shift >= args.m) return;
+    const int m0 = (int)(m_tile * BKT_TILE_M - (unsigned)shift);
     auto row_at = [m0](int at) { return (int)((unsigned)m0 + (unsigned)at); };
     const int m_first = row_at(4 * lane);
     const bool whole = m0 >= 0 && m0 <= args.m - BKT_TILE_M, whole_quad = m_first >= 0 && m_first <= args.m - 4;
