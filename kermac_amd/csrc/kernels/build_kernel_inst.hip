@@ -129,11 +129,36 @@ static bool small_applies(int load_a, int load_b, const kmc::BuildKernelArgs &ar
 // its rows per workgroup and a term at 3.5 cycles an instruction, where the ordinary kernel pays whole slices of 16 k.  Ordinary / this kernel,
 // us, p = 1, K = 6, 10, 16, 24: 10000 x 10000, rows 16-byte aligned 99 / 80, 103 / 92, 105 / 112, 153 / 150; 2 x 7000 x 7001, result not
 // aligned 182 / 84, 184 / 99, 160 / 117, 231 / 154; 5000 x 5000 35 / 24, 37 / 28, 37 / 32, 49 / 45; 3000 x 2500 16.8 / 13.9, 16.7 / 15.8, 16.2 / 17.8,
-// 21.6 / 24.4; 30000 rows against 300, whose loads of a
-// meet few columns, 17.6 / 14.8, 17.5 / 17.8, 17.7 / 19.8, 26.0 / 24.2 and with k contiguous 19.5 / 18.4, 19.6 / 23.0, 19.6 / 23.8, 27.6 / 33.9.  A set against
-// itself, computed in full here, 2 x 10000, K = 6 and 12, Laplace kernel 226 / 196 and 223 / 233.
+// 21.6 / 24.4.  A set against itself, computed in full here, 2 x 10000, K = 6 and 12, Laplace kernel 226 / 196 and 223 / 233.
+// Up to 8 terms no size of result was found that loses more than it varies (ordinary / this, K = 8, both operands k contiguous and both not): 30000
+// x 300 18.3 / 15.1 and 17.6 / 15.3, 30001 x 300 1.43 and 1.40 times, 30001 x 40 0.97 and 0.96, 100 x 60000 16.5 / 15.6 and 16.2 / 16.7, 16 x 500000 62 / 61 and 60 / 63,
+// 300 x 100 x 100 1.02 both, 64 x 300 x 300 1.03 and 0.98.  With more terms few rows lose what the tiles of 256 rows leave
+// unused of them, where the ordinary kernel stores 16 bytes at a time: K = 12, 100 x 60000 0.84 and 0.78, 300 x 30000 0.90 and 0.91, but 504 x 40000 1.10 and 1.05; K = 18
+// and 24, 504 x 40000 0.87 and 0.78, 756 x 26000 0.86 and 0.79, but 1012 x 20000 1.06 and 0.97.  `short_waste` is
+// that, and the limits are 5 / 4 and 8 / 7 (some sizes of few rows beyond them would gain: 320 x 40000 1.04 and, K = 18 and 24, 1.10 and 1.02).  Few
+// columns, which share a load of all k, gain little or nothing: 10000 x 300 at K = 12 and 24 1.02 and 0.96 .. 1.00, 30000 x 40 0.8 and 0.5.
 // KERMAC_AMD_DIRECT_SHORT_MAX_K=n replaces the rule by "at most n terms" (read on every call, so that a test can choose the kernel).
 constexpr bool HAS_SHORT = !HAS_ROOT_OR_POWER;
+
+// Columns this many apart start at the same place in a line of 32 floats
+static int short_classes(const kmc::BuildKernelArgs &args)
+{
+    int classes = kmc::BKT_LINE;
+    while (classes > 1 && args.c_ld % (2 * kmc::BKT_LINE / classes) == 0) classes /= 2;
+    return classes;
+}
+
+// Rows of this kernel's tiles per row of the ordinary kernel's, on average over where columns start in a line
+static double short_waste(const kmc::BuildKernelArgs &args)
+{
+    const int classes = short_classes(args);
+    int64_t tiles = 0;
+    for (int column = 0; column < classes; column++) {
+        const uint64_t start = reinterpret_cast<uintptr_t>(args.c) / 4 + static_cast<uint64_t>(column) * static_cast<uint64_t>(args.c_ld);
+        tiles += (static_cast<int64_t>(args.m) + static_cast<int64_t>(start % kmc::BKT_LINE) + kmc::BKT_TILE_M - 1) / kmc::BKT_TILE_M;
+    }
+    return static_cast<double>(tiles) * kmc::BKT_TILE_M / (static_cast<double>(classes) * args.tiles_m * kmc::BK_TILE_M);
+}
 
 static bool short_applies(int load_a, int load_b, const kmc::BuildKernelArgs &args)
 {
@@ -152,6 +177,7 @@ static bool short_applies(int load_a, int load_b, const kmc::BuildKernelArgs &ar
     if (args.k <= kmc_rules::DIRECT_SHORT_ANY_MAX_K) return true;
     if (args.symmetric) return false;
     if (args.n < kmc_rules::DIRECT_SHORT_MIN_COLUMNS) return false;
+    if (args.c_vec && short_waste(args) > (args.k <= kmc::BK_TILE_K ? 1.25 : 8.0 / 7)) return false;
     if (args.k <= 12) return true;
     if (args.k <= kmc::BK_TILE_K) return !args.c_vec;
     return tiles >= kmc_rules::DIRECT_SHORT_LONG_MIN_TILES;
@@ -160,9 +186,7 @@ static bool short_applies(int load_a, int load_b, const kmc::BuildKernelArgs &ar
 template <int DEPTH>
 static hipError_t launch_short(int load_a, int load_b, const kmc::BuildKernelArgs &args, hipStream_t stream)
 {
-    // columns this many apart start at the same place in a line of 32 floats
-    int classes = kmc::BKT_LINE;
-    while (classes > 1 && args.c_ld % (2 * kmc::BKT_LINE / classes) == 0) classes /= 2;
+    const int classes = short_classes(args);
     // floats between the start of a line and a column, at most
     uint64_t shift = args.l > 1 && args.c_bs % kmc::BKT_LINE ? kmc::BKT_LINE - 1 : 0;
     for (int column = 0; column < classes; column++) {
@@ -176,7 +200,7 @@ static hipError_t launch_short(int load_a, int load_b, const kmc::BuildKernelArg
     const int64_t per_group = static_cast<int64_t>(rounds) * kmc::BKT_COLUMNS * classes;
     const int64_t groups = (args.n + per_group - 1) / per_group * classes;
     kmc::BuildKernelArgs copy = args;
-    void *kernel_args[] = {&copy, &load_a, &load_b, &rounds, &classes};
+    void *kernel_args[] = {&copy, &load_a, &load_b, &rounds, const_cast<int *>(&classes)};
     return hipLaunchKernel(reinterpret_cast<const void *>(kmc::build_kernel_short<KMC_INNER_OP, KMC_INNER_POW, DEPTH>),
                            dim3(static_cast<unsigned>(m_tiles), static_cast<unsigned>(groups), args.l), dim3(kmc::BK_THREADS), kernel_args, 0, stream);
 }

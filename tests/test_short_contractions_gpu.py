@@ -5,6 +5,7 @@ import pytest
 import torch
 
 import kermac_amd as kermac
+from tests.helpers import kernels_of
 
 pytestmark = pytest.mark.gpu
 
@@ -23,13 +24,21 @@ DESCRIPTORS = {
     "dot": descriptor(DOT, POW.NOOP, POW.SQUARE),
     "laplace": descriptor(DIFF, POW.ABS, POW.NOOP, kermac.KernelType.LAPLACE),
     "gaussian": descriptor(DIFF, POW.SQUARE, POW.NOOP, kermac.KernelType.GAUSSIAN),
+    "cubes": descriptor(DIFF, POW.POW),
+    "fourth powers": descriptor(DIFF, POW.POW, POW.SQRT),
 }
+
+
+def launches_short(call):
+    return any("build_kernel_short" in name for name in kernels_of(call))
 
 
 def both(monkeypatch, call):
     monkeypatch.setenv("KERMAC_AMD_DIRECT_SHORT_MAX_K", "24")
+    assert launches_short(call)
     short = call()
     monkeypatch.setenv("KERMAC_AMD_DIRECT_SHORT_MAX_K", "0")
+    assert not launches_short(call)
     return short, call()
 
 
@@ -39,6 +48,8 @@ def test_the_bits_of_the_ordinary_kernel(device, monkeypatch, K, kind):
     g = torch.Generator().manual_seed(K)
     M, N = 531, 277
     options = dict(bandwidth=1.7, regularization=0.25, regularization_offset_x=3, regularization_offset_y=1) if kind in ("laplace", "gaussian") else {}
+    if kind in ("cubes", "fourth powers"):
+        options["inner_p"] = 3.0 if kind == "cubes" else 4.0
     a, b = torch.randn(M, K, generator=g).to(device), torch.randn(N, K, generator=g).to(device)
     for a_used in (a, a.t().contiguous().t()):
         for b_used in (b, b.t().contiguous().t()):
@@ -63,7 +74,7 @@ def test_every_place_in_a_line(device, monkeypatch, ld, offset):
     assert torch.equal(short, ordinary)
 
 
-@pytest.mark.parametrize("M,N", [(1, 1), (1, 1000), (1000, 1), (255, 15), (256, 16), (257, 17), (225, 129), (4000, 2100)])
+@pytest.mark.parametrize("M,N", [(1, 1), (1, 1000), (1000, 1), (255, 15), (256, 16), (257, 17), (225, 129), (512, 40), (4000, 2100)])
 def test_edges(device, monkeypatch, M, N):
     g = torch.Generator().manual_seed(M + N)
     a, b = torch.randn(M, 11, generator=g).to(device), torch.randn(N, 11, generator=g).to(device)
@@ -105,3 +116,21 @@ def test_a_result_of_nearly_2_to_the_31_rows(device, monkeypatch, M, k_contiguou
     assert bool((guard[:33] == -5.0).all()) and bool((guard[33 + M:] == -5.0).all())
     x.sub_(17.0).abs_()
     assert torch.equal(out, x)
+
+
+# (M, N, K): rows of the result contiguous.  More than 256 tiles of 128 x 128; above 8 terms 1024 columns and rows that fill the tiles of 256 (any
+# rows where they are not 16-byte aligned); 13 .. 16 terms of unaligned rows only; 17 .. 24 from 1024 tiles on
+@pytest.mark.parametrize("M,N,K,expected", [(2100, 2100, 8, True), (2048, 2048, 8, False), (100, 60000, 8, True), (30001, 150, 8, True), (5000, 1024, 9, True), (5000, 1023, 9, False),
+                                            (5000, 1024, 12, True), (5000, 1024, 13, False), (5001, 1024, 13, True), (5001, 1024, 16, True), (5000, 3300, 17, True), (5000, 3200, 17, False),
+                                            (5000, 3300, 24, True), (5000, 3300, 25, False), (300, 30000, 12, False), (301, 30000, 12, True), (256, 20000, 12, True), (100, 60000, 12, False),
+                                            (600, 8000, 12, True), (756, 26000, 20, False), (1012, 20000, 20, True)])
+def test_the_rule(device, M, N, K, expected):
+    a, b = torch.zeros(K, M, device=device).t(), torch.zeros(K, N, device=device).t()
+    out = torch.empty(N, M, device=device).t()
+    assert launches_short(lambda: kermac.cdist(a, b, out=out, p=1.0)) == expected
+
+
+@pytest.mark.parametrize("K,expected", [(8, True), (9, False)])
+def test_the_rule_for_a_set_against_itself(device, K, expected):
+    x = torch.zeros(2100, K, device=device)
+    assert launches_short(lambda: kermac.cdist(x, x, p=1.0)) == expected
