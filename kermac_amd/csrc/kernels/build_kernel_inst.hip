@@ -130,13 +130,8 @@ static bool small_applies(int load_a, int load_b, const kmc::BuildKernelArgs &ar
 // us, p = 1, K = 6, 10, 16, 24: 10000 x 10000, rows 16-byte aligned 99 / 80, 103 / 92, 105 / 112, 153 / 150; 2 x 7000 x 7001, result not
 // aligned 182 / 84, 184 / 99, 160 / 117, 231 / 154; 5000 x 5000 35 / 24, 37 / 28, 37 / 32, 49 / 45; 3000 x 2500 16.8 / 13.9, 16.7 / 15.8, 16.2 / 17.8,
 // 21.6 / 24.4.  A set against itself, computed in full here, 2 x 10000, K = 6 and 12, Laplace kernel 226 / 196 and 223 / 233.
-// Up to 8 terms no size of result was found that loses more than it varies (ordinary / this, K = 8, both operands k contiguous and both not): 30000
-// x 300 18.3 / 15.1 and 17.6 / 15.3, 30001 x 300 1.43 and 1.40 times, 30001 x 40 0.97 and 0.96, 100 x 60000 16.5 / 15.6 and 16.2 / 16.7, 16 x 500000 62 / 61 and 60 / 63,
-// 300 x 100 x 100 1.02 both, 64 x 300 x 300 1.03 and 0.98.  With more terms few rows lose what the tiles of 256 rows leave
-// unused of them, where the ordinary kernel stores 16 bytes at a time: K = 12, 100 x 60000 0.84 and 0.78, 300 x 30000 0.90 and 0.91, but 504 x 40000 1.10 and 1.05; K = 18
-// and 24, 504 x 40000 0.87 and 0.78, 756 x 26000 0.86 and 0.79, but 1012 x 20000 1.06 and 0.97.  `short_waste` is
-// that, and the limits are 5 / 4 and 8 / 7 (some sizes of few rows beyond them would gain: 320 x 40000 1.04 and, K = 18 and 24, 1.10 and 1.02).  Few
-// columns, which share a load of all k, gain little or nothing: 10000 x 300 at K = 12 and 24 1.02 and 0.96 .. 1.00, 30000 x 40 0.8 and 0.5.
+// Few columns, which share a load of all k, gain little or nothing above 8 terms: 10000 x 300 at K = 12 and 24 1.02 and 0.96 .. 1.00, 30000 x 40 0.8 and 0.5.
+// Few rows leave tiles of 256 rows unused, in which its arithmetic runs all the same (short_rows_pay).
 // KERMAC_AMD_DIRECT_SHORT_MAX_K=n replaces the rule by "at most n terms" (read on every call, so that a test can choose the kernel).
 constexpr bool HAS_SHORT = !HAS_ROOT_OR_POWER;
 
@@ -148,8 +143,19 @@ static int short_classes(const kmc::BuildKernelArgs &args)
     return classes;
 }
 
-// Rows of this kernel's tiles per row of the ordinary kernel's, on average over where columns start in a line
-static double short_waste(const kmc::BuildKernelArgs &args)
+// Whether the rows fill the tiles well enough.  `waste`: rows of this kernel's tiles of 256 per row of the ordinary kernel's of 128, on average over
+// where columns start in a line.  Up to which it pays depends on what an unused row costs, terms and an exponential or logarithm, and on whether
+// the ordinary kernel stores 16 bytes at a time; where it does not, it pays for each row that there is, which are few below 100.  Time of the ordinary
+// kernel over this one's, distances / Gaussian kernels, results of 4e6 to 6e7 elements, K = 1 .. 4, 5 .. 8, 9 .. 12, and 17 .. 24 (unaligned also 16):
+//   aligned, waste 1 (200, 256, 400, 700 rows)   1.04 .. 1.61 / 1.04 .. 1.63, 1.03 .. 1.58 / 1.05 .. 1.43, 1.02 .. 1.36 / 1.00 .. 1.20, 1.02 .. 1.31 / 0.99 .. 1.29
+//   aligned, 1.25 (500 rows)                     1.20 .. 1.55 / 1.18 .. 1.33, 1.14 .. 1.37 / 1.00 .. 1.10, 0.98 .. 1.08 / 0.85 .. 0.93, 0.82 .. 0.96 / 0.76 .. 0.88
+//   aligned, 1.33 (300, 384)                     1.08 .. 1.49 / 1.11 .. 1.36, 1.01 .. 1.31 / 1.00 .. 1.19, 0.91 .. 1.10 / 0.88 .. 1.07, 0.85 .. 0.98 / 0.84 .. 0.98
+//   aligned, 2 (8, 64, 100, 128)                 0.96 .. 1.48 / 0.93 .. 1.11, 0.95 .. 1.13 / 0.77 .. 1.09, 0.69 .. 1.03 / 0.64 .. 0.99, 0.59 .. 0.98 / 0.56 .. 0.97
+//   unaligned, 1 (129, 150 rows)                 1.20 .. 2.38 / 1.24 .. 1.97, 1.09 .. 1.98 / 1.16 .. 1.59, 1.07 .. 1.58 / 1.04 .. 1.34, 0.97 .. 1.36 / 1.03 .. 1.27
+//   unaligned, 1.2, 1.33 (257, 333, 513)         1.20 .. 2.25 / 1.28 .. 1.98, 1.10 .. 2.07 / 1.21 .. 1.65, 1.09 .. 1.60 / 1.10 .. 1.37, 1.00 .. 1.41 / 0.88 .. 1.37
+//   unaligned, 2 (127)                           1.23 .. 1.97 / 1.32 .. 1.45, 1.11 .. 1.75 / 1.16 .. 1.23, 1.06 .. 1.25 / 0.96 .. 1.03, 0.92 .. 1.06 / 0.81 .. 0.97
+//   unaligned, 2 (10, 17, 33)                    1.09 .. 1.42 / 0.90 .. 1.04, 0.87 .. 1.07 / 0.76 .. 0.89, 0.68 .. 0.86 / 0.64 .. 0.74, 0.57 .. 0.80 / 0.56 .. 0.72
+static bool short_rows_pay(const kmc::BuildKernelArgs &args)
 {
     const int classes = short_classes(args);
     int64_t tiles = 0;
@@ -157,7 +163,14 @@ static double short_waste(const kmc::BuildKernelArgs &args)
         const uint64_t start = reinterpret_cast<uintptr_t>(args.c) / 4 + static_cast<uint64_t>(column) * static_cast<uint64_t>(args.c_ld);
         tiles += (static_cast<int64_t>(args.m) + static_cast<int64_t>(start % kmc::BKT_LINE) + kmc::BKT_TILE_M - 1) / kmc::BKT_TILE_M;
     }
-    return static_cast<double>(tiles) * kmc::BKT_TILE_M / (static_cast<double>(classes) * args.tiles_m * kmc::BK_TILE_M);
+    const double waste = static_cast<double>(tiles) * kmc::BKT_TILE_M / (static_cast<double>(classes) * args.tiles_m * kmc::BK_TILE_M);
+    const bool heavy = args.kernel_type != kmc::KERNEL_NONE || args.outer_power == kmc::POW_POW || KMC_INNER_POW == kmc::POW_ABS_CUBE ||
+                       KMC_INNER_POW == kmc::POW_ABS_FOURTH;
+    const int k = args.k;
+    if (!heavy && k <= 4) return true;
+    if (args.c_vec) return waste <= (heavy ? k <= 8 ? 1.34 : 8.0 / 7 : k <= 8 ? 2.0 : k <= kmc::BK_TILE_K ? 1.25 : 8.0 / 7);
+    if (k <= (heavy ? 8 : kmc::BK_TILE_K) && args.m >= 100) return true;
+    return waste <= (heavy && k > 12 ? 1.25 : 1.34);
 }
 
 static bool short_applies(int load_a, int load_b, const kmc::BuildKernelArgs &args)
@@ -173,11 +186,10 @@ static bool short_applies(int load_a, int load_b, const kmc::BuildKernelArgs &ar
         (HAS_SCALAR_B && load_a == kmc::LOAD_COL_VEC && load_b == kmc::LOAD_COL_VEC && scalar_b_applies(args, &grid_width)))
         return false;
     const int64_t tiles = static_cast<int64_t>(args.tiles_m) * args.tiles_n * args.l;
-    if (tiles <= kmc_rules::DIRECT_SMALL_MAX_TILES) return false;          // for build_kernel_small
+    if (tiles <= kmc_rules::DIRECT_SMALL_MAX_TILES || !short_rows_pay(args)) return false;          // the first for build_kernel_small
     if (args.k <= kmc_rules::DIRECT_SHORT_ANY_MAX_K) return true;
     if (args.symmetric) return false;
     if (args.n < kmc_rules::DIRECT_SHORT_MIN_COLUMNS) return false;
-    if (args.c_vec && short_waste(args) > (args.k <= kmc::BK_TILE_K ? 1.25 : 8.0 / 7)) return false;
     if (args.k <= 12) return true;
     if (args.k <= kmc::BK_TILE_K) return !args.c_vec;
     return tiles >= kmc_rules::DIRECT_SHORT_LONG_MIN_TILES;

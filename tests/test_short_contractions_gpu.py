@@ -118,16 +118,22 @@ def test_a_result_of_nearly_2_to_the_31_rows(device, monkeypatch, M, k_contiguou
     assert torch.equal(out, x)
 
 
-# (M, N, K): rows of the result contiguous.  More than 256 tiles of 128 x 128; above 8 terms 1024 columns and rows that fill the tiles of 256 (any
-# rows where they are not 16-byte aligned); 13 .. 16 terms of unaligned rows only; 17 .. 24 from 1024 tiles on
-@pytest.mark.parametrize("M,N,K,expected", [(2100, 2100, 8, True), (2048, 2048, 8, False), (100, 60000, 8, True), (30001, 150, 8, True), (5000, 1024, 9, True), (5000, 1023, 9, False),
-                                            (5000, 1024, 12, True), (5000, 1024, 13, False), (5001, 1024, 13, True), (5001, 1024, 16, True), (5000, 3300, 17, True), (5000, 3200, 17, False),
-                                            (5000, 3300, 24, True), (5000, 3300, 25, False), (300, 30000, 12, False), (301, 30000, 12, True), (256, 20000, 12, True), (100, 60000, 12, False),
-                                            (600, 8000, 12, True), (756, 26000, 20, False), (1012, 20000, 20, True)])
-def test_the_rule(device, M, N, K, expected):
+# (M, N, K): rows of the result contiguous.  More than 256 tiles of 128 x 128; above 8 terms 1024 columns; 13 .. 16 terms of unaligned rows only;
+# 17 .. 24 from 1024 tiles on; and rows that fill the tiles of 256, more of them for more terms and for a kernel function
+@pytest.mark.parametrize("M,N,K,distance,gaussian", [
+    (2100, 2100, 8, True, True), (2048, 2048, 8, False, False), (30001, 150, 8, True, True), (5000, 1024, 9, True, True), (5000, 1023, 9, False, False),
+    (5000, 1024, 12, True, True), (5000, 1024, 13, False, False), (5001, 1024, 13, True, True), (5001, 1024, 16, True, True), (5000, 3300, 17, True, True),
+    (5000, 3200, 17, False, False), (5000, 3300, 24, True, True), (5000, 3300, 25, False, False),
+    (100, 60000, 4, True, False), (100, 60000, 8, True, False), (100, 60000, 12, False, False), (256, 20000, 12, True, True), (300, 30000, 8, True, True),
+    (300, 30000, 12, False, False), (504, 12000, 12, True, False), (504, 40000, 20, False, False), (1012, 20000, 20, True, True), (756, 26000, 20, False, False),
+    (17, 60000, 4, True, False), (17, 60000, 5, False, False), (127, 40000, 8, True, True), (127, 40000, 12, True, False), (301, 30000, 12, True, True),
+    (257, 30000, 15, True, False), (257, 60000, 20, True, False), (129, 90000, 20, True, True)])
+def test_the_rule(device, M, N, K, distance, gaussian):
     a, b = torch.zeros(K, M, device=device).t(), torch.zeros(K, N, device=device).t()
     out = torch.empty(N, M, device=device).t()
-    assert launches_short(lambda: kermac.cdist(a, b, out=out, p=1.0)) == expected
+    assert launches_short(lambda: kermac.cdist(a, b, out=out, p=1.0)) == distance
+    with kermac.l2_mode("direct"):
+        assert launches_short(lambda: kermac.run_kernel(DESCRIPTORS["gaussian"], a, b, out=out, bandwidth=1.0)) == gaussian
 
 
 @pytest.mark.parametrize("K,expected", [(8, True), (9, False)])
