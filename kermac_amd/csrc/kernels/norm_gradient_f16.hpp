@@ -18,15 +18,15 @@
 //                          sorted order -0 below +0, so that signed zeros and ties come out as copysign(1, d - b).
 //                          Rows of B longer than that are cut into chunks with positions of their own.
 //                          The same launch copies A into the order in which a wave reads it, scales C by a power of two per
-//                          row o, and estimates the largest |A[m, k] C[o, k]| over k for every m and o.
+//                          row o, and bounds |A[m, k] C[o, k]| for every m and o by its sum over 128 k or fewer.
 // norm_gradient_l1_f16     the product.
 //
-// Accuracy: S is exact.  w = a c 2^F with its largest value over k in [2^14, 2^15.2), F of every m and o from the estimate; w1 =
-// fp16(w), w2 = fp16(w - w1), so |w - w1 - w2| <= 2^-22 |w| + 2^-39 max_k|w|, however far max_k|a c| is below max|a| max|c|.  Doubled
+// Accuracy: S is exact.  w = a c 2^F with its largest sum over those k in [2^14, 2^15.2), F of every m and o from the launch before; w1 =
+// fp16(w), w2 = fp16(w - w1), so |w - w1 - w2| <= 2^-22 |w| + 2^-39 sum_k|w|, however far max_k|a c| is below max|a| max|c|.  Doubled
 // with the result, that is below 3 * 2^-22 sum_k |c a| up to K = 2^16, beside the fp32 accumulation.  (A scale per row m of A times one per
 // row o of C is not enough: in rows with a large value whose partner is zero, 1 beside 2^-16 say, fp16's smallest step takes the place
-// of the others' last bits, 6e-6 of sum_k |c a| and more.)  Zeros count as 2^-127 in the estimate, which shows where max|a| or max|c| is above
-// 2^100 times the products; rows of A below 2^-113 keep fewer bits.  The sums run over S W, so  1/2 sum_k W  is taken off them again: every 256
+// of the others' last bits, 6e-6 of sum_k |c a| and more.)  Sums of zero count as 2^-127, which shows where max|a| or max|c| is above
+// 2^100 times the products; rows of A below 2^-112 keep fewer bits.  The sums run over S W, so  1/2 sum_k W  is taken off them again: every 256
 // k, since a partial sum of S W alone drifts away from the one of the signed terms, and rounding follows the partial sums.
 //
 // Workgroup of norm_gradient_l1_f16: 8 waves, 16 m x 16 BLOCKS n x 16 o; wave w owns the 2 m  2w, 2w + 1  and all n, as
@@ -66,8 +66,9 @@ constexpr int NGF_COPY_M = 128;                // tile of the copy of A: m, and 
 constexpr int NGF_COPY_MAX_K = 512;
 constexpr int NGF_COPY_MIN_K = 64;
 constexpr int NGF_COPY_DEPTH = 16;             // k per lane at a time
-constexpr int NGF_COPY_C_PITCH = NGF_TILE_O + 4;       // words of LDS per two k of 16 o
-constexpr int NGF_EXPONENT_W = 14;             // largest W of a result in [2^14, 2^15.2): fp16 ends at 2^16
+constexpr int NGF_COPY_C_PITCH = 4 * NGF_TILE_O + 4;   // words of LDS per eight k of 16 o
+constexpr int NGF_COPY_C_WORDS = NGF_COPY_MAX_K / 8 * NGF_COPY_C_PITCH;
+constexpr int NGF_EXPONENT_W = 14;             // bound of a result's W in [2^14, 2^15.2): fp16 ends at 2^16
 constexpr int NGF_EXPONENT_C = 14;             // largest C of a row as it is copied, in [2^14, 2^15): A, which takes the rest of W's scale, is
                                                // then brought to 1 or a little more
 constexpr int NGF_MAX_CHUNK = 14272;           // k per sorted chunk: whole stages, counts up to 14334 (signs_half)
@@ -80,7 +81,7 @@ struct NormGradientF16Args {
     i64 positions_bs, counts_bs;               // in halves
     const float *a_copy; i64 a_copy_bs;        // [batch][m_pad / 2][k_pad / 32][4][2][8]: 8 k of each of 2 m, 4 times
     const float *a_magnitudes; i64 a_magnitudes_bs;    // [batch][ranges][m_pad]
-    const unsigned short *products; i64 products_bs;   // [batch][ranges][o_pad / 16][m_pad][16 o]: signs_product
+    const unsigned short *products; i64 products_bs;   // [batch][ranges][o_pad / 16][m_pad][16 o]: sums of |a c|, bfloat16
     const float *c_copy; i64 c_copy_bs;        // [batch][o_pad / 16][k_pad / 4][16 o][4 k], times 2^c_exponents
     const int *c_exponents; i64 c_exponents_bs;        // [batch][o_pad]
     int n_pad, m_pad, k_pad, o_pad, ranges;
@@ -257,21 +258,51 @@ __device__ __forceinline__ void signs_rank_row(const GradientPrepareArgs &args, 
     }
 }
 
-typedef unsigned short ngf_ushort2 __attribute__((ext_vector_type(2)));
+typedef unsigned short ngf_ushort8 __attribute__((ext_vector_type(8)));
 
-// The upper halves of |x0| and |x1|.  As an integer, that of x is 128 (127 + log2|x|), below it by no more than 128 * 0.094 (the
-// mantissa stands for its logarithm, and its last bits are missing), so the sum of two of them is the logarithm of a
-// product, and finding the largest product of a row takes an addition and a maximum of 16 bits per term.
-__device__ __forceinline__ ngf_ushort2 signs_logarithms(float x0, float x1)
+typedef short ngf_short4 __attribute__((ext_vector_type(4)));
+
+// |x0| and |x1| as bfloat16, rounded down
+__device__ __forceinline__ unsigned signs_magnitudes(float x0, float x1)
 {
-    return __builtin_bit_cast(ngf_ushort2, __builtin_amdgcn_perm(__float_as_uint(x1), __float_as_uint(x0), 0x07060302u) & 0x7fff7fffu);
+    return __builtin_amdgcn_perm(__float_as_uint(x1), __float_as_uint(x0), 0x07060302u) & 0x7fff7fffu;
 }
 
-// 128 m x copy_k k of A into the order of the product's waves, the largest magnitude per m, and the logarithm of the largest |a c| per m
-// and o of one block of 16 outputs (the blocks after the first only that).  A lane holds 2 m and 16 k at a time, which are 128
-// bytes of the copy; a wave takes a quarter of the k; the logarithms of C stand in LDS and are read as broadcasts.  Memory-bound
-// together with the sorts beside it for 16 outputs (8192 x 512 x 16 x 8192: the launch 0.18 ms without the products, 0.20 with them), beyond that
-// bound by the vector ALU, 4.6 cycles of a SIMD per 64 terms: 4000 x 32 x 128 x 4000 0.05 without, 0.13 with them.
+// Chunk j of a lane becomes its chunk of the four that lane j of its group of four holds
+__device__ __forceinline__ void signs_transpose_quad(float4 (&chunk)[4], int lane)
+{
+#pragma unroll
+    for (int bit = 1; bit <= 2; bit *= 2) {
+        const bool upper = lane & bit;
+        auto exchange = [&](float &low, float &high) {
+            const int sent = __float_as_int(upper ? low : high);
+            const float received = __int_as_float(bit == 1 ? __builtin_amdgcn_update_dpp(0, sent, 0xB1, 0xF, 0xF, true)      // quad_perm 1, 0, 3, 2
+                                                           : __builtin_amdgcn_update_dpp(0, sent, 0x4E, 0xF, 0xF, true));    // quad_perm 2, 3, 0, 1
+            low = upper ? received : low;
+            high = upper ? high : received;
+        };
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            if (j & bit) continue;
+            exchange(chunk[j].x, chunk[j + bit].x);
+            exchange(chunk[j].y, chunk[j + bit].y);
+            exchange(chunk[j].z, chunk[j + bit].z);
+            exchange(chunk[j].w, chunk[j + bit].w);
+        }
+    }
+}
+
+// Half word of LDS of the sum of row m and output 0 of a tile: 4 words of padding per 8 rows, or lanes that own them meet in one bank
+__device__ __forceinline__ int signs_sum_at(int m)
+{
+    return 16 * m + 8 * (m >> 3);
+}
+
+// 128 m x copy_k k of A into the order of the product's waves, the largest magnitude per m, and for one block of 16 outputs (the blocks after
+// the first only that) sum_k |a c| per m and o, the largest of four quarters of the k.  No |a c| is above its sum, and the sum, unlike a
+// maximum, is work for the matrix instruction: v_mfma_f32_4x4x4_16B_bf16 takes 4 k of a lane's own row with 4 outputs, which are read as broadcasts
+// of LDS.  (bfloat16 has the range of fp32; rounded down, |a|, |c| and the sum are up to 2.4 % too small.)  A lane holds 2 m and 16 k at a time,
+// which are 128 bytes of the copy; a wave takes a quarter of the k.
 __device__ __forceinline__ void signs_copy_tile(const GradientPrepareArgs &args, int block, int batch, unsigned *shared)
 {
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -283,26 +314,6 @@ __device__ __forceinline__ void signs_copy_tile(const GradientPrepareArgs &args,
     const int o_count = min(args.o - NGF_TILE_O * o_block, NGF_TILE_O);
     const int k_first = range * args.copy_k, k_count = min(args.copy_k, args.k_pad - k_first);
     const bool copies = o_block == 0 && batch < args.a_batches;
-
-    // loads of what does not exist, of C and of A, go to the last element that does and are dropped: with a branch for each they would be
-    // waited for one by one
-    const float *c = args.c + batch * args.c_bs + (i64)NGF_TILE_O * o_block * args.c_ld;
-    for (int pair = tid; pair < k_count / 2; pair += NGF_PREPARE_THREADS) {
-        const int k = k_first + 2 * pair, at0 = min(k, args.k - 1), at1 = min(k + 1, args.k - 1);
-        float x[NGF_TILE_O][2];
-#pragma unroll
-        for (int o = 0; o < NGF_TILE_O; o++) {
-            const float *row = c + (i64)min(o, o_count - 1) * args.c_ld;
-            x[o][0] = row[at0];
-            x[o][1] = row[at1];
-        }
-#pragma unroll
-        for (int o = 0; o < NGF_TILE_O; o++) {
-            const bool live = o < o_count;
-            shared[pair * NGF_COPY_C_PITCH + o] =
-                __builtin_bit_cast(unsigned, signs_logarithms(live && k < args.k ? x[o][0] : 0.0f, live && k + 1 < args.k ? x[o][1] : 0.0f));
-        }
-    }
 
     const int m = m0 + 2 * lane;
     const float *a = args.a + batch * args.a_bs;
@@ -327,20 +338,52 @@ __device__ __forceinline__ void signs_copy_tile(const GradientPrepareArgs &args,
         }
     };
     float magnitude[2] = {0.0f, 0.0f};
-    ngf_ushort2 largest[2][NGF_TILE_O];                    // over even and odd k
+    const int k_wave = k_first + wave * (k_count / 4), k_end = k_wave + k_count / 4;        // k_count: a multiple of 64
+    load(k_wave);
+    // C while these are under way: four outputs per wave, two k per lane.  Loads of what does not exist, of C and of A, go to the
+    // last element that does and are dropped: with a branch for each they would be waited for one by one
+    {
+        constexpr int ROWS = NGF_TILE_O / 4;
+        const float *c = args.c + batch * args.c_bs + (i64)NGF_TILE_O * o_block * args.c_ld;
+        constexpr int TIMES = 2;
+        for (int first = 0; first < k_count / 2; first += 64 * TIMES) {
+            float x[TIMES][ROWS][2];
+#pragma unroll
+            for (int t = 0; t < TIMES; t++) {
+                const int k = k_first + 2 * (first + 64 * t + lane), at0 = min(k, args.k - 1), at1 = min(k + 1, args.k - 1);
+#pragma unroll
+                for (int j = 0; j < ROWS; j++) {
+                    const float *row = c + (i64)min(ROWS * wave + j, o_count - 1) * args.c_ld;
+                    x[t][j][0] = row[at0];
+                    x[t][j][1] = row[at1];
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < TIMES; t++) {
+                const int pair = first + 64 * t + lane, k = k_first + 2 * pair;
+#pragma unroll
+                for (int j = 0; j < ROWS; j++) {
+                    const int o = ROWS * wave + j;
+                    if (pair < k_count / 2)
+                        shared[pair / 4 * NGF_COPY_C_PITCH + 4 * o + pair % 4] =
+                            signs_magnitudes(o < o_count && k < args.k ? x[t][j][0] : 0.0f, o < o_count && k + 1 < args.k ? x[t][j][1] : 0.0f);
+                }
+            }
+        }
+    }
+    // sums[i][o4][j]: m = m0 + 8 (lane / 4) + 2 j + i, the row of lane 4 (lane / 4) + j, o = 4 o4 + lane % 4
+    ngf_float4 sums[2][NGF_TILE_O / 4];
 #pragma unroll
     for (int i = 0; i < 2; i++)
 #pragma unroll
-        for (int o = 0; o < NGF_TILE_O; o++) largest[i][o] = ngf_ushort2{0, 0};
-    const int k_wave = k_first + wave * (k_count / 4), k_end = k_wave + k_count / 4;        // k_count: a multiple of 64
-    load(k_wave);
+        for (int o4 = 0; o4 < NGF_TILE_O / 4; o4++) sums[i][o4] = ngf_float4{0.0f, 0.0f, 0.0f, 0.0f};
     __syncthreads();
     for (int k0 = k_wave; k0 < k_end; k0 += NGF_COPY_DEPTH) {
-        ngf_ushort2 logarithms[2][NGF_COPY_DEPTH / 2];
+        uint2 magnitudes[2][NGF_COPY_DEPTH / 4];           // 4 k
 #pragma unroll
-        for (int j = 0; j < NGF_COPY_DEPTH / 2; j++) {
-            logarithms[0][j] = signs_logarithms(v[2 * j].x, v[2 * j + 1].x);
-            logarithms[1][j] = signs_logarithms(v[2 * j].y, v[2 * j + 1].y);
+        for (int j = 0; j < NGF_COPY_DEPTH / 4; j++) {
+            magnitudes[0][j] = make_uint2(signs_magnitudes(v[4 * j].x, v[4 * j + 1].x), signs_magnitudes(v[4 * j + 2].x, v[4 * j + 3].x));
+            magnitudes[1][j] = make_uint2(signs_magnitudes(v[4 * j].y, v[4 * j + 1].y), signs_magnitudes(v[4 * j + 2].y, v[4 * j + 3].y));
         }
         if (copies) {
 #pragma unroll
@@ -348,63 +391,70 @@ __device__ __forceinline__ void signs_copy_tile(const GradientPrepareArgs &args,
                 magnitude[0] = fmaxf(magnitude[0], fabsf(v[j].x));
                 magnitude[1] = fmaxf(magnitude[1], fabsf(v[j].y));
             }
-            if (m < args.m_pad) {
-                float4 *dst = reinterpret_cast<float4 *>(args.a_copy + batch * args.a_copy_bs + ((i64)(m / 2) * args.k_pad + k0) * 2);
+            // 8 k of a lane's two m are 64 bytes of the copy: four lanes exchange theirs and store 64 bytes side by side (a lane's own stores, 16
+            // bytes of 64 lines each, take half as long again as the memory)
 #pragma unroll
-                for (int eight = 0; eight < NGF_COPY_DEPTH; eight += 8)
+            for (int eight = 0; eight < NGF_COPY_DEPTH; eight += 8) {
+                float4 chunk[4];
 #pragma unroll
-                    for (int j = 0; j < 8; j += 4) {
-                        dst[eight / 2 + j / 4] = make_float4(v[eight + j].x, v[eight + j + 1].x, v[eight + j + 2].x, v[eight + j + 3].x);
-                        dst[eight / 2 + 2 + j / 4] = make_float4(v[eight + j].y, v[eight + j + 1].y, v[eight + j + 2].y, v[eight + j + 3].y);
-                    }
+                for (int j = 0; j < 8; j += 4) {
+                    chunk[j / 4] = make_float4(v[eight + j].x, v[eight + j + 1].x, v[eight + j + 2].x, v[eight + j + 3].x);
+                    chunk[2 + j / 4] = make_float4(v[eight + j].y, v[eight + j + 1].y, v[eight + j + 2].y, v[eight + j + 3].y);
+                }
+                signs_transpose_quad(chunk, lane);
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const int pair = m0 / 2 + (lane & ~3) + j;
+                    if (2 * pair < args.m_pad)
+                        *reinterpret_cast<float4 *>(args.a_copy + batch * args.a_copy_bs + ((i64)pair * args.k_pad + k0 + eight) * 2 + 4 * (lane & 3)) = chunk[j];
+                }
             }
         }
         if (k0 + NGF_COPY_DEPTH < k_end) load(k0 + NGF_COPY_DEPTH);
-        const uint4 *of_c = reinterpret_cast<const uint4 *>(shared + (k0 - k_first) / 2 * NGF_COPY_C_PITCH);
-        // four outputs at a time, so that the reads of their logarithms stand side by side behind one branch
+        // (outputs that do not exist are zeros: a branch for them would have their reads waited for one by one)
 #pragma unroll
-        for (int o4 = 0; o4 < NGF_TILE_O / 4; o4++) {
-            if (4 * o4 >= o_count) continue;
+        for (int eight = 0; eight < NGF_COPY_DEPTH / 8; eight++) {
+            uint4 c8[NGF_TILE_O / 4];
 #pragma unroll
-            for (int j = 0; j < NGF_COPY_DEPTH / 2; j++) {
-                const uint4 x = of_c[j * (NGF_COPY_C_PITCH / 4) + o4];
-                const unsigned words[4] = {x.x, x.y, x.z, x.w};
+            for (int o4 = 0; o4 < NGF_TILE_O / 4; o4++)
+                c8[o4] = *reinterpret_cast<const uint4 *>(shared + ((k0 - k_first) / 8 + eight) * NGF_COPY_C_PITCH + 16 * o4 + 4 * (lane & 3));
 #pragma unroll
-                for (int o = 0; o < 4; o++)
+            for (int four = 0; four < 2; four++)
+#pragma unroll
+                for (int o4 = 0; o4 < NGF_TILE_O / 4; o4++)
 #pragma unroll
                     for (int i = 0; i < 2; i++)
-                        largest[i][4 * o4 + o] = __builtin_elementwise_max(largest[i][4 * o4 + o], logarithms[i][j] + __builtin_bit_cast(ngf_ushort2, words[o]));
-            }
+                        sums[i][o4] = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(
+                            __builtin_bit_cast(ngf_short4, magnitudes[i][2 * eight + four]),
+                            __builtin_bit_cast(ngf_short4, four == 0 ? make_uint2(c8[o4].x, c8[o4].y) : make_uint2(c8[o4].z, c8[o4].w)), sums[i][o4], 0, 0, 0);
         }
     }
-    // the four waves' largest: [wave][i][two outputs to a word][lane], and behind them the magnitudes
-    constexpr int WORDS = NGF_TILE_O / 2;
-    float *const magnitudes = reinterpret_cast<float *>(shared + 4 * 2 * WORDS * 64);
+    // the four waves' sums, as bfloat16, and behind them the magnitudes
+    constexpr int WAVE_WORDS = NGF_COPY_M * NGF_TILE_O / 2 + NGF_COPY_M / 2;
+    unsigned short *const wave_sums = reinterpret_cast<unsigned short *>(shared);
+    float *const magnitudes = reinterpret_cast<float *>(shared + 4 * WAVE_WORDS);
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < 2; i++) {
 #pragma unroll
-        for (int j = 0; j < WORDS; j++) {
-            const ngf_ushort2 first = largest[i][2 * j], second = largest[i][2 * j + 1];
-            shared[((wave * 2 + i) * WORDS + j) * 64 + lane] = max(first.x, first.y) | (unsigned)max(second.x, second.y) << 16;
-        }
+        for (int o4 = 0; o4 < NGF_TILE_O / 4; o4++)
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                wave_sums[2 * wave * WAVE_WORDS + signs_sum_at(8 * (lane >> 2) + 2 * j + i) + 4 * o4 + (lane & 3)] =
+                    (unsigned short)(__float_as_uint(sums[i][o4][j]) >> 16 & 0x7fff);
         magnitudes[(wave * 2 + i) * 64 + lane] = magnitude[i];
     }
     __syncthreads();
     const int to = m0 + (tid >> 1), i = tid >> 1 & 1;      // half of the outputs of one m per thread
     if (to >= args.m_pad) return;
     if (batch < args.product_batches) {
-        unsigned word[WORDS / 2];
+        ngf_ushort8 largest = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
-        for (int j = 0; j < WORDS / 2; j++) {
-            ngf_ushort2 x = {0, 0};
-#pragma unroll
-            for (int part = 0; part < 4; part++)
-                x = __builtin_elementwise_max(x, __builtin_bit_cast(ngf_ushort2, shared[((part * 2 + i) * WORDS + WORDS / 2 * (tid & 1) + j) * 64 + (tid >> 2)]));
-            word[j] = __builtin_bit_cast(unsigned, x);
-        }
+        for (int part = 0; part < 4; part++)
+            largest = __builtin_elementwise_max(
+                largest, *reinterpret_cast<const ngf_ushort8 *>(wave_sums + 2 * part * WAVE_WORDS + signs_sum_at(tid >> 1) + 8 * (tid & 1)));
         unsigned short *products = args.products + batch * args.products_bs + (((i64)range * o_blocks + o_block) * args.m_pad + to) * NGF_TILE_O;
-        reinterpret_cast<uint4 *>(products)[tid & 1] = make_uint4(word[0], word[1], word[2], word[3]);
+        reinterpret_cast<ngf_ushort8 *>(products)[tid & 1] = largest;
     }
     if (copies && !(tid & 1)) {
         float x = 0.0f;
@@ -454,11 +504,12 @@ __device__ __forceinline__ void signs_scale_row(const GradientPrepareArgs &args,
 // CU, spread evenly over the launch (all sorts within its first half: 214 us in the place of 200 at 8192 x 512 x 16 x 8192).  The rows of C, few
 // and slow, come first.
 template <int LOG_R>
-__global__ __launch_bounds__(NGF_PREPARE_THREADS, LOG_R < 6 ? 4 : 2) void gradient_signs_prepare(const GradientPrepareArgs args)
+__global__ __launch_bounds__(NGF_PREPARE_THREADS, LOG_R < 5 ? 4 : LOG_R < 6 ? 3 : 2) void gradient_signs_prepare(const GradientPrepareArgs args)
 {
     constexpr int WORDS = (256 << LOG_R) + (8 << LOG_R);
-    constexpr int TILE_WORDS = NGF_COPY_MAX_K / 2 * NGF_COPY_C_PITCH;
-    static_assert(TILE_WORDS >= 4 * 64 * (NGF_TILE_O + 2), "the waves' results");
+    // C of a tile, then the waves' sums and magnitudes
+    constexpr int SUM_WORDS = 4 * (NGF_COPY_M * (NGF_TILE_O + 1) / 2 + NGF_COPY_M);
+    constexpr int TILE_WORDS = NGF_COPY_C_WORDS > SUM_WORDS ? NGF_COPY_C_WORDS : SUM_WORDS;
     __shared__ __attribute__((aligned(16))) unsigned words[WORDS > TILE_WORDS ? WORDS : TILE_WORDS];
     const int batch = blockIdx.y, block_behind_c = (int)blockIdx.x - args.o_pad;
     if (block_behind_c < 0) {
@@ -595,7 +646,7 @@ __global__ __launch_bounds__(NGF_THREADS, BLOCKS >= 8 ? 2 : 4) void norm_gradien
                 magnitude[i] = fmaxf(magnitude[i], __shfl_xor(magnitude[i], bit));
                 product[i] = max(product[i], __shfl_xor(product[i], bit));
             }
-            const int exponent = min(min(NGF_EXPONENT_W - ((product[i] >> 7) - 254) - c_exponent, 126 - signs_exponent(magnitude[i])), 127);
+            const int exponent = min(min(NGF_EXPONENT_W - ((product[i] >> 7) - 127) - c_exponent, 126 - signs_exponent(magnitude[i])), 126);
             scale[i] = __builtin_ldexpf(1.0f, exponent);
             unscale[i] = 1 - exponent - c_exponent;          // doubled: 2 S - 1 is summed as S - 1/2
         }

@@ -237,6 +237,21 @@ def test_small_products_beside_large_values(device, f16_route, kind, M, N, O, K,
     assert worst <= 1.0, f"{worst:.3g} times the bound"
 
 
+@pytest.mark.parametrize("small", ["c", "a"])
+def test_products_of_subnormal_values_count(device, f16_route, small):
+    """2^-130 in one operand and 2^100 in the other make the largest product by far: a scale that missed it would end in infinities."""
+    M, N, O, K = 70, 40, 16, 64
+    g = torch.Generator().manual_seed(3)
+    a, c = torch.rand(K, M, generator=g) + 0.5, torch.rand(O, K, generator=g) + 0.5
+    (a if small == "c" else c).mul_(2.0 ** -100)
+    (c if small == "c" else a.T)[:, 5], (a.T if small == "c" else c)[:, 5] = 2.0 ** -130, 2.0 ** 100
+    b, d = torch.randn(N, K, generator=g), torch.randn(N, M, generator=g)
+    got = kermac.cdist_grad(*(t.to(device) for t in (a, b, c, d)), p=1.0)[0].double().cpu()
+    sign = torch.copysign(torch.ones(()), d[:, None, :] - b[:, :, None]).double()                       # [N, K, M]
+    truth = torch.einsum("ok,km,nkm->onm", c.double(), a.double(), sign)
+    torch.testing.assert_close(got, truth, rtol=1e-6, atol=0.0)
+
+
 @pytest.mark.parametrize("M,N,O,tiles", [(2000, 700, 18, {"<12, false", "<12, true"}),      # two launches of 500 tiles of 192 n, two rounds each
                                          (9000, 200, 20, {"<16, false", "<16, true"}),      # 563 of 256 n: three
                                          (1500, 300, 17, {"<4, false", "<4, true"}),        # 470 of 64 n, two on a CU
