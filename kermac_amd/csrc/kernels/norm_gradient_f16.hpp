@@ -632,11 +632,15 @@ __global__ __launch_bounds__(NGF_THREADS, BLOCKS >= 8 ? 2 : 4) void norm_gradien
         const unsigned short *products = args.products + batch * args.products_bs + ((i64)(o0 / NGF_TILE_O) * args.m_pad + m0 + 2 * wave) * NGF_TILE_O + column;
         float magnitude[2] = {0.0f, 0.0f};
         int product[2] = {0, 0};
-        for (int range = q; range < args.ranges; range += 4)
+        for (int first = q; first < args.ranges; first += 16)
 #pragma unroll
-            for (int i = 0; i < 2; i++) {
-                magnitude[i] = fmaxf(magnitude[i], magnitudes[(i64)range * args.m_pad + i]);
-                product[i] = max(product[i], (int)products[(i64)range * args.o_pad * args.m_pad + NGF_TILE_O * i]);
+            for (int j = 0; j < 4; j++) {                  // loads side by side; beyond the end the last one again
+                const i64 range = min(first + 4 * j, args.ranges - 1);
+#pragma unroll
+                for (int i = 0; i < 2; i++) {
+                    magnitude[i] = fmaxf(magnitude[i], magnitudes[range * args.m_pad + i]);
+                    product[i] = max(product[i], (int)products[range * args.o_pad * args.m_pad + NGF_TILE_O * i]);
+                }
             }
         const int c_exponent = args.c_exponents[batch * args.c_exponents_bs + o0 + column];
 #pragma unroll

@@ -112,26 +112,31 @@ bool gradient_layout(const kmc_norm_gradient_params *p, GradientLayout *layout)
     return true;
 }
 
-// Tile of the product in n: 16, 12, 8, 4 or 2 blocks of 16, as blocks and us of two rounds of the 256 CUs at K = 8192, the second with the pieces in the
-// columns.  A step costs about as much as 8 blocks beside its blocks, W above all, so wide tiles are cheaper per result, unless they are too few for the
-// CUs or their last round is nearly empty.  Up to 4 blocks two workgroups share a CU and take as long as one behind the other, but need
-// no whole rounds; 8 % are taken off for what they hide of each other's ends (378, 431, 338 and 377 with the chip full; 2100 x 260 x 10 x 5000 in tiles
-// of 4 and 12 blocks 329 and 363 us, 1500 x 300 x 17 x 1500 138 and 146).
+// Tile of the product in n: 16, 12, 8, 4 or 2 blocks of 16, as blocks and the cost of a workgroup, the second with the pieces in the
+// columns, in us of two rounds of the 256 CUs at K = 8192 for those that have a CU to themselves.  A step costs about as much as 8 blocks beside its
+// blocks, W above all, so wide tiles are cheaper per result, unless they are too few for the CUs or their last round is nearly empty.  Up to 4 blocks
+// two workgroups share a CU and hide each other's ends: their cost is fitted to 120 shapes with every tile, K = 250 .. 5000.  12 / 4 blocks, us:
+// 3264 x 304 x 16 x K, K = 800 119 / 106, K = 5000 482 / 461; 6000 x 147 x 16 x 5000 502 / 561; 16 / 4 blocks: 9000 x 200 x 16 x 5000 882 / 965.  (Below about 500 k
+// the ends weigh more than this counts: K = 250 there 120 / 102.)
 // 12 is for n that fill little of the second half of a larger tile: with the others only / with
 // 12, us: 3000 x 147 x 64 x 4000 714 / 577, 2000 x 300 x 20 x 2000 301 / 212, 4000 x 147 x 32 x 4000 481 / 399.
-constexpr struct { int blocks, us, us_in_columns; } PRODUCT_TILES[] = {{16, 936, 743}, {12, 772, 642}, {8, 621, 536}, {4, 397, 347}, {2, 348, 311}};
+constexpr struct { int blocks, cost, cost_in_columns; } PRODUCT_TILES[] = {{16, 936, 743}, {12, 772, 642}, {8, 621, 536}, {4, 355, 295}, {2, 255, 225}};
 
-int blocks_for(const kmc_norm_gradient_params *p, int o_chunks, bool pieces_in_columns)
+struct ProductTile {
+    int blocks;
+    int64_t cost;
+};
+
+ProductTile tile_for(const kmc_norm_gradient_params *p, int o_chunks, bool pieces_in_columns)
 {
-    int best = 0;
-    int64_t best_cost = INT64_MAX;
+    ProductTile best = {0, o_chunks ? INT64_MAX : 0};
     for (const auto &tile : PRODUCT_TILES) {
         const int tile_n = 16 * tile.blocks;
         // 12 where its last tile ends inside the padded rows
         if (tile.blocks == 12 && round_up(p->n, tile_n) > round_up(p->n, kmc::NGF_N_PAD)) continue;
         const int64_t workgroups = static_cast<int64_t>((p->n + tile_n - 1) / tile_n) * ((p->m + kmc::NGF_TILE_M - 1) / kmc::NGF_TILE_M) * p->l * o_chunks;
-        const int64_t cost = (tile.blocks > 4 ? round_up(workgroups, 256) : workgroups > 256 ? workgroups : 256) * (pieces_in_columns ? tile.us_in_columns : tile.us);
-        if (cost < best_cost) { best = tile.blocks; best_cost = cost; }
+        const int64_t cost = round_up(workgroups, 256) / 256 * (pieces_in_columns ? tile.cost_in_columns : tile.cost);
+        if (cost < best.cost) best = {tile.blocks, cost};
     }
     return best;
 }
@@ -229,13 +234,18 @@ hipError_t launch_norm_gradient_f16(const kmc_norm_gradient_params *p, bool a_ve
     args.c_exponents = prepare.c_exponents; args.c_exponents_bs = layout.c_batches > 1 ? layout.o_pad : 0;
     args.n_pad = layout.n_pad; args.m_pad = layout.m_pad; args.k_pad = layout.k_pad; args.o_pad = layout.o_pad; args.ranges = layout.ranges;
     args.chunk_stages = layout.chunk_k / kmc::NGF_STAGE_K; args.stages = layout.stages;
-    // blocks of 16 outputs; what is left up to 8 in the first half of the columns, its second pieces in the other
-    const int left = p->o % kmc::NGF_TILE_O;
-    const int in_columns = left > 0 && left <= 8 ? 1 : 0;
-    const int full_chunks = (p->o + kmc::NGF_TILE_O - 1) / kmc::NGF_TILE_O - in_columns;
-    // two launches, one behind the other: a tile for each
-    if (full_chunks) status = launch_products<false>(blocks_for(p, full_chunks, false), args, 0, full_chunks, stream);
-    if (status == hipSuccess && in_columns) status = launch_products<true>(blocks_for(p, 1, true), args, p->o - left, 1, stream);
+    // Blocks of 16 outputs; what is left up to 8 in the first half of the columns, its second pieces in the other, in a launch behind the
+    // first, with a tile of its own, unless one launch with a block of 16 for them fills its rounds better: 2794 x 344 x 24 x 838, 350
+    // tiles of 192 n, 244 us in two launches and 196 in one
+    const int left = p->o % kmc::NGF_TILE_O, all_chunks = (p->o + kmc::NGF_TILE_O - 1) / kmc::NGF_TILE_O;
+    const bool may_split = left > 0 && left <= 8;
+    const ProductTile whole = tile_for(p, all_chunks, false), full = tile_for(p, all_chunks - 1, false), rest = tile_for(p, 1, true);
+    if (may_split && full.cost + rest.cost < whole.cost) {
+        if (all_chunks > 1) status = launch_products<false>(full.blocks, args, 0, all_chunks - 1, stream);
+        if (status == hipSuccess) status = launch_products<true>(rest.blocks, args, p->o - left, 1, stream);
+    } else {
+        status = launch_products<false>(whole.blocks, args, 0, all_chunks, stream);
+    }
     if (status == hipSuccess) *taken = true;
     return status;
 }

@@ -5,9 +5,10 @@ contraction on the fp16 matrix instruction.  Tolerance as for the other gradient
 result is a signed sum of K products, |got - truth| <= 1e-5 |truth| + 1e-4 mean |truth|.
 
 KERMAC_AMD_GRADIENT_F16_MIN_TERMS=1 sends the small shapes of these tests down the route, which by
-itself only takes problems of at least 4e8 terms and 3 outputs.
+itself only takes problems of at least 3 outputs, 24 n and 6.4e9 / outputs terms (1.5e7 above 16 outputs).
 """
 import importlib
+import re
 
 import pytest
 import torch
@@ -252,12 +253,15 @@ def test_products_of_subnormal_values_count(device, f16_route, small):
     torch.testing.assert_close(got, truth, rtol=1e-6, atol=0.0)
 
 
-@pytest.mark.parametrize("M,N,O,tiles", [(2000, 700, 18, {"<12, false", "<12, true"}),      # two launches of 500 tiles of 192 n, two rounds each
-                                         (9000, 200, 20, {"<16, false", "<16, true"}),      # 563 of 256 n: three
-                                         (1500, 300, 17, {"<4, false", "<4, true"}),        # 470 of 64 n, two on a CU
-                                         (2000, 200, 37, {"<16, false", "<8, true"})])      # 250 of 256 n, one round; 250 of 128 n, one round
-def test_each_launch_of_a_call_has_its_own_tile(device, f16_route, M, N, O, tiles):
-    """The blocks of 16 outputs and the rest of up to 8 are launches one behind the other."""
-    zeros = [torch.zeros(rows, columns, device=device) for rows, columns in ((40, M), (N, 40), (O, 40), (N, M))]
+@pytest.mark.parametrize("M,N,O,K,tiles", [(4000, 520, 24, 2000, {"12, false", "12, true"}),    # two launches of 750 tiles of 192 n, three rounds each
+                                           (4090, 250, 24, 500, {"16, false", "16, true"}),     # 256 of 256 n: one
+                                           (1500, 300, 17, 500, {"4, false", "4, true"}),       # 470 of 64 n, two on a CU
+                                           (2000, 200, 37, 2000, {"16, false", "8, true"}),     # 250 of 256 n, one round; 250 of 128 n, one round
+                                           (2794, 344, 24, 838, {"12, false"}),                 # one launch of 700 of 192 n, three rounds instead of four
+                                           (3264, 304, 16, 800, {"4, false"}),                  # 1020 of 64 n, two on a CU, fill their rounds better than 408 of 192 n
+                                           (9000, 200, 16, 800, {"16, false"})])                # 563 of 256 n
+def test_each_launch_of_a_call_has_its_own_tile(device, f16_route, M, N, O, K, tiles):
+    """The blocks of 16 outputs and the rest of up to 8 are launches one behind the other, unless one launch fills its rounds better."""
+    zeros = [torch.zeros(rows, columns, device=device) for rows, columns in ((K, M), (N, K), (O, K), (N, M))]
     names = kernels_of(lambda: kermac.cdist_grad(*zeros, p=1.0))
-    assert {tile for tile in tiles if any("norm_gradient_l1_f16" + tile in name for name in names)} == tiles, names
+    assert {tile for name in names for tile in re.findall(r"norm_gradient_l1_f16<(\d+, \w+)>", name)} == tiles, names
