@@ -267,7 +267,7 @@ def bench_cdist_grad(kermac, device, args, steps=None, warmup=None):
     log(f"  p=2, same operands: {l2_ms:.2f} ms (slab err {l2_err:.2e}); on the fp32 matrix-core kernel {l2_fp32_ms:.2f} ms ({l2_fp32_err:.2e})")
     check_parity("cdist_grad p=2 slab, max abs err / mean |truth|", l2_err, 1e-4)
     check_parity("cdist_grad p=2 (fp32 kernels) slab, max abs err / mean |truth|", l2_fp32_err, 1e-4)
-    # Beside it: 32 outputs, p = 1 (the tile of 16 n x 32 outputs: the sign work is shared by two blocks of outputs).
+    # Beside it: 32 outputs, p = 1 (two blocks of 16; the ranking of b and d serves both).
     c32 = torch.randn(32, k_ref, device=device)
     out32 = torch.empty(1, 32, n_ref, m_ref, device=device)
     truth32 = torch.einsum("ok,km,nmk->onm", c32.double(), a[:, ms].double(), sign)
@@ -285,7 +285,7 @@ def bench_cdist_grad(kermac, device, args, steps=None, warmup=None):
     log(f"  p=1, 32 outputs: {o32_ms:.2f} ms (slab err {o32_err:.2e}); on the fp32 matrix-core kernel {o32_fp32_ms:.2f} ms")
     check_parity("cdist_grad p=1, 32 outputs, slab, max abs err / mean |truth|", o32_err, 1e-4)
     # Executed matrix work on the default route: two products (the signs as 0 or 1, times a c in two fp16 pieces), 2 * O flops
-    # each per (m, n, k), against the dense fp16 peak; vector instructions beside the matrix ones (3.3 for each) are what bounds it.
+    # each per (m, n, k), against the dense fp16 peak; vector instructions beside the matrix ones (3.7 for each) are what bounds it.
     ops = 2.0 * 2.0 * o * m_ref * n_ref * k_ref
     nbytes = 4.0 * (k_ref * m_ref + n_ref * k_ref + o * k_ref + n_ref * m_ref + o * n_ref * m_ref)
     return side_line("cdist_grad ms, Laplace-kernel RFM gradient M=8192 N=512 O=16 K=8192 p=1",

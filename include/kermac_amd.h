@@ -338,10 +338,10 @@ typedef struct kmc_norm_gradient_params {
      * aligned, of at least the size kmc_norm_gradient_workspace_bytes reports for these parameters.
      * With it, large problems run on the fp16 matrix instruction.  KMC_NORM_L1: the rows n of b and d are
      * ranked, so that d >= b is a comparison of 16-bit numbers, 0 or 1 and exact; its product with a * c, in two fp16
-     * pieces (a power-of-two scale per m and o from the largest |a c| over k), takes 2 matrix instructions per 32 k where the
+     * pieces (a power-of-two scale per m and o from sums of |a c| over parts of k), takes 2 matrix instructions per 32 k where the
      * fp32 kernel issues 8 of twice the duration.  Error of e from the pieces below
-     * 2^-21 sum_k |c a| + k * 2^-38 max_k |c a|, so below 3 * 2^-22 sum_k |c a| up to k = 2^16, beside the rounding of the fp32
-     * accumulation that both kernels have.
+     * 2^-21 sum_k |c a| + k * 2^-38 times the largest sum of |c a| over 128 k in a row, so below 3 * 2^-22 sum_k |c a| up to k = 2^16,
+     * beside the rounding of the fp32 accumulation that both kernels have.
      * KMC_NORM_L2 with e_ld_o = n * e_ld_n (the planes of e one matrix of o * n rows): large problems
      * run as e = (d - s) g - p a with g[m][o] = sum_k a c, p[o n_rows + n][k] = c[o][k] (b[n][k] - s[n])
      * and s[n] the mean of row n of b (any s gives the same e; this one keeps both terms as small

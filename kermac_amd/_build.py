@@ -160,8 +160,8 @@ def build_c_example(verbose: bool = False) -> Path:
 
 if __name__ == "__main__":
     # python -m kermac_amd._build [--incremental] [-v] [--define NAME[=VALUE]]... [--output PATH]
-    # --define / --output build a variant of the library elsewhere (the measurement switches of the kernel headers,
-    # e.g. --define NGF_ABLATE_NO_SIGN --output /tmp/no_sign/libkermac_amd.so; KERMAC_AMD_LIBRARY=PATH then loads it)
+    # --define / --output build a variant of the library elsewhere (the tunable constants of the kernel headers,
+    # e.g. --define GB_WAVES=3 --output /tmp/waves/libkermac_amd.so; KERMAC_AMD_LIBRARY=PATH then loads it)
     arguments = sys.argv[1:]
     defines, output = [], None
     while "--define" in arguments:

@@ -443,14 +443,15 @@ struct GradientL2Layout {
     int64_t bytes;
 };
 
-// The route pays where a model of both times says so by 15 %, in microseconds, fitted to sweeps:
+// The route pays where a model of both times says so by 15 %, in microseconds, fitted to sweeps with the kernels of the route before the present
+// ones (which make the pieces of the products straight from b and c and walk faster, so the rule leaves a few calls to the fp32 kernels
+// that the route would win, and takes none that it loses):
 //   fp32 kernels   30 + terms * t(o) with terms = m n k l and t(o) = 0.077, 0.10, 0.126, 0.137 ps for 1 .. 4
 //                  outputs, 0.028 o up to 8 (vector kernels), 0.27 up to 16, 0.56 up to 32, 0.0175 o beyond
 //                  (matrix-core kernels: a run of outputs costs what its 16 or 32 columns cost);
-//   this route     200 + 1.5e-6 (o n + m) k l for the products and the two splits, and for the walk
-//                  6.3e-9 per multiply-add of the padded tiles but not less than 0.056 k (fitted to the product kernel before
-//                  the present tiles: 1.7 us per 256 x 256 x 16 step of a CU with the chip full, 0.9 us alone; the present one takes
-//                  4.7e-9 with the chip full, so the rule leaves a few calls to the fp32 kernels that it would win).
+//   this route     200 + 1.5e-6 (o n + m) k l for the products in fp32 and the two splits, and for the walk
+//                  6.3e-9 per multiply-add of the padded tiles but not less than 0.056 k (1.7 us per 256 x 256 x 16 step of a CU
+//                  with the chip full, 0.9 us alone; the present kernel takes 4.7e-9 with the chip full).
 // Examples (fp32 / this route, measured with the present kernel): 8192 x 512 x 16 x 8192 3.0; o = 1 4.3, o = 32 3.2; n = 64 1.65;
 // m = 1024 1.6; k = 512 1.8, k = 256 1.2; 10000 x 1000 x 10 x 784 3.4.  With the kernel before: n = 32 0.96, n = 8 0.81;
 // m = 512 0.86; k = 64 0.40.  KERMAC_AMD_GRADIENT_L2_MIN_TERMS replaces the rule by a number of terms

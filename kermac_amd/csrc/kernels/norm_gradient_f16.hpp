@@ -35,7 +35,7 @@
 // thirds of them the cheap ones of fp32.
 // Bound by the two together: on registers alone a v_mfma_f32_16x16x32_f16 takes 16.5 cycles, 16.9 with two packed
 // subtractions beside it, and four more for every further packed instruction; the kernel takes about 26.
-// Measured at M = K = 8192, N = 512, O = 16: 1.95 ms with 0.20 ms of gradient_signs_prepare (3.65 ms for the kernel that
+// Measured at M = K = 8192, N = 512, O = 16: 1.94 ms with 0.18 ms of gradient_signs_prepare (3.65 ms for the kernel that
 // flipped the sign into both pieces of A: three products and 2.5 vector instructions per term), O = 32 3.75 ms (5.55).  W from
 // pieces of A and C under a scale per row each, which loses bits as said above, took 1.94 and 3.70.
 // Up to 8 outputs leave half of the columns unused: there the columns 8 .. 15 take the second pieces (PIECES_IN_COLUMNS),
@@ -302,7 +302,8 @@ __device__ __forceinline__ int signs_sum_at(int m)
 // the first only that) sum_k |a c| per m and o, the largest of four quarters of the k.  No |a c| is above its sum, and the sum, unlike a
 // maximum, is work for the matrix instruction: v_mfma_f32_4x4x4_16B_bf16 takes 4 k of a lane's own row with 4 outputs, which are read as broadcasts
 // of LDS.  (bfloat16 has the range of fp32; rounded down, |a|, |c| and the sum are up to 2.4 % too small.)  A lane holds 2 m and 16 k at a time,
-// which are 128 bytes of the copy; a wave takes a quarter of the k.
+// which are 128 bytes of the copy; a wave takes a quarter of the k.  Memory-bound together with the sorts beside it.  The launch with the maxima on the
+// vector ALU and stores of 16 bytes per lane / now, us: 8192 x 512 x 16 x 8192 197 / 179, 2 x 3200 x 32 x 10 x 10432 154 / 119, 4000 x 32 x 128 x 4000 126 / 67.
 __device__ __forceinline__ void signs_copy_tile(const GradientPrepareArgs &args, int block, int batch, unsigned *shared)
 {
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);

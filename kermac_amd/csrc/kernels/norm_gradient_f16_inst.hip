@@ -36,13 +36,14 @@ int64_t place(int64_t &cursor, int64_t bytes)
 int64_t round_up(int64_t value, int64_t multiple) { return (value + multiple - 1) / multiple * multiple; }
 
 // The route pays where the fp32 kernels are bound by their matrix or vector instructions: enough
-// terms to carry the five extra launches, and more than two outputs (its cost does not fall below
-// that of 16 outputs; the vector kernel for one or two is cheaper).  From sweeps, fp32 / fp16 time:
-// O = 16 at 3.4e10 terms 2.5, 1.1e9 1.8, 5.4e8 1.1 .. 1.4, 2.7e8 0.8 .. 1.1, 1.3e8 0.66; at 3.4e10
-// terms O = 1 0.73, O = 2 0.93, O = 3 1.21, O = 4 1.31, O = 8 2.1, O = 17 1.7, O = 48 2.6; with few
-// outputs the fp32 kernels are cheaper by nearly that factor and the route is not (16 results per
-// tile whatever O), so the terms are asked for in proportion: 4e8 at 16 outputs, 1.6e9 at 4.  Its
-// tiles hold 32 columns of the result: N = 8 0.90, N = 16 0.86, N = 32 1.37, N = 33 1.49.
+// terms to carry the extra launch and the ranking, and more than two outputs (a workgroup costs the same for 1 .. 8 and for
+// 9 .. 16 outputs; the vector kernel for one or two is cheap).  Few outputs make the fp32 kernels cheaper nearly in proportion and not the
+// route, so the terms are asked for in proportion: 4e8 at 16 outputs, 1.6e9 at 4.  Its smallest tile holds 32 n.
+// The limits are those of the kernel before this one, which needed five more launches and a third matrix instruction, fp32 / that kernel's time:
+// O = 16 at 3.4e10 terms 2.5, 1.1e9 1.8, 5.4e8 1.1 .. 1.4, 2.7e8 0.8 .. 1.1, 1.3e8 0.66; at 3.4e10 terms O = 1 0.73, O = 2 0.93, O = 3 1.21, O = 4
+// 1.31, O = 8 2.1; N = 16 0.86, N = 32 1.37.  Of 57 shapes that they send down the route the present kernel is 1.55 times as fast as the fp32
+// kernels or more (11200 x 112 x 16 x 320 1.55, 4000 x 32 x 16 x 4000 1.80, 6862 x 105 x 24 x 417 1.96): they lose nothing, and leave calls to
+// the fp32 kernels that the route would win.
 // KERMAC_AMD_GRADIENT_F16_MIN_TERMS replaces the conditions by a number of terms (read on every
 // call, so that a test can send small shapes down the route).
 bool f16_pays(const kmc_norm_gradient_params *p)
@@ -51,9 +52,8 @@ bool f16_pays(const kmc_norm_gradient_params *p)
     const double forced = text ? std::atof(text) : 0.0;
     const double terms = static_cast<double>(p->m) * p->n * p->k * p->l;
     if (forced > 0.0) return terms >= forced;
-    // more than 16 outputs: the wider tiles of the route share the sign work between blocks of outputs, while the
-    // fp32 kernels go to their 32-column tiles (O = 32: 98 against 75 us at 1.7e7 terms, 187 against 128 at 2.7e8;
-    // O = 128: 101 against 70 and 588 against 206)
+    // more than 16 outputs: the ranking serves all blocks of outputs, while the fp32 kernels go to their 32-column tiles (fp32 / route, us:
+    // 704 x 48 x 32 x 1024, 3.5e7 terms, 102 / 59; 832 x 352 x 128 x 320, 9.4e7, 250 / 122; 576 x 48 x 64 x 2816, 7.8e7, 218 / 131)
     namespace r = kmc_rules;
     if (p->o > 16) return p->n >= r::GRADIENT_F16_MIN_N && terms >= static_cast<double>(r::GRADIENT_F16_MANY_OUTPUTS_MIN_TERMS);
     return p->o >= r::GRADIENT_F16_MIN_OUTPUTS && p->n >= r::GRADIENT_F16_MIN_N &&

@@ -115,7 +115,7 @@ _ROWS = (
     ("`cdist_grad`, p = 1",
      "O ≥ {GRADIENT_F16_MIN_OUTPUTS}, N ≥ {GRADIENT_F16_MIN_N}, terms · O ≥ {GRADIENT_F16_MIN_TERMS_TIMES_OUTPUTS}; with O > 16: terms ≥ "
      "{GRADIENT_F16_MANY_OUTPUTS_MIN_TERMS}",
-     "`gradient_signs_prepare` (rows of b and d ranked, a and c copied, largest products), `norm_gradient_l1_f16` (16 outputs a tile; 8 with both pieces in its columns)"),
+     "`gradient_signs_prepare` (rows of b and d ranked, a and c copied, bounds of their products), `norm_gradient_l1_f16` (16 outputs a tile; 8 with both pieces in its columns)"),
     ("`cdist_grad`, p = 2", "a model of both times favours the route by {GRADIENT_L2_ADVANTAGE_PERCENT} %, and the planes of `out` form one matrix",
      "`gradient_l2_prepare`, `gradient_l2_pieces_stats` and `_split`, `gram_f16_wide<GW_EPILOGUE_GRADIENT_L2>`"),
     ("`cdist_grad`, otherwise", "O ≤ 8 / O > 8", "`norm_kernel_gradient` (vector ALU) / `norm_kernel_gradient_mfma` (fp32 matrix instruction), in runs of 32, 16 and ≤ 8 outputs; "

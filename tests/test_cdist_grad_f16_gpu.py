@@ -1,6 +1,6 @@
 """GPU tests of the route that large L1 gradients take when the caller brings a workspace
-(include/kermac_amd.h, kmc_norm_gradient_params::workspace): a and c split once into two fp16
-pieces per value with a power-of-two scale per row, the sign of d - b put on the pieces of a, the
+(include/kermac_amd.h, kmc_norm_gradient_params::workspace): the rows of b and d ranked, d >= b as an
+exact 0 or 1, times a c in two fp16 pieces with a power-of-two scale per row m and output, the
 contraction on the fp16 matrix instruction.  Tolerance as for the other gradient kernels: the
 result is a signed sum of K products, |got - truth| <= 1e-5 |truth| + 1e-4 mean |truth|.
 
