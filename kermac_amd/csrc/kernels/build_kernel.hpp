@@ -309,8 +309,8 @@ __device__ __forceinline__ void row_square_diff(float (&accrow)[8], const float 
 // three before, the accumulation of the one five before.  Every instruction that reads the result
 // of a transcendental one has at least one other in between, the wait state it needs.  The loop is
 // bound by the issue of the two transcendentals (8.5 cycles each of about 28 per element); 10000 x
-// 10000 x 1024: with the five steps as groups of 8 instructions 19.3 ms, in this order 19.1; the
-// pipeline kept running from row to row of the register tile 19.2.
+// 10000 x 1024: with the five steps as groups of 8 instructions 19.3 ms, in this order 19.1, about as
+// much as runs on different days differ; the pipeline kept running from row to row of the register tile 19.2.
 __device__ __forceinline__ void row_pow_diff(float (&accrow)[8], const float (&fa)[8], float b, float p)
 {
     float t0, t1, t2, t3, t4, t5, t6, t7;
