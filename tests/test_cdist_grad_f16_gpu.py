@@ -216,7 +216,8 @@ def _beside_large_values(kind, M, O, K, g):
 @pytest.mark.parametrize("kind", ["one c of 2^16 that meets a = 0", "one a of 1 that meets c = 0, the others 2^-16",
                                   "a Laplace kernel: 1 that meets c = 0, beside exp(-20 +- 3)", "one of 1 in each, apart, the others 2^-14",
                                   "neighbours of 1 in each that meet 0, the others 2^-30", "outputs that see different rows of a"])
-@pytest.mark.parametrize("M,N,O,K", [(70, 40, 16, 64), (130, 300, 5, 100), (40, 70, 20, 130), (4000, 150, 9, 40), (33, 40, 40, 600)])
+@pytest.mark.parametrize("M,N,O,K", [(70, 40, 16, 64), (130, 300, 5, 100), (40, 70, 20, 130), (4000, 150, 9, 40), (33, 40, 40, 600),
+                                     (9000, 25, 120, 1100)])     # ranges of 512 k and a rest for the scales of W
 @pytest.mark.parametrize("powers", [(0, 0), (100, -60), (-60, 100)])
 def test_small_products_beside_large_values(device, f16_route, kind, M, N, O, K, powers):
     """The error of every element is bounded by its own sum of |c a|, however small that is beside max |a| max |c|: 3 * 2^-22 of it
