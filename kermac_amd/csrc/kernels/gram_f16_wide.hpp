@@ -571,6 +571,12 @@ __device__ __forceinline__ void wide_lanes_exchange()
 // The matrix instructions are written out: left to itself the compiler gives their results other registers than their
 // sums came from, which does not fit beside the operands.  Two products into the same sums are at least 16 matrix
 // instructions apart (8 in EightWaves), and the walk ends with the wait states that vector instructions need before they read the sums.
+// The blocks are walked back and forth, so that an instruction always shares one operand with the one in front of it: the board
+// is power-limited here and a new operand costs energy.  With every row of blocks walked from its first, and now: 30000 x 30000 x 1024 4908 -> 4878 us,
+// 1000 x 60000 x 784 and its product 452 -> 449, where two runs differ by 0.2 %; four pairs of runs of the gradient at 2 x 10000 x 768 x 16 x 10000
+// 0.8 .. 1.5 % apart, a fifth level.  (Columns of blocks back and forth, where the first operand changes more often: half of that; column by column without
+// turning: nothing.  Tiles of 128 x 256, 64 x 128 per wave: level, but 13.3 against 12.5 ms for the gradient, whose epilogue fetches more; of 256 x 256 by 8
+// waves, one workgroup per CU: 2 .. 5 % slower, also at K = 10000.)
 // The compiler, which keeps such distances for instructions it knows, does not see these: nothing else may read or move a sum between
 // the first product and those wait states, which holds as long as the sums stay where they are (the test of the kernel's listing
 // looks at every instruction in between).
@@ -580,8 +586,10 @@ __device__ __forceinline__ void wide_multiply(gram_float4 (&acc)[MT][NT], const 
 #pragma unroll
     for (int mt = FIRST; mt < LAST; mt++)
 #pragma unroll
-        for (int nt = 0; nt < NT; nt++)
+        for (int turn = 0; turn < NT; turn++) {
+            const int nt = mt % 2 == 0 ? turn : NT - 1 - turn;
             asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(acc[mt][nt]) : "v"(fa[mt]), "v"(fb[nt]));
+        }
 }
 
 template <typename Tile>
