@@ -165,7 +165,12 @@ enum kmc_flags {
      * (4 bytes per element of the padded copies).  Without a workspace, or for a call the query reports 0
      * for, the direct kernels run on the operands as they are.  The reference has one kernel for all
      * storage orders (include/build_a_kernel.cuh:484-539). */
-    KMC_FLAG_DIRECT_PANELS = 2048
+    KMC_FLAG_DIRECT_PANELS = 2048,
+    /* With KMC_FLAG_L2_GRAM_BF16 and gram_workspace (ignored by a launch that does not go through the workspace): the
+     * call makes the centre itself, in the workspace, from up to 512 rows of a spread over the panel (per batch entry, or
+     * once where a_bs is 0), subtracts it where kmc_sample_mean's flag would say so, and does not read gram_centre.
+     * kmc_gram_workspace_bytes counts the room for it.  One launch instead of the two of kmc_sample_mean. */
+    KMC_FLAG_GRAM_OWN_CENTRE = 4096
 };
 
 /*

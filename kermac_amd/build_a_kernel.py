@@ -654,8 +654,7 @@ def run_kernel(
         plan.keepalive.append(workspace)
     cut = _cut_over_contraction(params)
     if params.flags & (_backend.FLAG_L2_GRAM | _backend.FLAG_L2_GRAM_BF16):
-        plan.keepalive.append(_attach_gram_centre(params, stream, a.device))
-        plan.keepalive.append(_attach_gram_workspace(params, a.device))
+        plan.keepalive.append(_attach_gram_memory(params, stream, a.device))
     elif (cut is None and not params.flags & (_backend.FLAG_DOT_PIECES | _backend.FLAG_L1_FIXED)
             and params.inner_operator == _backend.OP_DIFF
             and (params.inner_power in (_backend.POW_ABS, _backend.POW_SQUARE)
@@ -687,12 +686,30 @@ def _direct_panels_min_tiles() -> int:
     return int(_backend.dispatch_rules()["DIRECT_PANELS_MIN_TILES"])
 
 
+def _attach_gram_memory(params, stream, device):
+    """What a matrix-core launch for squared differences takes beside its operands: the workspace, and the centre, which the
+    route through the workspace makes for itself in there (include/kermac_amd.h, KMC_FLAG_GRAM_OWN_CENTRE)."""
+    if _centre_wanted():
+        params.flags |= _backend.FLAG_GRAM_OWN_CENTRE
+    needed = _backend.gram_workspace_bytes(params)
+    if needed:
+        workspace = _attach_gram_workspace(params, device, needed=needed)
+        if workspace is not None:
+            return workspace
+    params.flags &= ~_backend.FLAG_GRAM_OWN_CENTRE         # a one-step kernel
+    return _attach_gram_centre(params, stream, device), _attach_gram_workspace(params, device)
+
+
+def _centre_wanted():
+    return os.environ.get("KERMAC_AMD_L2_CENTRE", "1") not in ("", "0")
+
+
 def _attach_gram_centre(params, stream, device):
     """Matrix-core launches subtract a point near the data from both operands while staging them
     (include/kermac_amd.h, gram_centre): the mean of a sample of the rows of the first operand,
     computed by the library into a small buffer allocated here.  KERMAC_AMD_L2_CENTRE=0 keeps the
     operands as they are."""
-    if os.environ.get("KERMAC_AMD_L2_CENTRE", "1") in ("", "0") or params.m == 0 or params.k == 0 or params.l == 0:
+    if not _centre_wanted() or params.m == 0 or params.k == 0 or params.l == 0:
         return None
     # per batch entry: the centre padded to a multiple of 64 floats, a flag (subtract or not: the
     # library leaves it out when the centre is negligible against the spread) and the variances
@@ -820,16 +837,17 @@ def _workspace_route_applies(params, flags):
 _L2_SAMPLE_MIN_TERMS = 4_000_000_000
 
 
-def _attach_gram_workspace(params, device, switch="KERMAC_AMD_L2_WORKSPACE"):
+def _attach_gram_workspace(params, device, switch="KERMAC_AMD_L2_WORKSPACE", needed=None):
     """Large squared-difference problems in the split-bf16 mode go through a workspace (include/
     kermac_amd.h, gram_workspace: both operands split once into fp16 pieces, then their products);
     the library says how much it wants for this call, 0 when it would not use one.
-    KERMAC_AMD_L2_WORKSPACE=0 keeps every call on the one-step kernel."""
+    KERMAC_AMD_L2_WORKSPACE=0 keeps every call on the one-step kernel.  `needed`: what the library says, if the caller has asked."""
     if os.environ.get(switch, "1") in ("", "0"):
         return None
     if os.environ.get("KERMAC_AMD_L2_PROBE", "1") in ("", "0"):
         params.flags |= _backend.FLAG_NO_PROBE      # no sample of the result in front of the matrix-core kernel
-    needed = _backend.gram_workspace_bytes(params)
+    if needed is None:
+        needed = _backend.gram_workspace_bytes(params)
     if (needed == 0 and (params.flags & (_backend.FLAG_L2_GRAM | _backend.FLAG_L2_GRAM_BF16)) and not (params.flags & _backend.FLAG_NO_PROBE)
             and params.m * params.n * params.k * params.l >= _L2_SAMPLE_MIN_TERMS):
         needed = _backend.SAMPLE_BYTES              # a one-step kernel: room for the sample that is taken in front of it

@@ -160,7 +160,7 @@ int64_t gram_f16_wide_bytes(const kmc_build_kernel_params *p, const kmc::BuildKe
 hipError_t launch_gram_f16_wide(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &args, hipStream_t stream, bool *taken,
                                 const unsigned **sample = nullptr);
 hipError_t launch_scalar_b_if_the_sample_leaves(int load_a, int load_b, const kmc::BuildKernelArgs &args, hipStream_t stream, bool *launched);
-hipError_t launch_gram_probe(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &args, unsigned *sample, hipStream_t stream);
+hipError_t launch_gram_probe(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &args, unsigned *sample, int centre_pairs, hipStream_t stream);
 int64_t l1_fixed_bytes(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &args);
 hipError_t launch_l1_fixed(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &args, hipStream_t stream, bool *taken);
 int64_t direct_panels_bytes(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &args);
@@ -262,7 +262,7 @@ int kmc_build_kernel(const kmc_build_kernel_params *params, void *stream)
             if (!(params->flags & KMC_FLAG_NO_PROBE) && params->gram_workspace && params->gram_workspace_bytes >= KMC_SAMPLE_BYTES &&
                 (reinterpret_cast<uintptr_t>(params->gram_workspace) & 255) == 0 && args.k > 0) {
                 unsigned *sample = static_cast<unsigned *>(params->gram_workspace);
-                g = launch_gram_probe(params, args, sample, static_cast<hipStream_t>(stream));
+                g = launch_gram_probe(params, args, sample, 0, static_cast<hipStream_t>(stream));
                 if (g != hipSuccess) return fail_hip(g, "gram_probe_operands launch");
                 args.sample = sample;
             }

@@ -65,6 +65,7 @@ struct GramRowsArgs {
     const float *x; i64 ld, bs;
     int rows, k, row_major, vec;          // vec: 128-bit loads along k are allowed (row-major only)
     const float *centre; i64 centre_bs;   // as BuildKernelArgs::centre, or null
+    int centre_pairs;                     // as GramProbeArgs
     gram_chunk *pieces; i64 pieces_bs;    // per batch entry, in chunks
     float *squares; float *magnitudes;    // [batch][range][rows_pad]
     float *unscale;                       // [batch][rows_pad]: 1 / the row's scale
@@ -132,6 +133,11 @@ __device__ __forceinline__ const float *gram_rows_centre(const GramRowsArgs &arg
 {
     if (!args.centre) return nullptr;
     const float *centre = args.centre + batch * args.centre_bs;
+    if (args.centre_pairs) {
+        CentreSums sums;
+        sums.load(centre, args.k, args.centre_pairs);
+        return sums.needless() ? nullptr : centre;
+    }
     const int padded = (args.k + GRAM_CENTRE_PAD - 1) / GRAM_CENTRE_PAD * GRAM_CENTRE_PAD;
     return centre[padded] != 0.0f ? centre : nullptr;      // the flag behind the vector: see centre_to_subtract
 }
@@ -301,7 +307,9 @@ __device__ __forceinline__ void gram_rows_once_of(const GramRowsArgs &args, int 
     const int row = block * GRO_ROWS + r, batch = blockIdx.z;
     const bool live = row < args.rows;
     const float *src = args.x + batch * args.bs + (i64)(live ? row : args.rows - 1) * args.ld;
-    const float *centre = gram_rows_centre(args, batch);
+    const float *centre = args.centre ? args.centre + batch * args.centre_bs : nullptr;
+    CentreSums sums;
+    if (centre && args.centre_pairs) sums.load(centre, args.k, args.centre_pairs);
     const int groups = (args.k + 63) / 64;
     const int k0 = BK_TILE_K * wave + 4 * quarter;             // and every 64 behind it
     float v[GROUPS][4];
@@ -319,7 +327,7 @@ __device__ __forceinline__ void gram_rows_once_of(const GramRowsArgs &args, int 
 #pragma unroll
             for (int e = 0; e < 4; e++) v[g][e] = src[min(64 * g + k0 + e, args.k - 1)];
     }
-    if (centre) {
+    if (centre && args.centre_pairs ? !sums.needless() : gram_rows_centre(args, batch) != nullptr) {
         // padded with zeros to whole groups of 64 k
         const bool aligned = (reinterpret_cast<unsigned long>(centre) & 15) == 0;
         const int last = 64 * (groups - 1);

@@ -35,6 +35,8 @@ struct WideLayout {
     int tiles_m, tiles_n;       // of GW_TILE x GW_TILE
     OperandRegions a, b;
     int64_t sample;         // byte offset of the words of gram_probe_operands
+    int64_t centre = 0, centre_floats = 0;      // byte offset of the centre that the route takes for itself, floats per batch entry (0: it takes none)
+    int centre_batches = 1;
     int64_t bytes;
 };
 
@@ -138,6 +140,8 @@ bool place_wide(int m, int n, int k, int l, bool a_shared, bool b_shared, bool a
     int64_t cursor = 0;
     const bool fits = k <= kmc::GRO_MAX_K;
     place_operand(layout->a, m, a_shared, l, a_rows && fits, *layout, cursor);
+    // behind the region of a, where it stays when b grows or shrinks: the split of a may be kept
+    layout->centre = layout->centre_floats ? place(cursor, 4 * layout->centre_floats * layout->centre_batches) : 0;
     if (symmetric) layout->b = layout->a;      // one panel, split once
     else place_operand(layout->b, n, b_shared, l, b_rows && fits, *layout, cursor);
     layout->sample = place(cursor, kmc::BK_SAMPLE_BYTES);
@@ -161,13 +165,17 @@ bool wide_layout(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &a
     if (!asked_for && !wide_pays(args.m, args.n, layout->tiles_m, layout->tiles_n, tiles * args.l, args.k, products, k_contiguous, args.l > 1, args.symmetric)) return false;
     // an operand that is the same for every batch entry is split once, unless the centre differs
     // (products have no centre: the caller's parameter block carries none into `args`)
-    const bool one_centre = products || !args.centre || args.centre_bs == 0;
+    const bool own_centre = squared_differences && (p->flags & KMC_FLAG_GRAM_OWN_CENTRE);
+    layout->centre_batches = own_centre && args.a_bs != 0 ? args.l : 1;
+    layout->centre_floats = own_centre ? 2 * ((args.k + kmc::GRAM_CENTRE_PAD - 1) / kmc::GRAM_CENTRE_PAD * kmc::GRAM_CENTRE_PAD) + kmc::GRAM_CENTRE_PAD : 0;
+    const bool one_centre = products || (own_centre ? layout->centre_batches == 1 : !args.centre || args.centre_bs == 0);
     return place_wide(args.m, args.n, args.k, args.l, args.a_bs == 0 && one_centre, args.b_bs == 0 && one_centre,
                       p->a_majorness == KMC_ROW_MAJOR, p->b_majorness == KMC_ROW_MAJOR, args.symmetric, layout);
 }
 
 kmc::GramRowsArgs rows_args(const float *x, int64_t ld, int64_t bs, int rows, int majorness, bool scalar_only,
-                            const kmc::BuildKernelArgs &args, const WideLayout &layout, const OperandRegions &r, char *workspace)
+                            const kmc::BuildKernelArgs &args, const WideLayout &layout, const OperandRegions &r, char *workspace,
+                            int centre_pairs = 0)
 {
     kmc::GramRowsArgs rows_of = {};
     rows_of.x = x; rows_of.ld = ld; rows_of.bs = bs;
@@ -175,6 +183,7 @@ kmc::GramRowsArgs rows_args(const float *x, int64_t ld, int64_t bs, int rows, in
     rows_of.row_major = majorness == KMC_ROW_MAJOR;
     rows_of.vec = rows_of.row_major && !scalar_only && aligned16(x) && ld % 4 == 0 && bs % 4 == 0;
     rows_of.centre = args.centre; rows_of.centre_bs = args.centre_bs;
+    rows_of.centre_pairs = centre_pairs;
     rows_of.pieces = reinterpret_cast<kmc::gram_chunk *>(workspace + r.pieces); rows_of.pieces_bs = r.pieces_bs;
     rows_of.squares = reinterpret_cast<float *>(workspace + r.squares);
     rows_of.magnitudes = reinterpret_cast<float *>(workspace + r.magnitudes);
@@ -232,8 +241,10 @@ void forget_split_in(const void *workspace)
 }
 
 // Statistics and split of one operand (also used by the gradient's fp16 route).
-hipError_t launch_gram_probe(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &args, unsigned *sample, hipStream_t stream);   // gram_probe.hip
-kmc::GramProbeArgs gram_probe_args(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &args, unsigned *sample);                 // gram_probe.hip
+hipError_t launch_gram_probe(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &args, unsigned *sample, int centre_pairs, hipStream_t stream);   // gram_probe.hip
+kmc::GramProbeArgs gram_probe_args(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &args, unsigned *sample, int centre_pairs);                 // gram_probe.hip
+hipError_t launch_route_centre(const float *x, int majorness, int rows, int k, int64_t ld, int64_t bs, int l, float *mean, int64_t mean_bs, hipStream_t stream);   // sample_mean.hip
+int route_centre_pairs(int majorness, int rows, int k, int l);                                                                                                    // sample_mean.hip
 
 hipError_t launch_gram_rows(const kmc::GramRowsArgs &rows_of, int batches, hipStream_t stream)
 {
@@ -363,9 +374,10 @@ int64_t gram_f16_wide_bytes(const kmc_build_kernel_params *p, const kmc::BuildKe
 
 // Row statistics and split of both operands, then the product kernel.  `*taken` says whether the
 // path applied (and the launches were made); if not, nothing was launched.
-hipError_t launch_gram_f16_wide(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &args, hipStream_t stream, bool *taken,
+hipError_t launch_gram_f16_wide(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &as_given, hipStream_t stream, bool *taken,
                                 const unsigned **sample_taken)
 {
+    kmc::BuildKernelArgs args = as_given;
     *taken = false;
     if (sample_taken) *sample_taken = nullptr;
     WideLayout layout;
@@ -374,8 +386,14 @@ hipError_t launch_gram_f16_wide(const kmc_build_kernel_params *p, const kmc::Bui
         return hipSuccess;
     char *workspace = static_cast<char *>(p->gram_workspace);
     const bool scalar_only = (p->flags & KMC_FLAG_FORCE_SCALAR_ACCESS) != 0;
-    const kmc::GramRowsArgs rows_a = rows_args(args.a, args.a_ld, args.a_bs, args.m, p->a_majorness, scalar_only, args, layout, layout.a, workspace);
-    const kmc::GramRowsArgs rows_b = rows_args(args.b, args.b_ld, args.b_bs, args.n, p->b_majorness, scalar_only, args, layout, layout.b, workspace);
+    const bool own_centre = layout.centre_floats != 0;
+    if (own_centre) {
+        args.centre = reinterpret_cast<float *>(workspace + layout.centre);
+        args.centre_bs = layout.centre_batches > 1 ? layout.centre_floats : 0;
+    }
+    const int centre_pairs = own_centre ? route_centre_pairs(p->a_majorness, args.m, args.k, layout.centre_batches) : 0;
+    const kmc::GramRowsArgs rows_a = rows_args(args.a, args.a_ld, args.a_bs, args.m, p->a_majorness, scalar_only, args, layout, layout.a, workspace, centre_pairs);
+    const kmc::GramRowsArgs rows_b = rows_args(args.b, args.b_ld, args.b_bs, args.n, p->b_majorness, scalar_only, args, layout, layout.b, workspace, centre_pairs);
     // The caller's trust rule grows with sqrt(k) (the error of a sum of k terms against the norms) and
     // passes 1 near k = 18000, where it would send every part to the repair launch -- whose own
     // fp32 sum over k is no better by then (measured at k = 20000 .. 200000: products of pieces, rounded once
@@ -395,9 +413,14 @@ hipError_t launch_gram_f16_wide(const kmc_build_kernel_params *p, const kmc::Bui
     const bool split_a = !a_is_kept, split_b = !args.symmetric;
     bool sampled = false;
     hipError_t status = hipSuccess;
+    // (a kept split of a was made around the centre that is still there)
+    if (own_centre && split_a)
+        status = launch_route_centre(args.a, p->a_majorness, args.m, args.k, args.a_ld, args.a_bs, layout.centre_batches,
+                                     reinterpret_cast<float *>(workspace + layout.centre), layout.centre_floats, stream);
+    if (status != hipSuccess) return status;
     if ((split_a && layout.a.once) || (split_b && layout.b.once)) {
         status = launch_gram_rows_once(split_a && layout.a.once ? &rows_a : nullptr, layout.a.batches, split_b && layout.b.once ? &rows_b : nullptr,
-                                       layout.b.batches, sample ? gram_probe_args(p, wide.kernel, sample) : kmc::GramProbeArgs{}, sample != nullptr, stream);
+                                       layout.b.batches, sample ? gram_probe_args(p, wide.kernel, sample, centre_pairs) : kmc::GramProbeArgs{}, sample != nullptr, stream);
         sampled = true;
     }
     if (status == hipSuccess && split_a && split_b && !layout.a.once && !layout.b.once) {
@@ -406,7 +429,7 @@ hipError_t launch_gram_f16_wide(const kmc_build_kernel_params *p, const kmc::Bui
         if (status == hipSuccess && split_a && !layout.a.once) status = launch_gram_rows(rows_a, layout.a.batches, stream);
         if (status == hipSuccess && split_b && !layout.b.once) status = launch_gram_rows(rows_b, layout.b.batches, stream);
     }
-    if (status == hipSuccess && sample && !sampled) status = launch_gram_probe(p, wide.kernel, sample, stream);
+    if (status == hipSuccess && sample && !sampled) status = launch_gram_probe(p, wide.kernel, sample, centre_pairs, stream);
     if (status != hipSuccess) return status;
     if (sample) {
         wide.kernel.sample = sample;

@@ -22,7 +22,7 @@ __global__ __launch_bounds__(GP_THREADS) void gram_probe_operands(const GramProb
 namespace kmc_host {
 
 // What the kernel needs for the problem of `p` (squared differences; m, n, k, l at least 1).
-kmc::GramProbeArgs gram_probe_args(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &args, unsigned *sample)
+kmc::GramProbeArgs gram_probe_args(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &args, unsigned *sample, int centre_pairs)
 {
     kmc::GramProbeArgs probe;
     probe.a = p->a; probe.b = p->b;
@@ -31,15 +31,16 @@ kmc::GramProbeArgs gram_probe_args(const kmc_build_kernel_params *p, const kmc::
     probe.b_k_contiguous = p->b_majorness == KMC_COL_MAJOR ? 0 : 1;
     probe.m = args.m; probe.n = args.n; probe.k = args.k; probe.l = args.l;
     probe.centre = args.centre; probe.centre_bs = args.centre_bs;
+    probe.centre_pairs = centre_pairs;
     probe.trust = args.gram_trust;
     probe.sample = sample;
     return probe;
 }
 
 // Fills sample[0 .. BK_SAMPLE_TILES) for the problem of `p` (squared differences; m, n, k, l at least 1).
-hipError_t launch_gram_probe(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &args, unsigned *sample, hipStream_t stream)
+hipError_t launch_gram_probe(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &args, unsigned *sample, int centre_pairs, hipStream_t stream)
 {
-    const kmc::GramProbeArgs probe = gram_probe_args(p, args, sample);
+    const kmc::GramProbeArgs probe = gram_probe_args(p, args, sample, centre_pairs);
     return launch(kmc::gram_probe_operands, dim3(kmc::BK_SAMPLE_TILES), dim3(kmc::GP_THREADS), stream, probe);
 }
 

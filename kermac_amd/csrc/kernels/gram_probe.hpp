@@ -26,8 +26,41 @@ struct GramProbeArgs {
     int a_k_contiguous, b_k_contiguous;
     int m, n, k, l;
     const float *centre; i64 centre_bs;        // as in BuildKernelArgs; the flag sits behind the padded centre
+    int centre_pairs;                          // > 0: no flag was stored, these many pairs say it (CentreSums)
     float trust;
     unsigned *sample;                          // [BK_SAMPLE_TILES]
+};
+
+// Whether subtracting the centre would lower the norms, and with them the error of the expansion, by under 2 %: |c|^2 against the variances.
+// sample_mean.hip leaves both as one pair of floats per workgroup of its own behind the centre ([centre, padded][64 unused][pairs]).  Every wave
+// adds them up in the same order, so that all of a call decide alike.  Data that are not numbers keep the subtraction (the
+// comparison is false), the repair decides.  In place of a launch that stores the answer for all: at 2000 x 2000 x 784 that
+// launch was 3 of 55 us on the stream, and one call of the host.  (From the means and variances of all k, by a workgroup with a barrier: 2 us dearer than the launch.)
+// (`load` in front of other loads, `needless` behind them, so that its wait is not one more round trip.)
+struct CentreSums {
+    float norm = 0.0f, spread = 0.0f;
+
+    __device__ __forceinline__ void load(const float *centre, int k, int pairs)
+    {
+        const float2 *pair = reinterpret_cast<const float2 *>(centre + (k + GRAM_CENTRE_PAD - 1) / GRAM_CENTRE_PAD * GRAM_CENTRE_PAD + GRAM_CENTRE_PAD);
+        const int q = threadIdx.x & 63;
+        const float2 of = pair[min(q, pairs - 1)];
+        norm = q < pairs ? of.x : 0.0f;
+        spread = q < pairs ? of.y : 0.0f;
+        for (int more = q + 64; more < pairs; more += 64) {
+            norm += pair[more].x;
+            spread += pair[more].y;
+        }
+    }
+    __device__ __forceinline__ bool needless()
+    {
+#pragma unroll
+        for (int offset = 32; offset > 0; offset >>= 1) {
+            norm += __shfl_xor(norm, offset);
+            spread += __shfl_xor(spread, offset);
+        }
+        return norm <= spread * (1.0f / 64.0f);
+    }
 };
 
 __device__ __forceinline__ float probe_element(const float *x, i64 ld, int k_contiguous, int row, int k)
@@ -54,7 +87,9 @@ __device__ __forceinline__ void gram_probe_tile(const GramProbeArgs &args, int t
     const float *a = args.a + batch * args.a_bs, *b = args.b + batch * args.b_bs;
     const int k_padded = (args.k + GRAM_CENTRE_PAD - 1) / GRAM_CENTRE_PAD * GRAM_CENTRE_PAD;
     const float *centre = args.centre ? args.centre + batch * args.centre_bs : nullptr;
-    if (centre && centre[k_padded] == 0.0f) centre = nullptr;        // the flag: this batch entry is taken as it is
+    CentreSums sums;
+    if (centre && args.centre_pairs) sums.load(centre, args.k, args.centre_pairs);
+    else if (centre && centre[k_padded] == 0.0f) centre = nullptr;        // the flag: this batch entry is taken as it is
 
     // Lane t fetches, for each run, one value of a and one of b: 16 rows x 16 k per run, along whichever
     // direction is contiguous.  Rows beyond the panel repeat its last row (a pair counted twice biases nothing
@@ -75,7 +110,7 @@ __device__ __forceinline__ void gram_probe_tile(const GramProbeArgs &args, int t
         va[r] = probe_element(a, args.a_ld, args.a_k_contiguous, m, min(first_of(r) + k_a, args.k - 1));
         vb[r] = probe_element(b, args.b_ld, args.b_k_contiguous, n, min(first_of(r) + k_b, args.k - 1));
     }
-    if (centre) {
+    if (centre && !(args.centre_pairs && sums.needless())) {
 #pragma unroll
         for (int r = 0; r < GP_RUNS; r++) {
             va[r] -= centre[min(first_of(r) + k_a, args.k - 1)];

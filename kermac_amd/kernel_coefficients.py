@@ -126,9 +126,9 @@ def run_kernel_coefficients(
             kernel.flags &= ~(_backend.FLAG_L2_GRAM | _backend.FLAG_L2_GRAM_BF16)
             matrix_core = False
         else:
-            plan.keepalive.append(_attach_gram_centre(kernel, stream, a.device))
             if panels is not None and _run_in_panels(plan, panels, stream, a.device, debug):
                 return plan.out
+            plan.keepalive.append(_attach_gram_centre(kernel, stream, a.device))
     elif _products_in_panels(plan) and _backend.build_kernel_has_variant(kernel.inner_operator, kernel.inner_power):
         panels = _panel_shape(plan, _backend.FLAG_DOT_PIECES)
         if panels is not None and _run_in_panels(plan, panels, stream, a.device, debug):
@@ -354,7 +354,7 @@ def _panel_shape(plan, route):
 
 def _run_in_panels(plan, shape, stream, device, debug):
     """The product in the panels of `shape` (_panel_shape); False when memory for them is missing."""
-    from .build_a_kernel import _attach_gram_workspace
+    from .build_a_kernel import _attach_gram_workspace, _centre_wanted
 
     rows, panels, ld, splits, route = shape
     L, M, N, O = plan.L, plan.M, plan.N, plan.O
@@ -362,6 +362,8 @@ def _run_in_panels(plan, shape, stream, device, debug):
     params = plan.params
     block = _backend.BuildKernelParams.from_buffer_copy(params.kernel)
     block.flags |= route
+    if block.flags & _backend.FLAG_L2_GRAM_BF16 and route and _centre_wanted():
+        block.flags |= _backend.FLAG_GRAM_OWN_CENTRE
     block.n, block.c_ld, block.c_bs = rows, ld, rows * ld
     panel = _scratch.allocate_floats((L * rows * ld,), device)
     if panel is None:
