@@ -71,6 +71,7 @@ struct GramRowsArgs {
     float *unscale;                       // [batch][rows_pad]: 1 / the row's scale
     i64 stats_bs, unscale_bs;
     int rows_pad, slices, slices_per_range, ranges;
+    int magnitude_ranges;                 // partial magnitudes per row: `ranges`, or what another launch has left
     int zero_slices;                      // slices behind the last that gram_f16_split fills with zeros (for
                                           // walks in steps of more than one slice)
 };
@@ -210,7 +211,7 @@ __device__ __forceinline__ void gram_f16_split_of(const GramRowsArgs &args, int 
     const float *centre = gram_rows_centre(args, batch);
 
     float magnitude = 0.0f;
-    for (int r = 0; r < args.ranges; r++) {
+    for (int r = 0; r < args.magnitude_ranges; r++) {
         const float part = args.magnitudes[batch * args.stats_bs + (i64)r * args.rows_pad + row];
         magnitude = part != part ? part : fmaxf(magnitude, part);
         if (part != part) break;

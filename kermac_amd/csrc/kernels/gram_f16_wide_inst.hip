@@ -190,7 +190,7 @@ kmc::GramRowsArgs rows_args(const float *x, int64_t ld, int64_t bs, int rows, in
     rows_of.unscale = reinterpret_cast<float *>(workspace + r.unscale);
     rows_of.stats_bs = r.stats_bs; rows_of.unscale_bs = r.rows_pad;
     rows_of.rows_pad = r.rows_pad; rows_of.slices = layout.slices;
-    rows_of.slices_per_range = r.slices_per_range; rows_of.ranges = r.ranges;
+    rows_of.slices_per_range = r.slices_per_range; rows_of.ranges = rows_of.magnitude_ranges = r.ranges;
     rows_of.zero_slices = layout.slices & 1;      // the walk takes two slices per step
     return rows_of;
 }
@@ -457,12 +457,16 @@ hipError_t launch_gram_f16_wide(const kmc_build_kernel_params *p, const kmc::Bui
 
 // ---- the gradient of the L2 norm as one product of pieces (norm_gradient_l2_wide.hpp) ----
 
+bool matrix_coefficients_by_rows4(const kmc_matrix_coefficients_params *p);                            // matrix_times_coefficients.hip
+int matrix_times_coefficients(const kmc_matrix_coefficients_params *p, float *magnitudes, int64_t magnitudes_bs, int64_t magnitudes_split_stride,
+                              hipStream_t stream);                                                   // matrix_times_coefficients.hip
+
 namespace {
 
 struct GradientL2Layout {
     WideLayout wide;                 // a: the columns m of a; b: the rows (o, n) of the products
     int g_parts;                     // ranges of k that g is summed in (partial products, then their sum)
-    int64_t shift, c_transposed, g, g_partial;      // byte offsets behind the regions of `wide`
+    int64_t shift, c_transposed, g, g_partial, magnitudes;      // byte offsets behind the regions of `wide`
     int64_t bytes;
 };
 
@@ -511,13 +515,14 @@ bool gradient_l2_layout(const kmc_norm_gradient_params *p, GradientL2Layout *lay
     layout->shift = place(cursor, static_cast<int64_t>(p->l) * p->n * 4);
     layout->c_transposed = place(cursor, static_cast<int64_t>(p->l) * p->k * p->o * 4);
     layout->g = place(cursor, static_cast<int64_t>(p->l) * p->m * p->o * 4);
-    // kmc_matrix_times_coefficients wants a workgroup per CU: 128 columns m and 32 outputs each
-    const int64_t workgroups = static_cast<int64_t>((p->m + 127) / 128) * ((p->o + 31) / 32) * p->l;
+    // kmc_matrix_times_coefficients wants a workgroup per CU: 256 columns m and 32 outputs each (of 128: 287 us where these take 269)
+    const int64_t workgroups = static_cast<int64_t>((p->m + 255) / 256) * ((p->o + 31) / 32) * p->l;
     int parts = workgroups >= 256 ? 1 : static_cast<int>((256 + workgroups - 1) / workgroups);
     if (parts > p->k / 512) parts = p->k / 512 > 1 ? p->k / 512 : 1;
     if (static_cast<int64_t>(parts) * p->l > 65535) parts = 1;
     layout->g_parts = parts;
     layout->g_partial = parts > 1 ? place(cursor, static_cast<int64_t>(parts) * p->l * p->m * p->o * 4) : 0;
+    layout->magnitudes = place(cursor, static_cast<int64_t>(parts) * wide.a.batches * wide.a.rows_pad * 4);
     layout->bytes = cursor;
     return true;
 }
@@ -565,7 +570,11 @@ int launch_norm_gradient_l2_wide(const kmc_norm_gradient_params *p, hipStream_t 
         weights.n_splits = layout.g_parts;
         weights.out_split_stride = static_cast<int64_t>(p->l) * weights.out_bs;
     }
-    const int contracted = kmc_matrix_times_coefficients(&weights, stream);
+    // the largest magnitudes of a's columns come with it (of a broadcast a from every batch entry, the same words)
+    const bool with_magnitudes = matrix_coefficients_by_rows4(&weights);
+    float *magnitudes = reinterpret_cast<float *>(workspace + layout.magnitudes);
+    const int64_t magnitudes_bs = static_cast<int64_t>(layout.g_parts) * wide.a.rows_pad;
+    const int contracted = matrix_times_coefficients(&weights, with_magnitudes ? magnitudes : nullptr, wide.a.batches > 1 ? magnitudes_bs : 0, wide.a.rows_pad, stream);
     if (contracted != KMC_OK) return contracted;
     if (layout.g_parts > 1) {
         kmc::GradientL2SumArgs sum = {};
@@ -584,15 +593,23 @@ int launch_norm_gradient_l2_wide(const kmc_norm_gradient_params *p, hipStream_t 
     const kmc::GramRowsArgs rows_b = rows_args(nullptr, 0, 0, rows, KMC_ROW_MAJOR, scalar_only, walk, wide, wide.b, workspace);
     kmc::GradientL2PiecesArgs pieces = {};
     pieces.a = rows_a; pieces.p = rows_b;
-    pieces.a_blocks = rows_a.rows_pad / kmc::GW_ROW_THREADS; pieces.a_batches = wide.a.batches;
+    // the columns that pad a hold zeros whatever their scale, of which the workspace may hold any
+    pieces.a_blocks = with_magnitudes ? 0 : rows_a.rows_pad / kmc::GW_ROW_THREADS; pieces.a_batches = wide.a.batches;
     pieces.from = prepare;
     // four outputs share a read of b, unless that leaves p fewer workgroups than three per CU
     const int ranges = rows_a.ranges > rows_b.ranges ? rows_a.ranges : rows_b.ranges, blocks_n = (p->n + kmc::GL2_ROWS - 1) / kmc::GL2_ROWS;
     pieces.outputs = kmc::GL2_OUTPUTS;
     while (pieces.outputs > 1 && static_cast<int64_t>(blocks_n) * ((p->o + pieces.outputs - 1) / pieces.outputs) * ranges * p->l < 768) pieces.outputs /= 2;
-    const dim3 grid(pieces.a_blocks + blocks_n * ((p->o + pieces.outputs - 1) / pieces.outputs), ranges, p->l);
+    dim3 grid(pieces.a_blocks + blocks_n * ((p->o + pieces.outputs - 1) / pieces.outputs), ranges, p->l);
     static_assert(kmc::GW_ROW_THREADS == kmc::GL2_THREADS, "one launch for both operands");
     status = launch(kmc::gradient_l2_pieces_stats, grid, dim3(kmc::GL2_THREADS), stream, pieces);
+    if (with_magnitudes) {
+        pieces.a.magnitudes = magnitudes;
+        pieces.a.stats_bs = magnitudes_bs;
+        pieces.a.magnitude_ranges = layout.g_parts;
+        pieces.a_blocks = rows_a.rows_pad / kmc::GW_ROW_THREADS;
+        grid.x += pieces.a_blocks;
+    }
     if (status == hipSuccess) status = launch(kmc::gradient_l2_pieces_split, grid, dim3(kmc::GL2_THREADS), stream, pieces);
     if (status != hipSuccess) return fail_hip(status, "gradient_l2_pieces launches");
 

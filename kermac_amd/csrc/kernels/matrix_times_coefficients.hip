@@ -43,6 +43,8 @@ struct MatrixCoefArgs {
     int m, n, o;
     int accumulate;
     int splits; i64 out_split_stride;      // the n in `splits` ranges, each with a partial product of its own
+    // rows4<.., true> only: magnitudes[batch bs + split stride + m], the largest |matrix[n, m]| of the split's n, not a number where one of them is not
+    float *magnitudes; i64 magnitudes_bs, magnitudes_split_stride;
 };
 
 // The rows n of split `split`, in whole groups of `group` except at the end of the panel.
@@ -138,10 +140,13 @@ __global__ __launch_bounds__(MC_THREADS) void matrix_times_coefficients(const Ma
 constexpr int MC4_WAVE_ROWS = 128;
 constexpr int MC4_GROUP = 4;         // loads of 16 bytes per group: 8 n, 16 matrix instructions
 
-template <int WAVES_M, int WAVES_N>
+// MAGNITUDES: the largest magnitude per row m on the way, for a caller that would otherwise read the panel once more for it
+// (the L2 gradient, whose pieces of a need it: 2 x 10000 x 10000 263 us without them, 269 with).
+template <int WAVES_M, int WAVES_N, bool MAGNITUDES>
 __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void matrix_times_coefficients_rows4(const MatrixCoefArgs args)
 {
     __shared__ float passed[WAVES_M][64][64];
+    __shared__ unsigned largest_of[MAGNITUDES ? WAVES_N : 1][MAGNITUDES ? WAVES_M * MC4_WAVE_ROWS : 1];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wave_m = wave % WAVES_M, wave_n = wave / WAVES_M;
@@ -168,6 +173,16 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void matrix_times_coefficie
     for (int c = 0; c < 4; ++c) sum[c] = mc_floatx16{0};
     float4 from_matrix[2][MC4_GROUP];
     float from_coef[2][MC4_GROUP];
+    // magnitudes as integers: the order of floats without a sign, NaNs above infinity
+    unsigned largest[4] = {0u, 0u, 0u, 0u};
+    auto note = [&](const float4 &v) {
+        if constexpr (MAGNITUDES) {
+            largest[0] = max(largest[0], __float_as_uint(v.x) & 0x7fffffffu);
+            largest[1] = max(largest[1], __float_as_uint(v.y) & 0x7fffffffu);
+            largest[2] = max(largest[2], __float_as_uint(v.z) & 0x7fffffffu);
+            largest[3] = max(largest[3], __float_as_uint(v.w) & 0x7fffffffu);
+        }
+    };
     auto load = [&](auto buffer, int at) {
 #pragma unroll
         for (int u = 0; u < MC4_GROUP; ++u) {
@@ -180,6 +195,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void matrix_times_coefficie
 #pragma unroll
         for (int u = 0; u < MC4_GROUP; ++u) {
             const float of_coef = from_coef[buffer][u] * column_exists;
+            note(from_matrix[buffer][u]);
             sum[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(of_coef, from_matrix[buffer][u].x, sum[0], 0, 0, 0);
             sum[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(of_coef, from_matrix[buffer][u].y, sum[1], 0, 0, 0);
             sum[2] = __builtin_amdgcn_mfma_f32_32x32x2f32(of_coef, from_matrix[buffer][u].z, sum[2], 0, 0, 0);
@@ -211,6 +227,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void matrix_times_coefficie
             const i64 read = row < end ? row : end - 1;
             const float of_coef = row < end ? coef[read * args.coef_ld] * column_exists : 0.0f;
             float4 of_matrix = *reinterpret_cast<const float4 *>(matrix + read * args.matrix_ld);
+            note(of_matrix);                       // a row beyond the end is the last one once more
             if (row >= end) of_matrix = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             sum[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(of_coef, of_matrix.x, sum[0], 0, 0, 0);
             sum[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(of_coef, of_matrix.y, sum[1], 0, 0, 0);
@@ -219,6 +236,22 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void matrix_times_coefficie
         }
     }
 
+    if constexpr (MAGNITUDES) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            largest[c] = max(largest[c], (unsigned)__shfl_xor((int)largest[c], 32));
+            if (half == 0) largest_of[wave_n][wave_m * MC4_WAVE_ROWS + 4 * column + c] = largest[c];
+        }
+        __syncthreads();
+        if (blockIdx.y == 0)
+            for (int r = threadIdx.x; r < WAVES_M * MC4_WAVE_ROWS; r += 64 * WAVES_M * WAVES_N) {
+                unsigned of_row = 0u;
+#pragma unroll
+                for (int team = 0; team < WAVES_N; ++team) of_row = max(of_row, largest_of[team][r]);
+                const int at = blockIdx.x * WAVES_M * MC4_WAVE_ROWS + r;
+                if (at < args.m) args.magnitudes[batch * args.magnitudes_bs + split * args.magnitudes_split_stride + at] = __uint_as_float(of_row);
+            }
+    }
     // the partial sums of teams 1 .. WAVES_N - 1 reach team 0 one after the other
     for (int team = 1; team < WAVES_N; ++team) {
         if (wave_n == team) {
@@ -252,10 +285,17 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void matrix_times_coefficie
 
 }  // namespace kmc
 
-extern "C" int kmc_matrix_times_coefficients(const kmc_matrix_coefficients_params *p, void *stream_handle)
+namespace kmc_host {
+
+bool matrix_coefficients_by_rows4(const kmc_matrix_coefficients_params *p)
 {
-    using kmc_host::fail;
-    kmc_host::clear_error();
+    return p->n > 0 && aligned16(p->matrix) && p->matrix_ld % 4 == 0 && p->matrix_bs % 4 == 0;
+}
+
+// `magnitudes`: null, or where matrix_coefficients_by_rows4 the largest magnitude of every row m goes, per batch entry and split.
+int matrix_times_coefficients(const kmc_matrix_coefficients_params *p, float *magnitudes, int64_t magnitudes_bs, int64_t magnitudes_split_stride,
+                              hipStream_t stream)
+{
     if (!p) return fail(KMC_ERR_INVALID_ARGUMENT, "null parameter block");
     if (p->m < 0 || p->n < 0 || p->o < 0 || p->l < 0) return fail(KMC_ERR_INVALID_ARGUMENT, "negative extent");
     if (p->matrix_ld < 0 || p->matrix_bs < 0 || p->coef_ld < 0 || p->coef_bs < 0 || p->out_ld < 0 || p->out_bs < 0)
@@ -279,10 +319,10 @@ extern "C" int kmc_matrix_times_coefficients(const kmc_matrix_coefficients_param
     args.accumulate = p->accumulate != 0;
     args.splits = p->n_splits > 1 ? p->n_splits : 1;
     args.out_split_stride = p->out_split_stride;
-    hipStream_t stream = static_cast<hipStream_t>(stream_handle);
+    args.magnitudes = magnitudes; args.magnitudes_bs = magnitudes_bs; args.magnitudes_split_stride = magnitudes_split_stride;
 
     const int column_tiles = (p->o + kmc::MC_COLUMNS - 1) / kmc::MC_COLUMNS;
-    const bool rows4 = p->n > 0 && kmc_host::aligned16(p->matrix) && p->matrix_ld % 4 == 0 && p->matrix_bs % 4 == 0;
+    const bool rows4 = matrix_coefficients_by_rows4(p);
     const unsigned z = static_cast<unsigned>(p->l) * args.splits;
     hipError_t e;
     if (rows4) {
@@ -291,12 +331,22 @@ extern "C" int kmc_matrix_times_coefficients(const kmc_matrix_coefficients_param
         auto grid = [&](int waves_m) { return dim3((p->m + waves_m * kmc::MC4_WAVE_ROWS - 1) / (waves_m * kmc::MC4_WAVE_ROWS), column_tiles, z); };
         const dim3 wide = grid(2);
         if (static_cast<int64_t>(wide.x) * wide.y * wide.z >= 256)
-            e = kmc_host::launch(kmc::matrix_times_coefficients_rows4<2, 4>, wide, dim3(512), stream, args);
+            e = magnitudes ? launch(kmc::matrix_times_coefficients_rows4<2, 4, true>, wide, dim3(512), stream, args)
+                           : launch(kmc::matrix_times_coefficients_rows4<2, 4, false>, wide, dim3(512), stream, args);
         else
-            e = kmc_host::launch(kmc::matrix_times_coefficients_rows4<1, 8>, grid(1), dim3(512), stream, args);
+            e = magnitudes ? launch(kmc::matrix_times_coefficients_rows4<1, 8, true>, grid(1), dim3(512), stream, args)
+                           : launch(kmc::matrix_times_coefficients_rows4<1, 8, false>, grid(1), dim3(512), stream, args);
     } else
         e = kmc_host::launch(kmc::matrix_times_coefficients, dim3((p->m + kmc::MC_ROWS - 1) / kmc::MC_ROWS, column_tiles, z),
                              dim3(kmc::MC_THREADS), stream, args);
     if (e != hipSuccess) return kmc_host::fail_hip(e, "matrix_times_coefficients launch");
     return KMC_OK;
+}
+
+}  // namespace kmc_host
+
+extern "C" int kmc_matrix_times_coefficients(const kmc_matrix_coefficients_params *p, void *stream)
+{
+    kmc_host::clear_error();
+    return kmc_host::matrix_times_coefficients(p, nullptr, 0, 0, static_cast<hipStream_t>(stream));
 }

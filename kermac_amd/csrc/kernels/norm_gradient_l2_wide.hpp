@@ -18,7 +18,9 @@
 // This header: the kernels that prepare s, the transposed c, and the pieces of a and p (g itself comes from
 // kmc_matrix_times_coefficients with a as the stored panel).  p is never stored: its values are made from b and c
 // twice, for the largest magnitude of every row and for the pieces (written in fp32 and read twice it cost 0.9 of 13.5 ms at
-// 2 x 10000 x 768 x 16 x 10000; now 12.7 .. 12.9, of which statistics 370 us and split 650, both mostly the bytes of a and the pieces).
+// 2 x 10000 x 768 x 16 x 10000).  The magnitudes of a come from the kernel that makes g, which reads all of a anyway.  Everything in front of the
+// product is its bytes there, us: g 254 -> 269, statistics of p 61 (of a and p 321), split 621 (667; c by vector loads), 982 (1273) in all, where 2.4 GB of a and
+// 1 GB of p take 700 at a copy's rate.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -76,14 +78,14 @@ __global__ __launch_bounds__(GL2_THREADS) void gradient_l2_prepare(const Gradien
     if (threadIdx.x == 0) args.shift[batch * args.shift_bs + n] = (mean - mean == 0.0f) ? mean : 0.0f;
 }
 
-// For 64 rows n, GL2_OUTPUTS outputs and one range of k: `use(output, slice, values)` for every slice of 16 values of p, lane = row
-// n, wave = every fourth slice.  b passes through LDS, since a lane's k are contiguous in memory and the lanes' rows are not.
+// For 64 rows n, GL2_OUTPUTS outputs from o_begin on and one range of k: `use(j, slice, values)` for every slice of 16 values of p of output
+// o_begin + j, lane = row n, wave = every fourth slice (uniform, so that c comes by scalar loads).  b passes through LDS, since a lane's k are contiguous in memory and the lanes' rows are not.
 template <typename Use>
 __device__ __forceinline__ void gradient_l2_walk(const GradientL2PiecesArgs &args, int n0, int o_begin, int o_end, int first, int last, Use &&use)
 {
     __shared__ float tile[GL2_DEPTH * (GL2_ROWS + 1)];
     const GradientL2PrepareArgs &from = args.from;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, batch = blockIdx.z;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), batch = blockIdx.z;
     const float *b = from.b + batch * from.b_bs, *c = from.c + batch * from.c_bs;
     const int n = n0 + lane;
     const float shift = n < from.n ? from.shift[batch * from.shift_bs + n] : 0.0f;
@@ -110,12 +112,19 @@ __device__ __forceinline__ void gradient_l2_walk(const GradientL2PiecesArgs &arg
 #pragma unroll
         for (int e = 0; e < BK_TILE_K; e++) centred[e] = tile[(BK_TILE_K * wave + e) * (GL2_ROWS + 1) + lane] - shift;
         const int k0 = slice * BK_TILE_K;
-        for (int o = o_begin; o < o_end; o++) {
-            const float *c_row = c + (i64)o * from.c_ld;
-            float value[BK_TILE_K];
 #pragma unroll
-            for (int e = 0; e < BK_TILE_K; e++) value[e] = k0 + e < from.k ? c_row[k0 + e] * centred[e] : 0.0f;
-            use(o, slice, value);
+        for (int j = 0; j < GL2_OUTPUTS; j++) {
+            if (o_begin + j >= o_end) break;
+            const float *c_row = c + (i64)(o_begin + j) * from.c_ld + k0;
+            float value[BK_TILE_K];
+            if (k0 + BK_TILE_K <= from.k) {
+#pragma unroll
+                for (int e = 0; e < BK_TILE_K; e++) value[e] = c_row[e] * centred[e];
+            } else {
+#pragma unroll
+                for (int e = 0; e < BK_TILE_K; e++) value[e] = k0 + e < from.k ? c_row[e] * centred[e] : 0.0f;
+            }
+            use(j, slice, value);
         }
     }
 }
@@ -126,38 +135,26 @@ __global__ __launch_bounds__(GL2_THREADS) void gradient_l2_pieces_stats(const Gr
         if ((int)blockIdx.z < args.a_batches && (int)blockIdx.y < args.a.ranges) gram_row_stats_of(args.a, blockIdx.x);
         return;
     }
-    __shared__ float shared[4][GL2_OUTPUTS][GL2_ROWS];
+    __shared__ unsigned shared[4][GL2_OUTPUTS][GL2_ROWS];
     const int groups = (args.from.o + args.outputs - 1) / args.outputs, block = blockIdx.x - args.a_blocks;
     const int n0 = block / groups * GL2_ROWS, o_begin = block % groups * args.outputs, o_end = min(o_begin + args.outputs, args.from.o);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, range = blockIdx.y;
     const int first = range * args.p.slices_per_range, last = min(first + args.p.slices_per_range, args.p.slices);
     if (first >= last) return;
-    float magnitude[GL2_OUTPUTS] = {};
-    bool not_a_number[GL2_OUTPUTS] = {};
-    gradient_l2_walk(args, n0, o_begin, o_end, first, last, [&](int o, int, const float (&value)[BK_TILE_K]) {
-        float largest = 0.0f;
-        bool wrong = false;
+    // as integers: the order of floats without a sign, NaNs above infinity, whose scale they take
+    unsigned magnitude[GL2_OUTPUTS] = {};
+    gradient_l2_walk(args, n0, o_begin, o_end, first, last, [&](int j, int, const float (&value)[BK_TILE_K]) {
 #pragma unroll
-        for (int e = 0; e < BK_TILE_K; e++) {
-            largest = fmaxf(largest, fabsf(value[e]));       // skips NaNs
-            wrong |= value[e] != value[e];
-        }
-#pragma unroll
-        for (int j = 0; j < GL2_OUTPUTS; j++)
-            if (o == o_begin + j) {
-                magnitude[j] = fmaxf(magnitude[j], largest);
-                not_a_number[j] |= wrong;
-            }
+        for (int e = 0; e < BK_TILE_K; e++) magnitude[j] = max(magnitude[j], __float_as_uint(value[e]) & 0x7fffffffu);
     });
-    // a NaN takes the scale of an infinity, as in gram_rows_once
 #pragma unroll
-    for (int j = 0; j < GL2_OUTPUTS; j++) shared[wave][j][lane] = not_a_number[j] ? __builtin_inff() : magnitude[j];
+    for (int j = 0; j < GL2_OUTPUTS; j++) shared[wave][j][lane] = magnitude[j];
     __syncthreads();
     const int n = n0 + lane, o = o_begin + wave;
     static_assert(GL2_OUTPUTS == 4, "a wave each");
     if (n < args.from.n && o < o_end)
         args.p.magnitudes[blockIdx.z * args.p.stats_bs + (i64)range * args.p.rows_pad + (i64)o * args.from.n + n] =
-            fmaxf(fmaxf(shared[0][wave][lane], shared[1][wave][lane]), fmaxf(shared[2][wave][lane], shared[3][wave][lane]));
+            __uint_as_float(max(max(shared[0][wave][lane], shared[1][wave][lane]), max(shared[2][wave][lane], shared[3][wave][lane])));
 }
 
 // Bound by the chunks it writes: a wave stores 1 KB of consecutive rows per piece and half.
@@ -181,18 +178,20 @@ __global__ __launch_bounds__(GL2_THREADS) void gradient_l2_pieces_split(const Gr
         const i64 row = (i64)(o_begin + j) * args.from.n + n;
         float magnitude = 0.0f;
         if (live && o_begin + j < o_end)
-            for (int r = 0; r < args.p.ranges; r++) magnitude = fmaxf(magnitude, args.p.magnitudes[batch * args.p.stats_bs + (i64)r * args.p.rows_pad + row]);
+            for (int r = 0; r < args.p.ranges; r++)
+                magnitude = __uint_as_float(max(__float_as_uint(magnitude),
+                                                __float_as_uint(args.p.magnitudes[batch * args.p.stats_bs + (i64)r * args.p.rows_pad + row])));
         const int exponent_field = gram_scale_exponent(magnitude);
         scale[j] = gram_scale(exponent_field);
         if (range == 0 && threadIdx.x < 64 && live && o_begin + j < o_end) args.p.unscale[batch * args.p.unscale_bs + row] = gram_unscale(exponent_field);
     }
     gram_chunk *pieces = args.p.pieces + batch * args.p.pieces_bs;
-    gradient_l2_walk(args, n0, o_begin, o_end, first, last, [&](int o, int slice, const float (&value)[BK_TILE_K]) {
-        const float s = o == o_begin ? scale[0] : o == o_begin + 1 ? scale[1] : o == o_begin + 2 ? scale[2] : scale[3];
+    gradient_l2_walk(args, n0, o_begin, o_end, first, last, [&](int j, int slice, const float (&value)[BK_TILE_K]) {
+        const float s = scale[j];
         unsigned piece[GW_PIECES][8];
 #pragma unroll
         for (int q = 0; q < 8; q++) gram_split_pair(value[2 * q] * s, value[2 * q + 1] * s, piece[0][q], piece[1][q]);
-        gram_chunk *dst = pieces + (i64)slice * GW_SEGMENTS * args.p.rows_pad + (i64)o * args.from.n + n;
+        gram_chunk *dst = pieces + (i64)slice * GW_SEGMENTS * args.p.rows_pad + (i64)(o_begin + j) * args.from.n + n;
 #pragma unroll
         for (int p = 0; p < GW_PIECES; p++)
 #pragma unroll
