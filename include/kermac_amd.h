@@ -170,7 +170,15 @@ enum kmc_flags {
      * call makes the centre itself, in the workspace, from up to 512 rows of a spread over the panel (per batch entry, or
      * once where a_bs is 0), subtracts it where kmc_sample_mean's flag would say so, and does not read gram_centre.
      * kmc_gram_workspace_bytes counts the room for it.  One launch instead of the two of kmc_sample_mean. */
-    KMC_FLAG_GRAM_OWN_CENTRE = 4096
+    KMC_FLAG_GRAM_OWN_CENTRE = 4096,
+    /* kmc_kernel_times_coefficients, with KMC_FLAG_L2_GRAM_BF16 or KMC_FLAG_DOT_PIECES and gram_workspace (in kernel): up to 32
+     * columns of coefficients are contracted where the route through the workspace makes the kernel matrix, tile by tile, in fp32;
+     * the products of the tiles of 128 centres go to the workspace and are added in an order that the shape fixes.  Tiles whose squared
+     * differences are not trusted are made again by the fused kernel.  n_ranges is not read.  kmc_kernel_coefficients_workspace_bytes says how
+     * much memory it wants; without it, or where that says 0, the call is as without this flag. */
+    KMC_FLAG_PRODUCT_PIECES = 8192,
+    /* With KMC_FLAG_PRODUCT_PIECES: added to `out` instead of stored (an error where the call cannot take that route). */
+    KMC_FLAG_PRODUCT_ACCUMULATE = 16384
 };
 
 /*
@@ -405,6 +413,11 @@ typedef struct kmc_kernel_coefficients_params {
  * KMC_ERR_UNSUPPORTED_VARIANT when the (inner_operator, inner_power) pair is not
  * among the ahead-of-time compiled ones. */
 int kmc_kernel_times_coefficients(const kmc_kernel_coefficients_params *params, void *stream);
+
+/* Bytes of kernel.gram_workspace that kmc_kernel_times_coefficients would use for these parameters with KMC_FLAG_PRODUCT_PIECES: the pieces of
+ * both operands (kmc_gram_workspace_bytes, whose rules decide), and 4 bytes per row, column (padded to 4) and tile of 128 centres
+ * for the products.  0: it would not.  No counterpart in the reference. */
+int kmc_kernel_coefficients_workspace_bytes(const kmc_kernel_coefficients_params *params, int64_t *bytes);
 /* 1 when (inner_operator, inner_power) is compiled ahead of time for the fused
  * coefficient kernel. */
 int kmc_kernel_times_coefficients_has_variant(int32_t inner_operator, int32_t inner_power);

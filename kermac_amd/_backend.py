@@ -50,6 +50,8 @@ FLAG_L1_FIXED = 512
 FLAG_NO_PROBE = 1024
 FLAG_DIRECT_PANELS = 2048
 FLAG_GRAM_OWN_CENTRE = 4096
+FLAG_PRODUCT_PIECES = 8192
+FLAG_PRODUCT_ACCUMULATE = 16384
 SAMPLE_BYTES = 1024             # KMC_SAMPLE_BYTES: what the sample in front of a matrix-core launch takes of the workspace
 
 _float_p = c_void_p  # device pointers are passed as integers
@@ -135,6 +137,7 @@ SIGNATURES = {
     "kmc_norm_gradient_workspace_bytes": (ctypes.c_int, [POINTER(NormGradientParams), POINTER(c_int64)]),
     "kmc_kernel_times_coefficients": (ctypes.c_int, [POINTER(KernelCoefficientsParams), c_void_p]),
     "kmc_matrix_times_coefficients": (ctypes.c_int, [POINTER(MatrixCoefficientsParams), c_void_p]),
+    "kmc_kernel_coefficients_workspace_bytes": (ctypes.c_int, [POINTER(KernelCoefficientsParams), POINTER(c_int64)]),
     "kmc_kernel_times_coefficients_has_variant": (ctypes.c_int, [c_int32, c_int32]),
     "kmc_kernel_times_coefficients_jit": (ctypes.c_int, [c_void_p, POINTER(KernelCoefficientsParams), c_void_p]),
     "kmc_jit_compile": (ctypes.c_int, [
@@ -263,6 +266,13 @@ def norm_kernel_gradient(params: NormGradientParams, stream: int) -> None:
 
 def kernel_times_coefficients(params: KernelCoefficientsParams, stream: int) -> None:
     check(library().kmc_kernel_times_coefficients(byref(params), c_void_p(stream)))
+
+
+def kernel_coefficients_workspace_bytes(params: KernelCoefficientsParams) -> int:
+    """Bytes of kernel.gram_workspace that the product from pieces would use for these parameters (0: it would not run)."""
+    needed = c_int64(0)
+    check(library().kmc_kernel_coefficients_workspace_bytes(byref(params), byref(needed)))
+    return needed.value
 
 
 def kernel_times_coefficients_jit(function: int, params: KernelCoefficientsParams, stream: int) -> None:

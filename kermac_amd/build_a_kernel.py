@@ -634,14 +634,16 @@ def run_kernel(
             _backend.build_kernel_jit(function, block, stream)
 
     matrix_core = _backend.FLAG_L2_GRAM | _backend.FLAG_L2_GRAM_BF16 | _backend.FLAG_DOT_PIECES
+    route_bytes = None
     if plan.l2_auto and params.flags & matrix_core:
         asked = params.flags & matrix_core
         params.flags &= ~matrix_core
-        params.flags |= _auto_matrix_core_flags(params, asked)
+        chosen, route_bytes = _auto_matrix_cores(params, asked)
+        params.flags |= chosen
     if params.flags & _backend.FLAG_DOT_PIECES:
         # products have no matrix-core kernel beside the route through the workspace: a call the
         # library has no use for a workspace for is an ordinary call of the direct kernel
-        workspace = _attach_gram_workspace(params, a.device)
+        workspace = _attach_gram_workspace(params, a.device, needed=route_bytes)
         if workspace is None:
             params.flags &= ~_backend.FLAG_DOT_PIECES
         plan.keepalive.append(workspace)
@@ -654,7 +656,7 @@ def run_kernel(
         plan.keepalive.append(workspace)
     cut = _cut_over_contraction(params)
     if params.flags & (_backend.FLAG_L2_GRAM | _backend.FLAG_L2_GRAM_BF16):
-        plan.keepalive.append(_attach_gram_memory(params, stream, a.device))
+        plan.keepalive.append(_attach_gram_memory(params, stream, a.device, route_bytes))
     elif (cut is None and not params.flags & (_backend.FLAG_DOT_PIECES | _backend.FLAG_L1_FIXED)
             and params.inner_operator == _backend.OP_DIFF
             and (params.inner_power in (_backend.POW_ABS, _backend.POW_SQUARE)
@@ -686,18 +688,20 @@ def _direct_panels_min_tiles() -> int:
     return int(_backend.dispatch_rules()["DIRECT_PANELS_MIN_TILES"])
 
 
-def _attach_gram_memory(params, stream, device):
+def _attach_gram_memory(params, stream, device, route_bytes=None):
     """What a matrix-core launch for squared differences takes beside its operands: the workspace, and the centre, which the
     route through the workspace makes for itself in there (include/kermac_amd.h, KMC_FLAG_GRAM_OWN_CENTRE)."""
-    if _centre_wanted():
-        params.flags |= _backend.FLAG_GRAM_OWN_CENTRE
-    needed = _backend.gram_workspace_bytes(params)
-    if needed:
-        workspace = _attach_gram_workspace(params, device, needed=needed)
+    if route_bytes is None:
+        route_bytes = _route_bytes(params, 0)
+    if route_bytes:
+        if _centre_wanted():
+            params.flags |= _backend.FLAG_GRAM_OWN_CENTRE
+        workspace = _attach_gram_workspace(params, device, needed=route_bytes)
         if workspace is not None:
             return workspace
-    params.flags &= ~_backend.FLAG_GRAM_OWN_CENTRE         # a one-step kernel
-    return _attach_gram_centre(params, stream, device), _attach_gram_workspace(params, device)
+        params.flags &= ~_backend.FLAG_GRAM_OWN_CENTRE
+        route_bytes = _backend.gram_workspace_bytes(params)
+    return _attach_gram_centre(params, stream, device), _attach_gram_workspace(params, device, needed=route_bytes)     # a one-step kernel
 
 
 def _centre_wanted():
@@ -759,9 +763,20 @@ _AUTO_UNCUT_MIN_TILES_K_CONTIGUOUS = 192
 
 
 def _auto_matrix_core_flags(params, asked):
-    """Which of the matrix-core flags `asked` (those the descriptor allows) this call gets in the l2 mode "auto"."""
-    if _workspace_route_applies(params, asked) and not _small_set_is_cut(params, asked):
-        return asked
+    return _auto_matrix_cores(params, asked)[0]
+
+
+def _auto_matrix_cores(params, asked):
+    """Which of the matrix-core flags `asked` (those the descriptor allows) this call gets in the l2 mode "auto", and the bytes that the
+    library wants for its route through a workspace with them (0: it has none for this call)."""
+    route_bytes = _route_bytes(params, asked)
+    if _workspace_allowed(route_bytes) and not _small_set_is_cut(params, asked):
+        return asked, route_bytes
+    chosen = _auto_one_step_flags(params, asked)
+    return chosen, route_bytes if chosen == asked else 0
+
+
+def _auto_one_step_flags(params, asked):
     # operands with the rows contiguous (m or n, the kernels' own order) stage faster in the split kernel
     rows_contiguous = params.a_majorness == _backend.COL_MAJOR and params.b_majorness == _backend.COL_MAJOR
     if not asked & _backend.FLAG_L2_GRAM or params.k < _AUTO_ONE_STEP_MIN_K or params.gram_trust >= 1.0:
@@ -818,13 +833,19 @@ def _small_set_is_cut(params, asked):
                 and _direct_path_would_cut(params, asked))
 
 
-def _workspace_route_applies(params, flags):
-    """Whether kmc_build_kernel would take this call through a workspace, given these matrix-core flags."""
+def _workspace_allowed(route_bytes):
+    # the environment last: a small call, which the library has no workspace for, is bound by the host
+    return route_bytes > 0 and os.environ.get("KERMAC_AMD_L2_WORKSPACE", "1") not in ("", "0")
+
+
+def _route_bytes(params, flags):
+    """The workspace that kmc_build_kernel would take this call through, given these matrix-core flags (0: none), with room for the centre."""
     kept = params.flags
     params.flags |= flags
+    if params.flags & _backend.FLAG_L2_GRAM_BF16:
+        params.flags |= _backend.FLAG_GRAM_OWN_CENTRE
     try:
-        # the environment last: a small call, which the library has no workspace for, is bound by the host
-        return _backend.gram_workspace_bytes(params) > 0 and os.environ.get("KERMAC_AMD_L2_WORKSPACE", "1") not in ("", "0")
+        return _backend.gram_workspace_bytes(params)
     finally:
         params.flags = kept
 

@@ -1,6 +1,7 @@
 // C-ABI entry points for the fused kernel-matrix x coefficients contraction.
 #include "host_common.hpp"
 #include "../kernels/kernel_coefficients.hpp"
+#include "contraction.hpp"
 #include "launchers.hpp"
 
 using namespace kmc_host;
@@ -49,6 +50,7 @@ int prepare(const kmc_kernel_coefficients_params *p, bool wide_allowed, kmc::Ker
     if (ranges > 1 && p->out_range_stride < 0) return fail(KMC_ERR_INVALID_ARGUMENT, "negative out_range_stride");
     kc->split_tiles = k.tiles_n > 0 ? ceil_div(k.tiles_n, ranges) : 1;
     kc->out_split_stride = ranges > 1 ? p->out_range_stride : 0;
+    kc->stamps = nullptr;
     *grid = dim3(k.tiles_m, static_cast<unsigned>(grid_y), static_cast<unsigned>(ranges));
     return KMC_OK;
 }
@@ -62,9 +64,48 @@ kmc_host::coef_launcher_fn find_launcher(int inner_operator, int inner_power)
     return nullptr;
 }
 
+// Squared differences and sums of products with KMC_FLAG_PRODUCT_PIECES: the matrix from products of fp16 pieces, contracted tile by tile where it
+// is made; tiles that are not trusted again by the fused kernel; the sum of all tiles.  *taken: the launches were made.
+hipError_t launch_contraction(const kmc_kernel_coefficients_params *p, const kmc::KernelCoefficientsArgs &kc, int load_a, int load_b, hipStream_t stream, bool *taken)
+{
+    kmc_host::Contraction contraction = {p->coef, p->coef_ld, p->coef_bs, p->o, nullptr, nullptr};
+    hipError_t status = kmc_host::launch_gram_f16_wide(&p->kernel, kc.kernel, stream, taken, nullptr, &contraction);
+    if (status != hipSuccess || !*taken) return status;
+    if (p->kernel.inner_operator == KMC_OP_DIFF) {
+        kmc::KernelCoefficientsArgs repair = kc;
+        repair.columns = kmc::KC_COLUMNS;
+        repair.o_chunks = 1;
+        repair.stamps = contraction.stamps;
+        repair.split_tiles = 1;
+        repair.out = contraction.products;
+        repair.out_ld = (p->o + 3) / 4 * 4;
+        repair.out_bs = repair.out_ld * kc.kernel.m;
+        repair.out_split_stride = repair.out_bs * kc.kernel.l;
+        const dim3 grid(kc.kernel.tiles_m, kc.kernel.l, kc.kernel.tiles_n);
+        status = find_launcher(p->kernel.inner_operator, p->kernel.inner_power)(load_a, load_b, repair, grid, stream);
+        if (status != hipSuccess) return status;
+    }
+    return kmc_host::launch_sum_products(contraction.products, kc.kernel.tiles_n, kc.kernel.l, kc.kernel.m, p->o, p->out, p->out_ld, p->out_bs,
+                                         (p->kernel.flags & KMC_FLAG_PRODUCT_ACCUMULATE) != 0, stream);
+}
+
 }  // namespace
 
 extern "C" {
+
+int kmc_kernel_coefficients_workspace_bytes(const kmc_kernel_coefficients_params *params, int64_t *bytes)
+{
+    if (!bytes) return fail(KMC_ERR_INVALID_ARGUMENT, "bytes: null pointer");
+    kmc::KernelCoefficientsArgs kc;
+    int load_a = 0, load_b = 0;
+    dim3 grid;
+    bool empty = false;
+    const int status = prepare(params, false, &kc, &load_a, &load_b, &grid, &empty);
+    if (status != KMC_OK) return status;
+    *bytes = !empty && kc.kernel.n > 0 && (params->kernel.flags & KMC_FLAG_PRODUCT_PIECES)
+                 ? kmc_host::gram_f16_wide_contraction_bytes(&params->kernel, kc.kernel, params->o) : 0;
+    return KMC_OK;
+}
 
 int kmc_kernel_times_coefficients_has_variant(int32_t inner_operator, int32_t inner_power)
 {
@@ -86,6 +127,14 @@ int kmc_kernel_times_coefficients(const kmc_kernel_coefficients_params *params, 
             return fail(KMC_ERR_INVALID_ARGUMENT, "KMC_FLAG_L2_GRAM needs inner_operator DIFF and inner_power SQUARE");
         launch = kmc_host::launch_gram_coefficients;   // kernel values from the matrix cores
     }
+    if ((params->kernel.flags & KMC_FLAG_PRODUCT_PIECES) && !empty && kc.kernel.n > 0) {
+        status = require_gfx950();
+        if (status != KMC_OK) return status;
+        bool taken = false;
+        const hipError_t made = launch_contraction(params, kc, load_a, load_b, static_cast<hipStream_t>(stream), &taken);
+        if (made != hipSuccess) return fail_hip(made, "kernel matrix times coefficients from pieces");
+        if (taken) return KMC_OK;
+    }
     if (!launch) {
         return fail(KMC_ERR_UNSUPPORTED_VARIANT,
                     "inner_operator=%d inner_power=%d is not compiled ahead of time; compile it at run time",
@@ -94,6 +143,8 @@ int kmc_kernel_times_coefficients(const kmc_kernel_coefficients_params *params, 
     if (empty) return KMC_OK;
     status = require_gfx950();
     if (status != KMC_OK) return status;
+    if (params->kernel.flags & KMC_FLAG_PRODUCT_ACCUMULATE)
+        return fail(KMC_ERR_INVALID_ARGUMENT, "KMC_FLAG_PRODUCT_ACCUMULATE needs the route of KMC_FLAG_PRODUCT_PIECES");
     hipError_t e = launch(load_a, load_b, kc, grid, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return fail_hip(e, "kernel_times_coefficients launch");
     return KMC_OK;

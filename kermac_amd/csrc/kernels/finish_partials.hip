@@ -106,9 +106,83 @@ __global__ __launch_bounds__(256) void finish_partials(const FinishArgs fa)
     for (int n = blockIdx.y; n < args.n; n += gridDim.y) finish_row(fa, group_sums, batch, n, p_outer, neg_gamma, regularization);
 }
 
+// out[l][m][o] (+)= the sum of the products of the tiles, in an order that the shape fixes.  A workgroup holds 64 consecutive quads of a product
+// [m][o padded to 4], so that a load reads 1 KB; where there are few of them its waves share the tiles among themselves (wave w the tiles
+// w, w + W, ..) and the first adds up what they have.  Eight loads under way per lane.
+struct SumProductsArgs {
+    const float4 *products;      // [tile][l][m][quads]
+    i64 tile;                    // quads from one tile's product to the next
+    i64 count;                   // l m quads
+    float *out; i64 out_ld, out_bs;
+    int m, outputs, quads, tiles, accumulate;
+};
+
+constexpr int SUM_PRODUCTS_MAX_WAVES = 16;
+
+template <int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void sum_products(const SumProductsArgs args)
+{
+    __shared__ float4 of_waves[WAVES][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const i64 at = (i64)blockIdx.x * 64 + lane;
+    float4 sum = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (at < args.count) {
+        const float4 *from = args.products + at;
+        int tile = wave;
+        for (; tile + 7 * WAVES < args.tiles; tile += 8 * WAVES) {
+            float4 v[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) v[u] = from[(tile + u * WAVES) * args.tile];
+#pragma unroll
+            for (int u = 0; u < 8; u++) { sum.x += v[u].x; sum.y += v[u].y; sum.z += v[u].z; sum.w += v[u].w; }
+        }
+        for (; tile < args.tiles; tile += WAVES) {
+            const float4 v = from[tile * args.tile];
+            sum.x += v.x; sum.y += v.y; sum.z += v.z; sum.w += v.w;
+        }
+    }
+    if (WAVES > 1) {
+        of_waves[wave][lane] = sum;
+        __syncthreads();
+        if (wave > 0) return;
+#pragma unroll
+        for (int w = 1; w < WAVES; w++) {
+            const float4 v = of_waves[w][lane];
+            sum.x += v.x; sum.y += v.y; sum.z += v.z; sum.w += v.w;
+        }
+    }
+    if (at >= args.count) return;
+    const i64 row = at / args.quads;
+    const int o = 4 * (int)(at - row * args.quads), l = (int)(row / args.m);
+    float *to = args.out + l * args.out_bs + (row - (i64)l * args.m) * args.out_ld + o;
+    const float values[4] = {sum.x, sum.y, sum.z, sum.w};
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+        if (o + e < args.outputs) to[e] = args.accumulate ? to[e] + values[e] : values[e];
+}
+
 }  // namespace kmc
 
 namespace kmc_host {
+
+// products: [tile][l][m][outputs padded to 4], 16-byte aligned.
+hipError_t launch_sum_products(const float *products, int tiles, int l, int m, int outputs, float *out, int64_t out_ld, int64_t out_bs, bool accumulate,
+                               hipStream_t stream)
+{
+    kmc::SumProductsArgs args;
+    args.products = reinterpret_cast<const float4 *>(products);
+    args.quads = (outputs + 3) / 4;
+    args.count = args.tile = static_cast<int64_t>(l) * m * args.quads;
+    args.out = out; args.out_ld = out_ld; args.out_bs = out_bs;
+    args.m = m; args.outputs = outputs; args.tiles = tiles; args.accumulate = accumulate;
+    const int64_t blocks = (args.count + 63) / 64;
+    if (blocks > 0x7fffffff) return hipErrorInvalidValue;
+    const dim3 grid(static_cast<unsigned>(blocks));
+    // one wave each from eight per CU on
+    if (blocks >= 2048 || tiles < 16) return launch(kmc::sum_products<1>, grid, dim3(64), stream, args);
+    if (blocks >= 512 || tiles < 64) return launch(kmc::sum_products<4>, grid, dim3(256), stream, args);
+    return launch(kmc::sum_products<kmc::SUM_PRODUCTS_MAX_WAVES>, grid, dim3(64 * kmc::SUM_PRODUCTS_MAX_WAVES), stream, args);
+}
 
 hipError_t launch_finish_partials(const kmc::BuildKernelArgs &kernel, const float *partials, int64_t partial_ld,
                                   int64_t partial_bs, int64_t partial_slice, int slices, int vec, hipStream_t stream)

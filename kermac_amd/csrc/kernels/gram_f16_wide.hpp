@@ -93,6 +93,11 @@ struct GramWideArgs {
     const float *gradient_g; i64 gradient_g_ld, gradient_g_bs;
     const float *gradient_shift; i64 gradient_shift_bs;
     int gradient_n;
+    // COLUMNS > 0 only: the matrix times coefficients, tile by tile (gram_f16_wide)
+    const float *coef; i64 coef_ld, coef_bs;      // [n][o], o contiguous
+    int outputs;
+    float *products; i64 products_ld, products_bs, products_tile;      // [tile of 128 n][batch][m][o], products_ld a multiple of 4
+    int *stamps; int stamps_m, stamps_n;          // [batch][tile of 128 m][tile of 128 n]: 1 where the repair launch recomputes the tile's product
 };
 
 constexpr int GW_MAX_RANGES = 9;      // ranges of K per row: ceil(slices / 8) up to 71 slices, 8 beyond
@@ -100,6 +105,8 @@ constexpr int GW_MAX_RANGES = 9;      // ranges of K per row: ceil(slices / 8) u
 constexpr int GW_EPILOGUE_DISTANCE = 0;
 constexpr int GW_EPILOGUE_GRADIENT_L2 = 1;
 constexpr int GW_EPILOGUE_DOT = 2;
+// added to GW_EPILOGUE_DISTANCE or GW_EPILOGUE_DOT: contracted with up to 16 or 32 columns of coefficients instead of stored
+constexpr int GW_CONTRACT_16 = 4, GW_CONTRACT_32 = 8;
 
 // The 16 values of row `row` in slice `slice`, centre subtracted; zeros where the row or k does not exist.
 __device__ __forceinline__ void gram_load_row_slice(const GramRowsArgs &args, const float *x, const float *centre, int row,
@@ -716,9 +723,19 @@ __device__ __forceinline__ void wide_walk_steps(gram_float4 (&acc)[Tile::MT][Til
 // EPILOGUE GW_EPILOGUE_DOT: the inner operator DOT (sum_k a b): the product of the pieces is the
 // value itself, nothing cancels, so there is no trust check and no repair; outer power, kernel
 // function, regularised diagonal and the stores, mirrored ones included, are those of the distance.
-template <typename Tile, bool SYMMETRIC, int EPILOGUE = GW_EPILOGUE_DISTANCE>
+//
+// GW_CONTRACT_16, GW_CONTRACT_32 (COLUMNS = 16, 32): the values are not stored but contracted with up to COLUMNS columns of coefficients, and the product of
+// every tile of 128 n goes to a place of its own, to be added up by sum_products: out[m, o] = sum_n C(m, n) coef[n, o].  A wave stages 16
+// columns n as for the stores and multiplies them with v_mfma_f32_16x16x4_f32 (fp32 operands and sums), lane q of four
+// groups on n = 4 q + step, so that its reads of the staged values fall into banks of their own.  Panels of the matrix stored
+// and contracted by a kernel of their own / this, us: 1000 x 60000 x 784, 10 columns 461 / 391, 32 columns 457 / 414; 4 x 16384 x 16384 x 256, 32 columns
+// 3679 / 2967, 10 columns 3664 / 2407; 30000 x 30000 x 1024, 16 columns 5846 / 5070; 8192 x 65536 x 128, 8 columns 1436 / 1002; 4096 x 4096 x 256,
+// 32 columns 87 / 76; 500 x 500 x 2000, 10 columns 113 / 101; none of 24 shapes was slower.
+template <typename Tile, bool SYMMETRIC, int WHAT = GW_EPILOGUE_DISTANCE>
 __global__ __launch_bounds__(Tile::THREADS, Tile::MIN_WAVES) void gram_f16_wide(const GramWideArgs args)
 {
+    constexpr int EPILOGUE = WHAT % GW_CONTRACT_16, COLUMNS = WHAT / GW_CONTRACT_16 * 16;
+    static_assert(COLUMNS == 0 || (!SYMMETRIC && EPILOGUE != GW_EPILOGUE_GRADIENT_L2 && Tile::TILE_N == 128), "what the contraction is for");
     constexpr int TILE_M = Tile::TILE_M, TILE_N = Tile::TILE_N, MT = Tile::MT, NT = Tile::NT;
     __shared__ gram_chunk ring[Tile::SLOTS * Tile::GRANULE_CHUNKS];
     __shared__ __attribute__((aligned(16))) float lds_norm_a[TILE_M], lds_norm_b[TILE_N];
@@ -740,7 +757,9 @@ __global__ __launch_bounds__(Tile::THREADS, Tile::MIN_WAVES) void gram_f16_wide(
             if (tid < Tile::PARTS) {
                 const int part_m = tid % Tile::PARTS_M * 128, part_n = tid / Tile::PARTS_M * 128;
                 const bool above = SYMMETRIC && m0 + part_m < n0 + part_n;
-                if (!above && part_m < m_valid && part_n < n_valid)
+                if constexpr (COLUMNS > 0) {
+                    if (part_m < m_valid) args.stamps[((i64)batch * args.stamps_m + (m0 + part_m) / 128) * args.stamps_n + tile_n] = 1;
+                } else if (!above && part_m < m_valid && part_n < n_valid)
                     args.kernel.c[batch * args.kernel.c_bs + (i64)(n0 + part_n) * args.kernel.c_ld + m0 + part_m] =
                         __uint_as_float(BK_REPAIR_MARKER);
             }
@@ -894,8 +913,28 @@ __global__ __launch_bounds__(Tile::THREADS, Tile::MIN_WAVES) void gram_f16_wide(
         static_assert(16 * PITCH <= 4 * Tile::SLOTS * Tile::GRANULE_CHUNKS / Tile::WAVES, "the staging fits a wave's share of the ring");
         const int row = wave_m + 4 * (lane_after % LANES);
         const bool whole = c_vec && row + 3 < rows;
+        constexpr int OB = COLUMNS > 0 ? COLUMNS / 16 : 1;
+        gram_float4 products[COLUMNS > 0 ? MT : 1][OB];          // [m block][o block]: o = 16 ob + 4 q + v, m = wave_m + 16 mt + i
+        const float *coef = nullptr;
+        if constexpr (COLUMNS > 0) {
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+                for (int ob = 0; ob < OB; ob++) products[mt][ob] = gram_float4{0.0f, 0.0f, 0.0f, 0.0f};
+            coef = late->coef + batch * late->coef_bs;
+        }
 #pragma unroll
         for (int nt = 0; nt < NT; nt++) {
+            float weights[COLUMNS > 0 ? 4 : 1][OB];              // of n = 16 nt + 4 q + step, o = 16 ob + i
+            if constexpr (COLUMNS > 0) {
+#pragma unroll
+                for (int step = 0; step < 4; step++)
+#pragma unroll
+                    for (int ob = 0; ob < OB; ob++) {
+                        const int n_local = wave_n + 16 * nt + 4 * q + step, o = 16 * ob + i;
+                        weights[step][ob] = n_local < columns && o < late->outputs ? coef[(i64)(n0 + n_local) * late->coef_ld + o] : 0.0f;
+                    }
+            }
             const float norm_b = EPILOGUE == GW_EPILOGUE_DISTANCE ? lds_norm_b[wave_n + nt * 16 + i] : 0.0f;
             const float unscale_b = (EPILOGUE == GW_EPILOGUE_DISTANCE ? -2.0f : 1.0f) * lds_unscale_b[wave_n + nt * 16 + i];
 #pragma unroll
@@ -949,6 +988,25 @@ __global__ __launch_bounds__(Tile::THREADS, Tile::MIN_WAVES) void gram_f16_wide(
                 }
             }
             if (above) continue;
+            if constexpr (COLUMNS > 0) {
+                // columns that do not exist may hold anything, which is no factor of a zero coefficient
+                const bool exists = wave_n + 16 * nt + i < columns;
+                wide_lanes_exchange();
+#pragma unroll
+                for (int mt = 0; mt < MT; mt++)
+                    *reinterpret_cast<gram_float4 *>(stage + i * PITCH + 16 * mt + 4 * q) = exists ? acc[mt][nt] : gram_float4{0.0f, 0.0f, 0.0f, 0.0f};
+                wide_lanes_exchange();
+#pragma unroll
+                for (int step = 0; step < 4; step++)
+#pragma unroll
+                    for (int mt = 0; mt < MT; mt++) {
+                        const float value = stage[(4 * q + step) * PITCH + 16 * mt + i];
+#pragma unroll
+                        for (int ob = 0; ob < OB; ob++)
+                            products[mt][ob] = __builtin_amdgcn_mfma_f32_16x16x4f32(weights[step][ob], value, products[mt][ob], 0, 0, 0);
+                    }
+                continue;
+            }
             wide_lanes_exchange();
 #pragma unroll
             for (int mt = 0; mt < MT; mt++) *reinterpret_cast<gram_float4 *>(stage + i * PITCH + 16 * mt + 4 * q) = acc[mt][nt];
@@ -970,6 +1028,37 @@ __global__ __launch_bounds__(Tile::THREADS, Tile::MIN_WAVES) void gram_f16_wide(
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (COLUMNS > 0) {
+            // The products of the waves side by side along n, added in their order.  (The ring holds the staged values of every wave until here.)
+            constexpr int QUADS = MT * OB;
+            static_assert(64 * QUADS * (Tile::WAVES - Tile::WAVES_M) <= Tile::SLOTS * Tile::GRANULE_CHUNKS, "the products of all but the first fit the ring");
+            gram_float4 *shared = reinterpret_cast<gram_float4 *>(ring);
+            const int along_m = wave % Tile::WAVES_M, along_n = wave / Tile::WAVES_M;
+            if (EPILOGUE == GW_EPILOGUE_DISTANCE && !(least_margin >= 0.0f)) lds_distrust[part] = 1;
+            __syncthreads();
+            if (along_n > 0) {
+#pragma unroll
+                for (int at = 0; at < QUADS; at++)
+                    shared[(((along_n - 1) * Tile::WAVES_M + along_m) * QUADS + at) * 64 + lane_after] = products[at / OB][at % OB];
+            }
+            __syncthreads();
+            if (EPILOGUE == GW_EPILOGUE_DISTANCE && wave == 0 && lane_after < Tile::PARTS && 128 * lane_after < rows)
+                late->stamps[((i64)batch * late->stamps_m + m0 / 128 + lane_after) * late->stamps_n + tile_n] = lds_distrust[lane_after];
+            if (along_n > 0) return;
+            float *to = late->products + tile_n * late->products_tile + batch * late->products_bs + (i64)m0 * late->products_ld;
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+                for (int ob = 0; ob < OB; ob++) {
+                    gram_float4 sum = products[mt][ob];
+#pragma unroll
+                    for (int team = 1; team < Tile::WAVES_N; team++)
+                        sum += shared[(((team - 1) * Tile::WAVES_M + along_m) * QUADS + mt * OB + ob) * 64 + lane_after];
+                    const int m_local = wave_m + 16 * mt + i, o = 16 * ob + 4 * q;
+                    if (m_local < rows && o < late->outputs) *reinterpret_cast<gram_float4 *>(to + m_local * late->products_ld + o) = sum;
+                }
+            return;
         }
     }
     if constexpr (EPILOGUE == GW_EPILOGUE_DISTANCE) {

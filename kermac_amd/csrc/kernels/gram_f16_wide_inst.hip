@@ -12,6 +12,7 @@
 #include "../host/host_common.hpp"
 #include "../host/dispatch_rules.hpp"
 #include "launch.hpp"
+#include "../host/contraction.hpp"
 #include "gram_f16_wide.hpp"
 #include "norm_gradient_l2_wide.hpp"
 
@@ -37,6 +38,7 @@ struct WideLayout {
     int64_t sample;         // byte offset of the words of gram_probe_operands
     int64_t centre = 0, centre_floats = 0;      // byte offset of the centre that the route takes for itself, floats per batch entry (0: it takes none)
     int centre_batches = 1;
+    int64_t products = 0, stamps = 0;           // byte offsets of a contraction's products and stamps
     int64_t bytes;
 };
 
@@ -337,6 +339,10 @@ hipError_t launch_product_in(kmc::GramWideArgs &wide, hipStream_t stream)
 // K = 784 210 / 185, of K = 4096 1072 / 934; 784, 3584 x 3584 of K = 784 100 / 96, of K = 4096 395 / 371; 938, 200 x 60000 of K = 784 194.4 / 197.5,
 // of K = 2048 568 / 561; 1024, 4096 x 4096 of K = 784 103.1 / 103.8, of K = 4096 432 / 421; more than one round of either: 1156,
 // 4352 x 4352 of K = 2048 276 / 306.  A set against itself: 780, 4900 points of K = 784 110 / 120; 990, 5632 of K = 784 130 / 127.
+//
+// A contraction stays with the small tiles: the large one's sums and products leave no registers for its operands, and it has no stores to save on
+// (large / small, us: 4 x 16384 x 16384 x 256, 32 columns 3073 / 2967, 10 columns 2477 / 2407; 30000 x 30000 x 1024, 16 columns 5012 / 5054, 32
+// columns 5418 / 5406; 16384 x 16384 x 128, 32 columns 622 / 613).
 constexpr int64_t SMALL_TILES_PER_ROUND = kmc::WideTileSmall::PER_CU * 256, LARGE_TILES_PER_ROUND = kmc::WideTileLarge::PER_CU * 256;
 constexpr int64_t LITTLE_OF_A_ROUND = SMALL_TILES_PER_ROUND / 6;
 constexpr int LONG_CONTRACTION_SLICES = 2048 / kmc::BK_TILE_K;
@@ -360,9 +366,31 @@ hipError_t launch_product(kmc::GramWideArgs &wide, hipStream_t stream)
                            (small <= SMALL_TILES_PER_ROUND + LITTLE_OF_A_ROUND || wide.slices >= LONG_CONTRACTION_SLICES);
     // KERMAC_AMD_WIDE_LARGE_TILE_MIN_TILES=n replaces the number (read on every call, so that a test can send small shapes to the large tiles)
     const char *text = std::getenv("KERMAC_AMD_WIDE_LARGE_TILE_MIN_TILES");
-    if (large >= (text ? std::atoi(text) : kmc_rules::WIDE_LARGE_TILE_MIN_TILES) || one_round) return launch_product_in<Large, SYMMETRIC, EPILOGUE>(wide, stream);
+    if constexpr (EPILOGUE < kmc::GW_CONTRACT_16) {
+        if (large >= (text ? std::atoi(text) : kmc_rules::WIDE_LARGE_TILE_MIN_TILES) || one_round) return launch_product_in<Large, SYMMETRIC, EPILOGUE>(wide, stream);
+    } else if (text && std::atoi(text) > 0) {
+        return launch_product_in<Small, SYMMETRIC, EPILOGUE>(wide, stream);
+    }
     if (small <= FEW_TILES) return launch_product_in<kmc::WideTileFew, SYMMETRIC, EPILOGUE>(wide, stream);
     return launch_product_in<Small, SYMMETRIC, EPILOGUE>(wide, stream);
+}
+
+// Room for the products of a contraction's tiles, behind everything else; false where the kernels behind it could not take the problem.
+bool place_contraction(const kmc::BuildKernelArgs &args, int outputs, WideLayout *layout)
+{
+    if (outputs < 1 || outputs > CONTRACTION_MAX_OUTPUTS || args.tiles_n > 65535) return false;
+    int64_t cursor = layout->bytes;
+    layout->products = place(cursor, static_cast<int64_t>(args.tiles_n) * args.l * args.m * ((outputs + 3) / 4 * 4) * 4);
+    layout->stamps = place(cursor, static_cast<int64_t>(args.l) * args.tiles_m * args.tiles_n * 4);
+    layout->bytes = cursor;
+    return true;
+}
+
+// Bytes of workspace for the matrix times coefficients by this path; 0 when it does not apply.
+int64_t gram_f16_wide_contraction_bytes(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &args, int outputs)
+{
+    WideLayout layout;
+    return wide_layout(p, args, &layout) && place_contraction(args, outputs, &layout) ? layout.bytes : 0;
 }
 
 // Bytes of workspace the path needs for this problem; 0 when it does not apply.
@@ -375,13 +403,13 @@ int64_t gram_f16_wide_bytes(const kmc_build_kernel_params *p, const kmc::BuildKe
 // Row statistics and split of both operands, then the product kernel.  `*taken` says whether the
 // path applied (and the launches were made); if not, nothing was launched.
 hipError_t launch_gram_f16_wide(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &as_given, hipStream_t stream, bool *taken,
-                                const unsigned **sample_taken)
+                                const unsigned **sample_taken, Contraction *contraction)
 {
     kmc::BuildKernelArgs args = as_given;
     *taken = false;
     if (sample_taken) *sample_taken = nullptr;
     WideLayout layout;
-    if (!p->gram_workspace || !wide_layout(p, args, &layout) || p->gram_workspace_bytes < layout.bytes ||
+    if (!p->gram_workspace || !wide_layout(p, args, &layout) || (contraction && !place_contraction(args, contraction->outputs, &layout)) || p->gram_workspace_bytes < layout.bytes ||
         (reinterpret_cast<uintptr_t>(p->gram_workspace) & (REGION_ALIGN - 1)) != 0)
         return hipSuccess;
     char *workspace = static_cast<char *>(p->gram_workspace);
@@ -447,6 +475,23 @@ hipError_t launch_gram_f16_wide(const kmc_build_kernel_params *p, const kmc::Bui
     wide.unscale_b_bs = layout.b.batches > 1 ? layout.b.rows_pad : 0;
     wide.rows_pad_a = layout.a.rows_pad; wide.rows_pad_b = layout.b.rows_pad;
     wide.slices = layout.slices; wide.ranges_a = layout.a.ranges; wide.ranges_b = layout.b.ranges;
+    if (contraction) {
+        wide.coef = contraction->coef; wide.coef_ld = contraction->coef_ld; wide.coef_bs = contraction->coef_bs;
+        wide.outputs = contraction->outputs;
+        wide.products = contraction->products = reinterpret_cast<float *>(workspace + layout.products);
+        wide.products_ld = (contraction->outputs + 3) / 4 * 4;
+        wide.products_bs = wide.products_ld * args.m;
+        wide.products_tile = wide.products_bs * args.l;
+        wide.stamps = contraction->stamps = reinterpret_cast<int *>(workspace + layout.stamps);
+        wide.stamps_m = args.tiles_m; wide.stamps_n = args.tiles_n;
+        const bool few = contraction->outputs <= 16;
+        if (products)
+            status = few ? launch_product<false, kmc::GW_EPILOGUE_DOT + kmc::GW_CONTRACT_16>(wide, stream) : launch_product<false, kmc::GW_EPILOGUE_DOT + kmc::GW_CONTRACT_32>(wide, stream);
+        else
+            status = few ? launch_product<false, kmc::GW_EPILOGUE_DISTANCE + kmc::GW_CONTRACT_16>(wide, stream) : launch_product<false, kmc::GW_EPILOGUE_DISTANCE + kmc::GW_CONTRACT_32>(wide, stream);
+        if (status == hipSuccess) *taken = true;
+        return status;
+    }
     if (args.symmetric)
         status = products ? launch_product<true, kmc::GW_EPILOGUE_DOT>(wide, stream) : launch_product<true, kmc::GW_EPILOGUE_DISTANCE>(wide, stream);
     else

@@ -40,6 +40,9 @@ struct KernelCoefficientsArgs {
     // out + z * out_split_stride; the caller adds the ranges.  One range: the whole product.
     int split_tiles;
     i64 out_split_stride;
+    // Null, or (one tile of centres per range): the tiles to compute, [batch][tile m][tile n], the others are left alone.  The repair launch
+    // behind the contraction in gram_f16_wide.
+    const int *stamps;
 };
 
 // First centre and one past the last centre of the range this workgroup walks.
@@ -87,6 +90,7 @@ __global__ __launch_bounds__(BK_THREADS, COLUMNS == KC_COLUMNS ? KC_MIN_WAVES : 
     const int tx = tid & 15;
     const int ty = tid >> 4;
     const int batch = blockIdx.y / kc.o_chunks;
+    if (kc.stamps && kc.stamps[((i64)batch * gridDim.x + blockIdx.x) * gridDim.z + blockIdx.z] == 0) return;
     const int o_base = (blockIdx.y % kc.o_chunks) * COLUMNS;
     const int m0 = blockIdx.x * BK_TILE_M;
     const int m_valid = args.m - m0;

@@ -358,6 +358,8 @@ def _run_in_panels(plan, shape, stream, device, debug):
 
     rows, panels, ld, splits, route = shape
     L, M, N, O = plan.L, plan.M, plan.N, plan.O
+    if route and _products_of_tiles(plan, shape, stream, device, debug):
+        return True
     parts = panels * splits                                      # 0: no partial products, the panels accumulate
     params = plan.params
     block = _backend.BuildKernelParams.from_buffer_copy(params.kernel)
@@ -436,6 +438,48 @@ def _run_in_panels(plan, shape, stream, device, debug):
     if partial is not None:
         _sum_partials(partial, plan.out)
     plan.keepalive += [panel, partial, workspace, product]
+    return True
+
+
+# Up to 32 columns: the panel is not stored but contracted tile by tile where it is made (include/kermac_amd.h, KMC_FLAG_PRODUCT_PIECES).
+_PRODUCTS_OF_TILES_MAX_COLUMNS = 32
+
+
+def _products_of_tiles(plan, shape, stream, device, debug):
+    """The product in the panels of `shape` without the panels; False when it cannot be (more columns, no memory)."""
+    from .build_a_kernel import _centre_wanted
+
+    rows, panels, _, splits, route = shape
+    if plan.O > _PRODUCTS_OF_TILES_MAX_COLUMNS or os.environ.get("KERMAC_AMD_PRODUCTS_OF_TILES", "1") in ("", "0"):
+        return False
+    params = _backend.KernelCoefficientsParams.from_buffer_copy(plan.params)
+    kernel = params.kernel
+    kernel.flags |= route | _backend.FLAG_PRODUCT_PIECES
+    if kernel.flags & _backend.FLAG_L2_GRAM_BF16 and _centre_wanted():
+        kernel.flags |= _backend.FLAG_GRAM_OWN_CENTRE
+    if os.environ.get("KERMAC_AMD_L2_PROBE", "1") in ("", "0"):
+        kernel.flags |= _backend.FLAG_NO_PROBE
+    if os.environ.get("KERMAC_AMD_L2_WORKSPACE", "1") in ("", "0"):
+        return False
+    kernel.n = rows
+    needed = _backend.kernel_coefficients_workspace_bytes(params)
+    workspace = _scratch.allocate(needed, device) if needed else None
+    if workspace is None:
+        return False
+    kernel.gram_workspace, kernel.gram_workspace_bytes = workspace.data_ptr(), needed
+    if debug:
+        print(f"(Kermac Debug) Kernel matrix x coefficients in {panels} panels of {rows} centres, {splits} partial products each, "
+              "contracted where they are made")
+    first_b, first_offset = kernel.b, kernel.regularization_offset_y
+    for index in range(panels):
+        n0 = index * rows
+        kernel.n = min(rows, plan.N - n0)
+        kernel.b = first_b + 4 * n0 * (kernel.b_ld if kernel.b_majorness == _backend.ROW_MAJOR else 1)
+        kernel.regularization_offset_y = first_offset + n0
+        params.coef = plan.params.coef + 4 * n0 * plan.params.coef_ld
+        _backend.kernel_times_coefficients(params, stream)
+        kernel.flags |= _backend.FLAG_GRAM_A_KEPT | _backend.FLAG_PRODUCT_ACCUMULATE       # the rows are the same for every panel: split once
+    plan.keepalive.append(workspace)
     return True
 
 
