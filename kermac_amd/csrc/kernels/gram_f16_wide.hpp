@@ -8,6 +8,7 @@
 //
 //   gram_row_stats   per row of an operand: sum of squares (the norms of the expansion) and
 //                    largest magnitude, both after the centre has been subtracted.
+//                    (Operands of up to 1024 k: both steps in one pass, gram_rows_once and gram_columns_once.)
 //   gram_f16_split   scales every row by a power of two that puts its largest magnitude into
 //                    [2^14, 2^15), splits every scaled value x into h1 = fp16(x), h2 = fp16(x - h1)
 //                    and writes the pieces in the order the matrix instruction reads them.
@@ -165,12 +166,14 @@ __device__ __forceinline__ void gram_row_stats_of(const GramRowsArgs &args, int 
     for (int slice = first; slice < last; slice++) {
         float v[BK_TILE_K];
         gram_load_row_slice(args, x, centre, row, slice, v);
+        float of_slice = 0.0f;                              // its own sum first: a longer one rounds more
 #pragma unroll
         for (int e = 0; e < BK_TILE_K; e++) {
-            square += v[e] * v[e];
+            of_slice += v[e] * v[e];
             magnitude = fmaxf(magnitude, fabsf(v[e]));      // skips NaNs
             not_a_number |= v[e] != v[e];
         }
+        square += of_slice;
     }
     const i64 at = batch * args.stats_bs + (i64)range * args.rows_pad + row;
     args.squares[at] = square;
@@ -414,6 +417,106 @@ __global__ __launch_bounds__(GW_ROW_THREADS, 2) void gram_rows_once(const GramRo
     const bool first = block < args.first_blocks;
     if ((int)blockIdx.z < (first ? args.first_batches : args.second_batches))
         gram_rows_once_of<GROUPS>(first ? args.first : args.second, first ? block : block - args.first_blocks);
+}
+
+// The same for operands with the rows contiguous: a workgroup holds 32 whole rows, a line of memory per k.  Wave w takes the slices w, w + 4, ..; a half
+// wave has one half of each, so that a lane makes whole chunks.  In place of gram_row_stats_pair, gram_f16_split_pair and the sample in three launches, which read
+// the operands twice: 30000 + 30000 rows of K = 1024 178 -> 121 us and the call 4911 -> 4753, calls of 2000 x 2000 x 784 64 -> 43.5, 4000 x 4000 x 256
+// 77 -> 51, 2 x 1503 x 1503 x 128 57 -> 34.5, 8000 x 8000 x 512 235 -> 212, 10000 x 10000 x 128 188 -> 155 (with the centre in one launch).
+constexpr int GCO_ROWS = 32;                                  // per workgroup
+
+template <int GROUPS>
+__device__ __forceinline__ void gram_columns_once_of(const GramRowsArgs &args, int block)
+{
+    __shared__ float squares[GRO_WAVES][GCO_ROWS], magnitudes[GRO_WAVES][GCO_ROWS];
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), r = threadIdx.x & 31, half = (threadIdx.x >> 5) & 1;
+    const int row = block * GCO_ROWS + r, batch = blockIdx.z;
+    const bool live = row < args.rows;
+    const float *src = args.x + batch * args.bs + (live ? row : args.rows - 1);
+    const float *centre = args.centre ? args.centre + batch * args.centre_bs : nullptr;
+    CentreSums sums;
+    if (centre && args.centre_pairs) sums.load(centre, args.k, args.centre_pairs);
+    float v[GROUPS][8];
+#pragma unroll
+    for (int g = 0; g < GROUPS; g++) {
+        const int slice = wave + GRO_WAVES * g, k0 = BK_TILE_K * slice + 8 * half;
+        if (BK_TILE_K * (slice + 1) <= args.k) {              // uniform: a wave has whole slices
+            const float *from = src + (i64)k0 * args.ld;
+#pragma unroll
+            for (int e = 0; e < 8; e++) v[g][e] = from[e * args.ld];
+        } else {
+            // loads of what does not exist go to the last k that does, as in gram_rows_once_of
+#pragma unroll
+            for (int e = 0; e < 8; e++) v[g][e] = src[(i64)min(k0 + e, args.k - 1) * args.ld];
+        }
+    }
+    if (centre && args.centre_pairs ? !sums.needless() : gram_rows_centre(args, batch) != nullptr) {
+        // padded with zeros to whole groups of 64 k, and 16-byte aligned
+        const int last = (args.k + GRAM_CENTRE_PAD - 1) / GRAM_CENTRE_PAD * GRAM_CENTRE_PAD - 8;
+#pragma unroll
+        for (int g = 0; g < GROUPS; g++) {
+            const float4 *of = reinterpret_cast<const float4 *>(centre + min(BK_TILE_K * (wave + GRO_WAVES * g) + 8 * half, last));
+            const float4 lo = of[0], hi = of[1];
+            v[g][0] -= lo.x; v[g][1] -= lo.y; v[g][2] -= lo.z; v[g][3] -= lo.w;
+            v[g][4] -= hi.x; v[g][5] -= hi.y; v[g][6] -= hi.z; v[g][7] -= hi.w;
+        }
+    }
+    float square = 0.0f, magnitude = 0.0f;
+    bool not_a_number = false;
+#pragma unroll
+    for (int g = 0; g < GROUPS; g++) {
+        const int k0 = BK_TILE_K * (wave + GRO_WAVES * g) + 8 * half;
+        float of_group = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            v[g][e] = live && k0 + e < args.k ? v[g][e] : 0.0f;
+            of_group += v[g][e] * v[g][e];
+            magnitude = fmaxf(magnitude, fabsf(v[g][e]));      // skips NaNs
+            not_a_number |= v[g][e] != v[g][e];
+        }
+        square += of_group;
+    }
+    if (not_a_number) magnitude = __builtin_inff();            // takes the same scale as a NaN
+    square += __shfl_xor(square, 32);
+    magnitude = fmaxf(magnitude, __shfl_xor(magnitude, 32));
+    if (half == 0) {
+        squares[wave][r] = square;
+        magnitudes[wave][r] = magnitude;
+    }
+    __syncthreads();
+    magnitude = fmaxf(fmaxf(magnitudes[0][r], magnitudes[1][r]), fmaxf(magnitudes[2][r], magnitudes[3][r]));
+    const int exponent_field = gram_scale_exponent(magnitude);
+    const float scale = gram_scale(exponent_field);
+    if (threadIdx.x < GCO_ROWS) {
+        args.squares[batch * args.stats_bs + row] = (squares[0][r] + squares[1][r]) + (squares[2][r] + squares[3][r]);
+        args.unscale[batch * args.unscale_bs + row] = gram_unscale(exponent_field);
+    }
+    gram_chunk *pieces = args.pieces + batch * args.pieces_bs;
+    const int all_slices = args.slices + args.zero_slices;
+#pragma unroll
+    for (int g = 0; g < GROUPS; g++) {
+        const int slice = wave + GRO_WAVES * g;
+        if (slice >= all_slices) break;
+        unsigned h1[4], h2[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) gram_split_pair(v[g][2 * q] * scale, v[g][2 * q + 1] * scale, h1[q], h2[q]);
+        gram_chunk *dst = pieces + ((i64)slice * GW_SEGMENTS + half) * args.rows_pad + row;
+        dst[0] = gram_chunk{h1[0], h1[1], h1[2], h1[3]};
+        dst[2 * (i64)args.rows_pad] = gram_chunk{h2[0], h2[1], h2[2], h2[3]};
+    }
+}
+
+template <int GROUPS>
+__global__ __launch_bounds__(GW_ROW_THREADS, 2) void gram_columns_once(const GramRowsOnceArgs args)
+{
+    const int block = (int)blockIdx.x - args.samples;
+    if (block < 0) {
+        if (blockIdx.z == 0) gram_probe_tile(args.probe, blockIdx.x);
+        return;
+    }
+    const bool first = block < args.first_blocks;
+    if ((int)blockIdx.z < (first ? args.first_batches : args.second_batches))
+        gram_columns_once_of<GROUPS>(first ? args.first : args.second, first ? block : block - args.first_blocks);
 }
 
 // Tile shapes of the product kernel.  A workgroup is 4 waves (8: EightWaves); a wave owns WAVE_M rows of a and WAVE_N rows of b as

@@ -132,20 +132,19 @@ void place_operand(OperandRegions &r, int rows, bool broadcast, int l, bool once
 }
 
 // Grid, slices and the regions of both operands in the workspace; tiles_m and tiles_n are set.
-// a_shared, b_shared: one operand for all batch entries.  a_rows, b_rows: its k are contiguous, so that one pass can make the
-// pieces of a short row (gram_rows_once).
-bool place_wide(int m, int n, int k, int l, bool a_shared, bool b_shared, bool a_rows, bool b_rows, bool symmetric, WideLayout *layout)
+// a_shared, b_shared: one operand for all batch entries.  once: one pass makes the pieces of a short row (gram_rows_once, gram_columns_once).
+bool place_wide(int m, int n, int k, int l, bool a_shared, bool b_shared, bool once, bool symmetric, WideLayout *layout)
 {
     // room for any tile of the product kernel in a grid, n tiles padded to the XCDs
     if (static_cast<int64_t>(layout->tiles_m) * (layout->tiles_n + kmc::BK_XCDS) * 4 > 0x7fffffff) return false;
     layout->slices = (k + kmc::BK_TILE_K - 1) / kmc::BK_TILE_K;
     int64_t cursor = 0;
     const bool fits = k <= kmc::GRO_MAX_K;
-    place_operand(layout->a, m, a_shared, l, a_rows && fits, *layout, cursor);
+    place_operand(layout->a, m, a_shared, l, once && fits, *layout, cursor);
     // behind the region of a, where it stays when b grows or shrinks: the split of a may be kept
     layout->centre = layout->centre_floats ? place(cursor, 4 * layout->centre_floats * layout->centre_batches) : 0;
     if (symmetric) layout->b = layout->a;      // one panel, split once
-    else place_operand(layout->b, n, b_shared, l, b_rows && fits, *layout, cursor);
+    else place_operand(layout->b, n, b_shared, l, once && fits, *layout, cursor);
     layout->sample = place(cursor, kmc::BK_SAMPLE_BYTES);
     layout->bytes = cursor;
     return true;
@@ -171,8 +170,7 @@ bool wide_layout(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &a
     layout->centre_batches = own_centre && args.a_bs != 0 ? args.l : 1;
     layout->centre_floats = own_centre ? 2 * ((args.k + kmc::GRAM_CENTRE_PAD - 1) / kmc::GRAM_CENTRE_PAD * kmc::GRAM_CENTRE_PAD) + kmc::GRAM_CENTRE_PAD : 0;
     const bool one_centre = products || (own_centre ? layout->centre_batches == 1 : !args.centre || args.centre_bs == 0);
-    return place_wide(args.m, args.n, args.k, args.l, args.a_bs == 0 && one_centre, args.b_bs == 0 && one_centre,
-                      p->a_majorness == KMC_ROW_MAJOR, p->b_majorness == KMC_ROW_MAJOR, args.symmetric, layout);
+    return place_wide(args.m, args.n, args.k, args.l, args.a_bs == 0 && one_centre, args.b_bs == 0 && one_centre, true, args.symmetric, layout);
 }
 
 kmc::GramRowsArgs rows_args(const float *x, int64_t ld, int64_t bs, int rows, int majorness, bool scalar_only,
@@ -274,30 +272,45 @@ hipError_t launch_gram_rows_pair(const kmc::GramRowsArgs &first, int first_batch
     return launch(kmc::gram_f16_split_pair<0>, grid, dim3(kmc::GW_ROW_THREADS), stream, pair);
 }
 
-// The pieces of the operands that are not null, and in front of them the sample if there is one, in one launch.
-hipError_t launch_gram_rows_once(const kmc::GramRowsArgs *first, int first_batches, const kmc::GramRowsArgs *second, int second_batches,
-                                 const kmc::GramProbeArgs &probe, bool take_sample, hipStream_t stream)
+// The pieces of the operands that are not null and of one storage order, and in front of them the sample if there is one, in one launch.
+hipError_t launch_gram_once(const kmc::GramRowsArgs *first, int first_batches, const kmc::GramRowsArgs *second, int second_batches,
+                            const kmc::GramProbeArgs &probe, bool take_sample, hipStream_t stream)
 {
+    const bool rows = (first ? first : second)->row_major;
+    const int rows_per_block = rows ? kmc::GRO_ROWS : kmc::GCO_ROWS;
     kmc::GramRowsOnceArgs args = {};
     args.probe = probe;
     args.samples = take_sample ? kmc::BK_SAMPLE_TILES : 0;
     int blocks = args.samples, k = 0, batches = 1;
     if (first) {
         args.first = *first; args.first_batches = batches = first_batches;
-        args.first_blocks = first->rows_pad / kmc::GRO_ROWS;
+        args.first_blocks = first->rows_pad / rows_per_block;
         blocks += args.first_blocks;
         k = first->k;
     }
     if (second) {
         args.second = *second; args.second_batches = second_batches;
         if (second_batches > batches) batches = second_batches;
-        blocks += second->rows_pad / kmc::GRO_ROWS;
+        blocks += second->rows_pad / rows_per_block;
         k = second->k;
     }
     const dim3 grid(blocks, 1, batches), threads(kmc::GW_ROW_THREADS);
-    // registers for 64, 128 or 256 values of a row per lane group: the smallest that holds a row
-    return k <= 256 ? launch(kmc::gram_rows_once<4>, grid, threads, stream, args)
-         : k <= 512 ? launch(kmc::gram_rows_once<8>, grid, threads, stream, args) : launch(kmc::gram_rows_once<16>, grid, threads, stream, args);
+    // registers for 256, 512 or 1024 k: the smallest that holds a row
+    if (rows)
+        return k <= 256 ? launch(kmc::gram_rows_once<4>, grid, threads, stream, args)
+             : k <= 512 ? launch(kmc::gram_rows_once<8>, grid, threads, stream, args) : launch(kmc::gram_rows_once<16>, grid, threads, stream, args);
+    return k <= 256 ? launch(kmc::gram_columns_once<4>, grid, threads, stream, args)
+         : k <= 512 ? launch(kmc::gram_columns_once<8>, grid, threads, stream, args) : launch(kmc::gram_columns_once<16>, grid, threads, stream, args);
+}
+
+// Both operands, in one launch if they are stored alike; the sample in the first.
+hipError_t launch_gram_once_both(const kmc::GramRowsArgs *first, int first_batches, const kmc::GramRowsArgs *second, int second_batches,
+                                 const kmc::GramProbeArgs &probe, bool take_sample, hipStream_t stream)
+{
+    if (!first || !second || first->row_major == second->row_major)
+        return launch_gram_once(first, first_batches, second, second_batches, probe, take_sample, stream);
+    const hipError_t status = launch_gram_once(first, first_batches, nullptr, 0, probe, take_sample, stream);
+    return status != hipSuccess ? status : launch_gram_once(nullptr, 0, second, second_batches, probe, false, stream);
 }
 
 // The product kernel in tiles of TILE; extents, batch entries and operands of `wide` are set.
@@ -447,7 +460,7 @@ hipError_t launch_gram_f16_wide(const kmc_build_kernel_params *p, const kmc::Bui
                                      reinterpret_cast<float *>(workspace + layout.centre), layout.centre_floats, stream);
     if (status != hipSuccess) return status;
     if ((split_a && layout.a.once) || (split_b && layout.b.once)) {
-        status = launch_gram_rows_once(split_a && layout.a.once ? &rows_a : nullptr, layout.a.batches, split_b && layout.b.once ? &rows_b : nullptr,
+        status = launch_gram_once_both(split_a && layout.a.once ? &rows_a : nullptr, layout.a.batches, split_b && layout.b.once ? &rows_b : nullptr,
                                        layout.b.batches, sample ? gram_probe_args(p, wide.kernel, sample, centre_pairs) : kmc::GramProbeArgs{}, sample != nullptr, stream);
         sampled = true;
     }
@@ -555,7 +568,7 @@ bool gradient_l2_layout(const kmc_norm_gradient_params *p, GradientL2Layout *lay
     wide.tiles_m = (p->m + kmc::GW_TILE - 1) / kmc::GW_TILE;
     wide.tiles_n = static_cast<int>((rows + kmc::GW_TILE - 1) / kmc::GW_TILE);
     if (!gradient_l2_pays(p, wide.tiles_m, wide.tiles_n)) return false;
-    if (!place_wide(p->m, static_cast<int>(rows), p->k, p->l, p->a_bs == 0, false, false, false, false, &wide)) return false;
+    if (!place_wide(p->m, static_cast<int>(rows), p->k, p->l, p->a_bs == 0, false, false, false, &wide)) return false;
     int64_t cursor = wide.bytes;
     layout->shift = place(cursor, static_cast<int64_t>(p->l) * p->n * 4);
     layout->c_transposed = place(cursor, static_cast<int64_t>(p->l) * p->k * p->o * 4);
