@@ -8,7 +8,7 @@
 //
 //   gram_row_stats   per row of an operand: sum of squares (the norms of the expansion) and
 //                    largest magnitude, both after the centre has been subtracted.
-//                    (Operands of up to 1024 k: both steps in one pass, gram_rows_once and gram_columns_once.)
+//                    (As a rule by one launch, gram_rows_once or gram_columns_once.)
 //   gram_f16_split   scales every row by a power of two that puts its largest magnitude into
 //                    [2^14, 2^15), splits every scaled value x into h1 = fp16(x), h2 = fp16(x - h1)
 //                    and writes the pieces in the order the matrix instruction reads them.
@@ -290,7 +290,7 @@ __global__ __launch_bounds__(GW_ROW_THREADS) void gram_f16_split_pair(const Gram
     }
 }
 
-// Both steps in one pass for operands with k contiguous and at most GRO_MAX_K of them: a workgroup holds 16 whole rows in its
+// Both steps in one pass for operands with k contiguous and up to 2048 of them: a workgroup holds 16 whole rows in its
 // registers, so the values are read once and the scale is known before the pieces are written.  Wave w takes the slices w,
 // w + 4, ..; four lanes share a slice of a row, 4 k each (a load instruction reads 64 consecutive bytes of 16 rows, the four
 // waves together 256); two neighbours exchange halves so that one stores the chunk of the first piece and the other that
@@ -301,7 +301,8 @@ __global__ __launch_bounds__(GW_ROW_THREADS) void gram_f16_split_pair(const Gram
 // 1000 + 60000 rows of K = 784 53 + 89 + 12 -> 110 us, 10000 rows 12 + 13 + 10 -> 27 us, 2 x 2000 rows 10 + 12 + 11 -> 18 us.
 constexpr int GRO_ROWS = 16;                                  // per workgroup
 constexpr int GRO_WAVES = GW_ROW_THREADS / 64;
-constexpr int GRO_MAX_K = 1024;
+constexpr int GRO_HELD_K = 1024;                              // k of a row in the registers: twice as many in the widest gram_rows_once
+constexpr int GRO_MAX_K = 8192;                               // ... and in all
 
 struct GramRowsOnceArgs {
     GramRowsArgs first, second;
@@ -310,7 +311,90 @@ struct GramRowsOnceArgs {
     GramProbeArgs probe;
 };
 
+// The values of a lane of a row workgroup: 4 k of every 64 from k_base on, of row `row`, with the centre subtracted; zeros where the row or k does not exist.
 template <int GROUPS>
+struct RowValues {
+    float v[GROUPS][4];
+
+    __device__ __forceinline__ void load(const GramRowsArgs &args, const float *src, int k0)
+    {
+        // Loads of what does not exist go to the last element that does and are dropped: with a branch per load they would be
+        // waited for one by one (198 instead of 110 us for 61000 rows).
+        if (args.vec && args.k % 4 == 0) {
+#pragma unroll
+            for (int g = 0; g < GROUPS; g++) {
+                const float4 f = *reinterpret_cast<const float4 *>(src + min(64 * g + k0, args.k - 4));
+                v[g][0] = f.x; v[g][1] = f.y; v[g][2] = f.z; v[g][3] = f.w;
+            }
+        } else {
+#pragma unroll
+            for (int g = 0; g < GROUPS; g++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) v[g][e] = src[min(64 * g + k0 + e, args.k - 1)];
+        }
+    }
+    __device__ __forceinline__ void centre(const GramRowsArgs &args, const float *centre, int k0, bool subtract, bool live)
+    {
+        if (subtract) {
+            // padded with zeros to whole groups of 64 k
+            const bool aligned = (reinterpret_cast<unsigned long>(centre) & 15) == 0;
+            const int last = (args.k + 63) / 64 * 64 - 4;
+            if (aligned) {
+#pragma unroll
+                for (int g = 0; g < GROUPS; g++) {
+                    const float4 f = *reinterpret_cast<const float4 *>(centre + min(64 * g + k0, last));
+                    v[g][0] -= f.x; v[g][1] -= f.y; v[g][2] -= f.z; v[g][3] -= f.w;
+                }
+            } else {
+#pragma unroll
+                for (int g = 0; g < GROUPS; g++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) v[g][e] -= centre[min(64 * g + k0, last) + e];
+            }
+        }
+#pragma unroll
+        for (int g = 0; g < GROUPS; g++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[g][e] = live && 64 * g + k0 + e < args.k ? v[g][e] : 0.0f;
+    }
+    __device__ __forceinline__ void statistics(float &square, float &magnitude) const
+    {
+        bool not_a_number = false;
+        float of_chunk = 0.0f;
+#pragma unroll
+        for (int g = 0; g < GROUPS; g++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                of_chunk += v[g][e] * v[g][e];
+                magnitude = fmaxf(magnitude, fabsf(v[g][e]));      // skips NaNs
+                not_a_number |= v[g][e] != v[g][e];
+            }
+        square += of_chunk;
+        if (not_a_number) magnitude = __builtin_inff();            // takes the same scale as a NaN
+    }
+    // the chunks of slices slice0, slice0 + 4, ..; two neighbours exchange halves
+    __device__ __forceinline__ void split(const GramRowsArgs &args, gram_chunk *pieces, int row, int slice0, int quarter, float scale) const
+    {
+        const int all_slices = args.slices + args.zero_slices;
+        const bool second = quarter & 1;
+        const int segment = 2 * (second ? 1 : 0) + (quarter >> 1);
+#pragma unroll
+        for (int g = 0; g < GROUPS; g++) {
+            const int slice = 4 * g + slice0;
+            unsigned h1[2], h2[2];
+#pragma unroll
+            for (int q = 0; q < 2; q++) gram_split_pair(v[g][2 * q] * scale, v[g][2 * q + 1] * scale, h1[q], h2[q]);
+            // the even lane holds the first half of both pieces' chunks, the odd one the second half
+            const unsigned give0 = second ? h1[0] : h2[0], give1 = second ? h1[1] : h2[1];
+            const unsigned got0 = (unsigned)__shfl_xor((int)give0, 1), got1 = (unsigned)__shfl_xor((int)give1, 1);
+            const gram_chunk chunk = second ? gram_chunk{got0, got1, h2[0], h2[1]} : gram_chunk{h1[0], h1[1], got0, got1};
+            if (slice < all_slices) pieces[((i64)slice * GW_SEGMENTS + segment) * args.rows_pad + row] = chunk;
+        }
+    }
+};
+
+// LONG: rows of more than 64 GROUPS k, in chunks of that many: read for the statistics, and once more, as a rule from a cache, for the pieces.
+template <int GROUPS, bool LONG>
 __device__ __forceinline__ void gram_rows_once_of(const GramRowsArgs &args, int block)
 {
     __shared__ float squares[GRO_WAVES][GRO_ROWS], magnitudes[GRO_WAVES][GRO_ROWS];
@@ -321,55 +405,20 @@ __device__ __forceinline__ void gram_rows_once_of(const GramRowsArgs &args, int 
     const float *centre = args.centre ? args.centre + batch * args.centre_bs : nullptr;
     CentreSums sums;
     if (centre && args.centre_pairs) sums.load(centre, args.k, args.centre_pairs);
-    const int groups = (args.k + 63) / 64;
     const int k0 = BK_TILE_K * wave + 4 * quarter;             // and every 64 behind it
-    float v[GROUPS][4];
-    // Loads of what does not exist go to the last element that does and are dropped: with a branch per load they would be
-    // waited for one by one (198 instead of 110 us for 61000 rows).
-    if (args.vec && args.k % 4 == 0) {
-#pragma unroll
-        for (int g = 0; g < GROUPS; g++) {
-            const float4 f = *reinterpret_cast<const float4 *>(src + min(64 * g + k0, args.k - 4));
-            v[g][0] = f.x; v[g][1] = f.y; v[g][2] = f.z; v[g][3] = f.w;
-        }
-    } else {
-#pragma unroll
-        for (int g = 0; g < GROUPS; g++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) v[g][e] = src[min(64 * g + k0 + e, args.k - 1)];
-    }
-    if (centre && args.centre_pairs ? !sums.needless() : gram_rows_centre(args, batch) != nullptr) {
-        // padded with zeros to whole groups of 64 k
-        const bool aligned = (reinterpret_cast<unsigned long>(centre) & 15) == 0;
-        const int last = 64 * (groups - 1);
-        if (aligned) {
-#pragma unroll
-            for (int g = 0; g < GROUPS; g++) {
-                const float4 f = *reinterpret_cast<const float4 *>(centre + min(64 * g, last) + k0);
-                v[g][0] -= f.x; v[g][1] -= f.y; v[g][2] -= f.z; v[g][3] -= f.w;
-            }
-        } else {
-#pragma unroll
-            for (int g = 0; g < GROUPS; g++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) v[g][e] -= centre[min(64 * g, last) + k0 + e];
-        }
-    }
-#pragma unroll
-    for (int g = 0; g < GROUPS; g++)
-#pragma unroll
-        for (int e = 0; e < 4; e++) v[g][e] = live && 64 * g + k0 + e < args.k ? v[g][e] : 0.0f;
+    constexpr int CHUNK = 64 * GROUPS;
+    RowValues<GROUPS> values;
+    values.load(args, src, k0);
+    const bool subtract = centre && args.centre_pairs ? !sums.needless() : gram_rows_centre(args, batch) != nullptr;
+    values.centre(args, centre, k0, subtract, live);
     float square = 0.0f, magnitude = 0.0f;
-    bool not_a_number = false;
-#pragma unroll
-    for (int g = 0; g < GROUPS; g++)
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            square += v[g][e] * v[g][e];
-            magnitude = fmaxf(magnitude, fabsf(v[g][e]));      // skips NaNs
-            not_a_number |= v[g][e] != v[g][e];
+    values.statistics(square, magnitude);
+    if constexpr (LONG)
+        for (int at = CHUNK; at < args.k; at += CHUNK) {
+            values.load(args, src, at + k0);
+            values.centre(args, centre, at + k0, subtract, live);
+            values.statistics(square, magnitude);
         }
-    if (not_a_number) magnitude = __builtin_inff();            // takes the same scale as a NaN
 #pragma unroll
     for (int offset = 2; offset > 0; offset >>= 1) {
         square += __shfl_xor(square, offset);
@@ -388,24 +437,21 @@ __device__ __forceinline__ void gram_rows_once_of(const GramRowsArgs &args, int 
         args.unscale[batch * args.unscale_bs + row] = gram_unscale(exponent_field);
     }
     gram_chunk *pieces = args.pieces + batch * args.pieces_bs;
-    const int all_slices = args.slices + args.zero_slices;
-    const bool second = quarter & 1;
-    const int segment = 2 * (second ? 1 : 0) + (quarter >> 1);
-#pragma unroll
-    for (int g = 0; g < GROUPS; g++) {
-        const int slice = 4 * g + wave;
-        unsigned h1[2], h2[2];
-#pragma unroll
-        for (int q = 0; q < 2; q++) gram_split_pair(v[g][2 * q] * scale, v[g][2 * q + 1] * scale, h1[q], h2[q]);
-        // the even lane holds the first half of both pieces' chunks, the odd one the second half
-        const unsigned give0 = second ? h1[0] : h2[0], give1 = second ? h1[1] : h2[1];
-        const unsigned got0 = (unsigned)__shfl_xor((int)give0, 1), got1 = (unsigned)__shfl_xor((int)give1, 1);
-        const gram_chunk chunk = second ? gram_chunk{got0, got1, h2[0], h2[1]} : gram_chunk{h1[0], h1[1], got0, got1};
-        if (slice < all_slices) pieces[((i64)slice * GW_SEGMENTS + segment) * args.rows_pad + row] = chunk;
+    if constexpr (LONG) {
+        // the last chunk is still here: backwards, so that the next one is the one read last
+        const int last = (args.k - 1) / CHUNK * CHUNK;
+        values.split(args, pieces, row, last / BK_TILE_K + wave, quarter, scale);
+        for (int at = last - CHUNK; at >= 0; at -= CHUNK) {
+            values.load(args, src, at + k0);
+            values.centre(args, centre, at + k0, subtract, live);
+            values.split(args, pieces, row, at / BK_TILE_K + wave, quarter, scale);
+        }
+    } else {
+        values.split(args, pieces, row, wave, quarter, scale);
     }
 }
 
-template <int GROUPS>
+template <int GROUPS, bool LONG = false>
 __global__ __launch_bounds__(GW_ROW_THREADS, 2) void gram_rows_once(const GramRowsOnceArgs args)
 {
     static_assert(GW_ROW_THREADS == GP_THREADS, "both parts of the launch");
@@ -416,7 +462,7 @@ __global__ __launch_bounds__(GW_ROW_THREADS, 2) void gram_rows_once(const GramRo
     }
     const bool first = block < args.first_blocks;
     if ((int)blockIdx.z < (first ? args.first_batches : args.second_batches))
-        gram_rows_once_of<GROUPS>(first ? args.first : args.second, first ? block : block - args.first_blocks);
+        gram_rows_once_of<GROUPS, LONG>(first ? args.first : args.second, first ? block : block - args.first_blocks);
 }
 
 // The same for operands with the rows contiguous: a workgroup holds 32 whole rows, a line of memory per k.  Wave w takes the slices w, w + 4, ..; a half
@@ -425,7 +471,82 @@ __global__ __launch_bounds__(GW_ROW_THREADS, 2) void gram_rows_once(const GramRo
 // 77 -> 51, 2 x 1503 x 1503 x 128 57 -> 34.5, 8000 x 8000 x 512 235 -> 212, 10000 x 10000 x 128 188 -> 155 (with the centre in one launch).
 constexpr int GCO_ROWS = 32;                                  // per workgroup
 
+// The values of a lane of such a workgroup: one half of the slices slice0, slice0 + 4, .. of a row.
 template <int GROUPS>
+struct ColumnValues {
+    float v[GROUPS][8];
+
+    __device__ __forceinline__ void load(const GramRowsArgs &args, const float *src, int slice0, int half)
+    {
+#pragma unroll
+        for (int g = 0; g < GROUPS; g++) {
+            const int slice = slice0 + GRO_WAVES * g, k0 = BK_TILE_K * slice + 8 * half;
+            if (BK_TILE_K * (slice + 1) <= args.k) {              // uniform: a wave has whole slices
+                const float *from = src + (i64)k0 * args.ld;
+#pragma unroll
+                for (int e = 0; e < 8; e++) v[g][e] = from[e * args.ld];
+            } else {
+                // loads of what does not exist go to the last k that does, as in RowValues
+#pragma unroll
+                for (int e = 0; e < 8; e++) v[g][e] = src[(i64)min(k0 + e, args.k - 1) * args.ld];
+            }
+        }
+    }
+    __device__ __forceinline__ void centre(const GramRowsArgs &args, const float *centre, int slice0, int half, bool subtract, bool live)
+    {
+        if (subtract) {
+            // padded with zeros to whole groups of 64 k, and 16-byte aligned
+            const int last = (args.k + GRAM_CENTRE_PAD - 1) / GRAM_CENTRE_PAD * GRAM_CENTRE_PAD - 8;
+#pragma unroll
+            for (int g = 0; g < GROUPS; g++) {
+                const float4 *of = reinterpret_cast<const float4 *>(centre + min(BK_TILE_K * (slice0 + GRO_WAVES * g) + 8 * half, last));
+                const float4 lo = of[0], hi = of[1];
+                v[g][0] -= lo.x; v[g][1] -= lo.y; v[g][2] -= lo.z; v[g][3] -= lo.w;
+                v[g][4] -= hi.x; v[g][5] -= hi.y; v[g][6] -= hi.z; v[g][7] -= hi.w;
+            }
+        }
+#pragma unroll
+        for (int g = 0; g < GROUPS; g++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) v[g][e] = live && BK_TILE_K * (slice0 + GRO_WAVES * g) + 8 * half + e < args.k ? v[g][e] : 0.0f;
+    }
+    __device__ __forceinline__ void statistics(float &square, float &magnitude) const
+    {
+        bool not_a_number = false;
+        float of_chunk = 0.0f;
+#pragma unroll
+        for (int g = 0; g < GROUPS; g++) {
+            float of_group = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                of_group += v[g][e] * v[g][e];
+                magnitude = fmaxf(magnitude, fabsf(v[g][e]));      // skips NaNs
+                not_a_number |= v[g][e] != v[g][e];
+            }
+            of_chunk += of_group;
+        }
+        square += of_chunk;
+        if (not_a_number) magnitude = __builtin_inff();            // takes the same scale as a NaN
+    }
+    __device__ __forceinline__ void split(const GramRowsArgs &args, gram_chunk *pieces, int row, int slice0, int half, float scale) const
+    {
+        const int all_slices = args.slices + args.zero_slices;
+#pragma unroll
+        for (int g = 0; g < GROUPS; g++) {
+            const int slice = slice0 + GRO_WAVES * g;
+            if (slice >= all_slices) break;
+            unsigned h1[4], h2[4];
+#pragma unroll
+            for (int q = 0; q < 4; q++) gram_split_pair(v[g][2 * q] * scale, v[g][2 * q + 1] * scale, h1[q], h2[q]);
+            gram_chunk *dst = pieces + ((i64)slice * GW_SEGMENTS + half) * args.rows_pad + row;
+            dst[0] = gram_chunk{h1[0], h1[1], h1[2], h1[3]};
+            dst[2 * (i64)args.rows_pad] = gram_chunk{h2[0], h2[1], h2[2], h2[3]};
+        }
+    }
+};
+
+// LONG: as in gram_rows_once_of, in chunks of 64 GROUPS k.
+template <int GROUPS, bool LONG>
 __device__ __forceinline__ void gram_columns_once_of(const GramRowsArgs &args, int block)
 {
     __shared__ float squares[GRO_WAVES][GCO_ROWS], magnitudes[GRO_WAVES][GCO_ROWS];
@@ -436,47 +557,19 @@ __device__ __forceinline__ void gram_columns_once_of(const GramRowsArgs &args, i
     const float *centre = args.centre ? args.centre + batch * args.centre_bs : nullptr;
     CentreSums sums;
     if (centre && args.centre_pairs) sums.load(centre, args.k, args.centre_pairs);
-    float v[GROUPS][8];
-#pragma unroll
-    for (int g = 0; g < GROUPS; g++) {
-        const int slice = wave + GRO_WAVES * g, k0 = BK_TILE_K * slice + 8 * half;
-        if (BK_TILE_K * (slice + 1) <= args.k) {              // uniform: a wave has whole slices
-            const float *from = src + (i64)k0 * args.ld;
-#pragma unroll
-            for (int e = 0; e < 8; e++) v[g][e] = from[e * args.ld];
-        } else {
-            // loads of what does not exist go to the last k that does, as in gram_rows_once_of
-#pragma unroll
-            for (int e = 0; e < 8; e++) v[g][e] = src[(i64)min(k0 + e, args.k - 1) * args.ld];
-        }
-    }
-    if (centre && args.centre_pairs ? !sums.needless() : gram_rows_centre(args, batch) != nullptr) {
-        // padded with zeros to whole groups of 64 k, and 16-byte aligned
-        const int last = (args.k + GRAM_CENTRE_PAD - 1) / GRAM_CENTRE_PAD * GRAM_CENTRE_PAD - 8;
-#pragma unroll
-        for (int g = 0; g < GROUPS; g++) {
-            const float4 *of = reinterpret_cast<const float4 *>(centre + min(BK_TILE_K * (wave + GRO_WAVES * g) + 8 * half, last));
-            const float4 lo = of[0], hi = of[1];
-            v[g][0] -= lo.x; v[g][1] -= lo.y; v[g][2] -= lo.z; v[g][3] -= lo.w;
-            v[g][4] -= hi.x; v[g][5] -= hi.y; v[g][6] -= hi.z; v[g][7] -= hi.w;
-        }
-    }
+    constexpr int CHUNK = GRO_WAVES * GROUPS;                  // slices
+    ColumnValues<GROUPS> values;
+    values.load(args, src, wave, half);
+    const bool subtract = centre && args.centre_pairs ? !sums.needless() : gram_rows_centre(args, batch) != nullptr;
+    values.centre(args, centre, wave, half, subtract, live);
     float square = 0.0f, magnitude = 0.0f;
-    bool not_a_number = false;
-#pragma unroll
-    for (int g = 0; g < GROUPS; g++) {
-        const int k0 = BK_TILE_K * (wave + GRO_WAVES * g) + 8 * half;
-        float of_group = 0.0f;
-#pragma unroll
-        for (int e = 0; e < 8; e++) {
-            v[g][e] = live && k0 + e < args.k ? v[g][e] : 0.0f;
-            of_group += v[g][e] * v[g][e];
-            magnitude = fmaxf(magnitude, fabsf(v[g][e]));      // skips NaNs
-            not_a_number |= v[g][e] != v[g][e];
+    values.statistics(square, magnitude);
+    if constexpr (LONG)
+        for (int at = CHUNK; at < args.slices; at += CHUNK) {
+            values.load(args, src, at + wave, half);
+            values.centre(args, centre, at + wave, half, subtract, live);
+            values.statistics(square, magnitude);
         }
-        square += of_group;
-    }
-    if (not_a_number) magnitude = __builtin_inff();            // takes the same scale as a NaN
     square += __shfl_xor(square, 32);
     magnitude = fmaxf(magnitude, __shfl_xor(magnitude, 32));
     if (half == 0) {
@@ -492,21 +585,20 @@ __device__ __forceinline__ void gram_columns_once_of(const GramRowsArgs &args, i
         args.unscale[batch * args.unscale_bs + row] = gram_unscale(exponent_field);
     }
     gram_chunk *pieces = args.pieces + batch * args.pieces_bs;
-    const int all_slices = args.slices + args.zero_slices;
-#pragma unroll
-    for (int g = 0; g < GROUPS; g++) {
-        const int slice = wave + GRO_WAVES * g;
-        if (slice >= all_slices) break;
-        unsigned h1[4], h2[4];
-#pragma unroll
-        for (int q = 0; q < 4; q++) gram_split_pair(v[g][2 * q] * scale, v[g][2 * q + 1] * scale, h1[q], h2[q]);
-        gram_chunk *dst = pieces + ((i64)slice * GW_SEGMENTS + half) * args.rows_pad + row;
-        dst[0] = gram_chunk{h1[0], h1[1], h1[2], h1[3]};
-        dst[2 * (i64)args.rows_pad] = gram_chunk{h2[0], h2[1], h2[2], h2[3]};
+    if constexpr (LONG) {
+        const int last = (args.slices - 1) / CHUNK * CHUNK;
+        values.split(args, pieces, row, last + wave, half, scale);
+        for (int at = last - CHUNK; at >= 0; at -= CHUNK) {
+            values.load(args, src, at + wave, half);
+            values.centre(args, centre, at + wave, half, subtract, live);
+            values.split(args, pieces, row, at + wave, half, scale);
+        }
+    } else {
+        values.split(args, pieces, row, wave, half, scale);
     }
 }
 
-template <int GROUPS>
+template <int GROUPS, bool LONG = false>
 __global__ __launch_bounds__(GW_ROW_THREADS, 2) void gram_columns_once(const GramRowsOnceArgs args)
 {
     const int block = (int)blockIdx.x - args.samples;
@@ -516,7 +608,7 @@ __global__ __launch_bounds__(GW_ROW_THREADS, 2) void gram_columns_once(const Gra
     }
     const bool first = block < args.first_blocks;
     if ((int)blockIdx.z < (first ? args.first_batches : args.second_batches))
-        gram_columns_once_of<GROUPS>(first ? args.first : args.second, first ? block : block - args.first_blocks);
+        gram_columns_once_of<GROUPS, LONG>(first ? args.first : args.second, first ? block : block - args.first_blocks);
 }
 
 // Tile shapes of the product kernel.  A workgroup is 4 waves (8: EightWaves); a wave owns WAVE_M rows of a and WAVE_N rows of b as

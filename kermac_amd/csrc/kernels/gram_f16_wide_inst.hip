@@ -132,22 +132,37 @@ void place_operand(OperandRegions &r, int rows, bool broadcast, int l, bool once
 }
 
 // Grid, slices and the regions of both operands in the workspace; tiles_m and tiles_n are set.
-// a_shared, b_shared: one operand for all batch entries.  once: one pass makes the pieces of a short row (gram_rows_once, gram_columns_once).
-bool place_wide(int m, int n, int k, int l, bool a_shared, bool b_shared, bool once, bool symmetric, WideLayout *layout)
+// a_shared, b_shared: one operand for all batch entries.  a_once, b_once: one launch makes its pieces (made_once).
+bool place_wide(int m, int n, int k, int l, bool a_shared, bool b_shared, bool a_once, bool b_once, bool symmetric, WideLayout *layout)
 {
     // room for any tile of the product kernel in a grid, n tiles padded to the XCDs
     if (static_cast<int64_t>(layout->tiles_m) * (layout->tiles_n + kmc::BK_XCDS) * 4 > 0x7fffffff) return false;
     layout->slices = (k + kmc::BK_TILE_K - 1) / kmc::BK_TILE_K;
     int64_t cursor = 0;
-    const bool fits = k <= kmc::GRO_MAX_K;
-    place_operand(layout->a, m, a_shared, l, once && fits, *layout, cursor);
+    place_operand(layout->a, m, a_shared, l, a_once, *layout, cursor);
     // behind the region of a, where it stays when b grows or shrinks: the split of a may be kept
     layout->centre = layout->centre_floats ? place(cursor, 4 * layout->centre_floats * layout->centre_batches) : 0;
     if (symmetric) layout->b = layout->a;      // one panel, split once
-    else place_operand(layout->b, n, b_shared, l, once && fits, *layout, cursor);
+    else place_operand(layout->b, n, b_shared, l, b_once, *layout, cursor);
     layout->sample = place(cursor, kmc::BK_SAMPLE_BYTES);
     layout->bytes = cursor;
     return true;
+}
+
+bool rows_vec(const float *x, int64_t ld, int64_t bs, int majorness, bool scalar_only)
+{
+    return majorness == KMC_ROW_MAJOR && !scalar_only && aligned16(x) && ld % 4 == 0 && bs % 4 == 0;
+}
+
+// Whether gram_rows_once or gram_columns_once makes the pieces of an operand: up to 2048 k its values, in chunks up to 1024, stay in registers; longer ones are read twice by
+// the same workgroup (LONG), which is ahead of two launches for rows that lie apart or cannot be read 16 bytes at a time, and behind for others, whose k
+// the two launches share among nine workgroups.  Two launches / LONG, us of a call: rows contiguous 197 x 7052 x 3328 166 / 154, 3000 x 3000 x 8000 637 / 547, 8000 x 8000 x 3000
+// 1018 / 980, 20000 x 20000 x 2304 4490 / 4414; k contiguous, not aligned, 4 x 3840 x 347 x 2767 767 / 317, 2 x 192 x 7002 x 3730 683 / 345; aligned 197 x 7052 x 3328
+// 167 / 184, 3000 x 3000 x 8000 631 / 656, 8000 x 8000 x 3000 1060 / 1059, 20000 x 20000 x 2304 4552 / 4718.  Two launches / one pass of 2048 k: 2000 x 2000 x 2048 109 / 84,
+// 8000 x 8000 x 1300 504 / 476, 200 x 60000 x 1030 793 / 295.
+bool made_once(const float *x, int64_t ld, int64_t bs, int majorness, int flags, int k)
+{
+    return k <= 2 * kmc::GRO_HELD_K || (k <= kmc::GRO_MAX_K && !rows_vec(x, ld, bs, majorness, (flags & KMC_FLAG_FORCE_SCALAR_ACCESS) != 0));
 }
 
 bool wide_layout(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &args, WideLayout *layout)
@@ -170,7 +185,9 @@ bool wide_layout(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &a
     layout->centre_batches = own_centre && args.a_bs != 0 ? args.l : 1;
     layout->centre_floats = own_centre ? 2 * ((args.k + kmc::GRAM_CENTRE_PAD - 1) / kmc::GRAM_CENTRE_PAD * kmc::GRAM_CENTRE_PAD) + kmc::GRAM_CENTRE_PAD : 0;
     const bool one_centre = products || (own_centre ? layout->centre_batches == 1 : !args.centre || args.centre_bs == 0);
-    return place_wide(args.m, args.n, args.k, args.l, args.a_bs == 0 && one_centre, args.b_bs == 0 && one_centre, true, args.symmetric, layout);
+    return place_wide(args.m, args.n, args.k, args.l, args.a_bs == 0 && one_centre, args.b_bs == 0 && one_centre,
+                      made_once(args.a, args.a_ld, args.a_bs, p->a_majorness, p->flags, args.k), made_once(args.b, args.b_ld, args.b_bs, p->b_majorness, p->flags, args.k),
+                      args.symmetric, layout);
 }
 
 kmc::GramRowsArgs rows_args(const float *x, int64_t ld, int64_t bs, int rows, int majorness, bool scalar_only,
@@ -181,7 +198,7 @@ kmc::GramRowsArgs rows_args(const float *x, int64_t ld, int64_t bs, int rows, in
     rows_of.x = x; rows_of.ld = ld; rows_of.bs = bs;
     rows_of.rows = rows; rows_of.k = args.k;
     rows_of.row_major = majorness == KMC_ROW_MAJOR;
-    rows_of.vec = rows_of.row_major && !scalar_only && aligned16(x) && ld % 4 == 0 && bs % 4 == 0;
+    rows_of.vec = rows_vec(x, ld, bs, majorness, scalar_only);
     rows_of.centre = args.centre; rows_of.centre_bs = args.centre_bs;
     rows_of.centre_pairs = centre_pairs;
     rows_of.pieces = reinterpret_cast<kmc::gram_chunk *>(workspace + r.pieces); rows_of.pieces_bs = r.pieces_bs;
@@ -296,6 +313,10 @@ hipError_t launch_gram_once(const kmc::GramRowsArgs *first, int first_batches, c
     }
     const dim3 grid(blocks, 1, batches), threads(kmc::GW_ROW_THREADS);
     // registers for 256, 512 or 1024 k: the smallest that holds a row
+    if (k > kmc::GRO_HELD_K) {
+        if (!rows) return launch(kmc::gram_columns_once<16, true>, grid, threads, stream, args);
+        return k <= 2 * kmc::GRO_HELD_K ? launch(kmc::gram_rows_once<32>, grid, threads, stream, args) : launch(kmc::gram_rows_once<32, true>, grid, threads, stream, args);
+    }
     if (rows)
         return k <= 256 ? launch(kmc::gram_rows_once<4>, grid, threads, stream, args)
              : k <= 512 ? launch(kmc::gram_rows_once<8>, grid, threads, stream, args) : launch(kmc::gram_rows_once<16>, grid, threads, stream, args);
@@ -568,7 +589,7 @@ bool gradient_l2_layout(const kmc_norm_gradient_params *p, GradientL2Layout *lay
     wide.tiles_m = (p->m + kmc::GW_TILE - 1) / kmc::GW_TILE;
     wide.tiles_n = static_cast<int>((rows + kmc::GW_TILE - 1) / kmc::GW_TILE);
     if (!gradient_l2_pays(p, wide.tiles_m, wide.tiles_n)) return false;
-    if (!place_wide(p->m, static_cast<int>(rows), p->k, p->l, p->a_bs == 0, false, false, false, &wide)) return false;
+    if (!place_wide(p->m, static_cast<int>(rows), p->k, p->l, p->a_bs == 0, false, false, false, false, &wide)) return false;
     int64_t cursor = wide.bytes;
     layout->shift = place(cursor, static_cast<int64_t>(p->l) * p->n * 4);
     layout->c_transposed = place(cursor, static_cast<int64_t>(p->l) * p->k * p->o * 4);

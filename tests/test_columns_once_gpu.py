@@ -1,5 +1,5 @@
-"""GPU tests of gram_columns_once: the pieces of operands with the rows contiguous in one pass, at the edges of its groups of k (256, 512, 1024), of
-its 32 rows and of the slices that pad K.  Distances keep the route's 1e-5 of the float64 truth; rows that differ by powers of two keep their bits."""
+"""GPU tests of gram_columns_once: the pieces of operands with the rows contiguous by one launch, at the edges of its groups of k (256, 512, 1024), of
+its chunks of longer rows (512, those of gram_rows_once 1024), of its 32 rows and of the slices that pad K.  Distances keep the route's 1e-5 of the float64 truth; rows that differ by powers of two keep their bits."""
 import pytest
 import torch
 
@@ -16,19 +16,20 @@ def wide(monkeypatch):
         yield
 
 
-@pytest.mark.parametrize("K", [1, 7, 8, 9, 15, 16, 17, 31, 33, 64, 65, 255, 256, 257, 511, 512, 513, 1009, 1023, 1024, 1025])
+@pytest.mark.parametrize("K", [1, 7, 8, 9, 15, 16, 17, 31, 33, 64, 65, 255, 256, 257, 511, 512, 513, 1009, 1023, 1024, 1025, 1040, 1536, 1537, 2047, 2048, 2049, 3001, 8192, 8193])
 @pytest.mark.parametrize("M,N", [(1, 33), (31, 32), (255, 257), (130, 300)])
 def test_edges_of_k_and_of_the_rows(device, K, M, N):
     g = torch.Generator().manual_seed(K + M)
     # neither base nor leading dimension aligned; a common offset, so that the centre is subtracted
     a, b = ((torch.randn(K, rows + 3, generator=g) + 30.0).to(device)[:, 1:rows + 1].t() for rows in (M, N))
     names = kernels_of(lambda: kermac.cdist(a, b, p=2.0))
-    assert K == 1 or M == 1 or sum("gram_columns_once" in name for name in names) == (1 if K <= 1024 else 0)       # one row or k: of either order
+    assert K == 1 or M == 1 or sum("gram_columns_once" in name for name in names) == (1 if K <= 8192 else 0)       # one row or k: of either order
     truth = torch.cdist(a.double(), b.double())[None]
     assert_close_to_truth(kermac.cdist(a, b, p=2.0), truth, rtol=1e-5, what="columns")
     other = b.contiguous()                                  # one operand of either order: a launch each
     names = kernels_of(lambda: kermac.cdist(a, other, p=2.0))
-    assert K > 1024 or K == 1 or M == 1 or (sum("gram_columns_once" in name for name in names), sum("gram_rows_once" in name for name in names)) == (1, 1)
+    # rows that cannot be read 16 bytes at a time take one launch up to 8192 k, others up to 2048
+    assert (K > 2048 and K % 4 == 0) or K > 8192 or K == 1 or M == 1 or (sum("gram_columns_once" in name for name in names), sum("gram_rows_once" in name for name in names)) == (1, 1)
     assert_close_to_truth(kermac.cdist(a, other, p=2.0), truth, rtol=1e-5, what="columns and rows")
 
 
