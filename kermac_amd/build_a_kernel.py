@@ -638,8 +638,16 @@ def run_kernel(
     if plan.l2_auto and params.flags & matrix_core:
         asked = params.flags & matrix_core
         params.flags &= ~matrix_core
-        chosen, route_bytes = _auto_matrix_cores(params, asked)
+        chosen, route_bytes, otherwise = _auto_matrix_cores(params, asked)
         params.flags |= chosen
+        if route_bytes and chosen & _backend.FLAG_L2_GRAM_BF16:
+            workspace = _attach_route_workspace(params, a.device, route_bytes)
+            if workspace is not None:
+                plan.keepalive.append(workspace)
+                launch(params)
+                return plan.out
+            params.flags = params.flags & ~(matrix_core | _backend.FLAG_GRAM_WORKSPACE_ANY_SIZE) | otherwise       # no memory for it
+            route_bytes = None
     if params.flags & _backend.FLAG_DOT_PIECES:
         # products have no matrix-core kernel beside the route through the workspace: a call the
         # library has no use for a workspace for is an ordinary call of the direct kernel
@@ -688,18 +696,26 @@ def _direct_panels_min_tiles() -> int:
     return int(_backend.dispatch_rules()["DIRECT_PANELS_MIN_TILES"])
 
 
+def _attach_route_workspace(params, device, route_bytes):
+    """The workspace of the route for squared differences, which makes the centre for itself in there (include/kermac_amd.h,
+    KMC_FLAG_GRAM_OWN_CENTRE); None, and the flags as they were, when the memory for it is refused."""
+    if _centre_wanted():
+        params.flags |= _backend.FLAG_GRAM_OWN_CENTRE
+    workspace = _attach_gram_workspace(params, device, needed=route_bytes)
+    if workspace is None:
+        params.flags &= ~_backend.FLAG_GRAM_OWN_CENTRE
+    return workspace
+
+
 def _attach_gram_memory(params, stream, device, route_bytes=None):
-    """What a matrix-core launch for squared differences takes beside its operands: the workspace, and the centre, which the
-    route through the workspace makes for itself in there (include/kermac_amd.h, KMC_FLAG_GRAM_OWN_CENTRE)."""
+    """What a matrix-core launch for squared differences takes beside its operands: the route's workspace, or for a one-step kernel the centre
+    and room for the sample."""
     if route_bytes is None:
         route_bytes = _route_bytes(params, 0)
     if route_bytes:
-        if _centre_wanted():
-            params.flags |= _backend.FLAG_GRAM_OWN_CENTRE
-        workspace = _attach_gram_workspace(params, device, needed=route_bytes)
+        workspace = _attach_route_workspace(params, device, route_bytes)
         if workspace is not None:
             return workspace
-        params.flags &= ~_backend.FLAG_GRAM_OWN_CENTRE
         route_bytes = _backend.gram_workspace_bytes(params)
     return _attach_gram_centre(params, stream, device), _attach_gram_workspace(params, device, needed=route_bytes)     # a one-step kernel
 
@@ -763,17 +779,48 @@ _AUTO_UNCUT_MIN_TILES_K_CONTIGUOUS = 192
 
 
 def _auto_matrix_core_flags(params, asked):
-    return _auto_matrix_cores(params, asked)[0]
+    """Which of the matrix-core flags `asked` this call gets where only the library's own rule sends calls through a workspace."""
+    return _auto_matrix_cores(params, asked)[2]
 
 
 def _auto_matrix_cores(params, asked):
-    """Which of the matrix-core flags `asked` (those the descriptor allows) this call gets in the l2 mode "auto", and the bytes that the
-    library wants for its route through a workspace with them (0: it has none for this call)."""
+    """Which of the matrix-core flags `asked` (those the descriptor allows) this call gets in the l2 mode "auto", the bytes that the
+    library wants for its route through a workspace with them (0: not that route), and the flags to do without that memory."""
     route_bytes = _route_bytes(params, asked)
     if _workspace_allowed(route_bytes) and not _small_set_is_cut(params, asked):
-        return asked, route_bytes
+        return asked, route_bytes, asked
     chosen = _auto_one_step_flags(params, asked)
-    return chosen, route_bytes if chosen == asked else 0
+    if asked & _backend.FLAG_L2_GRAM_BF16 and (_auto_route_beats_one_step(params) if chosen else _auto_route_beats_direct(params)):
+        any_size = asked | _backend.FLAG_GRAM_WORKSPACE_ANY_SIZE
+        route_bytes = _route_bytes(params, any_size)
+        if _workspace_allowed(route_bytes):
+            return any_size, route_bytes, chosen
+    return chosen, 0, chosen
+
+
+# "auto" beyond the library's rule, which weighs the route against the one-step kernels as they were when its launches in front of the product
+# were more.  On 200 calls of 64 <= K <= 4096 (k and rows contiguous, batches, sets against themselves) no one-step kernel is ahead of both the
+# route and the direct kernel; they serve calls without the memory for the route.  Best one-step kernel / route, us: 128 x 128 x 200 34 / 26,
+# 600 x 3000 x 250 71 / 34, 4 x 600 x 750 x 1440 175 / 76, 1950 x 15808 x 213 226 / 79, rows contiguous 768 x 223 x 234 37 / 32, 2624 x 3233 x 126 49 / 41.
+# The route's error is nowhere above that of the kernels it takes the place of (70 calls, normal, uniform, heavy-tailed and scaled points, relative to
+# the 2-norm: 2.9e-8 .. 1.2e-7, the split one-step kernel 3.9e-8 .. 1.7e-7, the direct one below K = 128 5.9e-8 .. 9.2e-8).  Where the direct path
+# cuts a call over k it stays there: its short sums hold more of heavy-tailed points (K = 4022 4.3e-8 / 5.1e-7).
+# Below K = 128 the alternative is the direct kernel: direct / route, us, k contiguous, 270 tiles of K = 64 26 / 28, 315 34 / 36, 592 47 / 43,
+# 867 65 / 52; 160 of K = 93 22 / 26; 1220 of K = 96 95 / 63; rows contiguous 1692 of K = 64 99 / 85.
+_AUTO_ROUTE_MIN_TILES_TIMES_K = 32768
+# One row of tiles over operands that no cache holds: the route writes their pieces and reads them back for a single use, the one-step kernel reads
+# them once (best one-step / route, us: 2 x 64 x 42624 x 1667 248 / 430, 81 x 4 x 49438 x 1094 397 / 866, 96 x 16706 x 2338 184 / 216; below 5e7
+# values 2 x 64 x 14400 x 1024 91 / 75, 69 x 52697 x 896 222 / 166, 105 x 33233 x 1067 218 / 166; from 129 rows on 140 x 39940 x 722 133 / 111).
+_AUTO_ROUTE_ONE_ROW_OF_TILES_MAX_VALUES = 5e7
+
+
+def _auto_route_beats_one_step(params):
+    return min(params.m, params.n) > 128 or (params.m + params.n) * params.k * params.l <= _AUTO_ROUTE_ONE_ROW_OF_TILES_MAX_VALUES
+
+
+def _auto_route_beats_direct(params):
+    return (params.k < _AUTO_ONE_STEP_MIN_K
+            and -(-params.m // 128) * -(-params.n // 128) * params.l * params.k >= _AUTO_ROUTE_MIN_TILES_TIMES_K)
 
 
 def _auto_one_step_flags(params, asked):

@@ -14,6 +14,8 @@
     X(WIDE_MIN_TILES, 128)                                                                              \
     X(WIDE_MIN_TILES_TIMES_K, 147456)      /* unless there are ... */                                   \
     X(WIDE_TILES_FOR_ANY_K, 768)           /* ... this many tiles */                                    \
+    X(WIDE_LONG_MIN_K, 2048)               /* from here on already ... */                               \
+    X(WIDE_LONG_MIN_TILES, 128)            /* ... this many tiles of 128 x 128 per batch entry, of two sets with the rows contiguous */ \
     X(WIDE_MIN_TILES_PER_SIDE_X2, 5)       /* 2 tiles_m tiles_n >= 5 (tiles_m + tiles_n), per batch entry */ \
     X(WIDE_MAX_PADDING_PERCENT, 20)        /* of the tiles' area */                                     \
     /* ... both operands with k contiguous: the one-step kernels stage those slowly */                  \

@@ -102,7 +102,9 @@ bool wide_pays(int64_t m, int64_t n, int64_t tiles_m, int64_t tiles_n, int64_t t
     if (products) return k >= r::DOT_MIN_K && tiles >= r::DOT_MIN_TILES && tiles * k >= r::DOT_MIN_TILES_TIMES_K && little_padding;
     // (from 768 tiles on the route is as fast as the one-step kernel also for the shortest contractions
     // it takes, 8192 x 8192 x 64 180 us against 187, and ahead of the direct kernel, 236)
-    if (k < r::WIDE_MIN_K || tiles < r::WIDE_MIN_TILES || (tiles * k < r::WIDE_MIN_TILES_TIMES_K && tiles < r::WIDE_TILES_FOR_ANY_K)) return false;
+    // (long contractions of few tiles, today, one-step / route, us: 1500 x 1500 x 2048 129 / 75, 2048 x 2048 x 2048 173 / 88, 1800 x 1500 x 4000 294 / 126)
+    const bool long_walk = k >= r::WIDE_LONG_MIN_K && ((m + 127) / 128) * ((n + 127) / 128) >= r::WIDE_LONG_MIN_TILES && !k_contiguous && !symmetric;
+    if (!long_walk && (k < r::WIDE_MIN_K || tiles < r::WIDE_MIN_TILES || (tiles * k < r::WIDE_MIN_TILES_TIMES_K && tiles < r::WIDE_TILES_FOR_ANY_K))) return false;
     if (2 * tiles_m * tiles_n < r::WIDE_MIN_TILES_PER_SIDE_X2 * (tiles_m + tiles_n)) return false;
     return little_padding;
 }

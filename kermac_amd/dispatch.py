@@ -49,16 +49,21 @@ _ROWS = (
      "K < {build_a_kernel.L2_DEFAULT_MIN_K}", "direct `build_kernel<DIFF, SQUARE>`"),
     ("",
      "the library's rule for the workspace route: K ≥ {WIDE_MIN_K}, ≥ {WIDE_MIN_TILES} tiles of 256 × 256 over the batch, "
-     "tiles · K ≥ {WIDE_MIN_TILES_TIMES_K} or ≥ {WIDE_TILES_FOR_ANY_K} tiles, per batch entry 2 · tiles_m · tiles_n ≥ "
+     "tiles · K ≥ {WIDE_MIN_TILES_TIMES_K} or ≥ {WIDE_TILES_FOR_ANY_K} tiles (of two sets with the rows contiguous and from K = {WIDE_LONG_MIN_K} on ≥ {WIDE_LONG_MIN_TILES} of 128 × 128 per entry), per batch entry 2 · tiles_m · tiles_n ≥ "
      "{WIDE_MIN_TILES_PER_SIDE_X2} · (tiles_m + tiles_n), ≤ {WIDE_MAX_PADDING_PERCENT} % of the tiles' area padding; with k contiguous in both "
      "operands instead: K ≥ {WIDE_K_CONTIGUOUS_MIN_K}, ≥ {WIDE_K_CONTIGUOUS_MIN_TILES} tiles, tiles · K ≥ {WIDE_K_CONTIGUOUS_MIN_TILES_TIMES_K}, M and N ≥ "
      "{WIDE_K_CONTIGUOUS_MIN_ROWS}; or a set against itself of ≥ {WIDE_SYMMETRIC_MIN_TILES} tiles (of its triangle), tiles · K ≥ "
      "{WIDE_SYMMETRIC_MIN_TILES_TIMES_K}, with k contiguous K ≥ {WIDE_SYMMETRIC_K_CONTIGUOUS_MIN_K}, ≥ {WIDE_SYMMETRIC_K_CONTIGUOUS_MIN_TILES} tiles, "
      "tiles · K ≥ {WIDE_SYMMETRIC_K_CONTIGUOUS_MIN_TILES_TIMES_K} (mode `\"auto\"`: not one that "
      "the direct path would cut over k on fewer than {build_a_kernel.AUTO_UNCUT_MIN_TILES_K_CONTIGUOUS} tiles of 128 × 128)",
-     "`gram_rows_once` (k contiguous and K ≤ 1024, the sample in the same launch) or `gram_row_stats_pair` + `gram_f16_split_pair` + `gram_probe_operands`, "
+     "the centre (`sample_mean_rows` or `_columns`), `gram_rows_once` or `gram_columns_once` (with the sample in the same launch) or, k contiguous and aligned from K = 2049 on, "
+     "`gram_row_stats_pair` + `gram_f16_split_pair` + `gram_probe_operands`, "
      "`gram_f16_wide` (fp16 pieces, tiles of 256 × 128 from {WIDE_LARGE_TILE_MIN_TILES} on or where those fit the chip at once and 128 × 128 do not, else 128 × 128; in batches of ≥ 8 entries of ≤ {WIDE_ENTRY_PER_XCD_MAX_TILES} tiles of 128 × 128 each entry on one XCD), repair launch "
      "of the direct kernel"),
+    ("",
+     "mode `\"auto\"` with memory for it, what the next line describes, or K < {build_a_kernel.AUTO_ONE_STEP_MIN_K} and tiles of 128 × 128 over the batch · K ≥ "
+     "{build_a_kernel.AUTO_ROUTE_MIN_TILES_TIMES_K}; not a result of one row of tiles over more than {build_a_kernel.AUTO_ROUTE_ONE_ROW_OF_TILES_MAX_VALUES} values of both operands",
+     "the same route (`KMC_FLAG_GRAM_WORKSPACE_ANY_SIZE`)"),
     ("",
      "K ≥ {build_a_kernel.AUTO_ONE_STEP_MIN_K}, trust < 1, "
      "and not (a call the direct path would cut over k on fewer than {build_a_kernel.AUTO_UNCUT_MIN_TILES_K_CONTIGUOUS} tiles of 128 × 128, "

@@ -122,6 +122,10 @@ def run_kernel_coefficients(
     if matrix_core:
         from .build_a_kernel import _attach_gram_centre
         panels = _panel_shape(plan, _backend.FLAG_L2_GRAM_BF16) if aot else None
+        if aot and panels is None and plan.l2_auto and _auto_products_of_tiles(plan):
+            whole = _centres_at_once(plan, _backend.FLAG_L2_GRAM_BF16 | _backend.FLAG_GRAM_WORKSPACE_ANY_SIZE)
+            if whole is not None and _products_of_tiles(plan, whole, stream, a.device, debug):
+                return plan.out
         if panels is None and plan.l2_auto and not _auto_fused_on_matrix_cores(plan):
             kernel.flags &= ~(_backend.FLAG_L2_GRAM | _backend.FLAG_L2_GRAM_BF16)
             matrix_core = False
@@ -445,6 +449,36 @@ def _run_in_panels(plan, shape, stream, device, debug):
 _PRODUCTS_OF_TILES_MAX_COLUMNS = 32
 
 
+# "auto", squared differences: from K = 128 on at any size, from K = 64 on where the tiles fill the chip.  Best fused kernel / this, us, over 200 calls
+# (both storage orders, batches, 1, 10 and 32 columns): 303 x 192 x 118 48 / 42, 640 x 204 x 269 71 / 42, 500 x 256 x 958 137 / 48,
+# 1728 x 2240 x 320 81 / 43, 3826 x 640 x 239 x 2 88 / 45, 896 x 4354 x 739 201 / 55, 3001 x 8960 x 97 207 / 88; K below 128: 320 x 11439 x 64 43 / 42.5,
+# 12224 x 576 x 64 42 / 43, 2 x 6080 x 1144 x 64 70 / 52, 1110 x 23184 x 64 130 / 69, 217 x 4928 x 92 45 / 43; none from K = 128 on was slower.
+_AUTO_TILES_MIN_K = 128
+_AUTO_TILES_MIN_TILES_TIMES_K = 32768          # below that K, tiles of 128 x 128 over the batch
+
+
+def _auto_products_of_tiles(plan):
+    from .build_a_kernel import _auto_route_beats_one_step
+
+    if plan.O > _PRODUCTS_OF_TILES_MAX_COLUMNS or 0 in (plan.L, plan.M, plan.N, plan.K, plan.O):
+        return False
+    tiles = -(-plan.M // 128) * -(-plan.N // 128) * plan.L
+    return ((plan.K >= _AUTO_TILES_MIN_K or tiles * plan.K >= _AUTO_TILES_MIN_TILES_TIMES_K)
+            and _auto_route_beats_one_step(plan.params.kernel))
+
+
+def _centres_at_once(plan, route):
+    """(centres, panels, -, -, route): as _panel_shape, by the room for the products of the tiles alone."""
+    budget = int(os.environ.get("KERMAC_AMD_COEFFICIENT_PANEL_BYTES", _PANEL_BYTES))
+    per_tile = 4 * plan.L * plan.M * (-(-plan.O // 4) * 4)          # of 128 centres
+    if budget < per_tile:
+        return None
+    rows = min(plan.N, budget // per_tile * 128, 65535 * 128)
+    panels = -(-plan.N // rows)
+    rows = min(plan.N, -(-(-(-plan.N // panels)) // 256) * 256)
+    return rows, -(-plan.N // rows), None, None, route
+
+
 def _products_of_tiles(plan, shape, stream, device, debug):
     """The product in the panels of `shape` without the panels; False when it cannot be (more columns, no memory)."""
     from .build_a_kernel import _centre_wanted
@@ -469,7 +503,8 @@ def _products_of_tiles(plan, shape, stream, device, debug):
     kernel.gram_workspace, kernel.gram_workspace_bytes = workspace.data_ptr(), needed
     if debug:
         print(f"(Kermac Debug) Kernel matrix x coefficients in {panels} panels of {rows} centres, {splits} partial products each, "
-              "contracted where they are made")
+              "contracted where they are made" if splits is not None else
+              f"(Kermac Debug) Kernel matrix x coefficients tile by tile, {rows} centres at once")
     first_b, first_offset = kernel.b, kernel.regularization_offset_y
     for index in range(panels):
         n0 = index * rows
