@@ -373,7 +373,8 @@ typedef struct kmc_norm_gradient_params {
  * bytes of a, b and c.  KMC_NORM_L2:
  * when a model of both times favours the route by 15 % (tiles of 256 x 256 over m and o * n, in
  * both directions, and a contraction of about 512 or more); about 4 (m + o n) k bytes.
- * KMC_NORM_P: never.  No counterpart in the reference. */
+ * KMC_NORM_P: never.  KMC_FLAG_GRAM_WORKSPACE_ANY_SIZE in flags sets the size rules of both aside, in this query and in the
+ * call.  No counterpart in the reference. */
 int kmc_norm_gradient_workspace_bytes(const kmc_norm_gradient_params *params, int64_t *bytes);
 
 /* Stands in for launch(stream, config, cute_norm_kernel_gradient<NormType>, *args)

@@ -653,7 +653,7 @@ def run_kernel(
         # library has no use for a workspace for is an ordinary call of the direct kernel
         workspace = _attach_gram_workspace(params, a.device, needed=route_bytes)
         if workspace is None:
-            params.flags &= ~_backend.FLAG_DOT_PIECES
+            params.flags &= ~(_backend.FLAG_DOT_PIECES | _backend.FLAG_GRAM_WORKSPACE_ANY_SIZE)
         plan.keepalive.append(workspace)
     if params.flags & _backend.FLAG_L1_FIXED:
         # the fixed-point route exists only through a workspace: without one (a problem too small
@@ -795,6 +795,11 @@ def _auto_matrix_cores(params, asked):
         route_bytes = _route_bytes(params, any_size)
         if _workspace_allowed(route_bytes):
             return any_size, route_bytes, chosen
+    if asked & _backend.FLAG_DOT_PIECES and not route_bytes and _auto_route_beats_direct_products(params, asked):
+        any_size = asked | _backend.FLAG_GRAM_WORKSPACE_ANY_SIZE
+        route_bytes = _route_bytes(params, any_size)
+        if _workspace_allowed(route_bytes):
+            return any_size, route_bytes, chosen
     return chosen, 0, chosen
 
 
@@ -821,6 +826,19 @@ def _auto_route_beats_one_step(params):
 def _auto_route_beats_direct(params):
     return (params.k < _AUTO_ONE_STEP_MIN_K
             and -(-params.m // 128) * -(-params.n // 128) * params.l * params.k >= _AUTO_ROUTE_MIN_TILES_TIMES_K)
+
+
+# Sums of products, below what the library's rule asks for.  Direct / route, us: 919 x 657 x 64 four times (tiles * K 12288) 15.0 / 18.7, 1728 x 619 x 64 four
+# times (17920) 19.1 / 19.7, 6110 x 382 x 87 twice (25056) 30.9 / 25.7, 640 x 4045 x 200 (32000) 32 / 21, 652 x 3100 x 419 63 / 21, 4320 x 5541 x 161
+# 130 / 58, 7181 x 26944 x 84 607 / 345.  The route's error against 64 bits (2-norm) is 0.58 .. 0.82 of the direct kernel's on normal and uniform values,
+# 0.33 .. 1.15 on heavy-tailed ones; columns that span six decades sum few terms, and each product of the pieces carries 2^-22
+# (K = 64 1.0e-7 / 3.3e-8).  A call that the direct path cuts over k stays there: its short sums are more exact.
+_AUTO_PRODUCTS_MIN_TILES_TIMES_K = 20000
+
+
+def _auto_route_beats_direct_products(params, asked):
+    return (-(-params.m // 128) * -(-params.n // 128) * params.l * params.k >= _AUTO_PRODUCTS_MIN_TILES_TIMES_K
+            and not _direct_path_would_cut(params, asked))
 
 
 def _auto_one_step_flags(params, asked):

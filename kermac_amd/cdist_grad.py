@@ -158,6 +158,9 @@ def cdist_grad(
         ValueError: bad shapes, strides, batch sizes or devices.
     """
     plan = _plan_cdist_grad(a, b, c, d, out, p)
+    route = _route_of_any_size(plan) if _may_split else None
+    if route is not None and _run_cut((*route, True), plan, a, b, c, d, p, debug, any_size=True):
+        return plan.out
     if _may_split:
         for cut in _cuts_over_contraction(plan):
             if _run_cut(cut, plan, a, b, c, d, p, debug):
@@ -166,10 +169,13 @@ def cdist_grad(
     return plan.out
 
 
-def _launch(plan, device, debug, needs_workspace=False):
-    """Launches the call as it is; with `needs_workspace` only if it gets the workspace that the library wants for it."""
+def _launch(plan, device, debug, needs_workspace=False, any_size=False):
+    """Launches the call as it is; with `needs_workspace` only if it gets the workspace that the library wants for it, which
+    with `any_size` does not ask whether the route pays."""
+    plan.params.flags = _backend.FLAG_GRAM_WORKSPACE_ANY_SIZE if any_size else 0
     workspace = _attach_workspace(plan.params, device)
     if needs_workspace and workspace is None:
+        plan.params.flags = 0
         return False
     if debug:
         print(f"(Kermac Debug) Launching kernel: norm_kernel_gradient<{('L1', 'L2', 'P')[plan.params.norm_type]}>")
@@ -220,6 +226,101 @@ _SPLIT_MAX_PARTIAL_BYTES = 512 << 20
 _SPLIT_F16_TARGET_WORKGROUPS = 512
 
 
+def _shape_of_cuts(plan):
+    """(workgroups of the fp32 kernels, the most slices over k), or None for a call that is not cut."""
+    if plan.L != 1 or plan.M == 0 or plan.N == 0 or plan.O == 0 or not launch_cuts_enabled():
+        return None
+    M, N, O, K = plan.M, plan.N, plan.O, plan.K
+    n_tile = 32 if O <= 8 else 16
+    workgroups = -(-M // 64) * -(-N // n_tile) * max(1, -(-O // 32))
+    min_depth = _SPLIT_MIN_DEPTH * (1 if workgroups < 512 else 2 if O <= 8 else 4)
+    if workgroups >= _SPLIT_BELOW_WORKGROUPS or K < 2 * min_depth:
+        return None
+    return workgroups, min(K // min_depth, _SPLIT_MAX_SLICES, _SPLIT_MAX_PARTIAL_BYTES // (4 * O * N * M) - 1)
+
+
+def _cut_into(K, wanted, most):
+    depth = K // min(wanted, most) // 64 * 64           # whole K slices of the kernels; 16-byte alignment survives
+    slices = K // depth
+    return slices, depth, K - slices * depth
+
+
+def _f16_slices(M, N, O):
+    """Slices over k that the L1 route wants: the number that fills the CUs, and the fewer that reach its number of workgroups."""
+    f16_workgroups = -(-M // 16) * -(-N // 128) * -(-O // 16)
+    wanted = -(-_SPLIT_F16_TARGET_WORKGROUPS // f16_workgroups)
+    filled = wanted
+    # a workgroup has its CU to itself: up to twice as many slices where their last round of 256 would be nearly empty
+    # (1408 x 128 x 32 x 9522, 176 workgroups: 3 slices 424 us, 4 slices 354)
+    if wanted > 1:
+        parts = [n * f16_workgroups / (256 * -(-n * f16_workgroups // 256)) for n in range(wanted, 2 * wanted + 1)]
+        filled += next((extra for extra, part in enumerate(parts) if part >= 0.85), parts.index(max(parts)))
+    return filled, wanted
+
+
+# The library's own rules for the fp16 routes (kmc_norm_gradient_workspace_bytes) take the calls that are large enough for the routes to win
+# everywhere; below them stand calls that the fp32 kernels, a workgroup walking the whole of k, take far longer for.  Which is
+# the faster one there follows from launch times in microseconds, fitted to 797 calls (M 64 .. 12000, N 8 .. 1024, K 64 .. 12000, O 1 .. 64, one
+# problem or a batch of two; the fits are off by 13 .. 19 %).  A route that they favour by 15 % is taken: over these calls the L1 gradient takes
+# 0.55 and the L2 gradient 0.67 of the fp32 kernels' time, 0.02 more than with the better one each time, and 9 calls of
+# them are slower by more than 5 % (the worst, 1009 x 254 x 1 x 1044, 69 -> 91 us).
+# fp32 / route, us: p = 1, 768 x 28 x 1 x 1651 twice 191 / 56; 192 x 22 x 32 x 1088 118 / 39; 428 x 18 x 4 x 256 40 / 23; 10304 x 675 x 1 x 175 117 / 227.
+# p = 2, 64 x 37 x 1 x 10691 twice 1229 / 358; 768 x 28 x 1 x 1651 twice 175 / 95; 256 x 62 x 4 x 832 124 / 74; 128 x 1013 x 32 x 135 twice 41 / 81.
+_ROUTE_ADVANTAGE = 1.15
+# The sums of the fp32 kernels hold their rounding, which short slices keep small: the route's error (in the 2-norm, against 64 bits,
+# 87 calls of normal, uniform and heavy-tailed values) is 0.35 .. 0.8 of theirs on slices of the same depth, 0.9 at four times the depth, above theirs
+# from seven times on (1602 x 178 x 10 x 4485 uncut against 8 slices 5.8e-7 / 4.2e-7).
+_ROUTE_MAX_DEPTH_RATIO = 4
+_ROUTE_MIN_FP32_US = 24.0
+
+
+def _fp32_us(plan, slices, depth):
+    L, M, N, O = plan.L, plan.M, plan.N, plan.O
+    rounds = max(1.0, -(-M // 64) * -(-N // (32 if O <= 8 else 16)) * -(-O // 32) * L * slices / 256)
+    outputs = O if O <= 2 else 4 if O <= 4 else 8 if O <= 8 else 16 if O <= 16 else 32
+    us = 4.5 + depth * (0.081 + rounds * (0.0356 + 0.0035 * outputs)) + 1.84e-6 * L * M * N * O
+    return us + 30.0 + 1.84e-6 * slices * M * N * O if slices > 1 else us
+
+
+def _route_us(plan, slices, depth):
+    L, M, N, O, K = plan.L, plan.M, plan.N, plan.O, plan.K
+    parts = L if slices == 1 else slices
+    if plan.params.norm_type == _NORM_L1:
+        workgroups = -(-M // 16) * -(-N // 128) * -(-O // 16) * parts
+        us = (18.5 + 0.0194 * depth * max(1.0, workgroups / 256) + (11e-6 * N + 2.6e-6 * M) * K * L + 23e-6 * N * (M + 256) * parts
+              + 1.7e-6 * L * M * N * O)
+        return us + 36.0 + 1.7e-6 * slices * M * N * O if slices > 1 else us
+    tiles = -(-M // 128) * -(-O * N // 128) * parts
+    us = 40.5 + depth * (0.0174 + 0.0168 * max(1.0, tiles / 256)) + 2.1e-6 * (O * N + M) * K * L + 3.3e-6 * L * M * N * O
+    return us + 47.0 + 3.3e-6 * slices * M * N * O if slices > 1 else us
+
+
+def _route_of_any_size(plan):
+    """(slices, k per slice, leftover k) with which an L1 or L2 gradient that the library's rule leaves to the fp32 kernels is faster on the fp16
+    matrix instruction, or None."""
+    if plan.params.norm_type == _NORM_P or min(plan.L, plan.M, plan.N, plan.O, plan.K) < 1 or not _workspace_enabled():
+        return None
+    shape = _shape_of_cuts(plan)
+    fp32 = (1, plan.K, 0)
+    forms = [fp32]
+    if shape is not None and shape[1] >= 2:
+        workgroups, most = shape
+        fp32 = _cut_into(plan.K, max(2, round(_SPLIT_TARGET_WORKGROUPS / workgroups)), most)
+        wanted = _f16_slices(plan.M, plan.N, plan.O)[0] if plan.params.norm_type == _NORM_L1 else fp32[0]
+        if min(wanted, most) >= 2:
+            forms.append(_cut_into(plan.K, wanted, most))
+    fp32_us = _fp32_us(plan, *fp32[:2])
+    if fp32_us < _ROUTE_MIN_FP32_US:
+        return None
+    forms = [form for form in forms if form[1] <= _ROUTE_MAX_DEPTH_RATIO * fp32[1]]
+    if not forms:
+        return None
+    route_us, route = min((_route_us(plan, *form[:2]), form) for form in forms)
+    if _ROUTE_ADVANTAGE * route_us >= fp32_us or _backend.norm_gradient_workspace_bytes(plan.params) > 0:
+        return None
+    return route
+
+
 def _takes_f16_route(params, slices=1, depth=None):
     """Whether the library wants a workspace for this L1 gradient, or for `slices` of `depth` k each as a batch of one launch."""
     if params.norm_type != _NORM_L1 or not _workspace_enabled():
@@ -234,30 +335,17 @@ def _takes_f16_route(params, slices=1, depth=None):
 def _cuts_over_contraction(plan):
     """How the call is cut over k: (slices, k per slice, leftover k, whether only with a workspace), the best first.  Behind the cuts for the fp16
     matrix instruction stands the one for the fp32 kernels, which run where the workspace is refused; the last resort is the call as it is."""
-    if plan.L != 1 or plan.M == 0 or plan.N == 0 or plan.O == 0 or not launch_cuts_enabled():
+    shape = _shape_of_cuts(plan)
+    if shape is None:
         return
+    workgroups, most = shape
     M, N, O, K = plan.M, plan.N, plan.O, plan.K
-    n_tile = 32 if O <= 8 else 16
-    workgroups = -(-M // 64) * -(-N // n_tile) * max(1, -(-O // 32))
-    min_depth = _SPLIT_MIN_DEPTH * (1 if workgroups < 512 else 2 if O <= 8 else 4)
-    if workgroups >= _SPLIT_BELOW_WORKGROUPS or K < 2 * min_depth:
-        return
-    most = min(K // min_depth, _SPLIT_MAX_SLICES, _SPLIT_MAX_PARTIAL_BYTES // (4 * O * N * M) - 1)
 
     def cut(wanted):
-        depth = K // min(wanted, most) // 64 * 64       # whole K slices of the kernels; 16-byte alignment survives
-        slices = K // depth
-        return slices, depth, K - slices * depth
+        return _cut_into(K, wanted, most)
 
     if _takes_f16_route(plan.params):
-        f16_workgroups = -(-M // 16) * -(-N // 128) * -(-O // 16)
-        wanted = -(-_SPLIT_F16_TARGET_WORKGROUPS // f16_workgroups)
-        filled = wanted
-        # a workgroup has its CU to itself: up to twice as many slices where their last round of 256 would be nearly empty
-        # (1408 x 128 x 32 x 9522, 176 workgroups: 3 slices 424 us, 4 slices 354)
-        if wanted > 1:
-            parts = [n * f16_workgroups / (256 * -(-n * f16_workgroups // 256)) for n in range(wanted, 2 * wanted + 1)]
-            filled += next((extra for extra, part in enumerate(parts) if part >= 0.85), parts.index(max(parts)))
+        filled, wanted = _f16_slices(M, N, O)
         # more slices take more memory: where that is refused, the fewer ones
         for slices in dict.fromkeys((filled, wanted)):
             if min(slices, most) < 2:
@@ -274,20 +362,20 @@ def _split_over_contraction(plan):
     return best[:3] if best is not None and best[0] > 1 else None
 
 
-def _run_cut(cut, plan, a, b, c, d, p, debug):
+def _run_cut(cut, plan, a, b, c, d, p, debug, any_size=False):
     """Launches the call in slices, or returns False with nothing launched: no memory for the partial results, or for the workspace of a
     cut that is none without."""
     slices, depth, leftover, needs_workspace = cut
     if slices == 1:
-        return _launch(plan, a.device, debug, needs_workspace)
+        return _launch(plan, a.device, debug, needs_workspace, any_size)
     taken = _scratch.mark()
-    if _run_slices(slices, depth, leftover, needs_workspace, plan, a, b, c, d, p, debug):
+    if _run_slices(slices, depth, leftover, needs_workspace, plan, a, b, c, d, p, debug, any_size):
         return True
     _scratch.give_back_to(taken)
     return False
 
 
-def _run_slices(slices, depth, leftover, needs_workspace, plan, a, b, c, d, p, debug):
+def _run_slices(slices, depth, leftover, needs_workspace, plan, a, b, c, d, p, debug, any_size=False):
     a2, b2, c2, d2 = (t[0] if t.dim() == 3 else t for t in (a, b, c, d))
     M, N, O = plan.M, plan.N, plan.O
     partial = _scratch.allocate_floats((slices + (1 if leftover else 0), O, N, M), a.device)
@@ -300,7 +388,7 @@ def _run_slices(slices, depth, leftover, needs_workspace, plan, a, b, c, d, p, d
     a_slices = a2.as_strided((slices, depth, M), (depth * a2.stride(0), a2.stride(0), a2.stride(1)), a2.storage_offset())
     b_slices = b2.as_strided((slices, N, depth), (depth * b2.stride(1), b2.stride(0), b2.stride(1)), b2.storage_offset())
     c_slices = c2.as_strided((slices, O, depth), (depth * c2.stride(1), c2.stride(0), c2.stride(1)), c2.storage_offset())
-    if not _launch(_plan_cdist_grad(a_slices, b_slices, c_slices, d2, partial[:slices], p), a.device, debug, needs_workspace):
+    if not _launch(_plan_cdist_grad(a_slices, b_slices, c_slices, d2, partial[:slices], p), a.device, debug, needs_workspace, any_size):
         return False
     if leftover:
         done = slices * depth

@@ -570,6 +570,7 @@ bool gradient_l2_pays(const kmc_norm_gradient_params *p, int64_t tiles_m, int64_
     const double forced = text ? std::atof(text) : 0.0;
     const double terms = static_cast<double>(p->m) * p->n * p->k * p->l;
     if (forced > 0.0) return terms >= forced;
+    if (p->flags & KMC_FLAG_GRAM_WORKSPACE_ANY_SIZE) return true;
     const int o = p->o;
     const double per_term = o == 1 ? 0.077 : o == 2 ? 0.10 : o == 3 ? 0.126 : o == 4 ? 0.137 : o <= 8 ? 0.028 * o
                           : o <= 16 ? 0.27 : o <= 32 ? 0.56 : 0.0175 * o;

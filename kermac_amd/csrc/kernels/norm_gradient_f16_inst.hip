@@ -52,6 +52,7 @@ bool f16_pays(const kmc_norm_gradient_params *p)
     const double forced = text ? std::atof(text) : 0.0;
     const double terms = static_cast<double>(p->m) * p->n * p->k * p->l;
     if (forced > 0.0) return terms >= forced;
+    if (p->flags & KMC_FLAG_GRAM_WORKSPACE_ANY_SIZE) return true;
     // more than 16 outputs: the ranking serves all blocks of outputs, while the fp32 kernels go to their 32-column tiles (fp32 / route, us:
     // 704 x 48 x 32 x 1024, 3.5e7 terms, 102 / 59; 832 x 352 x 128 x 320, 9.4e7, 250 / 122; 576 x 48 x 64 x 2816, 7.8e7, 218 / 131)
     namespace r = kmc_rules;

@@ -21,7 +21,7 @@ def rules() -> dict:
 
     merged = dict(_backend.dispatch_rules())
     for module, prefixes in ((build_a_kernel, ("_AUTO_", "_CUT_", "_L2_")),
-                             (cdist_grad, ("_SPLIT_",)),
+                             (cdist_grad, ("_SPLIT_", "_ROUTE_")),
                              (kernel_coefficients, ("_AUTO_", "_PANEL_", "_PIECES_", "_FUSED_", "_MANY_", "_SPLIT_"))):
         short = module.__name__.rsplit(".", 1)[-1]
         for name, value in vars(module).items():
@@ -83,6 +83,8 @@ _ROWS = (
      "≤ {WIDE_MAX_PADDING_PERCENT} % padding; or K ≥ {DOT_LONG_K}, tiles · K ≥ {DOT_LONG_MIN_TILES_TIMES_K}, ≥ {DOT_LONG_MIN_TILES_BATCHED} tiles "
      "over a batch ({DOT_LONG_MIN_TILES_SINGLE} of a single problem)",
      "the workspace route with `gram_f16_wide<GW_EPILOGUE_DOT>` (no trust check, no repair)"),
+    ("", "with memory for it: tiles of 128 × 128 over the batch · K ≥ {build_a_kernel.AUTO_PRODUCTS_MIN_TILES_TIMES_K}, but for a call that the direct path would cut over k",
+     "the same route (`KMC_FLAG_GRAM_WORKSPACE_ANY_SIZE`)"),
     ("", "otherwise", "direct `build_kernel<DOT, NOOP>`"),
     ("`cdist(p=1)`, `run_kernel` of DIFF + ABS (L1 norm, Laplace-L1)",
      "l1 mode `\"fixed\"` (opt-in) and ≥ {L1_FIXED_MIN_TILES} tiles of 128 × 128 over the batch, K ≥ {L1_FIXED_MIN_K}",
@@ -123,6 +125,8 @@ _ROWS = (
      "`gradient_signs_prepare` (rows of b and d ranked, a and c copied, bounds of their products), `norm_gradient_l1_f16` (16 outputs a tile; 8 with both pieces in its columns)"),
     ("`cdist_grad`, p = 2", "a model of both times favours the route by {GRADIENT_L2_ADVANTAGE_PERCENT} %, and the planes of `out` form one matrix",
      "`gradient_l2_prepare`, `gradient_l2_pieces_stats` and `_split`, `gram_f16_wide<GW_EPILOGUE_GRADIENT_L2>`"),
+    ("`cdist_grad`, p = 1 or 2, below those rules", "with memory for it, where models of the launch times favour the route, uncut or cut over k, over the fp32 kernels by a factor of "
+     "{cdist_grad.ROUTE_ADVANTAGE}, its slices at most {cdist_grad.ROUTE_MAX_DEPTH_RATIO} times as deep as theirs", "the same routes (`KMC_FLAG_GRAM_WORKSPACE_ANY_SIZE`)"),
     ("`cdist_grad`, otherwise", "O ≤ 8 / O > 8", "`norm_kernel_gradient` (vector ALU) / `norm_kernel_gradient_mfma` (fp32 matrix instruction), in runs of 32, 16 and ≤ 8 outputs; "
      "unbatched calls of fewer than {cdist_grad.SPLIT_BELOW_WORKGROUPS} workgroups are cut over k"),
     ("`run_kernel(..., coefficients=)`, squared differences, l2 mode `\"auto\"`",
