@@ -7,6 +7,7 @@ and the stream handle.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 import threading
 from ctypes import POINTER, Structure, byref, c_char_p, c_float, c_int32, c_int64, c_size_t, c_void_p
@@ -207,7 +208,9 @@ def check(status: int) -> None:
 
 
 def build_kernel(params: BuildKernelParams, stream: int) -> None:
-    check(library().kmc_build_kernel(byref(params), c_void_p(stream)))
+    status = library().kmc_build_kernel(byref(params), stream)
+    if status != OK:
+        check(status)
 
 
 def build_kernel_finish(params: BuildKernelParams, partials: int, partial_ld: int, partial_bs: int, partial_slice: int,
@@ -243,6 +246,7 @@ def build_kernel_jit(function: int, params: BuildKernelParams, stream: int) -> N
     check(library().kmc_build_kernel_jit(c_void_p(function), byref(params), c_void_p(stream)))
 
 
+@functools.lru_cache(maxsize=None)         # a property of the library
 def build_kernel_has_variant(inner_operator: int, inner_power: int) -> bool:
     return bool(library().kmc_build_kernel_has_variant(inner_operator, inner_power))
 

@@ -27,7 +27,7 @@ import torch
 from . import _backend
 from . import _scratch
 from .common import (Alignment, Majorness, PyTorchStreamWrapper, TensorStats, ceil_div, launch_cuts_enabled,
-                     merge_batch_size, tensor_stats)
+                     matrix_layout, merge_batch_size)
 from .module_cache.module_cache import ModuleCache, build_kernel_function_name
 
 
@@ -402,9 +402,13 @@ def _plan_run_kernel(
         raise TypeError("a and b must be PyTorch tensors")
     if out is not None and not isinstance(out, torch.Tensor):
         raise TypeError("out must be a PyTorch tensor if provided")
-    L = merge_batch_size("a", L, a, expected_dims=2, can_be_none=False)
-    L = merge_batch_size("b", L, b, expected_dims=2, can_be_none=False)
-    L = merge_batch_size("out", L, out, expected_dims=2, can_be_none=True)
+    # (a matrix without a batch leaves L as it is)
+    if a.dim() != 2:
+        L = merge_batch_size("a", L, a, expected_dims=2, can_be_none=False)
+    if b.dim() != 2:
+        L = merge_batch_size("b", L, b, expected_dims=2, can_be_none=False)
+    if out is not None and out.dim() != 2:
+        L = merge_batch_size("out", L, out, expected_dims=2, can_be_none=True)
 
     if a.dtype != torch.float32 or b.dtype != torch.float32:
         raise TypeError("a and b must have dtype torch.float32")
@@ -421,16 +425,15 @@ def _plan_run_kernel(
     if out is not None and out.device != device:
         raise ValueError(f"out must be on the same CUDA device as inputs: got {out.device}, expected {device}")
 
-    stats_a, stats_b = tensor_stats(a), tensor_stats(b)
-    _, M, K_a = stats_a.shape
-    _, N, K_b = stats_b.shape
+    _, M, K_a, a_majorness, a_ld, a_bs = matrix_layout(a)
+    _, N, K_b, b_majorness, b_ld, b_bs = matrix_layout(b)
     if K_a != K_b:
         raise ValueError(f"K dimensions must match: got {K_a} for a and {K_b} for b")
     K = K_a
 
+    has_out = True
     if out is not None:
-        stats_c = tensor_stats(out)
-        L_c, M_c, N_c = stats_c.shape
+        L_c, M_c, N_c, c_majorness, c_ld, c_bs = matrix_layout(out)
         if (M_c, N_c) != (M, N):
             raise ValueError(f"out must have shape (M={M}, N={N}), got {(M_c, N_c)}")
         if L_c != L and L != 1:
@@ -439,9 +442,9 @@ def _plan_run_kernel(
         # every element is written by the kernel (also for K = 0), so no fill is needed; the
         # reference allocates zeros (build_a_kernel.py:259), which costs 0.6 ms at 30000 x 30000
         out = torch.empty((L, M, N), dtype=torch.float32, device=device)
-        stats_c = tensor_stats(out)
+        c_majorness, c_ld, c_bs = Majorness.ROW_MAJOR, max(N, 1), max(M, 1) * max(N, 1) if L != 1 else 0
     else:
-        stats_c = None
+        has_out = False
 
     keepalive = [a, b, out]
 
@@ -462,10 +465,11 @@ def _plan_run_kernel(
             outer_p = 1.0 / inner_p
     # only those that are set: the parameter block starts as zeros
     hyper_parameters = []
-    for name, field, value in (("inner_p", "p_inner", inner_p), ("outer_p", "p_outer", outer_p), ("bandwidth", "bandwidth", bandwidth),
-                               ("regularization", "regularization", regularization)):
-        if value is not None:
-            hyper_parameters.append((field, *_hyper_parameter(name, value, L, device, require_device)))
+    if inner_p is not None or outer_p is not None or bandwidth is not None or regularization is not None:
+        for name, field, value in (("inner_p", "p_inner", inner_p), ("outer_p", "p_outer", outer_p), ("bandwidth", "bandwidth", bandwidth),
+                                   ("regularization", "regularization", regularization)):
+            if value is not None:
+                hyper_parameters.append((field, *_hyper_parameter(name, value, L, device, require_device)))
 
     # The kernel writes C with m contiguous.  A row-major out is the transpose of
     # that, so swap the operands (reference: :323-336).  The reference swaps neither the
@@ -476,28 +480,22 @@ def _plan_run_kernel(
     # with offset_x + n == offset_y + m.  The kernel itself computes B - A and tests
     # offset_x + (row of A) == offset_y + (row of B), so the swapped launch passes
     # through as it is and the unswapped one exchanges the offsets and negates.
-    swapped = stats_c is not None and stats_c.majorness is Majorness.ROW_MAJOR
+    swapped = has_out and c_majorness is Majorness.ROW_MAJOR
     off_x, off_y = int(regularization_offset_x), int(regularization_offset_y)
     if swapped:
         M, N = N, M
         a, b = b, a
-        stats_a, stats_b = stats_b, stats_a
+        a_majorness, a_ld, a_bs, b_majorness, b_ld, b_bs = b_majorness, b_ld, b_bs, a_majorness, a_ld, a_bs
     else:
         off_x, off_y = off_y, off_x
 
-    params = _backend.BuildKernelParams()
-    params.inner_operator = d._inner_operator.abi
-    params.inner_power = d._inner_power.abi
-    params.outer_power = d._outer_power.abi
-    params.kernel_type = d._kernel_type.abi
-    params.a_majorness = stats_a.majorness.abi
-    params.b_majorness = stats_b.majorness.abi
-    params.flags = 0 if swapped else _backend.FLAG_NEGATE_DIFF
+    flags = 0 if swapped else _backend.FLAG_NEGATE_DIFF
+    gram_trust = 0.0
     a_pointer, b_pointer = a.data_ptr(), b.data_ptr()
     if a_pointer == b_pointer and os.environ.get("KERMAC_AMD_NO_SYMMETRY", "0") not in ("", "0"):
         # the library computes x-against-x matrices from the tiles on and below the diagonal
         # (bit-identical result, about half the time); this keeps it to the full computation
-        params.flags |= _backend.FLAG_NO_SYMMETRY
+        flags |= _backend.FLAG_NO_SYMMETRY
     l2 = _l2_current()
     l2_auto = False
     if (l2["mode"] != "direct" and d._inner_operator is InnerOperator.DIFF
@@ -506,31 +504,34 @@ def _plan_run_kernel(
         # (_auto_matrix_core_flags), run_kernel_coefficients for the coefficient product (no out matrix
         # here), whose fused kernel has a matrix-core variant too
         l2_auto = l2["mode"] == "auto"
-        params.flags |= _backend.FLAG_L2_GRAM
-        if l2["mode"] == "gram_bf16" or (l2_auto and stats_c is not None):
-            params.flags |= _backend.FLAG_L2_GRAM_BF16
-        params.gram_trust = _gram_trust(K, l2)
+        flags |= _backend.FLAG_L2_GRAM
+        if l2["mode"] == "gram_bf16" or (l2_auto and has_out):
+            flags |= _backend.FLAG_L2_GRAM_BF16
+        gram_trust = _gram_trust(K, l2)
     elif (l2["mode"] in ("auto", "gram_bf16") and d._inner_operator is InnerOperator.DOT
-            and d._inner_power is PowerType.NOOP and K >= l2["min_k"] and stats_c is not None):
+            and d._inner_power is PowerType.NOOP and K >= l2["min_k"] and has_out):
         # sums of products (linear and polynomial kernels): large ones on the fp16 matrix instruction from two
         # fp16 pieces per value, when the library has a use for the workspace that run_kernel offers it
         l2_auto = l2["mode"] == "auto"
-        params.flags |= _backend.FLAG_DOT_PIECES
+        flags |= _backend.FLAG_DOT_PIECES
     l1 = _l1_current()
     if (l1["mode"] == "fixed" and d._inner_operator is InnerOperator.DIFF and d._inner_power is PowerType.ABS
-            and stats_c is not None):
+            and has_out):
         # sums of absolute differences: large stored matrices on fixed point, when the library has a
         # use for the workspace that run_kernel offers it
-        params.flags |= _backend.FLAG_L1_FIXED
+        flags |= _backend.FLAG_L1_FIXED
         if os.environ.get("KERMAC_AMD_L1_FIXED_ANY_SIZE", "0") not in ("", "0"):
-            params.flags |= _backend.FLAG_GRAM_WORKSPACE_ANY_SIZE      # tests send small shapes down the route
+            flags |= _backend.FLAG_GRAM_WORKSPACE_ANY_SIZE      # tests send small shapes down the route
         if l1["tolerance"] is not None:
-            params.gram_trust = float(l1["tolerance"])
-    params.m, params.n, params.k, params.l = M, N, K, L
-    params.a, params.a_ld, params.a_bs = a_pointer, stats_a.leading_dimension_stride, stats_a.batch_stride
-    params.b, params.b_ld, params.b_bs = b_pointer, stats_b.leading_dimension_stride, stats_b.batch_stride
-    if stats_c is not None:
-        params.c, params.c_ld, params.c_bs = out.data_ptr(), stats_c.leading_dimension_stride, stats_c.batch_stride
+            gram_trust = float(l1["tolerance"])
+    # the block's fields in their order, in one call: an assignment each is a microsecond of every call
+    params = _backend.BuildKernelParams(
+        d._inner_operator.abi, d._inner_power.abi, d._outer_power.abi, d._kernel_type.abi, a_majorness.abi, b_majorness.abi, flags,
+        M, N, K, L, a_pointer, a_ld, a_bs, b_pointer, b_ld, b_bs)
+    if has_out:
+        params.c, params.c_ld, params.c_bs = out.data_ptr(), c_ld, c_bs
+    if gram_trust:
+        params.gram_trust = gram_trust
     for field, pointer, batch_stride, by_value, keep in hyper_parameters:
         if keep is None:
             setattr(params, field + "_value", by_value)
@@ -538,7 +539,8 @@ def _plan_run_kernel(
             setattr(params, field, pointer)
             setattr(params, field + "_bs", batch_stride)
             keepalive.append(keep)
-    params.regularization_offset_x, params.regularization_offset_y = off_x, off_y
+    if off_x or off_y:
+        params.regularization_offset_x, params.regularization_offset_y = off_x, off_y
     params.epsilon = 1e-5 if epsilon is None else float(epsilon)
 
     plan = _LaunchPlan()
@@ -549,13 +551,14 @@ def _plan_run_kernel(
 
 
 _raw_current_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)      # of a process that has tensors there
 
 
 def _current_stream_for(device: torch.device) -> int:
     """The hipStream_t of torch's current stream, which must be on the tensors' device
     (reference: build_a_kernel.py:314-321).  The raw-handle accessor saves the construction of
     a Stream object on every call; a launch costs about 10 microseconds of host time."""
-    current = torch.cuda.current_device()
+    current = _current_device()
     index = current if device.index is None else device.index
     if current != index:
         raise ValueError(f"cuda stream must be on the same device as the tensors: got cuda:{current}, expected {device}")

@@ -14,7 +14,7 @@ import torch
 from . import _backend
 from . import _scratch
 from .build_a_kernel import _current_stream_for
-from .common import launch_cuts_enabled, merge_batch_size, tensor_stats
+from .common import launch_cuts_enabled, matrix_layout, merge_batch_size
 
 _NORM_L1, _NORM_L2, _NORM_P = 0, 1, 2
 
@@ -26,44 +26,48 @@ class _GradPlan:
 def _plan_cdist_grad(a, b, c, d, out, p, require_device=True) -> _GradPlan:
     """Validation and parameter marshalling of ``cdist_grad``
     (reference: cdist_grad.py:62-235), without the launch."""
-    if not all(isinstance(x, torch.Tensor) for x in (a, b, c, d)):
-        raise TypeError("All inputs must be PyTorch tensors")
+    inputs = (a, b, c, d)
+    for x in inputs:
+        if not isinstance(x, torch.Tensor):
+            raise TypeError("All inputs must be PyTorch tensors")
     if out is not None and not isinstance(out, torch.Tensor):
         raise TypeError("out must be a PyTorch tensor if provided")
-    if not all(x.dtype == torch.float32 for x in (a, b, c, d)):
-        raise TypeError("All inputs must have dtype torch.float32")
+    for x in inputs:
+        if x.dtype is not torch.float32:
+            raise TypeError("All inputs must have dtype torch.float32")
     if out is not None and out.dtype != torch.float32:
         raise TypeError("out must have dtype torch.float32")
-    if not all(x.dim() in (2, 3) for x in (a, b, c, d)):
-        raise ValueError("All inputs must be 2-dimensional or 3-dimensional with a batch mode")
+    for x in inputs:
+        if x.dim() not in (2, 3):
+            raise ValueError("All inputs must be 2-dimensional or 3-dimensional with a batch mode")
     if out is not None and out.dim() not in (3, 4):
         raise ValueError("out must be 3-dimensional or 4-dimensional with a batch mode")
     if require_device:
-        if not all(x.is_cuda for x in (a, b, c, d)):
-            raise ValueError("All inputs must be on a CUDA device")
+        for x in inputs:
+            if not x.is_cuda:
+                raise ValueError("All inputs must be on a CUDA device")
         if out is not None and not out.is_cuda:
             raise ValueError("out must be on a CUDA device")
     device = a.device
-    if not all(x.device == device for x in (a, b, c, d)):
-        raise ValueError(f"All inputs must be on the same CUDA device: got {[x.device for x in (a, b, c, d)]}")
+    for x in inputs[1:]:
+        if x.device != device:
+            raise ValueError(f"All inputs must be on the same CUDA device: got {[x.device for x in inputs]}")
     if out is not None and out.device != device:
         raise ValueError(f"out must be on the same CUDA device as inputs: got {out.device}, expected {device}")
 
     if isinstance(p, int) and not isinstance(p, bool):
         p = float(p)
 
-    stats_a, stats_b, stats_c, stats_d = tensor_stats(a), tensor_stats(b), tensor_stats(c), tensor_stats(d)
-    _, K, M = stats_a.shape
-    _, N, K_b = stats_b.shape
-    _, O, K_c = stats_c.shape
-    _, N_d, M_d = stats_d.shape
+    _, K, M, _, a_ld, a_bs = matrix_layout(a)
+    _, N, K_b, _, b_ld, b_bs = matrix_layout(b)
+    _, O, K_c, _, c_ld, c_bs = matrix_layout(c)
+    _, N_d, M_d, _, d_ld, d_bs = matrix_layout(d)
 
     L = 1
     L = merge_batch_size("p", L, p, expected_dims=0, can_be_none=False)
-    L = merge_batch_size("a", L, a, expected_dims=2, can_be_none=False)
-    L = merge_batch_size("b", L, b, expected_dims=2, can_be_none=False)
-    L = merge_batch_size("c", L, c, expected_dims=2, can_be_none=False)
-    L = merge_batch_size("d", L, d, expected_dims=2, can_be_none=False)
+    for name, x in zip("abcd", inputs):
+        if x.dim() != 2:            # (a matrix without a batch leaves L as it is)
+            L = merge_batch_size(name, L, x, expected_dims=2, can_be_none=False)
     L = merge_batch_size("out", L, out, expected_dims=3, can_be_none=True)
 
     if (N, K_b) != (N, K):
@@ -79,7 +83,7 @@ def _plan_cdist_grad(a, b, c, d, out, p, require_device=True) -> _GradPlan:
         elif tuple(out.shape) != (L, O, N, M):
             raise ValueError(f"Expected shape {(L, O, N, M)} for out, got {tuple(out.shape)}")
 
-    for name, x in (("a", a), ("b", b), ("c", c), ("d", d)):
+    for name, x in zip("abcd", inputs):
         if x.stride(-1) != 1:
             raise ValueError(f"{name} must have stride 1 in last dimension")
     if out is not None and out.stride(-1) != 1:
@@ -114,14 +118,8 @@ def _plan_cdist_grad(a, b, c, d, out, p, require_device=True) -> _GradPlan:
         # every element is written by the kernel, so no fill is needed
         out = torch.empty((L, O, N, M), dtype=torch.float32, device=device)
 
-    params = _backend.NormGradientParams()
-    params.norm_type = norm_type
-    params.flags = 0
-    params.m, params.n, params.o, params.k, params.l = M, N, O, K, L
-    params.a, params.a_ld, params.a_bs = a.data_ptr(), stats_a.leading_dimension_stride, stats_a.batch_stride
-    params.b, params.b_ld, params.b_bs = b.data_ptr(), stats_b.leading_dimension_stride, stats_b.batch_stride
-    params.c, params.c_ld, params.c_bs = c.data_ptr(), stats_c.leading_dimension_stride, stats_c.batch_stride
-    params.d, params.d_ld, params.d_bs = d.data_ptr(), stats_d.leading_dimension_stride, stats_d.batch_stride
+    params = _backend.NormGradientParams(norm_type, 0, M, N, O, K, L, a.data_ptr(), a_ld, a_bs, b.data_ptr(), b_ld, b_bs,
+                                         c.data_ptr(), c_ld, c_bs, d.data_ptr(), d_ld, d_bs)
     params.e = out.data_ptr()
     params.e_ld_n = out.stride(-2)
     params.e_ld_o = out.stride(-3)

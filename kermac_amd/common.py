@@ -114,6 +114,34 @@ def merge_batch_size(
     raise TypeError(f"{name} must be a float or a torch.Tensor, got {type(a).__name__}")
 
 
+def matrix_layout(tensor: torch.Tensor):
+    """(batches, rows, columns, majorness, leading dimension, batch stride) of a 2-D or batched 3-D fp32 tensor, as ``TensorStats``
+    holds them: the operators, whose small calls are bound by the host, take them without the object."""
+    if tensor.dtype is not torch.float32 and tensor.dim() in (2, 3):
+        raise TypeError("Input tensor must have dtype torch.float32")
+    strides = tensor.stride()
+    if len(strides) == 2:
+        rows, cols = tensor.shape
+        row_stride, col_stride = strides
+        batches, batch_stride = 1, 0
+    elif len(strides) == 3:
+        batches, rows, cols = tensor.shape
+        batch_stride, row_stride, col_stride = strides
+        if batches == 1:
+            batch_stride = 0
+    else:
+        raise ValueError("Input tensor must be 2 or 3-dimensional")
+    if col_stride == 1 and row_stride >= cols:
+        majorness = Majorness.ROW_MAJOR
+    elif row_stride == 1 and col_stride >= rows:
+        majorness = Majorness.COL_MAJOR
+    else:
+        raise ValueError(
+            f"Tensor has non-standard memory layout: strides={tensor.stride()}, shape={tensor.size()}"
+        )
+    return batches, rows, cols, majorness, row_stride if row_stride > col_stride else col_stride, batch_stride
+
+
 class TensorStats:
     """Batch count/stride, majorness, alignment and leading dimension of a 2-D or
     batched 3-D fp32 tensor (reference: common.py:72-141).
@@ -131,30 +159,9 @@ class TensorStats:
     __slots__ = ("_shape", "_num_batches", "_batch_stride", "_majorness", "_alignment", "_ld")
 
     def __init__(self, tensor: torch.Tensor):
-        shape, strides = tensor.shape, tensor.stride()
-        if len(shape) not in (2, 3):
-            raise ValueError("Input tensor must be 2 or 3-dimensional")
-        if tensor.dtype != torch.float32:
-            raise TypeError("Input tensor must have dtype torch.float32")
-
-        batched = len(shape) == 3
-        self._num_batches = shape[0] if batched else 1
-        self._batch_stride = strides[0] if batched and self._num_batches != 1 else 0
-
-        rows, cols = shape[-2:]
-        row_stride, col_stride = strides[-2:]
-        self._shape = (self._num_batches, rows, cols)
-
-        if col_stride == 1 and row_stride >= cols:
-            self._majorness = Majorness.ROW_MAJOR
-        elif row_stride == 1 and col_stride >= rows:
-            self._majorness = Majorness.COL_MAJOR
-        else:
-            raise ValueError(
-                f"Tensor has non-standard memory layout: strides={tensor.stride()}, shape={tensor.size()}"
-            )
-
-        self._ld = max(row_stride, col_stride)
+        batches, rows, cols, self._majorness, self._ld, self._batch_stride = matrix_layout(tensor)
+        self._num_batches = batches
+        self._shape = (batches, rows, cols)
         if self._majorness is Majorness.COL_MAJOR and self._ld % 4 == 0 and tensor.data_ptr() % 16 == 0:
             self._alignment = Alignment.ALIGN_4
         else:
