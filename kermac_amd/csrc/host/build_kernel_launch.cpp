@@ -123,6 +123,7 @@ int prepare(const kmc_build_kernel_params *p, bool need_c, kmc::BuildKernelArgs 
     args->centre = nullptr;
     args->centre_bs = 0;
     args->sample = nullptr;
+    args->repair_queue = nullptr;
     args->panels = 0;
     if ((p->flags & (KMC_FLAG_L2_GRAM | KMC_FLAG_L2_GRAM_BF16)) && p->gram_centre) {
         if (!aligned16(p->gram_centre) || p->gram_centre_bs % 4 != 0 || p->gram_centre_bs < 0)
@@ -159,7 +160,7 @@ hipError_t launch_gram_l2(int load_a, int load_b, const kmc::BuildKernelArgs &ar
 hipError_t launch_gram_bf16_l2(int load_a, int load_b, const kmc::BuildKernelArgs &args, dim3 grid, hipStream_t stream);
 int64_t gram_f16_wide_bytes(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &args);
 hipError_t launch_scalar_b_if_the_sample_leaves(int load_a, int load_b, const kmc::BuildKernelArgs &args, hipStream_t stream, bool *launched);
-hipError_t launch_gram_probe(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &args, unsigned *sample, int centre_pairs, hipStream_t stream);
+hipError_t launch_gram_probe(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &args, unsigned *sample, int centre_pairs, int queues, hipStream_t stream);
 int64_t l1_fixed_bytes(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &args);
 hipError_t launch_l1_fixed(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &args, hipStream_t stream, bool *taken);
 int64_t direct_panels_bytes(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &args);
@@ -255,13 +256,15 @@ int kmc_build_kernel(const kmc_build_kernel_params *params, void *stream)
         hipError_t g = launch_gram_f16_wide(params, args, static_cast<hipStream_t>(stream), &wide, &sample_taken);
         if (g != hipSuccess) return fail_hip(g, "gram_f16_wide launches");
         if (wide) args.sample = sample_taken;
+        // (the route's workspace has the queues of the repair launch behind the sample, which clears them)
+        if (sample_taken) args.repair_queue = const_cast<unsigned *>(sample_taken) + kmc::BK_SAMPLE_TILES;
         if (!wide) {
             // The one-step kernels: with KMC_SAMPLE_BYTES of workspace, a sample of the result first (gram_probe.hip),
             // so that data whose near-duplicates sit in every tile costs the direct kernel's time, not both.
             if (!(params->flags & KMC_FLAG_NO_PROBE) && params->gram_workspace && params->gram_workspace_bytes >= KMC_SAMPLE_BYTES &&
                 (reinterpret_cast<uintptr_t>(params->gram_workspace) & 255) == 0 && args.k > 0) {
                 unsigned *sample = static_cast<unsigned *>(params->gram_workspace);
-                g = launch_gram_probe(params, args, sample, 0, static_cast<hipStream_t>(stream));
+                g = launch_gram_probe(params, args, sample, 0, 0, static_cast<hipStream_t>(stream));
                 if (g != hipSuccess) return fail_hip(g, "gram_probe_operands launch");
                 args.sample = sample;
             }
@@ -276,7 +279,8 @@ int kmc_build_kernel(const kmc_build_kernel_params *params, void *stream)
             bool launched = false;
             g = launch_scalar_b_if_the_sample_leaves(load_a, load_b, args, static_cast<hipStream_t>(stream), &launched);
             if (g != hipSuccess) return fail_hip(g, "build_kernel_scalar_b launch");
-            args.sample = nullptr;
+            // (else the repair launch of many tiles does, and asks the sample itself)
+            if (launched || !args.repair_queue) args.sample = nullptr;
         }
         args.repair_only = 1;
     }

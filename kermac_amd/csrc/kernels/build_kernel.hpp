@@ -66,6 +66,8 @@ struct BuildKernelArgs {
     // where m == n + same_shift (a set against itself or against a run of its own rows): their distance is zero, which
     // |a|^2 + |b|^2 - 2 a.b cannot tell.  (The last fields, so that kernels that know nothing of them are compiled as they were.)
     int same_points, same_shift;
+    // build_kernel_repair only: what its workgroups take tiles from, behind the sample
+    unsigned *repair_queue;
 };
 
 constexpr int BK_PANELS_COPIED = 1;
@@ -571,15 +573,16 @@ __device__ __forceinline__ void finish_tile(
 // heights are rounded up to a multiple of 8 to keep that ownership in the last
 // band; the padding workgroups get `false` and exit at once.  The host drops the
 // rounding for problems of few n tiles, where it would add many such workgroups.
-__device__ __forceinline__ bool tile_of_workgroup(const BuildKernelArgs &args, int &tile_m, int &tile_n)
+// `workgroup` is one of the `width` ids of a batch entry: blockIdx.x of a launch with a workgroup per tile.
+__device__ __forceinline__ bool tile_of_workgroup(const BuildKernelArgs &args, int workgroup, int width, int batch, int &tile_m, int &tile_n)
 {
     // Batches rotate the order by one: the hardware derives the XCD from the launch-wide
     // workgroup id, which is blockIdx.x modulo 8 for every batch when the grid width is a
     // multiple of 8, so without the rotation a batch of problems of 8 tiles each would
     // run every tile n on a single XCD.  The residue classes modulo 8, and with them the ownership
     // described above, survive the rotation.
-    const int rotated = blockIdx.x + blockIdx.y % gridDim.x;
-    const int linear = rotated >= (int)gridDim.x ? rotated - (int)gridDim.x : rotated;
+    const int rotated = workgroup + (int)((unsigned)batch % (unsigned)width);
+    const int linear = rotated >= width ? rotated - width : rotated;
     if (args.symmetric) {
         // Symmetric result: the ids count through the tiles on and below the diagonal, row r
         // of the triangle starting at id r (r + 1) / 2.  (In the band order half the
@@ -600,6 +603,11 @@ __device__ __forceinline__ bool tile_of_workgroup(const BuildKernelArgs &args, i
     tile_m = in_band / band_height;
     tile_n = band * BK_BAND_N + in_band % band_height;
     return tile_n < args.tiles_n;
+}
+
+__device__ __forceinline__ bool tile_of_workgroup(const BuildKernelArgs &args, int &tile_m, int &tile_n)
+{
+    return tile_of_workgroup(args, blockIdx.x, gridDim.x, blockIdx.y, tile_m, tile_n);
 }
 
 // Marker the matrix-core L2 kernel (gram_kernel.hpp) leaves in the first element
@@ -700,14 +708,12 @@ __device__ __forceinline__ void store_tile(
 }
 
 // One output tile from start to finish; `lds_a` / `lds_b`: two slices per operand plus one pad row (see the fragment
-// prefetch).  The body of the two kernels below.
+// prefetch).  The body of the kernels below; `workgroup` and `width` as for tile_of_workgroup.
 template <int INNER_OP, int INNER_POW, int LOAD_A, int LOAD_B>
-__device__ __forceinline__ void build_kernel_tile(const BuildKernelArgs &args, float *lds_a, float *lds_b)
+__device__ __forceinline__ void build_kernel_tile(const BuildKernelArgs &args, float *lds_a, float *lds_b, int tid, int workgroup, int width, int batch)
 {
-    const int tid = threadIdx.x;
-    const int batch = blockIdx.y;
     int tile_m, tile_n;
-    if (!tile_of_workgroup(args, tile_m, tile_n)) return;
+    if (!tile_of_workgroup(args, workgroup, width, batch, tile_m, tile_n)) return;
     const int m0 = tile_m * BK_TILE_M;
     const int n0 = tile_n * BK_TILE_N;
     const int m_valid = args.m - m0;   // rows of A that exist from m0 on (may exceed 128)
@@ -762,7 +768,7 @@ __global__ __launch_bounds__(BK_THREADS) void build_kernel(const BuildKernelArgs
 {
     __shared__ __attribute__((aligned(16))) float lds_a[2 * BK_LDS_SLICE + BK_LDS_PITCH];
     __shared__ __attribute__((aligned(16))) float lds_b[2 * BK_LDS_SLICE + BK_LDS_PITCH];
-    build_kernel_tile<INNER_OP, INNER_POW, LOAD_A, LOAD_B>(args, lds_a, lds_b);
+    build_kernel_tile<INNER_OP, INNER_POW, LOAD_A, LOAD_B>(args, lds_a, lds_b, threadIdx.x, blockIdx.x, gridDim.x, blockIdx.y);
 }
 
 // The same kernel for panels with contiguous rows (both loaders LOAD_COL_VEC), compiled for four waves per SIMD.
@@ -777,7 +783,57 @@ __global__ __launch_bounds__(BK_THREADS, 4) void build_kernel_four_waves(const B
 {
     __shared__ __attribute__((aligned(16))) float lds_a[2 * BK_LDS_SLICE + BK_LDS_PITCH];
     __shared__ __attribute__((aligned(16))) float lds_b[2 * BK_LDS_SLICE + BK_LDS_PITCH];
-    build_kernel_tile<INNER_OP, INNER_POW, LOAD_COL_VEC, LOAD_COL_VEC>(args, lds_a, lds_b);
+    build_kernel_tile<INNER_OP, INNER_POW, LOAD_COL_VEC, LOAD_COL_VEC>(args, lds_a, lds_b, threadIdx.x, blockIdx.x, gridDim.x, blockIdx.y);
+}
+
+// The repair launch of a result of many tiles, of which as a rule none carries the marker: with a workgroup per tile it is bound by the
+// latency of a load each, four workgroups to a CU (30000 x 30000, 56400 tiles, 65 us, now 25; 12000 x 9000 x 512,
+// 6768 tiles, the call 369 -> 348).  Here as many workgroups as the chip holds look at
+// BK_REPAIR_CHUNK tiles at a time and recompute those that carry it.  They take the tiles, in their order, from eight queues, one per XCD
+// (tile_of_workgroup), so that a result with many marked ones stays balanced; where the sample left everything to this
+// launch (`sample` null: to another one in front of it), tile by tile.  (A fixed share for every workgroup: such results 5 to 12 % slower.)
+constexpr int BK_REPAIR_WORKGROUPS = 768;
+constexpr int BK_REPAIR_CHUNK = 32;                   // at most 32
+constexpr int BK_REPAIR_QUEUES = 8;
+
+template <int INNER_OP, int INNER_POW, int LOAD_A, int LOAD_B>
+__global__ __launch_bounds__(BK_THREADS, 3) void build_kernel_repair(const BuildKernelArgs args)
+{
+    __shared__ __attribute__((aligned(16))) float lds_a[2 * BK_LDS_SLICE + BK_LDS_PITCH];
+    __shared__ __attribute__((aligned(16))) float lds_b[2 * BK_LDS_SLICE + BK_LDS_PITCH];
+    __shared__ int next;
+    const int lane = threadIdx.x & 63;
+    const int width = args.grid_width, total = width * args.l;             // (the host checks that these fit)
+    const int queue = blockIdx.x % BK_REPAIR_QUEUES, begin = gridDim.x / BK_REPAIR_QUEUES;
+    const int chunk = args.sample && sample_leaves_it_to_the_direct_kernel(args.sample) ? 1 : BK_REPAIR_CHUNK;
+    int first = (int)blockIdx.x / BK_REPAIR_QUEUES * chunk;                // tile BK_REPAIR_QUEUES * first + queue of the launch
+    while (BK_REPAIR_QUEUES * (i64)first + queue < total) {
+        const i64 id = BK_REPAIR_QUEUES * ((i64)first + lane) + queue;
+        int tile_m, tile_n;
+        bool marked = false;
+        if (lane < chunk && id < total) {
+            const int batch = (int)id / width;
+            if (tile_of_workgroup(args, (int)id - batch * width, width, batch, tile_m, tile_n))
+                marked = __float_as_uint(args.c[batch * args.c_bs + (i64)tile_n * BK_TILE_N * args.c_ld + tile_m * BK_TILE_M]) == BK_REPAIR_MARKER;
+        }
+        // the same in every wave: none of them stores before all have passed the barriers of the walk
+        unsigned found = (unsigned)__ballot(marked);
+        while (found) {
+            const int here = BK_REPAIR_QUEUES * (first + __builtin_ctz(found)) + queue, batch = here / width;
+            found &= found - 1;
+            // a copy of the lane's id that the compiler cannot see through: what it derives from it before the loop costs 50 registers and a
+            // wave per SIMD
+            int tid = threadIdx.x;
+            asm volatile("" : "+v"(tid));
+            build_kernel_tile<INNER_OP, INNER_POW, LOAD_A, LOAD_B>(args, lds_a, lds_b, tid, here - batch * width, width, batch);
+            __syncthreads();            // the staging arrays, which the mirrored stores read
+        }
+        // (taken in front of the chunk, so that it arrives meanwhile, the last tiles wait for workgroups that are still at others: 5 % of 6768 marked ones)
+        if (threadIdx.x == 0) next = begin * chunk + (int)atomicAdd(args.repair_queue + queue, (unsigned)chunk);
+        __syncthreads();
+        first = __builtin_amdgcn_readfirstlane(next);
+        __syncthreads();
+    }
 }
 
 }  // namespace kmc

@@ -146,7 +146,7 @@ bool place_wide(int m, int n, int k, int l, bool a_shared, bool b_shared, bool a
     layout->centre = layout->centre_floats ? place(cursor, 4 * layout->centre_floats * layout->centre_batches) : 0;
     if (symmetric) layout->b = layout->a;      // one panel, split once
     else place_operand(layout->b, n, b_shared, l, b_once, *layout, cursor);
-    layout->sample = place(cursor, kmc::BK_SAMPLE_BYTES);
+    layout->sample = place(cursor, kmc::BK_SAMPLE_BYTES + 4 * kmc::BK_REPAIR_QUEUES);
     layout->bytes = cursor;
     return true;
 }
@@ -260,8 +260,8 @@ void forget_split_in(const void *workspace)
 }
 
 // Statistics and split of one operand (also used by the gradient's fp16 route).
-hipError_t launch_gram_probe(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &args, unsigned *sample, int centre_pairs, hipStream_t stream);   // gram_probe.hip
-kmc::GramProbeArgs gram_probe_args(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &args, unsigned *sample, int centre_pairs);                 // gram_probe.hip
+hipError_t launch_gram_probe(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &args, unsigned *sample, int centre_pairs, int queues, hipStream_t stream);   // gram_probe.hip
+kmc::GramProbeArgs gram_probe_args(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &args, unsigned *sample, int centre_pairs, int queues);                 // gram_probe.hip
 hipError_t launch_route_centre(const float *x, int majorness, int rows, int k, int64_t ld, int64_t bs, int l, float *mean, int64_t mean_bs, hipStream_t stream);   // sample_mean.hip
 int route_centre_pairs(int majorness, int rows, int k, int l);                                                                                                    // sample_mean.hip
 
@@ -484,7 +484,7 @@ hipError_t launch_gram_f16_wide(const kmc_build_kernel_params *p, const kmc::Bui
     if (status != hipSuccess) return status;
     if ((split_a && layout.a.once) || (split_b && layout.b.once)) {
         status = launch_gram_once_both(split_a && layout.a.once ? &rows_a : nullptr, layout.a.batches, split_b && layout.b.once ? &rows_b : nullptr,
-                                       layout.b.batches, sample ? gram_probe_args(p, wide.kernel, sample, centre_pairs) : kmc::GramProbeArgs{}, sample != nullptr, stream);
+                                       layout.b.batches, sample ? gram_probe_args(p, wide.kernel, sample, centre_pairs, kmc::BK_REPAIR_QUEUES) : kmc::GramProbeArgs{}, sample != nullptr, stream);
         sampled = true;
     }
     if (status == hipSuccess && split_a && split_b && !layout.a.once && !layout.b.once) {
@@ -493,7 +493,7 @@ hipError_t launch_gram_f16_wide(const kmc_build_kernel_params *p, const kmc::Bui
         if (status == hipSuccess && split_a && !layout.a.once) status = launch_gram_rows(rows_a, layout.a.batches, stream);
         if (status == hipSuccess && split_b && !layout.b.once) status = launch_gram_rows(rows_b, layout.b.batches, stream);
     }
-    if (status == hipSuccess && sample && !sampled) status = launch_gram_probe(p, wide.kernel, sample, centre_pairs, stream);
+    if (status == hipSuccess && sample && !sampled) status = launch_gram_probe(p, wide.kernel, sample, centre_pairs, kmc::BK_REPAIR_QUEUES, stream);
     if (status != hipSuccess) return status;
     if (sample) {
         wide.kernel.sample = sample;

@@ -22,7 +22,7 @@ __global__ __launch_bounds__(GP_THREADS) void gram_probe_operands(const GramProb
 namespace kmc_host {
 
 // What the kernel needs for the problem of `p` (squared differences; m, n, k, l at least 1).
-kmc::GramProbeArgs gram_probe_args(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &args, unsigned *sample, int centre_pairs)
+kmc::GramProbeArgs gram_probe_args(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &args, unsigned *sample, int centre_pairs, int queues)
 {
     kmc::GramProbeArgs probe;
     probe.a = p->a; probe.b = p->b;
@@ -34,13 +34,14 @@ kmc::GramProbeArgs gram_probe_args(const kmc_build_kernel_params *p, const kmc::
     probe.centre_pairs = centre_pairs;
     probe.trust = args.gram_trust;
     probe.sample = sample;
+    probe.queues = queues;
     return probe;
 }
 
-// Fills sample[0 .. BK_SAMPLE_TILES) for the problem of `p` (squared differences; m, n, k, l at least 1).
-hipError_t launch_gram_probe(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &args, unsigned *sample, int centre_pairs, hipStream_t stream)
+// Fills sample[0 .. BK_SAMPLE_TILES), and clears `queues` words behind it, for the problem of `p` (squared differences; m, n, k, l at least 1).
+hipError_t launch_gram_probe(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &args, unsigned *sample, int centre_pairs, int queues, hipStream_t stream)
 {
-    const kmc::GramProbeArgs probe = gram_probe_args(p, args, sample, centre_pairs);
+    const kmc::GramProbeArgs probe = gram_probe_args(p, args, sample, centre_pairs, queues);
     return launch(kmc::gram_probe_operands, dim3(kmc::BK_SAMPLE_TILES), dim3(kmc::GP_THREADS), stream, probe);
 }
 

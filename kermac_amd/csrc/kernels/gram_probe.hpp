@@ -29,6 +29,7 @@ struct GramProbeArgs {
     int centre_pairs;                          // > 0: no flag was stored, these many pairs say it (CentreSums)
     float trust;
     unsigned *sample;                          // [BK_SAMPLE_TILES]
+    int queues;                                // that many words behind it are cleared, for build_kernel_repair
 };
 
 // Whether subtracting the centre would lower the norms, and with them the error of the expansion, by under 2 %: |c|^2 against the variances.
@@ -76,6 +77,7 @@ __device__ __forceinline__ void gram_probe_tile(const GramProbeArgs &args, int t
     __shared__ unsigned below_in_tile;
     const int t = threadIdx.x;
     if (t == 0) below_in_tile = 0u;
+    if (tile == 0 && t < args.queues) args.sample[BK_SAMPLE_TILES + t] = 0u;
     unsigned h = (unsigned)tile * 2654435761u + 0x9e3779b9u;
     h ^= h >> 15; h *= 0x846ca68bu; h ^= h >> 13;
     const int batch = (int)(h % (unsigned)args.l);
