@@ -22,7 +22,7 @@ def rules() -> dict:
     merged = dict(_backend.dispatch_rules())
     for module, prefixes in ((build_a_kernel, ("_AUTO_", "_CUT_", "_L2_")),
                              (cdist_grad, ("_SPLIT_", "_ROUTE_")),
-                             (kernel_coefficients, ("_AUTO_", "_PANEL_", "_PIECES_", "_FUSED_", "_MANY_", "_SPLIT_"))):
+                             (kernel_coefficients, ("_AUTO_", "_PANEL_", "_PIECES_", "_FUSED_", "_MANY_", "_SPLIT_", "_PRODUCTS_"))):
         short = module.__name__.rsplit(".", 1)[-1]
         for name, value in vars(module).items():
             if name.startswith(prefixes) and isinstance(value, (int, float)) and not isinstance(value, bool):
@@ -59,7 +59,7 @@ _ROWS = (
      "the centre (`sample_mean_rows` or `_columns`), `gram_rows_once` or `gram_columns_once` (with the sample in the same launch) or, k contiguous and aligned from K = 2049 on, "
      "`gram_row_stats_pair` + `gram_f16_split_pair` + `gram_probe_operands`, "
      "`gram_f16_wide` (fp16 pieces, tiles of 256 × 128 from {WIDE_LARGE_TILE_MIN_TILES} on or where those fit the chip at once and 128 × 128 do not, else 128 × 128; in batches of ≥ 8 entries of ≤ {WIDE_ENTRY_PER_XCD_MAX_TILES} tiles of 128 × 128 each entry on one XCD), repair launch "
-     "of the direct kernel"),
+     "of the direct kernel (more than 4096 tiles: `build_kernel_repair`)"),
     ("",
      "mode `\"auto\"` with memory for it, what the next line describes, or K < {build_a_kernel.AUTO_ONE_STEP_MIN_K} and tiles of 128 × 128 over the batch · K ≥ "
      "{build_a_kernel.AUTO_ROUTE_MIN_TILES_TIMES_K}; not a result of one row of tiles over more than {build_a_kernel.AUTO_ROUTE_ONE_ROW_OF_TILES_MAX_VALUES} values of both operands",
@@ -130,6 +130,11 @@ _ROWS = (
     ("`cdist_grad`, otherwise", "O ≤ 8 / O > 8", "`norm_kernel_gradient` (vector ALU) / `norm_kernel_gradient_mfma` (fp32 matrix instruction), in runs of 32, 16 and ≤ 8 outputs; "
      "unbatched calls of fewer than {cdist_grad.SPLIT_BELOW_WORKGROUPS} workgroups are cut over k"),
     ("`run_kernel(..., coefficients=)`, squared differences, l2 mode `\"auto\"`",
+     "O ≤ {kernel_coefficients.PRODUCTS_OF_TILES_MAX_COLUMNS} with memory for it, K ≥ {kernel_coefficients.AUTO_TILES_MIN_K} or tiles of 128 × 128 over the batch · K ≥ "
+     "{kernel_coefficients.AUTO_TILES_MIN_TILES_TIMES_K}; not a matrix of one row of tiles over more than {build_a_kernel.AUTO_ROUTE_ONE_ROW_OF_TILES_MAX_VALUES} values of both "
+     "operands",
+     "the workspace route with `gram_f16_wide<GW_CONTRACT_16 | _32>`: every tile contracted where it is made; distrusted parts by `kernel_times_coefficients`, `sum_products`"),
+    ("",
      "K ≥ {kernel_coefficients.AUTO_PANEL_MIN_K} and (the library's workspace rule for a panel, or K ≥ {kernel_coefficients.AUTO_PANEL_LONG_K}, or K ≥ "
      "{kernel_coefficients.AUTO_PANEL_MID_K} with ≥ {kernel_coefficients.AUTO_PANEL_MID_TILES} tiles — both with {panel_used_percent} % of the tiles' area used — or "
      "O > {kernel_coefficients.AUTO_FUSED_MAX_COLUMNS} with K ≥ {kernel_coefficients.AUTO_PANEL_WIDE_K} and ≥ {kernel_coefficients.AUTO_PANEL_WIDE_TILES} tiles)",
