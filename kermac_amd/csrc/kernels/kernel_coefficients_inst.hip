@@ -21,6 +21,14 @@ template <int LOAD_A, int LOAD_B>
 static hipError_t launch_one(const kmc::KernelCoefficientsArgs &args, dim3 grid, hipStream_t stream)
 {
     hipError_t status;
+#if KMC_INNER_OP == 0 && KMC_INNER_POW == 2
+    if (args.stamps)
+        return args.columns == kmc::KC_COLUMNS ? launch(kmc::kernel_times_coefficients<KMC_INNER_OP, KMC_INNER_POW, LOAD_A, LOAD_B, kmc::KC_COLUMNS, true>, grid,
+                                                        dim3(kmc::BK_THREADS), stream, args)
+                                               : hipErrorInvalidValue;
+#else
+    if (args.stamps) return hipErrorInvalidValue;
+#endif
     if (args.columns == 64) {
         status = launch(kmc::kernel_times_coefficients<KMC_INNER_OP, KMC_INNER_POW, LOAD_A, LOAD_B, 64>, grid, dim3(kmc::BK_THREADS), stream, args);
     } else if (args.columns == kmc::KC_COLUMNS) {
