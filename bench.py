@@ -373,8 +373,8 @@ def bench_kernel_coef(kermac, device, args, steps=None, warmup=None, with_gaussi
                                         "default_panels_ms": round(gaussian_panels_ms, 3),
                                         "matrix_core_parity_max_err_over_mean": gaussian_err,
                                         "default_panels_parity_max_err_over_mean": panels_err,
-                                        "note": "the default l2 mode 'auto' builds the kernel matrix in panels of 4096 centres "
-                                                "(1 GiB, reused) on the fp16 matrix instruction and contracts each panel; "
+                                        "note": "the default l2 mode 'auto' builds the kernel matrix on the fp16 matrix instruction and "
+                                                "contracts each tile where it is made; "
                                                 "l2 mode 'gram' is the fused kernel on the fp32 matrix instruction"}
     if with_gaussian:
         # Beside it: the Laplace kernel of the headline with 100 coefficient columns.  The fused kernel holds 64 per
