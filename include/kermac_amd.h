@@ -177,7 +177,8 @@ enum kmc_flags {
      * differences are not trusted are made again by the fused kernel.  n_ranges is not read.  kmc_kernel_coefficients_workspace_bytes says how
      * much memory it wants; without it, or where that says 0, the call is as without this flag. */
     KMC_FLAG_PRODUCT_PIECES = 8192,
-    /* With KMC_FLAG_PRODUCT_PIECES: added to `out` instead of stored (an error where the call cannot take that route). */
+    /* With KMC_FLAG_PRODUCT_PIECES: added to `out` instead of stored (an error where the call cannot take that route; the size rules
+     * look at a launch alone, so that a product in several runs of centres sets KMC_FLAG_GRAM_WORKSPACE_ANY_SIZE in all of them). */
     KMC_FLAG_PRODUCT_ACCUMULATE = 16384
 };
 

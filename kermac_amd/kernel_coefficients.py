@@ -362,8 +362,11 @@ def _run_in_panels(plan, shape, stream, device, debug):
 
     rows, panels, ld, splits, route = shape
     L, M, N, O = plan.L, plan.M, plan.N, plan.O
-    if route and _products_of_tiles(plan, shape, stream, device, debug):
-        return True
+    if route:
+        # decided for the whole call: the library's rule, asked for the last panel alone, refuses one that is much shorter than the others
+        route |= _backend.FLAG_GRAM_WORKSPACE_ANY_SIZE
+        if _products_of_tiles(plan, (rows, panels, ld, splits, route), stream, device, debug):
+            return True
     parts = panels * splits                                      # 0: no partial products, the panels accumulate
     params = plan.params
     block = _backend.BuildKernelParams.from_buffer_copy(params.kernel)
