@@ -123,8 +123,7 @@ def run_kernel_coefficients(
         from .build_a_kernel import _attach_gram_centre
         panels = _panel_shape(plan, _backend.FLAG_L2_GRAM_BF16) if aot else None
         if aot and panels is None and plan.l2_auto and _auto_products_of_tiles(plan):
-            whole = _centres_at_once(plan, _backend.FLAG_L2_GRAM_BF16 | _backend.FLAG_GRAM_WORKSPACE_ANY_SIZE)
-            if whole is not None and _products_of_tiles(plan, whole, stream, a.device, debug):
+            if _products_of_tiles_at_any_size(plan, stream, a.device, debug):
                 return plan.out
         if panels is None and plan.l2_auto and not _auto_fused_on_matrix_cores(plan):
             kernel.flags &= ~(_backend.FLAG_L2_GRAM | _backend.FLAG_L2_GRAM_BF16)
@@ -470,16 +469,35 @@ def _auto_products_of_tiles(plan):
             and _auto_route_beats_one_step(plan.params.kernel))
 
 
-def _centres_at_once(plan, route):
-    """(centres, panels, -, -, route): as _panel_shape, by the room for the products of the tiles alone."""
-    budget = int(os.environ.get("KERMAC_AMD_COEFFICIENT_PANEL_BYTES", _PANEL_BYTES))
-    per_tile = 4 * plan.L * plan.M * (-(-plan.O // 4) * 4)          # of 128 centres
-    if budget < per_tile:
+def _centres_at_once(plan, route, share=1):
+    """(centres, panels, -, -, route): as _panel_shape, but what the budget (a `share`-th of it) bounds is the products of the tiles and the pieces of
+    the centres; None when it does not hold 256 of them."""
+    budget = int(os.environ.get("KERMAC_AMD_COEFFICIENT_PANEL_BYTES", _PANEL_BYTES)) // share
+    pieces = plan.L if plan.L > 1 and (plan.params.kernel.b_bs != 0 or plan.params.kernel.a_bs != 0) else 1      # entries with a centre or points of their own
+    per_run = 256 * 4 * (pieces * (-(-plan.K // 32) * 32) + plan.L * plan.M * (-(-plan.O // 4) * 4) // 128)      # of 256 centres, two tiles
+    if budget < per_run:
         return None
-    rows = min(plan.N, budget // per_tile * 128, 65535 * 128)
+    rows = min(plan.N, budget // per_run * 256, 65535 * 128)
     panels = -(-plan.N // rows)
     rows = min(plan.N, -(-(-(-plan.N // panels)) // 256) * 256)
     return rows, -(-plan.N // rows), None, None, route
+
+
+# Where the memory is refused, a quarter and a sixteenth of the budget are tried: 200 x 3000000 x 100 with 10 columns, 1.7 GB in all, goes in
+# two runs of centres as a rule and in seven under a limit of 300 MB.
+_PRODUCTS_OF_TILES_SHARES = (1, 4, 16)
+
+
+def _products_of_tiles_at_any_size(plan, stream, device, debug):
+    tried = None
+    for share in _PRODUCTS_OF_TILES_SHARES:
+        shape = _centres_at_once(plan, _backend.FLAG_L2_GRAM_BF16 | _backend.FLAG_GRAM_WORKSPACE_ANY_SIZE, share)
+        if shape is None:
+            return False
+        if shape != tried and _products_of_tiles(plan, shape, stream, device, debug):
+            return True
+        tried = shape
+    return False
 
 
 def _products_of_tiles(plan, shape, stream, device, debug):

@@ -61,6 +61,50 @@ def test_every_panel_gets_the_workspace_of_the_first(monkeypatch, descriptor, L,
         assert 0 < wanted <= given, f"a panel of {n} centres: the library wants {wanted} bytes for its route, {given} are there"
 
 
+@pytest.mark.parametrize("limit,runs", [(None, 2), (300 << 20, 7), (100 << 20, 27), (10 << 20, None)])
+def test_the_memory_of_a_run_of_centres_is_bounded(monkeypatch, limit, runs):
+    """Few rows against many centres: the pieces of the centres, 512 bytes each here, are most of what a run takes."""
+    L, M, N, K, O = 1, 200, 3000000, 100, 10
+    plan = module._plan_run_kernel_coefficients(GAUSSIAN, torch.empty(M, K), torch.empty(N, K), torch.empty(N, O), torch.empty(L, M, O), None, None, None, 10.0, None, None, 0, 0,
+                                                require_device=False)
+    assert module._auto_products_of_tiles(plan) and module._panel_shape(plan, _backend.FLAG_L2_GRAM_BF16) is None
+    taken, launched = [], []
+
+    def allocate(nbytes, device):
+        if limit is not None and nbytes > limit:
+            return None
+        taken.append(nbytes)
+        return Somewhere()
+
+    monkeypatch.setattr(_scratch, "allocate", allocate)
+    monkeypatch.setattr(_backend, "kernel_times_coefficients", lambda params, stream: launched.append((params.kernel.n, params.kernel.b - plan.params.kernel.b)))
+    assert module._products_of_tiles_at_any_size(plan, 0, torch.device("cpu"), False) == (runs is not None)
+    assert len(launched) == (runs or 0)
+    if runs is not None:
+        assert len(taken) == 1 and taken[0] <= 1 << 30
+        assert sum(n for n, _ in launched) == N and [b for _, b in launched] == [4 * K * launched[0][0] * i for i in range(runs)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("limit,runs", [(None, 1), (12 << 20, 4), (1 << 20, 0)])
+def test_fewer_centres_at_once_where_the_memory_is_refused(device, monkeypatch, capsys, limit, runs):
+    M, N, K, O = 200, 60000, 100, 10
+    monkeypatch.setenv("KERMAC_AMD_COEFFICIENT_PANEL_BYTES", str(40 << 20))
+    g = torch.Generator().manual_seed(3)
+    a, b, coef = (torch.randn(*shape, generator=g).to(device) for shape in ((M, K), (N, K), (N, O)))
+    kermac.set_max_scratch_bytes(limit)
+    try:
+        got = kermac.run_kernel(GAUSSIAN, a, b, coefficients=coef, bandwidth=10.0, debug=True)
+    finally:
+        kermac.set_max_scratch_bytes(None)
+    said = capsys.readouterr().out
+    rows = -(-N // max(runs, 1) // 256) * 256 if runs != 1 else N
+    assert (f"tile by tile, {rows} centres at once" in said) == (runs > 0), said
+    matrix = torch.exp(-torch.cdist(a.double(), b.double()) ** 2 / 200)
+    error, size = (got.double()[0] - matrix @ coef.double()).abs(), (1e-5 + N * 2.0 ** -24) * matrix @ coef.double().abs()
+    assert torch.all(error <= size), f"{(error / size).max().item():.3g} of the bound"
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("O", [10, 40])
 @pytest.mark.parametrize("descriptor,M", [(GAUSSIAN, 3072), (LINEAR, 4096)])
