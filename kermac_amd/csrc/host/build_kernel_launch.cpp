@@ -256,7 +256,7 @@ int kmc_build_kernel(const kmc_build_kernel_params *params, void *stream)
         hipError_t g = launch_gram_f16_wide(params, args, static_cast<hipStream_t>(stream), &wide, &sample_taken);
         if (g != hipSuccess) return fail_hip(g, "gram_f16_wide launches");
         if (wide) args.sample = sample_taken;
-        // (the route's workspace has the queues of the repair launch behind the sample, which clears them)
+        // (the route's workspace has the queues and the list of the repair launches behind the sample, whose launch clears the counters)
         if (sample_taken) args.repair_queue = const_cast<unsigned *>(sample_taken) + kmc::BK_SAMPLE_TILES;
         if (!wide) {
             // The one-step kernels: with KMC_SAMPLE_BYTES of workspace, a sample of the result first (gram_probe.hip),

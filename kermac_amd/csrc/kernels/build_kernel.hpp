@@ -66,7 +66,7 @@ struct BuildKernelArgs {
     // where m == n + same_shift (a set against itself or against a run of its own rows): their distance is zero, which
     // |a|^2 + |b|^2 - 2 a.b cannot tell.  (The last fields, so that kernels that know nothing of them are compiled as they were.)
     int same_points, same_shift;
-    // build_kernel_repair only: what its workgroups take tiles from, behind the sample
+    // repair_scan and build_kernel_repair only: BK_REPAIR_WORDS words, which the launch that takes the sample clears, and the list of marked tiles
     unsigned *repair_queue;
 };
 
@@ -786,15 +786,42 @@ __global__ __launch_bounds__(BK_THREADS, 4) void build_kernel_four_waves(const B
     build_kernel_tile<INNER_OP, INNER_POW, LOAD_COL_VEC, LOAD_COL_VEC>(args, lds_a, lds_b, threadIdx.x, blockIdx.x, gridDim.x, blockIdx.y);
 }
 
-// The repair launch of a result of many tiles, of which as a rule none carries the marker: with a workgroup per tile it is bound by the
-// latency of a load each, four workgroups to a CU (30000 x 30000, 56400 tiles, 65 us, now 25; 12000 x 9000 x 512,
-// 6768 tiles, the call 369 -> 348).  Here as many workgroups as the chip holds look at
-// BK_REPAIR_CHUNK tiles at a time and recompute those that carry it.  They take the tiles, in their order, from eight queues, one per XCD
-// (tile_of_workgroup), so that a result with many marked ones stays balanced; where the sample left everything to this
-// launch (`sample` null: to another one in front of it), tile by tile.  (A fixed share for every workgroup: such results 5 to 12 % slower.)
+// The repair of a result of many tiles, of which as a rule none carries the marker, in two launches.  With a workgroup per tile it is bound by the
+// latency of a load each, four workgroups to a CU.  repair_scan looks at a tile per lane and collects the marked ones in a list;
+// build_kernel_repair, as many workgroups as the chip holds, takes them from there one by one, so that marked tiles that lie together
+// are shared out like any others.  Where the sample left everything to this launch (`sample` null: to another one in front of it) it takes
+// all tiles, in their order, from eight queues, one per XCD (tile_of_workgroup).
+// A workgroup per tile / one per 32 tiles in turn / this, us: no tile marked, 30000 x 30000 x 1024, 56400 tiles, the launches 65 / 25 / 10, the call 12000 x 9000 x 512,
+// 6768 tiles, 389 / 362 / 362; 64 clusters stored one after the other, a tile in 64 marked, those calls 5830 / 6905 / 5390 and 582 / 1143 / 495, eight clusters
+// 10100 / 14200 / 8600; all tiles marked 29350 / 29250 / 29300 and 2130 / 2140 / 2070.
 constexpr int BK_REPAIR_WORKGROUPS = 768;
-constexpr int BK_REPAIR_CHUNK = 32;                   // at most 32
 constexpr int BK_REPAIR_QUEUES = 8;
+constexpr int BK_REPAIR_COUNT = BK_REPAIR_QUEUES, BK_REPAIR_NEXT = BK_REPAIR_QUEUES + 1;      // of the list: its length, how many are taken
+constexpr int BK_REPAIR_WORDS = 16;                                                           // queues and counters, in front of the list
+constexpr int BK_REPAIR_MIN_TILES = 4097;             // a workgroup per tile looks at 4096 of them in 5 us
+constexpr int BK_REPAIR_MAX_TILES = 0x3fffffff;
+
+template <int>
+__global__ __launch_bounds__(BK_THREADS) void repair_scan(const BuildKernelArgs args)
+{
+    if (args.sample && sample_leaves_it_to_the_direct_kernel(args.sample)) return;
+    const int width = args.grid_width;
+    const i64 id = (i64)blockIdx.x * BK_THREADS + threadIdx.x;
+    bool marked = false;
+    if (id < (i64)width * args.l) {
+        const int batch = (int)id / width;
+        int tile_m, tile_n;
+        if (tile_of_workgroup(args, (int)id - batch * width, width, batch, tile_m, tile_n))
+            marked = __float_as_uint(args.c[batch * args.c_bs + (i64)tile_n * BK_TILE_N * args.c_ld + tile_m * BK_TILE_M]) == BK_REPAIR_MARKER;
+    }
+    const unsigned long long found = __ballot(marked);
+    if (!found) return;
+    unsigned first = 0;
+    const int lane = threadIdx.x & 63;
+    if (lane == 0) first = atomicAdd(args.repair_queue + BK_REPAIR_COUNT, (unsigned)__popcll(found));
+    first = (unsigned)__builtin_amdgcn_readfirstlane((int)first);
+    if (marked) args.repair_queue[BK_REPAIR_WORDS + first + __popcll(found & ((1ull << lane) - 1))] = (unsigned)id;
+}
 
 template <int INNER_OP, int INNER_POW, int LOAD_A, int LOAD_B>
 __global__ __launch_bounds__(BK_THREADS, 3) void build_kernel_repair(const BuildKernelArgs args)
@@ -802,37 +829,25 @@ __global__ __launch_bounds__(BK_THREADS, 3) void build_kernel_repair(const Build
     __shared__ __attribute__((aligned(16))) float lds_a[2 * BK_LDS_SLICE + BK_LDS_PITCH];
     __shared__ __attribute__((aligned(16))) float lds_b[2 * BK_LDS_SLICE + BK_LDS_PITCH];
     __shared__ int next;
-    const int lane = threadIdx.x & 63;
-    const int width = args.grid_width, total = width * args.l;             // (the host checks that these fit)
-    const int queue = blockIdx.x % BK_REPAIR_QUEUES, begin = gridDim.x / BK_REPAIR_QUEUES;
-    const int chunk = args.sample && sample_leaves_it_to_the_direct_kernel(args.sample) ? 1 : BK_REPAIR_CHUNK;
-    int first = (int)blockIdx.x / BK_REPAIR_QUEUES * chunk;                // tile BK_REPAIR_QUEUES * first + queue of the launch
-    while (BK_REPAIR_QUEUES * (i64)first + queue < total) {
-        const i64 id = BK_REPAIR_QUEUES * ((i64)first + lane) + queue;
-        int tile_m, tile_n;
-        bool marked = false;
-        if (lane < chunk && id < total) {
-            const int batch = (int)id / width;
-            if (tile_of_workgroup(args, (int)id - batch * width, width, batch, tile_m, tile_n))
-                marked = __float_as_uint(args.c[batch * args.c_bs + (i64)tile_n * BK_TILE_N * args.c_ld + tile_m * BK_TILE_M]) == BK_REPAIR_MARKER;
-        }
-        // the same in every wave: none of them stores before all have passed the barriers of the walk
-        unsigned found = (unsigned)__ballot(marked);
-        while (found) {
-            const int here = BK_REPAIR_QUEUES * (first + __builtin_ctz(found)) + queue, batch = here / width;
-            found &= found - 1;
-            // a copy of the lane's id that the compiler cannot see through: what it derives from it before the loop costs 50 registers and a
-            // wave per SIMD
-            int tid = threadIdx.x;
-            asm volatile("" : "+v"(tid));
-            build_kernel_tile<INNER_OP, INNER_POW, LOAD_A, LOAD_B>(args, lds_a, lds_b, tid, here - batch * width, width, batch);
-            __syncthreads();            // the staging arrays, which the mirrored stores read
-        }
-        // (taken in front of the chunk, so that it arrives meanwhile, the last tiles wait for workgroups that are still at others: 5 % of 6768 marked ones)
-        if (threadIdx.x == 0) next = begin * chunk + (int)atomicAdd(args.repair_queue + queue, (unsigned)chunk);
+    const int width = args.grid_width;
+    const bool everything = args.sample && sample_leaves_it_to_the_direct_kernel(args.sample);
+    const int queue = blockIdx.x % BK_REPAIR_QUEUES;
+    // of the queue or of the list: the entry at hand, the first that is not handed out with the launch, all of them (the host checks that they fit)
+    int at = everything ? (int)blockIdx.x / BK_REPAIR_QUEUES : (int)blockIdx.x;
+    const int handed_out = everything ? (int)gridDim.x / BK_REPAIR_QUEUES : (int)gridDim.x;
+    const int all = everything ? (width * args.l - queue + BK_REPAIR_QUEUES - 1) / BK_REPAIR_QUEUES : (int)args.repair_queue[BK_REPAIR_COUNT];
+    unsigned *taken = args.repair_queue + (everything ? queue : BK_REPAIR_NEXT);
+    while (at < all) {
+        const int id = everything ? BK_REPAIR_QUEUES * at + queue : (int)args.repair_queue[BK_REPAIR_WORDS + at], batch = id / width;
+        // a copy of the lane's id that the compiler cannot see through: what it derives from it before the loop costs 50 registers and a
+        // wave per SIMD
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));
+        build_kernel_tile<INNER_OP, INNER_POW, LOAD_A, LOAD_B>(args, lds_a, lds_b, tid, id - batch * width, width, batch);
+        __syncthreads();            // the staging arrays, which the mirrored stores read, and `next`
+        if (threadIdx.x == 0) next = handed_out + (int)atomicAdd(taken, 1u);
         __syncthreads();
-        first = __builtin_amdgcn_readfirstlane(next);
-        __syncthreads();
+        at = __builtin_amdgcn_readfirstlane(next);
     }
 }
 

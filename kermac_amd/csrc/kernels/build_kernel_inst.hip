@@ -80,10 +80,13 @@ static hipError_t launch_one(const kmc::BuildKernelArgs &args, dim3 grid, hipStr
             return launch(kmc::build_kernel_four_waves<KMC_INNER_OP, KMC_INNER_POW>, grid, dim3(kmc::BK_THREADS), stream, args);
     }
 #if KMC_INNER_OP == 0 && KMC_INNER_POW == 2
-    // A workgroup per tile scans 4096 of them in 5 us, and there the queues would be most of the launch
     const int64_t tiles = static_cast<int64_t>(args.grid_width) * args.l;
-    if (args.repair_only && args.repair_queue && tiles > 4096 && tiles <= 0x3fffffff)
+    if (args.repair_only && args.repair_queue && tiles >= kmc::BK_REPAIR_MIN_TILES && tiles <= kmc::BK_REPAIR_MAX_TILES) {
+        const dim3 scan(static_cast<unsigned>((tiles + kmc::BK_THREADS - 1) / kmc::BK_THREADS));
+        const hipError_t status = launch(kmc::repair_scan<0>, scan, dim3(kmc::BK_THREADS), stream, args);
+        if (status != hipSuccess) return status;
         return launch(kmc::build_kernel_repair<KMC_INNER_OP, KMC_INNER_POW, LOAD_A, LOAD_B>, dim3(kmc::BK_REPAIR_WORKGROUPS), dim3(kmc::BK_THREADS), stream, args);
+    }
 #endif
     return launch(kmc::build_kernel<KMC_INNER_OP, KMC_INNER_POW, LOAD_A, LOAD_B>, grid, dim3(kmc::BK_THREADS), stream, args);
 }

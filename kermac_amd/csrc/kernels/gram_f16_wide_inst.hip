@@ -135,7 +135,8 @@ void place_operand(OperandRegions &r, int rows, bool broadcast, int l, bool once
 
 // Grid, slices and the regions of both operands in the workspace; tiles_m and tiles_n are set.
 // a_shared, b_shared: one operand for all batch entries.  a_once, b_once: one launch makes its pieces (made_once).
-bool place_wide(int m, int n, int k, int l, bool a_shared, bool b_shared, bool a_once, bool b_once, bool symmetric, WideLayout *layout)
+// repair_tiles: the list of the repair launch, as long as all tiles of the result.
+bool place_wide(int m, int n, int k, int l, bool a_shared, bool b_shared, bool a_once, bool b_once, bool symmetric, int64_t repair_tiles, WideLayout *layout)
 {
     // room for any tile of the product kernel in a grid, n tiles padded to the XCDs
     if (static_cast<int64_t>(layout->tiles_m) * (layout->tiles_n + kmc::BK_XCDS) * 4 > 0x7fffffff) return false;
@@ -146,7 +147,7 @@ bool place_wide(int m, int n, int k, int l, bool a_shared, bool b_shared, bool a
     layout->centre = layout->centre_floats ? place(cursor, 4 * layout->centre_floats * layout->centre_batches) : 0;
     if (symmetric) layout->b = layout->a;      // one panel, split once
     else place_operand(layout->b, n, b_shared, l, b_once, *layout, cursor);
-    layout->sample = place(cursor, kmc::BK_SAMPLE_BYTES + 4 * kmc::BK_REPAIR_QUEUES);
+    layout->sample = place(cursor, kmc::BK_SAMPLE_BYTES + 4 * (kmc::BK_REPAIR_WORDS + repair_tiles));
     layout->bytes = cursor;
     return true;
 }
@@ -186,10 +187,11 @@ bool wide_layout(const kmc_build_kernel_params *p, const kmc::BuildKernelArgs &a
     const bool own_centre = squared_differences && (p->flags & KMC_FLAG_GRAM_OWN_CENTRE);
     layout->centre_batches = own_centre && args.a_bs != 0 ? args.l : 1;
     layout->centre_floats = own_centre ? 2 * ((args.k + kmc::GRAM_CENTRE_PAD - 1) / kmc::GRAM_CENTRE_PAD * kmc::GRAM_CENTRE_PAD) + kmc::GRAM_CENTRE_PAD : 0;
+    const int64_t ids = static_cast<int64_t>(args.grid_width) * args.l;
     const bool one_centre = products || (own_centre ? layout->centre_batches == 1 : !args.centre || args.centre_bs == 0);
     return place_wide(args.m, args.n, args.k, args.l, args.a_bs == 0 && one_centre, args.b_bs == 0 && one_centre,
                       made_once(args.a, args.a_ld, args.a_bs, p->a_majorness, p->flags, args.k), made_once(args.b, args.b_ld, args.b_bs, p->b_majorness, p->flags, args.k),
-                      args.symmetric, layout);
+                      args.symmetric, squared_differences && ids >= kmc::BK_REPAIR_MIN_TILES && ids <= kmc::BK_REPAIR_MAX_TILES ? ids : 0, layout);
 }
 
 kmc::GramRowsArgs rows_args(const float *x, int64_t ld, int64_t bs, int rows, int majorness, bool scalar_only,
@@ -484,7 +486,7 @@ hipError_t launch_gram_f16_wide(const kmc_build_kernel_params *p, const kmc::Bui
     if (status != hipSuccess) return status;
     if ((split_a && layout.a.once) || (split_b && layout.b.once)) {
         status = launch_gram_once_both(split_a && layout.a.once ? &rows_a : nullptr, layout.a.batches, split_b && layout.b.once ? &rows_b : nullptr,
-                                       layout.b.batches, sample ? gram_probe_args(p, wide.kernel, sample, centre_pairs, kmc::BK_REPAIR_QUEUES) : kmc::GramProbeArgs{}, sample != nullptr, stream);
+                                       layout.b.batches, sample ? gram_probe_args(p, wide.kernel, sample, centre_pairs, kmc::BK_REPAIR_WORDS) : kmc::GramProbeArgs{}, sample != nullptr, stream);
         sampled = true;
     }
     if (status == hipSuccess && split_a && split_b && !layout.a.once && !layout.b.once) {
@@ -493,7 +495,7 @@ hipError_t launch_gram_f16_wide(const kmc_build_kernel_params *p, const kmc::Bui
         if (status == hipSuccess && split_a && !layout.a.once) status = launch_gram_rows(rows_a, layout.a.batches, stream);
         if (status == hipSuccess && split_b && !layout.b.once) status = launch_gram_rows(rows_b, layout.b.batches, stream);
     }
-    if (status == hipSuccess && sample && !sampled) status = launch_gram_probe(p, wide.kernel, sample, centre_pairs, kmc::BK_REPAIR_QUEUES, stream);
+    if (status == hipSuccess && sample && !sampled) status = launch_gram_probe(p, wide.kernel, sample, centre_pairs, kmc::BK_REPAIR_WORDS, stream);
     if (status != hipSuccess) return status;
     if (sample) {
         wide.kernel.sample = sample;
@@ -592,7 +594,7 @@ bool gradient_l2_layout(const kmc_norm_gradient_params *p, GradientL2Layout *lay
     wide.tiles_m = (p->m + kmc::GW_TILE - 1) / kmc::GW_TILE;
     wide.tiles_n = static_cast<int>((rows + kmc::GW_TILE - 1) / kmc::GW_TILE);
     if (!gradient_l2_pays(p, wide.tiles_m, wide.tiles_n)) return false;
-    if (!place_wide(p->m, static_cast<int>(rows), p->k, p->l, p->a_bs == 0, false, false, false, false, &wide)) return false;
+    if (!place_wide(p->m, static_cast<int>(rows), p->k, p->l, p->a_bs == 0, false, false, false, false, 0, &wide)) return false;
     int64_t cursor = wide.bytes;
     layout->shift = place(cursor, static_cast<int64_t>(p->l) * p->n * 4);
     layout->c_transposed = place(cursor, static_cast<int64_t>(p->l) * p->k * p->o * 4);

@@ -29,7 +29,7 @@ struct GramProbeArgs {
     int centre_pairs;                          // > 0: no flag was stored, these many pairs say it (CentreSums)
     float trust;
     unsigned *sample;                          // [BK_SAMPLE_TILES]
-    int queues;                                // that many words behind it are cleared, for build_kernel_repair
+    int queues;                                // that many words behind it are cleared, for the repair launches
 };
 
 // Whether subtracting the centre would lower the norms, and with them the error of the expansion, by under 2 %: |c|^2 against the variances.

@@ -59,7 +59,7 @@ _ROWS = (
      "the centre (`sample_mean_rows` or `_columns`), `gram_rows_once` or `gram_columns_once` (with the sample in the same launch) or, k contiguous and aligned from K = 2049 on, "
      "`gram_row_stats_pair` + `gram_f16_split_pair` + `gram_probe_operands`, "
      "`gram_f16_wide` (fp16 pieces, tiles of 256 × 128 from {WIDE_LARGE_TILE_MIN_TILES} on or where those fit the chip at once and 128 × 128 do not, else 128 × 128; in batches of ≥ 8 entries of ≤ {WIDE_ENTRY_PER_XCD_MAX_TILES} tiles of 128 × 128 each entry on one XCD), repair launch "
-     "of the direct kernel (more than 4096 tiles: `build_kernel_repair`)"),
+     "of the direct kernel (more than 4096 tiles: `repair_scan` and `build_kernel_repair`)"),
     ("",
      "mode `\"auto\"` with memory for it, what the next line describes, or K < {build_a_kernel.AUTO_ONE_STEP_MIN_K} and tiles of 128 × 128 over the batch · K ≥ "
      "{build_a_kernel.AUTO_ROUTE_MIN_TILES_TIMES_K}; not a result of one row of tiles over more than {build_a_kernel.AUTO_ROUTE_ONE_ROW_OF_TILES_MAX_VALUES} values of both operands",
