@@ -112,7 +112,7 @@ enum kmc_flags {
      * from two fp16 pieces per value and a scale per row, by the route that
      * KMC_FLAG_L2_GRAM_BF16 describes (kmc_gram_workspace_bytes says which, and how much memory it
      * wants).  Error below 3 * 2^-22 sum_k |a b| + k * 2^-38 max|a[m]| max|b[n]| (a value below
-     * 2^-28 of the largest of its row is kept to 2^-40 of that largest one, not to 2^-22 of
+     * 2^-17 of the largest of its row is kept to 2^-39 of that largest one, not to 2^-22 of
      * itself): the size of the rounding of an fp32 sum of k >= 100 terms; nothing cancels, so
      * nothing is checked or repaired.  Without a workspace, or
      * for a problem the query reports 0 for, the direct kernel runs. */

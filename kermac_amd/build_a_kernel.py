@@ -798,11 +798,6 @@ def _auto_matrix_cores(params, asked):
         route_bytes = _route_bytes(params, any_size)
         if _workspace_allowed(route_bytes):
             return any_size, route_bytes, chosen
-    if asked & _backend.FLAG_DOT_PIECES and not route_bytes and _auto_route_beats_direct_products(params, asked):
-        any_size = asked | _backend.FLAG_GRAM_WORKSPACE_ANY_SIZE
-        route_bytes = _route_bytes(params, any_size)
-        if _workspace_allowed(route_bytes):
-            return any_size, route_bytes, chosen
     return chosen, 0, chosen
 
 
@@ -831,17 +826,11 @@ def _auto_route_beats_direct(params):
             and -(-params.m // 128) * -(-params.n // 128) * params.l * params.k >= _AUTO_ROUTE_MIN_TILES_TIMES_K)
 
 
-# Sums of products, below what the library's rule asks for.  Direct / route, us: 919 x 657 x 64 four times (tiles * K 12288) 15.0 / 18.7, 1728 x 619 x 64 four
-# times (17920) 19.1 / 19.7, 6110 x 382 x 87 twice (25056) 30.9 / 25.7, 640 x 4045 x 200 (32000) 32 / 21, 652 x 3100 x 419 63 / 21, 4320 x 5541 x 161
-# 130 / 58, 7181 x 26944 x 84 607 / 345.  The route's error against 64 bits (2-norm) is 0.58 .. 0.82 of the direct kernel's on normal and uniform values,
-# 0.33 .. 1.15 on heavy-tailed ones; columns that span six decades sum few terms, and each product of the pieces carries 2^-22
-# (K = 64 1.0e-7 / 3.3e-8).  A call that the direct path cuts over k stays there: its short sums are more exact.
-_AUTO_PRODUCTS_MIN_TILES_TIMES_K = 20000
-
-
-def _auto_route_beats_direct_products(params, asked):
-    return (-(-params.m // 128) * -(-params.n // 128) * params.l * params.k >= _AUTO_PRODUCTS_MIN_TILES_TIMES_K
-            and not _direct_path_would_cut(params, asked))
+# Sums of products below what the library's rule asks for stay with the direct kernel, whose error is below K 2^-24 sum_k |a b| whatever the values are.  Pieces
+# are scaled by a row's largest magnitude and hold what lies more than 2^17 below it to 2^-39 of it: where the large values of one operand meet the small ones of the
+# other, as features in units of their own against weights of the inverse units do, and nothing in a product of two sets tells a route that its result is off.
+# Error / sum |a b| of the direct kernel and of the route at K = 200, scales of the features spread over 6 decades 3e-7 / 3e-7, over 8 4e-7 / 2e-5, over 10
+# 3e-7 / 2e-3.  (Direct / route, us: 640 x 4045 x 200 32 / 21, 652 x 3100 x 419 63 / 21, 4320 x 5541 x 161 130 / 58.)
 
 
 def _auto_one_step_flags(params, asked):

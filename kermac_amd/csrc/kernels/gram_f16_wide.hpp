@@ -18,7 +18,7 @@
 // Accuracy.  x - h1 is exact in fp32 and h2 keeps 11 of its bits: |x - h1 - h2| <= 2^-22 |x|, or
 // 2^-25 where h2 is subnormal, which is 2^-39 of the row's largest magnitude.  The dropped product
 // a2 b2 is below 2^-22 |a_k b_k|.  The error of a dot product from the pieces is therefore below
-// 3 * 2^-22 sum_k |a_k b_k| <= 3.6e-7 (|a|^2 + |b|^2), in practice far less since the roundings
+// 3 * 2^-22 sum_k |a_k b_k| + k 2^-38 max|a| max|b| <= (3.6e-7 + k 2^-39) (|a|^2 + |b|^2), in practice far less since the roundings
 // do not line up, beside the rounding of the fp32 accumulation that every matrix-core path has
 // (products of fp16 pieces are exact in fp32).  The scale per row is what makes the bound relative
 // to that row's norm, which is what the trust rule of gram_kernel.hpp needs: with one scale per

@@ -12,8 +12,8 @@
 // the pieces (GW_EPILOGUE_GRADIENT_L2: three piece products per 32 k); its epilogue fetches d and g
 // and stores e.  Where the fp32 kernels build c a (d - b) value by value on the vector ALU and
 // contract it on the fp32 matrix instruction, this route has no work per (o, n, m, k) outside the
-// matrix instruction.  Error of the product from the pieces below 3 * 2^-22 sum_k |c a (b - s)|;
-// g and the rest are fp32.
+// matrix instruction.  Error of the product from the pieces below 3 * 2^-22 sum_k |c a (b - s)| +
+// k 2^-38 max|a| max|c (b - s)|; g and the rest are fp32.
 //
 // This header: the kernels that prepare s, the transposed c, and the pieces of a and p (g itself comes from
 // kmc_matrix_times_coefficients with a as the stored panel).  p is never stored: its values are made from b and c

@@ -83,8 +83,6 @@ _ROWS = (
      "≤ {WIDE_MAX_PADDING_PERCENT} % padding; or K ≥ {DOT_LONG_K}, tiles · K ≥ {DOT_LONG_MIN_TILES_TIMES_K}, ≥ {DOT_LONG_MIN_TILES_BATCHED} tiles "
      "over a batch ({DOT_LONG_MIN_TILES_SINGLE} of a single problem)",
      "the workspace route with `gram_f16_wide<GW_EPILOGUE_DOT>` (no trust check, no repair)"),
-    ("", "with memory for it: tiles of 128 × 128 over the batch · K ≥ {build_a_kernel.AUTO_PRODUCTS_MIN_TILES_TIMES_K}, but for a call that the direct path would cut over k",
-     "the same route (`KMC_FLAG_GRAM_WORKSPACE_ANY_SIZE`)"),
     ("", "otherwise", "direct `build_kernel<DOT, NOOP>`"),
     ("`cdist(p=1)`, `run_kernel` of DIFF + ABS (L1 norm, Laplace-L1)",
      "l1 mode `\"fixed\"` (opt-in) and ≥ {L1_FIXED_MIN_TILES} tiles of 128 × 128 over the batch, K ≥ {L1_FIXED_MIN_K}",

@@ -543,7 +543,7 @@ def _products_of_tiles(plan, shape, stream, device, debug):
 # bound by it from about 128 columns on (O = 1000 above: 20 of 31 ms).  The contraction of a panel is itself a
 # sum of products, out[m, o] = sum_n panel[n, m] coef[n, o], with both operands stored the way kmc_build_kernel reads
 # them (m and o contiguous), so from _PIECES_MIN_COLUMNS columns on it runs on kmc_build_kernel's route for sums of
-# products (KMC_FLAG_DOT_PIECES: two fp16 pieces per value, scale per row m and o, error below 3 * 2^-22 sum_n |k c|)
+# products (KMC_FLAG_DOT_PIECES: two fp16 pieces per value, scale per row m and o, error below 3 * 2^-22 sum_n |k c| + N 2^-38 max|k| max|c|)
 # into the result for the first panel and into a buffer that is added to the result for the others.  Gaussian
 # kernel, fp32 contraction -> pieces: L = 4, M = N = 16384, K = 256 at O = 256 9.6 -> 8.1 ms, O = 512 15.6 -> 9.4,
 # O = 1000 25.5 -> 12.0; M = 10000, N = 100000, K = 784, O = 1000 28.5 -> 17.2 ms.  The split of a panel costs what

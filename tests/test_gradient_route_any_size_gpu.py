@@ -1,4 +1,4 @@
-"""Gradients below the library's rules for the fp16 routes, and products below its rule for theirs: the route that the launch-time models choose
+"""Gradients below the library's rules for the fp16 routes: the route that the launch-time models choose
 against float64 and against the kernels it takes the place of, in every form the calls come in."""
 import importlib
 
@@ -77,35 +77,5 @@ def test_gradient_without_memory_for_the_route_runs_as_before(device, monkeypatc
     kermac.set_max_scratch_bytes(300000)
     try:
         assert torch.equal(got, kermac.cdist_grad(*operands, p=p))
-    finally:
-        kermac.set_max_scratch_bytes(None)
-
-
-@pytest.mark.parametrize("L,M,N,K,k_contiguous", [(1, 640, 4045, 200, True), (2, 6110, 382, 87, False), (1, 1263, 1263, 320, False), (4, 917, 375, 230, True),
-                                                  (3, 129, 4500, 131, False), (1, 131, 16001, 93, True)])
-def test_products_on_the_route_of_any_size(device, L, M, N, K, k_contiguous):
-    g = torch.Generator(device=device).manual_seed(M + N + K)
-
-    def points(rows):
-        x = torch.randn(L, *((rows, K) if k_contiguous else (K, rows)), device=device, generator=g)
-        return x if k_contiguous else x.transpose(-1, -2)
-
-    a, b = points(M), points(N)
-    call = lambda: kermac.run_kernel(kermac.kernel_descriptor_mma, a, b)
-    assert any("gram_f16_wide" in name for name in kernels_of(call))
-    want, size = a.double() @ b.double().mT, a.double().abs() @ b.double().abs().mT
-
-    def errors(got):
-        off = (got.double() - want).abs()
-        return float(off.norm()), float((off / size).max())
-
-    on_route = errors(call())
-    with kermac.l2_mode("direct"):
-        direct = call()
-    on_direct = errors(direct)
-    assert on_route[0] <= 1.05 * on_direct[0] and on_route[1] <= on_direct[1] + 3 * 2.0 ** -22
-    kermac.set_max_scratch_bytes(4096)
-    try:
-        assert torch.equal(call(), direct)
     finally:
         kermac.set_max_scratch_bytes(None)
