@@ -256,17 +256,18 @@ def _f16_slices(M, N, O):
     return filled, wanted
 
 
-# The library's own rules for the fp16 routes (kmc_norm_gradient_workspace_bytes) take the calls that are large enough for the routes to win
-# everywhere; below them stand calls that the fp32 kernels, a workgroup walking the whole of k, take far longer for.  Which is
-# the faster one there follows from launch times in microseconds, fitted to 797 calls (M 64 .. 12000, N 8 .. 1024, K 64 .. 12000, O 1 .. 64, one
-# problem or a batch of two; the fits are off by 13 .. 19 %).  A route that they favour by 15 % is taken: over these calls the L1 gradient takes
-# 0.55 and the L2 gradient 0.67 of the fp32 kernels' time, 0.02 more than with the better one each time, and 9 calls of
-# them are slower by more than 5 % (the worst, 1009 x 254 x 1 x 1044, 69 -> 91 us).
-# fp32 / route, us: p = 1, 768 x 28 x 1 x 1651 twice 191 / 56; 192 x 22 x 32 x 1088 118 / 39; 428 x 18 x 4 x 256 40 / 23; 10304 x 675 x 1 x 175 117 / 227.
-# p = 2, 64 x 37 x 1 x 10691 twice 1229 / 358; 768 x 28 x 1 x 1651 twice 175 / 95; 256 x 62 x 4 x 832 124 / 74; 128 x 1013 x 32 x 135 twice 41 / 81.
+# The library's own rule for the L1 gradient's fp16 route (kmc_norm_gradient_workspace_bytes) takes the calls that are large enough for the route to win
+# everywhere; below it stand calls that the fp32 kernels, a workgroup walking the whole of k, take far longer for.  Which is
+# the faster one there follows from launch times in microseconds, fitted to sweeps of M 64 .. 12000, N 8 .. 1024, K 64 .. 12000, O 1 .. 64, one
+# problem or a batch of two (the fits are off by 13 .. 19 %).  A route that they favour by 15 % is taken.
+# fp32 / route, us: 768 x 28 x 1 x 1651 twice 191 / 56; 192 x 22 x 32 x 1088 118 / 39; 428 x 18 x 4 x 256 40 / 23; 10304 x 675 x 1 x 175 117 / 227.
+# Not the L2 gradient, below its own rule: the pieces of a and of c (b - s) are scaled by the largest magnitude of a row and hold what lies far below it to
+# fewer bits, and nothing in the sum of their products tells the call that its result is off.  Error (2-norm) of fp32 / route with the rows of a scaled over 8 decades and those of
+# c by the inverse: 717 x 52 x 16 x 390 twice 3.7e-7 / 1.6e-5, 2432 x 256 x 4 x 1984 4.9e-7 / 4.0e-5 (on normal values 0.4 to 0.6 of the fp32 kernels',
+# at 732 x 22 x 10 x 11840 twice 1650 / 468 us).  In the L1 gradient the pieces of a c meet 0 or 1: the route's error is 0.2 to 0.8 of theirs on such values too.
 _ROUTE_ADVANTAGE = 1.15
 # The sums of the fp32 kernels hold their rounding, which short slices keep small: the route's error (in the 2-norm, against 64 bits,
-# 87 calls of normal, uniform and heavy-tailed values) is 0.35 .. 0.8 of theirs on slices of the same depth, 0.9 at four times the depth, above theirs
+# normal, uniform, heavy-tailed and scaled values) is 0.2 .. 0.8 of theirs on slices of the same depth, 0.9 at four times the depth, above theirs
 # from seven times on (1602 x 178 x 10 x 4485 uncut against 8 slices 5.8e-7 / 4.2e-7).
 _ROUTE_MAX_DEPTH_RATIO = 4
 _ROUTE_MIN_FP32_US = 24.0
@@ -283,20 +284,16 @@ def _fp32_us(plan, slices, depth):
 def _route_us(plan, slices, depth):
     L, M, N, O, K = plan.L, plan.M, plan.N, plan.O, plan.K
     parts = L if slices == 1 else slices
-    if plan.params.norm_type == _NORM_L1:
-        workgroups = -(-M // 16) * -(-N // 128) * -(-O // 16) * parts
-        us = (18.5 + 0.0194 * depth * max(1.0, workgroups / 256) + (11e-6 * N + 2.6e-6 * M) * K * L + 23e-6 * N * (M + 256) * parts
-              + 1.7e-6 * L * M * N * O)
-        return us + 36.0 + 1.7e-6 * slices * M * N * O if slices > 1 else us
-    tiles = -(-M // 128) * -(-O * N // 128) * parts
-    us = 40.5 + depth * (0.0174 + 0.0168 * max(1.0, tiles / 256)) + 2.1e-6 * (O * N + M) * K * L + 3.3e-6 * L * M * N * O
-    return us + 47.0 + 3.3e-6 * slices * M * N * O if slices > 1 else us
+    workgroups = -(-M // 16) * -(-N // 128) * -(-O // 16) * parts
+    us = (18.5 + 0.0194 * depth * max(1.0, workgroups / 256) + (11e-6 * N + 2.6e-6 * M) * K * L + 23e-6 * N * (M + 256) * parts
+          + 1.7e-6 * L * M * N * O)
+    return us + 36.0 + 1.7e-6 * slices * M * N * O if slices > 1 else us
 
 
 def _route_of_any_size(plan):
-    """(slices, k per slice, leftover k) with which an L1 or L2 gradient that the library's rule leaves to the fp32 kernels is faster on the fp16
+    """(slices, k per slice, leftover k) with which an L1 gradient that the library's rule leaves to the fp32 kernels is faster on the fp16
     matrix instruction, or None."""
-    if plan.params.norm_type == _NORM_P or min(plan.L, plan.M, plan.N, plan.O, plan.K) < 1 or not _workspace_enabled():
+    if plan.params.norm_type != _NORM_L1 or min(plan.L, plan.M, plan.N, plan.O, plan.K) < 1 or not _workspace_enabled():
         return None
     shape = _shape_of_cuts(plan)
     fp32 = (1, plan.K, 0)
@@ -304,7 +301,7 @@ def _route_of_any_size(plan):
     if shape is not None and shape[1] >= 2:
         workgroups, most = shape
         fp32 = _cut_into(plan.K, max(2, round(_SPLIT_TARGET_WORKGROUPS / workgroups)), most)
-        wanted = _f16_slices(plan.M, plan.N, plan.O)[0] if plan.params.norm_type == _NORM_L1 else fp32[0]
+        wanted = _f16_slices(plan.M, plan.N, plan.O)[0]
         if min(wanted, most) >= 2:
             forms.append(_cut_into(plan.K, wanted, most))
     fp32_us = _fp32_us(plan, *fp32[:2])

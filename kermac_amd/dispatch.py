@@ -123,8 +123,8 @@ _ROWS = (
      "`gradient_signs_prepare` (rows of b and d ranked, a and c copied, bounds of their products), `norm_gradient_l1_f16` (16 outputs a tile; 8 with both pieces in its columns)"),
     ("`cdist_grad`, p = 2", "a model of both times favours the route by {GRADIENT_L2_ADVANTAGE_PERCENT} %, and the planes of `out` form one matrix",
      "`gradient_l2_prepare`, `gradient_l2_pieces_stats` and `_split`, `gram_f16_wide<GW_EPILOGUE_GRADIENT_L2>`"),
-    ("`cdist_grad`, p = 1 or 2, below those rules", "with memory for it, where models of the launch times favour the route, uncut or cut over k, over the fp32 kernels by a factor of "
-     "{cdist_grad.ROUTE_ADVANTAGE}, its slices at most {cdist_grad.ROUTE_MAX_DEPTH_RATIO} times as deep as theirs", "the same routes (`KMC_FLAG_GRAM_WORKSPACE_ANY_SIZE`)"),
+    ("`cdist_grad`, p = 1, below its rule", "with memory for it, where models of the launch times favour the route, uncut or cut over k, over the fp32 kernels by a factor of "
+     "{cdist_grad.ROUTE_ADVANTAGE}, its slices at most {cdist_grad.ROUTE_MAX_DEPTH_RATIO} times as deep as theirs", "the same route (`KMC_FLAG_GRAM_WORKSPACE_ANY_SIZE`)"),
     ("`cdist_grad`, otherwise", "O ≤ 8 / O > 8", "`norm_kernel_gradient` (vector ALU) / `norm_kernel_gradient_mfma` (fp32 matrix instruction), in runs of 32, 16 and ≤ 8 outputs; "
      "unbatched calls of fewer than {cdist_grad.SPLIT_BELOW_WORKGROUPS} workgroups are cut over k"),
     ("`run_kernel(..., coefficients=)`, squared differences, l2 mode `\"auto\"`",
