@@ -259,13 +259,16 @@ def _f16_slices(M, N, O):
 # The library's own rule for the L1 gradient's fp16 route (kmc_norm_gradient_workspace_bytes) takes the calls that are large enough for the route to win
 # everywhere; below it stand calls that the fp32 kernels, a workgroup walking the whole of k, take far longer for.  Which is
 # the faster one there follows from launch times in microseconds, fitted to sweeps of M 64 .. 12000, N 8 .. 1024, K 64 .. 12000, O 1 .. 64, one
-# problem or a batch of two (the fits are off by 13 .. 19 %).  A route that they favour by 15 % is taken.
+# problem or a batch of two (the fits are off by 13 .. 19 %).  An uncut route that they favour by 25 % is taken, one cut
+# over k by 15 %.  Of 260 other calls that they favour at all, the 171 uncut ones beyond 25 % are 0.97 .. 8.1 times as fast and the 41 cut ones beyond 15 % 0.94 .. 2.0 (two
+# slower, 68 x 13 x 2 x 3117 77 -> 82 us); the 16 uncut ones favoured by 15 to 25 % were 0.82 .. 1.6 (8808 x 37 x 16 x 174 44 -> 53 us).
 # fp32 / route, us: 768 x 28 x 1 x 1651 twice 191 / 56; 192 x 22 x 32 x 1088 118 / 39; 428 x 18 x 4 x 256 40 / 23; 10304 x 675 x 1 x 175 117 / 227.
 # Not the L2 gradient, below its own rule: the pieces of a and of c (b - s) are scaled by the largest magnitude of a row and hold what lies far below it to
 # fewer bits, and nothing in the sum of their products tells the call that its result is off.  Error (2-norm) of fp32 / route with the rows of a scaled over 8 decades and those of
 # c by the inverse: 717 x 52 x 16 x 390 twice 3.7e-7 / 1.6e-5, 2432 x 256 x 4 x 1984 4.9e-7 / 4.0e-5 (on normal values 0.4 to 0.6 of the fp32 kernels',
 # at 732 x 22 x 10 x 11840 twice 1650 / 468 us).  In the L1 gradient the pieces of a c meet 0 or 1: the route's error is 0.2 to 0.8 of theirs on such values too.
-_ROUTE_ADVANTAGE = 1.15
+_ROUTE_ADVANTAGE = 1.25
+_ROUTE_ADVANTAGE_CUT = 1.15
 # The sums of the fp32 kernels hold their rounding, which short slices keep small: the route's error (in the 2-norm, against 64 bits,
 # normal, uniform, heavy-tailed and scaled values) is 0.2 .. 0.8 of theirs on slices of the same depth, 0.9 at four times the depth, above theirs
 # from seven times on (1602 x 178 x 10 x 4485 uncut against 8 slices 5.8e-7 / 4.2e-7).
@@ -311,7 +314,7 @@ def _route_of_any_size(plan):
     if not forms:
         return None
     route_us, route = min((_route_us(plan, *form[:2]), form) for form in forms)
-    if _ROUTE_ADVANTAGE * route_us >= fp32_us or _backend.norm_gradient_workspace_bytes(plan.params) > 0:
+    if (_ROUTE_ADVANTAGE if route[0] == 1 else _ROUTE_ADVANTAGE_CUT) * route_us >= fp32_us or _backend.norm_gradient_workspace_bytes(plan.params) > 0:
         return None
     return route
 

@@ -124,7 +124,7 @@ _ROWS = (
     ("`cdist_grad`, p = 2", "a model of both times favours the route by {GRADIENT_L2_ADVANTAGE_PERCENT} %, and the planes of `out` form one matrix",
      "`gradient_l2_prepare`, `gradient_l2_pieces_stats` and `_split`, `gram_f16_wide<GW_EPILOGUE_GRADIENT_L2>`"),
     ("`cdist_grad`, p = 1, below its rule", "with memory for it, where models of the launch times favour the route, uncut or cut over k, over the fp32 kernels by a factor of "
-     "{cdist_grad.ROUTE_ADVANTAGE}, its slices at most {cdist_grad.ROUTE_MAX_DEPTH_RATIO} times as deep as theirs", "the same route (`KMC_FLAG_GRAM_WORKSPACE_ANY_SIZE`)"),
+     "{cdist_grad.ROUTE_ADVANTAGE} (cut {cdist_grad.ROUTE_ADVANTAGE_CUT}), its slices at most {cdist_grad.ROUTE_MAX_DEPTH_RATIO} times as deep as theirs", "the same route (`KMC_FLAG_GRAM_WORKSPACE_ANY_SIZE`)"),
     ("`cdist_grad`, otherwise", "O ≤ 8 / O > 8", "`norm_kernel_gradient` (vector ALU) / `norm_kernel_gradient_mfma` (fp32 matrix instruction), in runs of 32, 16 and ≤ 8 outputs; "
      "unbatched calls of fewer than {cdist_grad.SPLIT_BELOW_WORKGROUPS} workgroups are cut over k"),
     ("`run_kernel(..., coefficients=)`, squared differences, l2 mode `\"auto\"`",
