@@ -260,7 +260,7 @@ def _f16_slices(M, N, O):
 # everywhere; below it stand calls that the fp32 kernels, a workgroup walking the whole of k, take far longer for.  Which is
 # the faster one there follows from launch times in microseconds, fitted to sweeps of M 64 .. 12000, N 8 .. 1024, K 64 .. 12000, O 1 .. 64, one
 # problem or a batch of two (the fits are off by 13 .. 19 %).  An uncut route that they favour by 25 % is taken, one cut
-# over k by 15 %.  Of 260 other calls that they favour at all, the 171 uncut ones beyond 25 % are 0.97 .. 8.1 times as fast and the 41 cut ones beyond 15 % 0.94 .. 2.0 (two
+# over k by 15 %.  Of 260 other calls that they favour at all, the 171 uncut ones beyond 25 % are 0.97 .. 8.1 times as fast and the 41 cut ones beyond 15 % 0.94 .. 2.1 (two
 # slower, 68 x 13 x 2 x 3117 77 -> 82 us); the 16 uncut ones favoured by 15 to 25 % were 0.82 .. 1.6 (8808 x 37 x 16 x 174 44 -> 53 us).
 # fp32 / route, us: 768 x 28 x 1 x 1651 twice 191 / 56; 192 x 22 x 32 x 1088 118 / 39; 428 x 18 x 4 x 256 40 / 23; 10304 x 675 x 1 x 175 117 / 227.
 # Not the L2 gradient, below its own rule: the pieces of a and of c (b - s) are scaled by the largest magnitude of a row and hold what lies far below it to

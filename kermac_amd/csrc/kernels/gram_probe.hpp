@@ -6,7 +6,7 @@
 // This kernel looks first, at the operands as the caller holds them: BK_SAMPLE_TILES tiles of the result over
 // the batch, 16 consecutive rows of each operand from each, their 256 pairs over up to 128 of the k (8 runs of
 // 16 spread over the contraction), judged by the matrix-core kernels' own criterion on those k -- near-duplicates
-// fail it on any subset of k.  A workgroup owns one sampled tile and one word of the result, which it writes
+// fail it on any subset of k -- and one of those that a wave finds close there on all k.  A workgroup owns one sampled tile and one word of the result, which it writes
 // whole: nothing is accumulated across workgroups, so nothing has to be cleared and the order of the workgroups
 // does not matter.  build_kernel.hpp's sample_leaves_it_to_the_direct_kernel turns the words into the decision,
 // inside the matrix-core kernels.  The reference has no counterpart (it has no matrix-core path).
@@ -112,7 +112,8 @@ __device__ __forceinline__ void gram_probe_tile(const GramProbeArgs &args, int t
         va[r] = probe_element(a, args.a_ld, args.a_k_contiguous, m, min(first_of(r) + k_a, args.k - 1));
         vb[r] = probe_element(b, args.b_ld, args.b_k_contiguous, n, min(first_of(r) + k_b, args.k - 1));
     }
-    if (centre && !(args.centre_pairs && sums.needless())) {
+    if (centre && args.centre_pairs && sums.needless()) centre = nullptr;
+    if (centre) {
 #pragma unroll
         for (int r = 0; r < GP_RUNS; r++) {
             va[r] -= centre[min(first_of(r) + k_a, args.k - 1)];
@@ -138,7 +139,32 @@ __device__ __forceinline__ void gram_probe_tile(const GramProbeArgs &args, int t
         d2 += (y - x) * (y - x);
         norms += x * x + y * y;
     }
-    if (!(d2 >= args.trust * norms)) atomicAdd(&below_in_tile, 1u);
+    const unsigned long long close = __ballot(!(d2 >= args.trust * norms));
+    unsigned below = (unsigned)__popcll(close);
+    if (below > 0u && slices > GP_RUNS) {
+        // A pair that is close on these k need not be on all of them: where a few k hold most of every distance, as features of very different scales do, the others
+        // say nothing.  The wave takes the first of its close pairs, over all k, for all of them.  (Calls of such data that were mistaken for
+        // near-duplicates, without / with this, us and the error's 2-norm: 390 x 448 x 1552 twice, scales over 3 decades, 550 / 89, 6.3e-7 / 4.0e-8; 734 x 3776 x 3805 times 10
+        // coefficients, 6 decades, 1258 / 227, 2.0e-6 / 1.7e-7; 7358 x 1472 x 426, 8 decades, 272 / 76.  Near-duplicates: 2000 x 2000 x 784 265 / 265, 3000 x 3000 x 3072 1644 / 1649;
+        // with all pairs of such a tile looked at through LDS, 64 k at a time, 287 and 1745.)
+        const int pair = (t & ~63) + __builtin_ctzll(close);
+        const int pair_m = min(m0 + pair % BK_SAMPLE_ROWS, args.m - 1), pair_n = min(n0 + pair / BK_SAMPLE_ROWS, args.n - 1);
+        d2 = norms = 0.0f;
+#pragma unroll 4
+        for (int k = t & 63; k < args.k; k += 64) {
+            const float at = centre ? centre[k] : 0.0f;
+            const float x = probe_element(a, args.a_ld, args.a_k_contiguous, pair_m, k) - at, y = probe_element(b, args.b_ld, args.b_k_contiguous, pair_n, k) - at;
+            d2 += (y - x) * (y - x);
+            norms += x * x + y * y;
+        }
+#pragma unroll
+        for (int offset = 32; offset > 0; offset >>= 1) {
+            d2 += __shfl_xor(d2, offset);
+            norms += __shfl_xor(norms, offset);
+        }
+        if (d2 >= args.trust * norms) below = 0u;
+    }
+    if ((t & 63) == 0 && below > 0u) atomicAdd(&below_in_tile, below);
     __syncthreads();
     if (t == 0) args.sample[tile] = below_in_tile | (below_in_tile > 0u ? 0x10000u : 0u);
 }
