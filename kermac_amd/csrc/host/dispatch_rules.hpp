@@ -1,9 +1,10 @@
 // Every threshold by which the library decides, from the shape of a call alone, whether a route
-// through a workspace applies, and which variant of the direct kernel is launched.  This table is the only place where these numbers live: the rules
+// through a workspace applies, and which variant of the direct kernel is launched.  This table is the only place where the library's numbers live (the Python layer's default
+// mode, which asks for a route where it has measured it to be the faster one, has rules of its own on top, as constants beside their figures): the rules
 // (launch_one in kernels/build_kernel_inst.hip, wide_pays in kernels/gram_f16_wide_inst.hip, fixed_pays in kernels/l1_fixed_inst.hip, f16_pays in
 // kernels/norm_gradient_f16_inst.hip, gradient_l2_pays in kernels/gram_f16_wide_inst.hip) read them
 // from here, kmc_dispatch_rules() prints them, and the Python layer builds its "which kernel runs
-// when" table from that print-out.  Where each number comes from (the sweeps) is told next to the rule
+// when" table from that print-out and from its own constants.  Where each number comes from (the sweeps) is told next to the rule
 // that uses it.  Tiles are counted in 256 x 256 for the matrix-core routes and in 128 x 128 for the others, where a line does not say otherwise.
 #pragma once
 

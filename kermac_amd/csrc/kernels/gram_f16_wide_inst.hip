@@ -42,20 +42,14 @@ struct WideLayout {
     int64_t bytes;
 };
 
-// Whether the route pays for its extra launches.  Tiles are counted in 256 x 256, the rows that an operand is padded to.  The sweeps
-// against the one-step kernel below are of the product kernel before the present tiles of 256 x 128 and 128 x 128, one workgroup of
-// 256 x 256 per CU; the present one is faster almost everywhere, so that these lines keep some calls on a slower kernel and send hardly any to one
-// (one-step / route, us, today, calls that the rule leaves to the one-step kernel: k contiguous 1500 x 1500 x 784 102 / 50, 2000 x 2000 x 256
-// 60 / 41, 8 x 512 x 512 x 784 64 / 53, 100 x 50000 x 784 185 / 142; rows contiguous 2000 x 2000 x 2048 173 / 117, 3000 x 3000 x 784
-// 140 / 98, 1000 x 30000 x 256 161 / 111; the other way round, 16 x 512 x 512 x 2048 with k contiguous, 144 / 171).  One-step / wide time then:
-//   * over all tiles of the batch: K = 1024 1.09 at 144 tiles, 1.3 at 256, 1.6 from 1024 on; K = 256 0.99
-//     at 576, 1.15 at 1024, 1.25 at 4096; K = 64 1.0 at 1024, 1.07 from 2304 on; K = 32 never above 1;
-//   * the split of the operands is paid once per row and earned back once per tile the row meets, so
-//     each batch entry needs tiles in both directions: at K = 1024, 64 entries of 2 x 2 tiles 0.74,
-//     of 4 x 4 1.03, of 8 x 8 1.25, of 16 x 16 1.46; 118 x 4 tiles 1.26, 118 x 2 0.83, 391 x 2 0.84.
-//     The rule asks tiles_m * tiles_n / (tiles_m + tiles_n) >= 2.5 (5 x 5, or 4 x 7, or 3 x 15);
-//   * rows that pad the last tile are computed and thrown away: 8 entries of 1280 x 1280 1.24, of
-//     1290 x 1290 (6 x 6 tiles, 30 % padding) 0.86.  The rule asks for at most 20 % padding.
+// Whether the route pays for its extra launches, for a caller who leaves that to the library.  (With KMC_FLAG_GRAM_WORKSPACE_ANY_SIZE the caller has decided: the Python
+// layer's default mode does for nearly all squared differences from K = 128 on and for products with coefficients, by the rules and figures in
+// build_a_kernel.py and kernel_coefficients.py.)  Tiles are counted in 256 x 256, the rows that an operand is padded to.
+// The lines for squared differences stand where the one-step kernels and a slower product kernel, one workgroup of 256 x 256 per CU, crossed: tiles over the batch and tiles * k; tiles
+// in both directions of an entry, since the split is paid per row and earned back per tile the row meets; little padding.  The present kernel is
+// faster almost everywhere, so that they keep some calls on a slower kernel and send hardly any to one.  One-step / route, us, of calls that they leave to
+// the one-step kernel: k contiguous 1500 x 1500 x 784 102 / 50, 2000 x 2000 x 256 60 / 41, 8 x 512 x 512 x 784 64 / 53, 100 x 50000 x 784 185 / 142; rows contiguous 3000 x 3000 x 784
+// 140 / 98, 1000 x 30000 x 256 161 / 111; the other way round, 16 x 512 x 512 x 2048 with k contiguous, 144 / 171.
 // KERMAC_AMD_WIDE_MIN_TILES = t replaces the rule by "at least t tiles" (read on every call, so that
 // a test can send small shapes down the route).
 // Sums of products have no one-step matrix-core kernel to fall back to: the alternative is the direct
@@ -68,18 +62,13 @@ struct WideLayout {
 // only from 64 tiles on: the direct path cuts such a call over k (1500 x 1500, 36 tiles: 0.77 .. 0.84).
 //
 // Operands with k contiguous (row-major, as torch allocates them): the one-step kernels stage such operands
-// more slowly, the route splits them once and walks pieces whose layout is its own, so it pays much earlier
-// and whatever the shape of a batch entry (one-step / route time: 64 tiles 1.2 at K = 784, 1.5 at K = 3072, also
-// as 16 entries of 2 x 2 tiles with a third of the tiles padding; 144 tiles 1.1 at K = 256, 1.8 at K = 784;
-// 2 x 118 tiles 1.07 at K = 256, 1.3 at K = 784; 36 tiles 0.9 / 1.2; 32 tiles as 8 entries of 2 x 2 0.75 / 0.8;
-// K = 128 never above 1).  Not for a dimension that half a tile holds, where the 128 x 128 tiles of the
-// one-step kernels waste half as much (100 x 50000: 0.87 at K = 784, 4 entries 0.73; 128 x 20000 0.8).
+// more slowly, the route splits them once and walks pieces whose layout is its own, so it pays earlier
+// and whatever the shape of a batch entry.  Not for a dimension that half a tile holds, where the 128 x 128 tiles of the
+// one-step kernels waste half as much.
 //
 // A set against itself (the tiles of one triangle): one round of workgroups either way, whose walk is the route's faster one
 // (one-step split kernel / route, us, k contiguous: 1400 points, 21 tiles, at K = 784 77 / 63; 2000 at K = 256 66 / 52, at
-// K = 784 152 / 65, at K = 3072 502 / 160; 3000 at K = 128 59 / 50; 4 x 1000 at K = 784 163 / 67; 1000 at K = 784, 10 tiles, 63 / 61;
-// rows contiguous: 2000 at K = 784 82 / 85, at K = 3072 248 / 167; 2400 at K = 1024 106 / 90; 3500 at K = 512 95 / 88, a hair below the line; 3000 at
-// K = 128 46 / 70).
+// K = 784 152 / 65; rows contiguous: 2400 at K = 1024 106 / 90; 3000 at K = 128 46 / 70).
 bool wide_pays(int64_t m, int64_t n, int64_t tiles_m, int64_t tiles_n, int64_t tiles, int k, bool products, bool k_contiguous,
                bool batched, bool symmetric)
 {
@@ -102,7 +91,7 @@ bool wide_pays(int64_t m, int64_t n, int64_t tiles_m, int64_t tiles_n, int64_t t
     if (products) return k >= r::DOT_MIN_K && tiles >= r::DOT_MIN_TILES && tiles * k >= r::DOT_MIN_TILES_TIMES_K && little_padding;
     // (from 768 tiles on the route is as fast as the one-step kernel also for the shortest contractions
     // it takes, 8192 x 8192 x 64 180 us against 187, and ahead of the direct kernel, 236)
-    // (long contractions of few tiles, today, one-step / route, us: 1500 x 1500 x 2048 129 / 75, 2048 x 2048 x 2048 173 / 88, 1800 x 1500 x 4000 294 / 126)
+    // (long contractions of few tiles, one-step / route, us: 1500 x 1500 x 2048 129 / 75, 2048 x 2048 x 2048 173 / 88, 1800 x 1500 x 4000 294 / 126)
     const bool long_walk = k >= r::WIDE_LONG_MIN_K && ((m + 127) / 128) * ((n + 127) / 128) >= r::WIDE_LONG_MIN_TILES && !k_contiguous && !symmetric;
     if (!long_walk && (k < r::WIDE_MIN_K || tiles < r::WIDE_MIN_TILES || (tiles * k < r::WIDE_MIN_TILES_TIMES_K && tiles < r::WIDE_TILES_FOR_ANY_K))) return false;
     if (2 * tiles_m * tiles_n < r::WIDE_MIN_TILES_PER_SIDE_X2 * (tiles_m + tiles_n)) return false;
@@ -355,10 +344,9 @@ hipError_t launch_product_in(kmc::GramWideArgs &wide, hipStream_t stream)
     const int64_t width = SYMMETRIC ? blocks * (blocks + 1) / 2 * (kmc::GW_TILE / Tile::TILE_M) * (kmc::GW_TILE / Tile::TILE_N)
                                     : static_cast<int64_t>(wide.wide_tiles_m) * padded;
     if (width > 0x7fffffff) return hipErrorInvalidValue;
-    // An entry of a batch on one XCD, with how it was spread over all of them and with the kernel before these tiles (half as many reads of
-    // an operand), us: 64 x 300 x 300 x 4096, products, 866 / 1009 / 946; 16 x 1280 x 1280 x 4096 1010 / 1174 / 1108; 10 x 1100 x 1100 x 4096
-    // 637 / 733 / 664; 64 x 600 x 600 x 4096 1593 / 1993 / 1886; 500 x 300 x 300 x 784 1207 / 1408 / 1793; 40 sets of 900 points of K = 784
-    // against themselves 224 / 251; 10 x 1500 x 100 x 8 x 4000, the gradient, 738 / 836 / 754.  Larger entries keep an XCD's L2 busy by themselves
+    // An entry of a batch on one XCD / spread over all of them, us: 64 x 300 x 300 x 4096, products, 866 / 1009; 16 x 1280 x 1280 x 4096 1010 / 1174;
+    // 10 x 1100 x 1100 x 4096 637 / 733; 64 x 600 x 600 x 4096 1593 / 1993; 500 x 300 x 300 x 784 1207 / 1408; 40 sets of 900 points of K = 784
+    // against themselves 224 / 251; 10 x 1500 x 100 x 8 x 4000, the gradient, 738 / 836.  Larger entries keep an XCD's L2 busy by themselves
     // and gain nothing: 20 x 2000 x 2000 (256 tiles each) 248 / 236 at K = 256, 536 / 535 at K = 784; 8 x 4096 x 4096 x 784 752 / 702.
     wide.entry_per_xcd = wide.kernel.l >= kmc::BK_XCDS &&
                          static_cast<int64_t>((wide.kernel.m + 127) / 128) * ((wide.kernel.n + 127) / 128) <= kmc_rules::WIDE_ENTRY_PER_XCD_MAX_TILES;
@@ -373,7 +361,7 @@ hipError_t launch_product_in(kmc::GramWideArgs &wide, hipStream_t stream)
 // Above one round of small tiles (three on each of 256 CUs) the few of the second round have the chip to themselves; where the large
 // tiles are one round (two per CU) they are taken instead, as long as the second round of small ones is little or the contraction long.
 // Not for a set against itself, whose rounds are of unequal tiles.  Small / large, us, k contiguous: 800 small tiles, 8 x 1280 x 1280 of
-// K = 784 129.4 / 127.5, of K = 4096 644 / 617 (a workgroup of 256 x 256 per CU, the kernel before these, 147 and 570); 840, 28 x 640 x 768 of
+// K = 784 129.4 / 127.5, of K = 4096 644 / 617; 840, 28 x 640 x 768 of
 // K = 784 210 / 185, of K = 4096 1072 / 934; 784, 3584 x 3584 of K = 784 100 / 96, of K = 4096 395 / 371; 938, 200 x 60000 of K = 784 194.4 / 197.5,
 // of K = 2048 568 / 561; 1024, 4096 x 4096 of K = 784 103.1 / 103.8, of K = 4096 432 / 421; more than one round of either: 1156,
 // 4352 x 4352 of K = 2048 276 / 306.  A set against itself: 780, 4900 points of K = 784 110 / 120; 990, 5632 of K = 784 130 / 127.
@@ -563,8 +551,8 @@ struct GradientL2Layout {
 //                  6.3e-9 per multiply-add of the padded tiles but not less than 0.056 k (1.7 us per 256 x 256 x 16 step of a CU
 //                  with the chip full, 0.9 us alone; the present kernel takes 4.7e-9 with the chip full).
 // Examples (fp32 / this route, measured with the present kernel): 8192 x 512 x 16 x 8192 3.0; o = 1 4.3, o = 32 3.2; n = 64 1.65;
-// m = 1024 1.6; k = 512 1.8, k = 256 1.2; 10000 x 1000 x 10 x 784 3.4.  With the kernel before: n = 32 0.96, n = 8 0.81;
-// m = 512 0.86; k = 64 0.40.  KERMAC_AMD_GRADIENT_L2_MIN_TERMS replaces the rule by a number of terms
+// m = 1024 1.6; k = 512 1.8, k = 256 1.2; 10000 x 1000 x 10 x 784 3.4.  Calls below stay on the fp32 kernels, which
+// are more exact where the rows of a and c have opposite scales (cdist_grad.py).  KERMAC_AMD_GRADIENT_L2_MIN_TERMS replaces the rule by a number of terms
 // (read on every call, so that a test can send small shapes down the route).
 bool gradient_l2_pays(const kmc_norm_gradient_params *p, int64_t tiles_m, int64_t tiles_n)
 {

@@ -39,11 +39,9 @@ int64_t round_up(int64_t value, int64_t multiple) { return (value + multiple - 1
 // terms to carry the extra launch and the ranking, and more than two outputs (a workgroup costs the same for 1 .. 8 and for
 // 9 .. 16 outputs; the vector kernel for one or two is cheap).  Few outputs make the fp32 kernels cheaper nearly in proportion and not the
 // route, so the terms are asked for in proportion: 4e8 at 16 outputs, 1.6e9 at 4.  Its smallest tile holds 32 n.
-// The limits are those of the kernel before this one, which needed five more launches and a third matrix instruction, fp32 / that kernel's time:
-// O = 16 at 3.4e10 terms 2.5, 1.1e9 1.8, 5.4e8 1.1 .. 1.4, 2.7e8 0.8 .. 1.1, 1.3e8 0.66; at 3.4e10 terms O = 1 0.73, O = 2 0.93, O = 3 1.21, O = 4
-// 1.31, O = 8 2.1; N = 16 0.86, N = 32 1.37.  Of 57 shapes that they send down the route the present kernel is 1.55 times as fast as the fp32
+// The limits are those of a slower kernel with five more launches.  Of 57 shapes that they send down the route the present one is 1.55 times as fast as the fp32
 // kernels or more (11200 x 112 x 16 x 320 1.55, 4000 x 32 x 16 x 4000 1.80, 6862 x 105 x 24 x 417 1.96): they lose nothing, and leave calls to
-// the fp32 kernels that the route would win.
+// the fp32 kernels that the route would win; the Python layer takes those by models of both times (cdist_grad.py).
 // KERMAC_AMD_GRADIENT_F16_MIN_TERMS replaces the conditions by a number of terms (read on every
 // call, so that a test can send small shapes down the route).
 bool f16_pays(const kmc_norm_gradient_params *p)
