@@ -541,7 +541,7 @@ def main():
         per_p["2.0"]["l2_mode"] = kermac.get_l2_mode()
         per_p["2.0"]["note"] = ("default mode 'auto': |a-c|^2 + |b-c|^2 - 2 (a-c).(b-c), c = sample mean, with the cross term on "
                                 "the fp16 matrix instruction (both operands split once into two fp16 pieces per value, scaled per "
-                                "row, in a workspace; 256 x 256 tiles; three piece products), ill-conditioned 128 x 128 parts "
+                                "row, in a workspace; 256 x 128 tiles; three piece products), ill-conditioned 128 x 128 parts "
                                 "recomputed by the direct kernel; the vector-ALU kernel is per_p['2.0_direct']")
         # The default mode on data that defeats the matrix-core route: 64 tight clusters far apart (centres N(0, 10^2),
         # noise 1e-3, seed 11), so one pair in 64 is a pair of near-duplicates and every 128 x 128 part holds some.  The
