@@ -656,7 +656,7 @@ def run_kernel(
         # library has no use for a workspace for is an ordinary call of the direct kernel
         workspace = _attach_gram_workspace(params, a.device, needed=route_bytes)
         if workspace is None:
-            params.flags &= ~(_backend.FLAG_DOT_PIECES | _backend.FLAG_GRAM_WORKSPACE_ANY_SIZE)
+            params.flags &= ~_backend.FLAG_DOT_PIECES
         plan.keepalive.append(workspace)
     if params.flags & _backend.FLAG_L1_FIXED:
         # the fixed-point route exists only through a workspace: without one (a problem too small
